@@ -340,6 +340,16 @@ int tnn_grid_backward(const tnn_grid_desc *desc, const float *d_x, const void *d
 int tnn_grid_backward_ordered(const tnn_grid_desc *desc, const void *d_order, const void *d_dLdy, int dy_dtype,
                               uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, tnn_stream_t stream);
 
+/* tnn_grid_backward (d_x given) or tnn_grid_backward_ordered (d_order given, with d_x beside it or NULL) with scratch
+ * memory, for large batches: the contributions to levels beyond an LDS copy are sorted by destination into the workspace and
+ * summed on chip, where the calls above add each of them to the table with atomics. The same contributions in another order
+ * of addition. Workspace: tnn_grid_backward_workspace_bytes, which grows with the batch up to 2^18 points (config 4: 96 MiB)
+ * and no further; nothing in it has to be cleared. */
+size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size_t M);
+int tnn_grid_backward_binned(const tnn_grid_desc *desc, const float *d_x, const void *d_order, const void *d_dLdy, int dy_dtype,
+                             uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
+                             tnn_stream_t stream);
+
 /* The same scatter into an fp16 gradient table, two features of an entry per packed atomic (global_atomic_pk_add_f16): half
  * as many atomic operations as the fp32 route and half the gradient table; the same number of 32-byte requests at the memory
  * side, which is what bounds the pass, so about the same time. No counterpart in the reference, whose

@@ -1,0 +1,63 @@
+"""The scatter that sorts its contributions by destination (tnn_grid_backward_binned) against the oracle and the plain scatter."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from tolerances import BF16, FP16, FP32
+
+pytestmark = pytest.mark.gpu
+
+CFG2 = dict(n_dims=2, n_levels=16, n_features_per_level=2, log2_hashmap_size=15, base_resolution=16, per_level_scale=1.5)
+CFG3 = dict(n_dims=3, n_levels=16, n_features_per_level=2, log2_hashmap_size=19, base_resolution=16, per_level_scale=1.447)
+DT = {FP32: torch.float32, FP16: torch.float16, BF16: torch.bfloat16}
+
+
+def binned(tnn, d, x, g, dtype, ordered=False, grad=None, overwrite=True, short=0):
+    from tiny_dpcpp_nn import _lib
+    M = x.shape[0]
+    p = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None  # noqa: E731
+    need = tnn.lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), M)
+    work = torch.full((max(need - short, 1),), 0xA5, dtype=torch.uint8, device=tnn.dev)  # nothing in it has to be cleared
+    order = tnn.grid_order(d, x) if ordered else None
+    if grad is None:
+        grad = torch.full((tnn.grid_n_params(d),), 0.123, dtype=torch.float32, device=tnn.dev)
+    _lib.check(tnn.lib.tnn_grid_backward_binned(ctypes.byref(d), None if ordered else p(x), p(order), p(g), dtype, g.shape[1], p(grad), int(overwrite), M,
+                                                p(work), work.numel(), tnn.stream()))
+    return grad
+
+
+@pytest.mark.parametrize("cfg", [CFG2, CFG3, dict(CFG3, log2_hashmap_size=22, n_levels=12), dict(CFG2, n_features_per_level=1, hash="Prime"),
+                                 dict(CFG3, n_features_per_level=4, n_levels=8, interpolation="Smoothstep"), dict(CFG2, n_features_per_level=8, n_levels=7),
+                                 dict(CFG3, interpolation="Nearest"), dict(CFG2, grid_type="Dense", n_levels=9), dict(CFG2, grid_type="Tiled")])
+@pytest.mark.parametrize("M,ordered,kind", [(1, False, "uniform"), (513, False, "uniform"), (40007, True, "uniform"), (40007, False, "few"), (2 ** 18 + 9, False, "uniform")])
+def test_binned_scatter_matches_the_oracle(tnn, oracle, cfg, M, ordered, kind):
+    """Bins that overflow ("few": all points on some twenty cells), a batch of more than one part, edges of bins, every kind of level. fp32 sums
+    in another order against the oracle's double sum, at the plain scatter's bar; accumulate mode adds on top."""
+    rng = np.random.default_rng(M + cfg["n_dims"])
+    x = rng.uniform(0, 1, (M, cfg["n_dims"])).astype(np.float32)
+    if kind == "few":
+        x = x[rng.integers(0, 20, M)]
+    x[0] = 1.0
+    pw = cfg["n_levels"] * cfg["n_features_per_level"] + 4
+    d = tnn.grid_desc(cfg)
+    g = torch.from_numpy(rng.standard_normal((M, pw)).astype(np.float32)).to(tnn.dev)
+    xt = torch.from_numpy(x).to(tnn.dev)
+    for dtype in (FP32, BF16, FP16) if M == 513 else (FP32,):
+        gt = g.to(DT[dtype]).contiguous()
+        grad = binned(tnn, d, xt, gt, dtype, ordered)
+        ref = oracle.grid_backward(cfg, x, gt.float().cpu().numpy(), tnn.grid_n_params(d))
+        bar = 1e-5 * max(1.0, np.abs(ref).max())
+        assert np.abs(grad.cpu().numpy() - ref).max() <= bar
+        twice = binned(tnn, d, xt, gt, dtype, ordered, grad=grad.clone(), overwrite=False)
+        assert np.abs(twice.cpu().numpy() - 2 * ref).max() <= 2 * bar
+
+
+def test_binned_workspace_is_checked(tnn):
+    from tiny_dpcpp_nn import _lib
+    d = tnn.grid_desc(CFG3)
+    x = torch.rand((4096, 3), device=tnn.dev)
+    with pytest.raises(_lib.TnnError):
+        binned(tnn, d, x, torch.rand((4096, 32), device=tnn.dev), FP32, short=4096)
+    assert tnn.lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), 0) == 0

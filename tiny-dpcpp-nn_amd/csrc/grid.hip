@@ -10,11 +10,12 @@
 // written as contiguous 16-byte pieces. Per-level constants (scale, resolution, table offset, size,
 // how many dimensions enter the dense index, whether the level is hashed) are evaluated once on the
 // host and reach the kernel as scalar kernel arguments; no thread evaluates exp2.
-#include "grid_device.h"
+#include "grid_binned.h"
 
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 namespace tnn {
 
@@ -146,11 +147,12 @@ __global__ void __launch_bounds__(kGridThreads)
 
 // Which levels the backward pass accumulates in LDS first, and how the 1-D grid is split between the two routes.
 struct BackwardPlan {
-    uint32_t n_small;          // levels whose whole gradient slice fits the LDS budget
-    uint32_t small_blocks;     // workgroups per such level, each takes `chunk` consecutive points
+    uint32_t n_small;          // levels, or single features of levels, of which a copy fits the LDS budget
+    uint32_t small_blocks;     // workgroups per such part, each takes `chunk` consecutive points
     uint32_t chunk;
     uint32_t big_blocks;       // workgroups per other level, a group of lanes per point
     uint8_t small_level[TNN_GRID_MAX_LEVELS];
+    uint8_t small_feature[TNN_GRID_MAX_LEVELS];
     uint8_t big_level[TNN_GRID_MAX_LEVELS];
     // Points in cell order only: levels too large for a private copy of the whole level, where a stretch of consecutive
     // points still lands on few enough cells for a private copy of the box around them (kMaxTiled such levels).
@@ -164,6 +166,7 @@ struct BackwardPlan {
     uint32_t n_rows;
 };
 constexpr uint32_t kMaxTiled = 16;
+constexpr uint8_t kAllFeatures = 255;
 #ifndef TNN_BOXED_MIN_PER_CELL
 #define TNN_BOXED_MIN_PER_CELL 0.3
 #endif
@@ -274,10 +277,10 @@ template <int STEP, int FV> __device__ __forceinline__ void segmented_step(float
 //     are dispatched together, so its slice of the table is the hot one in L2.
 template <int D, int F, typename G, typename GT>
 __global__ void __launch_bounds__(kBwdThreads)
-    grid_backward_kernel(const GridLevels lv, const GridParams gp, const BackwardPlan bp, const float *__restrict__ xin,
+    grid_backward_kernel(const GridLevels lv, const GridParams gp, const BackwardPlan bp, const GradLayout dl, const float *__restrict__ xin,
                          const float4 *__restrict__ order, const uint32_t *__restrict__ bin_start, const G *__restrict__ dLdy,
                          GT *__restrict__ grad, long long M) {
-    extern __shared__ float priv[];
+    extern __shared__ double priv[];
     const uint32_t n_small_blocks = bp.n_small * bp.small_blocks;
     // Workgroups start in the order of their numbers. Those of the LDS routes and those of the direct route are bound by
     // different things (LDS atomics; atomic requests to memory), so their numbers are interleaved in proportion: both kinds
@@ -290,36 +293,55 @@ __global__ void __launch_bounds__(kBwdThreads)
                                  : blockIdx.x >= n_lds_blocks;
     const uint32_t lds_block = blockIdx.x - n_direct_before; // this workgroup's number among those of its kind
     if (!is_direct && lds_block < n_small_blocks) {
-        const uint32_t l = bp.small_level[lds_block / bp.small_blocks];
+        // the features of the level this workgroup adds: all, or one where a copy of all of them does not fit
+        const uint32_t part = lds_block / bp.small_blocks, l = bp.small_level[part];
+        const uint32_t f_first = bp.small_feature[part] == kAllFeatures ? 0 : bp.small_feature[part];
+        const uint32_t n_f = bp.small_feature[part] == kAllFeatures ? F : 1;
         const uint32_t size = lv.size[l], res = lv.resolution[l], flags = lv.flags[l];
         const float scale = lv.scale[l];
-        const uint32_t n = size * F;
-        for (uint32_t e = threadIdx.x; e < n; e += kBwdThreads) priv[e] = 0.0f;
+        for (uint32_t e = threadIdx.x; e < size * n_f; e += kBwdThreads) priv[e] = 0.0;
         __syncthreads();
         const long long first = (long long)(lds_block % bp.small_blocks) * bp.chunk;
         const long long last = first + bp.chunk < M ? first + bp.chunk : M;
-        for (long long i = first + threadIdx.x; i < last; i += kBwdThreads) {
+        // In cell order the lanes of a wave take points a stripe apart, as below: neighbours would queue up on one LDS address.
+        const uint32_t wave_no = threadIdx.x / kGridWave, lane = threadIdx.x % kGridWave;
+        const uint32_t start = order ? lane * (bp.chunk / kGridWave) + wave_no : threadIdx.x;
+        const uint32_t step = order ? kBwdThreads / kGridWave : kBwdThreads, turns = bp.chunk / kBwdThreads;
+        for (uint32_t t = 0; t < turns; ++t) {
+            const long long i = first + start + (long long)t * step;
+            if (i >= last) continue;
             float x[D];
             const long long row = load_point<D>(xin, order, i, x);
+            const G *dy = dLdy + (dl.by_position ? i : row) * dl.row_stride + l * dl.level_stride + f_first;
             float gy[F];
 #pragma unroll
-            for (int f = 0; f < F; ++f) gy[f] = (float)dLdy[row * gp.padded_width + l * F + f];
+            for (int f = 0; f < F; ++f)
+                if (f < (int)n_f) gy[f] = (float)dy[f];
             for_each_corner<D>(x, scale, size, res, flags, gp.hash_type, gp.interpolation, [&](uint32_t idx, float w) {
 #pragma unroll
-                for (int f = 0; f < F; ++f) atomicAdd(&priv[idx * F + f], w * gy[f]);
+                for (int f = 0; f < F; ++f)
+                    if (f < (int)n_f) lds_add(&priv[idx * n_f + f], w * gy[f]);
             });
         }
         __syncthreads();
-        GT *g = grad + (size_t)lv.offset[l] * F;
-        for (uint32_t e = threadIdx.x; e < size; e += kBwdThreads) {
-            float v[F];
-            bool any = false;
-#pragma unroll
-            for (int f = 0; f < F; ++f) {
-                v[f] = priv[e * F + f];
-                any |= v[f] != 0.0f;
+        GT *g = grad + (size_t)lv.offset[l] * F + f_first;
+        if constexpr (std::is_same<GT, float>::value) {
+            // neighbouring lanes take neighbouring values, so that the values of a 32-byte sector leave in one request
+            for (uint32_t e = threadIdx.x; e < size * n_f; e += kBwdThreads) {
+                const float v = (float)priv[e];
+                if (v != 0.0f) unsafeAtomicAdd(g + (n_f == F ? e : (size_t)e * F), v);
             }
-            if (any) add_entry<F>(g + (size_t)e * F, v);
+        } else {
+            for (uint32_t e = threadIdx.x; e < size; e += kBwdThreads) {
+                float v[F];
+                bool any = false;
+#pragma unroll
+                for (int f = 0; f < F; ++f) {
+                    v[f] = (float)priv[e * F + f];
+                    any |= v[f] != 0.0f;
+                }
+                if (any) add_entry<F>(g + (size_t)e * F, v);
+            }
         }
         return;
     }
@@ -327,7 +349,7 @@ __global__ void __launch_bounds__(kBwdThreads)
         // Cell order, a level whose workgroups each take stretches of consecutive points of one row of the order's coarse
         // cells (grid_order.hip walks the coarse cells row by row, x fastest, and leaves the first position of every
         // coarse cell behind the records): such a stretch lies in a few neighbouring cells, so the corners it touches fill
-        // a small box of the level's cells. The workgroup finds that box, accumulates in a private fp32 copy of it in LDS,
+        // a small box of the level's cells. The workgroup accumulates in a private fp32 copy of it in LDS,
         // and adds every touched entry to the table once. A stretch whose box does not fit (points far apart: the bins of
         // the points outside the unit cube, a sparse region) adds to the table directly.
         const uint32_t tb = lds_block - n_small_blocks;
@@ -340,68 +362,34 @@ __global__ void __launch_bounds__(kBwdThreads)
         const float scale = lv.scale[l];
         const long long row_first = bin_start[rowno * bp.bins_per_row];
         const long long row_end = rowno + 1 < bp.n_rows ? (long long)bin_start[(rowno + 1) * bp.bins_per_row] : M;
-        __shared__ int box_lo[D], box_hi[D];
         // lane L of wave w takes the points L * stripe + w + n_waves * k of the stretch: the lanes of an instruction are a
         // stripe apart and rarely in the same cell, where consecutive points would queue up on one LDS address
         constexpr uint32_t n_waves = kBwdThreads / kGridWave;
         const uint32_t stripe = chunk / kGridWave, wv = threadIdx.x / kGridWave, ln = threadIdx.x % kGridWave;
-        const bool nearest = gp.interpolation == TNN_INTERP_NEAREST;
         GT *g = grad + (size_t)lv.offset[l] * F;
         for (long long first = row_first + (long long)piece * chunk; first < row_end; first += (long long)pieces * chunk) {
             const uint32_t count = (uint32_t)((first + chunk < row_end ? first + chunk : row_end) - first);
-            __syncthreads(); // the box and the private copy of the stretch before are done with
-            if (threadIdx.x < D) {
-                box_lo[threadIdx.x] = 0x7fffffff;
-                box_hi[threadIdx.x] = (int)0x80000000;
-            }
-            __syncthreads();
-            int lo[D], hi[D];
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                lo[d] = 0x7fffffff;
-                hi[d] = (int)0x80000000;
-            }
-            for (uint32_t k = wv; k < stripe; k += n_waves) {
-                const uint32_t pl = ln * stripe + k;
-                if (pl >= count) continue;
-                float x[D];
-                load_point<D>(xin, order, first + pl, x);
-                uint32_t cell[D];
-                float frac[D];
-                cell_of<D>(x, scale, gp.interpolation, cell, frac);
+            // The cells the points of the coarse cells between the stretch's first and last can be in. Points outside the unit
+            // cube are in an end cell of the order; what lies outside the box adds to the table directly.
+            int lo[D];
+            uint32_t ext[D];
+            long long n_local = 1;
+            {
+                constexpr int bits = OrderBits<D>::coarse;
+                const uint32_t c0 = quantise(order[first].x, bits), c1 = quantise(order[first + count - 1].x, bits);
 #pragma unroll
                 for (int d = 0; d < D; ++d) {
-                    const int c = (int)cell[d];
-                    lo[d] = c < lo[d] ? c : lo[d];
-                    hi[d] = c > hi[d] ? c : hi[d];
+                    const uint32_t from = d == 0 ? c0 : (rowno >> (bits * (d - 1))) & ((1u << bits) - 1), to = d == 0 ? c1 : from;
+                    lo[d] = (int)floorf(__builtin_fmaf(scale, (float)from / (float)(1 << bits), 0.5f));
+                    const int hi = (int)floorf(__builtin_fmaf(scale, (float)(to + 1) / (float)(1 << bits), 0.5f));
+                    ext[d] = (uint32_t)(hi - lo[d] + 2); // the far corners are one cell further
+                    n_local *= ext[d];
                 }
             }
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-#pragma unroll
-                for (int off = kGridWave / 2; off > 0; off >>= 1) {
-                    const int a = __shfl_xor(lo[d], off, kGridWave), b2 = __shfl_xor(hi[d], off, kGridWave);
-                    lo[d] = a < lo[d] ? a : lo[d];
-                    hi[d] = b2 > hi[d] ? b2 : hi[d];
-                }
-                if (ln == 0 && lo[d] <= hi[d]) {
-                    atomicMin(&box_lo[d], lo[d]);
-                    atomicMax(&box_hi[d], hi[d]);
-                }
-            }
-            __syncthreads();
-            long long n_local = 1;
-            uint32_t ext[D];
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                lo[d] = box_lo[d];
-                const long long e = (long long)box_hi[d] - lo[d] + (nearest ? 1 : 2); // the far corners are one cell further
-                ext[d] = (uint32_t)e;
-                n_local = (e <= 0 || n_local > (1ll << 40)) ? (1ll << 41) : n_local * e;
-            }
-            const bool fits = n_local * F * (long long)sizeof(float) <= (long long)bp.budget;
+            const bool fits = n_local * F * (long long)sizeof(double) <= (long long)bp.budget;
             if (fits) {
-                for (uint32_t e = threadIdx.x; e < (uint32_t)n_local * F; e += kBwdThreads) priv[e] = 0.0f;
+                __syncthreads(); // the private copy of the stretch before is done with
+                for (uint32_t e = threadIdx.x; e < (uint32_t)n_local * F; e += kBwdThreads) priv[e] = 0.0;
                 __syncthreads();
             }
             for (uint32_t k = wv; k < stripe; k += n_waves) {
@@ -409,29 +397,32 @@ __global__ void __launch_bounds__(kBwdThreads)
                 if (pl >= count) continue;
                 float x[D];
                 const long long row = load_point<D>(xin, order, first + pl, x);
+                const G *dy = dLdy + (dl.by_position ? first + pl : row) * dl.row_stride + l * dl.level_stride;
                 float gy[F];
 #pragma unroll
-                for (int f = 0; f < F; ++f) gy[f] = (float)dLdy[row * gp.padded_width + l * F + f];
+                for (int f = 0; f < F; ++f) gy[f] = (float)dy[f];
                 uint32_t cell[D];
                 float frac[D];
                 cell_of<D>(x, scale, gp.interpolation, cell, frac);
+                bool inside = fits;
+#pragma unroll
+                for (int d = 0; d < D; ++d) inside &= (uint32_t)((int)cell[d] - lo[d]) < ext[d] - 1;
 #pragma unroll
                 for (int c = 0; c < (1 << D); ++c) {
-                    if (nearest && c > 0) break;
                     float weight = 1.0f;
                     uint32_t loc[D];
                     uint32_t local = 0, stride = 1;
 #pragma unroll
                     for (int d = 0; d < D; ++d) {
-                        const bool far = !nearest && (c & (1 << d));
-                        weight *= nearest ? 1.0f : (far ? frac[d] : 1 - frac[d]); // the products of for_each_corner
+                        const bool far = (c & (1 << d)) != 0;
+                        weight *= far ? frac[d] : 1 - frac[d]; // the products of for_each_corner
                         loc[d] = far ? cell[d] + 1 : cell[d];
                         local += (uint32_t)((int)loc[d] - lo[d]) * stride;
                         stride *= ext[d];
                     }
-                    if (fits) {
+                    if (inside) {
 #pragma unroll
-                        for (int f = 0; f < F; ++f) atomicAdd(&priv[local * F + f], weight * gy[f]);
+                        for (int f = 0; f < F; ++f) lds_add(&priv[local * F + f], weight * gy[f]);
                     } else {
                         float v[F];
 #pragma unroll
@@ -442,12 +433,14 @@ __global__ void __launch_bounds__(kBwdThreads)
             }
             if (!fits) continue;
             __syncthreads();
-            for (uint32_t e = threadIdx.x; e < (uint32_t)n_local; e += kBwdThreads) {
-                float v[F];
+            constexpr uint32_t VL = std::is_same<GT, float>::value ? F : 1; // lanes per entry (fp16 tables take features in pairs)
+            for (uint32_t n = threadIdx.x; n < (uint32_t)n_local * VL; n += kBwdThreads) {
+                const uint32_t e = n / VL;
+                float v[F / VL];
                 bool any = false;
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    v[f] = priv[e * F + f];
+                for (uint32_t f = 0; f < F / VL; ++f) {
+                    v[f] = (float)priv[n * (F / VL) + f];
                     any |= v[f] != 0.0f;
                 }
                 if (!any) continue;
@@ -457,7 +450,7 @@ __global__ void __launch_bounds__(kBwdThreads)
                     loc[d] = (uint32_t)(lo[d] + (int)(rest % ext[d]));
                     rest /= ext[d];
                 }
-                add_entry<F>(g + (size_t)level_index<D>(loc, size, res, flags, gp.hash_type) * F, v);
+                add_entry<F / VL>(g + (size_t)level_index<D>(loc, size, res, flags, gp.hash_type) * F + n % VL, v);
             }
         }
         return;
@@ -484,9 +477,10 @@ __global__ void __launch_bounds__(kBwdThreads)
     float x[D];
     const long long row = load_point<D>(xin, order, i, x);
     constexpr int FV = F / FL; // values per lane: 1 (fp32 table) or 2 (fp16 table)
+    const G *dy = dLdy + (dl.by_position ? i : row) * dl.row_stride + l * dl.level_stride + fl * FV;
     float gy[FV];
 #pragma unroll
-    for (int f = 0; f < FV; ++f) gy[f] = live ? (float)dLdy[row * gp.padded_width + l * F + fl * FV + f] : 0.0f;
+    for (int f = 0; f < FV; ++f) gy[f] = live ? (float)dy[f] : 0.0f;
     uint32_t cell[D];
     float frac[D];
     cell_of<D>(x, lv.scale[l], gp.interpolation, cell, frac);
@@ -539,11 +533,12 @@ __global__ void __launch_bounds__(kBwdThreads)
     }
 }
 
-__global__ void fill_zero_kernel(float4 *__restrict__ p, size_t n4, float *__restrict__ tail, size_t n_tail) {
+__global__ void fill_zero_kernel(float4 *__restrict__ p, size_t n4, float *__restrict__ tail, size_t n_tail, uint32_t *__restrict__ words, size_t n_words) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t k = i; k < n4; k += stride) p[k] = float4{0.f, 0.f, 0.f, 0.f};
     if (i < n_tail) tail[i] = 0.0f;
+    for (size_t k = i; k < n_words; k += stride) words[k] = 0;
 }
 
 int check_grid_desc(const tnn_grid_desc *d) {
@@ -588,25 +583,32 @@ static int launch_grid_forward_p(const tnn_grid_desc *d, const GridLevels &lv, c
     return launch_grid_forward_o<D, F, fp16_t>(lv, gp, x, order, table, out, out_dtype, M, s);
 }
 
-template <int D, int F, typename TAB>
-static int launch_grid_backward_g(const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *dLdy,
-                                  int dy_dtype, TAB *grad, size_t M, hipStream_t s) {
+// Which route every level takes: n_big levels are left for the direct one (bp->big_level), those of `bins` for the binned one
+// (grid_binned.hip), which needs scratch memory and is planned for only when `bins` is given.
+static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, uint32_t n_dims, uint32_t F, bool ordered, bool fp32_table, size_t M, BinPlan *bins,
+                                  uint32_t *n_big_levels, uint32_t *lds) {
+    const int D = (int)n_dims;
     // A level goes the LDS route when its slice fits the budget and a chunk of points makes clearly more atomics
     // than the flush of the private copy does (chunk * 2^D contributions against `size` entries).
     BackwardPlan bp{};
     bp.chunk = kPrivateChunk;
-    bp.budget = order ? kPrivateLdsBytesOrdered : kPrivateLdsBytes;
-    bp.small_blocks = (uint32_t)((M + bp.chunk - 1) / bp.chunk);
-    constexpr int per_block = kDirectPasses * kBwdThreads / (2 * BackwardLanes<F, TAB>::FL); // (point, level) pairs per workgroup on the direct route
-    bp.big_blocks = (uint32_t)((M + per_block - 1) / per_block);
+    bp.budget = ordered ? kPrivateLdsBytesOrdered : kPrivateLdsBytes;
     const size_t per_chunk = (M < bp.chunk ? M : (size_t)bp.chunk) << (gp.interpolation == TNN_INTERP_NEAREST ? 0 : D);
     uint32_t n_big = 0, lds_bytes = 0;
     for (uint32_t l = 0; l < gp.n_levels; ++l) {
-        const size_t bytes = (size_t)lv.size[l] * F * sizeof(float);
+        const size_t feature_bytes = (size_t)lv.size[l] * sizeof(double), bytes = feature_bytes * F;
         // (in cell order only the coarsest levels: the box of a stretch is far smaller than a level from 8 KiB on)
-        if (bytes <= (order ? 8192u : bp.budget) && per_chunk >= 2 * (size_t)lv.size[l]) {
+        const bool worth_it = per_chunk >= 2 * (size_t)lv.size[l];
+        if (worth_it && bytes <= (ordered ? 16384u : bp.budget)) {
+            bp.small_feature[bp.n_small] = kAllFeatures;
             bp.small_level[bp.n_small++] = (uint8_t)l;
             if (bytes > lds_bytes) lds_bytes = (uint32_t)bytes;
+        } else if (worth_it && !ordered && fp32_table && F == 2 && feature_bytes <= bp.budget && bp.n_small + 2 <= TNN_GRID_MAX_LEVELS) {
+            for (uint32_t f = 0; f < F; ++f) {
+                bp.small_feature[bp.n_small] = (uint8_t)f;
+                bp.small_level[bp.n_small++] = (uint8_t)l;
+            }
+            if (feature_bytes > lds_bytes) lds_bytes = (uint32_t)feature_bytes;
         } else {
             bp.big_level[n_big++] = (uint8_t)l;
         }
@@ -617,9 +619,7 @@ static int launch_grid_backward_g(const GridLevels &lv, const GridParams &gp, co
     // (grid_order.hip) walks a lattice of 64^2 (16^3) coarse cells row by row, x fastest: with the points spread evenly a
     // row holds M / 64 (M / 256) of them, and a stretch of C of these spans that share of the level's width plus a coarse
     // cell, and one coarse cell in the other dimensions. A stretch that breaks the estimate is caught in the kernel.
-    const uint32_t *bin_start = nullptr;
-    if (order && gp.n_levels > 0 && gp.interpolation != TNN_INTERP_NEAREST) {
-        bin_start = reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(order) + order_record_bytes(M));
+    if (ordered && gp.n_levels > 0 && gp.interpolation != TNN_INTERP_NEAREST) {
         bp.bins_per_row = (D == 2) ? 64 : 16;
         bp.n_rows = 4096 / bp.bins_per_row;
         const double per_row = (double)M / bp.n_rows, coarse = (double)bp.bins_per_row;
@@ -634,7 +634,7 @@ static int launch_grid_backward_g(const GridLevels &lv, const GridParams &gp, co
                 const double share = std::min(1.0, (double)(1u << c) / std::max(per_row, 1.0));
                 double cells = (share * R + R / coarse + 2.0) * (R / coarse + 2.0);
                 if (D == 3) cells *= R / coarse + 2.0;
-                if (cells * F * sizeof(float) <= 0.9 * (double)bp.budget) chunk_log2 = c;
+                if (cells * F * sizeof(double) <= 0.9 * (double)bp.budget) chunk_log2 = c;
             }
             if (chunk_log2 >= 0) {
                 const uint32_t pieces = (uint32_t)std::min(64.0, std::ceil(per_row / (double)(1u << chunk_log2)) + 1.0);
@@ -650,8 +650,31 @@ static int launch_grid_backward_g(const GridLevels &lv, const GridParams &gp, co
         }
         n_big = kept;
     }
+    // (few workgroups of the LDS route leave most of the chip idle: shorter ones then)
+    while (bp.chunk > 1024 && (M / bp.chunk) * bp.n_small < 256) bp.chunk /= 2;
+    bp.small_blocks = (uint32_t)((M + bp.chunk - 1) / bp.chunk);
+    if (bins) {
+        *bins = BinPlan{};
+        uint32_t kept = 0;
+        for (uint32_t i = 0; i < n_big; ++i)
+            if (!bin_plan_add(bins, bp.big_level[i], lv, gp, n_dims, F, M)) bp.big_level[kept++] = bp.big_level[i];
+        n_big = kept;
+    }
+    *n_big_levels = n_big;
+    *lds = lds_bytes;
+    return bp;
+}
+
+template <int D, int F, typename TAB>
+static int launch_grid_backward_g(const GridLevels &lv, const GridParams &gp, BackwardPlan bp, const GradLayout &dl, uint32_t n_big, uint32_t lds_bytes, const float *x,
+                                  const float4 *order, const void *dLdy, int dy_dtype, TAB *grad, size_t M, hipStream_t s) {
+    constexpr int per_block = kDirectPasses * kBwdThreads / (2 * BackwardLanes<F, TAB>::FL); // (point, level) pairs per workgroup on the direct route
+    bp.big_blocks = (uint32_t)((M + per_block - 1) / per_block);
+    const uint32_t *bin_start =
+        order ? reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(order) + order_record_bytes(M)) : nullptr;
     const unsigned long long blocks = (unsigned long long)bp.n_small * bp.small_blocks + bp.tiled_start[bp.n_tiled] + (unsigned long long)n_big * bp.big_blocks;
     if (blocks > 0x7fffffffull) return fail(TNN_ERR_UNSUPPORTED, "grid backward: batch too large for one launch");
+    if (blocks == 0) return TNN_OK;
     const dim3 grid((unsigned)blocks);
 #define TNN_BWD(GT)                                                                                                    \
     do {                                                                                                               \
@@ -659,7 +682,7 @@ static int launch_grid_backward_g(const GridLevels &lv, const GridParams &gp, co
         if (lds_bytes > 48 * 1024 &&                                                                                   \
             hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess) \
             return fail(TNN_ERR_HIP, "cannot reserve %u bytes of LDS", lds_bytes);                                     \
-        TNN_LAUNCH(k, grid, dim3(kBwdThreads), lds_bytes, s, lv, gp, bp, x, order, bin_start, (const GT *)dLdy, grad, (long long)M);    \
+        TNN_LAUNCH(k, grid, dim3(kBwdThreads), lds_bytes, s, lv, gp, bp, dl, x, order, bin_start, (const GT *)dLdy, grad, (long long)M);    \
     } while (0)
     switch (dy_dtype) {
     case TNN_FP32: TNN_BWD(float); break;
@@ -795,8 +818,12 @@ TNN_API int tnn_grid_forward_ordered(const tnn_grid_desc *desc, const void *d_or
     return rc;
 }
 
-static int grid_backward_any(const tnn_grid_desc *desc, const float *d_x, const float4 *d_order, const void *d_dLdy, int dy_dtype,
-                             uint32_t padded_width, void *d_grad_table, int grad_dtype, int overwrite, size_t M, tnn_stream_t stream) {
+namespace tnn {
+// by_position: dL/dy as the training kernel leaves it (GradLayout); d_x may be given beside d_order, for the routes that read
+// the rows of a row-major dL/dy better in the caller's order.
+int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4 *d_order, const void *d_dLdy, int dy_dtype, uint32_t padded_width,
+                       bool by_position, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
+                       hipStream_t s) {
     GridLevels lv;
     GridParams gp;
     int rc = grid_common(desc, padded_width, M, &lv, &gp);
@@ -806,25 +833,39 @@ static int grid_backward_any(const tnn_grid_desc *desc, const float *d_x, const 
     if (grad_dtype != TNN_FP32 && grad_dtype != TNN_FP16) return fail(TNN_ERR_UNSUPPORTED, "gradient table dtype %d", grad_dtype);
     if (grad_dtype == TNN_FP16 && desc->n_features_per_level % 2 != 0)
         return fail(TNN_ERR_UNSUPPORTED, "fp16 gradient tables need an even number of features per level (features are added in pairs)");
-    hipStream_t s = as_stream(stream);
-    if (overwrite) {
+    const uint32_t n_features = desc->n_features_per_level;
+    // With scratch memory the levels of the direct route are binned instead; without, and in fp16 tables, they are not.
+    BinPlan bins{};
+    uint32_t n_big = 0, lds_bytes = 0;
+    uintptr_t scratch = (reinterpret_cast<uintptr_t>(d_workspace) + 255) & ~(uintptr_t)255;
+    const bool binned = d_workspace && grad_dtype == TNN_FP32;
+    BackwardPlan bp = plan_backward(lv, gp, desc->n_dims, n_features, d_order != nullptr, grad_dtype == TNN_FP32, M, binned ? &bins : nullptr, &n_big, &lds_bytes);
+    if (bins.n_levels && workspace_bytes < bin_scratch_bytes(bins, n_features) + (scratch - reinterpret_cast<uintptr_t>(d_workspace)))
+        return fail(TNN_ERR_WORKSPACE, "grid backward: workspace of %zu bytes given, %zu needed", workspace_bytes, bin_scratch_bytes(bins, n_features) + 256);
+    if (overwrite || bins.n_levels) {
         // a fill kernel rather than a memset node, so the call can be captured into a HIP graph
-        const size_t bytes = tnn_grid_n_params(desc) * (grad_dtype == TNN_FP32 ? sizeof(float) : sizeof(fp16_t));
-        if (reinterpret_cast<uintptr_t>(d_grad_table) & 15) return fail(TNN_ERR_INVALID_ARGUMENT, "d_grad_table must be 16-byte aligned");
+        const size_t bytes = overwrite ? tnn_grid_n_params(desc) * (grad_dtype == TNN_FP32 ? sizeof(float) : sizeof(fp16_t)) : 0;
+        if (overwrite && (reinterpret_cast<uintptr_t>(d_grad_table) & 15)) return fail(TNN_ERR_INVALID_ARGUMENT, "d_grad_table must be 16-byte aligned");
         const size_t n4 = bytes / 16;
         const size_t n_tail = (bytes - n4 * 16) / sizeof(float); // level sizes are multiples of 8 entries: fp16 tables leave no tail
-        size_t blocks = (n4 + 255) / 256;
+        size_t blocks = (std::max<size_t>(n4, bins.n_bins) + 255) / 256;
         if (blocks > 4096) blocks = 4096;
         if (blocks < 4) blocks = 4;
         TNN_LAUNCH(fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (float4 *)d_grad_table, n4,
-                   reinterpret_cast<float *>(static_cast<char *>(d_grad_table) + n4 * 16), n_tail);
+                   reinterpret_cast<float *>(static_cast<char *>(d_grad_table) + n4 * 16), n_tail, reinterpret_cast<uint32_t *>(scratch), bins.n_bins);
         if ((rc = check_launch("fill_zero_kernel"))) return rc;
     }
+    const GradLayout dl{padded_width, n_features, by_position ? 1 : 0};
     if (grad_dtype == TNN_FP32) {
-        TNN_DISPATCH_DF(desc, rc = (launch_grid_backward_g<D_, F_, float>(lv, gp, d_x, d_order, d_dLdy, dy_dtype, (float *)d_grad_table, M, s)));
+        TNN_DISPATCH_DF(desc, rc = (launch_grid_backward_g<D_, F_, float>(lv, gp, bp, dl, n_big, lds_bytes, d_x, d_order, d_dLdy, dy_dtype,
+                                                                          (float *)d_grad_table, M, s)));
+        if (rc == TNN_OK && bins.n_levels)
+            rc = launch_grid_binned(bins, lv, gp, dl, desc->n_dims, n_features, d_x, d_x && !by_position ? nullptr : d_order, d_dLdy, dy_dtype, (float *)d_grad_table, overwrite != 0, M,
+                                    reinterpret_cast<void *>(scratch), s);
     } else {
         const uint32_t F = desc->n_features_per_level;
-#define TNN_PACKED(D_, F_) rc = launch_grid_backward_g<D_, F_, fp16_t>(lv, gp, d_x, d_order, d_dLdy, dy_dtype, (fp16_t *)d_grad_table, M, s)
+#define TNN_PACKED(D_, F_) \
+    rc = launch_grid_backward_g<D_, F_, fp16_t>(lv, gp, bp, dl, n_big, lds_bytes, d_x, d_order, d_dLdy, dy_dtype, (fp16_t *)d_grad_table, M, s)
         if (desc->n_dims == 2) {
             if (F == 2) TNN_PACKED(2, 2); else if (F == 4) TNN_PACKED(2, 4); else TNN_PACKED(2, 8);
         } else {
@@ -834,22 +875,45 @@ static int grid_backward_any(const tnn_grid_desc *desc, const float *d_x, const 
     }
     return rc;
 }
+} // namespace tnn
 
 TNN_API int tnn_grid_backward(const tnn_grid_desc *desc, const float *d_x, const void *d_dLdy, int dy_dtype,
                               uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, tnn_stream_t stream) {
-    return grid_backward_any(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, d_grad_table, TNN_FP32, overwrite, M, stream);
+    return grid_backward_impl(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, false, d_grad_table, TNN_FP32, overwrite, M, nullptr, 0, as_stream(stream));
 }
 
 TNN_API int tnn_grid_backward_ordered(const tnn_grid_desc *desc, const void *d_order, const void *d_dLdy, int dy_dtype,
                                       uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, tnn_stream_t stream) {
     if (!d_order) return tnn::fail(TNN_ERR_INVALID_ARGUMENT, "d_order is NULL");
-    return grid_backward_any(desc, nullptr, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, d_grad_table, TNN_FP32, overwrite,
-                             M, stream);
+    return grid_backward_impl(desc, nullptr, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, false, d_grad_table, TNN_FP32,
+                              overwrite, M, nullptr, 0, as_stream(stream));
+}
+
+TNN_API size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size_t M) {
+    GridLevels lv;
+    GridParams gp;
+    if (check_grid_desc(desc) || grid_common(desc, desc->n_levels * desc->n_features_per_level, M, &lv, &gp)) return 0;
+    size_t most = 0;
+    for (const bool ordered : {false, true}) {
+        BinPlan bins{};
+        uint32_t n_big, lds;
+        (void)plan_backward(lv, gp, desc->n_dims, desc->n_features_per_level, ordered, true, M, &bins, &n_big, &lds);
+        most = std::max(most, bin_scratch_bytes(bins, desc->n_features_per_level));
+    }
+    return most + 256;
+}
+
+TNN_API int tnn_grid_backward_binned(const tnn_grid_desc *desc, const float *d_x, const void *d_order, const void *d_dLdy, int dy_dtype,
+                                     uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
+                                     tnn_stream_t stream) {
+    if (!d_workspace) return tnn::fail(TNN_ERR_WORKSPACE, "grid backward: no workspace");
+    return grid_backward_impl(desc, d_x, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, false, d_grad_table, TNN_FP32, overwrite,
+                              M, d_workspace, workspace_bytes, as_stream(stream));
 }
 
 TNN_API int tnn_grid_backward_packed(const tnn_grid_desc *desc, const float *d_x, const void *d_dLdy, int dy_dtype,
                                      uint32_t padded_width, void *d_grad_table_f16, int overwrite, size_t M, tnn_stream_t stream) {
-    return grid_backward_any(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, d_grad_table_f16, TNN_FP16, overwrite, M, stream);
+    return grid_backward_impl(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, false, d_grad_table_f16, TNN_FP16, overwrite, M, nullptr, 0, as_stream(stream));
 }
 
 TNN_API int tnn_grid_indices(const tnn_grid_desc *desc, const float *d_x, uint32_t *d_indices, size_t M, tnn_stream_t stream) {

@@ -1,0 +1,32 @@
+// The binned route of the grid's backward pass (grid_binned.hip): which levels take it and where its scratch lies.
+#pragma once
+
+#include "grid_device.h"
+
+namespace tnn {
+
+constexpr uint32_t kMaxBinned = 32;         // levels one launch bins
+constexpr uint32_t kBinMaxBins = 1024;      // bins of a level
+constexpr uint32_t kBinSliceBytes = 128 * 1024; // most of a bin's slice of the table (LDS of a workgroup)
+
+struct BinPlan {
+    uint32_t n_levels;
+    uint32_t n_bins;                   // of all levels
+    uint8_t level[kMaxBinned];
+    uint8_t slice_log2[kMaxBinned];    // a bin holds 2^n consecutive entries of the level
+    uint32_t first_bin[kMaxBinned + 1]; // bins of the levels in front of this one
+    uint32_t capacity[kMaxBinned];     // records a bin has room for
+    uint32_t first_record[kMaxBinned]; // of the level's first bin
+    uint32_t n_records;                // room for all bins
+    uint32_t slice_lds;                // LDS bytes of the largest slice
+    uint32_t batch;                    // points binned at a time
+};
+
+// Adds level l to the plan if it can take the route.
+bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams &gp, uint32_t n_dims, uint32_t n_features, size_t M);
+size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_features);
+// d_cursors: the first p.n_bins words of the scratch, all zero.
+int launch_grid_binned(const BinPlan &p, const GridLevels &lv, const GridParams &gp, const GradLayout &dl, uint32_t n_dims, uint32_t n_features, const float *x,
+                       const float4 *order, const void *dLdy, int dy_dtype, float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s);
+
+} // namespace tnn

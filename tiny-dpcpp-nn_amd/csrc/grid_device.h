@@ -27,13 +27,39 @@ struct GridParams {
     uint32_t padded_width;
 };
 
+// Where dL/dy of a point and level lies: element (row, level, feature) at row * row_stride + level * level_stride + feature. A
+// caller's matrix is row-major in the caller's order; the training kernel writes its rows in the order it visits the points, so
+// that the scatter finds those of neighbouring points in the same lines (`by_position`: the row is the point's place).
+struct GradLayout {
+    uint32_t row_stride, level_stride;
+    int by_position;
+};
+
 // The buffer of tnn_grid_order_points (grid_order.hip): M records of 16 bytes, padded to 256 bytes, then the first position
 // of each of the 4096 coarse cells of the order (uint32, key order), which the scatter over ordered points reads.
 inline size_t order_record_bytes(size_t M) { return (M * 16 + 255) & ~(size_t)255; }
 
+// Pitch of the rows the training kernel writes for a grid of two features per level: whole 16-byte pieces.
+__host__ __device__ inline uint32_t gradient_pitch(uint32_t n_levels) { return (n_levels * 2 + 7) & ~7u; }
+
+// Leading `bits` bits of a coordinate taken as a number in [0, 1); anything else (outside, NaN) goes to an end bin.
+__device__ __forceinline__ uint32_t quantise(float v, int bits) {
+    const float s = v * (float)(1 << bits);
+    if (!(s > 0.0f)) return 0;
+    const uint32_t q = (uint32_t)s;
+    return q < (1u << bits) ? q : (1u << bits) - 1;
+}
+// Bits of every coordinate in the key of the order's coarse cells (first dimension fastest), and in the finer one inside a cell.
+template <int D> struct OrderBits;
+template <> struct OrderBits<2> { static constexpr int coarse = 6, fine = 3; };
+template <> struct OrderBits<3> { static constexpr int coarse = 4, fine = 2; };
+
 // Host side (grid.hip): validation of a descriptor, and of a call (include/encodings/grid.h:665-677) together with
 // the per-level constants the kernels take.
 int check_grid_desc(const tnn_grid_desc *d);
+int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4 *d_order, const void *d_dLdy, int dy_dtype, uint32_t padded_width,
+                       bool by_position, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
+                       hipStream_t s);
 int grid_common(const tnn_grid_desc *desc, uint32_t padded_width, size_t M, GridLevels *lv, GridParams *gp);
 
 template <int D> __device__ __forceinline__ uint32_t hash_pos(const uint32_t (&p)[D], uint32_t hash_type) {
@@ -102,6 +128,10 @@ template <typename P, int F> __device__ __forceinline__ void load_entry(const P 
         for (int f = 0; f < F; ++f) v[f] = (float)t[f];
     }
 }
+
+// Adds to a private sum in LDS. The sums are double on purpose: ds_add_f64 takes 20 cycles of a CU per wave instruction,
+// ds_add_f32 185 (any addresses; ds_add_u32 5), and the sums are rounded once, when they leave.
+__device__ __forceinline__ void lds_add(double *sum, float v) { unsafeAtomicAdd(sum, (double)v); }
 
 template <typename O> __device__ __forceinline__ O to_out(float v) { return (O)v; }
 

@@ -50,8 +50,8 @@ TNN_API size_t tnn_grid_mlp_train_step_workspace_bytes(const tnn_grid_desc *grid
     GridParams gp;
     FusedPlan plan;
     if (train_shape_check(grid, mlp, M ? M : 8, &lv, &gp, &plan)) return 0;
-    // dL/d(encoding) for the scatter, then the partial weight gradients and losses of the workgroups
-    return align256(M * 64 * 2) + align256(plan.loss_bytes) + align256(plan.partial_bytes) + 512;
+    // dL/d(encoding) for the scatter, then the partial weight gradients and losses of the workgroups, and what the scatter sorts the contributions into
+    return align256(M * gradient_pitch(grid->n_levels) * 2) + align256(plan.loss_bytes) + align256(plan.partial_bytes) + 512 + tnn_grid_backward_workspace_bytes(grid, M ? M : 8);
 }
 
 TNN_API int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order,
@@ -75,7 +75,7 @@ TNN_API int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn
     hipStream_t s = as_stream(stream);
     uintptr_t base = align256(reinterpret_cast<uintptr_t>(d_workspace));
     void *d_enc_grad = reinterpret_cast<void *>(base);
-    base += align256(M * 64 * 2);
+    base += align256(M * gradient_pitch(grid->n_levels) * 2);
     float *loss_partials = reinterpret_cast<float *>(base);
     base += align256(plan.loss_bytes);
     float *partials = reinterpret_cast<float *>(base);
@@ -92,9 +92,10 @@ TNN_API int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn
         rc = grid_mlp_train_launch_fp16(grid, mlp, plan, lv, gp, d_x, order, d_table, d_prepared_fwd, d_prepared_bwd, d_targets, loss_scale, d_y,
                                         d_loss_sum, d_enc_grad, M, partials, loss_partials, tail, s);
     if (rc) return rc;
-    // dL/d(encoding), in the network's type and at its padded width, into the table's gradient
-    if (d_order) return tnn_grid_backward_ordered(grid, d_order, d_enc_grad, mlp->dtype, 64, d_grad_table, overwrite, M, stream);
-    return tnn_grid_backward(grid, d_x, d_enc_grad, mlp->dtype, 64, d_grad_table, overwrite, M, stream);
+    // dL/d(encoding), in the network's type and in the order the kernel took the points, into the table's gradient
+    base += align256(plan.partial_bytes);
+    return grid_backward_impl(grid, d_order ? nullptr : d_x, order, d_enc_grad, mlp->dtype, gradient_pitch(grid->n_levels), true, d_grad_table, TNN_FP32, overwrite, M,
+                              reinterpret_cast<void *>(base), workspace_bytes - (base - reinterpret_cast<uintptr_t>(d_workspace)), s);
 }
 
 TNN_API int tnn_grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,
@@ -114,7 +115,7 @@ TNN_API int tnn_grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc 
     hipStream_t s = as_stream(stream);
     uintptr_t base = align256(reinterpret_cast<uintptr_t>(d_workspace));
     void *d_enc_grad = reinterpret_cast<void *>(base);
-    base += align256(M * 64 * 2);
+    base += align256(M * gradient_pitch(grid->n_levels) * 2);
     float *loss_partials = reinterpret_cast<float *>(base);
     base += align256(plan.loss_bytes);
     float *partials = reinterpret_cast<float *>(base);
@@ -128,6 +129,7 @@ TNN_API int tnn_grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc 
         rc = grid_mlp_given_launch_fp16(grid, mlp, plan, lv, gp, d_x, order, d_table, d_prepared_fwd, d_prepared_bwd, d_dLdy, d_dW, dW_is_fp32, enc_out,
                                         M, partials, loss_partials, s);
     if (rc || !d_grad_table) return rc;
-    if (d_order) return tnn_grid_backward_ordered(grid, d_order, d_enc_grad, mlp->dtype, 64, d_grad_table, overwrite, M, stream);
-    return tnn_grid_backward(grid, d_x, d_enc_grad, mlp->dtype, 64, d_grad_table, overwrite, M, stream);
+    base += align256(plan.partial_bytes);
+    return grid_backward_impl(grid, d_order ? nullptr : d_x, order, d_enc_grad, mlp->dtype, gradient_pitch(grid->n_levels), true, d_grad_table, TNN_FP32, overwrite, M,
+                              reinterpret_cast<void *>(base), workspace_bytes - (base - reinterpret_cast<uintptr_t>(d_workspace)), s);
 }

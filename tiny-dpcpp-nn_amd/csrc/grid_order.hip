@@ -44,18 +44,6 @@ static OrderPlan order_plan(size_t M) {
     return p;
 }
 
-// Leading `bits` bits of a coordinate taken as a number in [0, 1); anything else (outside, NaN) goes to an end bin.
-__device__ __forceinline__ uint32_t quantise(float v, int bits) {
-    const float s = v * (float)(1 << bits);
-    if (!(s > 0.0f)) return 0;
-    const uint32_t q = (uint32_t)s;
-    return q < (1u << bits) ? q : (1u << bits) - 1;
-}
-
-template <int D> struct OrderBits;
-template <> struct OrderBits<2> { static constexpr int coarse = 6, fine = 3; };
-template <> struct OrderBits<3> { static constexpr int coarse = 4, fine = 2; };
-
 template <int D> __device__ __forceinline__ uint32_t coarse_key(const float (&x)[D]) {
     constexpr int b = OrderBits<D>::coarse;
     uint32_t k = 0;

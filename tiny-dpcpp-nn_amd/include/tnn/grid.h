@@ -111,22 +111,13 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
         if (input.n() != this->get_input_width() || dL_doutput.n() != this->get_padded_output_width() || dL_doutput.m() != batch_size)
             throw std::invalid_argument("Dimension mismatch grid encoding backward_impl");
         check_max_level();
-        if (batch_size >= kCellOrderMinBackwardBatch) {
-            // large batches: the scatter over points in cell order sums neighbouring points on chip before it touches the table.
-            // The points are ordered here again (a tenth of the scatter's time): nothing says they are the forward pass's.
-            const size_t bytes = tnn_grid_order_bytes(&m_desc, batch_size);
-            if (!m_order || m_order->size() * sizeof(float) < bytes)
-                m_order = std::make_unique<DeviceMatrix<float>>((bytes + sizeof(float) - 1) / sizeof(float), 1, this->get_queue());
-            tnn::abi_check(tnn_grid_order_points(&m_desc, input.GetPointer(), batch_size, m_order->data(), m_order->size() * sizeof(float),
-                                                 this->get_queue().abi()));
-            tnn::abi_check(tnn_grid_backward_ordered(&m_desc, m_order->data(), dL_doutput.GetPointer(), TNN_FP32, this->get_padded_output_width(),
-                                                     gradients->GetPointer(), param_gradients_mode == GradientMode::Overwrite ? 1 : 0,
-                                                     batch_size, this->get_queue().abi()));
-            return;
-        }
-        tnn::abi_check(tnn_grid_backward(&m_desc, input.GetPointer(), dL_doutput.GetPointer(), TNN_FP32, this->get_padded_output_width(),
-                                         gradients->GetPointer(), param_gradients_mode == GradientMode::Overwrite ? 1 : 0, batch_size,
-                                         this->get_queue().abi()));
+        const size_t scratch = tnn_grid_backward_workspace_bytes(&m_desc, batch_size);
+        if (!m_scratch || m_scratch->size() * sizeof(float) < scratch)
+            m_scratch = std::make_unique<DeviceMatrix<float>>((scratch + sizeof(float) - 1) / sizeof(float), 1, this->get_queue());
+        tnn::abi_check(tnn_grid_backward_binned(&m_desc, input.GetPointer(), nullptr, dL_doutput.GetPointer(), TNN_FP32,
+                                                this->get_padded_output_width(), gradients->GetPointer(),
+                                                param_gradients_mode == GradientMode::Overwrite ? 1 : 0, batch_size, m_scratch->data(),
+                                                m_scratch->size() * sizeof(float), this->get_queue().abi()));
     }
 
     uint32_t n_pos_dims() const override { return m_desc.n_dims; }
@@ -152,10 +143,10 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
     // below this the ordering costs what it saves (2^18 points: 25 us + 42 us against 76 us in 2-D, 25 + 174 against 224 in 3-D
     // with a table of 2^22 entries per level; 2^17: 22 + 28 against 40 and 22 + 97 against 115)
     static constexpr size_t kCellOrderMinBatch = size_t(1) << 18;
-    static constexpr size_t kCellOrderMinBackwardBatch = size_t(1) << 17;
 
     tnn_grid_desc m_desc;
     std::unique_ptr<DeviceMatrix<float>> m_order; // records of the last large batch in cell order
+    std::unique_ptr<DeviceMatrix<float>> m_scratch; // what the backward pass sorts its contributions into; only grows
     uint32_t m_n_features;
     uint32_t m_n_features_per_level;
     GridOffsetTable m_offset_table;
