@@ -239,6 +239,38 @@ int tnn_mlp_backward_recompute(const tnn_mlp_desc *desc, const void *d_prepared_
                                const void *d_dLdy, void *d_dW, int dW_is_fp32, void *d_dLdx, size_t M, void *d_workspace,
                                size_t workspace_bytes, tnn_stream_t stream);
 
+/* ------------------------------------------------------------------------------------------
+ * The same passes on a caller's own rows, for callers whose matrices are not padded to the network's width and to 8 rows and
+ * whose gradients are loss-scaled. They stand in for what the reference's Python modules do around its kernels in separate
+ * operations: padding of rows and columns, the conversion of the input, the loss scale on the way in and out, and the packing
+ * of the weight gradients (dpcpp_bindings/tiny_dpcpp_nn/modules.py:84-136,206-262, include/tnn_api.h:541-603). Any M >= 1.
+ * ------------------------------------------------------------------------------------------ */
+
+/* dst (dst_rows x dst_cols, dense) := src (src_rows x src_cols, strides in elements) * scale, rounded to dst_dtype; columns
+ * beyond src's are `fill`, rows beyond src's are zero in src's columns. dtypes: bf16, fp16, fp32. */
+int tnn_resize_rows(int dst_dtype, void *d_dst, int dst_cols, size_t dst_rows, int src_dtype, const void *d_src, int src_cols,
+                    long long row_stride, long long col_stride, size_t src_rows, float fill, float scale, tnn_stream_t stream);
+/* tnn_mlp_inference on x (M x x_cols of T or fp32, rounded to T; the network's other input columns are `fill`), with the first
+ * y_cols columns of the output in y (M x y_cols). TNN_ERR_UNSUPPORTED for x other than M x width of T where the kernel takes
+ * whole rows only (width 128 with many matrices or a large batch): tnn_resize_rows first. */
+int tnn_mlp_inference_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_x, int x_dtype, int x_cols, float fill,
+                           void *d_y, int y_cols, size_t M, tnn_stream_t stream);
+/* tnn_mlp_backward_recompute with dL/dy of dy_cols columns (at most 16, or the width; the others are zero) multiplied by
+ * dy_scale as it is read, and results multiplied by result_scale: weight gradients in the packed parameter layout, rounded
+ * to T and stored as dW_dtype (T or fp32), and dL/dx (M x width of T, or NULL). */
+int tnn_mlp_backward_recompute_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_x,
+                                    const void *d_dLdy, int dy_cols, float dy_scale, float result_scale, void *d_dW_packed, int dW_dtype,
+                                    void *d_dLdx, size_t M, void *d_workspace, size_t workspace_bytes, tnn_stream_t stream);
+/* tnn_mlp_forward / tnn_mlp_backward at width 128 (TNN_ERR_UNSUPPORTED otherwise) without copies of what the caller holds anyway:
+ * d_hidden receives the n_hidden_layers hidden activations only (M x 128 each), the output goes to d_y (M x y_cols), and the
+ * backward pass reads x where it is. d_y of the backward pass: M x 128, or NULL for a network without an output activation.
+ * Scales and weight gradients as above. Workspace: tnn_mlp_backward_workspace_bytes. */
+int tnn_mlp_forward_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_x, void *d_hidden, void *d_y, int y_cols, size_t M,
+                         tnn_stream_t stream);
+int tnn_mlp_backward_rows(const tnn_mlp_desc *desc, const void *d_prepared_bwd, const void *d_x, const void *d_hidden, const void *d_y,
+                          const void *d_dLdy, float dy_scale, float result_scale, void *d_dW_packed, int dW_dtype, void *d_dLdx, size_t M,
+                          void *d_workspace, size_t workspace_bytes, tnn_stream_t stream);
+
 /* Testing aid, no counterpart in the reference. In the width-64 training and backward kernels the four waves that share
  * staged tiles meet at a counter in LDS; a wave waits there for at most `iterations` polls (default 2^22, far beyond any
  * real wait) so that a kernel always ends. A wave whose wait runs out marks its workgroup, and the call then delivers NaN
@@ -418,6 +450,15 @@ int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn_mlp_des
 int tnn_grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,
                           const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_dLdy, void *d_dW, int dW_is_fp32,
                           float *d_grad_table, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes, tnn_stream_t stream);
+/* tnn_grid_mlp_inference / _ordered (d_order given) with the first y_cols columns of the output in y (M x y_cols). */
+int tnn_grid_mlp_inference_rows(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,
+                                const void *d_prepared_fwd, void *d_y, int y_cols, size_t M, tnn_stream_t stream);
+/* tnn_grid_mlp_backward with dL/dy, scales and weight gradients as in tnn_mlp_backward_recompute_rows; the table's gradient is
+ * multiplied by result_scale too. */
+int tnn_grid_mlp_backward_rows(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,
+                               const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_dLdy, int dy_cols, float dy_scale,
+                               float result_scale, void *d_dW_packed, int dW_dtype, float *d_grad_table, int overwrite, size_t M,
+                               void *d_workspace, size_t workspace_bytes, tnn_stream_t stream);
 /* TNN_OK when tnn_grid_mlp_inference runs this pair of shapes, otherwise the status (and tnn_last_error the reason) it
  * would return: lets a caller choose between the fused call and the two calls once, when the modules are built. */
 int tnn_grid_mlp_supported(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp);

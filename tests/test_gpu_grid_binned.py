@@ -44,7 +44,7 @@ def test_binned_scatter_matches_the_oracle(tnn, oracle, cfg, M, ordered, kind):
     d = tnn.grid_desc(cfg)
     g = torch.from_numpy(rng.standard_normal((M, pw)).astype(np.float32)).to(tnn.dev)
     xt = torch.from_numpy(x).to(tnn.dev)
-    for dtype in (FP32, BF16, FP16) if M == 513 else (FP32,):
+    for dtype in (FP32, BF16, FP16) if M == 40007 else (FP32,):
         gt = g.to(DT[dtype]).contiguous()
         grad = binned(tnn, d, xt, gt, dtype, ordered)
         ref = oracle.grid_backward(cfg, x, gt.float().cpu().numpy(), tnn.grid_n_params(d))
@@ -57,7 +57,7 @@ def test_binned_scatter_matches_the_oracle(tnn, oracle, cfg, M, ordered, kind):
 def test_binned_workspace_is_checked(tnn):
     from tiny_dpcpp_nn import _lib
     d = tnn.grid_desc(CFG3)
-    x = torch.rand((4096, 3), device=tnn.dev)
+    x = torch.rand((40960, 3), device=tnn.dev)
     with pytest.raises(_lib.TnnError):
-        binned(tnn, d, x, torch.rand((4096, 32), device=tnn.dev), FP32, short=4096)
+        binned(tnn, d, x, torch.rand((40960, 32), device=tnn.dev), FP32, short=4096)
     assert tnn.lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), 0) == 0

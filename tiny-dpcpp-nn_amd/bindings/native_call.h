@@ -1,0 +1,123 @@
+// The autograd functions of the Python modules: one call into a native module, forward and backward, as nodes of PyTorch's
+// graph. They stand in for the reference's autograd function (dpcpp_bindings/tiny_dpcpp_nn/modules.py:65-136), which pads, scales,
+// converts and slices with PyTorch operations around the native calls; a training step on a small batch then spends
+// its time in Python and in a dozen launches. Here the step is one entry into C++ each way, and what surrounds the passes is
+// part of them (tnn::Module::forward_rows / backward_rows).
+#pragma once
+
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/torch.h>
+
+#include "tnn/tnn_api.h"
+
+namespace tnn_binding {
+
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+/// A network or an encoding: gradients of its input (a network's) and of its parameters.
+struct ModuleBackward : public torch::autograd::Node {
+    std::shared_ptr<tnn::Module> module;
+    tnn::Module::RowsPass pass; // its input tensor is in `input`
+    SavedVariable input, params;
+    double loss_scale = 1.0;
+    bool released = false;
+
+    variable_list apply(variable_list &&grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        TORCH_CHECK(!released, torch::autograd::ERR_BACKWARD_TWICE);
+        const torch::Tensor x = input.unpack(), p = params.unpack();
+        if (!grads[0].defined()) return {torch::Tensor(), torch::Tensor()};
+        const torch::AutoGradMode no_grad(false);
+        tnn::Module::RowsPass kept = pass;
+        kept.input = x;
+        auto [dx, dparams] = module->backward_rows(grads[0], kept, loss_scale, task_should_compute_output(0), p);
+        return {dx, dparams};
+    }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        input.reset_data();
+        params.reset_data();
+        pass.hidden.reset();
+        pass.output.reset();
+        released = true;
+    }
+    std::string name() const override { return "TnnModuleBackward"; }
+};
+
+/// A grid encoding and its network as one call: gradients of the network's parameters and of the table.
+struct EncodedNetworkBackward : public torch::autograd::Node {
+    std::shared_ptr<tnn::Module> network, encoding;
+    SavedVariable positions, params, table;
+    double loss_scale = 1.0;
+
+    variable_list apply(variable_list &&grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        const torch::Tensor x = positions.unpack(), p = params.unpack(), t = table.unpack();
+        if (!grads[0].defined()) return {torch::Tensor(), torch::Tensor()};
+        const torch::AutoGradMode no_grad(false);
+        auto [dparams, dtable] = network->backward_rows_with_encoding(*encoding, x, grads[0], loss_scale, p, t);
+        return {dparams, dtable};
+    }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        positions.reset_data();
+        params.reset_data();
+        table.reset_data();
+    }
+    std::string name() const override { return "TnnEncodedNetworkBackward"; }
+};
+
+/// y = module(x), recorded for autograd when that is on and anything asks for gradients.
+inline torch::Tensor call(const std::shared_ptr<tnn::Module> &module, const torch::Tensor &x, const torch::Tensor &params, bool push, bool training,
+                          double loss_scale) {
+    if (push && module->n_params()) module->push_params(params);
+    const torch::Tensor in = module->input_rows(x); // (PyTorch operations where any are needed: autograd sees them)
+    const bool record = torch::autograd::compute_requires_grad(in, params);
+    tnn::Module::RowsPass pass;
+    torch::Tensor y;
+    {
+        const torch::AutoGradMode no_grad(false);
+        y = module->forward_rows(in, record, training, pass);
+    }
+    if (!record) return y;
+    auto node = std::shared_ptr<ModuleBackward>(new ModuleBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(in, params));
+    node->module = module;
+    node->input = SavedVariable(pass.input, false);
+    pass.input.reset();
+    node->pass = std::move(pass);
+    node->params = SavedVariable(params, false);
+    node->loss_scale = loss_scale;
+    torch::autograd::set_history(y, node);
+    return y;
+}
+
+/// y = network(encoding(positions)) for a pair that can_train_with_encoding (or, without autograd, can_fuse_encoding) accepts.
+inline torch::Tensor call_with_encoding(const std::shared_ptr<tnn::Module> &network, const std::shared_ptr<tnn::Module> &encoding, const torch::Tensor &x,
+                                        const torch::Tensor &params, const torch::Tensor &table, bool push_network, bool push_table, double loss_scale) {
+    if (push_table) encoding->push_params(table);
+    if (push_network) network->push_params(params);
+    const torch::Tensor positions = x.detach().to(torch::kFloat32).contiguous();
+    const bool record = torch::autograd::compute_requires_grad(params, table);
+    torch::Tensor y;
+    {
+        const torch::AutoGradMode no_grad(false);
+        y = network->forward_rows_with_encoding(*encoding, positions, record);
+    }
+    if (!record) return y;
+    auto node = std::shared_ptr<EncodedNetworkBackward>(new EncodedNetworkBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(params, table));
+    node->network = network;
+    node->encoding = encoding;
+    node->positions = SavedVariable(positions, false);
+    node->params = SavedVariable(params, false);
+    node->table = SavedVariable(table, false);
+    node->loss_scale = loss_scale;
+    torch::autograd::set_history(y, node);
+    return y;
+}
+
+} // namespace tnn_binding

@@ -6,6 +6,7 @@
 #include <pybind11/stl.h>
 #include <torch/extension.h>
 
+#include "native_call.h"
 #include "tnn/tnn_api.h"
 
 namespace py = pybind11;
@@ -34,7 +35,7 @@ json to_json(const py::handle &h) {
 
 class PybindingModule {
   public:
-    PybindingModule(tnn::Module *module) : m_module{std::unique_ptr<tnn::Module>(module)} {}
+    PybindingModule(tnn::Module *module) : m_module{module} {}
 
     torch::Tensor fwd(torch::Tensor input) {
         CHECK_INPUT(input);
@@ -73,6 +74,14 @@ class PybindingModule {
         CHECK_INPUT(grad_output);
         return m_module->backward_with_encoding(*encoding.m_module, positions, grad_output, pack_gradient, positions_unchanged_since_forward);
     }
+    /// The module as an operator: parameters pushed (on request), forward pass, and a node of the autograd graph.
+    torch::Tensor call(const torch::Tensor &x, const torch::Tensor &params, bool push, bool training, double loss_scale) const {
+        return tnn_binding::call(m_module, x, params, push, training, loss_scale);
+    }
+    torch::Tensor call_with_encoding(const PybindingModule &encoding, const torch::Tensor &x, const torch::Tensor &params, const torch::Tensor &table,
+                                     bool push_network, bool push_table, double loss_scale) const {
+        return tnn_binding::call_with_encoding(m_module, encoding.m_module, x, params, table, push_network, push_table, loss_scale);
+    }
     torch::Tensor initial_params() { return m_module->initialize_params(); }
     torch::Tensor initial_params(torch::Tensor &tensor) { return m_module->initialize_params(tensor); }
     /// weights_are_packed: the tensor already is in the packed parameter layout, no packing is done
@@ -82,7 +91,7 @@ class PybindingModule {
     uint32_t n_output_dims() const { return (uint32_t)m_module->n_output_dims(); }
 
   private:
-    std::unique_ptr<tnn::Module> m_module;
+    std::shared_ptr<tnn::Module> m_module; // shared with the autograd nodes of its calls
 };
 
 template <typename T>
@@ -136,6 +145,10 @@ PYBIND11_MODULE(tiny_dpcpp_nn_pybind_module, m) {
         .def("can_train_with_encoding", &PybindingModule::can_train_with_encoding)
         .def("bwd_with_encoding", &PybindingModule::bwd_with_encoding, py::arg("encoding"), py::arg("positions"), py::arg("grad_output"),
              py::arg("pack_gradient"), py::arg("positions_unchanged_since_forward") = false)
+        .def("call", &PybindingModule::call, py::call_guard<py::gil_scoped_release>(), py::arg("x"), py::arg("params"), py::arg("push"), py::arg("training"),
+             py::arg("loss_scale"))
+        .def("call_with_encoding", &PybindingModule::call_with_encoding, py::call_guard<py::gil_scoped_release>(), py::arg("encoding"), py::arg("x"),
+             py::arg("params"), py::arg("table"), py::arg("push_network"), py::arg("push_table"), py::arg("loss_scale"))
         .def("bwd_no_encoding_grad", &PybindingModule::bwd_no_encoding_grad)
         .def("bwd_with_encoding_grad", &PybindingModule::bwd_with_encoding_grad)
         .def("initial_params", py::overload_cast<>(&PybindingModule::initial_params))

@@ -80,6 +80,23 @@ template <typename T> __device__ __forceinline__ void adam_update_element(const 
     adam_apply_element<T>(a, idx, adam_fetch_element(a, idx), g_raw);
 }
 
+// Weight gradients as the parameters are laid out (packed), rounded to the network's type first, as the raw gradients are.
+struct PackedGradient {
+    void *p = nullptr;
+    int dtype = TNN_FP32; // or the network's type
+    int W = 0;
+    float scale = 1.0f;
+};
+template <typename T> __device__ __forceinline__ void store_packed_gradient(const PackedGradient &g, int idx, float grad) {
+    const int per = g.W * g.W, l = idx / per, n = idx % per / g.W, k = idx % g.W;
+    const float v = (float)(T)grad * g.scale;
+    const int to = l * per + packed_coord(k, n, g.W);
+    if (g.dtype == TNN_FP32)
+        static_cast<float *>(g.p)[to] = v;
+    else
+        static_cast<T *>(g.p)[to] = (T)v;
+}
+
 // What follows the main kernel of the fused training step.
 struct TrainTail {
     bool use_adam = false;       // apply Adam to the reduced gradients inside the reduction kernel
@@ -87,6 +104,11 @@ struct TrainTail {
     hipEvent_t main_done = nullptr; // recorded between the main kernel and the reduction when not null
     void *dW = nullptr;             // launchers that have no dW argument of their own: where the reduced gradients go, if anywhere
     int dW_is_fp32 = 1;
+    // A caller's dL/dy (backward pass only): its columns where it has fewer than the network is wide (0: all), the factor it is
+    // multiplied by as it is read, and the one dL/dx and `packed` are multiplied by as they are written.
+    int dy_cols = 0;
+    float dy_scale = 1.0f, result_scale = 1.0f;
+    PackedGradient packed{};
 };
 
 } // namespace tnn

@@ -316,7 +316,7 @@ __global__ void __launch_bounds__(kBwdThreads)
             float gy[F];
 #pragma unroll
             for (int f = 0; f < F; ++f)
-                if (f < (int)n_f) gy[f] = (float)dy[f];
+                if (f < (int)n_f) gy[f] = (float)dy[f] * dl.scale;
             for_each_corner<D>(x, scale, size, res, flags, gp.hash_type, gp.interpolation, [&](uint32_t idx, float w) {
 #pragma unroll
                 for (int f = 0; f < F; ++f)
@@ -400,7 +400,7 @@ __global__ void __launch_bounds__(kBwdThreads)
                 const G *dy = dLdy + (dl.by_position ? first + pl : row) * dl.row_stride + l * dl.level_stride;
                 float gy[F];
 #pragma unroll
-                for (int f = 0; f < F; ++f) gy[f] = (float)dy[f];
+                for (int f = 0; f < F; ++f) gy[f] = (float)dy[f] * dl.scale;
                 uint32_t cell[D];
                 float frac[D];
                 cell_of<D>(x, scale, gp.interpolation, cell, frac);
@@ -480,7 +480,7 @@ __global__ void __launch_bounds__(kBwdThreads)
     const G *dy = dLdy + (dl.by_position ? i : row) * dl.row_stride + l * dl.level_stride + fl * FV;
     float gy[FV];
 #pragma unroll
-    for (int f = 0; f < FV; ++f) gy[f] = live ? (float)dy[f] : 0.0f;
+    for (int f = 0; f < FV; ++f) gy[f] = live ? (float)dy[f] * dl.scale : 0.0f;
     uint32_t cell[D];
     float frac[D];
     cell_of<D>(x, lv.scale[l], gp.interpolation, cell, frac);
@@ -653,8 +653,10 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
     // (few workgroups of the LDS route leave most of the chip idle: shorter ones then)
     while (bp.chunk > 1024 && (M / bp.chunk) * bp.n_small < 256) bp.chunk /= 2;
     bp.small_blocks = (uint32_t)((M + bp.chunk - 1) / bp.chunk);
-    if (bins) {
-        *bins = BinPlan{};
+    // Binned from where the atomics it saves (one request per pair of corners, 20e9 a second) take longer than its two launches:
+    // 2^18 requests. (2-D, 11 such levels, 12 000 points: 20 us either way; 2^16 points: 42 against 95.)
+    if (bins) *bins = BinPlan{};
+    if (bins && ((unsigned long long)M * n_big << (D - 1)) >= (1ull << 18)) {
         uint32_t kept = 0;
         for (uint32_t i = 0; i < n_big; ++i)
             if (!bin_plan_add(bins, bp.big_level[i], lv, gp, n_dims, F, M)) bp.big_level[kept++] = bp.big_level[i];
@@ -680,7 +682,7 @@ static int launch_grid_backward_g(const GridLevels &lv, const GridParams &gp, Ba
     do {                                                                                                               \
         auto k = grid_backward_kernel<D, F, GT, TAB>;                                                                  \
         if (lds_bytes > 48 * 1024 &&                                                                                   \
-            hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess) \
+            !reserve_lds(reinterpret_cast<const void *>(k), lds_bytes)) \
             return fail(TNN_ERR_HIP, "cannot reserve %u bytes of LDS", lds_bytes);                                     \
         TNN_LAUNCH(k, grid, dim3(kBwdThreads), lds_bytes, s, lv, gp, bp, dl, x, order, bin_start, (const GT *)dLdy, grad, (long long)M);    \
     } while (0)
@@ -822,7 +824,7 @@ namespace tnn {
 // by_position: dL/dy as the training kernel leaves it (GradLayout); d_x may be given beside d_order, for the routes that read
 // the rows of a row-major dL/dy better in the caller's order.
 int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4 *d_order, const void *d_dLdy, int dy_dtype, uint32_t padded_width,
-                       bool by_position, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
+                       bool by_position, float scale, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
                        hipStream_t s) {
     GridLevels lv;
     GridParams gp;
@@ -842,20 +844,24 @@ int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4
     BackwardPlan bp = plan_backward(lv, gp, desc->n_dims, n_features, d_order != nullptr, grad_dtype == TNN_FP32, M, binned ? &bins : nullptr, &n_big, &lds_bytes);
     if (bins.n_levels && workspace_bytes < bin_scratch_bytes(bins, n_features) + (scratch - reinterpret_cast<uintptr_t>(d_workspace)))
         return fail(TNN_ERR_WORKSPACE, "grid backward: workspace of %zu bytes given, %zu needed", workspace_bytes, bin_scratch_bytes(bins, n_features) + 256);
-    if (overwrite || bins.n_levels) {
+    if (overwrite && (reinterpret_cast<uintptr_t>(d_grad_table) & 15)) return fail(TNN_ERR_INVALID_ARGUMENT, "d_grad_table must be 16-byte aligned");
+    // The binned levels are written whole: where they are the last ones, as the finest are, only what lies in front of them is cleared.
+    size_t entries = overwrite ? desc->offsets[desc->n_levels] : 0;
+    if (bins.n_levels && bins.level[0] + bins.n_levels == desc->n_levels) entries = std::min<size_t>(entries, desc->offsets[bins.level[0]]);
+    if (entries || bins.n_levels) {
         // a fill kernel rather than a memset node, so the call can be captured into a HIP graph
-        const size_t bytes = overwrite ? tnn_grid_n_params(desc) * (grad_dtype == TNN_FP32 ? sizeof(float) : sizeof(fp16_t)) : 0;
-        if (overwrite && (reinterpret_cast<uintptr_t>(d_grad_table) & 15)) return fail(TNN_ERR_INVALID_ARGUMENT, "d_grad_table must be 16-byte aligned");
+        const size_t bytes = entries * n_features * (grad_dtype == TNN_FP32 ? sizeof(float) : sizeof(fp16_t));
         const size_t n4 = bytes / 16;
         const size_t n_tail = (bytes - n4 * 16) / sizeof(float); // level sizes are multiples of 8 entries: fp16 tables leave no tail
-        size_t blocks = (std::max<size_t>(n4, bins.n_bins) + 255) / 256;
+        const uint32_t n_words = bins.n_bins;
+        size_t blocks = (std::max<size_t>(n4, n_words) + 255) / 256;
         if (blocks > 4096) blocks = 4096;
         if (blocks < 4) blocks = 4;
         TNN_LAUNCH(fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (float4 *)d_grad_table, n4,
-                   reinterpret_cast<float *>(static_cast<char *>(d_grad_table) + n4 * 16), n_tail, reinterpret_cast<uint32_t *>(scratch), bins.n_bins);
+                   reinterpret_cast<float *>(static_cast<char *>(d_grad_table) + n4 * 16), n_tail, reinterpret_cast<uint32_t *>(scratch), n_words);
         if ((rc = check_launch("fill_zero_kernel"))) return rc;
     }
-    const GradLayout dl{padded_width, n_features, by_position ? 1 : 0};
+    const GradLayout dl{padded_width, n_features, by_position ? 1 : 0, scale};
     if (grad_dtype == TNN_FP32) {
         TNN_DISPATCH_DF(desc, rc = (launch_grid_backward_g<D_, F_, float>(lv, gp, bp, dl, n_big, lds_bytes, d_x, d_order, d_dLdy, dy_dtype,
                                                                           (float *)d_grad_table, M, s)));
@@ -879,13 +885,13 @@ int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4
 
 TNN_API int tnn_grid_backward(const tnn_grid_desc *desc, const float *d_x, const void *d_dLdy, int dy_dtype,
                               uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, tnn_stream_t stream) {
-    return grid_backward_impl(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, false, d_grad_table, TNN_FP32, overwrite, M, nullptr, 0, as_stream(stream));
+    return grid_backward_impl(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, false, 1.0f, d_grad_table, TNN_FP32, overwrite, M, nullptr, 0, as_stream(stream));
 }
 
 TNN_API int tnn_grid_backward_ordered(const tnn_grid_desc *desc, const void *d_order, const void *d_dLdy, int dy_dtype,
                                       uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, tnn_stream_t stream) {
     if (!d_order) return tnn::fail(TNN_ERR_INVALID_ARGUMENT, "d_order is NULL");
-    return grid_backward_impl(desc, nullptr, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, false, d_grad_table, TNN_FP32,
+    return grid_backward_impl(desc, nullptr, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, false, 1.0f, d_grad_table, TNN_FP32,
                               overwrite, M, nullptr, 0, as_stream(stream));
 }
 
@@ -907,13 +913,13 @@ TNN_API int tnn_grid_backward_binned(const tnn_grid_desc *desc, const float *d_x
                                      uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
                                      tnn_stream_t stream) {
     if (!d_workspace) return tnn::fail(TNN_ERR_WORKSPACE, "grid backward: no workspace");
-    return grid_backward_impl(desc, d_x, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, false, d_grad_table, TNN_FP32, overwrite,
+    return grid_backward_impl(desc, d_x, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, false, 1.0f, d_grad_table, TNN_FP32, overwrite,
                               M, d_workspace, workspace_bytes, as_stream(stream));
 }
 
 TNN_API int tnn_grid_backward_packed(const tnn_grid_desc *desc, const float *d_x, const void *d_dLdy, int dy_dtype,
                                      uint32_t padded_width, void *d_grad_table_f16, int overwrite, size_t M, tnn_stream_t stream) {
-    return grid_backward_impl(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, false, d_grad_table_f16, TNN_FP16, overwrite, M, nullptr, 0, as_stream(stream));
+    return grid_backward_impl(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, false, 1.0f, d_grad_table_f16, TNN_FP16, overwrite, M, nullptr, 0, as_stream(stream));
 }
 
 TNN_API int tnn_grid_indices(const tnn_grid_desc *desc, const float *d_x, uint32_t *d_indices, size_t M, tnn_stream_t stream) {

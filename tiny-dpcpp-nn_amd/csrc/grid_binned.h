@@ -13,7 +13,9 @@ struct BinPlan {
     uint32_t n_levels;
     uint32_t n_bins;                   // of all levels
     uint8_t level[kMaxBinned];
-    uint8_t slice_log2[kMaxBinned];    // a bin holds 2^n consecutive entries of the level
+    uint8_t bins_log2[kMaxBinned];     // the level's runs of 2^run_log2 entries go to its 2^bins_log2 bins in turn
+    uint8_t run_log2[kMaxBinned];
+    uint16_t places[kMaxBinned];       // entries a bin has room for
     uint32_t first_bin[kMaxBinned + 1]; // bins of the levels in front of this one
     uint32_t capacity[kMaxBinned];     // records a bin has room for
     uint32_t first_record[kMaxBinned]; // of the level's first bin
@@ -25,7 +27,8 @@ struct BinPlan {
 // Adds level l to the plan if it can take the route.
 bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams &gp, uint32_t n_dims, uint32_t n_features, size_t M);
 size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_features);
-// d_cursors: the first p.n_bins words of the scratch, all zero.
+// The first p.n_bins words of the scratch have to be zero when the kernels start. With `overwrite` every entry of the plan's levels
+// is written, whatever it held.
 int launch_grid_binned(const BinPlan &p, const GridLevels &lv, const GridParams &gp, const GradLayout &dl, uint32_t n_dims, uint32_t n_features, const float *x,
                        const float4 *order, const void *dLdy, int dy_dtype, float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s);
 

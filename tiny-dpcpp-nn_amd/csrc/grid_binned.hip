@@ -4,13 +4,17 @@
 // The memory side retires an atomic request per 32-byte sector, about 20 * 10^9 a second, and a point of a hashed level
 // needs 2^(D-1) or more of them: 2.1 ms for 2^20 points of a 3-D grid of 16 levels (2^19 entries). Here the contributions
 // are sorted by destination first:
-//   1. grid_bin_kernel cuts a level into bins of consecutive entries and writes every contribution as a record into its
+//   1. grid_bin_kernel deals runs of a level's entries out to bins and writes every contribution as a record into its
 //      bin. The two corners along the first dimension are neighbouring entries in a dense level and differ in the low bits
-//      of the index in a coherently hashed one, so they share a bin and travel as one record of two entries.
+//      of the index in a coherently hashed one, so nearly always they share a bin and travel as one record of two entries.
+//      (Long runs make long stores; but a hashed level's runs longer than its x range are dealt out by the other
+//      dimensions alone, and in 2-D the few hundred values of y fill the bins very unevenly: bin_plan_add.)
 //   2. grid_bin_sum_kernel takes a bin at a time, sums its records into a copy of the bin's entries in LDS and writes the
 //      entries to the table as whole lines.
 // A record of two features is 16 bytes written once and read once, where the two atomic requests it replaces occupy the
 // memory side for 64.
+// Measured, 2^20 points, 3-D, 2^19 entries, 15 levels this way: 2 x (165 + 177) us, 3 TB/s of records both ways; before, the
+// atomics of the ten finest of these levels alone took 1.5 ms.
 #include "grid_binned.h"
 
 #include <algorithm>
@@ -20,7 +24,17 @@ namespace tnn {
 
 constexpr int kBinThreads = 512;
 constexpr int kBinPoints = 2; // points of a thread
-constexpr int kBinSumThreads = 512;
+constexpr int kBinSumThreads = 1024; // at most
+
+// Entry e of a level: its bin and its place there.
+struct Bins {
+    uint32_t n_log2, run_log2;
+    __device__ __forceinline__ uint32_t bin(uint32_t e) const { return (e >> run_log2) & ((1u << n_log2) - 1); }
+    __device__ __forceinline__ uint32_t place(uint32_t e) const { return ((e >> (run_log2 + n_log2)) << run_log2) | (e & ((1u << run_log2) - 1)); }
+    __device__ __forceinline__ uint32_t entry(uint32_t bin, uint32_t place) const {
+        return ((((place >> run_log2) << n_log2) | bin) << run_log2) | (place & ((1u << run_log2) - 1));
+    }
+};
 
 // Two neighbouring entries of a bin, the position between them, and the gradient times the weights of the other dimensions.
 template <int F> struct alignas(F == 1 ? 4 : F == 2 ? 16 : 8) BinRecord {
@@ -79,12 +93,12 @@ __device__ __forceinline__ void pair_entries(const uint32_t (&cell)[D], uint32_t
 // gives every record its place among them, reserves that much of every bin with one atomic, and writes the records there, so
 // that a bin receives them in runs. The levels of the same points are consecutive workgroups of one XCD, which shares the
 // rows of dL/dy between them in its L2.
-// A record beyond a bin's capacity (points that cluster on few cells) goes to the table as atomics.
+// Records beyond a bin's capacity are counted and dropped.
 template <int D, int F, typename G>
 __global__ void __launch_bounds__(kBinThreads)
     grid_bin_kernel(const GridLevels lv, const GridParams gp, const BinPlan bp, const GradLayout dl, const float *__restrict__ xin,
                     const float4 *__restrict__ order, const G *__restrict__ dLdy, uint32_t *__restrict__ cursors, BinRecord<F> *__restrict__ records,
-                    float *__restrict__ grad, long long first, long long last, uint32_t per_wg) {
+                    long long first, long long last, uint32_t per_wg) {
     constexpr int NP = 1 << (D - 1); // pairs of a point
     static_assert(kBinThreads * kBinPoints * NP <= 4096 && kBinMaxBins <= 1024, "a record's place is packed into 12 + 10 + 10 bits");
     __shared__ uint32_t base[kBinMaxBins];  // records per bin, then the first place of them
@@ -93,7 +107,8 @@ __global__ void __launch_bounds__(kBinThreads)
     const long long begin = first + (long long)((turn / bp.n_levels) * 8 + blockIdx.x % 8) * per_wg;
     if (begin >= last) return;
     const long long end = begin + per_wg < last ? begin + per_wg : last;
-    const uint32_t l = bp.level[k], slice = bp.slice_log2[k], n_bins = bp.first_bin[k + 1] - bp.first_bin[k];
+    const Bins dealt{bp.bins_log2[k], bp.run_log2[k]};
+    const uint32_t l = bp.level[k], n_bins = 1u << dealt.n_log2;
     const uint32_t size = lv.size[l], res = lv.resolution[l], flags = lv.flags[l], capacity = bp.capacity[k];
     const float scale = lv.scale[l];
     uint32_t *const cursor = cursors + bp.first_bin[k];
@@ -101,7 +116,6 @@ __global__ void __launch_bounds__(kBinThreads)
 
     for (uint32_t b = threadIdx.x; b < n_bins; b += kBinThreads) base[b] = split[b] = 0;
     __syncthreads();
-    const uint32_t mask = (1u << slice) - 1;
     float frac[kBinPoints][D], gy[kBinPoints][F];
     uint32_t where[kBinPoints][NP], place[kBinPoints][NP]; // place: rank in the bin (12 bits), bin, bin of the far side
 #pragma unroll
@@ -112,15 +126,15 @@ __global__ void __launch_bounds__(kBinThreads)
         const long long row = bin_point<D>(xin, order, i, x);
         const G *dy = dLdy + (dl.by_position ? i : row) * dl.row_stride + l * dl.level_stride;
 #pragma unroll
-        for (int f = 0; f < F; ++f) gy[u][f] = (float)dy[f];
+        for (int f = 0; f < F; ++f) gy[u][f] = (float)dy[f] * dl.scale;
         uint32_t cell[D], near[NP], far[NP];
         cell_of<D>(x, scale, gp.interpolation, cell, frac[u]);
         pair_entries<D>(cell, size, res, flags, gp.hash_type, near, far);
 #pragma unroll
         for (int c = 0; c < NP; ++c) {
-            const uint32_t bin = near[c] >> slice, far_bin = far[c] >> slice;
+            const uint32_t bin = dealt.bin(near[c]), far_bin = dealt.bin(far[c]);
             place[u][c] = atomicAdd(&base[bin], 1u) | (bin << 12) | (far_bin << 22);
-            where[u][c] = (near[c] & mask) | ((far[c] & mask) << 15);
+            where[u][c] = dealt.place(near[c]) | (dealt.place(far[c]) << 15);
             if (far_bin != bin) atomicAdd(&split[far_bin], 1u);
         }
     }
@@ -147,16 +161,7 @@ __global__ void __launch_bounds__(kBinThreads)
             const uint32_t bin = (place[u][c] >> 12) & 1023u, far_bin = place[u][c] >> 22;
             const auto put = [&](uint32_t to, uint32_t at, uint32_t sides) {
                 r.where = where[u][c] | (sides << 30);
-                if (at < capacity) {
-                    bins[(size_t)to * capacity + at] = r;
-                    return;
-                }
-                float *const g = grad + ((size_t)lv.offset[l] + ((size_t)to << slice)) * F;
-#pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    if (sides & 1) unsafeAtomicAdd(g + (size_t)(r.where & 0x7fff) * F + f, (1 - r.frac) * r.g[f]);
-                    if (sides & 2) unsafeAtomicAdd(g + (size_t)((r.where >> 15) & 0x7fff) * F + f, r.frac * r.g[f]);
-                }
+                if (at < capacity) bins[(size_t)to * capacity + at] = r;
             };
             put(bin, base[bin] + (place[u][c] & 4095u), far_bin == bin ? 3u : 1u);
             if (far_bin != bin) put(far_bin, atomicAdd(&split[far_bin], 1u), 2u);
@@ -164,79 +169,126 @@ __global__ void __launch_bounds__(kBinThreads)
     }
 }
 
-// One workgroup sums one bin. Bound by the LDS atomics (two values of two features per record) and the records' bytes.
-template <int F>
+// One workgroup sums one bin and stores (or adds) its entries. Bound by the records' bytes and the LDS atomics (two values of two
+// features per record). A bin that more records were meant for than it has room for is summed from the points instead, all of them
+// passing its workgroup by. The bin's cursor is left at zero for the next part of the batch.
+template <int D, int F, typename G>
 __global__ void __launch_bounds__(kBinSumThreads)
-    grid_bin_sum_kernel(const GridLevels lv, const BinPlan bp, uint32_t *__restrict__ cursors, const BinRecord<F> *__restrict__ records,
-                        float *__restrict__ grad, int store) {
+    grid_bin_sum_kernel(const GridLevels lv, const GridParams gp, const BinPlan bp, const GradLayout dl, const float *__restrict__ xin,
+                        const float4 *__restrict__ order, const G *__restrict__ dLdy, uint32_t *__restrict__ cursors,
+                        const BinRecord<F> *__restrict__ records, float *__restrict__ grad, long long first, long long last, int store) {
     extern __shared__ double sums[];
     uint32_t k = 0;
     while (k + 1 < bp.n_levels && blockIdx.x >= bp.first_bin[k + 1]) ++k;
     const uint32_t l = bp.level[k], bin = blockIdx.x - bp.first_bin[k];
-    const uint32_t first = bin << bp.slice_log2[k], size = lv.size[l];
-    const uint32_t n = min(1u << bp.slice_log2[k], size - first);
-    for (uint32_t e = threadIdx.x; e < n * F; e += kBinSumThreads) sums[e] = 0.0;
+    const Bins dealt{bp.bins_log2[k], bp.run_log2[k]};
+    const uint32_t size = lv.size[l];
+    const uint32_t n = bp.places[k]; // the last ones may be beyond the level
+    for (uint32_t e = threadIdx.x; e < n * F; e += blockDim.x) sums[e] = 0.0;
     const uint32_t written = cursors[blockIdx.x];
-    const uint32_t n_records = min(written, bp.capacity[k]);
     const BinRecord<F> *const rec = records + bp.first_record[k] + (size_t)bin * bp.capacity[k];
     __syncthreads();
-    if (threadIdx.x == 0) cursors[blockIdx.x] = 0; // for the next part of the batch
-    constexpr int kAhead = 4; // records of a lane in flight
-    for (uint32_t i = threadIdx.x; i < n_records; i += kAhead * kBinSumThreads) {
-        BinRecord<F> r[kAhead];
+    if (threadIdx.x == 0) cursors[blockIdx.x] = 0;
+    if (written <= bp.capacity[k]) {
+        constexpr int kAhead = 4; // records of a lane in flight
+        for (uint32_t i = threadIdx.x; i < written; i += kAhead * blockDim.x) {
+            BinRecord<F> r[kAhead];
 #pragma unroll
-        for (int a = 0; a < kAhead; ++a) {
-            const uint32_t at = i + a * kBinSumThreads;
-            r[a] = rec[at < n_records ? at : i];
-            if (at >= n_records) r[a].where = 0;
-        }
-#pragma unroll
-        for (int a = 0; a < kAhead; ++a) {
-            const uint32_t near = r[a].where & 0x7fff, far = (r[a].where >> 15) & 0x7fff;
-            if (r[a].where & (1u << 30)) {
-#pragma unroll
-                for (int f = 0; f < F; ++f) lds_add(&sums[near * F + f], (1 - r[a].frac) * r[a].g[f]);
+            for (int a = 0; a < kAhead; ++a) {
+                const uint32_t at = i + a * blockDim.x;
+                r[a] = rec[at < written ? at : i];
+                if (at >= written) r[a].where = 0;
             }
-            if (r[a].where & (1u << 31)) {
 #pragma unroll
-                for (int f = 0; f < F; ++f) lds_add(&sums[far * F + f], r[a].frac * r[a].g[f]);
+            for (int a = 0; a < kAhead; ++a) {
+                const uint32_t near = r[a].where & 0x7fff, far = (r[a].where >> 15) & 0x7fff;
+                if (r[a].where & (1u << 30)) {
+#pragma unroll
+                    for (int f = 0; f < F; ++f) lds_add(&sums[near * F + f], (1 - r[a].frac) * r[a].g[f]);
+                }
+                if (r[a].where & (1u << 31)) {
+#pragma unroll
+                    for (int f = 0; f < F; ++f) lds_add(&sums[far * F + f], r[a].frac * r[a].g[f]);
+                }
+            }
+        }
+    } else {
+        for (long long i = first + threadIdx.x; i < last; i += blockDim.x) {
+            float x[D], frac[D];
+            const long long row = bin_point<D>(xin, order, i, x);
+            uint32_t cell[D], near[1 << (D - 1)], far[1 << (D - 1)];
+            cell_of<D>(x, lv.scale[l], gp.interpolation, cell, frac);
+            pair_entries<D>(cell, size, lv.resolution[l], lv.flags[l], gp.hash_type, near, far);
+            const G *dy = dLdy + (dl.by_position ? i : row) * dl.row_stride + l * dl.level_stride;
+#pragma unroll
+            for (int c = 0; c < (1 << (D - 1)); ++c) {
+                const bool near_mine = dealt.bin(near[c]) == bin, far_mine = dealt.bin(far[c]) == bin;
+                if (!near_mine && !far_mine) continue;
+                float weight = 1.0f;
+#pragma unroll
+                for (int d = 1; d < D; ++d) weight *= (c >> (d - 1)) & 1 ? frac[d] : 1 - frac[d];
+#pragma unroll
+                for (int f = 0; f < F; ++f) {
+                    const float v = weight * ((float)dy[f] * dl.scale);
+                    if (near_mine) lds_add(&sums[dealt.place(near[c]) * F + f], (1 - frac[0]) * v);
+                    if (far_mine) lds_add(&sums[dealt.place(far[c]) * F + f], frac[0] * v);
+                }
             }
         }
     }
     __syncthreads();
-    float *const g = grad + ((size_t)lv.offset[l] + first) * F;
-    if (store && written <= bp.capacity[k]) { // the bin's entries have no other contributions
-        for (uint32_t e = threadIdx.x; e < n * F; e += kBinSumThreads) g[e] = (float)sums[e];
-    } else {
-        for (uint32_t e = threadIdx.x; e < n * F; e += kBinSumThreads) g[e] += (float)sums[e];
+    float *const g = grad + (size_t)lv.offset[l] * F;
+    for (uint32_t v = threadIdx.x; v < n * F; v += blockDim.x) {
+        const uint32_t e = dealt.entry(bin, v / F);
+        if (e >= size) continue;
+        float *const to = g + (size_t)e * F + v % F;
+        *to = store ? (float)sums[v] : *to + (float)sums[v]; // (store: the bin's entries have no other contributions)
     }
 }
 
 bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams &gp, uint32_t n_dims, uint32_t n_features, size_t M) {
     if (p->n_levels >= kMaxBinned || gp.interpolation == TNN_INTERP_NEAREST) return false;
     const size_t size = lv.size[l], entry = n_features * sizeof(double);
-    // About 128 bins a level: a workgroup's share of a bin is then a run of several lines, and the bins of all levels are
-    // enough workgroups for the sums. Larger levels have bins as large as LDS allows.
-    uint32_t slice = 4;
-    while (slice < 15 && (size >> slice) > 128 && ((size_t)2 << slice) * entry <= kBinSliceBytes) ++slice;
-    const size_t bins = (size + ((size_t)1 << slice) - 1) >> slice;
+    // A bin stores all of its entries; atomics touch only those that have contributions, and cost as much when there is one for
+    // every 16 entries (3-D, 2^22 entries a level: 2^16 points).
+    if ((M << (n_dims - 1)) < size / 16) return false;
+    // 128 bins a level: a workgroup's share of a bin is then a run of several lines, and the bins of all levels are enough
+    // workgroups for the sums (64 or 256: the one pass gains what the other loses). Small levels have fewer, large ones as
+    // many as it takes for a bin to fit LDS.
+    uint32_t n_log2 = 7;
+    while (n_log2 > 0 && (size >> (n_log2 + 4)) == 0) --n_log2;
+    while (n_log2 < 31 && ((size >> n_log2) * entry > kBinSliceBytes || (size >> n_log2) > 0x7fff)) ++n_log2;
+    const size_t bins = (size_t)1 << n_log2;
     if (bins > kBinMaxBins) return false;
     p->batch = (uint32_t)std::min<size_t>(M, size_t(1) << 19);
-    // (other hashes than the coherent one send the two corners along the first dimension to different bins)
-    const bool apart = (lv.flags[l] & 16u) && gp.hash_type != TNN_HASH_COHERENT_PRIME;
-    const double mean = (double)p->batch * (double)(1u << (n_dims - 1)) * (apart ? 2.0 : 1.0) / ((double)size / (double)(1u << slice));
-    const double room = std::ceil((1.25 * mean + 8.0 * std::sqrt(mean) + 64.0) / 32.0) * 32.0;
+    // A hashed level deals out groups of cells that share a run of x and all of the other coordinates, at random: runs as long as
+    // leaves a bin 64 groups, down to 16 entries (a line of two features). Dense levels are dealt out in order: consecutive
+    // entries to a bin. (Other hashes than the coherent one send every corner by itself.)
+    const bool hashed = (lv.flags[l] & 16u) != 0, apart = hashed && gp.hash_type != TNN_HASH_COHERENT_PRIME;
+    const double R = (double)lv.resolution[l];
+    const auto groups = [&](uint32_t run) { return std::max(R / (double)((size_t)1 << run), 1.0) * std::pow(R, (double)n_dims - 1.0) / (double)bins; };
+    uint32_t run_log2 = 4;
+    while (((size_t)1 << (run_log2 + n_log2)) < size && (!hashed || apart || groups(run_log2 + 1) >= 64.0)) ++run_log2;
+    const size_t places = ((size + ((size_t)1 << (run_log2 + n_log2)) - 1) >> (run_log2 + n_log2)) << run_log2;
+    if (places > 0x7fff || places * entry > kBinSliceBytes) return false;
+    // What points spread evenly send a bin, and how far above it the fullest bin may be.
+    const double split = apart ? 2.0 : 1.0 + 1.0 / (double)((size_t)1 << run_log2);
+    const double mean = (double)p->batch * (double)(1u << (n_dims - 1)) * split * (double)places / (double)size;
+    const double uneven = hashed && !apart ? std::min(4.0 / std::sqrt(std::max(groups(run_log2), 1.0)), 3.0) : 0.0;
+    const double room = std::ceil(((1.2 + uneven) * mean + 8.0 * std::sqrt(mean) + 64.0) / 32.0) * 32.0;
     if (room * (double)bins + p->n_records > 4.0e9) return false;
     const uint32_t k = p->n_levels++;
     p->level[k] = (uint8_t)l;
-    p->slice_log2[k] = (uint8_t)slice;
+    p->bins_log2[k] = (uint8_t)n_log2;
+    p->run_log2[k] = (uint8_t)run_log2;
+    p->places[k] = (uint16_t)places;
     p->capacity[k] = (uint32_t)room;
     p->first_record[k] = p->n_records;
     p->n_records += (uint32_t)room * (uint32_t)bins;
     p->first_bin[k] = p->n_bins;
     p->n_bins += (uint32_t)bins;
     p->first_bin[k + 1] = p->n_bins;
-    p->slice_lds = std::max<uint32_t>(p->slice_lds, (uint32_t)(entry << slice));
+    p->slice_lds = std::max<uint32_t>(p->slice_lds, (uint32_t)(entry * places));
     return true;
 }
 
@@ -251,20 +303,21 @@ static int launch_binned(const BinPlan &p, const GridLevels &lv, const GridParam
                          float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s) {
     uint32_t *const cursors = static_cast<uint32_t *>(scratch);
     BinRecord<F> *const records = reinterpret_cast<BinRecord<F> *>(static_cast<char *>(scratch) + cursor_bytes(p));
-    const auto sum = grid_bin_sum_kernel<F>;
-    if (p.slice_lds > 48 * 1024 &&
-        hipFuncSetAttribute(reinterpret_cast<const void *>(sum), hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.slice_lds) != hipSuccess)
+    const auto sum = grid_bin_sum_kernel<D, F, G>;
+    if (!reserve_lds(reinterpret_cast<const void *>(sum), p.slice_lds))
         return fail(TNN_ERR_HIP, "cannot reserve %u bytes of LDS", p.slice_lds);
+    // (as many waves on a CU as it takes whatever LDS the bins need; small bins are over before 16 waves are under way)
+    const unsigned sum_threads = p.slice_lds > 32 * 1024 ? kBinSumThreads : kBinSumThreads / 2;
     for (size_t first = 0; first < M; first += p.batch) {
         const size_t last = std::min(M, first + p.batch), n = last - first;
         const uint32_t per_wg = n * p.n_levels < size_t(512) * kBinThreads * kBinPoints ? kBinThreads : kBinThreads * kBinPoints;
         const size_t stretches = (n + per_wg - 1) / per_wg;
         TNN_LAUNCH((grid_bin_kernel<D, F, G>), dim3((unsigned)((stretches + 7) / 8 * 8 * p.n_levels)), dim3(kBinThreads), 0, s, lv, gp, p, dl, x, order,
-                   (const G *)dLdy, cursors, records, grad, (long long)first, (long long)last, per_wg);
+                   (const G *)dLdy, cursors, records, (long long)first, (long long)last, per_wg);
         int rc = check_launch("grid_bin_kernel");
         if (rc) return rc;
-        TNN_LAUNCH(sum, dim3(p.n_bins), dim3(kBinSumThreads), p.slice_lds, s, lv, p, cursors, (const BinRecord<F> *)records, grad,
-                   (int)(overwrite && first == 0));
+        TNN_LAUNCH(sum, dim3(p.n_bins), dim3(sum_threads), p.slice_lds, s, lv, gp, p, dl, x, order, (const G *)dLdy, cursors,
+                   (const BinRecord<F> *)records, grad, (long long)first, (long long)last, (int)(overwrite && first == 0));
         if ((rc = check_launch("grid_bin_sum_kernel"))) return rc;
     }
     return TNN_OK;

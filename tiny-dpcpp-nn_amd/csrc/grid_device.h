@@ -33,6 +33,7 @@ struct GridParams {
 struct GradLayout {
     uint32_t row_stride, level_stride;
     int by_position;
+    float scale; // every value is multiplied by this as it is read
 };
 
 // The buffer of tnn_grid_order_points (grid_order.hip): M records of 16 bytes, padded to 256 bytes, then the first position
@@ -58,7 +59,7 @@ template <> struct OrderBits<3> { static constexpr int coarse = 4, fine = 2; };
 // the per-level constants the kernels take.
 int check_grid_desc(const tnn_grid_desc *d);
 int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4 *d_order, const void *d_dLdy, int dy_dtype, uint32_t padded_width,
-                       bool by_position, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
+                       bool by_position, float scale, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
                        hipStream_t s);
 int grid_common(const tnn_grid_desc *desc, uint32_t padded_width, size_t M, GridLevels *lv, GridParams *gp);
 

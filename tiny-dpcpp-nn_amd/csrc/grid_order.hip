@@ -248,8 +248,7 @@ TNN_API int tnn_grid_order_points(const tnn_grid_desc *desc, const float *d_x, s
     uint32_t *groups = reinterpret_cast<uint32_t *>(static_cast<char *>(d_order) + p.record_bytes + p.hist_bytes);
     hipStream_t s = as_stream(stream);
     const size_t scan_lds = ((size_t)p.n_wg * 64 + kScanParts * 64 + 64 + kScanParts) * sizeof(uint32_t);
-    if (scan_lds > 48 * 1024 &&
-        hipFuncSetAttribute(reinterpret_cast<const void *>(order_scan_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)scan_lds) != hipSuccess)
+    if (!reserve_lds(reinterpret_cast<const void *>(order_scan_kernel), scan_lds))
         return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", scan_lds);
 #define TNN_ORDER(D_)                                                                                                                  \
     do {                                                                                                                               \

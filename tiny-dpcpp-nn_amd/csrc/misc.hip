@@ -1,5 +1,7 @@
 // Error reporting, weight-layout permutations, L2 loss and the Adam step.
 #include "tnn_internal.h"
+
+#include <algorithm>
 #include "adam_update.h"
 
 #include <cstring>
@@ -25,6 +27,61 @@ int check_launch(const char *what) {
     return TNN_OK;
 }
 
+namespace {
+struct KernelFacts {
+    const void *kernel = nullptr;
+    int device = 0;
+    size_t reserved = 0;              // bytes of LDS the kernel may have
+    size_t lds = 0;                   // what `per_cu` was asked for
+    int threads = 0, per_cu = 0;
+};
+// Open addressing over kernel and device; a full table is started afresh (the library has some thousand kernels, a program
+// uses a few of them).
+KernelFacts &kernel_facts(const void *kernel) {
+    constexpr unsigned kSlots = 256;
+    static thread_local KernelFacts table[kSlots];
+    static thread_local unsigned used = 0;
+    int device = 0;
+    (void)hipGetDevice(&device);
+    if (used > kSlots / 2) {
+        for (KernelFacts &f : table) f = KernelFacts{};
+        used = 0;
+    }
+    unsigned i = (unsigned)((reinterpret_cast<uintptr_t>(kernel) >> 4) * 2654435761u + (unsigned)device) % kSlots;
+    while (table[i].kernel && (table[i].kernel != kernel || table[i].device != device)) i = (i + 1) % kSlots;
+    if (!table[i].kernel) {
+        table[i].kernel = kernel;
+        table[i].device = device;
+        ++used;
+    }
+    return table[i];
+}
+} // namespace
+
+bool reserve_lds(const void *kernel, size_t bytes) {
+    if (bytes <= 48 * 1024) return true;
+    KernelFacts &f = kernel_facts(kernel);
+    if (f.reserved >= bytes) return true;
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
+    f.reserved = bytes;
+    return true;
+}
+
+int resident_per_cu(const void *kernel, int threads, size_t lds_bytes) {
+    KernelFacts &f = kernel_facts(kernel);
+    if (f.per_cu == 0 || f.threads != threads || f.lds != lds_bytes) {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, lds_bytes) != hipSuccess || n < 1) {
+            (void)hipGetLastError();
+            n = 1;
+        }
+        f.per_cu = n;
+        f.threads = threads;
+        f.lds = lds_bytes;
+    }
+    return f.per_cu;
+}
+
 int check_mlp_desc(const tnn_mlp_desc *d) {
     if (!d) return fail(TNN_ERR_INVALID_ARGUMENT, "desc is NULL");
     if (d->dtype != TNN_BF16 && d->dtype != TNN_FP16)
@@ -40,6 +97,53 @@ int check_mlp_desc(const tnn_mlp_desc *d) {
         return fail(TNN_ERR_UNSUPPORTED, "activation %d / output activation %d: only None, ReLU and Sigmoid are supported",
                     d->activation, d->output_activation);
     return TNN_OK;
+}
+
+// dst[r][c] = src[r][c] * scale rounded to dst's type where src has that row and column; other columns of src's rows are `fill`,
+// other rows zero in the columns src has and `fill` in the others (rows are padded first, columns then). PER consecutive columns
+// of dst per thread.
+template <typename DST, typename SRC, int PER>
+__global__ void __launch_bounds__(256)
+    resize_rows_kernel(DST *__restrict__ dst, unsigned dst_cols, unsigned long long n_pieces, const SRC *__restrict__ src, unsigned src_cols,
+                       long long row_stride, long long col_stride, unsigned long long src_rows, float fill, float scale) {
+    const unsigned per_row = dst_cols / PER;
+    for (unsigned long long p = (unsigned long long)blockIdx.x * 256 + threadIdx.x; p < n_pieces; p += (unsigned long long)gridDim.x * 256) {
+        unsigned long long r;
+        unsigned c0;
+        if (n_pieces <= 0xffffffffull) {
+            r = (unsigned)p / per_row;
+            c0 = ((unsigned)p - (unsigned)r * per_row) * PER;
+        } else {
+            r = p / per_row;
+            c0 = (unsigned)(p - r * per_row) * PER;
+        }
+        const SRC *s = src + (long long)r * row_stride;
+        typedef DST dvec __attribute__((ext_vector_type(PER)));
+        dvec out;
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+            const unsigned c = c0 + e;
+            float v = c < src_cols ? 0.0f : fill;
+            if (c < src_cols && r < src_rows) v = as_fp32((float)s[c * col_stride] * scale);
+            out[e] = (DST)v;
+        }
+        *reinterpret_cast<dvec *>(dst + r * dst_cols + c0) = out;
+    }
+}
+
+template <typename DST, typename SRC>
+static int launch_resize_rows(void *dst, int dst_cols, size_t dst_rows, const void *src, int src_cols, long long row_stride, long long col_stride,
+                              size_t src_rows, float fill, float scale, hipStream_t s) {
+    const bool whole = dst_cols % 8 == 0 && (reinterpret_cast<uintptr_t>(dst) & 31) == 0;
+    const unsigned long long pieces = (unsigned long long)dst_rows * dst_cols / (whole ? 8 : 1);
+    const unsigned blocks = (unsigned)std::min<unsigned long long>((pieces + 255) / 256, 8192);
+    if (whole)
+        TNN_LAUNCH((resize_rows_kernel<DST, SRC, 8>), dim3(blocks), dim3(256), 0, s, (DST *)dst, (unsigned)dst_cols, pieces, (const SRC *)src, (unsigned)src_cols,
+                   row_stride, col_stride, (unsigned long long)src_rows, fill, scale);
+    else
+        TNN_LAUNCH((resize_rows_kernel<DST, SRC, 1>), dim3(blocks), dim3(256), 0, s, (DST *)dst, (unsigned)dst_cols, pieces, (const SRC *)src, (unsigned)src_cols,
+                   row_stride, col_stride, (unsigned long long)src_rows, fill, scale);
+    return check_launch("resize_rows_kernel");
 }
 
 enum PermuteOp { OP_PACK, OP_UNPACK, OP_PACKED_TRANSPOSE, OP_PACK_AND_TRANSPOSE };
@@ -144,6 +248,30 @@ __global__ void __launch_bounds__(256) mlp_adam_update_kernel(const AdamArgs a, 
 } // namespace tnn
 
 using namespace tnn;
+
+TNN_API int tnn_resize_rows(int dst_dtype, void *d_dst, int dst_cols, size_t dst_rows, int src_dtype, const void *d_src, int src_cols, long long row_stride,
+                            long long col_stride, size_t src_rows, float fill, float scale, tnn_stream_t stream) {
+    if (!d_dst || (!d_src && src_rows)) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    if (dst_cols < 1 || src_cols < 1) return fail(TNN_ERR_INVALID_ARGUMENT, "%d and %d columns", dst_cols, src_cols);
+    if (dst_rows == 0) return TNN_OK;
+#define TNN_RESIZE(D_, S_) return launch_resize_rows<D_, S_>(d_dst, dst_cols, dst_rows, d_src, src_cols, row_stride, col_stride, src_rows, fill, scale, as_stream(stream))
+#define TNN_RESIZE_FROM(D_)                                                                \
+    switch (src_dtype) {                                                                   \
+    case TNN_BF16: TNN_RESIZE(D_, bf16_t);                                                 \
+    case TNN_FP16: TNN_RESIZE(D_, fp16_t);                                                 \
+    case TNN_FP32: TNN_RESIZE(D_, float);                                                  \
+    default: return fail(TNN_ERR_UNSUPPORTED, "src_dtype %d", src_dtype);                  \
+    }
+    switch (dst_dtype) {
+    case TNN_BF16: TNN_RESIZE_FROM(bf16_t)
+    case TNN_FP16: TNN_RESIZE_FROM(fp16_t)
+    case TNN_FP32: TNN_RESIZE_FROM(float)
+    default: return fail(TNN_ERR_UNSUPPORTED, "dst_dtype %d", dst_dtype);
+    }
+#undef TNN_RESIZE_FROM
+#undef TNN_RESIZE
+}
+
 
 TNN_API const char *tnn_last_error(void) { return error_buffer(); }
 TNN_API int tnn_abi_version(void) { return TNN_HIP_ABI_VERSION; }

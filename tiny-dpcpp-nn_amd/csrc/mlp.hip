@@ -64,10 +64,12 @@ __global__ void prepare_weights_kernel(const SRC *__restrict__ packed, T *__rest
 // converted, and arrive while the conversion runs.
 // STAGED: every wave has a tile of LDS behind the weights and writes its rows through it (Tile::store_staged);
 // 2 = with the streaming hint.
-template <typename T, int W, int ACT, bool STORE_INTERM, bool W_IN_LDS, int THREADS, int STAGED = 0>
+// y: where the network's output goes (y_cols columns of it); for STORE_INTERM null means behind the activations. store_input = 0
+// leaves matrix 0 of the activations unwritten. NARROW: x has x_cols columns of T or (x_fp32) fp32, the others are `fill`.
+template <typename T, int W, int ACT, bool STORE_INTERM, bool W_IN_LDS, int THREADS, int STAGED = 0, bool NARROW = false>
 __global__ void __launch_bounds__(THREADS, (THREADS >= 512 && W <= 64) ? 4 : 1)
     mlp_forward_kernel(const typename Storage<T>::vec8 *__restrict__ wprep, const T *__restrict__ x, T *__restrict__ out,
-                       int n_mats, int out_act, long long M) {
+                       int n_mats, int out_act, long long M, T *__restrict__ y, int y_cols, int store_input, int x_cols, int x_fp32, float fill) {
     typedef Tile<T, W> TL;
     typedef typename Storage<T>::vec8 vec8;
     constexpr int NK = TL::NK, NI = TL::NI;
@@ -90,6 +92,12 @@ __global__ void __launch_bounds__(THREADS, (THREADS >= 512 && W <= 64) ? 4 : 1)
         }
     };
 
+    auto load_tile = [&](vec8(&r)[NK], long long row) __attribute__((always_inline)) {
+        if constexpr (NARROW)
+            TL::load_columns(r, x, x_fp32 != 0, x_cols, (T)fill, row, h, row < M);
+        else
+            TL::load(r, x, row, h, row < M);
+    };
     vec8 cur[NK];
     if constexpr (W_IN_LDS) {
         // The weights are requested first and the first tile behind them: the wait for the weights then leaves the tile's
@@ -108,7 +116,7 @@ __global__ void __launch_bounds__(THREADS, (THREADS >= 512 && W <= 64) ? 4 : 1)
         }
         asm volatile("" ::: "memory");
         const bool early = (wave & 1) == 0;
-        if (early && tile < n_tiles) TL::load(cur, x, tile * 32 + j, h, tile * 32 + j < M);
+        if (early && tile < n_tiles) load_tile(cur, tile * 32 + j);
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int i = 0; i < HELD; ++i) {
@@ -117,9 +125,9 @@ __global__ void __launch_bounds__(THREADS, (THREADS >= 512 && W <= 64) ? 4 : 1)
         }
         for (int f = threadIdx.x + HELD * THREADS; f < n; f += THREADS) lds_w[f] = wprep[f];
         __syncthreads();
-        if (!early && tile < n_tiles) TL::load(cur, x, tile * 32 + j, h, tile * 32 + j < M);
+        if (!early && tile < n_tiles) load_tile(cur, tile * 32 + j);
     } else {
-        if (tile < n_tiles) TL::load(cur, x, tile * 32 + j, h, tile * 32 + j < M);
+        if (tile < n_tiles) load_tile(cur, tile * 32 + j);
     }
     // Where a tile is waited for. The hardware counts outstanding memory operations in order, and the compiler, which
     // places the waits, only knows an upper bound per register at a loop header: left to itself it waits for `cur` inside
@@ -139,10 +147,10 @@ __global__ void __launch_bounds__(THREADS, (THREADS >= 512 && W <= 64) ? 4 : 1)
         // prefetch the next tile of this wave while the current one is being computed
         const long long next_tile = tile + stride;
         vec8 nxt[NK];
-        if (next_tile < n_tiles) TL::load(nxt, x, next_tile * 32 + j, h, next_tile * 32 + j < M);
+        if (next_tile < n_tiles) load_tile(nxt, next_tile * 32 + j);
 
         if constexpr (STAGED != 0) TL::row_offsets(st_off, tile, lane, M);
-        if (STORE_INTERM) put(cur, out, row, valid);
+        if (STORE_INTERM && store_input) put(cur, out, row, valid);
         f32x16 acc[NI];
         for (int l = 0; l < n_mats - 1; ++l) {
             TL::template matmul<W_IN_LDS>(acc, cur, lds_w, wprep, l, lane);
@@ -158,7 +166,12 @@ __global__ void __launch_bounds__(THREADS, (THREADS >= 512 && W <= 64) ? 4 : 1)
             for (int kb = 0; kb < NK; ++kb) cur[kb] = nxt[kb];
             settle();
         }
-        put(res, STORE_INTERM ? out + (size_t)n_mats * M * W : out, row, valid);
+        if (STAGED == 0 && y_cols < W) // (whole rows only where they leave through a staged tile)
+            TL::store_columns(res, y, y_cols, row, h, valid);
+        else if constexpr (STORE_INTERM)
+            put(res, y ? y : out + (size_t)n_mats * M * W, row, valid);
+        else
+            put(res, y, row, valid);
         if (STORE_INTERM && next_tile < n_tiles) {
 #pragma unroll
             for (int kb = 0; kb < NK; ++kb) cur[kb] = nxt[kb];
@@ -185,7 +198,7 @@ constexpr int kStreamTiles = 2;
 template <typename T, int W, int ACT, bool STORE_INTERM, int STAGED = 0>
 __global__ void __launch_bounds__(kStreamThreads, 1)
     mlp_forward_stream_kernel(const typename Storage<T>::vec8 *__restrict__ wprep, const T *__restrict__ x, T *__restrict__ out,
-                              int n_mats, int out_act, long long M, int store_input) {
+                              int n_mats, int out_act, long long M, int store_input, T *__restrict__ y, int y_cols) {
     typedef Tile<T, W> TL;
     typedef typename Storage<T>::vec8 vec8;
     constexpr int NK = TL::NK, NI = TL::NI, R = kStreamTiles;
@@ -263,7 +276,10 @@ __global__ void __launch_bounds__(kStreamThreads, 1)
                     if (STORE_INTERM) put(t, out + (size_t)(l + 1) * M * W);
                 } else {
                     TL::repack_rt(cur[t], acc[t], out_act);
-                    put(t, STORE_INTERM ? out + (size_t)n_mats * M * W : out);
+                    if (y_cols < W)
+                        TL::store_columns(cur[t], y, y_cols, row[t], h, valid[t]);
+                    else
+                        put(t, (STORE_INTERM && !y) ? out + (size_t)n_mats * M * W : y);
                 }
             }
             b ^= 1;
@@ -458,27 +474,9 @@ const DeviceInfo &device_info() {
 constexpr size_t kLdsBudget = 144 * 1024;
 
 // Grid of a streaming kernel: as many workgroups as the device holds at once (registers and LDS decide),
-// capped by the number of 32-row tiles. The result per kernel is cached.
+// capped by the number of 32-row tiles.
 static long long stream_grid(const void *kernel, size_t lds_bytes, size_t M, int n_cu) {
-    struct Entry {
-        const void *k;
-        size_t lds;
-        int per_cu;
-    };
-    static thread_local Entry cache[64];
-    static thread_local int n_cache = 0;
-    int per_cu = 0;
-    for (int i = 0; i < n_cache; ++i)
-        if (cache[i].k == kernel && cache[i].lds == lds_bytes) per_cu = cache[i].per_cu;
-    if (!per_cu) {
-        int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, kFwdThreads, lds_bytes) != hipSuccess || nb < 1) {
-            (void)hipGetLastError();
-            nb = 1;
-        }
-        per_cu = nb;
-        if (n_cache < 64) cache[n_cache++] = Entry{kernel, lds_bytes, per_cu};
-    }
+    const int per_cu = resident_per_cu(kernel, kFwdThreads, lds_bytes);
     const long long n_tiles = ((long long)M + 31) / 32;
     const int waves = kFwdThreads / 64;
     long long blocks = (n_tiles + waves - 1) / waves;
@@ -486,15 +484,25 @@ static long long stream_grid(const void *kernel, size_t lds_bytes, size_t M, int
     return blocks < 1 ? 1 : blocks;
 }
 
+// What a forward pass may be given beside the plain matrices: see mlp_forward_kernel. x_cols = 0: x is M x W of T.
+struct ForwardRows {
+    bool store_input = true;
+    void *y = nullptr; // null: `out` (inference), or behind the activations
+    int y_cols = 0;    // 0: all
+    int x_cols = 0, x_fp32 = 0;
+    float fill = 0.0f;
+};
+
 template <typename T, int W, int ACT, bool STORE_INTERM, int THREADS>
-static int launch_forward_v(const tnn_mlp_desc *d, const void *wprep, const void *x, void *out, size_t M, hipStream_t s, int per_cu,
-                            bool store_input = true) { // store_input = false: the width-128 streaming route may leave matrix 0 of `out` unwritten
+static int launch_forward_v(const tnn_mlp_desc *d, const void *wprep, const void *x, void *out, size_t M, hipStream_t s, int per_cu, const ForwardRows &io) {
     typedef typename Storage<T>::vec8 vec8;
     const int n_mats = d->n_hidden_layers + 1;
     const size_t wbytes = prepared_elems(d) * sizeof(T);
     const DeviceInfo &di = device_info();
     if (!di.ok) return fail(TNN_ERR_HIP, "no usable HIP device");
     const bool in_lds = wbytes <= kLdsBudget;
+    T *const y = static_cast<T *>(io.y ? io.y : (STORE_INTERM ? nullptr : out));
+    const int y_cols = io.y_cols ? io.y_cols : W;
     if constexpr (W == 128) {
         // also for large batches when the weights would fit: the staging tiles of the whole-row stores do not fit beside
         // 128 KiB of weights, and the stores are what these passes are bound by (forward with stored activations, 4 matrices:
@@ -513,10 +521,9 @@ static int launch_forward_v(const tnn_mlp_desc *d, const void *wprep, const void
             auto k2 = mlp_forward_stream_kernel<T, W, ACT, STORE_INTERM, 2>;
             auto k = !fits32 ? k0 : (streaming ? k2 : k1);
             const size_t lds_k = fits32 ? lds_staged : lds;
-            if (hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_k) != hipSuccess)
-                return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", lds_k);
+            if (!reserve_lds(reinterpret_cast<const void *>(k), lds_k)) return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", lds_k);
             TNN_LAUNCH(k, dim3((unsigned)g), dim3(kStreamThreads), lds_k, s, (const vec8 *)wprep, (const T *)x, (T *)out, n_mats,
-                       d->output_activation, (long long)M, store_input ? 1 : 0);
+                       d->output_activation, (long long)M, io.store_input ? 1 : 0, y, y_cols);
             return check_launch("mlp_forward_stream_kernel");
         }
     }
@@ -530,38 +537,22 @@ static int launch_forward_v(const tnn_mlp_desc *d, const void *wprep, const void
     // and the matrix fits 32-bit offsets; with the streaming hint for an inference result, and for activations whose
     // volume exceeds the 256 MB of cache in front of the HBM (below that the backward pass finds them there).
     const size_t staged_bytes = wbytes + (size_t)waves * Tile<T, W>::TILE_BYTES;
-    const bool staged = W <= 64 && in_lds && staged_bytes * per_cu <= 160 * 1024 &&
+    const bool staged = W <= 64 && in_lds && staged_bytes * per_cu <= 160 * 1024 && !io.x_cols && y_cols == W &&
                         (unsigned long long)M * W * sizeof(T) <= Tile<T, W>::kMaxBufferBytes;
     const bool streaming = !STORE_INTERM || (unsigned long long)(n_mats + 1) * M * W * sizeof(T) > (256ull << 20);
+    auto k = in_lds ? mlp_forward_kernel<T, W, ACT, STORE_INTERM, true, THREADS> : mlp_forward_kernel<T, W, ACT, STORE_INTERM, false, THREADS>;
+    size_t lds = in_lds ? wbytes : 0;
     if (staged) {
-        auto k1 = mlp_forward_kernel<T, W, ACT, STORE_INTERM, true, THREADS, (W <= 64 ? 1 : 0)>;
-        auto k2 = mlp_forward_kernel<T, W, ACT, STORE_INTERM, true, THREADS, (W <= 64 ? 2 : 0)>;
-        auto k = streaming ? k2 : k1;
-        // the reservation is a host round trip of several microseconds: once per kernel, device and size
-        static thread_local size_t reserved[2][16] = {};
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return fail(TNN_ERR_HIP, "no usable HIP device");
-        if (staged_bytes > 48 * 1024 && reserved[streaming][dev] < staged_bytes) {
-            if (hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)staged_bytes) != hipSuccess)
-                return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", staged_bytes);
-            reserved[streaming][dev] = staged_bytes;
-        }
-        TNN_LAUNCH(k, dim3((unsigned)blocks), dim3(THREADS), staged_bytes, s, (const vec8 *)wprep, (const T *)x,
-                           (T *)out, n_mats, d->output_activation, (long long)M);
-    } else if (in_lds) {
-        auto k = mlp_forward_kernel<T, W, ACT, STORE_INTERM, true, THREADS>;
-        if (wbytes > 48 * 1024 &&
-            hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)wbytes) != hipSuccess)
-            return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", wbytes);
-        TNN_LAUNCH(k, dim3((unsigned)blocks), dim3(THREADS), wbytes, s, (const vec8 *)wprep, (const T *)x,
-                           (T *)out, n_mats, d->output_activation, (long long)M);
-    } else {
-        auto k = mlp_forward_kernel<T, W, ACT, STORE_INTERM, false, THREADS>;
-        TNN_LAUNCH(k, dim3((unsigned)blocks), dim3(THREADS), 0, s, (const vec8 *)wprep, (const T *)x, (T *)out,
-                           n_mats, d->output_activation, (long long)M);
+        k = streaming ? mlp_forward_kernel<T, W, ACT, STORE_INTERM, true, THREADS, (W <= 64 ? 2 : 0)>
+                      : mlp_forward_kernel<T, W, ACT, STORE_INTERM, true, THREADS, (W <= 64 ? 1 : 0)>;
+        lds = staged_bytes;
     }
+    if constexpr (!STORE_INTERM && THREADS == 512) {
+        if (io.x_cols) k = in_lds ? mlp_forward_kernel<T, W, ACT, false, true, 512, 0, true> : mlp_forward_kernel<T, W, ACT, false, false, 512, 0, true>;
+    }
+    if (!reserve_lds(reinterpret_cast<const void *>(k), lds)) return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", lds);
+    TNN_LAUNCH(k, dim3((unsigned)blocks), dim3(THREADS), lds, s, (const vec8 *)wprep, (const T *)x, (T *)out, n_mats, d->output_activation, (long long)M, y,
+               y_cols, io.store_input ? 1 : 0, io.x_cols, io.x_fp32, io.fill);
     return check_launch("mlp_forward_kernel");
 }
 
@@ -569,25 +560,25 @@ static int launch_forward_v(const tnn_mlp_desc *d, const void *wprep, const void
 // measured faster than 256-thread workgroups at higher counts and than variants that hold the next matrix's
 // fragments in registers.
 template <typename T, int W, int ACT, bool STORE_INTERM>
-static int launch_forward_act(const tnn_mlp_desc *d, const void *wprep, const void *x, void *out, size_t M, hipStream_t s, bool store_input = true) {
+static int launch_forward_act(const tnn_mlp_desc *d, const void *wprep, const void *x, void *out, size_t M, hipStream_t s, const ForwardRows &io) {
     if constexpr (W <= 64) {
         // From two tiles per wave on a full chip: one workgroup of 16 waves per CU instead of two of 8, so that the weights
         // are staged once per CU (inference at 2^18 rows, w64 with 4 hidden layers: 13.7 -> 13.2 us); below that the
         // smaller workgroups spread over more CUs.
         const DeviceInfo &di = device_info();
         const size_t staged_bytes = prepared_elems(d) * sizeof(T) + 16 * (size_t)Tile<T, W>::TILE_BYTES;
-        if (di.ok && (M + 31) / 32 >= (size_t)di.n_cu * 32 && staged_bytes <= 160 * 1024)
-            return launch_forward_v<T, W, ACT, STORE_INTERM, 1024>(d, wprep, x, out, M, s, 1);
+        if (di.ok && (M + 31) / 32 >= (size_t)di.n_cu * 32 && staged_bytes <= 160 * 1024 && !io.x_cols)
+            return launch_forward_v<T, W, ACT, STORE_INTERM, 1024>(d, wprep, x, out, M, s, 1, io);
     }
-    return launch_forward_v<T, W, ACT, STORE_INTERM, 512>(d, wprep, x, out, M, s, 2, store_input);
+    return launch_forward_v<T, W, ACT, STORE_INTERM, 512>(d, wprep, x, out, M, s, 2, io);
 }
 
 template <typename T, int W, bool STORE_INTERM>
-static int launch_forward(const tnn_mlp_desc *d, const void *wprep, const void *x, void *out, size_t M, hipStream_t s, bool store_input = true) {
+static int launch_forward(const tnn_mlp_desc *d, const void *wprep, const void *x, void *out, size_t M, hipStream_t s, const ForwardRows &io = ForwardRows{}) {
     switch (d->activation) {
-    case TNN_ACT_RELU: return launch_forward_act<T, W, TNN_ACT_RELU, STORE_INTERM>(d, wprep, x, out, M, s, store_input);
-    case TNN_ACT_SIGMOID: return launch_forward_act<T, W, TNN_ACT_SIGMOID, STORE_INTERM>(d, wprep, x, out, M, s, store_input);
-    default: return launch_forward_act<T, W, TNN_ACT_NONE, STORE_INTERM>(d, wprep, x, out, M, s, store_input);
+    case TNN_ACT_RELU: return launch_forward_act<T, W, TNN_ACT_RELU, STORE_INTERM>(d, wprep, x, out, M, s, io);
+    case TNN_ACT_SIGMOID: return launch_forward_act<T, W, TNN_ACT_SIGMOID, STORE_INTERM>(d, wprep, x, out, M, s, io);
+    default: return launch_forward_act<T, W, TNN_ACT_NONE, STORE_INTERM>(d, wprep, x, out, M, s, io);
     }
 }
 
@@ -604,9 +595,7 @@ static int launch_backward(const tnn_mlp_desc *d, const void *wprep_bwd, const v
     const bool in_lds = wbytes <= kLdsBudget;
     if (in_lds) {
         auto k = mlp_backward_kernel<T, W, true>;
-        if (wbytes > 48 * 1024 &&
-            hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)wbytes) != hipSuccess)
+        if (!reserve_lds(reinterpret_cast<const void *>(k), wbytes))
             return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", wbytes);
         const long long blocks = stream_grid(reinterpret_cast<const void *>(k), wbytes, M, di.n_cu);
         TNN_LAUNCH(k, dim3((unsigned)blocks), dim3(kFwdThreads), wbytes, s, (const vec8 *)wprep_bwd,
@@ -653,11 +642,7 @@ static int launch_dw(const tnn_mlp_desc *d, const void *interm_bwd, const void *
                        (const T *)interm_bwd, (const T *)interm_fwd, partials, n_mats, (long long)M, p.rows_per_chunk);
     int rc = check_launch("mlp_dw_partial_kernel");
     if (rc) return rc;
-    const int n_elems = n_mats * W * W;
-    TNN_LAUNCH((train_reduce_kernel<T, false>), dim3(n_elems / 64), dim3(512), 0, s, partials, (const float *)nullptr,
-               (int)(p.n_chunks * p.partials_per_chunk), n_elems, dW_is_fp32 ? (T *)nullptr : (T *)dW,
-               dW_is_fp32 ? (float *)dW : (float *)nullptr, (float *)nullptr, AdamArgs{});
-    return check_launch("train_reduce_kernel");
+    return launch_train_reduce<T>(partials, nullptr, (int)(p.n_chunks * p.partials_per_chunk), n_mats * W * W, dW, dW_is_fp32, nullptr, TrainTail{}, s);
 }
 
 // Width 128: one launch per layer that forms delta_{l-1} and dW_l together (mlp_backward128.inc), then the reduction.
@@ -669,7 +654,7 @@ static int launch_backward128(const tnn_mlp_desc *d, const void *wprep_bwd, cons
                               bool keep_top_delta, void *dW, int dW_is_fp32, void *dLdx, size_t M, float *partials, hipStream_t s,
                               const float *targets = nullptr, float loss_scale = 0.0f, float *loss_sum = nullptr, const void *x0 = nullptr,
                               const void *wprep_fwd = nullptr, // (with targets): the network's output is not in interm_fwd, the top launch forms it
-                              const TrainTail &tail = TrainTail{}) {
+                              const TrainTail &tail = TrainTail{}, const void *y = nullptr) { // y: the network's output, null: behind the activations
     typedef typename Storage<T>::vec8 vec8;
     constexpr int W = 128;
     const int n_mats = d->n_hidden_layers + 1;
@@ -681,11 +666,11 @@ static int launch_backward128(const tnn_mlp_desc *d, const void *wprep_bwd, cons
     auto k_pair = mlp_layer_pair_backward128_kernel<T>;
     const float inv_n = 1.0f / (float)(M * W);
     const size_t top_lds = reform ? LayerBwd128::pair_lds_bytes : LayerBwd128::lds_bytes;
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k_top), hipFuncAttributeMaxDynamicSharedMemorySize, (int)top_lds) != hipSuccess)
+    if (!reserve_lds(reinterpret_cast<const void *>(k_top), top_lds))
         return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", top_lds);
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k_mid), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LayerBwd128::lds_bytes) != hipSuccess)
+    if (!reserve_lds(reinterpret_cast<const void *>(k_mid), LayerBwd128::lds_bytes))
         return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", LayerBwd128::lds_bytes);
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(k_pair), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LayerBwd128::pair_lds_bytes) != hipSuccess)
+    if (!reserve_lds(reinterpret_cast<const void *>(k_pair), LayerBwd128::pair_lds_bytes))
         return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", LayerBwd128::pair_lds_bytes);
     const T *fwd = static_cast<const T *>(interm_fwd);
     const T *input0 = x0 ? static_cast<const T *>(x0) : fwd; // the first matrix's input: the caller's x, or its copy in front of the activations
@@ -705,7 +690,7 @@ static int launch_backward128(const tnn_mlp_desc *d, const void *wprep_bwd, cons
             TNN_LAUNCH(k_pair, dim3((unsigned)p.n_chunks), dim3(kLayerBwdThreads), LayerBwd128::pair_lds_bytes, s, wb + (size_t)l * per_mat,
                        wb + (size_t)(l - 1) * per_mat, dl + (size_t)l * mat, fwd + (size_t)l * mat, l > 1 ? fwd + (size_t)(l - 1) * mat : input0,
                        keep_top_delta ? dl + (size_t)(l - 1) * mat : (T *)nullptr, delta_out, partials, n_mats, l, d->activation,
-                       l > 1 ? d->activation : TNN_ACT_NONE, (long long)M, p.rows_per_chunk);
+                       l > 1 ? d->activation : TNN_ACT_NONE, l > 1 ? 1.0f : tail.result_scale, (long long)M, p.rows_per_chunk);
             const int rc = check_launch("mlp_layer_pair_backward128_kernel");
             if (rc) return rc;
             l -= 2;
@@ -715,25 +700,16 @@ static int launch_backward128(const tnn_mlp_desc *d, const void *wprep_bwd, cons
         T *delta_out = l > 0 ? dl + (size_t)(l - 1) * mat : static_cast<T *>(dLdx);
         const int gate = l > 0 ? d->activation : TNN_ACT_NONE;
         TNN_LAUNCH((top ? k_top : k_mid), dim3((unsigned)p.n_chunks), dim3(kLayerBwdThreads), top ? top_lds : LayerBwd128::lds_bytes, s,
-                   wb + (size_t)l * per_mat, delta_in, l > 0 ? fwd + (size_t)l * mat : input0, fwd + (size_t)n_mats * mat,
+                   wb + (size_t)l * per_mat, delta_in, l > 0 ? fwd + (size_t)l * mat : input0, y ? static_cast<const T *>(y) : fwd + (size_t)n_mats * mat,
                    (top && keep_top_delta) ? dl + (size_t)l * mat : (T *)nullptr, delta_out, partials, n_mats, l, gate, d->output_activation, (long long)M,
-                   p.rows_per_chunk, targets, loss_scale, inv_n, loss_partials,
+                   p.rows_per_chunk, targets, targets ? loss_scale : tail.dy_scale, inv_n, loss_partials, l > 0 ? 1.0f : tail.result_scale,
                    (top && reform) ? static_cast<const vec8 *>(wprep_fwd) + (size_t)l * per_mat : (const vec8 *)nullptr);
         const int rc = check_launch("mlp_layer_backward128_kernel");
         if (rc) return rc;
         l -= 1;
     }
     if (tail.main_done && hipEventRecord(tail.main_done, s) != hipSuccess) return fail(TNN_ERR_HIP, "hipEventRecord failed");
-    const int n_elems = n_mats * W * W;
-    T *dW_T = (dW && !dW_is_fp32) ? (T *)dW : (T *)nullptr;
-    float *dW_f32 = (dW && dW_is_fp32) ? (float *)dW : (float *)nullptr;
-    if (tail.use_adam)
-        TNN_LAUNCH((train_reduce_kernel<T, true>), dim3(n_elems / 64), dim3(512), 0, s, partials, loss_partials, (int)p.n_chunks, n_elems, dW_T, dW_f32,
-                   loss_partials ? loss_sum : (float *)nullptr, tail.adam);
-    else
-        TNN_LAUNCH((train_reduce_kernel<T, false>), dim3(n_elems / 64), dim3(512), 0, s, partials, loss_partials, (int)p.n_chunks, n_elems, dW_T, dW_f32,
-                   loss_partials ? loss_sum : (float *)nullptr, tail.adam);
-    return check_launch("train_reduce_kernel");
+    return launch_train_reduce<T>(partials, loss_partials, (int)p.n_chunks, n_mats * W * W, dW, dW_is_fp32, loss_partials ? loss_sum : nullptr, tail, s);
 }
 
 // For tnn_mlp_train_step_l2 on width 128. The forward pass with stored activations that does not copy the input in front of
@@ -746,8 +722,10 @@ int forward128_for_training(const tnn_mlp_desc *desc, const void *wprep, const v
         d.n_hidden_layers -= 1;
         d.output_activation = d.activation; // the last matrix that runs is a hidden layer's
     }
-    if (desc->dtype == TNN_BF16) return launch_forward<bf16_t, 128, true>(&d, wprep, x, interm_fwd, M, s, false);
-    return launch_forward<fp16_t, 128, true>(&d, wprep, x, interm_fwd, M, s, false);
+    ForwardRows io;
+    io.store_input = false;
+    if (desc->dtype == TNN_BF16) return launch_forward<bf16_t, 128, true>(&d, wprep, x, interm_fwd, M, s, io);
+    return launch_forward<fp16_t, 128, true>(&d, wprep, x, interm_fwd, M, s, io);
 }
 
 // ... and loss and backward pass over those activations, the loss folded into the top layer's launch and the first matrix's
@@ -939,6 +917,69 @@ TNN_API int tnn_mlp_forward(const tnn_mlp_desc *desc, const void *d_prepared_fwd
     if (!d_prepared_fwd || !d_x || !d_interm_fwd) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
     TNN_DISPATCH_TW(desc, rc = (launch_forward<T_, W_, true>(desc, d_prepared_fwd, d_x, d_interm_fwd, M, as_stream(stream))));
     return rc;
+}
+
+TNN_API int tnn_mlp_inference_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_x, int x_dtype, int x_cols, float fill, void *d_y,
+                                   int y_cols, size_t M, tnn_stream_t stream) {
+    int rc = check_mlp_desc(desc);
+    if (rc) return rc;
+    if (M == 0) return fail(TNN_ERR_INVALID_ARGUMENT, "empty batch");
+    if (!d_prepared_fwd || !d_x || !d_y) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    if (x_cols < 1 || x_cols > desc->width || y_cols < 1 || y_cols > desc->width)
+        return fail(TNN_ERR_INVALID_ARGUMENT, "%d input and %d output columns for a network of width %d", x_cols, y_cols, desc->width);
+    if (x_dtype != desc->dtype && x_dtype != TNN_FP32) return fail(TNN_ERR_UNSUPPORTED, "x of dtype %d", x_dtype);
+    ForwardRows io;
+    io.y_cols = y_cols;
+    if (x_cols != desc->width || x_dtype != desc->dtype) {
+        io.x_cols = x_cols;
+        io.x_fp32 = x_dtype == TNN_FP32;
+        io.fill = fill;
+        if (desc->width == 128 && (prepared_elems(desc) * 2 > kLdsBudget || M >= 65536))
+            return fail(TNN_ERR_UNSUPPORTED, "the width-128 kernel for deep networks and large batches takes whole rows (tnn_resize_rows)");
+    }
+    TNN_DISPATCH_TW(desc, rc = (launch_forward<T_, W_, false>(desc, d_prepared_fwd, d_x, d_y, M, as_stream(stream), io)));
+    return rc;
+}
+
+TNN_API int tnn_mlp_forward_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_x, void *d_hidden, void *d_y, int y_cols, size_t M,
+                                 tnn_stream_t stream) {
+    int rc = check_mlp_desc(desc);
+    if (rc) return rc;
+    if (M == 0) return fail(TNN_ERR_INVALID_ARGUMENT, "empty batch");
+    if (!d_prepared_fwd || !d_x || !d_hidden || !d_y) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    if (y_cols < 1 || y_cols > desc->width) return fail(TNN_ERR_INVALID_ARGUMENT, "%d output columns for a network of width %d", y_cols, desc->width);
+    if (desc->width != 128) return fail(TNN_ERR_UNSUPPORTED, "built for width 128");
+    ForwardRows io;
+    io.store_input = false;
+    io.y = d_y;
+    io.y_cols = y_cols;
+    char *interm = static_cast<char *>(d_hidden) - M * 128 * 2; // matrix 0 is not touched
+    if (desc->dtype == TNN_BF16) return launch_forward<bf16_t, 128, true>(desc, d_prepared_fwd, d_x, interm, M, as_stream(stream), io);
+    return launch_forward<fp16_t, 128, true>(desc, d_prepared_fwd, d_x, interm, M, as_stream(stream), io);
+}
+
+TNN_API int tnn_mlp_backward_rows(const tnn_mlp_desc *desc, const void *d_prepared_bwd, const void *d_x, const void *d_hidden, const void *d_y,
+                                  const void *d_dLdy, float dy_scale, float result_scale, void *d_dW_packed, int dW_dtype, void *d_dLdx, size_t M,
+                                  void *d_workspace, size_t workspace_bytes, tnn_stream_t stream) {
+    int rc = check_mlp_desc(desc);
+    if (rc) return rc;
+    if (desc->width != 128) return fail(TNN_ERR_UNSUPPORTED, "built for width 128");
+    if (!d_prepared_bwd || !d_x || !d_hidden || !d_dLdy || (!d_y && desc->output_activation != TNN_ACT_NONE))
+        return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    TrainTail tail;
+    if ((rc = rows_tail(desc, desc->width, dy_scale, result_scale, d_dW_packed, dW_dtype, M, &tail))) return rc;
+    const size_t need = tnn_mlp_backward_workspace_bytes(desc, M);
+    if (!d_workspace || workspace_bytes < need) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
+    uintptr_t base = (reinterpret_cast<uintptr_t>(d_workspace) + 255) & ~(uintptr_t)255;
+    float *partials = reinterpret_cast<float *>(base);
+    void *deltas = reinterpret_cast<void *>(base + ((dw_plan(desc, M).partial_bytes + 255) & ~(size_t)255));
+    const char *interm = static_cast<const char *>(d_hidden) - M * 128 * 2;
+    const void *y = d_y ? d_y : d_hidden; // (not read without an output activation)
+    if (desc->dtype == TNN_BF16)
+        return launch_backward128<bf16_t>(desc, d_prepared_bwd, d_dLdy, interm, deltas, false, nullptr, 1, d_dLdx, M, partials, as_stream(stream), nullptr,
+                                          0.0f, nullptr, d_x, nullptr, tail, y);
+    return launch_backward128<fp16_t>(desc, d_prepared_bwd, d_dLdy, interm, deltas, false, nullptr, 1, d_dLdx, M, partials, as_stream(stream), nullptr, 0.0f,
+                                      nullptr, d_x, nullptr, tail, y);
 }
 
 TNN_API size_t tnn_mlp_backward_workspace_bytes(const tnn_mlp_desc *desc, size_t M) {

@@ -115,6 +115,14 @@ __device__ __forceinline__ typename Storage<T>::vec8 bwd_convert(const f32x16 &c
     return __builtin_bit_cast(typename Storage<T>::vec8, r);
 }
 
+// Every value times `by`, rounded to T.
+template <typename T> __device__ __forceinline__ typename Storage<T>::vec8 scaled(const typename Storage<T>::vec8 v, float by) {
+    f32x8 f = __builtin_convertvector(v, f32x8);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = as_fp32(f[e] * by);
+    return __builtin_convertvector(f, typename Storage<T>::vec8);
+}
+
 // "nt" bit of a buffer store: the line is written through instead of staying dirty in L2 until the kernel ends. Only
 // with stores that cover whole 128-byte lines; with partial lines it costs more than it saves.
 constexpr int kStreamingStore = 2;
@@ -142,6 +150,47 @@ template <typename T, int W> struct Tile {
         if (valid) {
 #pragma unroll
             for (int kb = 0; kb < NK; ++kb) p[2 * kb] = r[kb];
+        }
+    }
+
+    // The first `cols` columns of the rows, into a matrix of that many columns.
+    static __device__ __forceinline__ void store_columns(const vec8 (&r)[NK], T *__restrict__ base, int cols, long long row, int h, bool valid) {
+        if (!valid) return;
+        T *p = base + row * cols;
+#pragma unroll
+        for (int kb = 0; kb < NK; ++kb) {
+            const int c = 16 * kb + 8 * h;
+            if ((cols & 7) == 0) {
+                if (c < cols) *reinterpret_cast<vec8 *>(p + c) = r[kb];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (c + e < cols) p[c + e] = r[kb][e];
+            }
+        }
+    }
+    // A row of `cols` columns of T or fp32 (rounded to T), the others `fill`.
+    static __device__ __forceinline__ void load_columns(vec8 (&r)[NK], const void *__restrict__ base, bool fp32, int cols, T fill, long long row, int h,
+                                                        bool valid) {
+        if (!valid) row = 0;
+        const float *pf = static_cast<const float *>(base) + row * cols;
+        const T *pt = static_cast<const T *>(base) + row * cols;
+#pragma unroll
+        for (int kb = 0; kb < NK; ++kb) {
+            const int c = 16 * kb + 8 * h;
+            if (fp32 && (cols & 7) == 0 && c < cols) {
+                const f32x4 a = *reinterpret_cast<const f32x4 *>(pf + c), b = *reinterpret_cast<const f32x4 *>(pf + c + 4);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) r[kb][e] = (T)(e < 4 ? a[e & 3] : b[e & 3]);
+            } else if (!fp32 && (cols & 7) == 0 && c < cols) {
+                r[kb] = *reinterpret_cast<const vec8 *>(pt + c);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    r[kb][e] = fill;
+                    if (c + e < cols) r[kb][e] = fp32 ? (T)pf[c + e] : pt[c + e];
+                }
+            }
         }
     }
 

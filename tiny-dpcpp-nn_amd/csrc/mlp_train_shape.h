@@ -47,9 +47,12 @@ int fused_train_launch_fp16(const tnn_mlp_desc *d, const FusedPlan &p, const voi
 
 // The same kernels with dL/dy given by the caller (mlp_train_given_*.hip): backward pass with the activations formed again on chip.
 int fused_given_launch_bf16(const tnn_mlp_desc *d, const FusedPlan &p, const void *wf, const void *wb, const void *x, const void *dLdy, void *dW,
-                            int dW_is_fp32, void *dx, size_t M, float *partials, float *loss_partials, hipStream_t s);
+                            int dW_is_fp32, void *dx, size_t M, float *partials, float *loss_partials, const TrainTail &tail, hipStream_t s);
 int fused_given_launch_fp16(const tnn_mlp_desc *d, const FusedPlan &p, const void *wf, const void *wb, const void *x, const void *dLdy, void *dW,
-                            int dW_is_fp32, void *dx, size_t M, float *partials, float *loss_partials, hipStream_t s);
+                            int dW_is_fp32, void *dx, size_t M, float *partials, float *loss_partials, const TrainTail &tail, hipStream_t s);
+
+// Checks what the backward passes on a caller's rows are given (train.hip) and puts it into their tail.
+int rows_tail(const tnn_mlp_desc *desc, int dy_cols, float dy_scale, float result_scale, void *d_dW_packed, int dW_dtype, size_t M, TrainTail *tail);
 
 // Backward pass with the weight gradients in the same kernel (mlp_backward_fused.inc). TNN_ERR_UNSUPPORTED when the shape has
 // no such kernel or the workspace holds no partial tile; the caller then runs the separate kernels.

@@ -22,6 +22,11 @@ inline hipStream_t as_stream(tnn_stream_t s) { return reinterpret_cast<hipStream
 // Reports a failed launch as TNN_ERR_HIP. Does not synchronize.
 int check_launch(const char *what);
 
+// Reserves `bytes` of dynamic LDS for a kernel that wants more than every kernel may have, and how many of its workgroups a CU
+// holds at once (at least 1). Both ask the runtime, microseconds each time, so the answers are kept per thread, device and kernel.
+bool reserve_lds(const void *kernel, size_t bytes);
+int resident_per_cu(const void *kernel, int threads, size_t lds_bytes);
+
 // Every kernel goes out through this: an error that an earlier, unrelated runtime call of this thread left
 // behind (a failed allocation of the caller, say) is dropped first, so that check_launch reports this launch only.
 #define TNN_LAUNCH(...)                                                                                                \

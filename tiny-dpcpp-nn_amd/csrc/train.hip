@@ -164,6 +164,21 @@ TNN_API int tnn_mlp_train_step_l2_adam(const tnn_mlp_desc *desc, void *d_prepare
                                d_prepared_fwd, d_prepared_bwd, stream);
 }
 
+namespace tnn {
+int rows_tail(const tnn_mlp_desc *desc, int dy_cols, float dy_scale, float result_scale, void *d_dW_packed, int dW_dtype, size_t M, TrainTail *tail) {
+    if (M == 0) return fail(TNN_ERR_INVALID_ARGUMENT, "empty batch");
+    if (!d_dW_packed) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    if (dy_cols < 1 || (dy_cols > 16 && dy_cols != desc->width))
+        return fail(TNN_ERR_UNSUPPORTED, "dL/dy of %d columns: at most 16, or the network's width", dy_cols);
+    if (dW_dtype != TNN_FP32 && dW_dtype != desc->dtype) return fail(TNN_ERR_UNSUPPORTED, "weight gradients of dtype %d", dW_dtype);
+    tail->dy_cols = dy_cols == desc->width ? 0 : dy_cols;
+    tail->dy_scale = dy_scale;
+    tail->result_scale = result_scale;
+    tail->packed = PackedGradient{d_dW_packed, dW_dtype, desc->width, result_scale};
+    return TNN_OK;
+}
+} // namespace tnn
+
 TNN_API int tnn_mlp_backward_recompute_supported(const tnn_mlp_desc *desc) {
     int rc = check_mlp_desc(desc);
     if (rc) return rc;
@@ -171,13 +186,12 @@ TNN_API int tnn_mlp_backward_recompute_supported(const tnn_mlp_desc *desc) {
     return TNN_OK;
 }
 
-TNN_API int tnn_mlp_backward_recompute(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_x,
-                                       const void *d_dLdy, void *d_dW, int dW_is_fp32, void *d_dLdx, size_t M, void *d_workspace,
-                                       size_t workspace_bytes, tnn_stream_t stream) {
+static int backward_recompute(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_x, const void *d_dLdy,
+                              void *d_dW, int dW_is_fp32, void *d_dLdx, size_t M, void *d_workspace, size_t workspace_bytes, const TrainTail &tail,
+                              tnn_stream_t stream) {
     int rc = tnn_mlp_backward_recompute_supported(desc);
     if (rc) return rc;
-    if (!d_prepared_fwd || !d_prepared_bwd || !d_x || !d_dLdy || !d_dW) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
-    if (M == 0 || (M % 8) != 0) return fail(TNN_ERR_INVALID_ARGUMENT, "batch size %zu is not a positive multiple of 8", M);
+    if (!d_prepared_fwd || !d_prepared_bwd || !d_x || !d_dLdy || (!d_dW && !tail.packed.p)) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
     const FusedPlan p = fused_plan(desc, M);
     const size_t need = p.partial_bytes + p.loss_bytes + 512;
     if (!d_workspace || workspace_bytes < need) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
@@ -186,8 +200,29 @@ TNN_API int tnn_mlp_backward_recompute(const tnn_mlp_desc *desc, const void *d_p
     float *partials = reinterpret_cast<float *>(base + p.loss_bytes);
     hipStream_t s = as_stream(stream);
     if (desc->dtype == TNN_BF16)
-        return fused_given_launch_bf16(desc, p, d_prepared_fwd, d_prepared_bwd, d_x, d_dLdy, d_dW, dW_is_fp32, d_dLdx, M, partials, loss_partials, s);
-    return fused_given_launch_fp16(desc, p, d_prepared_fwd, d_prepared_bwd, d_x, d_dLdy, d_dW, dW_is_fp32, d_dLdx, M, partials, loss_partials, s);
+        return fused_given_launch_bf16(desc, p, d_prepared_fwd, d_prepared_bwd, d_x, d_dLdy, d_dW, dW_is_fp32, d_dLdx, M, partials, loss_partials, tail, s);
+    return fused_given_launch_fp16(desc, p, d_prepared_fwd, d_prepared_bwd, d_x, d_dLdy, d_dW, dW_is_fp32, d_dLdx, M, partials, loss_partials, tail, s);
+}
+
+TNN_API int tnn_mlp_backward_recompute(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_x,
+                                       const void *d_dLdy, void *d_dW, int dW_is_fp32, void *d_dLdx, size_t M, void *d_workspace,
+                                       size_t workspace_bytes, tnn_stream_t stream) {
+    int rc = tnn_mlp_backward_recompute_supported(desc);
+    if (rc) return rc;
+    if (!d_dW) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    if (M == 0 || (M % 8) != 0) return fail(TNN_ERR_INVALID_ARGUMENT, "batch size %zu is not a positive multiple of 8", M);
+    return backward_recompute(desc, d_prepared_fwd, d_prepared_bwd, d_x, d_dLdy, d_dW, dW_is_fp32, d_dLdx, M, d_workspace, workspace_bytes, TrainTail{},
+                              stream);
+}
+
+TNN_API int tnn_mlp_backward_recompute_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_x,
+                                            const void *d_dLdy, int dy_cols, float dy_scale, float result_scale, void *d_dW_packed, int dW_dtype,
+                                            void *d_dLdx, size_t M, void *d_workspace, size_t workspace_bytes, tnn_stream_t stream) {
+    int rc = check_mlp_desc(desc);
+    if (rc) return rc;
+    TrainTail tail;
+    if ((rc = rows_tail(desc, dy_cols, dy_scale, result_scale, d_dW_packed, dW_dtype, M, &tail))) return rc;
+    return backward_recompute(desc, d_prepared_fwd, d_prepared_bwd, d_x, d_dLdy, nullptr, 1, d_dLdx, M, d_workspace, workspace_bytes, tail, stream);
 }
 
 // ------------------------------------------------------------------------------------------------

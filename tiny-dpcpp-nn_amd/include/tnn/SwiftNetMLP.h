@@ -70,7 +70,7 @@ template <typename T, int WIDTH> class SwiftNetMLP : public Network<T> {
                                                 DeviceMatricesView<T> output, const bool a_backward_pass_follows = false) {
         if (Network<T>::get_input_width() != WIDTH) throw std::invalid_argument("The encoding must be padded to the network width.");
         const tnn_mlp_desc d = desc();
-        if (M >= (size_t(1) << (a_backward_pass_follows ? 17 : 18))) {
+        if (M >= OrderedFrom(a_backward_pass_follows)) {
             // large batches: points in cell order gather from shared lines of the table (same rows, bit for bit)
             OrderPoints(grid, positions, M);
             tnn::abi_check(tnn_grid_mlp_inference_ordered(&grid, &d, m_grid_order->data(), table, this->prepared_forward(),
@@ -151,7 +151,7 @@ template <typename T, int WIDTH> class SwiftNetMLP : public Network<T> {
         const tnn_mlp_desc d = desc();
         ReserveWorkspace(tnn_grid_mlp_train_step_workspace_bytes(&grid, &d, M));
         const void *order = nullptr;
-        if (M >= (size_t(1) << 17)) {
+        if (M >= OrderedFrom(true)) {
             if (!(positions_as_last_ordered && OrderIsOf(grid, positions, M))) OrderPoints(grid, positions, M);
             order = m_grid_order->data();
         }
@@ -159,6 +159,69 @@ template <typename T, int WIDTH> class SwiftNetMLP : public Network<T> {
                                              dL_doutput.GetPointer(), output.GetMatrixPointer(0), 0, grad_table, 1, M, workspace_, workspace_bytes_,
                                              this->get_queue().abi()));
         return {tnn::event(this->get_queue().get())};
+    }
+
+    // The passes on a caller's own rows (see the section of that name in tnn_hip.h), for the tensor-level modules: raw pointers and
+    // scratch memory of the caller's. `fill` of the input's padding columns: ones with the bias trick, zeros otherwise.
+    /// Whether inference_rows takes an input that is not M x WIDTH of T.
+    bool takes_narrow_rows(const size_t M) const {
+        return WIDTH < 128 || (M < 65536 && this->get_n_hidden_layers() + 1 <= 4);
+    }
+    void inference_rows(const void *x, const int x_dtype, const int x_cols, void *y, const int y_cols, const size_t M, const float fill) {
+        const tnn_mlp_desc d = desc();
+        tnn::abi_check(tnn_mlp_inference_rows(&d, this->prepared_forward(), x, x_dtype, x_cols, fill, y, y_cols, M, this->get_queue().abi()));
+    }
+    void inference_with_grid_rows(const tnn_grid_desc &grid, const void *table, const float *positions, const size_t M, void *y, const int y_cols,
+                                  const bool a_backward_pass_follows) {
+        const tnn_mlp_desc d = desc();
+        const void *order = nullptr;
+        if (M >= OrderedFrom(a_backward_pass_follows)) {
+            OrderPoints(grid, positions, M);
+            order = m_grid_order->data();
+        }
+        tnn::abi_check(tnn_grid_mlp_inference_rows(&grid, &d, positions, order, table, this->prepared_forward(), y, y_cols, M, this->get_queue().abi()));
+    }
+    size_t backward_recompute_scratch_bytes(const size_t M) const {
+        const tnn_mlp_desc d = desc();
+        return tnn_mlp_train_step_workspace_bytes(&d, M);
+    }
+    void backward_recompute_rows(const void *x, const void *dLdy, const int dy_cols, const float dy_scale, const float result_scale, void *dW_packed,
+                                 const int dW_dtype, void *dLdx, const size_t M, void *scratch, const size_t scratch_bytes) {
+        const tnn_mlp_desc d = desc();
+        tnn::abi_check(tnn_mlp_backward_recompute_rows(&d, this->prepared_forward(), this->prepared_backward(), x, dLdy, dy_cols, dy_scale, result_scale,
+                                                       dW_packed, dW_dtype, dLdx, M, scratch, scratch_bytes, this->get_queue().abi()));
+    }
+    size_t backward_with_grid_scratch_bytes(const tnn_grid_desc &grid, const size_t M) const {
+        const tnn_mlp_desc d = desc();
+        return tnn_grid_mlp_train_step_workspace_bytes(&grid, &d, M);
+    }
+    void backward_with_grid_rows(const tnn_grid_desc &grid, const void *table, const float *positions, const void *dLdy, const int dy_cols,
+                                 const float dy_scale, const float result_scale, void *dW_packed, const int dW_dtype, float *grad_table, const size_t M,
+                                 void *scratch, const size_t scratch_bytes, const bool positions_as_last_ordered) {
+        const tnn_mlp_desc d = desc();
+        const void *order = nullptr;
+        if (M >= OrderedFrom(true)) {
+            if (!(positions_as_last_ordered && OrderIsOf(grid, positions, M))) OrderPoints(grid, positions, M);
+            order = m_grid_order->data();
+        }
+        tnn::abi_check(tnn_grid_mlp_backward_rows(&grid, &d, positions, order, table, this->prepared_forward(), this->prepared_backward(), dLdy, dy_cols,
+                                                  dy_scale, result_scale, dW_packed, dW_dtype, grad_table, 1, M, scratch, scratch_bytes,
+                                                  this->get_queue().abi()));
+    }
+    /// Width 128: forward pass that keeps the hidden activations only, and the backward pass on them.
+    void forward_rows(const void *x, void *hidden, void *y, const int y_cols, const size_t M) {
+        const tnn_mlp_desc d = desc();
+        tnn::abi_check(tnn_mlp_forward_rows(&d, this->prepared_forward(), x, hidden, y, y_cols, M, this->get_queue().abi()));
+    }
+    size_t backward_scratch_bytes(const size_t M) const {
+        const tnn_mlp_desc d = desc();
+        return tnn_mlp_backward_workspace_bytes(&d, M);
+    }
+    void backward_rows(const void *x, const void *hidden, const void *y, const void *dLdy, const float dy_scale, const float result_scale, void *dW_packed,
+                       const int dW_dtype, void *dLdx, const size_t M, void *scratch, const size_t scratch_bytes) {
+        const tnn_mlp_desc d = desc();
+        tnn::abi_check(tnn_mlp_backward_rows(&d, this->prepared_backward(), x, hidden, y, dLdy, dy_scale, result_scale, dW_packed, dW_dtype, dLdx, M,
+                                             scratch, scratch_bytes, this->get_queue().abi()));
     }
 
     Activation get_activation() const { return m_activation; }
@@ -270,6 +333,8 @@ template <typename T, int WIDTH> class SwiftNetMLP : public Network<T> {
     size_t m_ordered_rows = 0;
     tnn_grid_desc m_ordered_grid{};
 
+    /// Batches of this many points and more are visited in cell order.
+    static constexpr size_t OrderedFrom(const bool for_training) { return size_t(1) << (for_training ? 17 : 18); }
     bool OrderIsOf(const tnn_grid_desc &grid, const float *positions, const size_t M) const {
         return m_grid_order && m_ordered_positions == positions && m_ordered_rows == M && std::memcmp(&m_ordered_grid, &grid, sizeof(grid)) == 0;
     }

@@ -111,13 +111,19 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
         if (input.n() != this->get_input_width() || dL_doutput.n() != this->get_padded_output_width() || dL_doutput.m() != batch_size)
             throw std::invalid_argument("Dimension mismatch grid encoding backward_impl");
         check_max_level();
-        const size_t scratch = tnn_grid_backward_workspace_bytes(&m_desc, batch_size);
-        if (!m_scratch || m_scratch->size() * sizeof(float) < scratch)
-            m_scratch = std::make_unique<DeviceMatrix<float>>((scratch + sizeof(float) - 1) / sizeof(float), 1, this->get_queue());
+        const size_t need = backward_scratch_bytes(batch_size);
+        void *scratch = m_lent_scratch;
+        size_t scratch_bytes = m_lent_scratch_bytes;
+        if (scratch_bytes < need) {
+            if (!m_scratch || m_scratch->size() * sizeof(float) < need)
+                m_scratch = std::make_unique<DeviceMatrix<float>>((need + sizeof(float) - 1) / sizeof(float), 1, this->get_queue());
+            scratch = m_scratch->data();
+            scratch_bytes = m_scratch->size() * sizeof(float);
+        }
         tnn::abi_check(tnn_grid_backward_binned(&m_desc, input.GetPointer(), nullptr, dL_doutput.GetPointer(), TNN_FP32,
                                                 this->get_padded_output_width(), gradients->GetPointer(),
-                                                param_gradients_mode == GradientMode::Overwrite ? 1 : 0, batch_size, m_scratch->data(),
-                                                m_scratch->size() * sizeof(float), this->get_queue().abi()));
+                                                param_gradients_mode == GradientMode::Overwrite ? 1 : 0, batch_size, scratch, scratch_bytes,
+                                                this->get_queue().abi()));
     }
 
     uint32_t n_pos_dims() const override { return m_desc.n_dims; }
@@ -134,6 +140,12 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
     const GridOffsetTable &grid_offset_table() const override { return m_offset_table; }
     const tnn_grid_desc &descriptor() const { return m_desc; }
     uint32_t n_levels() const { return m_desc.n_levels; }
+    size_t backward_scratch_bytes(const size_t batch_size) const { return tnn_grid_backward_workspace_bytes(&m_desc, batch_size); }
+    /// Memory for the backward passes from now on, instead of their own; (nullptr, 0) takes it back.
+    void lend_scratch(void *scratch, const size_t bytes) {
+        m_lent_scratch = scratch;
+        m_lent_scratch_bytes = bytes;
+    }
 
   private:
     void check_max_level() const {
@@ -146,7 +158,9 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
 
     tnn_grid_desc m_desc;
     std::unique_ptr<DeviceMatrix<float>> m_order; // records of the last large batch in cell order
-    std::unique_ptr<DeviceMatrix<float>> m_scratch; // what the backward pass sorts its contributions into; only grows
+    std::unique_ptr<DeviceMatrix<float>> m_scratch; // what the backward pass sorts its contributions into, when none is lent; only grows
+    void *m_lent_scratch = nullptr;
+    size_t m_lent_scratch_bytes = 0;
     uint32_t m_n_features;
     uint32_t m_n_features_per_level;
     GridOffsetTable m_offset_table;

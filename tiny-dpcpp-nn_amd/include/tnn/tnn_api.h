@@ -75,6 +75,38 @@ class Module {
         throw std::runtime_error("backward_with_encoding: not a network module");
     }
 
+    // ---- a module as an operator on a caller's rows -----------------------------------------------------------------------
+    // What the reference's Python modules do around the two passes in operations of their own (padding, conversion, loss scale,
+    // packing and slicing, dpcpp_bindings/tiny_dpcpp_nn/modules.py:84-136,206-262) is part of the passes here. The autograd
+    // function over them lives with the Python bindings.
+    /// What a forward pass leaves for its backward pass.
+    struct RowsPass {
+        torch::Tensor input;          // what the kernels read: the caller's tensor, or the padded and converted copy of it
+        torch::Tensor hidden, output; // width 128: the hidden activations, and the output where its activation needs it
+        int64_t rows = 0, cols = 0;   // of the caller's input
+        c10::ScalarType dtype = torch::kFloat32;
+        bool in_workspace = false; // the activations are in the module's own workspace (forward_pass / backward_pass)
+    };
+    /// The input as forward_rows takes it: dense, of a type the kernels read, with no more columns than the module has.
+    virtual torch::Tensor input_rows(const torch::Tensor &x) const = 0;
+    /// Columns a caller sees of the output.
+    virtual int64_t visible_columns() const = 0;
+    /// keep: a backward pass may follow. training: only where a network keeps its activations in the module's workspace.
+    virtual torch::Tensor forward_rows(const torch::Tensor &x, bool keep, bool training, RowsPass &pass) = 0;
+    /// Gradients of the input (undefined unless wanted and available) and of the parameters, in the type and shape of `params`.
+    virtual std::tuple<torch::Tensor, torch::Tensor> backward_rows(const torch::Tensor &dy, const RowsPass &pass, double loss_scale, bool want_dx,
+                                                                   const torch::Tensor &params) = 0;
+    /// The parameter tensor as the Python modules hold it (a network's is packed) becomes the module's parameters.
+    virtual void push_params(const torch::Tensor &params) = 0;
+    /// Network modules behind a grid encoding: the same two passes on positions.
+    virtual torch::Tensor forward_rows_with_encoding(const Module &, const torch::Tensor &, bool) {
+        throw std::runtime_error("forward_rows_with_encoding: not a network module");
+    }
+    virtual std::tuple<torch::Tensor, torch::Tensor> backward_rows_with_encoding(const Module &, const torch::Tensor &, const torch::Tensor &, double, const torch::Tensor &,
+                                                                                 const torch::Tensor &) {
+        throw std::runtime_error("backward_rows_with_encoding: not a network module");
+    }
+
     tnn::queue &get_queue() { return queue_; }
 
     /// First thing in every method: the module's kernels go to the stream the caller's tensor operations are on, so inputs
@@ -131,6 +163,24 @@ class Module {
   protected:
     virtual void FreeWorkspace() = 0;
     virtual void AllocateWorkspace(const size_t batch_size) = 0;
+    torch::Tensor fresh(at::IntArrayRef sizes, c10::ScalarType dtype) const { return torch::empty(sizes, torch::TensorOptions().dtype(dtype).device(device())); }
+    /// Scratch memory of one call, from the pool the caller's tensors come from (stream-ordered, like the results).
+    torch::Tensor scratch(size_t bytes) const { return fresh({(int64_t)bytes}, torch::kUInt8); }
+    static int abi_dtype(c10::ScalarType t) {
+        switch (t) {
+        case torch::kFloat32: return TNN_FP32;
+        case c10::ScalarType::Half: return TNN_FP16;
+        case c10::ScalarType::BFloat16: return TNN_BF16;
+        default: return -1;
+        }
+    }
+    /// rows x cols of dtype: src's values times `scale`, padded (tnn_resize_rows) or cut.
+    torch::Tensor resized(const torch::Tensor &src, int64_t rows, int64_t cols, c10::ScalarType dtype, float fill, float scale) {
+        torch::Tensor dst = fresh({rows, cols}, dtype);
+        tnn::abi_check(tnn_resize_rows(abi_dtype(dtype), dst.data_ptr(), (int)cols, (size_t)rows, abi_dtype(src.scalar_type()), src.data_ptr(), (int)src.size(1),
+                                       (long long)src.stride(0), (long long)src.stride(1), (size_t)src.size(0), fill, scale, queue_.abi()));
+        return dst;
+    }
     c10::Device device() const { return c10::Device(c10::DeviceType::CUDA, device_index_); }
 
   private:
@@ -209,10 +259,32 @@ template <typename T> class EncodingModule : public Module {
         last_gradients_ = torch::empty({(int64_t)encoding_->get_n_params(), 1}, torch::TensorOptions().dtype(torch_type<T>::dtype).device(device()));
         DeviceMatrixView<T> gradients_view(encoding_->get_n_params(), 1, 1, reinterpret_cast<T *>(last_gradients_.data_ptr()));
         Context ctx;
+        auto *grid = dynamic_cast<tinydpcppnn::encodings::grid::GridEncodingTemplated<T> *>(encoding_.get());
+        torch::Tensor lent;
+        if (grid) {
+            lent = this->scratch(grid->backward_scratch_bytes((size_t)batch_size));
+            grid->lend_scratch(lent.data_ptr(), (size_t)lent.numel());
+        }
         encoding_->backward_impl(ctx, input_encoding_dmv, dL_doutput_dmv, &gradients_view);
+        if (grid) grid->lend_scratch(nullptr, 0);
         this->finish();
         return {torch::Tensor(), last_gradients_};
     }
+
+    torch::Tensor input_rows(const torch::Tensor &x) const override { return x.to(torch::kFloat32).contiguous(); }
+    int64_t visible_columns() const override { return encoding_->get_padded_output_width(); }
+    torch::Tensor forward_rows(const torch::Tensor &x, bool keep, bool, RowsPass &pass) override {
+        if (keep) pass.input = x;
+        return forward_pass(x);
+    }
+    std::tuple<torch::Tensor, torch::Tensor> backward_rows(const torch::Tensor &dy, const RowsPass &pass, double loss_scale, bool,
+                                                           const torch::Tensor &params) override {
+        if (encoding_->get_n_params() == 0) return {torch::Tensor(), torch::Tensor()};
+        torch::Tensor g = std::get<1>(backward_pass((loss_scale != 1.0 ? dy * loss_scale : dy).contiguous(), pass.input, false, false));
+        if (loss_scale != 1.0) g = g / loss_scale;
+        return {torch::Tensor(), g.reshape(params.sizes()).to(params.scalar_type())};
+    }
+    void push_params(const torch::Tensor &params) override { set_params(params.detach().to(torch_type<T>::dtype).contiguous(), false); }
 
     torch::Tensor initialize_params() override { return get_params(); }
     torch::Tensor initialize_params(const torch::Tensor &tensor) override {
@@ -295,7 +367,7 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
                          network_.get_output_width(), this->get_queue()),
           net_gradients_packed_(network_.get_n_hidden_layers() + 1, network_.get_network_width(), WIDTH, WIDTH, WIDTH, WIDTH,
                                 network_.get_output_width(), this->get_queue()),
-          max_batch_size_(0), interm_forw_ptr_(nullptr), interm_backw_ptr_(nullptr), dL_dinput_ptr_(nullptr) {
+          max_batch_size_(0), interm_forw_ptr_(nullptr), interm_backw_ptr_(nullptr), dL_dinput_ptr_(nullptr), pad_value_(use_bias ? 1.0f : 0.0f) {
         net_gradients_.fill(T(0.0f)).wait();
     }
 
@@ -451,6 +523,128 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
         return {GradientsTensor(pack_transpose_gradient), table_grad};
     }
 
+    torch::Tensor input_rows(const torch::Tensor &x) const override {
+        TORCH_CHECK(x.dim() == 2, "input must have two dimensions");
+        torch::Tensor in = x.size(1) > WIDTH ? x.narrow(1, 0, WIDTH) : x;
+        if (in.scalar_type() != kType && in.scalar_type() != torch::kFloat32) in = in.to(kType);
+        return in.contiguous();
+    }
+    int64_t visible_columns() const override { return network_.get_unpadded_output_width(); }
+
+    torch::Tensor forward_rows(const torch::Tensor &x, bool keep, bool training, RowsPass &pass) override {
+        this->enter();
+        CHECK_INPUT(x);
+        const int64_t rows = x.size(0), n_out = visible_columns();
+        pass.rows = rows;
+        pass.cols = x.size(1);
+        pass.dtype = x.scalar_type();
+        if (rows == 0) {
+            pass.input = x;
+            return fresh({0, n_out}, kType);
+        }
+        const bool whole = x.size(1) == WIDTH && x.scalar_type() == kType;
+        const bool recompute = keep && can_recompute_backward();
+        if (!keep || recompute) {
+            // a backward pass forms the activations again from the matrix this one reads
+            torch::Tensor in = x;
+            if (!whole && (keep || !network_.takes_narrow_rows((size_t)rows))) in = this->resized(x, rows, WIDTH, kType, pad_value_, 1.0f);
+            if (keep) pass.input = in;
+            torch::Tensor y = fresh({rows, n_out}, kType);
+            network_.inference_rows(in.data_ptr(), this->abi_dtype(in.scalar_type()), (int)in.size(1), y.data_ptr(), (int)n_out, (size_t)rows, pad_value_);
+            return y;
+        }
+        if constexpr (WIDTH == 128) {
+            pass.input = whole ? x : this->resized(x, rows, WIDTH, kType, pad_value_, 1.0f);
+            pass.hidden = fresh({network_.get_n_hidden_layers(), rows, WIDTH}, kType);
+            // the derivative of an output activation needs whole rows of the output
+            const bool need_output = network_.get_output_activation() != Activation::None;
+            const int64_t cols = need_output ? WIDTH : n_out;
+            torch::Tensor y = fresh({rows, cols}, kType);
+            network_.forward_rows(pass.input.data_ptr(), pass.hidden.data_ptr(), y.data_ptr(), (int)cols, (size_t)rows);
+            if (!need_output) return y;
+            pass.output = y;
+            return this->resized(y, rows, n_out, kType, 0.0f, 1.0f);
+        }
+        // deeper networks of the other widths keep their activations in the module's workspace, as forward_pass does
+        const int64_t padded = (rows + 7) / 8 * 8;
+        pass.in_workspace = true;
+        pass.input = (whole && padded == rows) ? x : this->resized(x, padded, WIDTH, kType, pad_value_, 1.0f);
+        torch::Tensor y = training ? forward_pass(pass.input) : inference(pass.input);
+        return (padded == rows && n_out == WIDTH) ? y : this->resized(y, rows, n_out, kType, 0.0f, 1.0f);
+    }
+
+    std::tuple<torch::Tensor, torch::Tensor> backward_rows(const torch::Tensor &dy, const RowsPass &pass, double loss_scale, bool want_dx,
+                                                           const torch::Tensor &params) override {
+        this->enter();
+        CHECK_GPU(dy);
+        const int64_t rows = pass.rows;
+        if (rows == 0) return {torch::zeros({0, pass.cols}, pass.input.options()), torch::zeros_like(params)};
+        TORCH_CHECK(dy.dim() == 2 && dy.size(0) == rows && dy.size(1) == visible_columns() && dy.scalar_type() == kType, "grad_output does not match the output");
+        const float up = (float)loss_scale, down = (float)(1.0 / loss_scale);
+        torch::Tensor dx;
+        if (pass.in_workspace) {
+            const torch::Tensor g = this->resized(dy, pass.input.size(0), WIDTH, kType, 0.0f, up);
+            torch::Tensor dW;
+            std::tie(dx, dW) = backward_pass(g, true, want_dx);
+            if (dx.defined()) dx = this->resized(dx.view({pass.input.size(0), WIDTH}).narrow(0, 0, rows).narrow(1, 0, pass.cols), rows, pass.cols, pass.dtype, 0.0f, down);
+            dW = dW.to(torch::kFloat32);
+            if (loss_scale != 1.0) dW.mul_(down);
+            return {dx, dW.reshape(params.sizes()).to(params.scalar_type())};
+        }
+        const bool direct = dy.is_contiguous() && (dy.size(1) == WIDTH || (dy.size(1) <= 16 && WIDTH < 128));
+        const torch::Tensor g = direct ? dy : this->resized(dy, rows, WIDTH, kType, 0.0f, 1.0f);
+        const c10::ScalarType dW_type = params.scalar_type() == kType ? kType : torch::kFloat32;
+        torch::Tensor dW = fresh(params.sizes(), dW_type);
+        if (want_dx) dx = fresh({rows, WIDTH}, kType);
+        void *const dx_ptr = want_dx ? dx.data_ptr() : nullptr;
+        if (WIDTH == 128) {
+            const torch::Tensor work = this->scratch(network_.backward_scratch_bytes((size_t)rows));
+            network_.backward_rows(pass.input.data_ptr(), pass.hidden.data_ptr(), pass.output.defined() ? pass.output.data_ptr() : nullptr, g.data_ptr(), up, down,
+                                   dW.data_ptr(), this->abi_dtype(dW_type), dx_ptr, (size_t)rows, work.data_ptr(), (size_t)work.numel());
+        } else {
+            const torch::Tensor work = this->scratch(network_.backward_recompute_scratch_bytes((size_t)rows));
+            network_.backward_recompute_rows(pass.input.data_ptr(), g.data_ptr(), (int)g.size(1), up, down, dW.data_ptr(), this->abi_dtype(dW_type), dx_ptr,
+                                             (size_t)rows, work.data_ptr(), (size_t)work.numel());
+        }
+        if (want_dx && (pass.cols != WIDTH || pass.dtype != kType)) dx = this->resized(dx.narrow(1, 0, pass.cols), rows, pass.cols, pass.dtype, 0.0f, 1.0f);
+        return {dx, dW_type == params.scalar_type() ? dW : dW.to(params.scalar_type())};
+    }
+
+    /// A network on the GPU converts fp32 / fp16 / bf16 to its own type in the kernel that copies; everything else is cast here.
+    void push_params(const torch::Tensor &params) override {
+        torch::Tensor p = params.detach();
+        if (!p.is_cuda() || this->abi_dtype(p.scalar_type()) < 0) p = p.to(kType);
+        set_params(p, true);
+    }
+
+    torch::Tensor forward_rows_with_encoding(const Module &encoding, const torch::Tensor &positions, bool keep) override {
+        this->enter();
+        const tnn_grid_desc *grid = CheckedPositions(encoding, positions);
+        const int64_t rows = positions.size(0), n_out = visible_columns();
+        torch::Tensor y = fresh({rows, n_out}, kType);
+        network_.inference_with_grid_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), (size_t)rows, y.data_ptr(), (int)n_out, keep);
+        return y;
+    }
+
+    std::tuple<torch::Tensor, torch::Tensor> backward_rows_with_encoding(const Module &encoding, const torch::Tensor &positions, const torch::Tensor &dy,
+                                                                         double loss_scale, const torch::Tensor &params, const torch::Tensor &table) override {
+        this->enter();
+        const tnn_grid_desc *grid = CheckedPositions(encoding, positions);
+        CHECK_GPU(dy);
+        const int64_t rows = positions.size(0);
+        TORCH_CHECK(dy.dim() == 2 && dy.size(0) == rows && dy.size(1) == visible_columns() && dy.scalar_type() == kType, "grad_output does not match the output");
+        const bool direct = dy.is_contiguous() && (dy.size(1) == WIDTH || dy.size(1) <= 16);
+        const torch::Tensor g = direct ? dy : this->resized(dy, rows, WIDTH, kType, 0.0f, 1.0f);
+        const c10::ScalarType dW_type = params.scalar_type() == kType ? kType : torch::kFloat32;
+        torch::Tensor dW = fresh(params.sizes(), dW_type), dtable = fresh(table.sizes(), torch::kFloat32);
+        const torch::Tensor work = this->scratch(network_.backward_with_grid_scratch_bytes(*grid, (size_t)rows));
+        // the caller's tensor is one autograd saved: it is as it was in the forward pass, and so is its cell order
+        network_.backward_with_grid_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), g.data_ptr(), (int)g.size(1), (float)loss_scale,
+                                         (float)(1.0 / loss_scale), dW.data_ptr(), this->abi_dtype(dW_type), dtable.data_ptr<float>(), (size_t)rows,
+                                         work.data_ptr(), (size_t)work.numel(), true);
+        return {dW_type == params.scalar_type() ? dW : dW.to(params.scalar_type()), dtable.to(table.scalar_type())};
+    }
+
     torch::Tensor initialize_params() override { return get_params(); }
     torch::Tensor get_params() override {
         this->enter();
@@ -519,6 +713,18 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
     }
 
   private:
+    static constexpr c10::ScalarType kType = torch_type<T>::dtype;
+
+    const tnn_grid_desc *CheckedPositions(const Module &encoding, const torch::Tensor &positions) const {
+        const tnn_grid_desc *grid = encoding.grid_descriptor();
+        if (!grid || !network_.supports_grid_input(*grid))
+            throw std::invalid_argument("this encoding / network pair runs as two modules (" + std::string(tnn_last_error()) + ")");
+        CHECK_INPUT(positions);
+        TORCH_CHECK(positions.dim() == 2 && positions.scalar_type() == torch::kFloat32, "positions must be a float32 matrix");
+        if (positions.sizes()[1] != (int64_t)grid->n_dims) throw std::runtime_error("Input tensor has incorrect dimensions");
+        return grid;
+    }
+
     size_t CheckedBatch(const torch::Tensor &input_tensor, const uint32_t width) const {
         CHECK_INPUT(input_tensor);
         TORCH_CHECK(input_tensor.dim() == 2, "input_tensor must have two dimensions");
@@ -568,6 +774,7 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
     T *interm_forw_ptr_;
     T *interm_backw_ptr_;
     T *dL_dinput_ptr_;
+    const float pad_value_; // of the input's columns beyond the caller's: the bias trick's ones, or zeros
 };
 
 } // namespace tnn

@@ -91,6 +91,17 @@ SIGNATURES = {
     "tnn_grid_mlp_backward": (c_int, [ctypes.POINTER(GridDesc), ctypes.POINTER(MlpDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                       c_void_p, c_int, c_void_p, c_int, c_size_t, c_void_p, c_size_t, c_void_p]),
     "tnn_mlp_set_packed_weights": (c_int, [ctypes.POINTER(MlpDesc), c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "tnn_resize_rows": (c_int, [c_int, c_void_p, c_int, c_size_t, c_int, c_void_p, c_int, ctypes.c_longlong, ctypes.c_longlong, c_size_t, c_float, c_float,
+                                c_void_p]),
+    "tnn_mlp_inference_rows": (c_int, [POINTER(MlpDesc), c_void_p, c_void_p, c_int, c_int, c_float, c_void_p, c_int, c_size_t, c_void_p]),
+    "tnn_grid_mlp_inference_rows": (c_int, [POINTER(GridDesc), POINTER(MlpDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_size_t, c_void_p]),
+    "tnn_mlp_backward_recompute_rows": (c_int, [POINTER(MlpDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_float, c_float, c_void_p, c_int,
+                                                c_void_p, c_size_t, c_void_p, c_size_t, c_void_p]),
+    "tnn_grid_mlp_backward_rows": (c_int, [POINTER(GridDesc), POINTER(MlpDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_float,
+                                           c_float, c_void_p, c_int, c_void_p, c_int, c_size_t, c_void_p, c_size_t, c_void_p]),
+    "tnn_mlp_forward_rows": (c_int, [POINTER(MlpDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_size_t, c_void_p]),
+    "tnn_mlp_backward_rows": (c_int, [POINTER(MlpDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_float, c_void_p, c_int, c_void_p,
+                                      c_size_t, c_void_p, c_size_t, c_void_p]),
     "tnn_probe_line_gather": (c_int, [c_void_p, c_size_t, c_size_t, c_int, ctypes.c_uint32, c_void_p, c_void_p]),
     "tnn_debug_set_meeting_spin_limit": (c_int, [c_int, ctypes.POINTER(c_int)]),
     "tnn_mlp_train_step_l2_static_max_bytes": (c_size_t, []),
