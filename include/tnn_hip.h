@@ -255,6 +255,11 @@ int tnn_resize_rows(int dst_dtype, void *d_dst, int dst_cols, size_t dst_rows, i
  * whole rows only (width 128 with many matrices or a large batch): tnn_resize_rows first. */
 int tnn_mlp_inference_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_x, int x_dtype, int x_cols, float fill,
                            void *d_y, int y_cols, size_t M, tnn_stream_t stream);
+/* tnn_mlp_set_packed_weights of fp32 parameters followed by tnn_mlp_inference_rows, in one launch where the network's weights fit
+ * LDS (widths up to 64): what a module does in every forward pass. */
+int tnn_mlp_push_inference_rows(const tnn_mlp_desc *desc, const float *d_src_packed, int unpadded_input_width, int unpadded_output_width,
+                                int use_bias, void *d_packed_T, void *d_packed_transposed_T, void *d_prepared_fwd, void *d_prepared_bwd,
+                                const void *d_x, int x_dtype, int x_cols, float fill, void *d_y, int y_cols, size_t M, tnn_stream_t stream);
 /* tnn_mlp_backward_recompute with dL/dy of dy_cols columns (at most 16, or the width; the others are zero) multiplied by
  * dy_scale as it is read, and results multiplied by result_scale: weight gradients in the packed parameter layout, rounded
  * to T and stored as dW_dtype (T or fp32), and dL/dx (M x width of T, or NULL). */
@@ -453,6 +458,11 @@ int tnn_grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, co
 /* tnn_grid_mlp_inference / _ordered (d_order given) with the first y_cols columns of the output in y (M x y_cols). */
 int tnn_grid_mlp_inference_rows(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,
                                 const void *d_prepared_fwd, void *d_y, int y_cols, size_t M, tnn_stream_t stream);
+/* The same with tnn_mlp_set_packed_weights of fp32 parameters in front, in one launch. */
+int tnn_grid_mlp_push_inference_rows(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_src_packed, int unpadded_input_width,
+                                     int unpadded_output_width, int use_bias, void *d_packed_T, void *d_packed_transposed_T,
+                                     void *d_prepared_fwd, void *d_prepared_bwd, const float *d_x, const void *d_order, const void *d_table,
+                                     void *d_y, int y_cols, size_t M, tnn_stream_t stream);
 /* tnn_grid_mlp_backward with dL/dy, scales and weight gradients as in tnn_mlp_backward_recompute_rows; the table's gradient is
  * multiplied by result_scale too. */
 int tnn_grid_mlp_backward_rows(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,

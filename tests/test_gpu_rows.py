@@ -95,3 +95,46 @@ def test_backward_rows(tnn, oracle, dtype, W, hidden, M, dy_cols):
     step = 2.0 ** (-8 if dtype == BF16 else -10)  # one rounding of a sum taken from values four times as large
     assert float((packed - ref).abs().max()) <= 2 * step * float(ref.abs().max())
     assert float((dx.float() - dX[:M].float()).norm()) <= step * float(dX.float().norm())
+
+
+@pytest.mark.parametrize("dtype", [BF16, FP16])
+@pytest.mark.parametrize("W,hidden,n_in,n_out,bias,M", [(16, 2, 16, 16, 0, 31), (32, 4, 5, 7, 1, 9001), (64, 4, 64, 64, 0, 70001), (64, 18, 3, 1, 1, 500), (64, 2, 40, 16, 1, 2 ** 18),
+                                                        (128, 2, 100, 128, 0, 3000)])
+def test_push_and_inference_in_one_launch(tnn, dtype, W, hidden, n_in, n_out, bias, M):
+    """The copies that a push leaves and the pass on them, bit for bit those of the two calls: few workgroups (others write the copies), many
+    (those that compute do), depths whose weights do not fit LDS, padding weights."""
+    from tiny_dpcpp_nn import _lib
+    desc = tnn.mlp_desc(dtype, W, hidden, "relu", "none")
+    n = (hidden + 1) * W * W
+    nb = tnn.lib.tnn_mlp_prepared_bytes(ctypes.byref(desc)) // 2
+    params = torch.randn(n, device=tnn.dev) * W ** -0.5
+    sizes = (n, n, nb, nb)
+    one, two = ([torch.full((k,), 7.0, dtype=DT[dtype], device=tnn.dev) for k in sizes] for _ in range(2))
+    x = torch.rand((M, n_in), device=tnn.dev)
+    if W == 128:
+        x = torch.nn.functional.pad(x, [0, W - n_in], value=float(bias)).to(DT[dtype])
+    xd, xc = (FP32, n_in) if W < 128 else (dtype, W)
+    y1, y2 = (torch.empty((M, n_out), dtype=DT[dtype], device=tnn.dev) for _ in range(2))
+    _lib.check(tnn.lib.tnn_mlp_push_inference_rows(ctypes.byref(desc), p(params), n_in, n_out, bias, *[p(t) for t in one], p(x), xd, xc, float(bias), p(y1), n_out, M,
+                                                   tnn.stream()))
+    _lib.check(tnn.lib.tnn_mlp_set_packed_weights(ctypes.byref(desc), p(params), FP32, n_in, n_out, bias, *[p(t) for t in two], tnn.stream()))
+    _lib.check(tnn.lib.tnn_mlp_inference_rows(ctypes.byref(desc), p(two[2]), p(x), xd, xc, float(bias), p(y2), n_out, M, tnn.stream()))
+    for a, b in zip(one + [y1], two + [y2]):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("M", [40, 20000])
+def test_grid_push_and_inference_in_one_launch(tnn, M):
+    from tiny_dpcpp_nn import _lib
+    d = tnn.grid_desc(dict(n_dims=2, n_levels=16, n_features_per_level=2, log2_hashmap_size=12, base_resolution=16, per_level_scale=1.5))
+    desc = tnn.mlp_desc(BF16, 64, 2, "relu", "none")
+    n, nb = 3 * 64 * 64, tnn.lib.tnn_mlp_prepared_bytes(ctypes.byref(desc)) // 2
+    params, table, x = torch.randn(n, device=tnn.dev) * 0.1, torch.randn(tnn.grid_n_params(d), device=tnn.dev), torch.rand((M, 2), device=tnn.dev)
+    one, two = ([torch.full((k,), 7.0, dtype=torch.bfloat16, device=tnn.dev) for k in (n, n, nb, nb)] for _ in range(2))
+    y1, y2 = (torch.empty((M, 3), dtype=torch.bfloat16, device=tnn.dev) for _ in range(2))
+    g, m = ctypes.byref(d), ctypes.byref(desc)
+    _lib.check(tnn.lib.tnn_grid_mlp_push_inference_rows(g, m, p(params), 64, 3, 0, *[p(t) for t in one], p(x), None, p(table), p(y1), 3, M, tnn.stream()))
+    _lib.check(tnn.lib.tnn_mlp_set_packed_weights(m, p(params), FP32, 64, 3, 0, *[p(t) for t in two], tnn.stream()))
+    _lib.check(tnn.lib.tnn_grid_mlp_inference_rows(g, m, p(x), None, p(table), p(two[2]), p(y2), 3, M, tnn.stream()))
+    for a, b in zip(one + [y1], two + [y2]):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))

@@ -73,14 +73,13 @@ struct EncodedNetworkBackward : public torch::autograd::Node {
 /// y = module(x), recorded for autograd when that is on and anything asks for gradients.
 inline torch::Tensor call(const std::shared_ptr<tnn::Module> &module, const torch::Tensor &x, const torch::Tensor &params, bool push, bool training,
                           double loss_scale) {
-    if (push && module->n_params()) module->push_params(params);
     const torch::Tensor in = module->input_rows(x); // (PyTorch operations where any are needed: autograd sees them)
     const bool record = torch::autograd::compute_requires_grad(in, params);
     tnn::Module::RowsPass pass;
     torch::Tensor y;
     {
         const torch::AutoGradMode no_grad(false);
-        y = module->forward_rows(in, record, training, pass);
+        y = module->forward_rows(in, push && module->n_params() ? params : torch::Tensor(), record, training, pass);
     }
     if (!record) return y;
     auto node = std::shared_ptr<ModuleBackward>(new ModuleBackward(), torch::autograd::deleteNode);
@@ -99,13 +98,12 @@ inline torch::Tensor call(const std::shared_ptr<tnn::Module> &module, const torc
 inline torch::Tensor call_with_encoding(const std::shared_ptr<tnn::Module> &network, const std::shared_ptr<tnn::Module> &encoding, const torch::Tensor &x,
                                         const torch::Tensor &params, const torch::Tensor &table, bool push_network, bool push_table, double loss_scale) {
     if (push_table) encoding->push_params(table);
-    if (push_network) network->push_params(params);
     const torch::Tensor positions = x.detach().to(torch::kFloat32).contiguous();
     const bool record = torch::autograd::compute_requires_grad(params, table);
     torch::Tensor y;
     {
         const torch::AutoGradMode no_grad(false);
-        y = network->forward_rows_with_encoding(*encoding, positions, record);
+        y = network->forward_rows_with_encoding(*encoding, positions, push_network ? params : torch::Tensor(), record);
     }
     if (!record) return y;
     auto node = std::shared_ptr<EncodedNetworkBackward>(new EncodedNetworkBackward(), torch::autograd::deleteNode);

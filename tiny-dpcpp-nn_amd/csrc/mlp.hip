@@ -69,7 +69,8 @@ __global__ void prepare_weights_kernel(const SRC *__restrict__ packed, T *__rest
 template <typename T, int W, int ACT, bool STORE_INTERM, bool W_IN_LDS, int THREADS, int STAGED = 0, bool NARROW = false>
 __global__ void __launch_bounds__(THREADS, (THREADS >= 512 && W <= 64) ? 4 : 1)
     mlp_forward_kernel(const typename Storage<T>::vec8 *__restrict__ wprep, const T *__restrict__ x, T *__restrict__ out,
-                       int n_mats, int out_act, long long M, T *__restrict__ y, int y_cols, int store_input, int x_cols, int x_fp32, float fill) {
+                       int n_mats, int out_act, long long M, T *__restrict__ y, int y_cols, int store_input, int x_cols, int x_fp32, float fill,
+                       const WeightPush push) {
     typedef Tile<T, W> TL;
     typedef typename Storage<T>::vec8 vec8;
     constexpr int NK = TL::NK, NI = TL::NI;
@@ -79,7 +80,11 @@ __global__ void __launch_bounds__(THREADS, (THREADS >= 512 && W <= 64) ? 4 : 1)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int j = lane & 31, h = lane >> 5;
     const long long n_tiles = (M + 31) / 32;
-    const long long stride = (long long)gridDim.x * (blockDim.x >> 6);
+    if (!STORE_INTERM && (int)blockIdx.x >= push.blocks) { // (only with a push: a workgroup beside those that compute)
+        push_copies<T, W>(push, n_mats);
+        return;
+    }
+    const long long stride = (long long)push.blocks * (blockDim.x >> 6);
     long long tile = (long long)blockIdx.x * (blockDim.x >> 6) + wave;
     unsigned char *my_stage = smem_raw + (size_t)n_mats * (TL::NF * kWaveSize * sizeof(vec8)) + (size_t)wave * TL::TILE_BYTES;
     unsigned int st_off[NK];
@@ -107,23 +112,45 @@ __global__ void __launch_bounds__(THREADS, (THREADS >= 512 && W <= 64) ? 4 : 1)
         // tile and nothing else overlaps its loads; 1-4 % at 2^18 and 2^20 rows).
         constexpr int per_mat = NI * NK * kWaveSize;
         const int n = n_mats * per_mat;
-        constexpr int HELD = 4;
-        vec8 held[HELD];
-#pragma unroll
-        for (int i = 0; i < HELD; ++i) {
-            const int f = threadIdx.x + i * THREADS;
-            held[i] = wprep[f < n ? f : n - 1];
-        }
-        asm volatile("" ::: "memory");
         const bool early = (wave & 1) == 0;
-        if (early && tile < n_tiles) load_tile(cur, tile * 32 + j);
-        asm volatile("" ::: "memory");
+        if (!STORE_INTERM && push.master) {
+            constexpr int HELD = 2;
+            PushedFragment<T, W> held[HELD];
 #pragma unroll
-        for (int i = 0; i < HELD; ++i) {
-            const int f = threadIdx.x + i * THREADS;
-            if (f < n) lds_w[f] = held[i];
+            for (int i = 0; i < HELD; ++i) {
+                const int f = threadIdx.x + i * THREADS;
+                held[i].request(push, f < n ? f : n - 1);
+            }
+            asm volatile("" ::: "memory");
+            if (early && tile < n_tiles) load_tile(cur, tile * 32 + j);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int i = 0; i < HELD; ++i) {
+                const int f = threadIdx.x + i * THREADS;
+                if (f < n) lds_w[f] = held[i].convert(push, f, n_mats);
+            }
+            for (int f = threadIdx.x + HELD * THREADS; f < n; f += THREADS) {
+                held[0].request(push, f);
+                lds_w[f] = held[0].convert(push, f, n_mats);
+            }
+        } else {
+            constexpr int HELD = 4;
+            vec8 held[HELD];
+#pragma unroll
+            for (int i = 0; i < HELD; ++i) {
+                const int f = threadIdx.x + i * THREADS;
+                held[i] = wprep[f < n ? f : n - 1];
+            }
+            asm volatile("" ::: "memory");
+            if (early && tile < n_tiles) load_tile(cur, tile * 32 + j);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int i = 0; i < HELD; ++i) {
+                const int f = threadIdx.x + i * THREADS;
+                if (f < n) lds_w[f] = held[i];
+            }
+            for (int f = threadIdx.x + HELD * THREADS; f < n; f += THREADS) lds_w[f] = wprep[f];
         }
-        for (int f = threadIdx.x + HELD * THREADS; f < n; f += THREADS) lds_w[f] = wprep[f];
         __syncthreads();
         if (!early && tile < n_tiles) load_tile(cur, tile * 32 + j);
     } else {
@@ -140,6 +167,7 @@ __global__ void __launch_bounds__(THREADS, (THREADS >= 512 && W <= 64) ? 4 : 1)
         for (int kb = 0; kb < NK; ++kb) asm volatile("" : "+v"(cur[kb]));
     };
     settle();
+    if (!STORE_INTERM && push.master) push_copies<T, W>(push, n_mats);
 
     while (tile < n_tiles) {
         const long long row = tile * 32 + j;
@@ -491,6 +519,7 @@ struct ForwardRows {
     int y_cols = 0;    // 0: all
     int x_cols = 0, x_fp32 = 0;
     float fill = 0.0f;
+    WeightPush push{}; // inference with weights that fit LDS only
 };
 
 template <typename T, int W, int ACT, bool STORE_INTERM, int THREADS>
@@ -551,8 +580,10 @@ static int launch_forward_v(const tnn_mlp_desc *d, const void *wprep, const void
         if (io.x_cols) k = in_lds ? mlp_forward_kernel<T, W, ACT, false, true, 512, 0, true> : mlp_forward_kernel<T, W, ACT, false, false, 512, 0, true>;
     }
     if (!reserve_lds(reinterpret_cast<const void *>(k), lds)) return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", lds);
-    TNN_LAUNCH(k, dim3((unsigned)blocks), dim3(THREADS), lds, s, (const vec8 *)wprep, (const T *)x, (T *)out, n_mats, d->output_activation, (long long)M, y,
-               y_cols, io.store_input ? 1 : 0, io.x_cols, io.x_fp32, io.fill);
+    WeightPush push = io.push;
+    const int grid = push_grid(&push, (int)blocks, THREADS, prepared_elems(d));
+    TNN_LAUNCH(k, dim3((unsigned)grid), dim3(THREADS), lds, s, (const vec8 *)wprep, (const T *)x, (T *)out, n_mats, d->output_activation, (long long)M, y,
+               y_cols, io.store_input ? 1 : 0, io.x_cols, io.x_fp32, io.fill, push);
     return check_launch("mlp_forward_kernel");
 }
 
@@ -797,31 +828,30 @@ static int check_batch(size_t M) {
 template <typename T, typename SRC>
 __global__ void set_packed_weights_kernel(const SRC *__restrict__ src, T *__restrict__ packed, T *__restrict__ packed_t, T *__restrict__ fwd,
                                           T *__restrict__ bwd, int W, int n_mats, int live_in, int live_out) {
-    const int NI = (W + 31) / 32, NK = W / 16;
-    const int per_mat = NI * NK * 512;
-    const int total = n_mats * per_mat;
-    for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {
-        const int l = idx / per_mat;
-        int r = idx % per_mat;
-        const int t = r & 7;
-        const int lane = (r >> 3) & 63;
-        r >>= 9;
-        const int kb = r % NK, a = r / NK;
-        const int h = lane >> 5, i = lane & 31;
-        const int outer = 32 * a + swap23(i), inner = 16 * kb + 8 * h + t;
-        T vf = (T)0.0f, vb = (T)0.0f;
-        if (outer < W) {
-            const size_t m = (size_t)l * W * W;
-            // rows of the first matrix from live_in on and columns of the last matrix from live_out on only see padding
-            auto weight = [&](int k, int n) { return ((l == 0 && k >= live_in) || (l == n_mats - 1 && n >= live_out)) ? (T)0.0f : (T)(float)src[m + packed_coord(k, n, W)]; };
-            vf = weight(inner, outer);
-            vb = weight(outer, inner);
-            packed[m + packed_coord(inner, outer, W)] = vf;
-            packed_t[m + packed_coord(outer, inner, W)] = vf; // element (k, n) of W is element (n, k) of its transpose
-        }
-        fwd[idx] = vf;
-        bwd[idx] = vb;
-    }
+    const int total = n_mats * ((W + 31) / 32) * (W / 16) * 512;
+    WeightPush p;
+    p.live_in = live_in;
+    p.live_out = live_out;
+    for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x)
+        write_weight_copies<T>(idx, src, packed, packed_t, fwd, bwd, W, [&](float v, int l, int k, int n) { return pushed_weight<T>(p, v, l, k, n, n_mats); });
+}
+
+// The arguments of tnn_mlp_set_packed_weights, checked.
+int make_weight_push(const tnn_mlp_desc *desc, const void *src, int unpadded_input_width, int unpadded_output_width, int use_bias, void *packed, void *packed_t,
+                     void *fwd, void *bwd, WeightPush *p) {
+    if (!src || !packed || !packed_t || !fwd || !bwd) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    if (src == packed || src == packed_t) return fail(TNN_ERR_INVALID_ARGUMENT, "the source must not be one of the destinations");
+    const int W = desc->width;
+    if (unpadded_input_width > W || unpadded_output_width > W || unpadded_input_width <= 0 || unpadded_output_width <= 0)
+        return fail(TNN_ERR_INVALID_ARGUMENT, "Padded weights width cannot be less than the unpadded.");
+    // include/network/Network.h:191-202: with the bias trick the ones reach up to the next multiple of 16, and an input width
+    // that already is one leaves the whole padded width live
+    const int live_in = !use_bias ? unpadded_input_width : (unpadded_input_width % 16 == 0 ? W : (unpadded_input_width / 16 + 1) * 16);
+    if (live_in > W) return fail(TNN_ERR_INVALID_ARGUMENT, "one_padded_input_width > padded_input_width, the input width is too small.");
+    p->master = static_cast<const float *>(src);
+    p->packed = packed, p->packed_t = packed_t, p->fwd = fwd, p->bwd = bwd;
+    p->live_in = live_in, p->live_out = unpadded_output_width;
+    return TNN_OK;
 }
 
 } // namespace tnn
@@ -833,23 +863,18 @@ TNN_API int tnn_mlp_set_packed_weights(const tnn_mlp_desc *desc, const void *d_s
                                        void *d_prepared_fwd, void *d_prepared_bwd, tnn_stream_t stream) {
     int rc = check_mlp_desc(desc);
     if (rc) return rc;
-    if (!d_src_packed || !d_packed_T || !d_packed_transposed_T || !d_prepared_fwd || !d_prepared_bwd)
-        return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
-    if (d_src_packed == d_packed_T || d_src_packed == d_packed_transposed_T) return fail(TNN_ERR_INVALID_ARGUMENT, "the source must not be one of the destinations");
+    WeightPush push;
+    if ((rc = make_weight_push(desc, d_src_packed, unpadded_input_width, unpadded_output_width, use_bias, d_packed_T, d_packed_transposed_T, d_prepared_fwd,
+                               d_prepared_bwd, &push)))
+        return rc;
     const int W = desc->width;
-    if (unpadded_input_width > W || unpadded_output_width > W || unpadded_input_width <= 0 || unpadded_output_width <= 0)
-        return fail(TNN_ERR_INVALID_ARGUMENT, "Padded weights width cannot be less than the unpadded.");
-    // include/network/Network.h:191-202: with the bias trick the ones reach up to the next multiple of 16, and an input width
-    // that already is one leaves the whole padded width live
-    const int live_in = !use_bias ? unpadded_input_width : (unpadded_input_width % 16 == 0 ? W : (unpadded_input_width / 16 + 1) * 16);
-    if (live_in > W) return fail(TNN_ERR_INVALID_ARGUMENT, "one_padded_input_width > padded_input_width, the input width is too small.");
     const int n_mats = desc->n_hidden_layers + 1;
     const int total = (int)prepared_elems(desc);
     const int blocks = (total + 255) / 256;
     hipStream_t s = as_stream(stream);
 #define TNN_SPW(T_, S_)                                                                                                                          \
     TNN_LAUNCH((set_packed_weights_kernel<T_, S_>), dim3(blocks), dim3(256), 0, s, (const S_ *)d_src_packed, (T_ *)d_packed_T, (T_ *)d_packed_transposed_T, \
-               (T_ *)d_prepared_fwd, (T_ *)d_prepared_bwd, W, n_mats, live_in, unpadded_output_width)
+               (T_ *)d_prepared_fwd, (T_ *)d_prepared_bwd, W, n_mats, push.live_in, push.live_out)
     if (desc->dtype == TNN_BF16) {
         if (src_dtype == TNN_FP32) TNN_SPW(bf16_t, float);
         else if (src_dtype == TNN_BF16) TNN_SPW(bf16_t, bf16_t);
@@ -919,10 +944,9 @@ TNN_API int tnn_mlp_forward(const tnn_mlp_desc *desc, const void *d_prepared_fwd
     return rc;
 }
 
-TNN_API int tnn_mlp_inference_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_x, int x_dtype, int x_cols, float fill, void *d_y,
-                                   int y_cols, size_t M, tnn_stream_t stream) {
-    int rc = check_mlp_desc(desc);
-    if (rc) return rc;
+static int inference_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_x, int x_dtype, int x_cols, float fill, void *d_y, int y_cols,
+                          size_t M, const WeightPush &push, tnn_stream_t stream) {
+    int rc = TNN_OK;
     if (M == 0) return fail(TNN_ERR_INVALID_ARGUMENT, "empty batch");
     if (!d_prepared_fwd || !d_x || !d_y) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
     if (x_cols < 1 || x_cols > desc->width || y_cols < 1 || y_cols > desc->width)
@@ -930,6 +954,7 @@ TNN_API int tnn_mlp_inference_rows(const tnn_mlp_desc *desc, const void *d_prepa
     if (x_dtype != desc->dtype && x_dtype != TNN_FP32) return fail(TNN_ERR_UNSUPPORTED, "x of dtype %d", x_dtype);
     ForwardRows io;
     io.y_cols = y_cols;
+    io.push = push;
     if (x_cols != desc->width || x_dtype != desc->dtype) {
         io.x_cols = x_cols;
         io.x_fp32 = x_dtype == TNN_FP32;
@@ -939,6 +964,31 @@ TNN_API int tnn_mlp_inference_rows(const tnn_mlp_desc *desc, const void *d_prepa
     }
     TNN_DISPATCH_TW(desc, rc = (launch_forward<T_, W_, false>(desc, d_prepared_fwd, d_x, d_y, M, as_stream(stream), io)));
     return rc;
+}
+
+TNN_API int tnn_mlp_inference_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_x, int x_dtype, int x_cols, float fill, void *d_y,
+                                   int y_cols, size_t M, tnn_stream_t stream) {
+    const int rc = check_mlp_desc(desc);
+    return rc ? rc : inference_rows(desc, d_prepared_fwd, d_x, x_dtype, x_cols, fill, d_y, y_cols, M, WeightPush{}, stream);
+}
+
+TNN_API int tnn_mlp_push_inference_rows(const tnn_mlp_desc *desc, const float *d_src_packed, int unpadded_input_width, int unpadded_output_width, int use_bias,
+                                        void *d_packed_T, void *d_packed_transposed_T, void *d_prepared_fwd, void *d_prepared_bwd, const void *d_x, int x_dtype,
+                                        int x_cols, float fill, void *d_y, int y_cols, size_t M, tnn_stream_t stream) {
+    int rc = check_mlp_desc(desc);
+    if (rc) return rc;
+    WeightPush push;
+    if ((rc = make_weight_push(desc, d_src_packed, unpadded_input_width, unpadded_output_width, use_bias, d_packed_T, d_packed_transposed_T, d_prepared_fwd,
+                               d_prepared_bwd, &push)))
+        return rc;
+    // (width 128 passes its matrices through LDS round after round, and matrices that do not fit LDS are read where they are)
+    if (desc->width == 128 || prepared_elems(desc) * 2 > kLdsBudget || (reinterpret_cast<uintptr_t>(d_src_packed) & 7)) {
+        if ((rc = tnn_mlp_set_packed_weights(desc, d_src_packed, TNN_FP32, unpadded_input_width, unpadded_output_width, use_bias, d_packed_T,
+                                             d_packed_transposed_T, d_prepared_fwd, d_prepared_bwd, stream)))
+            return rc;
+        push = WeightPush{};
+    }
+    return inference_rows(desc, d_prepared_fwd, d_x, x_dtype, x_cols, fill, d_y, y_cols, M, push, stream);
 }
 
 TNN_API int tnn_mlp_forward_rows(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_x, void *d_hidden, void *d_y, int y_cols, size_t M,

@@ -321,6 +321,103 @@ template <typename T, int W> struct Tile {
     }
 };
 
+// A forward pass that takes the parameters where the optimiser left them (fp32, packed layout) instead of prepared operands,
+// and leaves everything tnn_mlp_set_packed_weights derives from them behind: the launch of its own that the push was took 2.5 to
+// 5 us in front of every forward pass. Every workgroup that computes stages its weights from the parameters (twice the bytes
+// of the prepared operands, out of L2); the copies are written by workgroups [first, ...), which are those that compute when
+// there are enough of them, and additional ones behind them otherwise (a small batch occupies few CUs).
+struct WeightPush {
+    const float *master = nullptr; // null: no push, the kernel reads prepared operands
+    void *packed = nullptr, *packed_t = nullptr, *fwd = nullptr, *bwd = nullptr;
+    int live_in = 0, live_out = 0; // rows of the first matrix / columns of the last one from here on only see padding
+    int blocks = 0;                // workgroups that compute
+    int first = 0;                 // first workgroup that writes copies
+};
+
+// A weight of matrix l as set_packed_weights takes it.
+template <typename T> __device__ __forceinline__ T pushed_weight(const WeightPush &p, float v, int l, int k, int n, int n_mats) {
+    return ((l == 0 && k >= p.live_in) || (l == n_mats - 1 && n >= p.live_out)) ? (T)0.0f : (T)v;
+}
+
+// One forward operand fragment (8 values of T): f counts fragments over all matrices and lanes.
+template <typename T, int W> struct PushedFragment {
+    f32x2 raw[4];
+    __device__ __forceinline__ void request(const WeightPush &p, int f) {
+        constexpr int NK = W / 16, per_mat = ((W + 31) / 32) * NK * kWaveSize;
+        const int l = f / per_mat, r = f % per_mat, lane = r & 63;
+        const int outer = 32 * ((r >> 6) / NK) + swap23(lane & 31), k0 = 16 * ((r >> 6) % NK) + 8 * (lane >> 5);
+        const float *src = p.master + (size_t)l * W * W + 2 * (outer < W ? outer : 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) raw[q] = *reinterpret_cast<const f32x2 *>(src + (k0 + 2 * q) * W); // rows k0 + 2 q and the next, side by side
+    }
+    __device__ __forceinline__ typename Storage<T>::vec8 convert(const WeightPush &p, int f, int n_mats) const {
+        constexpr int NK = W / 16, per_mat = ((W + 31) / 32) * NK * kWaveSize;
+        const int l = f / per_mat, r = f % per_mat, lane = r & 63;
+        const int outer = 32 * ((r >> 6) / NK) + swap23(lane & 31), k0 = 16 * ((r >> 6) % NK) + 8 * (lane >> 5);
+        typename Storage<T>::vec8 v = {};
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+            if (outer < W) v[t] = pushed_weight<T>(p, raw[t >> 1][t & 1], l, k0 + t, outer, n_mats);
+        return v;
+    }
+};
+
+// One slot of the operand-order index space of all matrices (it covers every matrix element once, plus the empty half-tile
+// at width 16): the element's place in the packed copy, its transpose and both operand orders.
+template <typename T, typename SRC, typename WEIGHT>
+__device__ __forceinline__ void write_weight_copies(int idx, const SRC *__restrict__ src, T *__restrict__ packed, T *__restrict__ packed_t, T *__restrict__ fwd,
+                                                    T *__restrict__ bwd, int W, WEIGHT weight) {
+    const int NI = (W + 31) / 32, NK = W / 16;
+    const int per_mat = NI * NK * 512;
+    const int l = idx / per_mat;
+    int r = idx % per_mat;
+    const int t = r & 7;
+    const int lane = (r >> 3) & 63;
+    r >>= 9;
+    const int kb = r % NK, a = r / NK;
+    const int h = lane >> 5, i = lane & 31;
+    const int outer = 32 * a + swap23(i), inner = 16 * kb + 8 * h + t;
+    T vf = (T)0.0f, vb = (T)0.0f;
+    if (outer < W) {
+        const size_t m = (size_t)l * W * W;
+        vf = weight((float)src[m + packed_coord(inner, outer, W)], l, inner, outer);
+        vb = weight((float)src[m + packed_coord(outer, inner, W)], l, outer, inner);
+        packed[m + packed_coord(inner, outer, W)] = vf;
+        packed_t[m + packed_coord(outer, inner, W)] = vf; // element (k, n) of W is element (n, k) of its transpose
+    }
+    fwd[idx] = vf;
+    bwd[idx] = vb;
+}
+
+template <typename T, int W> __device__ __forceinline__ void push_copies(const WeightPush &p, int n_mats) {
+    if ((int)blockIdx.x < p.first) return;
+    const int total = n_mats * ((W + 31) / 32) * (W / 16) * 512, step = ((int)gridDim.x - p.first) * (int)blockDim.x;
+    for (int idx = ((int)blockIdx.x - p.first) * (int)blockDim.x + (int)threadIdx.x; idx < total; idx += step)
+        write_weight_copies<T>(idx, p.master, static_cast<T *>(p.packed), static_cast<T *>(p.packed_t), static_cast<T *>(p.fwd), static_cast<T *>(p.bwd), W,
+                               [&](float v, int l, int k, int n) { return pushed_weight<T>(p, v, l, k, n, n_mats); });
+}
+
+// Weights of the forward pass into LDS, from prepared operands or from the parameters.
+template <typename T, int W>
+__device__ __forceinline__ void stage_weights(typename Storage<T>::vec8 *lds_w, const typename Storage<T>::vec8 *__restrict__ glb_w, int n_mats,
+                                              const WeightPush &p) {
+    constexpr int per_mat = Tile<T, W>::NI * Tile<T, W>::NK * kWaveSize;
+    const int n = n_mats * per_mat;
+    if (!p.master) {
+        for (int f = threadIdx.x; f < n; f += blockDim.x) lds_w[f] = glb_w[f];
+    } else {
+        for (int f = threadIdx.x; f < n; f += 2 * blockDim.x) {
+            const int g = f + (int)blockDim.x < n ? f + (int)blockDim.x : f;
+            PushedFragment<T, W> a, b;
+            a.request(p, f);
+            b.request(p, g);
+            lds_w[f] = a.convert(p, f, n_mats);
+            lds_w[g] = b.convert(p, g, n_mats);
+        }
+    }
+    __syncthreads();
+}
+
 template <typename T, int W>
 __device__ __forceinline__ void stage_weights(typename Storage<T>::vec8 *lds_w,
                                               const typename Storage<T>::vec8 *__restrict__ glb_w, int n_mats) {
@@ -337,6 +434,14 @@ struct DeviceInfo {
     bool ok = false;
 };
 const DeviceInfo &device_info();
+
+// The grid of a forward pass with a push and the rest of its plan; `blocks` workgroups compute.
+inline int push_grid(WeightPush *p, int blocks, int threads, size_t prepared_elements) {
+    p->blocks = blocks;
+    if (!p->master) return blocks;
+    p->first = blocks >= 64 ? 0 : blocks;
+    return blocks >= 64 ? blocks : blocks + (int)((prepared_elements + threads - 1) / threads);
+}
 
 inline size_t prepared_elems(const tnn_mlp_desc *d) {
     const int W = d->width, NI = (W + 31) / 32, NK = W / 16;

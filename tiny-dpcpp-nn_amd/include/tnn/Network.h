@@ -134,6 +134,14 @@ template <typename T> class Network : public NetworkBase<T> {
     virtual uint32_t get_unpadded_input_width() const { return shape_.raw_in; }
 
   protected:
+    // Where a push of the parameters writes, for the calls that push and run a pass in one launch.
+    int unpadded_in() const { return (int)shape_.raw_in; }
+    int unpadded_out() const { return (int)shape_.raw_out; }
+    int bias_flag() const { return shape_.bias ? 1 : 0; }
+    T *packed_weights() { return m_weights_matrices.data(); }
+    T *packed_weights_transposed() { return m_weightsT_matrices.data(); }
+    void *prepared_forward_storage() { return prepared_fwd_; }
+    void *prepared_backward_storage() { return prepared_bwd_; }
     // Operand-order copies of the weights for the forward and the backward kernels.
     const void *prepared_forward() const { return prepared_fwd_; }
     const void *prepared_backward() const { return prepared_bwd_; }

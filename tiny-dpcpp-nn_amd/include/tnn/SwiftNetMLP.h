@@ -167,17 +167,31 @@ template <typename T, int WIDTH> class SwiftNetMLP : public Network<T> {
     bool takes_narrow_rows(const size_t M) const {
         return WIDTH < 128 || (M < 65536 && this->get_n_hidden_layers() + 1 <= 4);
     }
-    void inference_rows(const void *x, const int x_dtype, const int x_cols, void *y, const int y_cols, const size_t M, const float fill) {
+    /// With `params` (fp32, packed, on the device): set_weights_matrices_from_device(params, true) first, in the same launch.
+    void inference_rows(const void *x, const int x_dtype, const int x_cols, void *y, const int y_cols, const size_t M, const float fill,
+                        const float *params = nullptr) {
         const tnn_mlp_desc d = desc();
+        if (params) {
+            tnn::abi_check(tnn_mlp_push_inference_rows(&d, params, this->unpadded_in(), this->unpadded_out(), this->bias_flag(), this->packed_weights(),
+                                                       this->packed_weights_transposed(), this->prepared_forward_storage(), this->prepared_backward_storage(),
+                                                       x, x_dtype, x_cols, fill, y, y_cols, M, this->get_queue().abi()));
+            return;
+        }
         tnn::abi_check(tnn_mlp_inference_rows(&d, this->prepared_forward(), x, x_dtype, x_cols, fill, y, y_cols, M, this->get_queue().abi()));
     }
     void inference_with_grid_rows(const tnn_grid_desc &grid, const void *table, const float *positions, const size_t M, void *y, const int y_cols,
-                                  const bool a_backward_pass_follows) {
+                                  const bool a_backward_pass_follows, const float *params = nullptr) {
         const tnn_mlp_desc d = desc();
         const void *order = nullptr;
         if (M >= OrderedFrom(a_backward_pass_follows)) {
             OrderPoints(grid, positions, M);
             order = m_grid_order->data();
+        }
+        if (params) {
+            tnn::abi_check(tnn_grid_mlp_push_inference_rows(&grid, &d, params, this->unpadded_in(), this->unpadded_out(), this->bias_flag(),
+                                                            this->packed_weights(), this->packed_weights_transposed(), this->prepared_forward_storage(),
+                                                            this->prepared_backward_storage(), positions, order, table, y, y_cols, M, this->get_queue().abi()));
+            return;
         }
         tnn::abi_check(tnn_grid_mlp_inference_rows(&grid, &d, positions, order, table, this->prepared_forward(), y, y_cols, M, this->get_queue().abi()));
     }

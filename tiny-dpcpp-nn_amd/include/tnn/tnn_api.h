@@ -92,14 +92,15 @@ class Module {
     /// Columns a caller sees of the output.
     virtual int64_t visible_columns() const = 0;
     /// keep: a backward pass may follow. training: only where a network keeps its activations in the module's workspace.
-    virtual torch::Tensor forward_rows(const torch::Tensor &x, bool keep, bool training, RowsPass &pass) = 0;
+    /// push: the parameters to take over first, or an undefined tensor.
+    virtual torch::Tensor forward_rows(const torch::Tensor &x, const torch::Tensor &push, bool keep, bool training, RowsPass &pass) = 0;
     /// Gradients of the input (undefined unless wanted and available) and of the parameters, in the type and shape of `params`.
     virtual std::tuple<torch::Tensor, torch::Tensor> backward_rows(const torch::Tensor &dy, const RowsPass &pass, double loss_scale, bool want_dx,
                                                                    const torch::Tensor &params) = 0;
     /// The parameter tensor as the Python modules hold it (a network's is packed) becomes the module's parameters.
     virtual void push_params(const torch::Tensor &params) = 0;
     /// Network modules behind a grid encoding: the same two passes on positions.
-    virtual torch::Tensor forward_rows_with_encoding(const Module &, const torch::Tensor &, bool) {
+    virtual torch::Tensor forward_rows_with_encoding(const Module &, const torch::Tensor &, const torch::Tensor &, bool) {
         throw std::runtime_error("forward_rows_with_encoding: not a network module");
     }
     virtual std::tuple<torch::Tensor, torch::Tensor> backward_rows_with_encoding(const Module &, const torch::Tensor &, const torch::Tensor &, double, const torch::Tensor &,
@@ -273,7 +274,8 @@ template <typename T> class EncodingModule : public Module {
 
     torch::Tensor input_rows(const torch::Tensor &x) const override { return x.to(torch::kFloat32).contiguous(); }
     int64_t visible_columns() const override { return encoding_->get_padded_output_width(); }
-    torch::Tensor forward_rows(const torch::Tensor &x, bool keep, bool, RowsPass &pass) override {
+    torch::Tensor forward_rows(const torch::Tensor &x, const torch::Tensor &push, bool keep, bool, RowsPass &pass) override {
+        if (push.defined()) push_params(push);
         if (keep) pass.input = x;
         return forward_pass(x);
     }
@@ -531,26 +533,28 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
     }
     int64_t visible_columns() const override { return network_.get_unpadded_output_width(); }
 
-    torch::Tensor forward_rows(const torch::Tensor &x, bool keep, bool training, RowsPass &pass) override {
+    torch::Tensor forward_rows(const torch::Tensor &x, const torch::Tensor &push, bool keep, bool training, RowsPass &pass) override {
         this->enter();
         CHECK_INPUT(x);
         const int64_t rows = x.size(0), n_out = visible_columns();
         pass.rows = rows;
         pass.cols = x.size(1);
         pass.dtype = x.scalar_type();
+        const bool recompute = keep && can_recompute_backward();
+        const float *pushed = PushedWithThePass(push, rows > 0 && (!keep || recompute)); // (otherwise they are pushed here)
         if (rows == 0) {
             pass.input = x;
             return fresh({0, n_out}, kType);
         }
         const bool whole = x.size(1) == WIDTH && x.scalar_type() == kType;
-        const bool recompute = keep && can_recompute_backward();
         if (!keep || recompute) {
             // a backward pass forms the activations again from the matrix this one reads
             torch::Tensor in = x;
             if (!whole && (keep || !network_.takes_narrow_rows((size_t)rows))) in = this->resized(x, rows, WIDTH, kType, pad_value_, 1.0f);
             if (keep) pass.input = in;
             torch::Tensor y = fresh({rows, n_out}, kType);
-            network_.inference_rows(in.data_ptr(), this->abi_dtype(in.scalar_type()), (int)in.size(1), y.data_ptr(), (int)n_out, (size_t)rows, pad_value_);
+            network_.inference_rows(in.data_ptr(), this->abi_dtype(in.scalar_type()), (int)in.size(1), y.data_ptr(), (int)n_out, (size_t)rows, pad_value_,
+                                    pushed);
             return y;
         }
         if constexpr (WIDTH == 128) {
@@ -617,12 +621,13 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
         set_params(p, true);
     }
 
-    torch::Tensor forward_rows_with_encoding(const Module &encoding, const torch::Tensor &positions, bool keep) override {
+    torch::Tensor forward_rows_with_encoding(const Module &encoding, const torch::Tensor &positions, const torch::Tensor &push, bool keep) override {
         this->enter();
         const tnn_grid_desc *grid = CheckedPositions(encoding, positions);
+        const float *pushed = PushedWithThePass(push, true);
         const int64_t rows = positions.size(0), n_out = visible_columns();
         torch::Tensor y = fresh({rows, n_out}, kType);
-        network_.inference_with_grid_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), (size_t)rows, y.data_ptr(), (int)n_out, keep);
+        network_.inference_with_grid_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), (size_t)rows, y.data_ptr(), (int)n_out, keep, pushed);
         return y;
     }
 
@@ -723,6 +728,15 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
         TORCH_CHECK(positions.dim() == 2 && positions.scalar_type() == torch::kFloat32, "positions must be a float32 matrix");
         if (positions.sizes()[1] != (int64_t)grid->n_dims) throw std::runtime_error("Input tensor has incorrect dimensions");
         return grid;
+    }
+
+    /// The parameters as the passes that push them in their own launch take them (fp32 on the device), or null after a push here.
+    const float *PushedWithThePass(const torch::Tensor &push, const bool the_pass_can) {
+        if (!push.defined()) return nullptr;
+        if (the_pass_can && push.is_cuda() && push.scalar_type() == torch::kFloat32 && push.is_contiguous() && (size_t)push.numel() == n_params())
+            return push.data_ptr<float>();
+        push_params(push);
+        return nullptr;
     }
 
     size_t CheckedBatch(const torch::Tensor &input_tensor, const uint32_t width) const {

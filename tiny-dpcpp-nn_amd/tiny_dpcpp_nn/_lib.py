@@ -95,6 +95,10 @@ SIGNATURES = {
                                 c_void_p]),
     "tnn_mlp_inference_rows": (c_int, [POINTER(MlpDesc), c_void_p, c_void_p, c_int, c_int, c_float, c_void_p, c_int, c_size_t, c_void_p]),
     "tnn_grid_mlp_inference_rows": (c_int, [POINTER(GridDesc), POINTER(MlpDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_size_t, c_void_p]),
+    "tnn_mlp_push_inference_rows": (c_int, [POINTER(MlpDesc), c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
+                                            c_float, c_void_p, c_int, c_size_t, c_void_p]),
+    "tnn_grid_mlp_push_inference_rows": (c_int, [POINTER(GridDesc), POINTER(MlpDesc), c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+                                                 c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_size_t, c_void_p]),
     "tnn_mlp_backward_recompute_rows": (c_int, [POINTER(MlpDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_float, c_float, c_void_p, c_int,
                                                 c_void_p, c_size_t, c_void_p, c_size_t, c_void_p]),
     "tnn_grid_mlp_backward_rows": (c_int, [POINTER(GridDesc), POINTER(MlpDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_float,
