@@ -830,3 +830,22 @@ def test_image_learning_sample_on_a_picture_file(tcnn, monkeypatch, tmp_path):
     np.testing.assert_allclose(got[4], pic[h - 1, w - 1], atol=1e-3)
     monkeypatch.setattr(sys, "argv", ["mlp_learning_an_image.py", "--n_steps", "300", "--image", path_png, "--seed", "3"])
     assert sample.main() < 3e-3
+
+
+def test_a_tangent_is_refused_and_a_failed_call_pushes_again(tcnn):
+    """The modules have no forward-mode derivative: a dual input or parameter is refused, not differentiated as a constant. With the push
+    switched off for unchanged parameters, a pass that raised has pushed nothing."""
+    import torch.autograd.forward_ad as fwAD
+    net = tcnn.Network(8, 4, net_config(16, 2), dtype=torch.bfloat16)
+    x = torch.rand((16, 8), device="cuda")
+    with fwAD.dual_level():
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            net(fwAD.make_dual(x, torch.ones_like(x)))
+    net.push_params_every_forward = False
+    with torch.no_grad():
+        before = net(x)
+        net.params.mul_(2.0)
+        with pytest.raises((RuntimeError, ValueError)):
+            net(torch.rand((16,), device="cuda"))
+        after = net(x)
+    assert not torch.equal(before, after)

@@ -70,9 +70,16 @@ struct EncodedNetworkBackward : public torch::autograd::Node {
     std::string name() const override { return "TnnEncodedNetworkBackward"; }
 };
 
+/// The nodes here have no forward-mode derivative: a tangent is refused, as PyTorch refuses it for a function without a jvp, not dropped.
+inline void refuse_tangents(std::initializer_list<torch::Tensor> inputs) {
+    for (const torch::Tensor &t : inputs)
+        TORCH_CHECK_NOT_IMPLEMENTED(!torch::autograd::isFwGradDefined(t), "tiny_dpcpp_nn modules have no forward-mode derivative");
+}
+
 /// y = module(x), recorded for autograd when that is on and anything asks for gradients.
 inline torch::Tensor call(const std::shared_ptr<tnn::Module> &module, const torch::Tensor &x, const torch::Tensor &params, bool push, bool training,
                           double loss_scale) {
+    refuse_tangents({x, params});
     const torch::Tensor in = module->input_rows(x); // (PyTorch operations where any are needed: autograd sees them)
     const bool record = torch::autograd::compute_requires_grad(in, params);
     tnn::Module::RowsPass pass;
@@ -97,6 +104,7 @@ inline torch::Tensor call(const std::shared_ptr<tnn::Module> &module, const torc
 /// y = network(encoding(positions)) for a pair that can_train_with_encoding (or, without autograd, can_fuse_encoding) accepts.
 inline torch::Tensor call_with_encoding(const std::shared_ptr<tnn::Module> &network, const std::shared_ptr<tnn::Module> &encoding, const torch::Tensor &x,
                                         const torch::Tensor &params, const torch::Tensor &table, bool push_network, bool push_table, double loss_scale) {
+    refuse_tangents({x, params, table});
     if (push_table) encoding->push_params(table);
     const torch::Tensor positions = x.detach().to(torch::kFloat32).contiguous();
     const bool record = torch::autograd::compute_requires_grad(params, table);

@@ -129,13 +129,12 @@ class Module(torch.nn.Module):
         """What the reference does in front of every forward (modules.py:253): set_params(). With push_params_every_forward
         switched off, only when `params` is known to have changed: in-place updates (optimizer steps, copy_, load_state_dict)
         raise the tensor's version and a replaced tensor has another identity or address; writes through `.data` do neither."""
-        if self.push_params_every_forward:
-            return True
-        state = self._params_state()
-        if self._pushed == state:
-            return False
-        self._pushed = state
-        return True
+        return self.push_params_every_forward or self._pushed != self._params_state()
+
+    def _has_pushed(self):
+        """Called once the pass has taken the parameters over: after one that raised, the next pushes again."""
+        if not self.push_params_every_forward:
+            self._pushed = self._params_state()
 
     def get_params(self):
         """The parameters as the native module holds them (a network's: packed layout)."""
@@ -144,7 +143,9 @@ class Module(torch.nn.Module):
     # ---- evaluation ----------------------------------------------------------------------------------------------
     def forward(self, x):
         # one entry into the native module: push, padding and conversion, the pass, and its node in the autograd graph
-        return self.tnn_module.call(x, self.params, self._must_push(), self.training, self.loss_scale)
+        y = self.tnn_module.call(x, self.params, self._must_push(), self.training, self.loss_scale)
+        self._has_pushed()
+        return y
 
 
 class Network(Module):
@@ -229,5 +230,8 @@ class NetworkWithInputEncoding(Module):
             return self.network_with_encoding(x)
         # a grid encoding and its network as one kernel (backward: one kernel plus the scatter), with the values of the two
         # modules in turn, the reference's only route; the encoded matrix is never stored
-        return network.tnn_module.call_with_encoding(encoding.tnn_module, x, network.params, encoding.params, network._must_push(), encoding._must_push(),
-                                                     network.loss_scale)
+        y = network.tnn_module.call_with_encoding(encoding.tnn_module, x, network.params, encoding.params, network._must_push(), encoding._must_push(),
+                                                  network.loss_scale)
+        network._has_pushed()
+        encoding._has_pushed()
+        return y
