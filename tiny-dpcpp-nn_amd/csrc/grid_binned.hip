@@ -13,7 +13,7 @@
 //      entries to the table as whole lines.
 // A record of two features is 16 bytes written once and read once, where the two atomic requests it replaces occupy the
 // memory side for 64.
-// Measured, 2^20 points, 3-D, 2^19 entries, 15 levels this way: 2 x (165 + 177) us, 3 TB/s of records both ways; before, the
+// Measured, 2^20 points, 3-D, 2^19 entries, 15 levels this way: 2 x (164 + 172) us, 3 TB/s of records both ways; before, the
 // atomics of the ten finest of these levels alone took 1.5 ms.
 #include "grid_binned.h"
 
@@ -22,9 +22,17 @@
 
 namespace tnn {
 
-constexpr int kBinThreads = 512;
-constexpr int kBinPoints = 2; // points of a thread
 constexpr int kBinSumThreads = 1024; // at most
+
+// A binning workgroup: its threads (at most), the points of a thread, and the most records it sorts in LDS. 2048 records of 16
+// bytes let four workgroups of 8 waves share a CU, whose phases (loads, LDS, stores) then overlap; wider records take half as many.
+// (3-D, 2^19 points, 15 levels of two features: 164 us; 4096 records 177, 1024 184.)
+template <int D, int F> struct BinShape {
+    static constexpr int kThreads = F <= 2 ? 512 : 256;
+    static constexpr int kPoints = D == 2 && F <= 2 ? 2 : 1;
+    static constexpr int kPairs = 1 << (D - 1);
+    static constexpr int kRecords = kThreads * kPoints * kPairs;
+};
 
 // Entry e of a level: its bin and its place there.
 struct Bins {
@@ -89,38 +97,47 @@ __device__ __forceinline__ void pair_entries(const uint32_t (&cell)[D], uint32_t
     }
 }
 
-// One workgroup bins up to kBinPoints x kBinThreads consecutive points of one level: it counts its records per bin, which
-// gives every record its place among them, reserves that much of every bin with one atomic, and writes the records there, so
-// that a bin receives them in runs. The levels of the same points are consecutive workgroups of one XCD, which shares the
-// rows of dL/dy between them in its L2.
+// One workgroup bins kPoints points a thread of one level: it counts its records per bin, which gives every record its place among
+// them, reserves that much of every bin with one atomic, sorts the records by bin in LDS and writes them from there, so that a
+// wave stores whole runs: neighbouring lanes, neighbouring records. Bound by the records' bytes on their way to memory, 3.0 TB/s
+// at 12, 16, 24 and 40 bytes a record. (Every lane storing its own records, as many L2 requests as records times pieces of 16
+// bytes: four features 166 -> 133 us, eight 138 -> 119, one 36 -> 27, two as fast either way, 3-D or 2-D, 2^18 points.) The levels of the same points are consecutive workgroups of one
+// XCD, which shares the rows of dL/dy between them in its L2.
 // Records beyond a bin's capacity are counted and dropped.
 template <int D, int F, typename G>
-__global__ void __launch_bounds__(kBinThreads)
+__global__ void __launch_bounds__((BinShape<D, F>::kThreads))
     grid_bin_kernel(const GridLevels lv, const GridParams gp, const BinPlan bp, const GradLayout dl, const float *__restrict__ xin,
                     const float4 *__restrict__ order, const G *__restrict__ dLdy, uint32_t *__restrict__ cursors, BinRecord<F> *__restrict__ records,
-                    long long first, long long last, uint32_t per_wg) {
-    constexpr int NP = 1 << (D - 1); // pairs of a point
-    static_assert(kBinThreads * kBinPoints * NP <= 4096 && kBinMaxBins <= 1024, "a record's place is packed into 12 + 10 + 10 bits");
-    __shared__ uint32_t base[kBinMaxBins];  // records per bin, then the first place of them
-    __shared__ uint32_t split[kBinMaxBins]; // the same for far sides that lie in another bin than the near side
-    const uint32_t turn = blockIdx.x / 8, k = turn % bp.n_levels;
+                    long long first, long long last) {
+    typedef BinShape<D, F> S;
+    constexpr int NP = S::kPairs, P = S::kPoints;
+    static_assert(S::kRecords <= 4096 && kBinMaxBins <= 1024, "a record's place is packed into 12 + 10 + 10 bits");
+    const int T = blockDim.x;
+    extern __shared__ __align__(16) unsigned char bin_smem[];
+    BinRecord<F> *const sorted = reinterpret_cast<BinRecord<F> *>(bin_smem);
+    uint16_t *const bin_of = reinterpret_cast<uint16_t *>(sorted + T * P * NP); // of a sorted record
+    uint32_t *const base = reinterpret_cast<uint32_t *>(bin_of + T * P * NP);    // records per bin, then the first sorted one of them
+    const uint32_t turn = blockIdx.x / 8, k = turn % bp.n_levels, per_wg = T * P;
     const long long begin = first + (long long)((turn / bp.n_levels) * 8 + blockIdx.x % 8) * per_wg;
     if (begin >= last) return;
     const long long end = begin + per_wg < last ? begin + per_wg : last;
     const Bins dealt{bp.bins_log2[k], bp.run_log2[k]};
     const uint32_t l = bp.level[k], n_bins = 1u << dealt.n_log2;
+    uint32_t *const split = base + n_bins; // records per bin of far sides that lie in another bin than the near side, then the next place of one
+    uint32_t *const shift = split + n_bins; // place in the bin less place among the sorted records
+    uint32_t *const wave_sum = shift + n_bins;
     const uint32_t size = lv.size[l], res = lv.resolution[l], flags = lv.flags[l], capacity = bp.capacity[k];
     const float scale = lv.scale[l];
     uint32_t *const cursor = cursors + bp.first_bin[k];
     BinRecord<F> *const bins = records + bp.first_record[k];
 
-    for (uint32_t b = threadIdx.x; b < n_bins; b += kBinThreads) base[b] = split[b] = 0;
+    for (uint32_t b = threadIdx.x; b < n_bins; b += T) base[b] = split[b] = 0;
     __syncthreads();
-    float frac[kBinPoints][D], gy[kBinPoints][F];
-    uint32_t where[kBinPoints][NP], place[kBinPoints][NP]; // place: rank in the bin (12 bits), bin, bin of the far side
+    float frac[P][D], gy[P][F];
+    uint32_t where[P][NP], place[P][NP]; // place: rank in the bin (12 bits), bin, bin of the far side
 #pragma unroll
-    for (int u = 0; u < kBinPoints; ++u) {
-        const long long i = begin + threadIdx.x + u * kBinThreads;
+    for (int u = 0; u < P; ++u) {
+        const long long i = begin + threadIdx.x + u * T;
         if (i >= end) continue;
         float x[D];
         const long long row = bin_point<D>(xin, order, i, x);
@@ -139,16 +156,45 @@ __global__ void __launch_bounds__(kBinThreads)
         }
     }
     __syncthreads();
-    for (uint32_t b = threadIdx.x; b < n_bins; b += kBinThreads) {
-        const uint32_t n = base[b], n_split = split[b];
-        const uint32_t at = n + n_split ? atomicAdd(&cursor[b], n + n_split) : 0u;
-        base[b] = at;
-        split[b] = at + n;
+    // A running sum over the bins' counts, `each` neighbouring bins a thread (at most 1024 bins over at least 128 threads).
+    constexpr int kEach = 8;
+    const uint32_t each = (n_bins + T - 1) / T, b0 = threadIdx.x * each;
+    uint32_t count[kEach], mine = 0;
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+        count[e] = (uint32_t)e < each && b0 + e < n_bins ? base[b0 + e] : 0u;
+        mine += count[e];
+    }
+    uint32_t upto = mine; // of the wave's lanes up to this one
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t below = __shfl_up(upto, off, 64);
+        if ((int)(threadIdx.x & 63) >= off) upto += below;
+    }
+    if ((threadIdx.x & 63) == 63) wave_sum[threadIdx.x >> 6] = upto;
+    __syncthreads();
+    uint32_t at = upto - mine, total = 0;
+    for (int w = 0; w < T / 64; ++w) {
+        const uint32_t sum = wave_sum[w];
+        if (w < (int)(threadIdx.x >> 6)) at += sum;
+        total += sum;
+    }
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+        const uint32_t b = b0 + e;
+        if ((uint32_t)e < each && b < n_bins) {
+            const uint32_t n_split = split[b];
+            const uint32_t reserved = count[e] + n_split ? atomicAdd(&cursor[b], count[e] + n_split) : 0u;
+            base[b] = at;
+            shift[b] = reserved - at;
+            split[b] = reserved + count[e];
+            at += count[e];
+        }
     }
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < kBinPoints; ++u) {
-        if (begin + threadIdx.x + u * kBinThreads >= end) continue;
+    for (int u = 0; u < P; ++u) {
+        if (begin + threadIdx.x + u * T >= end) continue;
 #pragma unroll
         for (int c = 0; c < NP; ++c) {
             float weight = 1.0f;
@@ -158,15 +204,29 @@ __global__ void __launch_bounds__(kBinThreads)
             r.frac = frac[u][0];
 #pragma unroll
             for (int f = 0; f < F; ++f) r.g[f] = weight * gy[u][f];
-            const uint32_t bin = (place[u][c] >> 12) & 1023u, far_bin = place[u][c] >> 22;
-            const auto put = [&](uint32_t to, uint32_t at, uint32_t sides) {
-                r.where = where[u][c] | (sides << 30);
-                if (at < capacity) bins[(size_t)to * capacity + at] = r;
-            };
-            put(bin, base[bin] + (place[u][c] & 4095u), far_bin == bin ? 3u : 1u);
-            if (far_bin != bin) put(far_bin, atomicAdd(&split[far_bin], 1u), 2u);
+            const uint32_t bin = (place[u][c] >> 12) & 1023u, far_bin = place[u][c] >> 22, slot = base[bin] + (place[u][c] & 4095u);
+            r.where = where[u][c] | ((far_bin == bin ? 3u : 1u) << 30);
+            sorted[slot] = r;
+            bin_of[slot] = (uint16_t)bin;
+            if (far_bin != bin) {
+                r.where = where[u][c] | (2u << 30);
+                const uint32_t to = atomicAdd(&split[far_bin], 1u);
+                if (to < capacity) bins[(size_t)far_bin * capacity + to] = r;
+            }
         }
     }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < total; i += T) {
+        const uint32_t bin = bin_of[i], to = shift[bin] + i;
+        if (to < capacity) bins[(size_t)bin * capacity + to] = sorted[i];
+    }
+}
+
+// LDS of it with T threads.
+template <int D, int F> static size_t bin_lds(const BinPlan &p, unsigned T) {
+    uint32_t n_bins = 0;
+    for (uint32_t k = 0; k < p.n_levels; ++k) n_bins = std::max(n_bins, 1u << p.bins_log2[k]);
+    return (size_t)T * BinShape<D, F>::kPoints * BinShape<D, F>::kPairs * (sizeof(BinRecord<F>) + sizeof(uint16_t)) + (3 * n_bins + 16) * sizeof(uint32_t);
 }
 
 // One workgroup sums one bin and stores (or adds) its entries. Bound by the records' bytes and the LDS atomics (two values of two
@@ -306,14 +366,19 @@ static int launch_binned(const BinPlan &p, const GridLevels &lv, const GridParam
     const auto sum = grid_bin_sum_kernel<D, F, G>;
     if (!reserve_lds(reinterpret_cast<const void *>(sum), p.slice_lds))
         return fail(TNN_ERR_HIP, "cannot reserve %u bytes of LDS", p.slice_lds);
+    typedef BinShape<D, F> S;
+    const auto bin = grid_bin_kernel<D, F, G>;
+    if (!reserve_lds(reinterpret_cast<const void *>(bin), bin_lds<D, F>(p, S::kThreads)))
+        return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", bin_lds<D, F>(p, S::kThreads));
     // (as many waves on a CU as it takes whatever LDS the bins need; small bins are over before 16 waves are under way)
     const unsigned sum_threads = p.slice_lds > 32 * 1024 ? kBinSumThreads : kBinSumThreads / 2;
     for (size_t first = 0; first < M; first += p.batch) {
         const size_t last = std::min(M, first + p.batch), n = last - first;
-        const uint32_t per_wg = n * p.n_levels < size_t(512) * kBinThreads * kBinPoints ? kBinThreads : kBinThreads * kBinPoints;
-        const size_t stretches = (n + per_wg - 1) / per_wg;
-        TNN_LAUNCH((grid_bin_kernel<D, F, G>), dim3((unsigned)((stretches + 7) / 8 * 8 * p.n_levels)), dim3(kBinThreads), 0, s, lv, gp, p, dl, x, order,
-                   (const G *)dLdy, cursors, records, (long long)first, (long long)last, per_wg);
+        // (a small batch: half as many threads, twice as many workgroups, while there are fewer than two for every CU)
+        const unsigned T = n * p.n_levels < size_t(512) * S::kThreads * S::kPoints ? S::kThreads / 2 : S::kThreads;
+        const size_t stretches = (n + T * S::kPoints - 1) / (T * S::kPoints);
+        TNN_LAUNCH(bin, dim3((unsigned)((stretches + 7) / 8 * 8 * p.n_levels)), dim3(T), (bin_lds<D, F>(p, T)), s, lv, gp, p, dl, x, order,
+                   (const G *)dLdy, cursors, records, (long long)first, (long long)last);
         int rc = check_launch("grid_bin_kernel");
         if (rc) return rc;
         TNN_LAUNCH(sum, dim3(p.n_bins), dim3(sum_threads), p.slice_lds, s, lv, gp, p, dl, x, order, (const G *)dLdy, cursors,
