@@ -167,10 +167,10 @@ struct BackwardPlan {
 };
 constexpr uint32_t kMaxTiled = 16;
 constexpr uint8_t kAllFeatures = 255;
-#ifndef TNN_BOXED_MIN_PER_CELL
-#define TNN_BOXED_MIN_PER_CELL 0.3
-#endif
-constexpr double kBoxedMinPerCell = TNN_BOXED_MIN_PER_CELL; // points of the batch per cell of a level, at least, for the boxed route
+// Points of the batch per cell of a level, at least, for the boxed route: against the direct route, and against the binned one,
+// whose levels cost the same whatever their cells (2-D, 2^18 points: a level of 0.31 points a cell takes 6.6 us boxed and 3.0
+// binned; one of 0.7, 4.8 and 7.7; 1.6: 3.8 and 6.4; 3.5: 3.1 and 7.5; 7.9: 2.6 and 6.3).
+constexpr double kBoxedMinPerCell = 0.3, kBoxedMinPerCellBinned = 0.5;
 
 constexpr int kGridWave = 64;                    // lanes of a wave
 constexpr int kBwdThreads = 512;                 // the backward kernel's workgroups
@@ -630,7 +630,7 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
             const double per_cell = (double)M / std::pow(R, (double)D);
             int chunk_log2 = -1;
             // (short stretches: many workgroups of some ten microseconds each spread over the CUs far more evenly than few long ones)
-            for (int c = 10; c >= 9 && chunk_log2 < 0 && bp.n_tiled < kMaxTiled && per_cell >= kBoxedMinPerCell; --c) {
+            for (int c = 10; c >= 9 && chunk_log2 < 0 && bp.n_tiled < kMaxTiled && per_cell >= (bins ? kBoxedMinPerCellBinned : kBoxedMinPerCell); --c) {
                 const double share = std::min(1.0, (double)(1u << c) / std::max(per_row, 1.0));
                 double cells = (share * R + R / coarse + 2.0) * (R / coarse + 2.0);
                 if (D == 3) cells *= R / coarse + 2.0;
