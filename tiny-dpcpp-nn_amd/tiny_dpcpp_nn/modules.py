@@ -9,7 +9,7 @@ layout conventions (`params` of a network is the packed layout, `set_params(tens
 is PyTorch-ROCm's "cuda" where the reference has "xpu".
 
 As in the reference (modules.py:253), every forward pushes `params` to the native module first, so that any way of
-writing them is seen, `params.data[...] = ...` included. The push is one small kernel on the device. A caller that only
+writing them is seen, `params.data[...] = ...` included. The push is part of the forward kernel, or one small kernel in front of it. A caller that only
 ever updates `params` through operations PyTorch's version counter sees (optimizers, copy_(), load_state_dict) can switch
 the push off for unchanged parameters with `module.push_params_every_forward = False`.
 
