@@ -807,7 +807,7 @@ class Bench:
         ach = bpp * M / (scatter_ms * 1e-3) / 1e9
         roof = {"bound": "hbm", "achieved": ach, "peak": PEAK_HBM, "unit": "GB/s", "frac": ach / PEAK_HBM,
                 "traffic": MEASURED_TRAFFIC_BYTES.get(("grid_train_packed" if args.packed_scatter else ("grid_train_ordered" if ordered else "grid_train"), lg)),
-                "kernel": "grid_backward_kernel (with the fill of the gradient table in front of it)" + (" over points in cell order" if ordered else ""),
+                "kernel": "grid_backward_kernel without scratch memory (with the fill of the gradient table in front of it; the step itself sorts its contributions)" + (" over points in cell order" if ordered else ""),
                 "kernel_ms": scatter_ms,
                 "algorithmic_bytes_per_launch": bpp * M}
         out = line("hash-grid + fused-MLP training samples/s (2-D, 16x2, log2 19; w64, 2 hidden layers; batch 2^18; whole step with both Adam updates)",
