@@ -849,3 +849,50 @@ def test_a_tangent_is_refused_and_a_failed_call_pushes_again(tcnn):
             net(torch.rand((16,), device="cuda"))
         after = net(x)
     assert not torch.equal(before, after)
+
+
+@pytest.mark.parametrize("own_streams", [False, True])
+def test_two_threads_on_one_module(tcnn, own_streams):
+    """Two Python threads, each with its own batch, on one stream or a stream each, share a field and its encoding. The batches are large
+    enough to be put in cell order, in a buffer the module shares between its passes: a pass that launched on the other thread's
+    order, stream or scratch memory would return the other thread's rows. Gradients are sums in no fixed order: the network's, rounded to bf16 at
+    the end, within a unit of its last place (2^-8), the table's within fp32 sums."""
+    import threading
+
+    field = tcnn.NetworkWithInputEncoding(2, 16, net_config(64, 2), {"otype": "HashGrid", "type": "Hash", "n_levels": 16, "n_features_per_level": 2,
+                                          "log2_hashmap_size": 15, "base_resolution": 16, "per_level_scale": 1.5}, dtype=torch.bfloat16, use_bias=False)
+    with torch.no_grad():
+        field.encoding.params.normal_(0, 0.1)
+    batches = [torch.rand((2 ** 18 + 8 * i, 2), device=DEVICE) for i in range(2)]
+    grads = [torch.randn((x.shape[0], 16), device=DEVICE).bfloat16() for x in batches]
+
+    def passes(i):
+        with torch.no_grad():
+            out = [field(batches[i]), field.encoding(batches[i])]
+        y = field(batches[i])
+        out += torch.autograd.grad(y, [field.network.params, field.encoding.params], grads[i])
+        return out
+
+    expected = [passes(i) for i in range(2)]
+    torch.cuda.synchronize()
+    worst, errors, start = [torch.zeros(4, device=DEVICE) for _ in range(2)], [], threading.Barrier(2)
+
+    def worker(i):
+        try:
+            start.wait()
+            with torch.cuda.stream(torch.cuda.Stream() if own_streams else torch.cuda.default_stream()):
+                for _ in range(25):
+                    off = [(a.float() - b.float()).abs().max() / b.float().abs().max() for a, b in zip(passes(i), expected[i])]
+                    worst[i] = torch.maximum(worst[i], torch.stack(off))
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=worker, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for w in worst:
+        assert w[0] == 0 and w[1] == 0 and w[2] <= 2.0 ** -8 and w[3] <= 1e-5, w

@@ -17,6 +17,11 @@ namespace tnn_binding {
 using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
+// The interpreter's lock is released before a module's is waited for, here and in every binding: a thread that holds a module's
+// may need the interpreter's for a moment (dropping the last reference to a tensor that Python has seen).
+typedef std::lock_guard<std::recursive_mutex> ModuleLock;
+typedef std::scoped_lock<std::recursive_mutex, std::recursive_mutex> ModulePairLock;
+
 /// A network or an encoding: gradients of its input (a network's) and of its parameters.
 struct ModuleBackward : public torch::autograd::Node {
     std::shared_ptr<tnn::Module> module;
@@ -33,6 +38,7 @@ struct ModuleBackward : public torch::autograd::Node {
         const torch::AutoGradMode no_grad(false);
         tnn::Module::RowsPass kept = pass;
         kept.input = x;
+        const ModuleLock pass_lock(module->pass_mutex());
         auto [dx, dparams] = module->backward_rows(grads[0], kept, loss_scale, task_should_compute_output(0), p);
         return {dx, dparams};
     }
@@ -58,6 +64,7 @@ struct EncodedNetworkBackward : public torch::autograd::Node {
         const torch::Tensor x = positions.unpack(), p = params.unpack(), t = table.unpack();
         if (!grads[0].defined()) return {torch::Tensor(), torch::Tensor()};
         const torch::AutoGradMode no_grad(false);
+        const ModulePairLock pass_lock(network->pass_mutex(), encoding->pass_mutex());
         auto [dparams, dtable] = network->backward_rows_with_encoding(*encoding, x, grads[0], loss_scale, p, t);
         return {dparams, dtable};
     }
@@ -86,6 +93,7 @@ inline torch::Tensor call(const std::shared_ptr<tnn::Module> &module, const torc
     torch::Tensor y;
     {
         const torch::AutoGradMode no_grad(false);
+        const ModuleLock pass_lock(module->pass_mutex());
         y = module->forward_rows(in, push && module->n_params() ? params : torch::Tensor(), record, training, pass);
     }
     if (!record) return y;
@@ -105,12 +113,13 @@ inline torch::Tensor call(const std::shared_ptr<tnn::Module> &module, const torc
 inline torch::Tensor call_with_encoding(const std::shared_ptr<tnn::Module> &network, const std::shared_ptr<tnn::Module> &encoding, const torch::Tensor &x,
                                         const torch::Tensor &params, const torch::Tensor &table, bool push_network, bool push_table, double loss_scale) {
     refuse_tangents({x, params, table});
-    if (push_table) encoding->push_params(table);
     const torch::Tensor positions = x.detach().to(torch::kFloat32).contiguous();
     const bool record = torch::autograd::compute_requires_grad(params, table);
     torch::Tensor y;
     {
         const torch::AutoGradMode no_grad(false);
+        const ModulePairLock pass_lock(network->pass_mutex(), encoding->pass_mutex());
+        if (push_table) encoding->push_params(table);
         y = network->forward_rows_with_encoding(*encoding, positions, push_network ? params : torch::Tensor(), record);
     }
     if (!record) return y;

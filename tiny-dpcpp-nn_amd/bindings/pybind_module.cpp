@@ -39,25 +39,30 @@ class PybindingModule {
 
     torch::Tensor fwd(torch::Tensor input) {
         CHECK_INPUT(input);
+        const auto pass_lock = lock();
         return m_module->forward_pass(input);
     }
     torch::Tensor inference(torch::Tensor input) {
         CHECK_INPUT(input);
+        const auto pass_lock = lock();
         return m_module->inference(input);
     }
     std::tuple<torch::Tensor, torch::Tensor> bwd_no_encoding_grad(torch::Tensor grad_output, bool pack_gradient, bool get_dl_dinput) {
         CHECK_INPUT(grad_output);
+        const auto pass_lock = lock();
         return m_module->backward_pass(grad_output, pack_gradient, get_dl_dinput);
     }
     std::tuple<torch::Tensor, torch::Tensor> bwd_with_encoding_grad(torch::Tensor grad_output, torch::Tensor input_from_fwd, bool pack_gradient,
                                                                     bool get_dl_dinput) {
         CHECK_INPUT(grad_output);
+        const auto pass_lock = lock();
         return m_module->backward_pass(grad_output, input_from_fwd, pack_gradient, get_dl_dinput);
     }
     /// Network modules: whether inference on `encoding`'s output can run as one kernel, and that inference.
     bool can_fuse_encoding(const PybindingModule &encoding) const { return m_module->can_fuse_encoding(*encoding.m_module); }
     torch::Tensor inference_with_encoding(const PybindingModule &encoding, torch::Tensor positions, bool a_backward_pass_follows) {
         CHECK_INPUT(positions);
+        const tnn_binding::ModulePairLock pass_lock(m_module->pass_mutex(), encoding.m_module->pass_mutex());
         return m_module->inference_with_encoding(*encoding.m_module, positions, a_backward_pass_follows);
     }
     /// Network modules, training without stored activations: inference() is the forward pass, these are the backward passes.
@@ -65,6 +70,7 @@ class PybindingModule {
     std::tuple<torch::Tensor, torch::Tensor> bwd_recompute(torch::Tensor grad_output, torch::Tensor input_from_fwd, bool pack_gradient, bool get_dl_dinput) {
         CHECK_INPUT(grad_output);
         CHECK_INPUT(input_from_fwd);
+        const auto pass_lock = lock();
         return m_module->backward_pass_recompute(grad_output, input_from_fwd, pack_gradient, get_dl_dinput);
     }
     bool can_train_with_encoding(const PybindingModule &encoding) const { return m_module->can_train_with_encoding(*encoding.m_module); }
@@ -72,6 +78,7 @@ class PybindingModule {
                                                                bool pack_gradient, bool positions_unchanged_since_forward) {
         CHECK_INPUT(positions);
         CHECK_INPUT(grad_output);
+        const tnn_binding::ModulePairLock pass_lock(m_module->pass_mutex(), encoding.m_module->pass_mutex());
         return m_module->backward_with_encoding(*encoding.m_module, positions, grad_output, pack_gradient, positions_unchanged_since_forward);
     }
     /// The module as an operator: parameters pushed (on request), forward pass, and a node of the autograd graph.
@@ -82,15 +89,28 @@ class PybindingModule {
                                      bool push_network, bool push_table, double loss_scale) const {
         return tnn_binding::call_with_encoding(m_module, encoding.m_module, x, params, table, push_network, push_table, loss_scale);
     }
-    torch::Tensor initial_params() { return m_module->initialize_params(); }
-    torch::Tensor initial_params(torch::Tensor &tensor) { return m_module->initialize_params(tensor); }
+    torch::Tensor initial_params() {
+        const auto pass_lock = lock();
+        return m_module->initialize_params();
+    }
+    torch::Tensor initial_params(torch::Tensor &tensor) {
+        const auto pass_lock = lock();
+        return m_module->initialize_params(tensor);
+    }
     /// weights_are_packed: the tensor already is in the packed parameter layout, no packing is done
-    void set_params(torch::Tensor &tensor, bool weights_are_packed) { m_module->set_params(tensor, weights_are_packed); }
-    torch::Tensor get_params() { return m_module->get_params(); }
+    void set_params(torch::Tensor &tensor, bool weights_are_packed) {
+        const auto pass_lock = lock();
+        m_module->set_params(tensor, weights_are_packed);
+    }
+    torch::Tensor get_params() {
+        const auto pass_lock = lock();
+        return m_module->get_params();
+    }
     uint32_t n_params() const { return (uint32_t)m_module->n_params(); }
     uint32_t n_output_dims() const { return (uint32_t)m_module->n_output_dims(); }
 
   private:
+    std::unique_lock<std::recursive_mutex> lock() const { return std::unique_lock<std::recursive_mutex>(m_module->pass_mutex()); }
     std::shared_ptr<tnn::Module> m_module; // shared with the autograd nodes of its calls
 };
 
@@ -134,27 +154,28 @@ PYBIND11_MODULE(tiny_dpcpp_nn_pybind_module, m) {
         .value("Linear", Activation::None)
         .export_values();
 
+    // Methods that run passes or touch parameters wait for the module's lock: without the interpreter's (native_call.h).
+    typedef py::call_guard<py::gil_scoped_release> Unlocked;
     py::class_<PybindingModule>(m, "Module")
-        .def("fwd", &PybindingModule::fwd)
-        .def("inference", &PybindingModule::inference)
+        .def("fwd", &PybindingModule::fwd, Unlocked())
+        .def("inference", &PybindingModule::inference, Unlocked())
         .def("can_fuse_encoding", &PybindingModule::can_fuse_encoding)
-        .def("inference_with_encoding", &PybindingModule::inference_with_encoding, py::arg("encoding"), py::arg("positions"),
+        .def("inference_with_encoding", &PybindingModule::inference_with_encoding, Unlocked(), py::arg("encoding"), py::arg("positions"),
              py::arg("a_backward_pass_follows") = false)
         .def("can_recompute_backward", &PybindingModule::can_recompute_backward)
-        .def("bwd_recompute", &PybindingModule::bwd_recompute)
+        .def("bwd_recompute", &PybindingModule::bwd_recompute, Unlocked())
         .def("can_train_with_encoding", &PybindingModule::can_train_with_encoding)
-        .def("bwd_with_encoding", &PybindingModule::bwd_with_encoding, py::arg("encoding"), py::arg("positions"), py::arg("grad_output"),
+        .def("bwd_with_encoding", &PybindingModule::bwd_with_encoding, Unlocked(), py::arg("encoding"), py::arg("positions"), py::arg("grad_output"),
              py::arg("pack_gradient"), py::arg("positions_unchanged_since_forward") = false)
-        .def("call", &PybindingModule::call, py::call_guard<py::gil_scoped_release>(), py::arg("x"), py::arg("params"), py::arg("push"), py::arg("training"),
-             py::arg("loss_scale"))
-        .def("call_with_encoding", &PybindingModule::call_with_encoding, py::call_guard<py::gil_scoped_release>(), py::arg("encoding"), py::arg("x"),
-             py::arg("params"), py::arg("table"), py::arg("push_network"), py::arg("push_table"), py::arg("loss_scale"))
-        .def("bwd_no_encoding_grad", &PybindingModule::bwd_no_encoding_grad)
-        .def("bwd_with_encoding_grad", &PybindingModule::bwd_with_encoding_grad)
-        .def("initial_params", py::overload_cast<>(&PybindingModule::initial_params))
-        .def("initial_params", py::overload_cast<torch::Tensor &>(&PybindingModule::initial_params))
-        .def("set_params", &PybindingModule::set_params)
-        .def("get_params", &PybindingModule::get_params)
+        .def("call", &PybindingModule::call, Unlocked(), py::arg("x"), py::arg("params"), py::arg("push"), py::arg("training"), py::arg("loss_scale"))
+        .def("call_with_encoding", &PybindingModule::call_with_encoding, Unlocked(), py::arg("encoding"), py::arg("x"), py::arg("params"), py::arg("table"),
+             py::arg("push_network"), py::arg("push_table"), py::arg("loss_scale"))
+        .def("bwd_no_encoding_grad", &PybindingModule::bwd_no_encoding_grad, Unlocked())
+        .def("bwd_with_encoding_grad", &PybindingModule::bwd_with_encoding_grad, Unlocked())
+        .def("initial_params", py::overload_cast<>(&PybindingModule::initial_params), Unlocked())
+        .def("initial_params", py::overload_cast<torch::Tensor &>(&PybindingModule::initial_params), Unlocked())
+        .def("set_params", &PybindingModule::set_params, Unlocked())
+        .def("get_params", &PybindingModule::get_params, Unlocked())
         .def("n_output_dims", &PybindingModule::n_output_dims)
         .def("n_params", &PybindingModule::n_params);
     m.def("set_initial_weight_seed", [](uint64_t seed) { tnn::set_initial_weight_seed(seed); }, py::arg("seed"),

@@ -8,6 +8,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/torch.h>
 
+#include <mutex>
 #include <tuple>
 
 #include "SwiftNetMLP.h"
@@ -110,6 +111,13 @@ class Module {
 
     tnn::queue &get_queue() { return queue_; }
 
+    /// A pass binds the module to the caller's stream, may put points in cell order into a buffer of the module's and then
+    /// launches on it, and reads parameter copies that the next pass may push again: two passes of one module must not
+    /// interleave on the host. Callers with several threads hold this from the first call of a pass to its last launch (the
+    /// Python bindings do, whose calls run without the interpreter's lock); a pair of modules, both. On the device enter() orders
+    /// the passes of different streams.
+    std::recursive_mutex &pass_mutex() const { return pass_mutex_; }
+
     /// First thing in every method: the module's kernels go to the stream the caller's tensor operations are on, so inputs
     /// produced there are complete when the kernels read them and the tensors handed back (allocated from that stream's
     /// pool) are written on it. When the caller has changed streams since the last call, the new stream first waits for
@@ -187,6 +195,7 @@ class Module {
   private:
     tnn::queue queue_;
     c10::DeviceIndex device_index_;
+    mutable std::recursive_mutex pass_mutex_; // (recursive: a tensor's own dispatch may come back to the module)
 };
 
 /************************************************ENCODING MODULE */
