@@ -851,6 +851,26 @@ def test_a_tangent_is_refused_and_a_failed_call_pushes_again(tcnn):
     assert not torch.equal(before, after)
 
 
+@pytest.mark.parametrize("kind", ["network", "encoding", "field", "frequency"])
+def test_backward_pass_on_no_rows(tcnn, kind):
+    """An empty batch gives zero gradients, as a PyTorch module's does: nothing is raised in either direction."""
+    grid = {"otype": "HashGrid", "type": "Hash", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": 12, "base_resolution": 16, "per_level_scale": 1.5}
+    frequency = {"otype": "Frequency", "n_frequencies": 6}
+    model = {"network": lambda: tcnn.Network(2, 5, net_config(32, 3)), "encoding": lambda: tcnn.Encoding(2, grid),
+             "field": lambda: tcnn.NetworkWithInputEncoding(2, 5, net_config(64, 2), grid),
+             "frequency": lambda: tcnn.NetworkWithInputEncoding(2, 5, net_config(64, 2), frequency)}[kind]()
+    for rows in (0, 16, 0):
+        model.zero_grad()
+        x = torch.rand((rows, 2), device=DEVICE, requires_grad=kind == "network")
+        y = model(x)
+        assert y.shape[0] == rows
+        y.float().sum().backward()
+        trained = [p for p in model.parameters() if p.requires_grad]
+        assert trained and all(p.grad is not None and bool(p.grad.any()) == (rows > 0) for p in trained)
+        if kind == "network":
+            assert x.grad.shape == x.shape
+
+
 @pytest.mark.parametrize("own_streams", [False, True])
 def test_two_threads_on_one_module(tcnn, own_streams):
     """Two Python threads, each with its own batch, on one stream or a stream each, share a field and its encoding. The batches are large

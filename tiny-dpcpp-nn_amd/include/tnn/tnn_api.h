@@ -291,6 +291,7 @@ template <typename T> class EncodingModule : public Module {
     std::tuple<torch::Tensor, torch::Tensor> backward_rows(const torch::Tensor &dy, const RowsPass &pass, double loss_scale, bool,
                                                            const torch::Tensor &params) override {
         if (encoding_->get_n_params() == 0) return {torch::Tensor(), torch::Tensor()};
+        if (pass.input.size(0) == 0) return {torch::Tensor(), torch::zeros_like(params)};
         torch::Tensor g = std::get<1>(backward_pass((loss_scale != 1.0 ? dy * loss_scale : dy).contiguous(), pass.input, false, false));
         if (loss_scale != 1.0) g = g / loss_scale;
         return {torch::Tensor(), g.reshape(params.sizes()).to(params.scalar_type())};
