@@ -559,6 +559,20 @@ static void test_grid(const char *config_text, uint32_t padded_width, size_t M) 
     CHECK(throws<std::invalid_argument>([&] { enc->forward_impl(xd.GetView(), &wrong_view); }, "Dimension mismatch"));
     CHECK(throws<std::invalid_argument>([&] { enc->forward_impl(xd.GetView(), &out_view, true); }, "inference params"));
     CHECK(enc->forward_impl(xd.GetView(), nullptr) == nullptr);
+
+    // a pass that throws keeps nothing of the scratch memory its caller gave it: the next one runs on the encoding's own
+    {
+        const size_t bytes = grid->backward_scratch_bytes(M);
+        DeviceMatrix<char> scratch(bytes, 1, q);
+        CHECK(throws<std::invalid_argument>([&] { grid->backward_with_scratch(xd.GetView(), wrong_view, &grads_view, scratch.data(), bytes); }, "Dimension mismatch"));
+        grid->backward_with_scratch(xd.GetView(), dyd.GetView(), &grads_view, scratch.data(), bytes);
+        q.wait();
+        CHECK(max_norm_rel(grads.copy_to_host(), gref) <= 1e-5);
+        CHECK(throws<std::invalid_argument>([&] { grid->backward_with_scratch(xd.GetView(), wrong_view, &grads_view, scratch.data(), bytes); }, "Dimension mismatch"));
+    }
+    enc->backward_impl(ctx, xd.GetView(), dyd.GetView(), &grads_view);
+    q.wait();
+    CHECK(max_norm_rel(grads.copy_to_host(), gref) <= 1e-5);
 }
 
 static double max_abs_diff(const std::vector<float> &a, const std::vector<float> &b) {

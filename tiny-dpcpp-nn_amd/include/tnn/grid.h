@@ -101,29 +101,18 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
     void backward_impl(const Context &, const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput,
                        DeviceMatrixView<T> *gradients, DeviceMatrix<float> *dL_dinput = nullptr, bool use_inference_params = false,
                        GradientMode param_gradients_mode = GradientMode::Overwrite) override {
-        const size_t batch_size = input.m();
-        if (batch_size == 0) throw std::invalid_argument("batch_size == 0");
-        if (use_inference_params) throw std::invalid_argument("Cannot use inference params.");
-        if (dL_dinput) throw std::invalid_argument("GridEncoding: gradients w.r.t. the input are not supported.");
-        if (param_gradients_mode == GradientMode::Ignore) return;
-        if (!gradients) throw std::invalid_argument("GridEncoding: gradients must not be null.");
-        if (gradients->nelements() != this->get_n_params()) throw std::invalid_argument("GridEncoding: gradients have the wrong size.");
-        if (input.n() != this->get_input_width() || dL_doutput.n() != this->get_padded_output_width() || dL_doutput.m() != batch_size)
-            throw std::invalid_argument("Dimension mismatch grid encoding backward_impl");
-        check_max_level();
-        const size_t need = backward_scratch_bytes(batch_size);
-        void *scratch = m_lent_scratch;
-        size_t scratch_bytes = m_lent_scratch_bytes;
-        if (scratch_bytes < need) {
-            if (!m_scratch || m_scratch->size() * sizeof(float) < need)
-                m_scratch = std::make_unique<DeviceMatrix<float>>((need + sizeof(float) - 1) / sizeof(float), 1, this->get_queue());
-            scratch = m_scratch->data();
-            scratch_bytes = m_scratch->size() * sizeof(float);
-        }
-        tnn::abi_check(tnn_grid_backward_binned(&m_desc, input.GetPointer(), nullptr, dL_doutput.GetPointer(), TNN_FP32,
-                                                this->get_padded_output_width(), gradients->GetPointer(),
-                                                param_gradients_mode == GradientMode::Overwrite ? 1 : 0, batch_size, scratch, scratch_bytes,
-                                                this->get_queue().abi()));
+        if (!check_backward(input, dL_doutput, gradients, dL_dinput, use_inference_params, param_gradients_mode)) return;
+        const size_t need = backward_scratch_bytes(input.m());
+        if (!m_scratch || m_scratch->size() * sizeof(float) < need)
+            m_scratch = std::make_unique<DeviceMatrix<float>>((need + sizeof(float) - 1) / sizeof(float), 1, this->get_queue());
+        run_backward(input, dL_doutput, gradients, m_scratch->data(), m_scratch->size() * sizeof(float), param_gradients_mode);
+    }
+
+    /// backward_impl with the caller's scratch memory (backward_scratch_bytes of it, used until the pass is over on the stream).
+    void backward_with_scratch(const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput, DeviceMatrixView<T> *gradients, void *scratch,
+                               const size_t scratch_bytes, GradientMode param_gradients_mode = GradientMode::Overwrite) {
+        if (check_backward(input, dL_doutput, gradients, nullptr, false, param_gradients_mode))
+            run_backward(input, dL_doutput, gradients, scratch, scratch_bytes, param_gradients_mode);
     }
 
     uint32_t n_pos_dims() const override { return m_desc.n_dims; }
@@ -141,13 +130,29 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
     const tnn_grid_desc &descriptor() const { return m_desc; }
     uint32_t n_levels() const { return m_desc.n_levels; }
     size_t backward_scratch_bytes(const size_t batch_size) const { return tnn_grid_backward_workspace_bytes(&m_desc, batch_size); }
-    /// Memory for the backward passes from now on, instead of their own; (nullptr, 0) takes it back.
-    void lend_scratch(void *scratch, const size_t bytes) {
-        m_lent_scratch = scratch;
-        m_lent_scratch_bytes = bytes;
-    }
 
   private:
+    /// Whether there is anything to do; throws where the arguments do not fit.
+    bool check_backward(const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput, const DeviceMatrixView<T> *gradients,
+                        const DeviceMatrix<float> *dL_dinput, bool use_inference_params, GradientMode param_gradients_mode) const {
+        if (input.m() == 0) throw std::invalid_argument("batch_size == 0");
+        if (use_inference_params) throw std::invalid_argument("Cannot use inference params.");
+        if (dL_dinput) throw std::invalid_argument("GridEncoding: gradients w.r.t. the input are not supported.");
+        if (param_gradients_mode == GradientMode::Ignore) return false;
+        if (!gradients) throw std::invalid_argument("GridEncoding: gradients must not be null.");
+        if (gradients->nelements() != this->get_n_params()) throw std::invalid_argument("GridEncoding: gradients have the wrong size.");
+        if (input.n() != this->get_input_width() || dL_doutput.n() != this->get_padded_output_width() || dL_doutput.m() != input.m())
+            throw std::invalid_argument("Dimension mismatch grid encoding backward_impl");
+        check_max_level();
+        return true;
+    }
+    void run_backward(const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput, DeviceMatrixView<T> *gradients, void *scratch,
+                      const size_t scratch_bytes, GradientMode param_gradients_mode) {
+        tnn::abi_check(tnn_grid_backward_binned(&m_desc, input.GetPointer(), nullptr, dL_doutput.GetPointer(), TNN_FP32,
+                                                this->get_padded_output_width(), gradients->GetPointer(),
+                                                param_gradients_mode == GradientMode::Overwrite ? 1 : 0, input.m(), scratch, scratch_bytes,
+                                                this->get_queue().abi()));
+    }
     void check_max_level() const {
         if (this->m_max_level < (float)m_desc.n_levels) throw std::invalid_argument("GridEncoding: max_level below the level count is not supported.");
     }
@@ -158,9 +163,7 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
 
     tnn_grid_desc m_desc;
     std::unique_ptr<DeviceMatrix<float>> m_order; // records of the last large batch in cell order
-    std::unique_ptr<DeviceMatrix<float>> m_scratch; // what the backward pass sorts its contributions into, when none is lent; only grows
-    void *m_lent_scratch = nullptr;
-    size_t m_lent_scratch_bytes = 0;
+    std::unique_ptr<DeviceMatrix<float>> m_scratch; // what backward_impl sorts its contributions into; only grows
     uint32_t m_n_features;
     uint32_t m_n_features_per_level;
     GridOffsetTable m_offset_table;

@@ -270,13 +270,12 @@ template <typename T> class EncodingModule : public Module {
         DeviceMatrixView<T> gradients_view(encoding_->get_n_params(), 1, 1, reinterpret_cast<T *>(last_gradients_.data_ptr()));
         Context ctx;
         auto *grid = dynamic_cast<tinydpcppnn::encodings::grid::GridEncodingTemplated<T> *>(encoding_.get());
-        torch::Tensor lent;
-        if (grid) {
-            lent = this->scratch(grid->backward_scratch_bytes((size_t)batch_size));
-            grid->lend_scratch(lent.data_ptr(), (size_t)lent.numel());
+        if (auto *grid = dynamic_cast<tinydpcppnn::encodings::grid::GridEncodingTemplated<T> *>(encoding_.get())) {
+            const torch::Tensor work = this->scratch(grid->backward_scratch_bytes((size_t)batch_size));
+            grid->backward_with_scratch(input_encoding_dmv, dL_doutput_dmv, &gradients_view, work.data_ptr(), (size_t)work.numel());
+        } else {
+            encoding_->backward_impl(ctx, input_encoding_dmv, dL_doutput_dmv, &gradients_view);
         }
-        encoding_->backward_impl(ctx, input_encoding_dmv, dL_doutput_dmv, &gradients_view);
-        if (grid) grid->lend_scratch(nullptr, 0);
         this->finish();
         return {torch::Tensor(), last_gradients_};
     }
