@@ -871,6 +871,34 @@ def test_backward_pass_on_no_rows(tcnn, kind):
             assert x.grad.shape == x.shape
 
 
+@pytest.mark.parametrize("with_gradients", [True, False])
+@pytest.mark.parametrize("kind", ["network", "encoding", "field", "frequency"])
+def test_a_trace_replays_the_module(tcnn, kind, with_gradients):
+    """torch.jit.trace records a module's call: replayed on other rows (another number of them, none among them) and after the parameters
+    have changed, the program gives the module's values, and its gradients."""
+    grid = {"otype": "HashGrid", "type": "Hash", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": 12, "base_resolution": 16, "per_level_scale": 1.5}
+    frequency = {"otype": "Frequency", "n_frequencies": 6}
+    model = {"network": lambda: tcnn.Network(2, 5, net_config(32, 3)), "encoding": lambda: tcnn.Encoding(2, grid),
+             "field": lambda: tcnn.NetworkWithInputEncoding(2, 5, net_config(64, 2), grid),
+             "frequency": lambda: tcnn.NetworkWithInputEncoding(2, 5, net_config(64, 2), frequency)}[kind]()
+    if kind in ("encoding", "field"):
+        with torch.no_grad():
+            next(p for n, p in model.named_parameters() if kind == "encoding" or "encoding" in n).normal_(0, 0.1)
+    trained = [p for p in model.parameters() if p.requires_grad]
+    with torch.set_grad_enabled(with_gradients):
+        program = torch.jit.trace(model, torch.rand((64, 2), device=DEVICE))
+        for rows in (64, 13, 0, 200):
+            x = torch.rand((rows, 2), device=DEVICE, requires_grad=kind == "network" and with_gradients)
+            with torch.no_grad():
+                trained[0].mul_(0.9)
+            y, z = model(x), program(x)
+            assert y.shape == z.shape and torch.equal(y, z)
+            if with_gradients and rows:
+                dy, wrt = torch.randn_like(y), trained + ([x] if x.requires_grad else [])
+                for a, b in zip(torch.autograd.grad(y, wrt, dy), torch.autograd.grad(z, wrt, dy)):
+                    assert bool(a.any()) and float((a - b).abs().max()) <= 1e-5 * float(a.abs().max())  # a table's: sums in no fixed order
+
+
 @pytest.mark.parametrize("own_streams", [False, True])
 def test_two_threads_on_one_module(tcnn, own_streams):
     """Two Python threads, each with its own batch, on one stream or a stream each, share a field and its encoding. The batches are large

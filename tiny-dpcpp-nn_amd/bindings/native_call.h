@@ -5,6 +5,7 @@
 // part of them (tnn::Module::forward_rows / backward_rows).
 #pragma once
 
+#include <ATen/TracerMode.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
@@ -83,9 +84,11 @@ inline void refuse_tangents(std::initializer_list<torch::Tensor> inputs) {
         TORCH_CHECK_NOT_IMPLEMENTED(!torch::autograd::isFwGradDefined(t), "tiny_dpcpp_nn modules have no forward-mode derivative");
 }
 
-/// y = module(x), recorded for autograd when that is on and anything asks for gradients.
-inline torch::Tensor call(const std::shared_ptr<tnn::Module> &module, const torch::Tensor &x, const torch::Tensor &params, bool push, bool training,
+/// y = module(x), recorded for autograd when that is on and anything asks for gradients. Nothing while torch.jit.trace records: it
+/// sees PyTorch's operators, of a call here the allocation of the result alone (modules.py then makes the call an operator).
+inline std::optional<torch::Tensor> call(const std::shared_ptr<tnn::Module> &module, const torch::Tensor &x, const torch::Tensor &params, bool push, bool training,
                           double loss_scale) {
+    if (at::tracer::impl::is_dispatch_enabled()) return std::nullopt;
     refuse_tangents({x, params});
     const torch::Tensor in = module->input_rows(x); // (PyTorch operations where any are needed: autograd sees them)
     const bool record = torch::autograd::compute_requires_grad(in, params);
@@ -109,9 +112,11 @@ inline torch::Tensor call(const std::shared_ptr<tnn::Module> &module, const torc
     return y;
 }
 
-/// y = network(encoding(positions)) for a pair that can_train_with_encoding (or, without autograd, can_fuse_encoding) accepts.
-inline torch::Tensor call_with_encoding(const std::shared_ptr<tnn::Module> &network, const std::shared_ptr<tnn::Module> &encoding, const torch::Tensor &x,
+/// y = network(encoding(positions)) for a pair that can_train_with_encoding (or, without autograd, can_fuse_encoding) accepts. Nothing
+/// for no positions, and while torch.jit.trace records.
+inline std::optional<torch::Tensor> call_with_encoding(const std::shared_ptr<tnn::Module> &network, const std::shared_ptr<tnn::Module> &encoding, const torch::Tensor &x,
                                         const torch::Tensor &params, const torch::Tensor &table, bool push_network, bool push_table, double loss_scale) {
+    if (at::tracer::impl::is_dispatch_enabled() || (x.dim() > 0 && x.size(0) == 0)) return std::nullopt;
     refuse_tangents({x, params, table});
     const torch::Tensor positions = x.detach().to(torch::kFloat32).contiguous();
     const bool record = torch::autograd::compute_requires_grad(params, table);

@@ -82,11 +82,11 @@ class PybindingModule {
         return m_module->backward_with_encoding(*encoding.m_module, positions, grad_output, pack_gradient, positions_unchanged_since_forward);
     }
     /// The module as an operator: parameters pushed (on request), forward pass, and a node of the autograd graph.
-    torch::Tensor call(const torch::Tensor &x, const torch::Tensor &params, bool push, bool training, double loss_scale) const {
+    std::optional<torch::Tensor> call(const torch::Tensor &x, const torch::Tensor &params, bool push, bool training, double loss_scale) const {
         return tnn_binding::call(m_module, x, params, push, training, loss_scale);
     }
-    torch::Tensor call_with_encoding(const PybindingModule &encoding, const torch::Tensor &x, const torch::Tensor &params, const torch::Tensor &table,
-                                     bool push_network, bool push_table, double loss_scale) const {
+    std::optional<torch::Tensor> call_with_encoding(const PybindingModule &encoding, const torch::Tensor &x, const torch::Tensor &params,
+                                                    const torch::Tensor &table, bool push_network, bool push_table, double loss_scale) const {
         return tnn_binding::call_with_encoding(m_module, encoding.m_module, x, params, table, push_network, push_table, loss_scale);
     }
     torch::Tensor initial_params() {

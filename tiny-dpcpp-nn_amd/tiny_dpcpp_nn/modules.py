@@ -67,6 +67,37 @@ def from_packed_layout_coord(idx, rows, cols):
     return (2 * pair + (within & 1)) * cols + within // 2
 
 
+class _RecordedCall(torch.autograd.Function):
+    """A module's call as torch.jit.trace can record it: one operator, which calls the module again when the trace is replayed."""
+
+    @staticmethod
+    def forward(ctx, owner, x, *params):
+        recorder = torch._C._get_tracing_state()  # None when a trace is replayed
+        torch._C._set_tracing_state(None)  # what the call consists of is not recorded
+        try:
+            with torch.set_grad_enabled(any(ctx.needs_input_grad)):
+                x = x.detach().requires_grad_(ctx.needs_input_grad[1])
+                y = owner.forward(x)
+            ctx.inner = (x, *params), y
+            shape, values = tuple(y.shape), y.data
+        finally:
+            torch._C._set_tracing_state(recorder)
+        if recorder is None:
+            return values
+        result = torch.empty(shape, dtype=values.dtype, device=values.device)  # (a tensor the recorder knows)
+        torch._C._set_tracing_state(None)
+        result.copy_(values)
+        torch._C._set_tracing_state(recorder)
+        return result
+
+    @staticmethod
+    def backward(ctx, dy):
+        inputs, y = ctx.inner
+        wanted = [t for t, needed in zip(inputs, ctx.needs_input_grad[1:]) if needed]
+        grads = iter(torch.autograd.grad(y, wanted, dy, retain_graph=True, allow_unused=True))
+        return (None, *(next(grads) if needed else None for needed in ctx.needs_input_grad[1:]))
+
+
 class Module(torch.nn.Module):
     """Base of the three front-end classes: owns the native module (`tnn_module`) and the PyTorch-side parameter tensor
     `params` (fp32 when `store_params_as_full_precision`, else the module's dtype; a network's is in the packed layout)."""
@@ -144,6 +175,8 @@ class Module(torch.nn.Module):
     def forward(self, x):
         # one entry into the native module: push, padding and conversion, the pass, and its node in the autograd graph
         y = self.tnn_module.call(x, self.params, self._must_push(), self.training, self.loss_scale)
+        if y is None:  # torch.jit.trace is recording
+            return _RecordedCall.apply(self, x, self.params)
         self._has_pushed()
         return y
 
@@ -226,12 +259,14 @@ class NetworkWithInputEncoding(Module):
         network, encoding = self.network, self.encoding
         if self._fused is None:  # (fixed once the two native modules exist)
             self._fused = (network.tnn_module.can_fuse_encoding(encoding.tnn_module), network.tnn_module.can_train_with_encoding(encoding.tnn_module))
-        if x.shape[0] == 0 or not self._fused[torch.is_grad_enabled()]:
+        if not self._fused[torch.is_grad_enabled()]:
             return self.network_with_encoding(x)
         # a grid encoding and its network as one kernel (backward: one kernel plus the scatter), with the values of the two
         # modules in turn, the reference's only route; the encoded matrix is never stored
         y = network.tnn_module.call_with_encoding(encoding.tnn_module, x, network.params, encoding.params, network._must_push(), encoding._must_push(),
                                                   network.loss_scale)
+        if y is None:
+            return _RecordedCall.apply(self, x, network.params, encoding.params) if torch.jit.is_tracing() else self.network_with_encoding(x)
         network._has_pushed()
         encoding._has_pushed()
         return y
