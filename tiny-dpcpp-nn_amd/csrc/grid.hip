@@ -533,12 +533,11 @@ __global__ void __launch_bounds__(kBwdThreads)
     }
 }
 
-__global__ void fill_zero_kernel(float4 *__restrict__ p, size_t n4, float *__restrict__ tail, size_t n_tail, uint32_t *__restrict__ words, size_t n_words) {
+__global__ void fill_zero_kernel(float4 *__restrict__ p, size_t n4, float *__restrict__ tail, size_t n_tail) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t k = i; k < n4; k += stride) p[k] = float4{0.f, 0.f, 0.f, 0.f};
     if (i < n_tail) tail[i] = 0.0f;
-    for (size_t k = i; k < n_words; k += stride) words[k] = 0;
 }
 
 int check_grid_desc(const tnn_grid_desc *d) {
@@ -842,23 +841,22 @@ int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4
     uintptr_t scratch = (reinterpret_cast<uintptr_t>(d_workspace) + 255) & ~(uintptr_t)255;
     const bool binned = d_workspace && grad_dtype == TNN_FP32;
     BackwardPlan bp = plan_backward(lv, gp, desc->n_dims, n_features, d_order != nullptr, grad_dtype == TNN_FP32, M, binned ? &bins : nullptr, &n_big, &lds_bytes);
-    if (bins.n_levels && workspace_bytes < bin_scratch_bytes(bins, n_features) + (scratch - reinterpret_cast<uintptr_t>(d_workspace)))
-        return fail(TNN_ERR_WORKSPACE, "grid backward: workspace of %zu bytes given, %zu needed", workspace_bytes, bin_scratch_bytes(bins, n_features) + 256);
+    if (bins.n_levels && workspace_bytes < bin_scratch_bytes(bins, desc->n_dims, n_features) + (scratch - reinterpret_cast<uintptr_t>(d_workspace)))
+        return fail(TNN_ERR_WORKSPACE, "grid backward: workspace of %zu bytes given, %zu needed", workspace_bytes, bin_scratch_bytes(bins, desc->n_dims, n_features) + 256);
     if (overwrite && (reinterpret_cast<uintptr_t>(d_grad_table) & 15)) return fail(TNN_ERR_INVALID_ARGUMENT, "d_grad_table must be 16-byte aligned");
     // The binned levels are written whole: where they are the last ones, as the finest are, only what lies in front of them is cleared.
     size_t entries = overwrite ? desc->offsets[desc->n_levels] : 0;
     if (bins.n_levels && bins.level[0] + bins.n_levels == desc->n_levels) entries = std::min<size_t>(entries, desc->offsets[bins.level[0]]);
-    if (entries || bins.n_levels) {
+    if (entries) {
         // a fill kernel rather than a memset node, so the call can be captured into a HIP graph
         const size_t bytes = entries * n_features * (grad_dtype == TNN_FP32 ? sizeof(float) : sizeof(fp16_t));
         const size_t n4 = bytes / 16;
         const size_t n_tail = (bytes - n4 * 16) / sizeof(float); // level sizes are multiples of 8 entries: fp16 tables leave no tail
-        const uint32_t n_words = bins.n_bins;
-        size_t blocks = (std::max<size_t>(n4, n_words) + 255) / 256;
+        size_t blocks = (n4 + 255) / 256;
         if (blocks > 4096) blocks = 4096;
         if (blocks < 4) blocks = 4;
         TNN_LAUNCH(fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (float4 *)d_grad_table, n4,
-                   reinterpret_cast<float *>(static_cast<char *>(d_grad_table) + n4 * 16), n_tail, reinterpret_cast<uint32_t *>(scratch), n_words);
+                   reinterpret_cast<float *>(static_cast<char *>(d_grad_table) + n4 * 16), n_tail);
         if ((rc = check_launch("fill_zero_kernel"))) return rc;
     }
     const GradLayout dl{padded_width, n_features, by_position ? 1 : 0, scale};
@@ -904,7 +902,7 @@ TNN_API size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size
         BinPlan bins{};
         uint32_t n_big, lds;
         (void)plan_backward(lv, gp, desc->n_dims, desc->n_features_per_level, ordered, true, M, &bins, &n_big, &lds);
-        most = std::max(most, bin_scratch_bytes(bins, desc->n_features_per_level));
+        most = std::max(most, bin_scratch_bytes(bins, desc->n_dims, desc->n_features_per_level));
     }
     return most + 256;
 }

@@ -17,17 +17,14 @@ struct BinPlan {
     uint8_t run_log2[kMaxBinned];
     uint16_t places[kMaxBinned];       // entries a bin has room for
     uint32_t first_bin[kMaxBinned + 1]; // bins of the levels in front of this one
-    uint32_t capacity[kMaxBinned];     // records a bin has room for
-    uint32_t first_record[kMaxBinned]; // of the level's first bin
-    uint32_t n_records;                // room for all bins
     uint32_t slice_lds;                // LDS bytes of the largest slice
     uint32_t batch;                    // points binned at a time
 };
 
 // Adds level l to the plan if it can take the route.
 bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams &gp, uint32_t n_dims, uint32_t n_features, size_t M);
-size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_features);
-// The first p.n_bins words of the scratch have to be zero when the kernels start. With `overwrite` every entry of the plan's levels
+size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_dims, uint32_t n_features);
+// Nothing in the scratch has to be cleared. With `overwrite` every entry of the plan's levels
 // is written, whatever it held.
 int launch_grid_binned(const BinPlan &p, const GridLevels &lv, const GridParams &gp, const GradLayout &dl, uint32_t n_dims, uint32_t n_features, const float *x,
                        const float4 *order, const void *dLdy, int dy_dtype, float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s);

@@ -4,17 +4,22 @@
 // The memory side retires an atomic request per 32-byte sector, about 20 * 10^9 a second, and a point of a hashed level
 // needs 2^(D-1) or more of them: 2.1 ms for 2^20 points of a 3-D grid of 16 levels (2^19 entries). Here the contributions
 // are sorted by destination first:
-//   1. grid_bin_kernel deals runs of a level's entries out to bins and writes every contribution as a record into its
-//      bin. The two corners along the first dimension are neighbouring entries in a dense level and differ in the low bits
-//      of the index in a coherently hashed one, so nearly always they share a bin and travel as one record of two entries.
-//      (Long runs make long stores; but a hashed level's runs longer than its x range are dealt out by the other
+//   1. grid_bin_kernel deals runs of a level's entries out to bins. A workgroup sorts the contributions of a stretch of points by
+//      bin in LDS and writes them as one piece of consecutive records, with a table of where each bin's begin. The two corners
+//      along the first dimension are neighbouring entries in a dense level and differ in the low bits of the index in a
+//      coherently hashed one, so nearly always they share a bin and travel as one record of two entries.
+//      (Long runs of entries share more; but a hashed level's runs longer than its x range are dealt out by the other
 //      dimensions alone, and in 2-D the few hundred values of y fill the bins very unevenly: bin_plan_add.)
-//   2. grid_bin_sum_kernel takes a bin at a time, sums its records into a copy of the bin's entries in LDS and writes the
-//      entries to the table as whole lines.
+//   2. grid_bin_sum_kernel takes a bin at a time, sums its records of all pieces into a copy of the bin's entries in LDS and
+//      writes the entries to the table as whole lines.
 // A record of two features is 16 bytes written once and read once, where the two atomic requests it replaces occupy the
-// memory side for 64.
-// Measured, 2^20 points, 3-D, 2^19 entries, 15 levels this way: 2 x (164 + 172) us, 3 TB/s of records both ways; before, the
-// atomics of the ten finest of these levels alone took 1.5 ms.
+// memory side for 64. A piece has room for whatever its points need, so no bin can be too full: points that crowd a few cells
+// make some bins longer than others, and that is all. (Bins of a fixed size, filled by all workgroups through shared cursors, are
+// as fast for points spread evenly, but what finds no room has to go elsewhere. 2^20 points, 3-D, 2^19 entries, whole scatter, from
+// points in the inner 90 % of the cube / in a cube of 5 % of the side: the overfull bins summed from the points 4.0 / 5.8 ms, the surplus
+// added with atomics 0.76 / 36 ms, pieces 0.75 / 3.9 ms; evenly spread 0.74, 0.76 and 0.75 ms.)
+// Measured, 2^20 points, 3-D, 2^19 entries, 15 levels this way: 2 x (161 + 184) us; before, the atomics of the ten finest of these
+// levels alone took 1.5 ms.
 #include "grid_binned.h"
 
 #include <algorithm>
@@ -23,10 +28,13 @@
 namespace tnn {
 
 constexpr int kBinSumThreads = 1024; // at most
+constexpr uint32_t kBinSumGroup = 8;    // lanes that walk through a share of a bin's records together
+constexpr int kBinPiecesEach = 4;        // pieces a thread of the sums looks up, at most
+constexpr uint32_t kBinNeighbours = 16;  // consecutive bins on an XCD
+constexpr uint32_t kBinPiecePad = 144; // records between two pieces, so that workgroups in step do not all write to the same channels
 
-// A binning workgroup: its threads (at most), the points of a thread, and the most records it sorts in LDS. 2048 records of 16
+// A binning workgroup: its threads (at most), the points of a thread, and the pairs of corners it sorts in LDS. 2048 records of 16
 // bytes let four workgroups of 8 waves share a CU, whose phases (loads, LDS, stores) then overlap; wider records take half as many.
-// (3-D, 2^19 points, 15 levels of two features: 164 us; 4096 records 177, 1024 184.)
 template <int D, int F> struct BinShape {
     static constexpr int kThreads = F <= 2 ? 512 : 256;
     static constexpr int kPoints = D == 2 && F <= 2 ? 2 : 1;
@@ -34,13 +42,16 @@ template <int D, int F> struct BinShape {
     static constexpr int kRecords = kThreads * kPoints * kPairs;
 };
 
-// Entry e of a level: its bin and its place there.
+// Entry e of a level: its bin and its place there. Runs of 2^run_log2 entries go to the bins in turn, every round of them starting
+// at another bin: a region of a dense level then meets all bins about equally, also where a row of the level is a multiple of a round.
 struct Bins {
     uint32_t n_log2, run_log2;
-    __device__ __forceinline__ uint32_t bin(uint32_t e) const { return (e >> run_log2) & ((1u << n_log2) - 1); }
+    __device__ __forceinline__ uint32_t turn(uint32_t round) const { return (round * 2654435769u) >> 22; }
+    __device__ __forceinline__ uint32_t bin(uint32_t e) const { return ((e >> run_log2) + turn(e >> (run_log2 + n_log2))) & ((1u << n_log2) - 1); }
     __device__ __forceinline__ uint32_t place(uint32_t e) const { return ((e >> (run_log2 + n_log2)) << run_log2) | (e & ((1u << run_log2) - 1)); }
     __device__ __forceinline__ uint32_t entry(uint32_t bin, uint32_t place) const {
-        return ((((place >> run_log2) << n_log2) | bin) << run_log2) | (place & ((1u << run_log2) - 1));
+        const uint32_t round = place >> run_log2, run = (bin - turn(round)) & ((1u << n_log2) - 1);
+        return (((round << n_log2) | run) << run_log2) | (place & ((1u << run_log2) - 1));
     }
 };
 
@@ -50,9 +61,6 @@ template <int F> struct alignas(F == 1 ? 4 : F == 2 ? 16 : 8) BinRecord {
     float frac;
     float g[F];
 };
-
-template <int F> static size_t record_bytes_of() { return sizeof(BinRecord<F>); }
-static size_t record_bytes(uint32_t F) { return F == 1 ? record_bytes_of<1>() : F == 2 ? record_bytes_of<2>() : F == 4 ? record_bytes_of<4>() : record_bytes_of<8>(); }
 
 template <int D>
 __device__ __forceinline__ long long bin_point(const float *__restrict__ xin, const float4 *__restrict__ order, long long i, float (&x)[D]) {
@@ -97,39 +105,60 @@ __device__ __forceinline__ void pair_entries(const uint32_t (&cell)[D], uint32_t
     }
 }
 
+// What the threads of a workgroup in front of this one have, and what all have. WAVES: room in wave_sum.
+template <int WAVES> __device__ __forceinline__ uint32_t running_sum(uint32_t mine, uint32_t *__restrict__ wave_sum, uint32_t &total) {
+    // of the wave's lanes up to this one: rows of 16 lanes first (DPP row_shr), then the last lane of a row to the rows above
+    uint32_t upto = mine;
+    upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x111, 0xf, 0xf, true);
+    upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x112, 0xf, 0xf, true);
+    upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x114, 0xf, 0xf, true);
+    upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x118, 0xf, 0xf, true);
+    upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
+    upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
+    if ((threadIdx.x & 63) == 63) wave_sum[threadIdx.x >> 6] = upto;
+    __syncthreads();
+    uint32_t before = upto - mine;
+    total = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < WAVES; ++w) {
+        const uint32_t sum = w < blockDim.x / 64 ? wave_sum[w] : 0u;
+        if (w < threadIdx.x >> 6) before += sum;
+        total += sum;
+    }
+    return before;
+}
+
 // One workgroup bins kPoints points a thread of one level: it counts its records per bin, which gives every record its place among
-// them, reserves that much of every bin with one atomic, sorts the records by bin in LDS and writes them from there, so that a
-// wave stores whole runs: neighbouring lanes, neighbouring records. Bound by the records' bytes on their way to memory, 3.0 TB/s
-// at 12, 16, 24 and 40 bytes a record. (Every lane storing its own records, as many L2 requests as records times pieces of 16
-// bytes: four features 166 -> 133 us, eight 138 -> 119, one 36 -> 27, two as fast either way, 3-D or 2-D, 2^18 points.) The levels of the same points are consecutive workgroups of one
-// XCD, which shares the rows of dL/dy between them in its L2.
-// Records beyond a bin's capacity are counted and dropped.
+// them, sorts the records in LDS and writes them to its piece of the scratch, so that a wave stores whole lines. A far side that
+// lies in another bin than the near side is a record of its own; LDS has room for one in eight, those beyond go to the
+// piece directly. The levels of the same points are consecutive workgroups of one XCD, which shares the rows of dL/dy between
+// them in its L2.
+// No one unit bounds it (3-D, 2^19 points, 15 levels, 161 us): 507 MB written, all in whole 64-byte requests, at 3.1 TB/s where a
+// fill reaches 6.9; the vector units are at work half of the time, LDS a quarter, and a wave waits for 43 % of its.
 template <int D, int F, typename G>
 __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
     grid_bin_kernel(const GridLevels lv, const GridParams gp, const BinPlan bp, const GradLayout dl, const float *__restrict__ xin,
-                    const float4 *__restrict__ order, const G *__restrict__ dLdy, uint32_t *__restrict__ cursors, BinRecord<F> *__restrict__ records,
-                    long long first, long long last) {
+                    const float4 *__restrict__ order, const G *__restrict__ dLdy, uint16_t *__restrict__ offsets, BinRecord<F> *__restrict__ records,
+                    long long first, long long last, uint32_t n_stretches, uint32_t pitch, uint32_t room) {
     typedef BinShape<D, F> S;
     constexpr int NP = S::kPairs, P = S::kPoints;
     static_assert(S::kRecords <= 4096 && kBinMaxBins <= 1024, "a record's place is packed into 12 + 10 + 10 bits");
-    const int T = blockDim.x;
+    const uint32_t T = blockDim.x;
     extern __shared__ __align__(16) unsigned char bin_smem[];
     BinRecord<F> *const sorted = reinterpret_cast<BinRecord<F> *>(bin_smem);
-    uint16_t *const bin_of = reinterpret_cast<uint16_t *>(sorted + T * P * NP); // of a sorted record
-    uint32_t *const base = reinterpret_cast<uint32_t *>(bin_of + T * P * NP);    // records per bin, then the first sorted one of them
-    const uint32_t turn = blockIdx.x / 8, k = turn % bp.n_levels, per_wg = T * P;
-    const long long begin = first + (long long)((turn / bp.n_levels) * 8 + blockIdx.x % 8) * per_wg;
-    if (begin >= last) return;
-    const long long end = begin + per_wg < last ? begin + per_wg : last;
+    uint32_t *const base = reinterpret_cast<uint32_t *>(sorted + room); // records per bin, then the place of the bin's first one
+    const uint32_t turn = blockIdx.x / 8, k = turn % bp.n_levels, stretch = (turn / bp.n_levels) * 8 + blockIdx.x % 8;
+    if (stretch >= n_stretches) return;
+    const long long begin = first + (long long)stretch * (T * P);
+    const long long end = begin + T * P < last ? begin + T * P : last;
     const Bins dealt{bp.bins_log2[k], bp.run_log2[k]};
     const uint32_t l = bp.level[k], n_bins = 1u << dealt.n_log2;
-    uint32_t *const split = base + n_bins; // records per bin of far sides that lie in another bin than the near side, then the next place of one
-    uint32_t *const shift = split + n_bins; // place in the bin less place among the sorted records
-    uint32_t *const wave_sum = shift + n_bins;
-    const uint32_t size = lv.size[l], res = lv.resolution[l], flags = lv.flags[l], capacity = bp.capacity[k];
+    uint32_t *const split = base + n_bins; // the same for far sides in another bin, then the place of the next of them
+    uint32_t *const wave_sum = split + n_bins;
+    const uint32_t size = lv.size[l], res = lv.resolution[l], flags = lv.flags[l];
     const float scale = lv.scale[l];
-    uint32_t *const cursor = cursors + bp.first_bin[k];
-    BinRecord<F> *const bins = records + bp.first_record[k];
+    uint16_t *const begins = offsets + (size_t)stretch * (bp.n_bins + bp.n_levels) + bp.first_bin[k] + k;
+    BinRecord<F> *const piece = records + ((size_t)k * n_stretches + stretch) * pitch;
 
     for (uint32_t b = threadIdx.x; b < n_bins; b += T) base[b] = split[b] = 0;
     __syncthreads();
@@ -156,41 +185,28 @@ __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
         }
     }
     __syncthreads();
-    // A running sum over the bins' counts, `each` neighbouring bins a thread (at most 1024 bins over at least 128 threads).
-    constexpr int kEach = 8;
+    constexpr int kEach = 8; // neighbouring bins of a thread, at most (1024 bins, 128 threads)
     const uint32_t each = (n_bins + T - 1) / T, b0 = threadIdx.x * each;
-    uint32_t count[kEach], mine = 0;
+    uint32_t count[kEach], apart[kEach], mine = 0, total;
 #pragma unroll
     for (int e = 0; e < kEach; ++e) {
-        count[e] = (uint32_t)e < each && b0 + e < n_bins ? base[b0 + e] : 0u;
-        mine += count[e];
+        const bool any = (uint32_t)e < each && b0 + e < n_bins;
+        count[e] = any ? base[b0 + e] : 0u;
+        apart[e] = any ? split[b0 + e] : 0u;
+        mine += count[e] + apart[e];
     }
-    uint32_t upto = mine; // of the wave's lanes up to this one
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t below = __shfl_up(upto, off, 64);
-        if ((int)(threadIdx.x & 63) >= off) upto += below;
-    }
-    if ((threadIdx.x & 63) == 63) wave_sum[threadIdx.x >> 6] = upto;
-    __syncthreads();
-    uint32_t at = upto - mine, total = 0;
-    for (int w = 0; w < T / 64; ++w) {
-        const uint32_t sum = wave_sum[w];
-        if (w < (int)(threadIdx.x >> 6)) at += sum;
-        total += sum;
-    }
+    uint32_t at = running_sum<S::kThreads / 64>(mine, wave_sum, total);
 #pragma unroll
     for (int e = 0; e < kEach; ++e) {
         const uint32_t b = b0 + e;
         if ((uint32_t)e < each && b < n_bins) {
-            const uint32_t n_split = split[b];
-            const uint32_t reserved = count[e] + n_split ? atomicAdd(&cursor[b], count[e] + n_split) : 0u;
+            begins[b] = (uint16_t)at;
             base[b] = at;
-            shift[b] = reserved - at;
-            split[b] = reserved + count[e];
-            at += count[e];
+            split[b] = at + count[e];
+            at += count[e] + apart[e];
         }
     }
+    if (threadIdx.x == 0) begins[n_bins] = (uint16_t)total;
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < P; ++u) {
@@ -204,105 +220,131 @@ __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
             r.frac = frac[u][0];
 #pragma unroll
             for (int f = 0; f < F; ++f) r.g[f] = weight * gy[u][f];
-            const uint32_t bin = (place[u][c] >> 12) & 1023u, far_bin = place[u][c] >> 22, slot = base[bin] + (place[u][c] & 4095u);
-            r.where = where[u][c] | ((far_bin == bin ? 3u : 1u) << 30);
-            sorted[slot] = r;
-            bin_of[slot] = (uint16_t)bin;
-            if (far_bin != bin) {
-                r.where = where[u][c] | (2u << 30);
-                const uint32_t to = atomicAdd(&split[far_bin], 1u);
-                if (to < capacity) bins[(size_t)far_bin * capacity + to] = r;
-            }
+            const uint32_t bin = (place[u][c] >> 12) & 1023u, far_bin = place[u][c] >> 22;
+            const auto put = [&](uint32_t to, uint32_t sides) {
+                r.where = where[u][c] | (sides << 30);
+                if (to < room) sorted[to] = r;
+                else piece[to] = r;
+            };
+            put(base[bin] + (place[u][c] & 4095u), far_bin == bin ? 3u : 1u);
+            if (far_bin != bin) put(atomicAdd(&split[far_bin], 1u), 2u);
         }
     }
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < total; i += T) {
-        const uint32_t bin = bin_of[i], to = shift[bin] + i;
-        if (to < capacity) bins[(size_t)bin * capacity + to] = sorted[i];
-    }
+    const uint32_t staged = total < room ? total : room;
+    for (uint32_t i = threadIdx.x; i < staged; i += T) piece[i] = sorted[i];
 }
 
-// LDS of it with T threads.
-template <int D, int F> static size_t bin_lds(const BinPlan &p, unsigned T) {
-    uint32_t n_bins = 0;
-    for (uint32_t k = 0; k < p.n_levels; ++k) n_bins = std::max(n_bins, 1u << p.bins_log2[k]);
-    return (size_t)T * BinShape<D, F>::kPoints * BinShape<D, F>::kPairs * (sizeof(BinRecord<F>) + sizeof(uint16_t)) + (3 * n_bins + 16) * sizeof(uint32_t);
-}
-
-// One workgroup sums one bin and stores (or adds) its entries. Bound by the records' bytes and the LDS atomics (two values of two
-// features per record). A bin that more records were meant for than it has room for is summed from the points instead, all of them
-// passing its workgroup by. The bin's cursor is left at zero for the next part of the batch.
-template <int D, int F, typename G>
+// One workgroup sums one bin and stores (or adds) its entries. Bound by the LDS atomics, two entries of F values a record: LDS is at
+// work 72 % of the time (3-D, 2^19 points, 15 levels, 184 us; 163 with the records read and not added). The bin's runs of records in the pieces follow each other here (`first`: records in front of a piece's run);
+// sixteen lanes take an equal share of them all, whatever the runs' lengths, and walk from run to run. Neighbouring bins, whose
+// runs share lines, are workgroups of one XCD, sixteen at a time.
+template <int F>
 __global__ void __launch_bounds__(kBinSumThreads)
-    grid_bin_sum_kernel(const GridLevels lv, const GridParams gp, const BinPlan bp, const GradLayout dl, const float *__restrict__ xin,
-                        const float4 *__restrict__ order, const G *__restrict__ dLdy, uint32_t *__restrict__ cursors,
-                        const BinRecord<F> *__restrict__ records, float *__restrict__ grad, long long first, long long last, int store) {
+    grid_bin_sum_kernel(const GridLevels lv, const BinPlan bp, const uint16_t *__restrict__ offsets, const BinRecord<F> *__restrict__ records,
+                        float *__restrict__ grad, uint32_t n_stretches, uint32_t pitch, int store) {
+    constexpr uint32_t kWaves = kBinSumThreads / 64, kGroup = kBinSumGroup;
     extern __shared__ double sums[];
+    const uint32_t number = (blockIdx.x / (8 * kBinNeighbours) * 8 + blockIdx.x % 8) * kBinNeighbours + blockIdx.x / 8 % kBinNeighbours;
+    if (number >= bp.n_bins) return;
     uint32_t k = 0;
-    while (k + 1 < bp.n_levels && blockIdx.x >= bp.first_bin[k + 1]) ++k;
-    const uint32_t l = bp.level[k], bin = blockIdx.x - bp.first_bin[k];
+    while (k + 1 < bp.n_levels && number >= bp.first_bin[k + 1]) ++k;
+    const uint32_t l = bp.level[k], bin = number - bp.first_bin[k];
     const Bins dealt{bp.bins_log2[k], bp.run_log2[k]};
     const uint32_t size = lv.size[l];
     const uint32_t n = bp.places[k]; // the last ones may be beyond the level
+    uint32_t *const wave_sum = reinterpret_cast<uint32_t *>(sums + n * F);
+    uint32_t *const wave_runs = wave_sum + kWaves;
+    uint32_t *const group_run = wave_runs + kWaves;       // run that a group's first record is in
+    uint32_t *const first = group_run + kBinSumThreads / kGroup; // records in front of a run
+    uint32_t *const start = first + n_stretches + 1;       // place of the run's first record in the pieces, less `first`
+    const uint16_t *const begins = offsets + bp.first_bin[k] + k + bin;
+    constexpr int kEach = kBinPiecesEach;
+    const uint32_t each = (n_stretches + blockDim.x - 1) / blockDim.x, s0 = threadIdx.x * each;
+    uint32_t ends[kEach]; // where the bin's records begin in the piece, and where the next bin's do
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+        ends[e] = 0;
+        if ((uint32_t)e < each && s0 + e < n_stretches) __builtin_memcpy(&ends[e], begins + (size_t)(s0 + e) * (bp.n_bins + bp.n_levels), sizeof(uint32_t));
+    }
     for (uint32_t e = threadIdx.x; e < n * F; e += blockDim.x) sums[e] = 0.0;
-    const uint32_t written = cursors[blockIdx.x];
-    const BinRecord<F> *const rec = records + bp.first_record[k] + (size_t)bin * bp.capacity[k];
+    uint32_t count[kEach], mine = 0, run = 0, runs = 0; // runs that hold any records: in front of this thread's, in its wave
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+        count[e] = (ends[e] >> 16) - (ends[e] & 0xffffu);
+        mine += count[e];
+        const unsigned long long any = __ballot(count[e] != 0);
+        run += __popcll(any & ((1ull << (threadIdx.x & 63)) - 1));
+        runs += __popcll(any);
+    }
+    if ((threadIdx.x & 63) == 0) wave_runs[threadIdx.x >> 6] = runs;
+    uint32_t total, at = running_sum<kWaves>(mine, wave_sum, total), n_runs = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kWaves; ++w) {
+        const uint32_t sum = w < blockDim.x / 64 ? wave_runs[w] : 0u;
+        if (w < threadIdx.x >> 6) run += sum;
+        n_runs += sum;
+    }
+    // (whole rounds of a group: all but the last groups then have all of their lanes at work)
+    const uint32_t share = (total + blockDim.x - 1) / blockDim.x * kGroup;
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+        if (count[e] == 0) continue;
+        for (uint32_t g = (at + share - 1) / share; g * share < at + count[e]; ++g) group_run[g] = run;
+        first[run] = at;
+        start[run++] = (s0 + e) * pitch + (ends[e] & 0xffffu) - at;
+        at += count[e];
+    }
+    if (threadIdx.x == 0) first[n_runs] = total;
     __syncthreads();
-    if (threadIdx.x == 0) cursors[blockIdx.x] = 0;
-    if (written <= bp.capacity[k]) {
-        constexpr int kAhead = 4; // records of a lane in flight
-        for (uint32_t i = threadIdx.x; i < written; i += kAhead * blockDim.x) {
-            BinRecord<F> r[kAhead];
+    const BinRecord<F> *const rec = records + (size_t)k * n_stretches * pitch;
+    const uint32_t group = threadIdx.x / kGroup, end = (group + 1) * share < total ? (group + 1) * share : total;
+    uint32_t i = group * share + threadIdx.x % kGroup, s = i < end ? group_run[group] : 0u;
+    constexpr int kAhead = 4; // records of a lane in flight
+    for (; i < end; i += kAhead * kGroup) {
+        uint32_t at_a[kAhead];
 #pragma unroll
-            for (int a = 0; a < kAhead; ++a) {
-                const uint32_t at = i + a * blockDim.x;
-                r[a] = rec[at < written ? at : i];
-                if (at >= written) r[a].where = 0;
-            }
-#pragma unroll
-            for (int a = 0; a < kAhead; ++a) {
-                const uint32_t near = r[a].where & 0x7fff, far = (r[a].where >> 15) & 0x7fff;
-                if (r[a].where & (1u << 30)) {
-#pragma unroll
-                    for (int f = 0; f < F; ++f) lds_add(&sums[near * F + f], (1 - r[a].frac) * r[a].g[f]);
-                }
-                if (r[a].where & (1u << 31)) {
-#pragma unroll
-                    for (int f = 0; f < F; ++f) lds_add(&sums[far * F + f], r[a].frac * r[a].g[f]);
-                }
-            }
+        for (int a = 0; a < kAhead; ++a) {
+            // (lanes past the end walk to the last run and read its last record)
+            const uint32_t wanted = i + a * kGroup < total ? i + a * kGroup : total - 1;
+            while (wanted >= first[s + 1]) ++s; // (first[n_runs] is beyond every record)
+            at_a[a] = start[s] + wanted;
         }
-    } else {
-        for (long long i = first + threadIdx.x; i < last; i += blockDim.x) {
-            float x[D], frac[D];
-            const long long row = bin_point<D>(xin, order, i, x);
-            uint32_t cell[D], near[1 << (D - 1)], far[1 << (D - 1)];
-            cell_of<D>(x, lv.scale[l], gp.interpolation, cell, frac);
-            pair_entries<D>(cell, size, lv.resolution[l], lv.flags[l], gp.hash_type, near, far);
-            const G *dy = dLdy + (dl.by_position ? i : row) * dl.row_stride + l * dl.level_stride;
+        BinRecord<F> r[kAhead];
 #pragma unroll
-            for (int c = 0; c < (1 << (D - 1)); ++c) {
-                const bool near_mine = dealt.bin(near[c]) == bin, far_mine = dealt.bin(far[c]) == bin;
-                if (!near_mine && !far_mine) continue;
-                float weight = 1.0f;
+        for (int a = 0; a < kAhead; ++a) r[a] = rec[at_a[a]];
 #pragma unroll
-                for (int d = 1; d < D; ++d) weight *= (c >> (d - 1)) & 1 ? frac[d] : 1 - frac[d];
+        for (int a = 0; a < kAhead; ++a) {
+            const uint32_t where = i + a * kGroup < end ? r[a].where : 0u, near = where & 0x7fff, far = (where >> 15) & 0x7fff;
+            if (where & (1u << 30)) {
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    const float v = weight * ((float)dy[f] * dl.scale);
-                    if (near_mine) lds_add(&sums[dealt.place(near[c]) * F + f], (1 - frac[0]) * v);
-                    if (far_mine) lds_add(&sums[dealt.place(far[c]) * F + f], frac[0] * v);
-                }
+                for (int f = 0; f < F; ++f) lds_add(&sums[near * F + f], (1 - r[a].frac) * r[a].g[f]);
+            }
+            if (where & (1u << 31)) {
+#pragma unroll
+                for (int f = 0; f < F; ++f) lds_add(&sums[far * F + f], r[a].frac * r[a].g[f]);
             }
         }
     }
     __syncthreads();
     float *const g = grad + (size_t)lv.offset[l] * F;
+    if (store) { // the bin's entries have no other contributions
+        typedef float entry_t __attribute__((ext_vector_type(F), aligned(F < 4 ? F * 4 : 16)));
+        for (uint32_t v = threadIdx.x; v < n; v += blockDim.x) {
+            const uint32_t e = dealt.entry(bin, v);
+            if (e >= size) continue;
+            entry_t sum;
+#pragma unroll
+            for (int f = 0; f < F; ++f) sum[f] = (float)sums[v * F + f];
+            *reinterpret_cast<entry_t *>(g + (size_t)e * F) = sum;
+        }
+        return;
+    }
     for (uint32_t v = threadIdx.x; v < n * F; v += blockDim.x) {
         const uint32_t e = dealt.entry(bin, v / F);
         if (e >= size) continue;
         float *const to = g + (size_t)e * F + v % F;
-        *to = store ? (float)sums[v] : *to + (float)sums[v]; // (store: the bin's entries have no other contributions)
+        *to += (float)sums[v];
     }
 }
 
@@ -313,38 +355,31 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
     // every 16 entries (3-D, 2^22 entries a level: 2^16 points).
     if ((M << (n_dims - 1)) < size / 16) return false;
     // 128 bins a level: a workgroup's share of a bin is then a run of several lines, and the bins of all levels are enough
-    // workgroups for the sums (64 or 256: the one pass gains what the other loses). Small levels have fewer, large ones as
-    // many as it takes for a bin to fit LDS.
-    uint32_t n_log2 = 7;
+    // workgroups for the sums. 256 where 128 would take more than 32 KB of LDS each, so that four workgroups share a CU while some wait
+    // for their first records (2-D, 2^18 points: 29 -> 27 us; 3-D, 2^16: 48 -> 40, 2^19: 182 either way; four features 262 -> 236). Small
+    // levels have fewer, large ones as many as it takes for a bin to fit LDS.
+    uint32_t n_log2 = (size >> 7) * entry > 32 * 1024 ? 8 : 7;
     while (n_log2 > 0 && (size >> (n_log2 + 4)) == 0) --n_log2;
     while (n_log2 < 31 && ((size >> n_log2) * entry > kBinSliceBytes || (size >> n_log2) > 0x7fff)) ++n_log2;
     const size_t bins = (size_t)1 << n_log2;
     if (bins > kBinMaxBins) return false;
     p->batch = (uint32_t)std::min<size_t>(M, size_t(1) << 19);
     // A hashed level deals out groups of cells that share a run of x and all of the other coordinates, at random: runs as long as
-    // leaves a bin 64 groups, down to 16 entries (a line of two features). Dense levels are dealt out in order: consecutive
-    // entries to a bin. (Other hashes than the coherent one send every corner by itself.)
+    // leaves a bin 64 groups, down to 16 entries (a line of two features). A dense level deals out runs of that length: points that
+    // crowd a region of it then still meet all of its bins. (Other hashes than the coherent one send every corner by itself,
+    // at random: consecutive entries to a bin.)
     const bool hashed = (lv.flags[l] & 16u) != 0, apart = hashed && gp.hash_type != TNN_HASH_COHERENT_PRIME;
     const double R = (double)lv.resolution[l];
     const auto groups = [&](uint32_t run) { return std::max(R / (double)((size_t)1 << run), 1.0) * std::pow(R, (double)n_dims - 1.0) / (double)bins; };
     uint32_t run_log2 = 4;
-    while (((size_t)1 << (run_log2 + n_log2)) < size && (!hashed || apart || groups(run_log2 + 1) >= 64.0)) ++run_log2;
+    while (((size_t)1 << (run_log2 + n_log2)) < size && (apart || (hashed && groups(run_log2 + 1) >= 64.0))) ++run_log2;
     const size_t places = ((size + ((size_t)1 << (run_log2 + n_log2)) - 1) >> (run_log2 + n_log2)) << run_log2;
     if (places > 0x7fff || places * entry > kBinSliceBytes) return false;
-    // What points spread evenly send a bin, and how far above it the fullest bin may be.
-    const double split = apart ? 2.0 : 1.0 + 1.0 / (double)((size_t)1 << run_log2);
-    const double mean = (double)p->batch * (double)(1u << (n_dims - 1)) * split * (double)places / (double)size;
-    const double uneven = hashed && !apart ? std::min(4.0 / std::sqrt(std::max(groups(run_log2), 1.0)), 3.0) : 0.0;
-    const double room = std::ceil(((1.2 + uneven) * mean + 8.0 * std::sqrt(mean) + 64.0) / 32.0) * 32.0;
-    if (room * (double)bins + p->n_records > 4.0e9) return false;
     const uint32_t k = p->n_levels++;
     p->level[k] = (uint8_t)l;
     p->bins_log2[k] = (uint8_t)n_log2;
     p->run_log2[k] = (uint8_t)run_log2;
     p->places[k] = (uint16_t)places;
-    p->capacity[k] = (uint32_t)room;
-    p->first_record[k] = p->n_records;
-    p->n_records += (uint32_t)room * (uint32_t)bins;
     p->first_bin[k] = p->n_bins;
     p->n_bins += (uint32_t)bins;
     p->first_bin[k + 1] = p->n_bins;
@@ -352,37 +387,65 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
     return true;
 }
 
-static size_t cursor_bytes(const BinPlan &p) { return ((size_t)p.n_bins * sizeof(uint32_t) + 255) & ~(size_t)255; }
+// The launches of a part of the batch.
+struct BinLaunch {
+    uint32_t threads, stretch, n_stretches; // of a binning workgroup, its points, and how many there are
+    uint32_t room, pitch;                   // records that fit its LDS; from one piece to the next
+    size_t offset_bytes, scratch_bytes;
+};
+template <int D, int F> static BinLaunch bin_launch(const BinPlan &p) {
+    typedef BinShape<D, F> S;
+    BinLaunch b;
+    // (a small batch: half as many threads, twice as many workgroups, while there are fewer than two for every CU)
+    b.threads = (size_t)p.batch * p.n_levels < size_t(512) * S::kThreads * S::kPoints ? S::kThreads / 2 : S::kThreads;
+    b.stretch = b.threads * S::kPoints;
+    b.n_stretches = (p.batch + b.stretch - 1) / b.stretch;
+    b.room = b.stretch * S::kPairs / 8 * 9;
+    b.pitch = 2 * b.stretch * S::kPairs + kBinPiecePad; // (were every far side a record of its own)
+    b.offset_bytes = ((size_t)b.n_stretches * (p.n_bins + p.n_levels) * sizeof(uint16_t) + 255) & ~(size_t)255;
+    b.scratch_bytes = b.offset_bytes + (size_t)p.n_levels * b.n_stretches * b.pitch * sizeof(BinRecord<F>);
+    return b;
+}
 
-size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_features) {
-    return p.n_levels ? cursor_bytes(p) + (size_t)p.n_records * record_bytes(n_features) : 0;
+size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_dims, uint32_t n_features) {
+    if (!p.n_levels) return 0;
+#define TNN_BIN_BYTES(F) (n_dims == 2 ? bin_launch<2, F>(p) : bin_launch<3, F>(p)).scratch_bytes
+    switch (n_features) {
+    case 1: return TNN_BIN_BYTES(1);
+    case 2: return TNN_BIN_BYTES(2);
+    case 4: return TNN_BIN_BYTES(4);
+    default: return TNN_BIN_BYTES(8);
+    }
+#undef TNN_BIN_BYTES
 }
 
 template <int D, int F, typename G>
 static int launch_binned(const BinPlan &p, const GridLevels &lv, const GridParams &gp, const GradLayout &dl, const float *x, const float4 *order, const void *dLdy,
                          float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s) {
-    uint32_t *const cursors = static_cast<uint32_t *>(scratch);
-    BinRecord<F> *const records = reinterpret_cast<BinRecord<F> *>(static_cast<char *>(scratch) + cursor_bytes(p));
-    const auto sum = grid_bin_sum_kernel<D, F, G>;
-    if (!reserve_lds(reinterpret_cast<const void *>(sum), p.slice_lds))
-        return fail(TNN_ERR_HIP, "cannot reserve %u bytes of LDS", p.slice_lds);
     typedef BinShape<D, F> S;
+    const BinLaunch b = bin_launch<D, F>(p);
+    uint16_t *const offsets = static_cast<uint16_t *>(scratch);
+    BinRecord<F> *const records = reinterpret_cast<BinRecord<F> *>(static_cast<char *>(scratch) + b.offset_bytes);
+    uint32_t most_bins = 0;
+    for (uint32_t k = 0; k < p.n_levels; ++k) most_bins = std::max(most_bins, 1u << p.bins_log2[k]);
     const auto bin = grid_bin_kernel<D, F, G>;
-    if (!reserve_lds(reinterpret_cast<const void *>(bin), bin_lds<D, F>(p, S::kThreads)))
-        return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", bin_lds<D, F>(p, S::kThreads));
-    // (as many waves on a CU as it takes whatever LDS the bins need; small bins are over before 16 waves are under way)
-    const unsigned sum_threads = p.slice_lds > 32 * 1024 ? kBinSumThreads : kBinSumThreads / 2;
+    const auto sum = grid_bin_sum_kernel<F>;
+    const size_t bin_lds = (size_t)b.room * sizeof(BinRecord<F>) + (2 * most_bins + 16) * sizeof(uint32_t);
+    const size_t sum_lds = p.slice_lds + (2 * kBinSumThreads / 64 + kBinSumThreads / kBinSumGroup + 2 * b.n_stretches + 1) * sizeof(uint32_t);
+    if (!reserve_lds(reinterpret_cast<const void *>(bin), bin_lds) || !reserve_lds(reinterpret_cast<const void *>(sum), sum_lds))
+        return fail(TNN_ERR_HIP, "cannot reserve %zu and %zu bytes of LDS", bin_lds, sum_lds);
+    // (about as many waves on a CU as it holds, whatever LDS the bins need: small bins are over before many are under way)
+    unsigned sum_threads = p.slice_lds > 48 * 1024 ? kBinSumThreads : p.slice_lds > 20 * 1024 ? kBinSumThreads / 2 : kBinSumThreads / 4;
+    while (sum_threads * kBinPiecesEach < b.n_stretches) sum_threads *= 2;
     for (size_t first = 0; first < M; first += p.batch) {
-        const size_t last = std::min(M, first + p.batch), n = last - first;
-        // (a small batch: half as many threads, twice as many workgroups, while there are fewer than two for every CU)
-        const unsigned T = n * p.n_levels < size_t(512) * S::kThreads * S::kPoints ? S::kThreads / 2 : S::kThreads;
-        const size_t stretches = (n + T * S::kPoints - 1) / (T * S::kPoints);
-        TNN_LAUNCH(bin, dim3((unsigned)((stretches + 7) / 8 * 8 * p.n_levels)), dim3(T), (bin_lds<D, F>(p, T)), s, lv, gp, p, dl, x, order,
-                   (const G *)dLdy, cursors, records, (long long)first, (long long)last);
+        const size_t last = std::min(M, first + p.batch);
+        const uint32_t n_stretches = (uint32_t)((last - first + b.stretch - 1) / b.stretch);
+        TNN_LAUNCH(bin, dim3((n_stretches + 7) / 8 * 8 * p.n_levels), dim3(b.threads), bin_lds, s, lv, gp, p, dl, x, order, (const G *)dLdy, offsets, records,
+                   (long long)first, (long long)last, n_stretches, b.pitch, b.room);
         int rc = check_launch("grid_bin_kernel");
         if (rc) return rc;
-        TNN_LAUNCH(sum, dim3(p.n_bins), dim3(sum_threads), p.slice_lds, s, lv, gp, p, dl, x, order, (const G *)dLdy, cursors,
-                   (const BinRecord<F> *)records, grad, (long long)first, (long long)last, (int)(overwrite && first == 0));
+        TNN_LAUNCH(sum, dim3((p.n_bins + 8 * kBinNeighbours - 1) / (8 * kBinNeighbours) * (8 * kBinNeighbours)), dim3(sum_threads), sum_lds, s, lv, p, (const uint16_t *)offsets, (const BinRecord<F> *)records, grad,
+                   n_stretches, b.pitch, (int)(overwrite && first == 0));
         if ((rc = check_launch("grid_bin_sum_kernel"))) return rc;
     }
     return TNN_OK;
