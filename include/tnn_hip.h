@@ -383,6 +383,9 @@ int tnn_grid_backward_ordered(const tnn_grid_desc *desc, const void *d_order, co
  * of addition. Workspace: tnn_grid_backward_workspace_bytes, which grows with the batch up to 2^18 points (config 4: 96 MiB)
  * and no further; nothing in it has to be cleared. */
 size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size_t M);
+/* Whether tnn_grid_backward_binned is faster over M points given in both orders (the ordering included) than over d_x alone: large
+ * batches on grids with levels that cannot be sorted on chip. */
+int tnn_grid_backward_wants_order(const tnn_grid_desc *desc, size_t M);
 int tnn_grid_backward_binned(const tnn_grid_desc *desc, const float *d_x, const void *d_order, const void *d_dLdy, int dy_dtype,
                              uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
                              tnn_stream_t stream);

@@ -14,13 +14,13 @@ CFG3 = dict(n_dims=3, n_levels=16, n_features_per_level=2, log2_hashmap_size=19,
 DT = {FP32: torch.float32, FP16: torch.float16, BF16: torch.bfloat16}
 
 
-def binned(tnn, d, x, g, dtype, ordered=False, grad=None, overwrite=True, short=0):
+def binned(tnn, d, x, g, dtype, ordered=False, grad=None, overwrite=True, short=0, both=False):
     from tiny_dpcpp_nn import _lib
     M = x.shape[0]
     p = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None  # noqa: E731
     need = tnn.lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), M)
     work = torch.full((max(need - short, 1),), 0xA5, dtype=torch.uint8, device=tnn.dev)  # nothing in it has to be cleared
-    order = tnn.grid_order(d, x) if ordered else None
+    order = tnn.grid_order(d, x) if ordered or both else None
     if grad is None:
         grad = torch.full((tnn.grid_n_params(d),), 0.123, dtype=torch.float32, device=tnn.dev)
     _lib.check(tnn.lib.tnn_grid_backward_binned(ctypes.byref(d), None if ordered else p(x), p(order), p(g), dtype, g.shape[1], p(grad), int(overwrite), M,
@@ -114,6 +114,38 @@ def test_crowded_points_take_about_as_long_as_even_ones(tnn, cfg):
     even = time("even")
     for kind in ("inner", "quarter", "shell"):
         assert time(kind) <= 2 * even, kind
+
+
+@pytest.mark.parametrize("cfg", [CFG2, CFG3, dict(CFG3, log2_hashmap_size=22, n_levels=12), dict(CFG3, n_features_per_level=8, n_levels=6, per_level_scale=2.0),
+                                 dict(CFG2, interpolation="Nearest"), dict(CFG2, n_features_per_level=1, grid_type="Dense", n_levels=9)])
+@pytest.mark.parametrize("kind", ["even", "small"])
+def test_points_in_both_orders(tnn, oracle, cfg, kind):
+    """Boxes and atomics take the cell order and the bins the caller's, where a call is given both: the contributions are the same."""
+    rng = np.random.default_rng(11)
+    M = 40007
+    x = crowded(kind, cfg, M, rng)
+    d = tnn.grid_desc(cfg)
+    for dtype in (FP32, FP16):
+        g = torch.from_numpy(rng.standard_normal((M, cfg["n_levels"] * cfg["n_features_per_level"])).astype(np.float32)).to(tnn.dev).to(DT[dtype])
+        grad = binned(tnn, d, torch.from_numpy(x).to(tnn.dev), g, dtype, both=True)
+        ref = oracle.grid_backward(cfg, x, g.float().cpu().numpy(), tnn.grid_n_params(d))
+        assert np.abs(grad.cpu().numpy() - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
+
+
+def test_encoding_orders_a_batch_whose_finest_levels_are_not_binned(tnn):
+    """Eight features in 2^22 entries are beyond what the bins hold in LDS: the encoding's backward pass hands both orders over from 2^18 points on."""
+    import tiny_dpcpp_nn
+    cfg = dict(CFG3, n_levels=5, n_features_per_level=8, log2_hashmap_size=22, per_level_scale=2.6)
+    d = tnn.grid_desc(cfg)
+    wants = lambda M, **kw: tnn.lib.tnn_grid_backward_wants_order(ctypes.byref(tnn.grid_desc(dict(cfg, **kw))), M)  # noqa: E731
+    assert wants(2 ** 18) == 1 and wants(2 ** 18 - 1) == 0 and wants(2 ** 20, interpolation="Nearest") == 0 and wants(2 ** 20, log2_hashmap_size=19) == 0
+    enc = tiny_dpcpp_nn.Encoding(3, {"otype": "HashGrid", "type": "Hash", "n_levels": 5, "n_features_per_level": 8, "log2_hashmap_size": 22,
+                                     "base_resolution": 16, "per_level_scale": 2.6})
+    x = torch.rand((2 ** 18 + 5, 3), device=tnn.dev)
+    dy = torch.randn((x.shape[0], 40), device=tnn.dev)
+    got, = torch.autograd.grad(enc(x), [enc.params], dy)
+    ref = tnn.grid_backward(d, x, dy, FP32)
+    assert float((got.reshape(-1) - ref.reshape(-1)).abs().max()) <= 1e-5 * float(ref.abs().max())
 
 
 def test_binned_workspace_is_checked(tnn):

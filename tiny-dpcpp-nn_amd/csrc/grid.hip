@@ -907,6 +907,22 @@ TNN_API size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size
     return most + 256;
 }
 
+TNN_API int tnn_grid_backward_wants_order(const tnn_grid_desc *desc, size_t M) {
+    GridLevels lv;
+    GridParams gp;
+    if (check_grid_desc(desc) || grid_common(desc, desc->n_levels * desc->n_features_per_level, M, &lv, &gp)) return 0;
+    // Where the bins take all levels they are as fast as the boxes of cell order, without the ordering. Where they refuse the finest
+    // (tables beyond 2^21 entries of eight features, 2^23 of two), with x alone and with both, us, evenly spread points:
+    // eight features, 2^22 entries, 2^17 points 990 and 960, 2^18 1512 and 1377, 2^20 4800 and 4054; two features, 2^24
+    // entries 777 and 808, 1081 and 1091, 3059 and 2810. Nearest sends a point to one entry a level, and the caller's order is the
+    // faster one at every size (3-D, 2^19 entries, 2^18 points 227 and 232, 2^20 862 and 859; 2-D 193 and 212, 775 and 945).
+    if (gp.interpolation == TNN_INTERP_NEAREST || M < (size_t(1) << 18)) return 0;
+    BinPlan bins{};
+    uint32_t n_big, lds;
+    (void)plan_backward(lv, gp, desc->n_dims, desc->n_features_per_level, false, true, M, &bins, &n_big, &lds);
+    return n_big != 0;
+}
+
 TNN_API int tnn_grid_backward_binned(const tnn_grid_desc *desc, const float *d_x, const void *d_order, const void *d_dLdy, int dy_dtype,
                                      uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
                                      tnn_stream_t stream) {

@@ -83,13 +83,8 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
         const size_t batch = input.m();
         if (batch >= kCellOrderMinBatch) {
             // large batches: order the points by cell first, so that neighbouring lanes gather from the same lines of the
-            // table (same rows, bit for bit; the buffer only grows)
-            const size_t bytes = tnn_grid_order_bytes(&m_desc, batch);
-            if (!m_order || m_order->size() * sizeof(float) < bytes)
-                m_order = std::make_unique<DeviceMatrix<float>>((bytes + sizeof(float) - 1) / sizeof(float), 1, this->get_queue());
-            tnn::abi_check(tnn_grid_order_points(&m_desc, input.GetPointer(), batch, m_order->data(), m_order->size() * sizeof(float),
-                                                 this->get_queue().abi()));
-            tnn::abi_check(tnn_grid_forward_ordered(&m_desc, m_order->data(), this->get_params()->data(), output->GetPointer(), TNN_FP32,
+            // table (same rows, bit for bit)
+            tnn::abi_check(tnn_grid_forward_ordered(&m_desc, ordered(input), this->get_params()->data(), output->GetPointer(), TNN_FP32,
                                                     this->get_padded_output_width(), batch, this->get_queue().abi()));
             return nullptr;
         }
@@ -148,10 +143,20 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
     }
     void run_backward(const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput, DeviceMatrixView<T> *gradients, void *scratch,
                       const size_t scratch_bytes, GradientMode param_gradients_mode) {
-        tnn::abi_check(tnn_grid_backward_binned(&m_desc, input.GetPointer(), nullptr, dL_doutput.GetPointer(), TNN_FP32,
+        // (The points are ordered here again: nothing says they are the forward pass's.)
+        const void *order = tnn_grid_backward_wants_order(&m_desc, input.m()) ? ordered(input) : nullptr;
+        tnn::abi_check(tnn_grid_backward_binned(&m_desc, input.GetPointer(), order, dL_doutput.GetPointer(), TNN_FP32,
                                                 this->get_padded_output_width(), gradients->GetPointer(),
                                                 param_gradients_mode == GradientMode::Overwrite ? 1 : 0, input.m(), scratch, scratch_bytes,
                                                 this->get_queue().abi()));
+    }
+    /// The points in cell order, in a buffer that only grows.
+    const void *ordered(const DeviceMatrixView<float> input) {
+        const size_t bytes = tnn_grid_order_bytes(&m_desc, input.m());
+        if (!m_order || m_order->size() * sizeof(float) < bytes)
+            m_order = std::make_unique<DeviceMatrix<float>>((bytes + sizeof(float) - 1) / sizeof(float), 1, this->get_queue());
+        tnn::abi_check(tnn_grid_order_points(&m_desc, input.GetPointer(), input.m(), m_order->data(), m_order->size() * sizeof(float), this->get_queue().abi()));
+        return m_order->data();
     }
     void check_max_level() const {
         if (this->m_max_level < (float)m_desc.n_levels) throw std::invalid_argument("GridEncoding: max_level below the level count is not supported.");

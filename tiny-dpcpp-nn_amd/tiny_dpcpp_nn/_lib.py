@@ -141,6 +141,7 @@ SIGNATURES = {
     "tnn_grid_backward": (c_int, [POINTER(GridDesc), c_void_p, c_void_p, c_int, c_uint32, c_void_p, c_int, c_size_t, c_void_p]),
     "tnn_grid_backward_ordered": (c_int, [POINTER(GridDesc), c_void_p, c_void_p, c_int, c_uint32, c_void_p, c_int, c_size_t, c_void_p]),
     "tnn_grid_backward_workspace_bytes": (c_size_t, [POINTER(GridDesc), c_size_t]),
+    "tnn_grid_backward_wants_order": (c_int, [POINTER(GridDesc), c_size_t]),
     "tnn_grid_backward_binned": (c_int, [POINTER(GridDesc), c_void_p, c_void_p, c_void_p, c_int, c_uint32, c_void_p, c_int, c_size_t, c_void_p, c_size_t,
                                          c_void_p]),
     "tnn_grid_backward_packed": (c_int, [POINTER(GridDesc), c_void_p, c_void_p, c_int, c_uint32, c_void_p, c_int, c_size_t, c_void_p]),
