@@ -5,7 +5,9 @@
 #include <cstdio>
 #include <functional>
 #include <random>
+#include <thread>
 
+#include "../../tiny-dpcpp-nn_amd/csrc/lds_reservation.h"
 #include "tnn/SwiftNetMLP.h"
 #include "tnn/encoding_factory.h"
 #include "tnn/io.h"
@@ -673,6 +675,25 @@ static void test_encoding_config_errors() {
         "Padded output width"));
 }
 
+// What a kernel may have of LDS is one setting of the process: a thread that asks for less must not lower it under another's feet.
+static void test_lds_reservations() {
+    tnn::LdsReservations reservations;
+    const int a = 0, b = 0;
+    size_t set = 0, of_b = 0, of_second = 0;
+    const auto ask = [&](const void *kernel, int device, size_t bytes, size_t &is) {
+        size_t got = 0;
+        std::thread([&] { got = reservations.at_least(kernel, device, bytes, [&](size_t n) { return (is = n) != 0; }); }).join();
+        return got;
+    };
+    CHECK(ask(&a, 0, 64000, set) == 64000 && set == 64000);
+    CHECK(ask(&a, 0, 52000, set) == 64000 && set == 64000); // another thread, fewer bytes: nothing is set
+    CHECK(ask(&a, 0, 80000, set) == 80000 && set == 80000);
+    CHECK(ask(&b, 0, 50000, of_b) == 50000 && of_b == 50000);           // another kernel
+    CHECK(ask(&a, 1, 50000, of_second) == 50000 && of_second == 50000); // another device
+    CHECK(reservations.at_least(&a, 0, 90000, [](size_t) { return false; }) == 0); // refused: as before
+    CHECK(ask(&a, 0, 90000, set) == 90000 && set == 90000);
+}
+
 int main(int argc, char **argv) {
     const bool cpu_only = argc > 1 && std::string(argv[1]) == "--cpu";
     std::printf("storage types\n");
@@ -683,6 +704,8 @@ int main(int argc, char **argv) {
     test_json();
     std::printf("io files\n");
     test_io_files();
+    std::printf("LDS reservations\n");
+    test_lds_reservations();
     if (!cpu_only) {
         tnn::abi_check(tnn_device_check());
         std::printf("swiftnet\n");

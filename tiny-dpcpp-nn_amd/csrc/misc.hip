@@ -1,4 +1,5 @@
 // Error reporting, weight-layout permutations, L2 loss and the Adam step.
+#include "lds_reservation.h"
 #include "tnn_internal.h"
 
 #include <algorithm>
@@ -31,7 +32,7 @@ namespace {
 struct KernelFacts {
     const void *kernel = nullptr;
     int device = 0;
-    size_t reserved = 0;              // bytes of LDS the kernel may have
+    size_t reserved = 0;              // bytes of LDS the kernel may have at least (process-wide it only rises)
     size_t lds = 0;                   // what `per_cu` was asked for
     int threads = 0, per_cu = 0;
 };
@@ -62,9 +63,11 @@ bool reserve_lds(const void *kernel, size_t bytes) {
     if (bytes <= 48 * 1024) return true;
     KernelFacts &f = kernel_facts(kernel);
     if (f.reserved >= bytes) return true;
-    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
-    f.reserved = bytes;
-    return true;
+    static LdsReservations &process = *new LdsReservations; // (never destroyed: threads may outlive main)
+    f.reserved = process.at_least(kernel, f.device, bytes, [&](size_t n) {
+        return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n) == hipSuccess;
+    });
+    return f.reserved >= bytes;
 }
 
 int resident_per_cu(const void *kernel, int threads, size_t lds_bytes) {

@@ -23,7 +23,8 @@ inline hipStream_t as_stream(tnn_stream_t s) { return reinterpret_cast<hipStream
 int check_launch(const char *what);
 
 // Reserves `bytes` of dynamic LDS for a kernel that wants more than every kernel may have, and how many of its workgroups a CU
-// holds at once (at least 1). Both ask the runtime, microseconds each time, so the answers are kept per thread, device and kernel.
+// holds at once (at least 1). Both ask the runtime, microseconds each time, so the answers are kept per thread, device and kernel;
+// what is reserved holds for the process (lds_reservation.h).
 bool reserve_lds(const void *kernel, size_t bytes);
 int resident_per_cu(const void *kernel, int threads, size_t lds_bytes);
 
