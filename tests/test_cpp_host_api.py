@@ -28,6 +28,12 @@ def test_host_api_cpu_cases():
     _run(["--cpu"])
 
 
+def test_a_module_needs_the_references_methods_only():
+    """A C++ subclass of tnn::Module as a program that came from the reference has it compiles against the header."""
+    proc = subprocess.run(["make", "-C", os.path.join(HERE, "cpp"), "module_subclass"], capture_output=True, text=True, timeout=600)
+    assert proc.returncode == 0, proc.stdout[-2000:] + proc.stderr[-4000:]
+
+
 @pytest.mark.gpu
 def test_host_api_gpu_cases():
     """SwiftNetMLP forward/inference/backward, Trainer, L2Loss, grid encoding and every error path, on the GPU."""

@@ -79,7 +79,7 @@ class Module {
     // ---- a module as an operator on a caller's rows -----------------------------------------------------------------------
     // What the reference's Python modules do around the two passes in operations of their own (padding, conversion, loss scale,
     // packing and slicing, dpcpp_bindings/tiny_dpcpp_nn/modules.py:84-136,206-262) is part of the passes here. The autograd
-    // function over them lives with the Python bindings.
+    // function over them lives with the Python bindings. A subclass that has the reference's methods only need not have these.
     /// What a forward pass leaves for its backward pass.
     struct RowsPass {
         torch::Tensor input;          // what the kernels read: the caller's tensor, or the padded and converted copy of it
@@ -89,17 +89,21 @@ class Module {
         bool in_workspace = false; // the activations are in the module's own workspace (forward_pass / backward_pass)
     };
     /// The input as forward_rows takes it: dense, of a type the kernels read, with no more columns than the module has.
-    virtual torch::Tensor input_rows(const torch::Tensor &x) const = 0;
+    virtual torch::Tensor input_rows(const torch::Tensor &) const { throw std::runtime_error("input_rows: not available for this module"); }
     /// Columns a caller sees of the output.
-    virtual int64_t visible_columns() const = 0;
+    virtual int64_t visible_columns() const { throw std::runtime_error("visible_columns: not available for this module"); }
     /// keep: a backward pass may follow. training: only where a network keeps its activations in the module's workspace.
     /// push: the parameters to take over first, or an undefined tensor.
-    virtual torch::Tensor forward_rows(const torch::Tensor &x, const torch::Tensor &push, bool keep, bool training, RowsPass &pass) = 0;
+    virtual torch::Tensor forward_rows(const torch::Tensor & /*x*/, const torch::Tensor & /*push*/, bool /*keep*/, bool /*training*/, RowsPass & /*pass*/) {
+        throw std::runtime_error("forward_rows: not available for this module");
+    }
     /// Gradients of the input (undefined unless wanted and available) and of the parameters, in the type and shape of `params`.
-    virtual std::tuple<torch::Tensor, torch::Tensor> backward_rows(const torch::Tensor &dy, const RowsPass &pass, double loss_scale, bool want_dx,
-                                                                   const torch::Tensor &params) = 0;
+    virtual std::tuple<torch::Tensor, torch::Tensor> backward_rows(const torch::Tensor & /*dy*/, const RowsPass & /*pass*/, double /*loss_scale*/, bool /*want_dx*/,
+                                                                   const torch::Tensor & /*params*/) {
+        throw std::runtime_error("backward_rows: not available for this module");
+    }
     /// The parameter tensor as the Python modules hold it (a network's is packed) becomes the module's parameters.
-    virtual void push_params(const torch::Tensor &params) = 0;
+    virtual void push_params(const torch::Tensor &) { throw std::runtime_error("push_params: not available for this module"); }
     /// Network modules behind a grid encoding: the same two passes on positions.
     virtual torch::Tensor forward_rows_with_encoding(const Module &, const torch::Tensor &, const torch::Tensor &, bool) {
         throw std::runtime_error("forward_rows_with_encoding: not a network module");
