@@ -380,8 +380,12 @@ int tnn_grid_backward_ordered(const tnn_grid_desc *desc, const void *d_order, co
 /* tnn_grid_backward (d_x given) or tnn_grid_backward_ordered (d_order given, with d_x beside it or NULL) with scratch
  * memory, for large batches: the contributions to levels beyond an LDS copy are sorted by destination into the workspace and
  * summed on chip, where the calls above add each of them to the table with atomics. The same contributions in another order
- * of addition. Workspace: tnn_grid_backward_workspace_bytes, which grows with the batch up to 2^18 points (config 4: 96 MiB)
- * and no further; nothing in it has to be cleared. */
+ * of addition. Nothing in the workspace has to be cleared. Its size, tnn_grid_backward_workspace_bytes, grows with the batch up to 2^19
+ * points, which are sorted at a time, and no further: room for two records a pair of corners along the first dimension (12, 16, 24
+ * or 40 bytes with 1, 2, 4 or 8 features), point and level that is sorted. 16 levels of two features and 2^19 entries: 183 MiB for 2^18
+ * points of a 2-D grid, 366 from 2^19 on; 500 and 1000 MiB in 3-D; 829 and 1658 MiB with four features, 1377 and 2754 with eight.
+ * A caller without that much to spare sorts parts of the batch (overwrite = 0 after the first) or calls the routines above, which need
+ * no workspace. */
 size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size_t M);
 /* Whether tnn_grid_backward_binned is faster over M points given in both orders (the ordering included) than over d_x alone: large
  * batches on grids with levels that cannot be sorted on chip. */
@@ -440,7 +444,8 @@ int tnn_grid_mlp_inference_ordered(const tnn_grid_desc *grid, const tnn_mlp_desc
  *   d_grad_table: n_params fp32, overwritten or accumulated into as in tnn_grid_backward; it holds loss_scale x the gradient.
  *   Network arguments as in tnn_mlp_train_step_l2_adam. Built for width 64, ReLU, at most 4 hidden layers and 2 features per
  *   level (tnn_grid_mlp_train_supported returns TNN_OK); other shapes get TNN_ERR_UNSUPPORTED and run the three calls.
- * Workspace: tnn_grid_mlp_train_step_workspace_bytes. */
+ * Workspace: tnn_grid_mlp_train_step_workspace_bytes: what tnn_grid_backward_binned needs, which is most of it, dL/d(encoding) and the
+ * workgroups' partial gradients (211 MiB for 2^18 points of a 2-D grid of 16 levels and 2^19 entries). */
 int tnn_grid_mlp_train_supported(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp);
 size_t tnn_grid_mlp_train_step_workspace_bytes(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, size_t M);
 int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order,

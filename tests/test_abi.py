@@ -59,3 +59,19 @@ def test_grid_descriptor_host_side(lib):
     assert lib.tnn_grid_desc_init(ctypes.byref(d), 3, 200, 2, 22, 16, 1.447, 0, 1, 1, _lib.TNN_FP16) == _lib.TNN_ERR_INVALID_ARGUMENT
     assert b"MAX_N_LEVELS" in lib.tnn_last_error()
     assert lib.tnn_grid_desc_init(ctypes.byref(d), 5, 16, 2, 22, 16, 1.447, 0, 1, 1, _lib.TNN_FP16) == _lib.TNN_ERR_UNSUPPORTED
+
+
+def test_scatter_workspace_is_as_large_as_the_header_says(lib):
+    """The sizes given at tnn_grid_backward_binned and tnn_grid_mlp_train_step_l2_adam, in MiB, and that they stop growing at 2^19 points."""
+    from tiny_dpcpp_nn import _lib
+    d = _lib.GridDesc()
+    header = open(os.path.join(ROOT, "include", "tnn_hip.h")).read()
+    for dims, features, sizes in ((2, 2, (183, 366)), (3, 2, (500, 1000)), (3, 4, (829, 1658)), (3, 8, (1377, 2754))):
+        assert lib.tnn_grid_desc_init(ctypes.byref(d), dims, 16, features, 19, 16, 1.5 if dims == 2 else 1.447, 0, 1, 1, _lib.TNN_FP32) == 0
+        got = [lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), 2 ** k) / 2 ** 20 for k in (18, 19, 20, 22)]
+        assert [int(g) for g in got] == [sizes[0], sizes[1], sizes[1], sizes[1]]
+        assert all(f"{size} " in header for size in sizes)
+    mlp = _lib.MlpDesc(_lib.TNN_FP16, 64, 2, _lib.ACT_RELU, _lib.ACT_NONE)
+    assert lib.tnn_grid_desc_init(ctypes.byref(d), 2, 16, 2, 19, 16, 1.5, 0, 1, 1, _lib.TNN_FP16) == 0
+    step = int(lib.tnn_grid_mlp_train_step_workspace_bytes(ctypes.byref(d), ctypes.byref(mlp), 2 ** 18) / 2 ** 20)
+    assert f"({step} MiB for 2^18 points" in header
