@@ -238,8 +238,8 @@ __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
 // One workgroup sums one bin and stores (or adds) its entries. Bound by the LDS atomics, two entries of F values a record: LDS is at
 // work 72 % of the time (3-D, 2^19 points, 15 levels, 184 us; 163 with the records read and not added). The bin's runs of records in the pieces follow each other here (`first`: records in front of a piece's run);
 // sixteen lanes take an equal share of them all, whatever the runs' lengths, and walk from run to run. Neighbouring bins, whose
-// runs share lines, are workgroups of one XCD, sixteen at a time.
-template <int F>
+// runs share lines, are workgroups of one XCD, sixteen at a time. kAhead: records of a lane in flight.
+template <int F, int kAhead>
 __global__ void __launch_bounds__(kBinSumThreads)
     grid_bin_sum_kernel(const GridLevels lv, const BinPlan bp, const uint16_t *__restrict__ offsets, const BinRecord<F> *__restrict__ records,
                         float *__restrict__ grad, uint32_t n_stretches, uint32_t pitch, int store) {
@@ -300,7 +300,6 @@ __global__ void __launch_bounds__(kBinSumThreads)
     const BinRecord<F> *const rec = records + (size_t)k * n_stretches * pitch;
     const uint32_t group = threadIdx.x / kGroup, end = (group + 1) * share < total ? (group + 1) * share : total;
     uint32_t i = group * share + threadIdx.x % kGroup, s = i < end ? group_run[group] : 0u;
-    constexpr int kAhead = 4; // records of a lane in flight
     for (; i < end; i += kAhead * kGroup) {
         uint32_t at_a[kAhead];
 #pragma unroll
@@ -429,14 +428,17 @@ static int launch_binned(const BinPlan &p, const GridLevels &lv, const GridParam
     uint32_t most_bins = 0;
     for (uint32_t k = 0; k < p.n_levels; ++k) most_bins = std::max(most_bins, 1u << p.bins_log2[k]);
     const auto bin = grid_bin_kernel<D, F, G>;
-    const auto sum = grid_bin_sum_kernel<F>;
     const size_t bin_lds = (size_t)b.room * sizeof(BinRecord<F>) + (2 * most_bins + 16) * sizeof(uint32_t);
     const size_t sum_lds = p.slice_lds + (2 * kBinSumThreads / 64 + kBinSumThreads / kBinSumGroup + 2 * b.n_stretches + 1) * sizeof(uint32_t);
-    if (!reserve_lds(reinterpret_cast<const void *>(bin), bin_lds) || !reserve_lds(reinterpret_cast<const void *>(sum), sum_lds))
-        return fail(TNN_ERR_HIP, "cannot reserve %zu and %zu bytes of LDS", bin_lds, sum_lds);
     // (about as many waves on a CU as it holds, whatever LDS the bins need: small bins are over before many are under way)
     unsigned sum_threads = p.slice_lds > 48 * 1024 ? kBinSumThreads : p.slice_lds > 20 * 1024 ? kBinSumThreads / 2 : kBinSumThreads / 4;
     while (sum_threads * kBinPiecesEach < b.n_stretches) sum_threads *= 2;
+    // Up to four records a lane of an even spread, and a few more that are split: five in flight make one round of them (2-D, 2^18 points 27.3 ->
+    // 24.9 us); long bins are no faster for it (3-D, 2^19: 184 and 191).
+    const bool short_bins = ((size_t)p.batch * S::kPairs) / most_bins <= (size_t)4 * sum_threads;
+    const auto sum = short_bins ? grid_bin_sum_kernel<F, 5> : grid_bin_sum_kernel<F, 4>;
+    if (!reserve_lds(reinterpret_cast<const void *>(bin), bin_lds) || !reserve_lds(reinterpret_cast<const void *>(sum), sum_lds))
+        return fail(TNN_ERR_HIP, "cannot reserve %zu and %zu bytes of LDS", bin_lds, sum_lds);
     for (size_t first = 0; first < M; first += p.batch) {
         const size_t last = std::min(M, first + p.batch);
         const uint32_t n_stretches = (uint32_t)((last - first + b.stretch - 1) / b.stretch);
