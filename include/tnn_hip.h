@@ -400,7 +400,7 @@ int tnn_grid_backward_binned(const tnn_grid_desc *desc, const float *d_x, const 
  * gradients are float (grad_t, include/encodings/grid.h:586, "we don't have atomics for half precision",
  * dpcpp_bindings/tiny_dpcpp_nn/modules.py:320-324); it is what tiny-cuda-nn does for half-precision grids. Sums are
  * rounded to fp16 at every addition: scale dL/dy (loss scale) so that contributions stay clear of fp16's denormal range.
- * n_features_per_level must be even. d_grad_table_f16: n_params fp16. Coarse levels are still accumulated in fp32 (LDS)
+ * n_features_per_level must be even. d_grad_table_f16: n_params fp16. Coarse levels are still accumulated in LDS (double)
  * and rounded once when they are flushed. */
 int tnn_grid_backward_packed(const tnn_grid_desc *desc, const float *d_x, const void *d_dLdy, int dy_dtype,
                              uint32_t padded_width, void *d_grad_table_f16, int overwrite, size_t M, tnn_stream_t stream);

@@ -206,7 +206,7 @@ def test_two_streams_give_the_single_stream_results(tnn):
 
 def test_two_host_threads(tnn):
     """Two host threads, a stream each, call the library at the same time (ctypes releases the GIL during a call): same
-    results as one thread. What the library caches per device lives in thread-local storage."""
+    results as one thread. What the library remembers of its kernels is thread-local, or (the LDS they may have) the process's and locked."""
     import ctypes
     import threading
 

@@ -349,7 +349,7 @@ __global__ void __launch_bounds__(kBwdThreads)
         // Cell order, a level whose workgroups each take stretches of consecutive points of one row of the order's coarse
         // cells (grid_order.hip walks the coarse cells row by row, x fastest, and leaves the first position of every
         // coarse cell behind the records): such a stretch lies in a few neighbouring cells, so the corners it touches fill
-        // a small box of the level's cells. The workgroup accumulates in a private fp32 copy of it in LDS,
+        // a small box of the level's cells. The workgroup accumulates in a private copy of it in LDS (double),
         // and adds every touched entry to the table once. A stretch whose box does not fit (points far apart: the bins of
         // the points outside the unit cube, a sparse region) adds to the table directly.
         const uint32_t tb = lds_block - n_small_blocks;
