@@ -90,6 +90,19 @@ def test_crowded_points_match_the_oracle(tnn, oracle, cfg, kind):
     assert np.abs(grad.cpu().numpy() - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
 
 
+@pytest.mark.parametrize("M", [33003, 50001, 2 ** 18 + 1])
+def test_as_many_bins_as_a_level_may_have(tnn, oracle, M):
+    """1024 bins a level (eight features, 2^21 entries), dealt out by the smallest workgroups and by the largest."""
+    cfg = dict(n_dims=3, n_levels=3, n_features_per_level=8, log2_hashmap_size=21, base_resolution=128, per_level_scale=1.2)
+    rng = np.random.default_rng(M)
+    x = rng.uniform(0, 1, (M, 3)).astype(np.float32)
+    d = tnn.grid_desc(cfg)
+    g = torch.from_numpy(rng.standard_normal((M, 24)).astype(np.float32)).to(tnn.dev)
+    grad = binned(tnn, d, torch.from_numpy(x).to(tnn.dev), g, FP32)
+    ref = oracle.grid_backward(cfg, x, g.cpu().numpy(), tnn.grid_n_params(d))
+    assert np.abs(grad.cpu().numpy() - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
+
+
 @pytest.mark.parametrize("cfg", [dict(CFG2, log2_hashmap_size=19), CFG3])
 def test_crowded_points_take_about_as_long_as_even_ones(tnn, cfg):
     """No distribution of an ordinary batch falls off the fast path: measured 0.95 to 1.05 of the time for evenly spread points, where one

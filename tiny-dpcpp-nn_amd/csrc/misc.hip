@@ -6,6 +6,7 @@
 #include "adam_update.h"
 
 #include <cstring>
+#include <exception>
 
 namespace tnn {
 
@@ -63,10 +64,14 @@ bool reserve_lds(const void *kernel, size_t bytes) {
     if (bytes <= 48 * 1024) return true;
     KernelFacts &f = kernel_facts(kernel);
     if (f.reserved >= bytes) return true;
-    static LdsReservations &process = *new LdsReservations; // (never destroyed: threads may outlive main)
-    f.reserved = process.at_least(kernel, f.device, bytes, [&](size_t n) {
-        return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n) == hipSuccess;
-    });
+    try { // (the callers are C entries)
+        static LdsReservations &process = *new LdsReservations; // (never destroyed: threads may outlive main)
+        f.reserved = process.at_least(kernel, f.device, bytes, [&](size_t n) {
+            return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n) == hipSuccess;
+        });
+    } catch (const std::exception &) {
+        return false; // out of host memory
+    }
     return f.reserved >= bytes;
 }
 
