@@ -1,0 +1,92 @@
+"""The grid encoding level by level (tnn_grid_forward_by_level, and tnn_grid_forward on small batches): the rows of the kernel that walks all
+levels of a point, bit for bit, which is checked against the oracle elsewhere (tests/test_gpu_grid.py, here through the larger batch)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_harness import BF16, FP16, FP32, ptr
+from tiny_dpcpp_nn import _lib
+
+pytestmark = pytest.mark.gpu
+DIRECT = 2 ** 14  # the most points whose rows tnn_grid_forward writes level by level
+TORCH = {FP32: torch.float32, BF16: torch.bfloat16, FP16: torch.float16}
+BASE = dict(n_dims=3, n_levels=16, n_features_per_level=2, log2_hashmap_size=15, base_resolution=16, per_level_scale=1.447)
+
+
+def bits(t):
+    return t.contiguous().view(torch.int32 if t.element_size() == 4 else torch.int16)
+
+
+def by_level(tnn, d, x, order, table, width, out_dtype):
+    M = x.shape[0]
+    need = d.n_levels * d.n_features_per_level * TORCH[out_dtype].itemsize * ((M + 63) // 64 * 64) + 256
+    work = torch.empty(need, dtype=torch.uint8, device=tnn.dev)
+    out = torch.full((M, width), 7.0, dtype=TORCH[out_dtype], device=tnn.dev)
+    args = (ctypes.byref(d), ptr(x) if order is None else None, ptr(order) if order is not None else None, ptr(table), ptr(out), out_dtype, width, M, ptr(work))
+    assert tnn.lib.tnn_grid_forward_by_level(*args, need - 300, tnn.stream()) == _lib.TNN_ERR_WORKSPACE
+    _lib.check(tnn.lib.tnn_grid_forward_by_level(*args, need, tnn.stream()))
+    return out
+
+
+@pytest.mark.parametrize("cfg,param_dtype,out_dtype,width", [
+    (BASE, FP32, FP32, 32), (BASE, FP16, FP16, 64), (BASE, FP32, BF16, 36), (dict(BASE, n_dims=2, per_level_scale=1.5), FP32, FP32, 33),
+    (dict(BASE, n_dims=2, log2_hashmap_size=19, per_level_scale=1.5), FP16, BF16, 32), (dict(BASE, n_features_per_level=1), FP32, FP32, 17),
+    (dict(BASE, n_features_per_level=4), FP32, FP32, 64), (dict(BASE, n_features_per_level=8, n_levels=3, n_dims=2), FP16, FP16, 24),
+    (dict(BASE, n_features_per_level=8, n_levels=7), FP32, FP32, 60), (dict(BASE, n_levels=1), FP32, FP32, 2), (dict(BASE, n_levels=5, interpolation="Smoothstep"), FP32, FP32, 10),
+    (dict(BASE, interpolation="Nearest"), FP32, FP32, 32), (dict(BASE, hash="Prime"), FP32, FP32, 32), (dict(BASE, hash="ReversedPrime", n_dims=2), FP16, FP16, 32),
+    (dict(BASE, hash="Rng"), FP32, FP32, 32), (dict(BASE, grid_type="Dense", n_levels=5), FP32, FP32, 12), (dict(BASE, grid_type="Tiled"), FP32, FP32, 32)])
+def test_levels_are_the_rows_of_the_points(tnn, cfg, param_dtype, out_dtype, width):
+    d = tnn.grid_desc(cfg, param_dtype)
+    gen = torch.Generator(device=tnn.dev).manual_seed(5)
+    table = (torch.rand(tnn.grid_n_params(d), device=tnn.dev, generator=gen) * 2 - 1).to(TORCH[param_dtype])
+    M = DIRECT + 77
+    x = torch.rand((M, cfg["n_dims"]), device=tnn.dev, generator=gen)
+    x[:6] = torch.tensor([0.0, 1.0, -0.25, 1.75, float("nan"), 0.999999], device=tnn.dev)[:, None]
+    expected = tnn.grid_forward(d, x, table, width, out_dtype)
+    assert torch.equal(bits(by_level(tnn, d, x, None, table, width, out_dtype)), bits(expected))
+    assert torch.equal(bits(by_level(tnn, d, x, tnn.grid_order(d, x), table, width, out_dtype)), bits(expected))
+    for m in (1, 2, 63, 129, 4097, DIRECT):  # written directly, odd numbers of lanes among them
+        part = x[:m].contiguous()
+        assert torch.equal(bits(tnn.grid_forward(d, part, table, width, out_dtype)), bits(expected[:m]))
+        assert torch.equal(bits(tnn.grid_forward_ordered(d, tnn.grid_order(d, part), table, width, m, out_dtype)), bits(expected[:m]))
+
+
+@pytest.mark.parametrize("dims,log2,M", [(3, 16, DIRECT), (3, 16, DIRECT + 1), (3, 19, 2 ** 19 + 3), (2, 16, 2 ** 19 - 1), (2, 16, 2 ** 19), (3, 22, 2 ** 17)])
+def test_encoding_module_on_both_sides_of_each_rule(tnn, dims, log2, M):
+    """The Python encoding takes whichever route its size says; the C ABI in two calls of half the points, or by points, gives the same rows."""
+    import tiny_dpcpp_nn
+    cfg = dict(BASE, n_dims=dims, log2_hashmap_size=log2)
+    enc = tiny_dpcpp_nn.Encoding(dims, {"otype": "HashGrid", "type": "Hash", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": log2, "base_resolution": 16,
+                                        "per_level_scale": 1.447})
+    gen = torch.Generator(device=tnn.dev).manual_seed(6)
+    with torch.no_grad():
+        enc.params.copy_(torch.rand(enc.params.shape, device=tnn.dev, generator=gen) - 0.5)
+        x = torch.rand((M, dims), device=tnn.dev, generator=gen)
+        y = enc(x)
+    d = tnn.grid_desc(cfg)
+    x2 = torch.cat([x, x[: DIRECT + 1]]) if M <= DIRECT else x  # (a batch beyond the small ones)
+    assert torch.equal(bits(y), bits(tnn.grid_forward(d, x2, enc.params.detach().reshape(-1), 32, FP32)[:M]))
+
+
+def test_a_small_batch_in_a_graph_replays(tnn):
+    d = tnn.grid_desc(BASE)
+    table = torch.rand(tnn.grid_n_params(d), device=tnn.dev)
+    x = torch.rand((1000, 3), device=tnn.dev)
+    out = torch.empty((1000, 32), device=tnn.dev)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        tnn.grid_forward(d, x, table, 32, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        tnn.grid_forward(d, x, table, 32, out=out)
+    for seed in range(4):
+        x.copy_(torch.rand(x.shape, device=tnn.dev, generator=torch.Generator(device=tnn.dev).manual_seed(seed)))
+        out.fill_(float(seed))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.clone()
+        assert np.isfinite(got.cpu().numpy()).all() and torch.equal(got, tnn.grid_forward(d, x, table, 32))

@@ -11,6 +11,7 @@
 // how many dimensions enter the dense index, whether the level is hashed) are evaluated once on the
 // host and reach the kernel as scalar kernel arguments; no thread evaluates exp2.
 #include "grid_binned.h"
+#include "grid_levels.h"
 
 #include <algorithm>
 #include <cmath>
@@ -802,6 +803,7 @@ TNN_API int tnn_grid_forward(const tnn_grid_desc *desc, const float *d_x, const 
     int rc = grid_common(desc, padded_width, M, &lv, &gp);
     if (rc) return rc;
     if (!d_x || !d_table || !d_out) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    if (grid_rows_direct(M)) return launch_grid_levels(desc, lv, gp, d_x, nullptr, d_table, d_out, out_dtype, padded_width, M, as_stream(stream));
     TNN_DISPATCH_DF(desc, rc = (launch_grid_forward_p<D_, F_>(desc, lv, gp, d_x, nullptr, d_table, d_out, out_dtype, M, as_stream(stream))));
     return rc;
 }
@@ -814,6 +816,8 @@ TNN_API int tnn_grid_forward_ordered(const tnn_grid_desc *desc, const void *d_or
     if (rc) return rc;
     if (!d_order || !d_table || !d_out) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
     if (reinterpret_cast<uintptr_t>(d_order) & 15) return fail(TNN_ERR_INVALID_ARGUMENT, "d_order must be 16-byte aligned");
+    if (grid_rows_direct(M))
+        return launch_grid_levels(desc, lv, gp, nullptr, static_cast<const float4 *>(d_order), d_table, d_out, out_dtype, padded_width, M, as_stream(stream));
     TNN_DISPATCH_DF(desc, rc = (launch_grid_forward_p<D_, F_>(desc, lv, gp, nullptr, static_cast<const float4 *>(d_order), d_table, d_out,
                                                               out_dtype, M, as_stream(stream))));
     return rc;

@@ -1,0 +1,334 @@
+// Grid encoding level by level (gfx950).
+//
+// Reference behaviour being reproduced: include/encodings/grid.h:37-135 (kernel_grid; the same sums, bit for bit, as
+// grid_forward_kernel). The reference, too, takes the levels as the slow dimension of its launch (:696-731).
+//
+// What bounds a gather is where its line comes from: lines of 128 bytes at random arrive 66 * 10^9 times a second from the memory
+// side and 265 * 10^9 times from an XCD's own 4 MB of L2 (64 bytes a cycle and CU), whether 4, 8 or 16 bytes of a line are wanted.
+// A kernel whose waves walk all levels of their points (grid_forward_kernel) has the whole table in use at once, in every XCD. Here
+// an XCD takes a level at a time, for all points: its L2 holds that level, and a level is fetched by one or two XCDs instead of eight.
+// The corners of a cell along the first dimension lie in one line nearly always. Two loads of a lane fetch it twice, because
+// the lines that a CU's waves have under way are many times what its vector cache holds; here two neighbouring lanes load the two
+// corners of a row, of one's point and then of the other's, and exchange what they loaded.
+// Measured, fp32 table and rows: 3-D, 16 levels, 2^19 entries, 2^20 points 253 us in cell order and 332 in the caller's (one load a lane: 547 and
+// 534; all levels of a point in one thread: 519 and 754), of which the levels beyond L2's reach of a thread a point 455 -> 170 for eight of them;
+// 2-D, 2^18 points 32 and 43 (42 and 76). 5001 points 3-D: 6 us (38).
+// A batch that is small then has a wave for every level, too, and not one wave that walks through all of them.
+#include "grid_levels.h"
+
+#include <algorithm>
+#include <cmath>
+
+namespace tnn {
+
+constexpr int kLevelThreads = 256;
+constexpr uint32_t kXcds = 8;
+
+// Points of a thread, so that it has 16 gathers and more in flight.
+template <int D, int F> struct LevelShape {
+    static constexpr int kPoints = F > 4 ? 1 : D == 2 && F <= 2 ? 4 : 2;
+    static constexpr int kChunk = kLevelThreads * kPoints; // points of a workgroup
+};
+
+// Workgroup b is the (b / 8)-th of XCD b % 8 (workgroups go to the XCDs in turn; were they not, nothing but locality would be lost);
+// XCD k takes the items [first[k], first[k + 1]) of the list of all (level, chunk of points), level by level.
+struct LevelPlan {
+    uint32_t first[kXcds + 1];
+    uint32_t n_chunks;
+};
+
+// The neighbouring lane's value: lanes 2 k and 2 k + 1 exchange (DPP quad_perm).
+__device__ __forceinline__ uint32_t swap_pair(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xf, 0xf, false); }
+__device__ __forceinline__ float swap_pair(float v) { return __uint_as_float(swap_pair(__float_as_uint(v))); }
+
+// Entries of a cell's corners on one side of it along the first dimension (side 1: the far one): bit d - 1 of a row's number says which
+// side of dimension d it lies on. The values of level_index.
+template <int D>
+__device__ __forceinline__ void row_entries(const uint32_t (&cell)[D], uint32_t side, uint32_t size, uint32_t res, uint32_t flags, uint32_t hash_type,
+                                            uint32_t (&entry)[1 << (D - 1)]) {
+    constexpr int R = 1 << (D - 1);
+    const uint32_t x = cell[0] + side;
+    if ((flags & 48u) == 48u && hash_type == TNN_HASH_COHERENT_PRIME) {
+        const uint32_t y0 = cell[1] * 2654435761u, y1 = y0 + 2654435761u;
+        const uint32_t z0 = D > 2 ? cell[D - 1] * 805459861u : 0u, z1 = z0 + 805459861u;
+#pragma unroll
+        for (int r = 0; r < R; ++r) entry[r] = (x ^ ((r & 1) ? y1 : y0) ^ (D > 2 ? ((r & 2) ? z1 : z0) : 0u)) & (size - 1);
+    } else if ((flags & 31u) == (uint32_t)D) {
+        const uint32_t first = D > 2 ? x + res * (cell[1] + res * cell[D - 1]) : x + res * cell[1];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            entry[r] = first + ((r & 1) ? res : 0u) + ((r & 2) ? res * res : 0u);
+            if (flags & 32u) entry[r] &= size - 1;
+            else if (entry[r] >= size) entry[r] %= size;
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            uint32_t loc[D];
+            loc[0] = x;
+#pragma unroll
+            for (int d = 1; d < D; ++d) loc[d] = cell[d] + ((r >> (d - 1)) & 1);
+            entry[r] = level_index<D>(loc, size, res, flags, hash_type);
+        }
+    }
+}
+
+template <int D, int F, typename P, typename O, bool ROWS>
+__global__ void __launch_bounds__(kLevelThreads)
+    grid_levels_kernel(const GridLevels lv, const GridParams gp, const LevelPlan plan, const float *__restrict__ xin, const float4 *__restrict__ order,
+                       const P *__restrict__ table, O *__restrict__ out, long long M, size_t pitch) {
+    constexpr int U = LevelShape<D, F>::kPoints, R = 1 << (D - 1); // R: rows of two corners along the first dimension
+    typedef O ovec __attribute__((ext_vector_type(F)));
+    const uint32_t xcd = blockIdx.x % kXcds, item = plan.first[xcd] + blockIdx.x / kXcds;
+    if (item >= plan.first[xcd + 1]) return;
+    const uint32_t l = item / plan.n_chunks;
+    const long long i0 = (long long)(item % plan.n_chunks) * LevelShape<D, F>::kChunk + threadIdx.x;
+    const uint32_t size = lv.size[l], res = lv.resolution[l], flags = lv.flags[l];
+    const float scale = lv.scale[l];
+    const P *const level = table + (size_t)lv.offset[l] * F;
+    const bool nearest = gp.interpolation == TNN_INTERP_NEAREST;
+    const uint32_t side = threadIdx.x & 1;
+
+    // (lanes past the end stay, as the last point's: their neighbours exchange with them)
+    float x[U][D];
+    uint32_t row[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const long long i = i0 + u * kLevelThreads < M ? i0 + u * kLevelThreads : M - 1;
+        if (order) {
+            const float4 r = order[i];
+            x[u][0] = r.x;
+            x[u][1] = r.y;
+            if (D > 2) x[u][D - 1] = r.z;
+            row[u] = __float_as_uint(r.w);
+        } else {
+#pragma unroll
+            for (int d = 0; d < D; ++d) x[u][d] = xin[i * D + d];
+        }
+    }
+    float even[U][R][F], odd[U][R][F], frac[U][D]; // what this lane loads for the even and the odd lane's point
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        uint32_t cell[D], of_even[D], of_odd[D], a[R], b[R];
+        cell_of<D>(x[u], scale, gp.interpolation, cell, frac[u]);
+        if (nearest) {
+            load_entry<P, F>(level + (size_t)level_index<D>(cell, size, res, flags, gp.hash_type) * F, even[u][0]);
+            continue;
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const uint32_t other = swap_pair(cell[d]);
+            of_even[d] = side ? other : cell[d];
+            of_odd[d] = side ? cell[d] : other;
+        }
+        row_entries<D>(of_even, side, size, res, flags, gp.hash_type, a);
+        row_entries<D>(of_odd, side, size, res, flags, gp.hash_type, b);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            load_entry<P, F>(level + (size_t)a[r] * F, even[u][r]);
+            load_entry<P, F>(level + (size_t)b[r] * F, odd[u][r]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const long long i = i0 + u * kLevelThreads;
+        ovec o;
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            float v = 0.0f;
+            if (nearest) {
+                v = even[u][0][f];
+            } else {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float mine = side ? odd[u][r][f] : even[u][r][f], other = swap_pair(side ? even[u][r][f] : odd[u][r][f]);
+                    const float near = side ? other : mine, far = side ? mine : other;
+                    // the products and the order of encode_levels
+                    float near_weight = 1 - frac[u][0], far_weight = frac[u][0];
+#pragma unroll
+                    for (int d = 1; d < D; ++d) {
+                        const float w = (r & (1 << (d - 1))) ? frac[u][d] : 1 - frac[u][d];
+                        near_weight *= w;
+                        far_weight *= w;
+                    }
+                    v = __builtin_fmaf(near_weight, near, v);
+                    v = __builtin_fmaf(far_weight, far, v);
+                }
+            }
+            o[f] = to_out<O>(as_fp32(v)); // (pinned as encode_levels pins it)
+        }
+        if (i >= M) continue;
+        if constexpr (ROWS) {
+            O *const to = out + (order ? (size_t)row[u] : (size_t)i) * gp.padded_width;
+#pragma unroll
+            for (int f = 0; f < F; ++f) to[l * F + f] = o[f];
+            if (l + 1 == gp.n_levels)
+                for (uint32_t c = gp.n_levels * F; c < gp.padded_width; ++c) to[c] = to_out<O>(0.0f);
+        } else {
+            __builtin_nontemporal_store(o, reinterpret_cast<ovec *>(out + ((size_t)l * pitch + i) * F));
+        }
+    }
+}
+
+// Rows of the encoded matrix from the levels: a thread a piece of PER values, so that a wave writes whole lines. Bound by the bytes (3-D,
+// 16 levels of two features, fp32, 2^20 points: 268 MB in 40 us).
+template <int F, typename O>
+__global__ void __launch_bounds__(256) grid_rows_kernel(const O *__restrict__ levels, const float4 *__restrict__ order, O *__restrict__ out, long long M, size_t pitch,
+                                                        uint32_t n_levels, uint32_t padded_width) {
+    constexpr uint32_t PER = 16 / sizeof(O), TOGETHER = F < (int)PER ? F : PER; // values of a piece; of those that lie side by side in `levels`
+    typedef O piece_t __attribute__((ext_vector_type(PER)));
+    typedef O part_t __attribute__((ext_vector_type(TOGETHER)));
+    const uint32_t pieces = (padded_width + PER - 1) / PER;
+    const bool whole = padded_width % PER == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    const long long n = M * pieces;
+    for (long long t = (long long)blockIdx.x * 256 + threadIdx.x; t < n; t += (long long)gridDim.x * 256) {
+        const long long i = t / pieces;
+        const uint32_t c0 = (uint32_t)(t % pieces) * PER;
+        piece_t v = {};
+#pragma unroll
+        for (uint32_t e = 0; e < PER; e += TOGETHER) {
+            const uint32_t l = (c0 + e) / F, f = (c0 + e) % F;
+            if (l >= n_levels) continue; // zero padding (include/encodings/grid.h:682-694)
+            const part_t part = *reinterpret_cast<const part_t *>(levels + ((size_t)l * pitch + i) * F + f);
+#pragma unroll
+            for (uint32_t k = 0; k < TOGETHER; ++k) v[e + k] = part[k];
+        }
+        O *const to = out + (order ? (size_t)__float_as_uint(order[i].w) : (size_t)i) * padded_width + c0;
+        if (whole) {
+            *reinterpret_cast<piece_t *>(to) = v;
+        } else {
+#pragma unroll
+            for (uint32_t e = 0; e < PER; ++e)
+                if (c0 + e < padded_width) to[e] = v[e];
+        }
+    }
+}
+
+// What 2^23 points cost in a level, us: the loads, and lines from L2 unless the level is a few lines or
+// (in cell order) the lanes of a wave share them; beyond the 4 MB of an XCD's L2 they come from the memory side.
+static double level_cost(const GridLevels &lv, uint32_t l, uint32_t n_dims, size_t entry_bytes, bool ordered, size_t M) {
+    const double bytes = (double)lv.size[l] * (double)entry_bytes, work = n_dims == 2 ? 29.0 : 49.0, lines = n_dims == 2 ? 50.0 : 110.0;
+    double miss = std::min(1.0, std::max(0.0, std::log2(bytes / 16384.0) / 4.0)) * (1.0 + 0.75 * std::max(0.0, std::log2(bytes / (4 << 20))));
+    if (ordered) miss /= 1.0 + 5.0 * (double)M / std::pow((double)lv.resolution[l], (double)n_dims);
+    return work + lines * miss;
+}
+
+// us a batch takes by levels (3-D, 2^19 entries, 2^20 points: 332 measured, 253 in cell order).
+static double levels_us(const GridLevels &lv, uint32_t n_levels, uint32_t n_dims, size_t entry_bytes, bool ordered, size_t M) {
+    double cost = 0.0;
+    for (uint32_t l = 0; l < n_levels; ++l) cost += level_cost(lv, l, n_dims, entry_bytes, ordered, M);
+    return cost * (double)M / (double)(1 << 23);
+}
+
+template <int D, int F, typename P, typename O>
+static int launch_levels(const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *table, void *out, bool rows, size_t M,
+                         hipStream_t s) {
+    LevelPlan plan;
+    const unsigned long long chunks = (M + LevelShape<D, F>::kChunk - 1) / LevelShape<D, F>::kChunk, items = chunks * gp.n_levels;
+    if (items > 0x0fffffffull) return fail(TNN_ERR_UNSUPPORTED, "grid encoding by levels: batch too large for one launch");
+    plan.n_chunks = (uint32_t)chunks;
+    double total = 0.0, cost[TNN_GRID_MAX_LEVELS], before = 0.0;
+    for (uint32_t l = 0; l < gp.n_levels; ++l) total += cost[l] = level_cost(lv, l, D, F * sizeof(P), order != nullptr, M);
+    uint32_t most = 0;
+    for (uint32_t k = 0, l = 0; k <= kXcds; ++k) {
+        const double until = total * k / kXcds;
+        while (l + 1 < gp.n_levels && before + cost[l] < until) before += cost[l++];
+        const double part = std::min(1.0, std::max(0.0, (until - before) / cost[l]));
+        plan.first[k] = k == kXcds ? (uint32_t)items : l * plan.n_chunks + (uint32_t)(part * plan.n_chunks + 0.5);
+        if (k > 0) most = std::max(most, plan.first[k] - plan.first[k - 1]);
+    }
+    auto k = grid_levels_kernel<D, F, P, O, false>;
+    if (rows) k = grid_levels_kernel<D, F, P, O, true>;
+    TNN_LAUNCH(k, dim3(most * kXcds), dim3(kLevelThreads), 0, s, lv, gp, plan, x, order, (const P *)table, (O *)out, (long long)M, level_pitch(M));
+    return check_launch("grid_levels_kernel");
+}
+
+int launch_grid_levels(const tnn_grid_desc *desc, const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *table, void *out,
+                       int out_dtype, uint32_t padded_width, size_t M, hipStream_t s) {
+    GridParams p = gp;
+    p.padded_width = padded_width;
+#define TNN_LEVELS_O(D, F, P)                                                                                                                \
+    switch (out_dtype) {                                                                                                                     \
+    case TNN_FP32: return launch_levels<D, F, P, float>(lv, p, x, order, table, out, padded_width != 0, M, s);                               \
+    case TNN_BF16: return launch_levels<D, F, P, bf16_t>(lv, p, x, order, table, out, padded_width != 0, M, s);                              \
+    case TNN_FP16: return launch_levels<D, F, P, fp16_t>(lv, p, x, order, table, out, padded_width != 0, M, s);                              \
+    default: return fail(TNN_ERR_UNSUPPORTED, "out_dtype %d", out_dtype);                                                                    \
+    }
+#define TNN_LEVELS_P(D, F)                                                                                                                   \
+    if (desc->param_dtype == TNN_FP32) TNN_LEVELS_O(D, F, float)                                                                              \
+    TNN_LEVELS_O(D, F, fp16_t)
+#define TNN_LEVELS_F(D)                                                                                                                      \
+    switch (desc->n_features_per_level) {                                                                                                    \
+    case 1: TNN_LEVELS_P(D, 1)                                                                                                               \
+    case 2: TNN_LEVELS_P(D, 2)                                                                                                               \
+    case 4: TNN_LEVELS_P(D, 4)                                                                                                               \
+    default: TNN_LEVELS_P(D, 8)                                                                                                              \
+    }
+    if (desc->n_dims == 2) { TNN_LEVELS_F(2) }
+    TNN_LEVELS_F(3)
+#undef TNN_LEVELS_F
+#undef TNN_LEVELS_P
+#undef TNN_LEVELS_O
+}
+
+bool grid_rows_direct(size_t M) { return M <= (size_t(1) << 14); }
+
+template <typename O>
+static int launch_rows(uint32_t F, const void *levels, const float4 *order, void *out, uint32_t n_levels, uint32_t padded_width, size_t M, hipStream_t s) {
+    auto k = F == 1 ? grid_rows_kernel<1, O> : F == 2 ? grid_rows_kernel<2, O> : F == 4 ? grid_rows_kernel<4, O> : grid_rows_kernel<8, O>;
+    const size_t pieces = M * ((padded_width * sizeof(O) + 15) / 16);
+    TNN_LAUNCH(k, dim3((unsigned)std::min<size_t>((pieces + 255) / 256, size_t(1) << 20)), dim3(256), 0, s, (const O *)levels, order, (O *)out, (long long)M, level_pitch(M), n_levels,
+               padded_width);
+    return check_launch("grid_rows_kernel");
+}
+
+} // namespace tnn
+
+using namespace tnn;
+
+static size_t dtype_bytes(int dtype) { return dtype == TNN_FP32 ? 4 : 2; }
+static size_t entry_bytes(const tnn_grid_desc *desc) { return desc->n_features_per_level * dtype_bytes(desc->param_dtype); }
+
+TNN_API size_t tnn_grid_forward_workspace_bytes(const tnn_grid_desc *desc, int out_dtype, size_t M) {
+    if (check_grid_desc(desc) || M == 0 || grid_rows_direct(M)) return 0;
+    // Points in cell order walk all levels (grid_forward_kernel) where lines come from the memory side in either case, and in 2-D from
+    // 2^19 points on, where few lines are not shared and the rows are a pass of their own. us, with the ordering (points / levels and
+    // rows): 3-D, 2^18 points, 2^19, 2^20, 2^22 entries 171 / 103, 208 / 163, 220 / 237; 2-D, 2^18 points, 2^19 entries 72 / 56,
+    // 2^20 points 171 / 177 ordered, 193 not.
+    size_t largest = 0;
+    for (uint32_t l = 0; l < desc->n_levels; ++l) largest = std::max<size_t>(largest, (desc->offsets[l + 1] - desc->offsets[l]) * entry_bytes(desc));
+    if (M >= (size_t(1) << 17) && largest > (size_t(8) << 20)) return 0;
+    if (M >= (size_t(1) << 19) && desc->n_dims == 2) return 0;
+    return (size_t)desc->n_levels * level_pitch(M) * desc->n_features_per_level * dtype_bytes(out_dtype) + 256;
+}
+
+TNN_API int tnn_grid_levels_want_order(const tnn_grid_desc *desc, size_t M) {
+    GridLevels lv;
+    GridParams gp;
+    if (check_grid_desc(desc) || grid_common(desc, desc->n_levels * desc->n_features_per_level, M, &lv, &gp)) return 0;
+    if (M < (size_t(1) << 18)) return 0;
+    const double ordering = 20.0 + 22.0 * (double)M / (double)(1 << 20); // us (2^18 points 25, 2^20 46, 2^21 65)
+    return levels_us(lv, gp.n_levels, desc->n_dims, entry_bytes(desc), false, M) - levels_us(lv, gp.n_levels, desc->n_dims, entry_bytes(desc), true, M) > ordering;
+}
+
+TNN_API int tnn_grid_forward_by_level(const tnn_grid_desc *desc, const float *d_x, const void *d_order, const void *d_table, void *d_out, int out_dtype, uint32_t padded_width,
+                                      size_t M, void *d_workspace, size_t workspace_bytes, tnn_stream_t stream) {
+    GridLevels lv;
+    GridParams gp;
+    int rc = grid_common(desc, padded_width, M, &lv, &gp);
+    if (rc) return rc;
+    if ((!d_x && !d_order) || !d_table || !d_out) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    if (reinterpret_cast<uintptr_t>(d_order) & 15) return fail(TNN_ERR_INVALID_ARGUMENT, "d_order must be 16-byte aligned");
+    if (out_dtype != TNN_FP32 && out_dtype != TNN_BF16 && out_dtype != TNN_FP16) return fail(TNN_ERR_UNSUPPORTED, "out_dtype %d", out_dtype);
+    const uintptr_t base = (reinterpret_cast<uintptr_t>(d_workspace) + 255) & ~(uintptr_t)255;
+    const size_t need = (size_t)desc->n_levels * level_pitch(M) * desc->n_features_per_level * dtype_bytes(out_dtype) + (base - reinterpret_cast<uintptr_t>(d_workspace));
+    if (!d_workspace || workspace_bytes < need) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
+    const float4 *order = static_cast<const float4 *>(d_order);
+    void *levels = reinterpret_cast<void *>(base);
+    hipStream_t s = as_stream(stream);
+    if ((rc = launch_grid_levels(desc, lv, gp, d_x, order, d_table, levels, out_dtype, 0, M, s))) return rc;
+    const uint32_t F = desc->n_features_per_level;
+    if (out_dtype == TNN_FP32) return launch_rows<float>(F, levels, order, d_out, desc->n_levels, padded_width, M, s);
+    if (out_dtype == TNN_BF16) return launch_rows<bf16_t>(F, levels, order, d_out, desc->n_levels, padded_width, M, s);
+    return launch_rows<fp16_t>(F, levels, order, d_out, desc->n_levels, padded_width, M, s);
+}

@@ -72,14 +72,7 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
 
     std::unique_ptr<Context> forward_impl(const DeviceMatrixView<float> input, DeviceMatrixView<T> *output = nullptr,
                                           bool use_inference_params = false, bool prepare_input_gradients = false) override {
-        if (this->get_padded_output_width() == 0) throw std::invalid_argument("Can't have width == 0");
-        if (use_inference_params) throw std::invalid_argument("Can't use inference params.");
-        if (prepare_input_gradients) throw std::invalid_argument("Can't prepare input gradients");
-        if (!output) return nullptr;
-        if (output->n() != this->get_padded_output_width()) throw std::invalid_argument("Dimension mismatch grid encoding forw_impl output");
-        if (input.n() != this->get_input_width()) throw std::invalid_argument("Dimension mismatch grid encoding forw_impl input");
-        if (input.stride() != input.n() || output->stride() != output->n()) throw std::invalid_argument("Only dense matrices are supported.");
-        check_max_level();
+        if (!check_forward(input, output, use_inference_params, prepare_input_gradients)) return nullptr;
         const size_t batch = input.m();
         if (batch >= kCellOrderMinBatch) {
             // large batches: order the points by cell first, so that neighbouring lanes gather from the same lines of the
@@ -91,6 +84,16 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
         tnn::abi_check(tnn_grid_forward(&m_desc, input.GetPointer(), this->get_params()->data(), output->GetPointer(), TNN_FP32,
                                         this->get_padded_output_width(), batch, this->get_queue().abi()));
         return nullptr; // enqueued on the encoding's in-order stream; the caller waits on the queue when it needs the host to see it
+    }
+
+    /// forward_impl with scratch memory of the caller's (forward_scratch_bytes of it, used until the pass is over on the stream), which
+    /// large batches are the faster for: same rows, bit for bit.
+    size_t forward_scratch_bytes(const size_t batch_size) const { return tnn_grid_forward_workspace_bytes(&m_desc, TNN_FP32, batch_size); }
+    void forward_with_scratch(const DeviceMatrixView<float> input, DeviceMatrixView<T> *output, void *scratch, const size_t scratch_bytes) {
+        if (!check_forward(input, output, false, false)) return;
+        const void *order = tnn_grid_levels_want_order(&m_desc, input.m()) ? ordered(input) : nullptr;
+        tnn::abi_check(tnn_grid_forward_by_level(&m_desc, input.GetPointer(), order, this->get_params()->data(), output->GetPointer(), TNN_FP32,
+                                                 this->get_padded_output_width(), input.m(), scratch, scratch_bytes, this->get_queue().abi()));
     }
 
     void backward_impl(const Context &, const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput,
@@ -128,6 +131,17 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
 
   private:
     /// Whether there is anything to do; throws where the arguments do not fit.
+    bool check_forward(const DeviceMatrixView<float> input, const DeviceMatrixView<T> *output, bool use_inference_params, bool prepare_input_gradients) const {
+        if (this->get_padded_output_width() == 0) throw std::invalid_argument("Can't have width == 0");
+        if (use_inference_params) throw std::invalid_argument("Can't use inference params.");
+        if (prepare_input_gradients) throw std::invalid_argument("Can't prepare input gradients");
+        if (!output) return false;
+        if (output->n() != this->get_padded_output_width()) throw std::invalid_argument("Dimension mismatch grid encoding forw_impl output");
+        if (input.n() != this->get_input_width()) throw std::invalid_argument("Dimension mismatch grid encoding forw_impl input");
+        if (input.stride() != input.n() || output->stride() != output->n()) throw std::invalid_argument("Only dense matrices are supported.");
+        check_max_level();
+        return true;
+    }
     bool check_backward(const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput, const DeviceMatrixView<T> *gradients,
                         const DeviceMatrix<float> *dL_dinput, bool use_inference_params, GradientMode param_gradients_mode) const {
         if (input.m() == 0) throw std::invalid_argument("batch_size == 0");

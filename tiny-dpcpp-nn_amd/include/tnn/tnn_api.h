@@ -233,7 +233,13 @@ template <typename T> class EncodingModule : public Module {
         // the kernel writes the tensor that is handed back (a fresh allocation as the reference's clone is, without the copy)
         torch::Tensor output = torch::empty({(int64_t)batch_size, (int64_t)out_w}, torch::TensorOptions().dtype(torch_type<T>::dtype).device(device()));
         DeviceMatrixView<T> output_encoding(batch_size, out_w, out_w, reinterpret_cast<T *>(output.data_ptr()));
-        std::unique_ptr<Context> model_ctx = encoding_->forward_impl(input_dmv, &output_encoding);
+        auto *grid = dynamic_cast<tinydpcppnn::encodings::grid::GridEncodingTemplated<T> *>(encoding_.get());
+        if (const size_t need = grid ? grid->forward_scratch_bytes(batch_size) : 0) {
+            const torch::Tensor work = this->scratch(need);
+            grid->forward_with_scratch(input_dmv, &output_encoding, work.data_ptr(), (size_t)work.numel());
+        } else {
+            encoding_->forward_impl(input_dmv, &output_encoding);
+        }
         this->finish();
         return output;
     }
@@ -273,7 +279,6 @@ template <typename T> class EncodingModule : public Module {
         last_gradients_ = torch::empty({(int64_t)encoding_->get_n_params(), 1}, torch::TensorOptions().dtype(torch_type<T>::dtype).device(device()));
         DeviceMatrixView<T> gradients_view(encoding_->get_n_params(), 1, 1, reinterpret_cast<T *>(last_gradients_.data_ptr()));
         Context ctx;
-        auto *grid = dynamic_cast<tinydpcppnn::encodings::grid::GridEncodingTemplated<T> *>(encoding_.get());
         if (auto *grid = dynamic_cast<tinydpcppnn::encodings::grid::GridEncodingTemplated<T> *>(encoding_.get())) {
             const torch::Tensor work = this->scratch(grid->backward_scratch_bytes((size_t)batch_size));
             grid->backward_with_scratch(input_encoding_dmv, dL_doutput_dmv, &gradients_view, work.data_ptr(), (size_t)work.numel());

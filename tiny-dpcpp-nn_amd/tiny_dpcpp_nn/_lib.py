@@ -137,6 +137,9 @@ SIGNATURES = {
     "tnn_grid_forward": (c_int, [POINTER(GridDesc), c_void_p, c_void_p, c_void_p, c_int, c_uint32, c_size_t, c_void_p]),
     "tnn_grid_order_bytes": (c_size_t, [POINTER(GridDesc), c_size_t]),
     "tnn_grid_order_points": (c_int, [POINTER(GridDesc), c_void_p, c_size_t, c_void_p, c_size_t, c_void_p]),
+    "tnn_grid_forward_workspace_bytes": (c_size_t, [POINTER(GridDesc), c_int, c_size_t]),
+    "tnn_grid_levels_want_order": (c_int, [POINTER(GridDesc), c_size_t]),
+    "tnn_grid_forward_by_level": (c_int, [POINTER(GridDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_uint32, c_size_t, c_void_p, c_size_t, c_void_p]),
     "tnn_grid_forward_ordered": (c_int, [POINTER(GridDesc), c_void_p, c_void_p, c_void_p, c_int, c_uint32, c_size_t, c_void_p]),
     "tnn_grid_backward": (c_int, [POINTER(GridDesc), c_void_p, c_void_p, c_int, c_uint32, c_void_p, c_int, c_size_t, c_void_p]),
     "tnn_grid_backward_ordered": (c_int, [POINTER(GridDesc), c_void_p, c_void_p, c_int, c_uint32, c_void_p, c_int, c_size_t, c_void_p]),
