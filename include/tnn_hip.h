@@ -367,7 +367,7 @@ int tnn_grid_forward_ordered(const tnn_grid_desc *desc, const void *d_order, con
  * second pass makes rows of them. Same values, bit for bit. d_order (may be NULL): the records of tnn_grid_order_points, then d_x may be
  * NULL. tnn_grid_forward_workspace_bytes: the workspace it takes where it is the faster call for M points, 0 where it is not (small
  * batches, whose rows tnn_grid_forward writes the same way; large ones of two dimensions or of levels beyond 8 MB). Any M runs, with
- * n_levels * n_features_per_level * sizeof(out_dtype) bytes for each of M points rounded up to 64, and 256 more.
+ * (n_levels * n_features_per_level rounded up to 16) * sizeof(out_dtype) bytes for each of M points rounded up to 64, and 256 more.
  * tnn_grid_levels_want_order: whether it (with tnn_grid_order_points in front) is the faster for cell order. */
 size_t tnn_grid_forward_workspace_bytes(const tnn_grid_desc *desc, int out_dtype, size_t M);
 int tnn_grid_levels_want_order(const tnn_grid_desc *desc, size_t M);
@@ -437,12 +437,12 @@ int tnn_grid_mlp_inference(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, c
 int tnn_grid_mlp_inference_ordered(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const void *d_order, const void *d_table,
                                    const void *d_prepared_fwd, void *d_y, size_t M, tnn_stream_t stream);
 
-/* One optimisation step of a network behind a hash-grid encoding without the encoded matrix (the training half of the
- * fused path above): what the reference's training loop does with Encoding.forward, Network.forward, the L2 loss,
+/* One optimisation step of a network behind a hash-grid encoding (the training half of the
+ * path above): what the reference's training loop does with Encoding.forward, Network.forward, the L2 loss,
  * loss.backward() through both modules and optimizer.step() on the network's parameters
  * (dpcpp_bindings/tiny_dpcpp_nn/modules.py:357-421 over include/encodings/grid.h:661-797 and include/trainer.h:23-46).
- * The encoding is evaluated inside the training kernel where tnn_mlp_train_step_l2_adam loads its input rows, so the
- * M x width encoded matrix is neither written nor read; dL/d(encoding) goes through the workspace into the scatter of
+ * The encoding is evaluated level by level (tnn_grid_forward_by_level) in the network's type, and the training kernel reads the levels
+ * where tnn_mlp_train_step_l2_adam loads its input rows; dL/d(encoding) goes through the workspace into the scatter of
  * tnn_grid_backward (tnn_grid_backward_ordered when d_order is given). Same values as tnn_grid_forward (out_dtype = network
  * type, padded_width = width) + tnn_mlp_train_step_l2_adam (with d_dLdx) + tnn_grid_backward. With d_x (the caller's order):
  * outputs, loss, Adam state and re-staged weights bit for bit, the table's gradient up to the order of its fp32 additions
@@ -455,8 +455,8 @@ int tnn_grid_mlp_inference_ordered(const tnn_grid_desc *grid, const tnn_mlp_desc
  *   d_grad_table: n_params fp32, overwritten or accumulated into as in tnn_grid_backward; it holds loss_scale x the gradient.
  *   Network arguments as in tnn_mlp_train_step_l2_adam. Built for width 64, ReLU, at most 4 hidden layers and 2 features per
  *   level (tnn_grid_mlp_train_supported returns TNN_OK); other shapes get TNN_ERR_UNSUPPORTED and run the three calls.
- * Workspace: tnn_grid_mlp_train_step_workspace_bytes: what tnn_grid_backward_binned needs, which is most of it, dL/d(encoding) and the
- * workgroups' partial gradients (211 MiB for 2^18 points of a 2-D grid of 16 levels and 2^19 entries). */
+ * Workspace: tnn_grid_mlp_train_step_workspace_bytes: what tnn_grid_backward_binned needs, which is most of it (and holds the encoded levels
+ * before), dL/d(encoding) and the workgroups' partial gradients (211 MiB for 2^18 points of a 2-D grid of 16 levels and 2^19 entries). */
 int tnn_grid_mlp_train_supported(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp);
 size_t tnn_grid_mlp_train_step_workspace_bytes(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, size_t M);
 int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order,
@@ -464,10 +464,10 @@ int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn_mlp_des
                                     float loss_scale, void *d_y, float *d_loss_sum, float *d_master_packed, float *d_m, float *d_v,
                                     int step, float lr, float beta1, float beta2, float eps, void *d_packed_T, float *d_grad_table,
                                     int overwrite, size_t M, void *d_workspace, size_t workspace_bytes, tnn_stream_t stream);
-/* The backward pass of a network behind a hash-grid encoding for a given dL/dy, without the encoded matrix: what
+/* The backward pass of a network behind a hash-grid encoding for a given dL/dy: what
  * loss.backward() does through NetworkWithInputEncoding in the reference (dpcpp_bindings/tiny_dpcpp_nn/modules.py:84-136 over
  * Network::backward_pass and GridEncoding::backward_impl, include/encodings/grid.h:752-797). The encoding and the
- * network's forward pass are formed again on chip from the positions (tnn_grid_mlp_inference is the forward pass that goes
+ * network's forward pass are formed again from the positions (tnn_grid_mlp_inference is the forward pass that goes
  * with it), the weight gradients leave as in tnn_mlp_backward_recompute, and dL/d(encoding) goes through the workspace into
  * the scatter of tnn_grid_backward (tnn_grid_backward_ordered when d_order is given). d_grad_table: n_params fp32, or NULL
  * when only the network's gradients are wanted. Shapes and workspace as tnn_grid_mlp_train_step_l2_adam. */

@@ -21,7 +21,7 @@ def bits(t):
 
 def by_level(tnn, d, x, order, table, width, out_dtype):
     M = x.shape[0]
-    need = d.n_levels * d.n_features_per_level * TORCH[out_dtype].itemsize * ((M + 63) // 64 * 64) + 256
+    need = (d.n_levels * d.n_features_per_level + 15) // 16 * 16 * TORCH[out_dtype].itemsize * ((M + 63) // 64 * 64) + 256
     work = torch.empty(need, dtype=torch.uint8, device=tnn.dev)
     out = torch.full((M, width), 7.0, dtype=TORCH[out_dtype], device=tnn.dev)
     args = (ctypes.byref(d), ptr(x) if order is None else None, ptr(order) if order is not None else None, ptr(table), ptr(out), out_dtype, width, M, ptr(work))

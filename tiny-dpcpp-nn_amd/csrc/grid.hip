@@ -824,10 +824,9 @@ TNN_API int tnn_grid_forward_ordered(const tnn_grid_desc *desc, const void *d_or
 }
 
 namespace tnn {
-// by_position: dL/dy as the training kernel leaves it (GradLayout); d_x may be given beside d_order, for the routes that read
-// the rows of a row-major dL/dy better in the caller's order.
+// d_x may be given beside d_order, for the routes that read the rows of a row-major dL/dy better in the caller's order.
 int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4 *d_order, const void *d_dLdy, int dy_dtype, uint32_t padded_width,
-                       bool by_position, float scale, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
+                       const GradLayout &dl, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
                        hipStream_t s) {
     GridLevels lv;
     GridParams gp;
@@ -863,12 +862,11 @@ int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4
                    reinterpret_cast<float *>(static_cast<char *>(d_grad_table) + n4 * 16), n_tail);
         if ((rc = check_launch("fill_zero_kernel"))) return rc;
     }
-    const GradLayout dl{padded_width, n_features, by_position ? 1 : 0, scale};
     if (grad_dtype == TNN_FP32) {
         TNN_DISPATCH_DF(desc, rc = (launch_grid_backward_g<D_, F_, float>(lv, gp, bp, dl, n_big, lds_bytes, d_x, d_order, d_dLdy, dy_dtype,
                                                                           (float *)d_grad_table, M, s)));
         if (rc == TNN_OK && bins.n_levels)
-            rc = launch_grid_binned(bins, lv, gp, dl, desc->n_dims, n_features, d_x, d_x && !by_position ? nullptr : d_order, d_dLdy, dy_dtype, (float *)d_grad_table, overwrite != 0, M,
+            rc = launch_grid_binned(bins, lv, gp, dl, desc->n_dims, n_features, d_x, d_x && !dl.by_position ? nullptr : d_order, d_dLdy, dy_dtype, (float *)d_grad_table, overwrite != 0, M,
                                     reinterpret_cast<void *>(scratch), s);
     } else {
         const uint32_t F = desc->n_features_per_level;
@@ -885,15 +883,18 @@ int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4
 }
 } // namespace tnn
 
+// A caller's row-major dL/dy.
+static GradLayout rows_of(const tnn_grid_desc *desc, uint32_t padded_width) { return GradLayout{padded_width, desc ? desc->n_features_per_level : 0, 0, 1.0f}; }
+
 TNN_API int tnn_grid_backward(const tnn_grid_desc *desc, const float *d_x, const void *d_dLdy, int dy_dtype,
                               uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, tnn_stream_t stream) {
-    return grid_backward_impl(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, false, 1.0f, d_grad_table, TNN_FP32, overwrite, M, nullptr, 0, as_stream(stream));
+    return grid_backward_impl(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, rows_of(desc, padded_width), d_grad_table, TNN_FP32, overwrite, M, nullptr, 0, as_stream(stream));
 }
 
 TNN_API int tnn_grid_backward_ordered(const tnn_grid_desc *desc, const void *d_order, const void *d_dLdy, int dy_dtype,
                                       uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, tnn_stream_t stream) {
     if (!d_order) return tnn::fail(TNN_ERR_INVALID_ARGUMENT, "d_order is NULL");
-    return grid_backward_impl(desc, nullptr, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, false, 1.0f, d_grad_table, TNN_FP32,
+    return grid_backward_impl(desc, nullptr, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, rows_of(desc, padded_width), d_grad_table, TNN_FP32,
                               overwrite, M, nullptr, 0, as_stream(stream));
 }
 
@@ -931,13 +932,13 @@ TNN_API int tnn_grid_backward_binned(const tnn_grid_desc *desc, const float *d_x
                                      uint32_t padded_width, float *d_grad_table, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
                                      tnn_stream_t stream) {
     if (!d_workspace) return tnn::fail(TNN_ERR_WORKSPACE, "grid backward: no workspace");
-    return grid_backward_impl(desc, d_x, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, false, 1.0f, d_grad_table, TNN_FP32, overwrite,
+    return grid_backward_impl(desc, d_x, static_cast<const float4 *>(d_order), d_dLdy, dy_dtype, padded_width, rows_of(desc, padded_width), d_grad_table, TNN_FP32, overwrite,
                               M, d_workspace, workspace_bytes, as_stream(stream));
 }
 
 TNN_API int tnn_grid_backward_packed(const tnn_grid_desc *desc, const float *d_x, const void *d_dLdy, int dy_dtype,
                                      uint32_t padded_width, void *d_grad_table_f16, int overwrite, size_t M, tnn_stream_t stream) {
-    return grid_backward_impl(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, false, 1.0f, d_grad_table_f16, TNN_FP16, overwrite, M, nullptr, 0, as_stream(stream));
+    return grid_backward_impl(desc, d_x, nullptr, d_dLdy, dy_dtype, padded_width, rows_of(desc, padded_width), d_grad_table_f16, TNN_FP16, overwrite, M, nullptr, 0, as_stream(stream));
 }
 
 TNN_API int tnn_grid_indices(const tnn_grid_desc *desc, const float *d_x, uint32_t *d_indices, size_t M, tnn_stream_t stream) {

@@ -28,10 +28,10 @@ struct GridParams {
 };
 
 // Where dL/dy of a point and level lies: element (row, level, feature) at row * row_stride + level * level_stride + feature. A
-// caller's matrix is row-major in the caller's order; the training kernel writes its rows in the order it visits the points, so
-// that the scatter finds those of neighbouring points in the same lines (`by_position`: the row is the point's place).
+// caller's matrix is row-major in the caller's order; the training kernel writes a row of points per level, in the order it visits the
+// points (`by_position`: the row is the point's place), so that the scatter, a level at a time, reads nothing else.
 struct GradLayout {
-    uint32_t row_stride, level_stride;
+    size_t row_stride, level_stride;
     int by_position;
     float scale; // every value is multiplied by this as it is read
 };
@@ -39,9 +39,6 @@ struct GradLayout {
 // The buffer of tnn_grid_order_points (grid_order.hip): M records of 16 bytes, padded to 256 bytes, then the first position
 // of each of the 4096 coarse cells of the order (uint32, key order), which the scatter over ordered points reads.
 inline size_t order_record_bytes(size_t M) { return (M * 16 + 255) & ~(size_t)255; }
-
-// Pitch of the rows the training kernel writes for a grid of two features per level: whole 16-byte pieces.
-__host__ __device__ inline uint32_t gradient_pitch(uint32_t n_levels) { return (n_levels * 2 + 7) & ~7u; }
 
 // Leading `bits` bits of a coordinate taken as a number in [0, 1); anything else (outside, NaN) goes to an end bin.
 __device__ __forceinline__ uint32_t quantise(float v, int bits) {
@@ -59,7 +56,7 @@ template <> struct OrderBits<3> { static constexpr int coarse = 4, fine = 2; };
 // the per-level constants the kernels take.
 int check_grid_desc(const tnn_grid_desc *d);
 int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4 *d_order, const void *d_dLdy, int dy_dtype, uint32_t padded_width,
-                       bool by_position, float scale, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
+                       const GradLayout &dl, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
                        hipStream_t s);
 int grid_common(const tnn_grid_desc *desc, uint32_t padded_width, size_t M, GridLevels *lv, GridParams *gp);
 

@@ -157,7 +157,7 @@ __global__ void __launch_bounds__(kLevelThreads)
             }
             o[f] = to_out<O>(as_fp32(v)); // (pinned as encode_levels pins it)
         }
-        if (i >= M) continue;
+        if (i >= (ROWS ? M : (long long)pitch)) continue;
         if constexpr (ROWS) {
             O *const to = out + (order ? (size_t)row[u] : (size_t)i) * gp.padded_width;
 #pragma unroll
@@ -166,6 +166,8 @@ __global__ void __launch_bounds__(kLevelThreads)
                 for (uint32_t c = gp.n_levels * F; c < gp.padded_width; ++c) to[c] = to_out<O>(0.0f);
         } else {
             __builtin_nontemporal_store(o, reinterpret_cast<ovec *>(out + ((size_t)l * pitch + i) * F));
+            if (l + 1 == gp.n_levels)
+                for (uint32_t p = l + 1; p < padded_levels(gp.n_levels, F); ++p) *reinterpret_cast<ovec *>(out + ((size_t)p * pitch + i) * F) = ovec{};
         }
     }
 }
@@ -299,7 +301,7 @@ TNN_API size_t tnn_grid_forward_workspace_bytes(const tnn_grid_desc *desc, int o
     for (uint32_t l = 0; l < desc->n_levels; ++l) largest = std::max<size_t>(largest, (desc->offsets[l + 1] - desc->offsets[l]) * entry_bytes(desc));
     if (M >= (size_t(1) << 17) && largest > (size_t(8) << 20)) return 0;
     if (M >= (size_t(1) << 19) && desc->n_dims == 2) return 0;
-    return (size_t)desc->n_levels * level_pitch(M) * desc->n_features_per_level * dtype_bytes(out_dtype) + 256;
+    return levels_elements(desc, M) * dtype_bytes(out_dtype) + 256;
 }
 
 TNN_API int tnn_grid_levels_want_order(const tnn_grid_desc *desc, size_t M) {
@@ -321,7 +323,7 @@ TNN_API int tnn_grid_forward_by_level(const tnn_grid_desc *desc, const float *d_
     if (reinterpret_cast<uintptr_t>(d_order) & 15) return fail(TNN_ERR_INVALID_ARGUMENT, "d_order must be 16-byte aligned");
     if (out_dtype != TNN_FP32 && out_dtype != TNN_BF16 && out_dtype != TNN_FP16) return fail(TNN_ERR_UNSUPPORTED, "out_dtype %d", out_dtype);
     const uintptr_t base = (reinterpret_cast<uintptr_t>(d_workspace) + 255) & ~(uintptr_t)255;
-    const size_t need = (size_t)desc->n_levels * level_pitch(M) * desc->n_features_per_level * dtype_bytes(out_dtype) + (base - reinterpret_cast<uintptr_t>(d_workspace));
+    const size_t need = levels_elements(desc, M) * dtype_bytes(out_dtype) + (base - reinterpret_cast<uintptr_t>(d_workspace));
     if (!d_workspace || workspace_bytes < need) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
     const float4 *order = static_cast<const float4 *>(d_order);
     void *levels = reinterpret_cast<void *>(base);

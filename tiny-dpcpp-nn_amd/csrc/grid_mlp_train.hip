@@ -1,24 +1,22 @@
-// C entry points of the training step on an encoded input without the encoded matrix: hash-grid encoding, network
+// C entry points of the training step on an encoded input: hash-grid encoding by levels (grid_levels.hip), network
 // forward, L2 loss, backward pass and Adam on the network's weights (kernels: grid_mlp_train.inc, built once per network
 // type), then the scatter of dL/d(encoding) into the table's gradient (grid.hip).
-#include "grid_device.h"
+#include "grid_levels.h"
 #include "mlp_train_shape.h"
 
+#include <algorithm>
+
 namespace tnn {
-int grid_mlp_train_launch_bf16(const tnn_grid_desc *g, const tnn_mlp_desc *d, const FusedPlan &p, const GridLevels &lv, const GridParams &gp,
-                               const float *x, const float4 *order, const void *table, const void *wf, const void *wb, const float *targets,
-                               float loss_scale, void *y, float *loss_sum, void *d_enc, size_t M, float *partials, float *loss_partials,
-                               const TrainTail &tail, hipStream_t s);
-int grid_mlp_train_launch_fp16(const tnn_grid_desc *g, const tnn_mlp_desc *d, const FusedPlan &p, const GridLevels &lv, const GridParams &gp,
-                               const float *x, const float4 *order, const void *table, const void *wf, const void *wb, const float *targets,
-                               float loss_scale, void *y, float *loss_sum, void *d_enc, size_t M, float *partials, float *loss_partials,
-                               const TrainTail &tail, hipStream_t s);
-int grid_mlp_given_launch_bf16(const tnn_grid_desc *g, const tnn_mlp_desc *d, const FusedPlan &p, const GridLevels &lv, const GridParams &gp,
-                               const float *x, const float4 *order, const void *table, const void *wf, const void *wb, const void *dLdy,
-                               void *d_enc, size_t M, float *partials, float *loss_partials, const TrainTail &tail, hipStream_t s);
-int grid_mlp_given_launch_fp16(const tnn_grid_desc *g, const tnn_mlp_desc *d, const FusedPlan &p, const GridLevels &lv, const GridParams &gp,
-                               const float *x, const float4 *order, const void *table, const void *wf, const void *wb, const void *dLdy,
-                               void *d_enc, size_t M, float *partials, float *loss_partials, const TrainTail &tail, hipStream_t s);
+#define TNN_DECLARE(T)                                                                                                                                 \
+    int grid_mlp_train_launch_##T(const tnn_mlp_desc *d, const FusedPlan &p, const void *levels, uint32_t n_levels, const float4 *order, const void *wf, \
+                                  const void *wb, const float *targets, float loss_scale, void *y, float *loss_sum, void *d_enc, size_t M,               \
+                                  float *partials, float *loss_partials, const TrainTail &tail, hipStream_t s);                                        \
+    int grid_mlp_given_launch_##T(const tnn_mlp_desc *d, const FusedPlan &p, const void *levels, uint32_t n_levels, const float4 *order, const void *wf, \
+                                  const void *wb, const void *dLdy, void *d_enc, size_t M, float *partials, float *loss_partials, const TrainTail &tail, \
+                                  hipStream_t s);
+TNN_DECLARE(bf16)
+TNN_DECLARE(fp16)
+#undef TNN_DECLARE
 } // namespace tnn
 
 using namespace tnn;
@@ -45,13 +43,45 @@ TNN_API int tnn_grid_mlp_train_supported(const tnn_grid_desc *grid, const tnn_ml
     return train_shape_check(grid, mlp, 8, &lv, &gp, &plan);
 }
 
+// Where a pass keeps what: dL/d(encoding) by levels for the scatter, the partial weight gradients and losses of the workgroups, and a
+// part that first holds the encoded levels and then, when the network is through with them, what the scatter sorts the contributions into.
+struct GridTrainMemory {
+    size_t levels_bytes, bytes;
+    void *enc_grad = nullptr, *levels = nullptr;
+    float *loss_partials = nullptr, *partials = nullptr;
+    void *scatter = nullptr;
+    size_t scatter_bytes = 0;
+
+    GridTrainMemory(const tnn_grid_desc *grid, const FusedPlan &plan, size_t M)
+        : levels_bytes(align256(levels_elements(grid, M) * 2)),
+          bytes(levels_bytes + align256(plan.loss_bytes) + align256(plan.partial_bytes) + 512 + std::max(levels_bytes, tnn_grid_backward_workspace_bytes(grid, M))) {}
+    void place(const FusedPlan &plan, void *workspace, size_t workspace_bytes) {
+        uintptr_t base = align256(reinterpret_cast<uintptr_t>(workspace));
+        enc_grad = reinterpret_cast<void *>(base);
+        base += levels_bytes;
+        loss_partials = reinterpret_cast<float *>(base);
+        base += align256(plan.loss_bytes);
+        partials = reinterpret_cast<float *>(base);
+        base += align256(plan.partial_bytes);
+        levels = scatter = reinterpret_cast<void *>(base);
+        scatter_bytes = workspace_bytes - (base - reinterpret_cast<uintptr_t>(workspace));
+    }
+};
+
+// dL/d(encoding), in the network's type, by levels and in the order the kernel took the points, into the table's gradient
+static int scatter_levels(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const float4 *order, const GridTrainMemory &m, float scale,
+                          float *d_grad_table, int overwrite, size_t M, hipStream_t s) {
+    const GradLayout dl{grid->n_features_per_level, level_pitch(M) * grid->n_features_per_level, 1, scale};
+    return grid_backward_impl(grid, order ? nullptr : d_x, order, m.enc_grad, mlp->dtype, (uint32_t)mlp->width, dl, d_grad_table, TNN_FP32, overwrite, M, m.scatter,
+                              m.scatter_bytes, s);
+}
+
 TNN_API size_t tnn_grid_mlp_train_step_workspace_bytes(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, size_t M) {
     GridLevels lv;
     GridParams gp;
     FusedPlan plan;
     if (train_shape_check(grid, mlp, M ? M : 8, &lv, &gp, &plan)) return 0;
-    // dL/d(encoding) for the scatter, then the partial weight gradients and losses of the workgroups, and what the scatter sorts the contributions into
-    return align256(M * gradient_pitch(grid->n_levels) * 2) + align256(plan.loss_bytes) + align256(plan.partial_bytes) + 512 + tnn_grid_backward_workspace_bytes(grid, M ? M : 8);
+    return GridTrainMemory(grid, plan, M ? M : 8).bytes;
 }
 
 TNN_API int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order,
@@ -70,32 +100,22 @@ TNN_API int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn
     if (reinterpret_cast<uintptr_t>(d_order) & 15) return fail(TNN_ERR_INVALID_ARGUMENT, "d_order must be 16-byte aligned");
     if (loss_scale == 0.0f) return fail(TNN_ERR_INVALID_ARGUMENT, "loss_scale must not be 0");
     if (step < 1) return fail(TNN_ERR_INVALID_ARGUMENT, "step counts from 1");
-    const size_t need = tnn_grid_mlp_train_step_workspace_bytes(grid, mlp, M);
-    if (!d_workspace || workspace_bytes < need) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
+    GridTrainMemory m(grid, plan, M);
+    if (!d_workspace || workspace_bytes < m.bytes) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, m.bytes);
+    m.place(plan, d_workspace, workspace_bytes);
     hipStream_t s = as_stream(stream);
-    uintptr_t base = align256(reinterpret_cast<uintptr_t>(d_workspace));
-    void *d_enc_grad = reinterpret_cast<void *>(base);
-    base += align256(M * gradient_pitch(grid->n_levels) * 2);
-    float *loss_partials = reinterpret_cast<float *>(base);
-    base += align256(plan.loss_bytes);
-    float *partials = reinterpret_cast<float *>(base);
 
     TrainTail tail;
     tail.use_adam = true;
     tail.adam = make_adam_args(d_master_packed, d_m, d_v, 1.0f / loss_scale, step, lr, beta1, beta2, eps, d_packed_T, d_prepared_fwd, d_prepared_bwd,
                                mlp->width);
     const float4 *order = static_cast<const float4 *>(d_order);
-    if (mlp->dtype == TNN_BF16)
-        rc = grid_mlp_train_launch_bf16(grid, mlp, plan, lv, gp, d_x, order, d_table, d_prepared_fwd, d_prepared_bwd, d_targets, loss_scale, d_y,
-                                        d_loss_sum, d_enc_grad, M, partials, loss_partials, tail, s);
-    else
-        rc = grid_mlp_train_launch_fp16(grid, mlp, plan, lv, gp, d_x, order, d_table, d_prepared_fwd, d_prepared_bwd, d_targets, loss_scale, d_y,
-                                        d_loss_sum, d_enc_grad, M, partials, loss_partials, tail, s);
-    if (rc) return rc;
-    // dL/d(encoding), in the network's type and in the order the kernel took the points, into the table's gradient
-    base += align256(plan.partial_bytes);
-    return grid_backward_impl(grid, d_order ? nullptr : d_x, order, d_enc_grad, mlp->dtype, gradient_pitch(grid->n_levels), true, 1.0f, d_grad_table, TNN_FP32, overwrite, M,
-                              reinterpret_cast<void *>(base), workspace_bytes - (base - reinterpret_cast<uintptr_t>(d_workspace)), s);
+    if ((rc = launch_grid_levels(grid, lv, gp, d_x, order, d_table, m.levels, mlp->dtype, 0, M, s))) return rc;
+    const auto launch = mlp->dtype == TNN_BF16 ? grid_mlp_train_launch_bf16 : grid_mlp_train_launch_fp16;
+    if ((rc = launch(mlp, plan, m.levels, grid->n_levels, order, d_prepared_fwd, d_prepared_bwd, d_targets, loss_scale, d_y, d_loss_sum, m.enc_grad, M, m.partials,
+                     m.loss_partials, tail, s)))
+        return rc;
+    return scatter_levels(grid, mlp, d_x, order, m, 1.0f, d_grad_table, overwrite, M, s);
 }
 
 static int grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,
@@ -109,28 +129,17 @@ static int grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp,
     if ((!d_x && !d_order) || !d_table || !d_prepared_fwd || !d_prepared_bwd || !d_dLdy || (!tail.dW && !tail.packed.p))
         return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
     if (reinterpret_cast<uintptr_t>(d_order) & 15) return fail(TNN_ERR_INVALID_ARGUMENT, "d_order must be 16-byte aligned");
-    const size_t need = tnn_grid_mlp_train_step_workspace_bytes(grid, mlp, M);
-    if (!d_workspace || workspace_bytes < need) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
-    uintptr_t base = align256(reinterpret_cast<uintptr_t>(d_workspace));
-    void *d_enc_grad = reinterpret_cast<void *>(base);
-    base += align256(M * gradient_pitch(grid->n_levels) * 2);
-    float *loss_partials = reinterpret_cast<float *>(base);
-    base += align256(plan.loss_bytes);
-    float *partials = reinterpret_cast<float *>(base);
+    GridTrainMemory m(grid, plan, M);
+    if (!d_workspace || workspace_bytes < m.bytes) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, m.bytes);
+    m.place(plan, d_workspace, workspace_bytes);
     const float4 *order = static_cast<const float4 *>(d_order);
+    if ((rc = launch_grid_levels(grid, lv, gp, d_x, order, d_table, m.levels, mlp->dtype, 0, M, s))) return rc;
     // without a gradient table the network's gradients are all that is asked for: no dL/d(encoding) leaves the kernel
-    void *enc_out = d_grad_table ? d_enc_grad : nullptr;
-    if (mlp->dtype == TNN_BF16)
-        rc = grid_mlp_given_launch_bf16(grid, mlp, plan, lv, gp, d_x, order, d_table, d_prepared_fwd, d_prepared_bwd, d_dLdy, enc_out, M, partials,
-                                        loss_partials, tail, s);
-    else
-        rc = grid_mlp_given_launch_fp16(grid, mlp, plan, lv, gp, d_x, order, d_table, d_prepared_fwd, d_prepared_bwd, d_dLdy, enc_out, M, partials,
-                                        loss_partials, tail, s);
+    const auto launch = mlp->dtype == TNN_BF16 ? grid_mlp_given_launch_bf16 : grid_mlp_given_launch_fp16;
+    rc = launch(mlp, plan, m.levels, grid->n_levels, order, d_prepared_fwd, d_prepared_bwd, d_dLdy, d_grad_table ? m.enc_grad : nullptr, M, m.partials, m.loss_partials,
+                tail, s);
     if (rc || !d_grad_table) return rc;
-    base += align256(plan.partial_bytes);
-    return grid_backward_impl(grid, d_order ? nullptr : d_x, order, d_enc_grad, mlp->dtype, gradient_pitch(grid->n_levels), true, tail.result_scale,
-                              d_grad_table, TNN_FP32, overwrite, M, reinterpret_cast<void *>(base),
-                              workspace_bytes - (base - reinterpret_cast<uintptr_t>(d_workspace)), s);
+    return scatter_levels(grid, mlp, d_x, order, m, tail.result_scale, d_grad_table, overwrite, M, s);
 }
 
 TNN_API int tnn_grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,
