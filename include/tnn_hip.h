@@ -488,6 +488,21 @@ int tnn_grid_mlp_backward_rows(const tnn_grid_desc *grid, const tnn_mlp_desc *ml
                                const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_dLdy, int dy_cols, float dy_scale,
                                float result_scale, void *d_dW_packed, int dW_dtype, float *d_grad_table, int overwrite, size_t M,
                                void *d_workspace, size_t workspace_bytes, tnn_stream_t stream);
+/* Forward and backward pass of a network behind a grid encoding by levels: tnn_grid_mlp_inference_rows (d_src_packed NULL) or
+ * tnn_grid_mlp_push_inference_rows with the encoding level by level, which leaves the encoded batch in d_levels (tnn_grid_levels_bytes, 16-byte
+ * aligned; values in the network's type); and tnn_grid_mlp_backward_rows on these levels instead of the table. The backward pass of a forward
+ * pass that was given d_order takes the same records. Same values as those calls, bit for bit.
+ * tnn_grid_mlp_wants_levels: whether the forward pass is the faster this way for M points (where not, its bytes of scratch buy nothing). */
+size_t tnn_grid_levels_bytes(const tnn_grid_desc *grid, size_t M);
+int tnn_grid_mlp_wants_levels(const tnn_grid_desc *grid, size_t M);
+int tnn_grid_mlp_forward_levels(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_src_packed, int unpadded_input_width,
+                                int unpadded_output_width, int use_bias, void *d_packed_T, void *d_packed_transposed_T, void *d_prepared_fwd,
+                                void *d_prepared_bwd, const float *d_x, const void *d_order, const void *d_table, void *d_levels, void *d_y,
+                                int y_cols, size_t M, tnn_stream_t stream);
+int tnn_grid_mlp_backward_levels_rows(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order,
+                                      const void *d_levels, const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_dLdy, int dy_cols,
+                                      float dy_scale, float result_scale, void *d_dW_packed, int dW_dtype, float *d_grad_table, int overwrite, size_t M,
+                                      void *d_workspace, size_t workspace_bytes, tnn_stream_t stream);
 /* TNN_OK when tnn_grid_mlp_inference runs this pair of shapes, otherwise the status (and tnn_last_error the reason) it
  * would return: lets a caller choose between the fused call and the two calls once, when the modules are built. */
 int tnn_grid_mlp_supported(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp);

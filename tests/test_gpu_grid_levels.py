@@ -90,3 +90,43 @@ def test_a_small_batch_in_a_graph_replays(tnn):
         torch.cuda.synchronize()
         got = out.clone()
         assert np.isfinite(got.cpu().numpy()).all() and torch.equal(got, tnn.grid_forward(d, x, table, 32))
+
+
+@pytest.mark.parametrize("W,F,n_levels,dims,dtype,n_hidden,M,y_cols", [
+    (64, 2, 16, 3, FP16, 2, 1001, 3), (64, 2, 12, 2, BF16, 4, 4096, 64), (64, 2, 32, 3, FP16, 3, 33, 16), (64, 2, 1, 2, FP16, 2, 31, 1), (16, 1, 16, 3, BF16, 2, 500, 5),
+    (32, 4, 5, 2, FP16, 3, 777, 32), (64, 8, 8, 3, BF16, 2, 2050, 24), (64, 8, 3, 3, FP16, 1, 65, 7), (128, 2, 20, 3, FP16, 2, 300, 128), (128, 1, 9, 2, BF16, 1, 1, 2)])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_network_behind_levels(tnn, W, F, n_levels, dims, dtype, n_hidden, M, y_cols, ordered):
+    """tnn_grid_mlp_forward_levels against the kernel that evaluates the encoding itself, and the backward pass on the levels it leaves against the one that forms
+    them from the table: the same values, whatever the buffers held before."""
+    cfg = dict(BASE, n_dims=dims, n_levels=n_levels, n_features_per_level=F, log2_hashmap_size=12)
+    L, gd, md = tnn.lib, tnn.grid_desc(cfg), tnn.mlp_desc(dtype, W, n_hidden, "relu", "sigmoid" if M % 2 else "none")
+    g, m = ctypes.byref(gd), ctypes.byref(md)
+    rng = np.random.default_rng(M)
+    gen = torch.Generator(device=tnn.dev).manual_seed(M)
+    x = torch.rand((M, dims), device=tnn.dev, generator=gen)
+    table = torch.rand(tnn.grid_n_params(gd), device=tnn.dev, generator=gen) - 0.5
+    _, pf, pb = tnn.prepare(md, rng.uniform(-0.3, 0.3, (n_hidden + 1, W, W)).astype(np.float32))
+    order = tnn.grid_order(gd, x) if ordered else None
+    o = ptr(order) if ordered else None
+    y, expected = (torch.full((M, y_cols), float("nan"), dtype=TORCH[dtype], device=tnn.dev) for _ in range(2))
+    levels = torch.full((L.tnn_grid_levels_bytes(g, M) // 2,), float("nan"), dtype=TORCH[dtype], device=tnn.dev)
+    _lib.check(L.tnn_grid_mlp_inference_rows(g, m, ptr(x), o, ptr(table), ptr(pf), ptr(expected), y_cols, M, tnn.stream()))
+    _lib.check(L.tnn_grid_mlp_forward_levels(g, m, None, W, W, 0, None, None, ptr(pf), None, ptr(x), o, ptr(table), ptr(levels), ptr(y), y_cols, M, tnn.stream()))
+    assert torch.equal(bits(y), bits(expected))
+    assert bool(torch.isfinite(levels).all())  # nothing of it is left unwritten: the kernels read whole groups of levels, of whole tiles
+    if L.tnn_grid_mlp_train_supported(g, m) != _lib.TNN_OK:
+        return
+    dy = (torch.randn((M, y_cols), device=tnn.dev, generator=gen) * 1e-2).to(TORCH[dtype])
+    dy_full = dy if y_cols <= 16 or y_cols == W else torch.nn.functional.pad(dy, (0, W - y_cols))
+    size = L.tnn_grid_mlp_train_step_workspace_bytes(g, m, M)
+    results = []
+    for call, source in ((L.tnn_grid_mlp_backward_rows, table), (L.tnn_grid_mlp_backward_levels_rows, levels)):
+        work = torch.full((size,), 255, dtype=torch.uint8, device=tnn.dev)
+        dW, dtable = torch.full(((n_hidden + 1) * W * W,), float("nan"), device=tnn.dev), torch.full_like(table, float("nan"))
+        _lib.check(call(g, m, ptr(x), o, ptr(source), ptr(pf), ptr(pb), ptr(dy_full), dy_full.shape[1], 8.0, 0.125, ptr(dW), FP32, ptr(dtable), 1, M, ptr(work), size,
+                        tnn.stream()))
+        results.append((dW, dtable))
+    assert torch.equal(results[0][0], results[1][0])
+    scale = float(results[0][1].abs().max())  # (sums of fp32 atomics in no defined order: the bar of tnn_grid_backward)
+    assert scale > 0 and float((results[0][1] - results[1][1]).abs().max()) <= 1e-5 * scale

@@ -57,6 +57,7 @@ struct ModuleBackward : public torch::autograd::Node {
 /// A grid encoding and its network as one call: gradients of the network's parameters and of the table.
 struct EncodedNetworkBackward : public torch::autograd::Node {
     std::shared_ptr<tnn::Module> network, encoding;
+    tnn::Module::RowsPass pass; // the encoded batch
     SavedVariable positions, params, table;
     double loss_scale = 1.0;
 
@@ -66,7 +67,7 @@ struct EncodedNetworkBackward : public torch::autograd::Node {
         if (!grads[0].defined()) return {torch::Tensor(), torch::Tensor()};
         const torch::AutoGradMode no_grad(false);
         const ModulePairLock pass_lock(network->pass_mutex(), encoding->pass_mutex());
-        auto [dparams, dtable] = network->backward_rows_with_encoding(*encoding, x, grads[0], loss_scale, p, t);
+        auto [dparams, dtable] = network->backward_rows_with_encoding(*encoding, x, grads[0], pass, loss_scale, p, t);
         return {dparams, dtable};
     }
     void release_variables() override {
@@ -74,6 +75,8 @@ struct EncodedNetworkBackward : public torch::autograd::Node {
         positions.reset_data();
         params.reset_data();
         table.reset_data();
+        pass.levels.reset();
+        pass.order.reset();
     }
     std::string name() const override { return "TnnEncodedNetworkBackward"; }
 };
@@ -120,18 +123,20 @@ inline std::optional<torch::Tensor> call_with_encoding(const std::shared_ptr<tnn
     refuse_tangents({x, params, table});
     const torch::Tensor positions = x.detach().to(torch::kFloat32).contiguous();
     const bool record = torch::autograd::compute_requires_grad(params, table);
+    tnn::Module::RowsPass pass;
     torch::Tensor y;
     {
         const torch::AutoGradMode no_grad(false);
         const ModulePairLock pass_lock(network->pass_mutex(), encoding->pass_mutex());
         if (push_table) encoding->push_params(table);
-        y = network->forward_rows_with_encoding(*encoding, positions, push_network ? params : torch::Tensor(), record);
+        y = network->forward_rows_with_encoding(*encoding, positions, push_network ? params : torch::Tensor(), record, pass);
     }
     if (!record) return y;
     auto node = std::shared_ptr<EncodedNetworkBackward>(new EncodedNetworkBackward(), torch::autograd::deleteNode);
     node->set_next_edges(torch::autograd::collect_next_edges(params, table));
     node->network = network;
     node->encoding = encoding;
+    node->pass = std::move(pass);
     node->positions = SavedVariable(positions, false);
     node->params = SavedVariable(params, false);
     node->table = SavedVariable(table, false);

@@ -1,0 +1,158 @@
+// Forward pass of a network behind a grid encoding, by levels: the encoding level by level (grid_levels.hip), then a kernel of the network that reads
+// the levels. C entry points of that pass and of the backward pass on the levels it leaves.
+//
+// Reference behaviour being reproduced: dpcpp_bindings/tiny_dpcpp_nn/modules.py:357-421, as grid_mlp.inc does in one kernel; the values are
+// the same, bit for bit. The one kernel moves fewer bytes, but its gathers are as the encoding of all levels of a point has them: lines from the memory
+// side, two waves a SIMD to wait for them. (2-D, 16 levels, 2^19 entries, fp32 table, 2^18 points in cell order, two hidden layers of 64: 45.5 us; 33 and 8
+// this way. 3-D, 3000 points: 37 and 5 + 5.)
+#include "grid_levels.h"
+#include "mlp_tile.h"
+
+#include <algorithm>
+
+namespace tnn {
+int make_weight_push(const tnn_mlp_desc *desc, const void *src, int unpadded_input_width, int unpadded_output_width, int use_bias, void *packed, void *packed_t,
+                     void *fwd, void *bwd, WeightPush *p); // mlp.hip
+
+constexpr int kLevelsMlpThreads = 512;
+
+// A wave owns a tile of 32 points; it asks for the next one's levels while it computes. Weights in LDS. Bound by the bytes and, in a small batch, by
+// the latency of one tile after the weights.
+template <typename T, int W, int F>
+__global__ void __launch_bounds__(kLevelsMlpThreads, W == 128 ? 2 : 4)
+    levels_mlp_kernel(const T *__restrict__ levels, size_t pitch, uint32_t n_levels, const float4 *__restrict__ order, const typename Storage<T>::vec8 *__restrict__ wprep,
+                      T *__restrict__ out, int n_mats, int act, int out_act, long long M, int y_cols, const WeightPush push) {
+    typedef Tile<T, W> TL;
+    typedef typename Storage<T>::vec8 vec8;
+    constexpr int NK = TL::NK, NI = TL::NI;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    vec8 *lds_w = reinterpret_cast<vec8 *>(smem_raw);
+    if ((int)blockIdx.x >= push.blocks) { // (only with a push: a workgroup beside those that compute)
+        push_copies<T, W>(push, n_mats);
+        return;
+    }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane & 31, h = lane >> 5;
+    const long long n_tiles = (M + 31) / 32, stride = (long long)push.blocks * (blockDim.x >> 6);
+    long long tile = (long long)blockIdx.x * (blockDim.x >> 6) + wave;
+    vec8 nxt[NK];
+    uint32_t next_row = 0;
+    auto request = [&](const long long t) __attribute__((always_inline)) {
+        const long long i = t * 32 + j < M ? t * 32 + j : M - 1;
+        load_level_pieces<T, W, F>(nxt, levels, pitch, n_levels, (size_t)t * 32, j, h);
+        next_row = order ? __float_as_uint(order[i].w) : (uint32_t)i;
+    };
+    if (tile < n_tiles) request(tile);
+    stage_weights<T, W>(lds_w, wprep, n_mats, push);
+    if (push.master) push_copies<T, W>(push, n_mats);
+    while (tile < n_tiles) {
+        const bool valid = tile * 32 + j < M;
+        const long long row = order ? (long long)next_row : tile * 32 + j;
+        vec8 cur[NK];
+#pragma unroll
+        for (int kb = 0; kb < NK; ++kb) {
+            cur[kb] = nxt[kb];
+            asm volatile("" : "+v"(cur[kb])); // (waited for here, before the next tile's are asked for)
+        }
+        tile += stride;
+        if (tile < n_tiles) request(tile);
+        f32x16 acc[NI];
+        for (int l = 0; l < n_mats - 1; ++l) {
+            TL::template matmul<true>(acc, cur, lds_w, wprep, l, lane);
+            TL::repack_rt(cur, acc, act);
+        }
+        TL::template matmul<true>(acc, cur, lds_w, wprep, n_mats - 1, lane);
+        TL::repack_rt(cur, acc, out_act);
+        if (y_cols < W)
+            TL::store_columns(cur, out, y_cols, row, h, valid);
+        else
+            TL::store(cur, out, row, h, valid);
+    }
+}
+
+template <typename T, int W, int F>
+static int launch_levels_mlp(const tnn_mlp_desc *mlp, const void *levels, uint32_t n_levels, const float4 *order, const void *wprep, void *y, int y_cols, size_t M,
+                             WeightPush push, hipStream_t s) {
+    typedef typename Storage<T>::vec8 vec8;
+    const int n_mats = mlp->n_hidden_layers + 1;
+    const size_t lds = prepared_elems(mlp) * sizeof(T); // checked against the device by the caller
+    auto k = levels_mlp_kernel<T, W, F>;
+    if (!reserve_lds(reinterpret_cast<const void *>(k), lds)) return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", lds);
+    const int per_cu = resident_per_cu(reinterpret_cast<const void *>(k), kLevelsMlpThreads, lds);
+    const long long tiles = ((long long)M + 31) / 32, per_block = kLevelsMlpThreads / 64;
+    const long long blocks = std::min((tiles + per_block - 1) / per_block, (long long)device_info().n_cu * per_cu);
+    const int grid = push_grid(&push, (int)blocks, kLevelsMlpThreads, prepared_elems(mlp));
+    TNN_LAUNCH(k, dim3((unsigned)grid), dim3(kLevelsMlpThreads), lds, s, (const T *)levels, level_pitch(M), n_levels, order, (const vec8 *)wprep, (T *)y, n_mats,
+               mlp->activation, mlp->output_activation, (long long)M, y_cols, push);
+    return check_launch("levels_mlp_kernel");
+}
+
+template <typename T>
+static int launch_levels_mlp_w(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const void *levels, const float4 *order, const void *wprep, void *y, int y_cols,
+                               size_t M, const WeightPush &push, hipStream_t s) {
+#define TNN_LM(W, F) return launch_levels_mlp<T, W, F>(mlp, levels, grid->n_levels, order, wprep, y, y_cols, M, push, s)
+#define TNN_LM_F(W)                                 \
+    switch (grid->n_features_per_level) {           \
+    case 1: TNN_LM(W, 1);                           \
+    case 2: TNN_LM(W, 2);                           \
+    case 4: TNN_LM(W, 4);                           \
+    default: TNN_LM(W, 8);                          \
+    }
+    switch (mlp->width) {
+    case 16: TNN_LM_F(16)
+    case 32: TNN_LM_F(32)
+    case 64: TNN_LM_F(64)
+    default: TNN_LM_F(128)
+    }
+#undef TNN_LM_F
+#undef TNN_LM
+}
+
+} // namespace tnn
+
+using namespace tnn;
+
+TNN_API size_t tnn_grid_levels_bytes(const tnn_grid_desc *grid, size_t M) {
+    return check_grid_desc(grid) || M == 0 ? 0 : levels_elements(grid, M) * 2;
+}
+
+TNN_API int tnn_grid_mlp_wants_levels(const tnn_grid_desc *grid, size_t M) {
+    if (check_grid_desc(grid) || M == 0) return 0;
+    // As tnn_grid_forward_workspace_bytes has it, but that the rows are no pass of their own here.
+    size_t largest = 0;
+    for (uint32_t l = 0; l < grid->n_levels; ++l)
+        largest = std::max<size_t>(largest, (grid->offsets[l + 1] - grid->offsets[l]) * grid->n_features_per_level * (grid->param_dtype == TNN_FP32 ? 4 : 2));
+    return M < (size_t(1) << 17) || largest <= (size_t(8) << 20);
+}
+
+TNN_API int tnn_grid_mlp_forward_levels(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_src_packed, int unpadded_input_width,
+                                        int unpadded_output_width, int use_bias, void *d_packed_T, void *d_packed_transposed_T, void *d_prepared_fwd,
+                                        void *d_prepared_bwd, const float *d_x, const void *d_order, const void *d_table, void *d_levels, void *d_y, int y_cols,
+                                        size_t M, tnn_stream_t stream) {
+    GridLevels lv;
+    GridParams gp;
+    int rc = tnn_grid_mlp_supported(grid, mlp);
+    if (rc) return rc;
+    if ((rc = grid_common(grid, (uint32_t)mlp->width, M, &lv, &gp))) return rc;
+    if (y_cols < 1 || y_cols > mlp->width) return fail(TNN_ERR_INVALID_ARGUMENT, "%d output columns for a network of width %d", y_cols, mlp->width);
+    if ((!d_x && !d_order) || !d_table || !d_prepared_fwd || !d_levels || !d_y) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    if ((reinterpret_cast<uintptr_t>(d_order) & 15) || (reinterpret_cast<uintptr_t>(d_levels) & 15))
+        return fail(TNN_ERR_INVALID_ARGUMENT, "d_order and d_levels must be 16-byte aligned");
+    WeightPush push;
+    if (d_src_packed) {
+        if ((rc = make_weight_push(mlp, d_src_packed, unpadded_input_width, unpadded_output_width, use_bias, d_packed_T, d_packed_transposed_T, d_prepared_fwd,
+                                   d_prepared_bwd, &push)))
+            return rc;
+        if (reinterpret_cast<uintptr_t>(d_src_packed) & 7) { // (read in pairs)
+            if ((rc = tnn_mlp_set_packed_weights(mlp, d_src_packed, TNN_FP32, unpadded_input_width, unpadded_output_width, use_bias, d_packed_T,
+                                                 d_packed_transposed_T, d_prepared_fwd, d_prepared_bwd, stream)))
+                return rc;
+            push = WeightPush{};
+        }
+    }
+    const float4 *order = static_cast<const float4 *>(d_order);
+    hipStream_t s = as_stream(stream);
+    if ((rc = launch_grid_levels(grid, lv, gp, d_x, order, d_table, d_levels, mlp->dtype, 0, M, s))) return rc;
+    if (mlp->dtype == TNN_BF16) return launch_levels_mlp_w<bf16_t>(grid, mlp, d_levels, order, d_prepared_fwd, d_y, y_cols, M, push, s);
+    return launch_levels_mlp_w<fp16_t>(grid, mlp, d_levels, order, d_prepared_fwd, d_y, y_cols, M, push, s);
+}

@@ -118,25 +118,30 @@ TNN_API int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn
     return scatter_levels(grid, mlp, d_x, order, m, 1.0f, d_grad_table, overwrite, M, s);
 }
 
+// d_levels: the encoded batch as a forward pass left it, or null, and it is formed from d_table.
 static int grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,
-                             const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_dLdy, float *d_grad_table, int overwrite, size_t M,
+                             const void *d_levels, const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_dLdy, float *d_grad_table, int overwrite, size_t M,
                              void *d_workspace, size_t workspace_bytes, const TrainTail &tail, hipStream_t s) {
     GridLevels lv;
     GridParams gp;
     FusedPlan plan;
     int rc = train_shape_check(grid, mlp, M, &lv, &gp, &plan);
     if (rc) return rc;
-    if ((!d_x && !d_order) || !d_table || !d_prepared_fwd || !d_prepared_bwd || !d_dLdy || (!tail.dW && !tail.packed.p))
+    if ((!d_x && !d_order) || (!d_table && !d_levels) || !d_prepared_fwd || !d_prepared_bwd || !d_dLdy || (!tail.dW && !tail.packed.p))
         return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
-    if (reinterpret_cast<uintptr_t>(d_order) & 15) return fail(TNN_ERR_INVALID_ARGUMENT, "d_order must be 16-byte aligned");
+    if ((reinterpret_cast<uintptr_t>(d_order) & 15) || (reinterpret_cast<uintptr_t>(d_levels) & 15))
+        return fail(TNN_ERR_INVALID_ARGUMENT, "d_order and d_levels must be 16-byte aligned");
     GridTrainMemory m(grid, plan, M);
     if (!d_workspace || workspace_bytes < m.bytes) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, m.bytes);
     m.place(plan, d_workspace, workspace_bytes);
     const float4 *order = static_cast<const float4 *>(d_order);
-    if ((rc = launch_grid_levels(grid, lv, gp, d_x, order, d_table, m.levels, mlp->dtype, 0, M, s))) return rc;
+    if (!d_levels) {
+        if ((rc = launch_grid_levels(grid, lv, gp, d_x, order, d_table, m.levels, mlp->dtype, 0, M, s))) return rc;
+        d_levels = m.levels;
+    }
     // without a gradient table the network's gradients are all that is asked for: no dL/d(encoding) leaves the kernel
     const auto launch = mlp->dtype == TNN_BF16 ? grid_mlp_given_launch_bf16 : grid_mlp_given_launch_fp16;
-    rc = launch(mlp, plan, m.levels, grid->n_levels, order, d_prepared_fwd, d_prepared_bwd, d_dLdy, d_grad_table ? m.enc_grad : nullptr, M, m.partials, m.loss_partials,
+    rc = launch(mlp, plan, d_levels, grid->n_levels, order, d_prepared_fwd, d_prepared_bwd, d_dLdy, d_grad_table ? m.enc_grad : nullptr, M, m.partials, m.loss_partials,
                 tail, s);
     if (rc || !d_grad_table) return rc;
     return scatter_levels(grid, mlp, d_x, order, m, tail.result_scale, d_grad_table, overwrite, M, s);
@@ -152,7 +157,7 @@ TNN_API int tnn_grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc 
     TrainTail tail;
     tail.dW = d_dW;
     tail.dW_is_fp32 = dW_is_fp32;
-    return grid_mlp_backward(grid, mlp, d_x, d_order, d_table, d_prepared_fwd, d_prepared_bwd, d_dLdy, d_grad_table, overwrite, M, d_workspace,
+    return grid_mlp_backward(grid, mlp, d_x, d_order, d_table, nullptr, d_prepared_fwd, d_prepared_bwd, d_dLdy, d_grad_table, overwrite, M, d_workspace,
                              workspace_bytes, tail, as_stream(stream));
 }
 
@@ -164,6 +169,19 @@ TNN_API int tnn_grid_mlp_backward_rows(const tnn_grid_desc *grid, const tnn_mlp_
     if (rc) return rc;
     TrainTail tail;
     if ((rc = rows_tail(mlp, dy_cols, dy_scale, result_scale, d_dW_packed, dW_dtype, M, &tail))) return rc;
-    return grid_mlp_backward(grid, mlp, d_x, d_order, d_table, d_prepared_fwd, d_prepared_bwd, d_dLdy, d_grad_table, overwrite, M, d_workspace,
+    return grid_mlp_backward(grid, mlp, d_x, d_order, d_table, nullptr, d_prepared_fwd, d_prepared_bwd, d_dLdy, d_grad_table, overwrite, M, d_workspace,
+                             workspace_bytes, tail, as_stream(stream));
+}
+
+TNN_API int tnn_grid_mlp_backward_levels_rows(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_levels,
+                                              const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_dLdy, int dy_cols, float dy_scale,
+                                              float result_scale, void *d_dW_packed, int dW_dtype, float *d_grad_table, int overwrite, size_t M,
+                                              void *d_workspace, size_t workspace_bytes, tnn_stream_t stream) {
+    int rc = check_mlp_desc(mlp);
+    if (rc) return rc;
+    if (!d_levels) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
+    TrainTail tail;
+    if ((rc = rows_tail(mlp, dy_cols, dy_scale, result_scale, d_dW_packed, dW_dtype, M, &tail))) return rc;
+    return grid_mlp_backward(grid, mlp, d_x, d_order, nullptr, d_levels, d_prepared_fwd, d_prepared_bwd, d_dLdy, d_grad_table, overwrite, M, d_workspace,
                              workspace_bytes, tail, as_stream(stream));
 }

@@ -179,11 +179,12 @@ template <typename T, int WIDTH> class SwiftNetMLP : public Network<T> {
         }
         tnn::abi_check(tnn_mlp_inference_rows(&d, this->prepared_forward(), x, x_dtype, x_cols, fill, y, y_cols, M, this->get_queue().abi()));
     }
+    /// Behind a grid encoding: in one kernel, large batches in cell order.
     void inference_with_grid_rows(const tnn_grid_desc &grid, const void *table, const float *positions, const size_t M, void *y, const int y_cols,
-                                  const bool a_backward_pass_follows, const float *params = nullptr) {
+                                  const float *params = nullptr) {
         const tnn_mlp_desc d = desc();
         const void *order = nullptr;
-        if (M >= OrderedFrom(a_backward_pass_follows)) {
+        if (M >= OrderedFrom(false)) {
             OrderPoints(grid, positions, M);
             order = m_grid_order->data();
         }
@@ -194,6 +195,20 @@ template <typename T, int WIDTH> class SwiftNetMLP : public Network<T> {
             return;
         }
         tnn::abi_check(tnn_grid_mlp_inference_rows(&grid, &d, positions, order, table, this->prepared_forward(), y, y_cols, M, this->get_queue().abi()));
+    }
+    /// By levels, which are left for backward_with_levels_rows: `levels` and (unless 0) `order` are the caller's memory. The batch of a training step
+    /// is put in cell order from the size on from which its scatter is the faster for it.
+    static size_t levels_order_bytes(const tnn_grid_desc &grid, const size_t M, const bool a_backward_pass_follows) {
+        const bool ordered = a_backward_pass_follows ? M >= OrderedFrom(true) : tnn_grid_levels_want_order(&grid, M) != 0;
+        return ordered ? tnn_grid_order_bytes(&grid, M) : 0;
+    }
+    void forward_with_levels_rows(const tnn_grid_desc &grid, const void *table, const float *positions, const size_t M, void *levels, void *order,
+                                  const size_t order_bytes, void *y, const int y_cols, const float *params) {
+        const tnn_mlp_desc d = desc();
+        if (order) tnn::abi_check(tnn_grid_order_points(&grid, positions, M, order, order_bytes, this->get_queue().abi()));
+        tnn::abi_check(tnn_grid_mlp_forward_levels(&grid, &d, params, this->unpadded_in(), this->unpadded_out(), this->bias_flag(), this->packed_weights(),
+                                                   this->packed_weights_transposed(), this->prepared_forward_storage(), this->prepared_backward_storage(), positions,
+                                                   order, table, levels, y, y_cols, M, this->get_queue().abi()));
     }
     size_t backward_recompute_scratch_bytes(const size_t M) const {
         const tnn_mlp_desc d = desc();
@@ -209,18 +224,13 @@ template <typename T, int WIDTH> class SwiftNetMLP : public Network<T> {
         const tnn_mlp_desc d = desc();
         return tnn_grid_mlp_train_step_workspace_bytes(&grid, &d, M);
     }
-    void backward_with_grid_rows(const tnn_grid_desc &grid, const void *table, const float *positions, const void *dLdy, const int dy_cols,
-                                 const float dy_scale, const float result_scale, void *dW_packed, const int dW_dtype, float *grad_table, const size_t M,
-                                 void *scratch, const size_t scratch_bytes, const bool positions_as_last_ordered) {
+    void backward_with_levels_rows(const tnn_grid_desc &grid, const float *positions, const void *levels, const void *order, const void *dLdy, const int dy_cols,
+                                   const float dy_scale, const float result_scale, void *dW_packed, const int dW_dtype, float *grad_table, const size_t M,
+                                   void *scratch, const size_t scratch_bytes) {
         const tnn_mlp_desc d = desc();
-        const void *order = nullptr;
-        if (M >= OrderedFrom(true)) {
-            if (!(positions_as_last_ordered && OrderIsOf(grid, positions, M))) OrderPoints(grid, positions, M);
-            order = m_grid_order->data();
-        }
-        tnn::abi_check(tnn_grid_mlp_backward_rows(&grid, &d, positions, order, table, this->prepared_forward(), this->prepared_backward(), dLdy, dy_cols,
-                                                  dy_scale, result_scale, dW_packed, dW_dtype, grad_table, 1, M, scratch, scratch_bytes,
-                                                  this->get_queue().abi()));
+        tnn::abi_check(tnn_grid_mlp_backward_levels_rows(&grid, &d, positions, order, levels, this->prepared_forward(), this->prepared_backward(), dLdy, dy_cols,
+                                                         dy_scale, result_scale, dW_packed, dW_dtype, grad_table, 1, M, scratch, scratch_bytes,
+                                                         this->get_queue().abi()));
     }
     /// Width 128: forward pass that keeps the hidden activations only, and the backward pass on them.
     void forward_rows(const void *x, void *hidden, void *y, const int y_cols, const size_t M) {

@@ -84,6 +84,7 @@ class Module {
     struct RowsPass {
         torch::Tensor input;          // what the kernels read: the caller's tensor, or the padded and converted copy of it
         torch::Tensor hidden, output; // width 128: the hidden activations, and the output where its activation needs it
+        torch::Tensor levels, order;  // behind a grid encoding: the encoded batch, and the cell order it is in (undefined: the caller's)
         int64_t rows = 0, cols = 0;   // of the caller's input
         c10::ScalarType dtype = torch::kFloat32;
         bool in_workspace = false; // the activations are in the module's own workspace (forward_pass / backward_pass)
@@ -105,11 +106,11 @@ class Module {
     /// The parameter tensor as the Python modules hold it (a network's is packed) becomes the module's parameters.
     virtual void push_params(const torch::Tensor &) { throw std::runtime_error("push_params: not available for this module"); }
     /// Network modules behind a grid encoding: the same two passes on positions.
-    virtual torch::Tensor forward_rows_with_encoding(const Module &, const torch::Tensor &, const torch::Tensor &, bool) {
+    virtual torch::Tensor forward_rows_with_encoding(const Module &, const torch::Tensor &, const torch::Tensor &, bool, RowsPass &) {
         throw std::runtime_error("forward_rows_with_encoding: not a network module");
     }
-    virtual std::tuple<torch::Tensor, torch::Tensor> backward_rows_with_encoding(const Module &, const torch::Tensor &, const torch::Tensor &, double, const torch::Tensor &,
-                                                                                 const torch::Tensor &) {
+    virtual std::tuple<torch::Tensor, torch::Tensor> backward_rows_with_encoding(const Module &, const torch::Tensor &, const torch::Tensor &, const RowsPass &, double,
+                                                                                 const torch::Tensor &, const torch::Tensor &) {
         throw std::runtime_error("backward_rows_with_encoding: not a network module");
     }
 
@@ -639,18 +640,30 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
         set_params(p, true);
     }
 
-    torch::Tensor forward_rows_with_encoding(const Module &encoding, const torch::Tensor &positions, const torch::Tensor &push, bool keep) override {
+    torch::Tensor forward_rows_with_encoding(const Module &encoding, const torch::Tensor &positions, const torch::Tensor &push, bool keep, RowsPass &pass) override {
         this->enter();
         const tnn_grid_desc *grid = CheckedPositions(encoding, positions);
         const float *pushed = PushedWithThePass(push, true);
         const int64_t rows = positions.size(0), n_out = visible_columns();
         torch::Tensor y = fresh({rows, n_out}, kType);
-        network_.inference_with_grid_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), (size_t)rows, y.data_ptr(), (int)n_out, keep, pushed);
+        if (!keep && !tnn_grid_mlp_wants_levels(grid, (size_t)rows)) {
+            network_.inference_with_grid_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), (size_t)rows, y.data_ptr(), (int)n_out, pushed);
+            return y;
+        }
+        const size_t order_bytes = network_.levels_order_bytes(*grid, (size_t)rows, keep);
+        const torch::Tensor levels = this->scratch(tnn_grid_levels_bytes(grid, (size_t)rows)), order = order_bytes ? this->scratch(order_bytes) : torch::Tensor();
+        network_.forward_with_levels_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), (size_t)rows, levels.data_ptr(),
+                                          order_bytes ? order.data_ptr() : nullptr, order_bytes, y.data_ptr(), (int)n_out, pushed);
+        if (keep) {
+            pass.levels = levels;
+            pass.order = order;
+        }
         return y;
     }
 
     std::tuple<torch::Tensor, torch::Tensor> backward_rows_with_encoding(const Module &encoding, const torch::Tensor &positions, const torch::Tensor &dy,
-                                                                         double loss_scale, const torch::Tensor &params, const torch::Tensor &table) override {
+                                                                         const RowsPass &pass, double loss_scale, const torch::Tensor &params,
+                                                                         const torch::Tensor &table) override {
         this->enter();
         const tnn_grid_desc *grid = CheckedPositions(encoding, positions);
         CHECK_GPU(dy);
@@ -661,10 +674,10 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
         const c10::ScalarType dW_type = params.scalar_type() == kType ? kType : torch::kFloat32;
         torch::Tensor dW = fresh(params.sizes(), dW_type), dtable = fresh(table.sizes(), torch::kFloat32);
         const torch::Tensor work = this->scratch(network_.backward_with_grid_scratch_bytes(*grid, (size_t)rows));
-        // the caller's tensor is one autograd saved: it is as it was in the forward pass, and so is its cell order
-        network_.backward_with_grid_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), g.data_ptr(), (int)g.size(1), (float)loss_scale,
-                                         (float)(1.0 / loss_scale), dW.data_ptr(), this->abi_dtype(dW_type), dtable.data_ptr<float>(), (size_t)rows,
-                                         work.data_ptr(), (size_t)work.numel(), true);
+        // the caller's tensor is one autograd saved: it is as it was in the forward pass, whose levels and cell order these are
+        network_.backward_with_levels_rows(*grid, positions.data_ptr<float>(), pass.levels.data_ptr(), pass.order.defined() ? pass.order.data_ptr() : nullptr,
+                                           g.data_ptr(), (int)g.size(1), (float)loss_scale, (float)(1.0 / loss_scale), dW.data_ptr(), this->abi_dtype(dW_type),
+                                           dtable.data_ptr<float>(), (size_t)rows, work.data_ptr(), (size_t)work.numel());
         return {dW_type == params.scalar_type() ? dW : dW.to(params.scalar_type()), dtable.to(table.scalar_type())};
     }
 
