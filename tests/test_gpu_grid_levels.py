@@ -70,6 +70,22 @@ def test_encoding_module_on_both_sides_of_each_rule(tnn, dims, log2, M):
     assert torch.equal(bits(y), bits(tnn.grid_forward(d, x2, enc.params.detach().reshape(-1), 32, FP32)[:M]))
 
 
+@pytest.mark.parametrize("dims,M", [(2, 2 ** 11 - 1), (2, 2 ** 11), (2, 2 ** 19 - 1), (2, 2 ** 19), (3, 1), (3, 2 ** 17)])
+def test_field_module_on_both_sides_of_each_rule(tnn, dims, M):
+    """NetworkWithInputEncoding without autograd takes the route its size says; with autograd the one that keeps the encoded batch: the same rows."""
+    import tiny_dpcpp_nn
+    tiny_dpcpp_nn.manual_seed(3)
+    model = tiny_dpcpp_nn.NetworkWithInputEncoding(
+        dims, 3, {"otype": "FullyFusedMLP", "activation": "ReLU", "output_activation": "None", "n_neurons": 64, "n_hidden_layers": 2},
+        {"otype": "HashGrid", "type": "Hash", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": 14, "base_resolution": 16, "per_level_scale": 1.5},
+        dtype=torch.float16, use_bias=False)
+    x = torch.rand((M, dims), device=tnn.dev)
+    with torch.no_grad():
+        model.encoding.params.copy_(torch.rand(model.encoding.params.shape, device=tnn.dev) - 0.5)
+        y = model(x)
+    assert torch.equal(bits(y), bits(model(x).detach()))
+
+
 def test_a_small_batch_in_a_graph_replays(tnn):
     d = tnn.grid_desc(BASE)
     table = torch.rand(tnn.grid_n_params(d), device=tnn.dev)

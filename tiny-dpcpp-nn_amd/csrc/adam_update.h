@@ -97,6 +97,18 @@ template <typename T> __device__ __forceinline__ void store_packed_gradient(cons
         static_cast<T *>(g.p)[to] = (T)v;
 }
 
+// Memory that is to hold zeros: n4 times 16 bytes, 16-byte aligned, and n_tail floats behind them.
+struct ClearRange {
+    float4 *p = nullptr;
+    size_t n4 = 0;
+    uint32_t n_tail = 0, reduce_blocks = 0; // workgroups in front of those that clear
+};
+__device__ __forceinline__ void clear_range(const ClearRange &c, uint32_t block, uint32_t blocks) {
+    const size_t i = (size_t)block * blockDim.x + threadIdx.x, stride = (size_t)blocks * blockDim.x;
+    for (size_t k = i; k < c.n4; k += stride) c.p[k] = float4{0.f, 0.f, 0.f, 0.f};
+    if (i < c.n_tail) reinterpret_cast<float *>(c.p + c.n4)[i] = 0.0f;
+}
+
 // What follows the main kernel of the fused training step.
 struct TrainTail {
     bool use_adam = false;       // apply Adam to the reduced gradients inside the reduction kernel
@@ -109,6 +121,7 @@ struct TrainTail {
     int dy_cols = 0;
     float dy_scale = 1.0f, result_scale = 1.0f;
     PackedGradient packed{};
+    ClearRange clear{}; // cleared by further workgroups of the reduction (a launch of its own in front of the scatter took 5 us)
 };
 
 } // namespace tnn

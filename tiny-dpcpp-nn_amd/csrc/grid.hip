@@ -11,6 +11,7 @@
 // how many dimensions enter the dense index, whether the level is hashed) are evaluated once on the
 // host and reach the kernel as scalar kernel arguments; no thread evaluates exp2.
 #include "grid_binned.h"
+#include "adam_update.h"
 #include "grid_levels.h"
 
 #include <algorithm>
@@ -534,12 +535,7 @@ __global__ void __launch_bounds__(kBwdThreads)
     }
 }
 
-__global__ void fill_zero_kernel(float4 *__restrict__ p, size_t n4, float *__restrict__ tail, size_t n_tail) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t k = i; k < n4; k += stride) p[k] = float4{0.f, 0.f, 0.f, 0.f};
-    if (i < n_tail) tail[i] = 0.0f;
-}
+__global__ void __launch_bounds__(256) fill_zero_kernel(const ClearRange clear) { clear_range(clear, blockIdx.x, gridDim.x); }
 
 int check_grid_desc(const tnn_grid_desc *d) {
     if (!d) return fail(TNN_ERR_INVALID_ARGUMENT, "desc is NULL");
@@ -824,10 +820,36 @@ TNN_API int tnn_grid_forward_ordered(const tnn_grid_desc *desc, const void *d_or
 }
 
 namespace tnn {
+// The binned levels are written whole: where they are the last ones, as the finest are, only what lies in front of them is cleared.
+static ClearRange range_to_clear(const tnn_grid_desc *desc, const BinPlan &bins, void *d_grad_table, int grad_dtype) {
+    size_t entries = desc->offsets[desc->n_levels];
+    if (bins.n_levels && bins.level[0] + bins.n_levels == desc->n_levels) entries = std::min<size_t>(entries, desc->offsets[bins.level[0]]);
+    const size_t bytes = entries * desc->n_features_per_level * (grad_dtype == TNN_FP32 ? sizeof(float) : sizeof(fp16_t));
+    ClearRange c;
+    c.p = static_cast<float4 *>(d_grad_table);
+    c.n4 = bytes / 16;
+    c.n_tail = (uint32_t)((bytes - c.n4 * 16) / sizeof(float)); // level sizes are multiples of 8 entries: fp16 tables leave no tail
+    return c;
+}
+
+int grid_backward_clear(const tnn_grid_desc *desc, bool ordered, bool with_workspace, void *d_grad_table, int grad_dtype, size_t M, ClearRange *clear) {
+    GridLevels lv;
+    GridParams gp;
+    const int rc = grid_common(desc, desc->n_levels * desc->n_features_per_level, M, &lv, &gp);
+    if (rc) return rc;
+    if (reinterpret_cast<uintptr_t>(d_grad_table) & 15) return fail(TNN_ERR_INVALID_ARGUMENT, "d_grad_table must be 16-byte aligned");
+    BinPlan bins{};
+    uint32_t n_big, lds;
+    const bool fp32 = grad_dtype == TNN_FP32;
+    (void)plan_backward(lv, gp, desc->n_dims, desc->n_features_per_level, ordered, fp32, M, with_workspace && fp32 ? &bins : nullptr, &n_big, &lds);
+    *clear = range_to_clear(desc, bins, d_grad_table, grad_dtype);
+    return TNN_OK;
+}
+
 // d_x may be given beside d_order, for the routes that read the rows of a row-major dL/dy better in the caller's order.
 int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4 *d_order, const void *d_dLdy, int dy_dtype, uint32_t padded_width,
                        const GradLayout &dl, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
-                       hipStream_t s) {
+                       hipStream_t s, bool cleared) {
     GridLevels lv;
     GridParams gp;
     int rc = grid_common(desc, padded_width, M, &lv, &gp);
@@ -847,20 +869,14 @@ int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4
     if (bins.n_levels && workspace_bytes < bin_scratch_bytes(bins, desc->n_dims, n_features) + (scratch - reinterpret_cast<uintptr_t>(d_workspace)))
         return fail(TNN_ERR_WORKSPACE, "grid backward: workspace of %zu bytes given, %zu needed", workspace_bytes, bin_scratch_bytes(bins, desc->n_dims, n_features) + 256);
     if (overwrite && (reinterpret_cast<uintptr_t>(d_grad_table) & 15)) return fail(TNN_ERR_INVALID_ARGUMENT, "d_grad_table must be 16-byte aligned");
-    // The binned levels are written whole: where they are the last ones, as the finest are, only what lies in front of them is cleared.
-    size_t entries = overwrite ? desc->offsets[desc->n_levels] : 0;
-    if (bins.n_levels && bins.level[0] + bins.n_levels == desc->n_levels) entries = std::min<size_t>(entries, desc->offsets[bins.level[0]]);
-    if (entries) {
+    if (overwrite && !cleared) {
         // a fill kernel rather than a memset node, so the call can be captured into a HIP graph
-        const size_t bytes = entries * n_features * (grad_dtype == TNN_FP32 ? sizeof(float) : sizeof(fp16_t));
-        const size_t n4 = bytes / 16;
-        const size_t n_tail = (bytes - n4 * 16) / sizeof(float); // level sizes are multiples of 8 entries: fp16 tables leave no tail
-        size_t blocks = (n4 + 255) / 256;
-        if (blocks > 4096) blocks = 4096;
-        if (blocks < 4) blocks = 4;
-        TNN_LAUNCH(fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (float4 *)d_grad_table, n4,
-                   reinterpret_cast<float *>(static_cast<char *>(d_grad_table) + n4 * 16), n_tail);
-        if ((rc = check_launch("fill_zero_kernel"))) return rc;
+        const ClearRange clear = range_to_clear(desc, bins, d_grad_table, grad_dtype);
+        if (clear.n4 || clear.n_tail) {
+            const size_t blocks = std::min<size_t>(4096, std::max<size_t>(4, (clear.n4 + 255) / 256));
+            TNN_LAUNCH(fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, s, clear);
+            if ((rc = check_launch("fill_zero_kernel"))) return rc;
+        }
     }
     if (grad_dtype == TNN_FP32) {
         TNN_DISPATCH_DF(desc, rc = (launch_grid_backward_g<D_, F_, float>(lv, gp, bp, dl, n_big, lds_bytes, d_x, d_order, d_dLdy, dy_dtype,

@@ -118,7 +118,9 @@ TNN_API size_t tnn_grid_levels_bytes(const tnn_grid_desc *grid, size_t M) {
 
 TNN_API int tnn_grid_mlp_wants_levels(const tnn_grid_desc *grid, size_t M) {
     if (check_grid_desc(grid) || M == 0) return 0;
-    // As tnn_grid_forward_workspace_bytes has it, but that the rows are no pass of their own here.
+    // As tnn_grid_forward_workspace_bytes has it; and few points of two dimensions are a launch of one tile's latency in one kernel, two otherwise (module,
+    // us, one kernel / levels: 100 points 10.3 / 13.1, 9000 21.4 / 13.1; 3-D 100 points 16.8 / 13.2).
+    if (grid->n_dims == 2 && (M < (size_t(1) << 11) || M >= (size_t(1) << 19))) return 0; // (2^18 points 69 / 55, 2^20 150 / 168)
     size_t largest = 0;
     for (uint32_t l = 0; l < grid->n_levels; ++l)
         largest = std::max<size_t>(largest, (grid->offsets[l + 1] - grid->offsets[l]) * grid->n_features_per_level * (grid->param_dtype == TNN_FP32 ? 4 : 2));

@@ -1,6 +1,7 @@
 // C entry points of the training step on an encoded input: hash-grid encoding by levels (grid_levels.hip), network
 // forward, L2 loss, backward pass and Adam on the network's weights (kernels: grid_mlp_train.inc, built once per network
 // type), then the scatter of dL/d(encoding) into the table's gradient (grid.hip).
+#include "adam_update.h"
 #include "grid_levels.h"
 #include "mlp_train_shape.h"
 
@@ -68,12 +69,13 @@ struct GridTrainMemory {
     }
 };
 
+// (The reduction behind the network's kernel has cleared the table's gradient where that is overwritten.)
 // dL/d(encoding), in the network's type, by levels and in the order the kernel took the points, into the table's gradient
 static int scatter_levels(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const float4 *order, const GridTrainMemory &m, float scale,
                           float *d_grad_table, int overwrite, size_t M, hipStream_t s) {
     const GradLayout dl{grid->n_features_per_level, level_pitch(M) * grid->n_features_per_level, 1, scale};
     return grid_backward_impl(grid, order ? nullptr : d_x, order, m.enc_grad, mlp->dtype, (uint32_t)mlp->width, dl, d_grad_table, TNN_FP32, overwrite, M, m.scatter,
-                              m.scatter_bytes, s);
+                              m.scatter_bytes, s, overwrite != 0);
 }
 
 TNN_API size_t tnn_grid_mlp_train_step_workspace_bytes(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, size_t M) {
@@ -110,6 +112,7 @@ TNN_API int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn
     tail.adam = make_adam_args(d_master_packed, d_m, d_v, 1.0f / loss_scale, step, lr, beta1, beta2, eps, d_packed_T, d_prepared_fwd, d_prepared_bwd,
                                mlp->width);
     const float4 *order = static_cast<const float4 *>(d_order);
+    if (overwrite && (rc = grid_backward_clear(grid, order != nullptr, true, d_grad_table, TNN_FP32, M, &tail.clear))) return rc;
     if ((rc = launch_grid_levels(grid, lv, gp, d_x, order, d_table, m.levels, mlp->dtype, 0, M, s))) return rc;
     const auto launch = mlp->dtype == TNN_BF16 ? grid_mlp_train_launch_bf16 : grid_mlp_train_launch_fp16;
     if ((rc = launch(mlp, plan, m.levels, grid->n_levels, order, d_prepared_fwd, d_prepared_bwd, d_targets, loss_scale, d_y, d_loss_sum, m.enc_grad, M, m.partials,
@@ -121,7 +124,7 @@ TNN_API int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn
 // d_levels: the encoded batch as a forward pass left it, or null, and it is formed from d_table.
 static int grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,
                              const void *d_levels, const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_dLdy, float *d_grad_table, int overwrite, size_t M,
-                             void *d_workspace, size_t workspace_bytes, const TrainTail &tail, hipStream_t s) {
+                             void *d_workspace, size_t workspace_bytes, TrainTail tail, hipStream_t s) {
     GridLevels lv;
     GridParams gp;
     FusedPlan plan;
@@ -135,6 +138,7 @@ static int grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp,
     if (!d_workspace || workspace_bytes < m.bytes) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, m.bytes);
     m.place(plan, d_workspace, workspace_bytes);
     const float4 *order = static_cast<const float4 *>(d_order);
+    if (d_grad_table && overwrite && (rc = grid_backward_clear(grid, order != nullptr, true, d_grad_table, TNN_FP32, M, &tail.clear))) return rc;
     if (!d_levels) {
         if ((rc = launch_grid_levels(grid, lv, gp, d_x, order, d_table, m.levels, mlp->dtype, 0, M, s))) return rc;
         d_levels = m.levels;
