@@ -3,6 +3,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 from tolerances import BF16, FP16, FP32, PROPAGATED, assert_close, assert_propagated, max_norm_rel
 
@@ -627,3 +628,21 @@ def test_backward_recompute_rejects_what_it_cannot_run(tnn):
     assert tnn.lib.tnn_mlp_backward_recompute(ctypes.byref(ok), ptr(t), ptr(t), ptr(t), ptr(t), ptr(t), 1, None, 8, ptr(ws), 16, tnn.stream()) == _lib.TNN_ERR_WORKSPACE
     assert tnn.lib.tnn_mlp_backward_recompute(ctypes.byref(ok), ptr(t), ptr(t), ptr(t), None, ptr(t), 1, None, 8, ptr(ws), 16, tnn.stream()) == _lib.TNN_ERR_INVALID_ARGUMENT
     assert tnn.lib.tnn_mlp_backward_recompute(ctypes.byref(ok), ptr(t), ptr(t), ptr(t), ptr(t), ptr(t), 1, None, 12, ptr(ws), 16, tnn.stream()) == _lib.TNN_ERR_INVALID_ARGUMENT
+
+
+@pytest.mark.parametrize("act", ["relu", "sigmoid", "none"])
+@pytest.mark.parametrize("M", [8, 1064, 32768 + 8, 65832, 100000, 131072 + 32, 150000])
+def test_width_128_shares_that_are_no_whole_rounds(tnn, act, M):
+    """The kernel that passes a deep network's matrices through LDS, on batches that leave waves with one tile or none, against the same rows in a batch that is
+    whole rounds for every workgroup (131 072 rows of 256 workgroups): the same bits, activations and inference."""
+    W, n_mats, whole = 128, 9, 2 * 131072
+    desc = tnn.mlp_desc(FP16, W, n_mats - 1, act, "none")
+    rng = np.random.default_rng(3)
+    lim = np.sqrt(6.0 / (2 * W))
+    _, pf, _ = tnn.prepare(desc, rng.uniform(-lim, lim, (n_mats, W, W)).astype(np.float32))
+    x = (torch.rand((whole, W), device=tnn.dev, generator=torch.Generator(device=tnn.dev).manual_seed(M)) * 2 - 1).to(torch.float16)
+    part = x[:M].contiguous()
+    assert torch.equal(tnn.inference(desc, pf, part).view(torch.int16), tnn.inference(desc, pf, x)[:M].view(torch.int16))
+    got, expected = tnn.forward(desc, pf, part), tnn.forward(desc, pf, x)
+    for l in range(n_mats + 1):
+        assert torch.equal(got.view(n_mats + 1, M, W)[l].view(torch.int16), expected.view(n_mats + 1, whole, W)[l, :M].view(torch.int16)), l

@@ -223,23 +223,26 @@ constexpr int kStreamTiles = 2;
 
 // STAGED as in mlp_forward_kernel: 0 plain stores, 1 whole rows through a tile of LDS per wave (behind the two slots),
 // 2 the same with the streaming hint.
-template <typename T, int W, int ACT, bool STORE_INTERM, int STAGED = 0>
+// The workgroups take equal shares of the tiles, and a share's last round is as short as what is left of it: a wave without a second tile leaves its half
+// of the round's products out. (With rounds of 512 rows dealt out whole, 200 003 rows were two rounds for half of the workgroups and one for the other half:
+// 68.7 us. And 1000 rows were two workgroups: 35 us, 21 with a workgroup for every four tiles.)
+// WHOLE: all shares are whole rounds, and no condition on a tile stands between the products (131 072 rows: 1 to 4 % faster for that).
+template <typename T, int W, int ACT, bool STORE_INTERM, int STAGED = 0, bool WHOLE = false>
 __global__ void __launch_bounds__(kStreamThreads, 1)
     mlp_forward_stream_kernel(const typename Storage<T>::vec8 *__restrict__ wprep, const T *__restrict__ x, T *__restrict__ out,
                               int n_mats, int out_act, long long M, int store_input, T *__restrict__ y, int y_cols) {
     typedef Tile<T, W> TL;
     typedef typename Storage<T>::vec8 vec8;
-    constexpr int NK = TL::NK, NI = TL::NI, R = kStreamTiles;
+    constexpr int NK = TL::NK, NI = TL::NI, R = kStreamTiles, WAVES = kStreamThreads / 64;
     constexpr int per_mat = NI * NK * kWaveSize;         // 16-byte fragments per matrix
     constexpr int SHARE = per_mat / kStreamThreads;      // fragments a thread carries per matrix
     static_assert(per_mat % kStreamThreads == 0, "matrix does not split evenly over the workgroup");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     vec8 *lds = reinterpret_cast<vec8 *>(smem_raw); // slot s starts at lds + s * per_mat
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 31, h = lane >> 5;
-    constexpr int ROUND = (kStreamThreads / 64) * R * 32;
-    const long long n_rounds = (M + ROUND - 1) / ROUND;
+    const long long n_tiles = (M + 31) / 32, last_tile = (blockIdx.x + 1) * n_tiles / gridDim.x;
 
     vec8 st[SHARE];
 #pragma unroll
@@ -247,7 +250,11 @@ __global__ void __launch_bounds__(kStreamThreads, 1)
     int b = 0; // slot that holds the matrix of the layer about to run
     unsigned char *my_stage = smem_raw + 2 * per_mat * sizeof(vec8) + (size_t)wave * TL::TILE_BYTES;
 
-    for (long long r = blockIdx.x; r < n_rounds; r += gridDim.x) {
+    for (long long first = blockIdx.x * n_tiles / gridDim.x; first < last_tile; first += WAVES * R) {
+        const bool whole = WHOLE || first + WAVES * R <= last_tile;
+        // a wave's tiles: two neighbouring ones of a whole round, or one of each half
+        const long long tile0 = first + (whole ? R * wave : wave), tile1 = tile0 + (whole ? 1 : WAVES);
+        const bool two = WHOLE || tile1 < last_tile;
         long long row[R];
         bool valid[R];
         vec8 cur[R][NK];
@@ -260,15 +267,17 @@ __global__ void __launch_bounds__(kStreamThreads, 1)
                 TL::store(cur[t], dst, row[t], h, valid[t]);
             }
         };
+        // (a wave without a tile computes with zeros and stores nothing)
+        const bool any = WHOLE || tile0 < last_tile;
 #pragma unroll
         for (int t = 0; t < R; ++t) {
-            row[t] = r * ROUND + (wave * R + t) * 32 + j;
-            valid[t] = row[t] < M;
-            if constexpr (STAGED != 0) st_base[t] = TL::staged_base(r * (ROUND / 32) + wave * R + t, lane);
+            row[t] = (t == 0 ? tile0 : tile1) * 32 + j;
+            valid[t] = row[t] < M && (t == 0 ? any : two);
+            if constexpr (STAGED != 0) st_base[t] = TL::staged_base(t == 0 ? tile0 : tile1, lane);
             TL::load(cur[t], x, row[t], h, valid[t]);
-            if (STORE_INTERM && store_input) put(t, out); // (a training step reads the input where it is: it leaves matrix 0 unwritten)
+            if (STORE_INTERM && store_input && (t == 0 ? any : two)) put(t, out); // (a training step reads the input where it is: it leaves matrix 0 unwritten)
         }
-        const bool more_rounds = r + gridDim.x < n_rounds;
+        const bool more_rounds = first + WAVES * R < last_tile;
         for (int l = 0; l < n_mats; ++l) {
             __syncthreads(); // the matrix of layer l is in slot b; nobody reads the other slot any more
             const bool last = l + 1 == n_mats;
@@ -279,31 +288,40 @@ __global__ void __launch_bounds__(kStreamThreads, 1)
                 for (int i = 0; i < SHARE; ++i) st[i] = next[threadIdx.x + kStreamThreads * i];
             }
             f32x16 acc[R][NI];
-#pragma unroll
-            for (int t = 0; t < R; ++t)
-#pragma unroll
-                for (int a = 0; a < NI; ++a) acc[t][a] = f32x16{};
             const vec8 *w = lds + b * per_mat + lane;
+            auto products = [&](auto tiles) __attribute__((always_inline)) {
+                constexpr int N = decltype(tiles)::value;
 #pragma unroll
-            for (int kb = 0; kb < NK; ++kb) {
+                for (int t = 0; t < N; ++t)
 #pragma unroll
-                for (int a = 0; a < NI; ++a) {
-                    const vec8 frag = w[(a * NK + kb) * kWaveSize];
+                    for (int a = 0; a < NI; ++a) acc[t][a] = f32x16{};
 #pragma unroll
-                    for (int t = 0; t < R; ++t) acc[t][a] = Storage<T>::mfma(frag, cur[t][kb], acc[t][a]);
+                for (int kb = 0; kb < NK; ++kb) {
+#pragma unroll
+                    for (int a = 0; a < NI; ++a) {
+                        const vec8 frag = w[(a * NK + kb) * kWaveSize];
+#pragma unroll
+                        for (int t = 0; t < N; ++t) acc[t][a] = Storage<T>::mfma(frag, cur[t][kb], acc[t][a]);
+                    }
                 }
-            }
+            };
+            if (two)
+                products(std::integral_constant<int, 2>{});
+            else
+                products(std::integral_constant<int, 1>{});
             if (stage) {
 #pragma unroll
                 for (int i = 0; i < SHARE; ++i) lds[(b ^ 1) * per_mat + threadIdx.x + kStreamThreads * i] = st[i];
             }
 #pragma unroll
             for (int t = 0; t < R; ++t) {
+                if (t == 1 && !two) break;
                 if (!last) {
                     TL::template repack<ACT>(cur[t], acc[t]);
-                    if (STORE_INTERM) put(t, out + (size_t)(l + 1) * M * W);
+                    if (STORE_INTERM && any) put(t, out + (size_t)(l + 1) * M * W);
                 } else {
                     TL::repack_rt(cur[t], acc[t], out_act);
+                    if (!any) continue;
                     if (y_cols < W)
                         TL::store_columns(cur[t], y, y_cols, row[t], h, valid[t]);
                     else
@@ -539,9 +557,8 @@ static int launch_forward_v(const tnn_mlp_desc *d, const void *wprep, const void
         // 197 -> 182 us at 2^20 rows, 2 matrices: 143 -> 105 us)
         if (!in_lds || M >= 65536) { // stream the matrices through LDS, one layer at a time
             constexpr size_t lds = 2 * (size_t)Tile<T, W>::NI * Tile<T, W>::NK * kWaveSize * sizeof(vec8);
-            constexpr long long round = (kStreamThreads / 64) * kStreamTiles * 32;
-            long long g = ((long long)M + round - 1) / round;
-            if (g > di.n_cu) g = di.n_cu;
+            // a workgroup a CU, each with a tile for every SIMD at least
+            const long long n_tiles = ((long long)M + 31) / 32, g = std::min<long long>((n_tiles + 3) / 4, di.n_cu);
             const bool fits32 = (unsigned long long)M * W * sizeof(T) <= Tile<T, W>::kMaxBufferBytes;
             const bool streaming = !STORE_INTERM || (unsigned long long)(n_mats + 1) * M * W * sizeof(T) > (256ull << 20);
             const size_t lds_staged = lds + (kStreamThreads / 64) * (size_t)Tile<T, W>::TILE_BYTES;
@@ -549,6 +566,10 @@ static int launch_forward_v(const tnn_mlp_desc *d, const void *wprep, const void
             auto k1 = mlp_forward_stream_kernel<T, W, ACT, STORE_INTERM, 1>;
             auto k2 = mlp_forward_stream_kernel<T, W, ACT, STORE_INTERM, 2>;
             auto k = !fits32 ? k0 : (streaming ? k2 : k1);
+            if (fits32 && n_tiles % (g * (kStreamThreads / 64) * kStreamTiles) == 0) {
+                k = mlp_forward_stream_kernel<T, W, ACT, STORE_INTERM, 1, true>;
+                if (streaming) k = mlp_forward_stream_kernel<T, W, ACT, STORE_INTERM, 2, true>;
+            }
             const size_t lds_k = fits32 ? lds_staged : lds;
             if (!reserve_lds(reinterpret_cast<const void *>(k), lds_k)) return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", lds_k);
             TNN_LAUNCH(k, dim3((unsigned)g), dim3(kStreamThreads), lds_k, s, (const vec8 *)wprep, (const T *)x, (T *)out, n_mats,
