@@ -24,11 +24,13 @@ namespace tnn {
 constexpr int kLevelThreads = 256;
 constexpr uint32_t kXcds = 8;
 
-// Points of a thread, so that it has 16 gathers and more in flight.
-template <int D, int F> struct LevelShape {
-    static constexpr int kPoints = F > 4 ? 1 : D == 2 && F <= 2 ? 4 : 2;
+// Points of a thread. Few, so that a batch is many workgroups (us with 1, 2, 4 and 8 points a thread, 2-D: 20 000 points 5.0, 5.6, 6.3, 7.8; 2^16 10.8, 10.7,
+// 11.5, 14.1; 2^18 29.4, 29.8, 32.0, 33.7), but two in three dimensions where the batch is large (2^20 points, one and two: 265, 254).
+template <int D, int F, bool LARGE> struct LevelShape {
+    static constexpr int kPoints = F > 4 ? 1 : D == 2 ? (F <= 2 ? 2 : 1) : LARGE ? 2 : 1;
     static constexpr int kChunk = kLevelThreads * kPoints; // points of a workgroup
 };
+constexpr size_t kLargeBatch = size_t(1) << 19;
 
 // Workgroup b is the (b / 8)-th of XCD b % 8 (workgroups go to the XCDs in turn; were they not, nothing but locality would be lost);
 // XCD k takes the items [first[k], first[k + 1]) of the list of all (level, chunk of points), level by level.
@@ -73,16 +75,17 @@ __device__ __forceinline__ void row_entries(const uint32_t (&cell)[D], uint32_t 
     }
 }
 
-template <int D, int F, typename P, typename O, bool ROWS>
+template <int D, int F, typename P, typename O, bool ROWS, bool LARGE>
 __global__ void __launch_bounds__(kLevelThreads)
     grid_levels_kernel(const GridLevels lv, const GridParams gp, const LevelPlan plan, const float *__restrict__ xin, const float4 *__restrict__ order,
                        const P *__restrict__ table, O *__restrict__ out, long long M, size_t pitch) {
-    constexpr int U = LevelShape<D, F>::kPoints, R = 1 << (D - 1); // R: rows of two corners along the first dimension
+    typedef LevelShape<D, F, LARGE> S;
+    constexpr int U = S::kPoints, R = 1 << (D - 1); // R: rows of two corners along the first dimension
     typedef O ovec __attribute__((ext_vector_type(F)));
     const uint32_t xcd = blockIdx.x % kXcds, item = plan.first[xcd] + blockIdx.x / kXcds;
     if (item >= plan.first[xcd + 1]) return;
     const uint32_t l = item / plan.n_chunks;
-    const long long i0 = (long long)(item % plan.n_chunks) * LevelShape<D, F>::kChunk + threadIdx.x;
+    const long long i0 = (long long)(item % plan.n_chunks) * S::kChunk + threadIdx.x;
     const uint32_t size = lv.size[l], res = lv.resolution[l], flags = lv.flags[l];
     const float scale = lv.scale[l];
     const P *const level = table + (size_t)lv.offset[l] * F;
@@ -226,7 +229,9 @@ template <int D, int F, typename P, typename O>
 static int launch_levels(const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *table, void *out, bool rows, size_t M,
                          hipStream_t s) {
     LevelPlan plan;
-    const unsigned long long chunks = (M + LevelShape<D, F>::kChunk - 1) / LevelShape<D, F>::kChunk, items = chunks * gp.n_levels;
+    const bool large = D == 3 && M >= kLargeBatch && !rows;
+    const size_t chunk = large ? LevelShape<D, F, D == 3>::kChunk : LevelShape<D, F, false>::kChunk;
+    const unsigned long long chunks = (M + chunk - 1) / chunk, items = chunks * gp.n_levels;
     if (items > 0x0fffffffull) return fail(TNN_ERR_UNSUPPORTED, "grid encoding by levels: batch too large for one launch");
     plan.n_chunks = (uint32_t)chunks;
     double total = 0.0, cost[TNN_GRID_MAX_LEVELS], before = 0.0;
@@ -239,8 +244,9 @@ static int launch_levels(const GridLevels &lv, const GridParams &gp, const float
         plan.first[k] = k == kXcds ? (uint32_t)items : l * plan.n_chunks + (uint32_t)(part * plan.n_chunks + 0.5);
         if (k > 0) most = std::max(most, plan.first[k] - plan.first[k - 1]);
     }
-    auto k = grid_levels_kernel<D, F, P, O, false>;
-    if (rows) k = grid_levels_kernel<D, F, P, O, true>;
+    auto k = grid_levels_kernel<D, F, P, O, false, false>;
+    if (rows) k = grid_levels_kernel<D, F, P, O, true, false>;
+    if (large) k = grid_levels_kernel<D, F, P, O, false, D == 3>;
     TNN_LAUNCH(k, dim3(most * kXcds), dim3(kLevelThreads), 0, s, lv, gp, plan, x, order, (const P *)table, (O *)out, (long long)M, level_pitch(M));
     return check_launch("grid_levels_kernel");
 }
