@@ -209,13 +209,21 @@ __global__ void __launch_bounds__(256) grid_rows_kernel(const O *__restrict__ le
     }
 }
 
-// What 2^23 points cost in a level, us: the loads, and lines from L2 unless the level is a few lines or
-// (in cell order) the lanes of a wave share them; beyond the 4 MB of an XCD's L2 they come from the memory side.
+// What 2^23 points cost in a level, us: the loads, and the lines they miss in a CU's cache. `misses` in units of lines that come from L2, by the level's
+// bytes: measured (3-D, 2^20 points) 32 KB 61 us, 95 KB 106, 281 KB 137, 2.7 MB 143, 4 MB 168, 8 MB 280, 24 MB 514, 32 MB 554, a few lines 49.
+// In cell order the lanes of a wave share lines: 0.34 points a cell leave 0.13 of them (of 4 MB; 0.04 of 24 MB), 0.036 0.83 (0.49).
 static double level_cost(const GridLevels &lv, uint32_t l, uint32_t n_dims, size_t entry_bytes, bool ordered, size_t M) {
-    const double bytes = (double)lv.size[l] * (double)entry_bytes, work = n_dims == 2 ? 29.0 : 49.0, lines = n_dims == 2 ? 50.0 : 110.0;
-    double miss = std::min(1.0, std::max(0.0, std::log2(bytes / 16384.0) / 4.0)) * (1.0 + 0.75 * std::max(0.0, std::log2(bytes / (4 << 20))));
-    if (ordered) miss /= 1.0 + 5.0 * (double)M / std::pow((double)lv.resolution[l], (double)n_dims);
-    return work + lines * miss;
+    constexpr double at[][2] = {{14.0, 0.0}, {15.0, 0.13}, {16.6, 0.6}, {18.1, 0.93}, {21.4, 1.0}, {22.0, 1.26}, {23.0, 2.4}, {24.6, 4.9}, {25.0, 5.3}};
+    constexpr int n = sizeof(at) / sizeof(at[0]);
+    const double size = std::min(at[n - 1][0], std::max(at[0][0], std::log2((double)lv.size[l] * (double)entry_bytes)));
+    int i = 1;
+    while (i + 1 < n && size > at[i][0]) ++i;
+    double misses = at[i - 1][1] + (at[i][1] - at[i - 1][1]) * (size - at[i - 1][0]) / (at[i][0] - at[i - 1][0]);
+    if (ordered) {
+        const double per_cell = (double)M / std::pow((double)lv.resolution[l], (double)n_dims);
+        misses /= 1.0 + std::pow(per_cell / (0.1 * std::pow(1.26 / std::max(misses, 1.26), 0.73)), 1.5);
+    }
+    return n_dims == 2 ? 29.0 + 43.0 * misses : 49.0 + 95.0 * misses;
 }
 
 // us a batch takes by levels (3-D, 2^19 entries, 2^20 points: 332 measured, 253 in cell order).
@@ -297,15 +305,19 @@ using namespace tnn;
 static size_t dtype_bytes(int dtype) { return dtype == TNN_FP32 ? 4 : 2; }
 static size_t entry_bytes(const tnn_grid_desc *desc) { return desc->n_features_per_level * dtype_bytes(desc->param_dtype); }
 
+size_t tnn::largest_level_bytes(const tnn_grid_desc *desc) {
+    size_t entries = 0;
+    for (uint32_t l = 0; l < desc->n_levels; ++l) entries = std::max<size_t>(entries, desc->offsets[l + 1] - desc->offsets[l]);
+    return entries * entry_bytes(desc);
+}
+
 TNN_API size_t tnn_grid_forward_workspace_bytes(const tnn_grid_desc *desc, int out_dtype, size_t M) {
     if (check_grid_desc(desc) || M == 0 || grid_rows_direct(M)) return 0;
     // Points in cell order walk all levels (grid_forward_kernel) where lines come from the memory side in either case, and in 2-D from
     // 2^19 points on, where few lines are not shared and the rows are a pass of their own. us, with the ordering (points / levels and
-    // rows): 3-D, 2^18 points, 2^19, 2^20, 2^22 entries 171 / 103, 208 / 163, 220 / 237; 2-D, 2^18 points, 2^19 entries 72 / 56,
+    // rows): 3-D, 2^18 points, 2^19, 2^20, 2^22 entries 171 / 103, 208 / 163, 217 / 240; 2-D, 2^18 points, 2^19 entries 72 / 54,
     // 2^20 points 171 / 177 ordered, 193 not.
-    size_t largest = 0;
-    for (uint32_t l = 0; l < desc->n_levels; ++l) largest = std::max<size_t>(largest, (desc->offsets[l + 1] - desc->offsets[l]) * entry_bytes(desc));
-    if (M >= (size_t(1) << 17) && largest > (size_t(8) << 20)) return 0;
+    if (M >= (size_t(1) << 17) && largest_level_bytes(desc) > (desc->n_dims == 3 ? size_t(16) << 20 : size_t(8) << 20)) return 0;
     if (M >= (size_t(1) << 19) && desc->n_dims == 2) return 0;
     return levels_elements(desc, M) * dtype_bytes(out_dtype) + 256;
 }
@@ -315,7 +327,7 @@ TNN_API int tnn_grid_levels_want_order(const tnn_grid_desc *desc, size_t M) {
     GridParams gp;
     if (check_grid_desc(desc) || grid_common(desc, desc->n_levels * desc->n_features_per_level, M, &lv, &gp)) return 0;
     if (M < (size_t(1) << 18)) return 0;
-    const double ordering = 20.0 + 22.0 * (double)M / (double)(1 << 20); // us (2^18 points 25, 2^20 46, 2^21 65)
+    const double ordering = 17.0 + 25.0 * (double)M / (double)(1 << 20); // us (2^18 points 21, 2^20 46, 2^21 65)
     return levels_us(lv, gp.n_levels, desc->n_dims, entry_bytes(desc), false, M) - levels_us(lv, gp.n_levels, desc->n_dims, entry_bytes(desc), true, M) > ordering;
 }
 

@@ -121,9 +121,9 @@ TNN_API int tnn_grid_mlp_wants_levels(const tnn_grid_desc *grid, size_t M) {
     // As tnn_grid_forward_workspace_bytes has it; and few points of two dimensions are a launch of one tile's latency in one kernel, two otherwise (module,
     // us, one kernel / levels: 100 points 10.3 / 13.1, 9000 21.4 / 13.1; 3-D 100 points 16.8 / 13.2).
     if (grid->n_dims == 2 && (M < (size_t(1) << 11) || M >= (size_t(1) << 19))) return 0; // (2^18 points 69 / 55, 2^20 150 / 168)
-    size_t largest = 0;
-    for (uint32_t l = 0; l < grid->n_levels; ++l)
-        largest = std::max<size_t>(largest, (grid->offsets[l + 1] - grid->offsets[l]) * grid->n_features_per_level * (grid->param_dtype == TNN_FP32 ? 4 : 2));
+    // 2^22 entries (32 MB a level), 3-D, 2^18 points, 2^20, 2^21: 212 / 224, 704 / 704, 1288 / 1265; 2^21 entries, 2^21 points 1271 / 1145.
+    const size_t largest = largest_level_bytes(grid);
+    if (grid->n_dims == 3) return M < (size_t(1) << 17) || M >= (size_t(1) << 20) || largest <= (size_t(16) << 20);
     return M < (size_t(1) << 17) || largest <= (size_t(8) << 20);
 }
 
