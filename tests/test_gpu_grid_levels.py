@@ -146,3 +146,23 @@ def test_network_behind_levels(tnn, W, F, n_levels, dims, dtype, n_hidden, M, y_
     assert torch.equal(results[0][0], results[1][0])
     scale = float(results[0][1].abs().max())  # (sums of fp32 atomics in no defined order: the bar of tnn_grid_backward)
     assert scale > 0 and float((results[0][1] - results[1][1]).abs().max()) <= 1e-5 * scale
+
+
+@pytest.mark.parametrize("dims,log2,M,interpolation", [(3, 19, 2 ** 19 + 5, "Linear"), (3, 16, 2 ** 19 + 5, "Smoothstep"), (3, 16, 2 ** 19, "Nearest"), (3, 22, 2 ** 18, "Linear"), (2, 16, 2 ** 19, "Linear")])
+def test_backward_takes_its_own_forward_passes_order(tnn, dims, log2, M, interpolation):
+    """Two forward passes on other points, then their backward passes in either order, one of them twice: the gradients of the plain scatter."""
+    import tiny_dpcpp_nn
+    cfg = dict(BASE, n_dims=dims, log2_hashmap_size=log2, interpolation=interpolation)
+    enc = tiny_dpcpp_nn.Encoding(dims, {"otype": "HashGrid", "type": "Hash", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": log2, "base_resolution": 16,
+                                        "per_level_scale": 1.447, "interpolation": interpolation})
+    d = tnn.grid_desc(cfg)
+    gen = torch.Generator(device=tnn.dev).manual_seed(8)
+    xs = [torch.rand((M, dims), device=tnn.dev, generator=gen) for _ in range(2)]
+    dys = [torch.randn((M, 32), device=tnn.dev, generator=gen) for _ in range(2)]
+    ys = [enc(x) for x in xs]
+    for i in (0, 1, 0):
+        enc.params.grad = None
+        ys[i].backward(dys[i], retain_graph=True)
+        expected = tnn.grid_backward(d, xs[i], dys[i], FP32)
+        scale = float(expected.abs().max())
+        assert float((enc.params.grad.reshape(-1) - expected.reshape(-1)).abs().max()) <= 1e-5 * scale  # (fp32 sums in another order: the bar of tnn_grid_backward)

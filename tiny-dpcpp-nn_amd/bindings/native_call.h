@@ -49,6 +49,7 @@ struct ModuleBackward : public torch::autograd::Node {
         params.reset_data();
         pass.hidden.reset();
         pass.output.reset();
+        pass.order.reset();
         released = true;
     }
     std::string name() const override { return "TnnModuleBackward"; }

@@ -86,14 +86,26 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
         return nullptr; // enqueued on the encoding's in-order stream; the caller waits on the queue when it needs the host to see it
     }
 
-    /// forward_impl with scratch memory of the caller's (forward_scratch_bytes of it, used until the pass is over on the stream), which
-    /// large batches are the faster for: same rows, bit for bit.
+    /// forward_impl with memory of the caller's, used until the pass is over on the stream: scratch (forward_scratch_bytes, 0: none is wanted) and the
+    /// batch in cell order (forward_order_bytes, 0: the batch is not ordered), which backward_with_scratch can take over. Same rows, bit for bit.
     size_t forward_scratch_bytes(const size_t batch_size) const { return tnn_grid_forward_workspace_bytes(&m_desc, TNN_FP32, batch_size); }
-    void forward_with_scratch(const DeviceMatrixView<float> input, DeviceMatrixView<T> *output, void *scratch, const size_t scratch_bytes) {
+    size_t forward_order_bytes(const size_t batch_size) const {
+        const bool ordered = forward_scratch_bytes(batch_size) ? tnn_grid_levels_want_order(&m_desc, batch_size) != 0 : batch_size >= kCellOrderMinBatch;
+        return ordered ? tnn_grid_order_bytes(&m_desc, batch_size) : 0;
+    }
+    void forward_with_scratch(const DeviceMatrixView<float> input, DeviceMatrixView<T> *output, void *scratch, const size_t scratch_bytes, void *order,
+                              const size_t order_bytes) {
         if (!check_forward(input, output, false, false)) return;
-        const void *order = tnn_grid_levels_want_order(&m_desc, input.m()) ? ordered(input) : nullptr;
-        tnn::abi_check(tnn_grid_forward_by_level(&m_desc, input.GetPointer(), order, this->get_params()->data(), output->GetPointer(), TNN_FP32,
-                                                 this->get_padded_output_width(), input.m(), scratch, scratch_bytes, this->get_queue().abi()));
+        const uint32_t width = this->get_padded_output_width();
+        const T *table = this->get_params()->data();
+        const tnn_stream_t s = this->get_queue().abi();
+        if (order) tnn::abi_check(tnn_grid_order_points(&m_desc, input.GetPointer(), input.m(), order, order_bytes, s));
+        if (scratch)
+            tnn::abi_check(tnn_grid_forward_by_level(&m_desc, input.GetPointer(), order, table, output->GetPointer(), TNN_FP32, width, input.m(), scratch, scratch_bytes, s));
+        else if (order)
+            tnn::abi_check(tnn_grid_forward_ordered(&m_desc, order, table, output->GetPointer(), TNN_FP32, width, input.m(), s));
+        else
+            tnn::abi_check(tnn_grid_forward(&m_desc, input.GetPointer(), table, output->GetPointer(), TNN_FP32, width, input.m(), s));
     }
 
     void backward_impl(const Context &, const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput,
@@ -106,11 +118,12 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
         run_backward(input, dL_doutput, gradients, m_scratch->data(), m_scratch->size() * sizeof(float), param_gradients_mode);
     }
 
-    /// backward_impl with the caller's scratch memory (backward_scratch_bytes of it, used until the pass is over on the stream).
+    /// backward_impl with the caller's scratch memory (backward_scratch_bytes of it, used until the pass is over on the stream). `order`: the same
+    /// points in cell order, as forward_with_scratch left them, or null.
     void backward_with_scratch(const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput, DeviceMatrixView<T> *gradients, void *scratch,
-                               const size_t scratch_bytes, GradientMode param_gradients_mode = GradientMode::Overwrite) {
+                               const size_t scratch_bytes, const void *order = nullptr, GradientMode param_gradients_mode = GradientMode::Overwrite) {
         if (check_backward(input, dL_doutput, gradients, nullptr, false, param_gradients_mode))
-            run_backward(input, dL_doutput, gradients, scratch, scratch_bytes, param_gradients_mode);
+            run_backward(input, dL_doutput, gradients, scratch, scratch_bytes, param_gradients_mode, order);
     }
 
     uint32_t n_pos_dims() const override { return m_desc.n_dims; }
@@ -156,9 +169,12 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
         return true;
     }
     void run_backward(const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput, DeviceMatrixView<T> *gradients, void *scratch,
-                      const size_t scratch_bytes, GradientMode param_gradients_mode) {
-        // (The points are ordered here again: nothing says they are the forward pass's.)
-        const void *order = tnn_grid_backward_wants_order(&m_desc, input.m()) ? ordered(input) : nullptr;
+                      const size_t scratch_bytes, GradientMode param_gradients_mode, const void *order = nullptr) {
+        // An order that is there is worth its boxes in three dimensions (2^19 entries, 2^20 points, whole scatter 723 -> 633 us), not in two, whose rows of
+        // dL/dy are then read in another order than they lie in (2^20 points, forward and backward 595 -> 603); made for this pass alone it is where the
+        // bins refuse levels. Nearest is the faster for the caller's order either way.
+        if (m_desc.interpolation == TNN_INTERP_NEAREST || m_desc.n_dims == 2) order = nullptr;
+        if (!order && tnn_grid_backward_wants_order(&m_desc, input.m())) order = ordered(input);
         tnn::abi_check(tnn_grid_backward_binned(&m_desc, input.GetPointer(), order, dL_doutput.GetPointer(), TNN_FP32,
                                                 this->get_padded_output_width(), gradients->GetPointer(),
                                                 param_gradients_mode == GradientMode::Overwrite ? 1 : 0, input.m(), scratch, scratch_bytes,

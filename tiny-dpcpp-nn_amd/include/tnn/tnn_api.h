@@ -221,6 +221,11 @@ template <typename T> class EncodingModule : public Module {
     ~EncodingModule() { this->FreeWorkspace(); }
 
     torch::Tensor forward_pass(const torch::Tensor &input_tensor) override {
+        torch::Tensor order;
+        return forward_pass(input_tensor, order);
+    }
+    /// order: the batch in cell order, where the pass put it in one.
+    torch::Tensor forward_pass(const torch::Tensor &input_tensor, torch::Tensor &order) {
         this->enter();
         CHECK_INPUT(input_tensor);
         TORCH_CHECK(input_tensor.scalar_type() == torch::kFloat32, "input_tensor must be float32");
@@ -235,9 +240,12 @@ template <typename T> class EncodingModule : public Module {
         torch::Tensor output = torch::empty({(int64_t)batch_size, (int64_t)out_w}, torch::TensorOptions().dtype(torch_type<T>::dtype).device(device()));
         DeviceMatrixView<T> output_encoding(batch_size, out_w, out_w, reinterpret_cast<T *>(output.data_ptr()));
         auto *grid = dynamic_cast<tinydpcppnn::encodings::grid::GridEncodingTemplated<T> *>(encoding_.get());
-        if (const size_t need = grid ? grid->forward_scratch_bytes(batch_size) : 0) {
-            const torch::Tensor work = this->scratch(need);
-            grid->forward_with_scratch(input_dmv, &output_encoding, work.data_ptr(), (size_t)work.numel());
+        if (grid) {
+            const size_t scratch_bytes = grid->forward_scratch_bytes(batch_size), order_bytes = grid->forward_order_bytes(batch_size);
+            const torch::Tensor work = scratch_bytes ? this->scratch(scratch_bytes) : torch::Tensor();
+            if (order_bytes) order = this->scratch(order_bytes);
+            grid->forward_with_scratch(input_dmv, &output_encoding, scratch_bytes ? work.data_ptr() : nullptr, scratch_bytes, order_bytes ? order.data_ptr() : nullptr,
+                                       order_bytes);
         } else {
             encoding_->forward_impl(input_dmv, &output_encoding);
         }
@@ -253,6 +261,11 @@ template <typename T> class EncodingModule : public Module {
 
     std::tuple<torch::Tensor, torch::Tensor> backward_pass(const torch::Tensor &grad_output, const torch::Tensor &input_from_fwd,
                                                            bool pack_transpose_gradient = false, bool get_dl_dinput = false) override {
+        return backward_pass(grad_output, input_from_fwd, torch::Tensor(), pack_transpose_gradient, get_dl_dinput);
+    }
+    /// order: of input_from_fwd, as forward_pass left it, or undefined.
+    std::tuple<torch::Tensor, torch::Tensor> backward_pass(const torch::Tensor &grad_output, const torch::Tensor &input_from_fwd, const torch::Tensor &order,
+                                                           bool pack_transpose_gradient, bool get_dl_dinput) {
         this->enter();
         if (encoding_->get_n_params() == 0) return {torch::Tensor(), torch::Tensor()};
         CHECK_INPUT(grad_output);
@@ -282,7 +295,8 @@ template <typename T> class EncodingModule : public Module {
         Context ctx;
         if (auto *grid = dynamic_cast<tinydpcppnn::encodings::grid::GridEncodingTemplated<T> *>(encoding_.get())) {
             const torch::Tensor work = this->scratch(grid->backward_scratch_bytes((size_t)batch_size));
-            grid->backward_with_scratch(input_encoding_dmv, dL_doutput_dmv, &gradients_view, work.data_ptr(), (size_t)work.numel());
+            grid->backward_with_scratch(input_encoding_dmv, dL_doutput_dmv, &gradients_view, work.data_ptr(), (size_t)work.numel(),
+                                        order.defined() ? order.data_ptr() : nullptr);
         } else {
             encoding_->backward_impl(ctx, input_encoding_dmv, dL_doutput_dmv, &gradients_view);
         }
@@ -294,14 +308,19 @@ template <typename T> class EncodingModule : public Module {
     int64_t visible_columns() const override { return encoding_->get_padded_output_width(); }
     torch::Tensor forward_rows(const torch::Tensor &x, const torch::Tensor &push, bool keep, bool, RowsPass &pass) override {
         if (push.defined()) push_params(push);
-        if (keep) pass.input = x;
-        return forward_pass(x);
+        torch::Tensor order;
+        const torch::Tensor y = forward_pass(x, order);
+        if (keep) {
+            pass.input = x;
+            pass.order = order;
+        }
+        return y;
     }
     std::tuple<torch::Tensor, torch::Tensor> backward_rows(const torch::Tensor &dy, const RowsPass &pass, double loss_scale, bool,
                                                            const torch::Tensor &params) override {
         if (encoding_->get_n_params() == 0) return {torch::Tensor(), torch::Tensor()};
         if (pass.input.size(0) == 0) return {torch::Tensor(), torch::zeros_like(params)};
-        torch::Tensor g = std::get<1>(backward_pass((loss_scale != 1.0 ? dy * loss_scale : dy).contiguous(), pass.input, false, false));
+        torch::Tensor g = std::get<1>(backward_pass((loss_scale != 1.0 ? dy * loss_scale : dy).contiguous(), pass.input, pass.order, false, false));
         if (loss_scale != 1.0) g = g / loss_scale;
         return {torch::Tensor(), g.reshape(params.sizes()).to(params.scalar_type())};
     }
