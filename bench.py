@@ -69,7 +69,7 @@ def parse():
     ap.add_argument("--no-cell-order", action="store_true",
                     help="grid and grid_mlp: encode the points as they come instead of ordering the batch by cell in every step")
     ap.add_argument("--unfused", action="store_true",
-                    help="grid_train: encoding, network step and scatter as three calls with the encoded matrix in memory")
+                    help="grid_train: encoding, network step and scatter as three calls")
     ap.add_argument("--push-only-when-changed", action="store_true",
                     help="py_* workloads: switch the modules' push of `params` before every forward off (push_params_every_forward = False)")
     ap.add_argument("--no-extra-legs", action="store_true",
@@ -739,7 +739,7 @@ class Bench:
         order_bytes = lib.tnn_grid_order_bytes(g, M)
         order = torch.empty(max(order_bytes, 16), dtype=torch.uint8, device=t.dev)
 
-        # one call for encoding + network step + scatter (the encoded matrix never exists) unless --unfused
+        # one call for encoding + network step + scatter unless --unfused
         fused = not args.unfused and not args.packed_scatter
         fws_bytes = lib.tnn_grid_mlp_train_step_workspace_bytes(g, md, M) if fused else 0
         if fused and fws_bytes == 0:

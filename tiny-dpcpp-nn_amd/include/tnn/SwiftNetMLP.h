@@ -139,7 +139,7 @@ template <typename T, int WIDTH> class SwiftNetMLP : public Network<T> {
 
     /// The backward pass of this network behind a grid encoding of `positions`, for `dL_doutput`: weight gradients into `output`
     /// (raw layout) and the table's gradient (fp32, overwritten) into `grad_table` when it is not null. Encoding and forward
-    /// pass are formed again on chip; the encoded matrix is never stored (inference_with_grid is the forward pass that goes
+    /// pass are formed again (inference_with_grid is the forward pass that goes
     /// with this). Batches from 2^17 rows on are visited in cell order, as GridEncoding's own backward pass does.
     /// `positions_as_last_ordered`: the caller vouches that the contents of `positions` have not changed since the last call
     /// that put them in cell order (inference_with_grid or this); if that call was for this pointer, batch size and grid, its

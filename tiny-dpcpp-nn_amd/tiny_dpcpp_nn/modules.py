@@ -243,7 +243,7 @@ class NetworkWithInputEncoding(Module):
         self.network = Network(self.width, n_output_dims, network_config, store_params_as_full_precision=store_params_as_full_precision,
                                device=device, dtype=dtype, use_bias=use_bias)
         self.network_with_encoding = torch.nn.Sequential(self.encoding, self.network)
-        self._fused = None  # whether the pair runs as one kernel: (without autograd, with it)
+        self._fused = None  # whether the pair runs as one call: (without autograd, with it)
 
     @property
     def params(self):
@@ -261,8 +261,8 @@ class NetworkWithInputEncoding(Module):
             self._fused = (network.tnn_module.can_fuse_encoding(encoding.tnn_module), network.tnn_module.can_train_with_encoding(encoding.tnn_module))
         if not self._fused[torch.is_grad_enabled()]:
             return self.network_with_encoding(x)
-        # a grid encoding and its network as one kernel (backward: one kernel plus the scatter), with the values of the two
-        # modules in turn, the reference's only route; the encoded matrix is never stored
+        # a grid encoding and its network as one call into the native module each way, with the values of the two
+        # modules in turn, the reference's only route
         y = network.tnn_module.call_with_encoding(encoding.tnn_module, x, network.params, encoding.params, network._must_push(), encoding._must_push(),
                                                   network.loss_scale)
         if y is None:
