@@ -12,7 +12,7 @@
 // corners of a row, of one's point and then of the other's, and exchange what they loaded.
 // Measured, fp32 table and rows: 3-D, 16 levels, 2^19 entries, 2^20 points 253 us in cell order and 332 in the caller's (one load a lane: 547 and
 // 534; all levels of a point in one thread: 519 and 754), of which the levels beyond L2's reach of a thread a point 455 -> 170 for eight of them;
-// 2-D, 2^18 points 32 and 43 (42 and 76). 5001 points 3-D: 6 us (38).
+// 2-D, 2^18 points 25.6 and 39 (42 and 76). 5001 points 3-D: 6 us (38).
 // A batch that is small then has a wave for every level, too, and not one wave that walks through all of them.
 #include "grid_levels.h"
 
@@ -25,7 +25,7 @@ constexpr int kLevelThreads = 256;
 constexpr uint32_t kXcds = 8;
 
 // Points of a thread. Few, so that a batch is many workgroups (us with 1, 2, 4 and 8 points a thread, 2-D: 20 000 points 5.0, 5.6, 6.3, 7.8; 2^16 10.8, 10.7,
-// 11.5, 14.1; 2^18 29.4, 29.8, 32.0, 33.7), but two in three dimensions where the batch is large (2^20 points, one and two: 265, 254).
+// 11.5, 14.1; 2^18 29.4, 29.8, 32.0, 33.7, before two corners were one load), but two in three dimensions where the batch is large (2^20 points, one and two: 265, 254).
 template <int D, int F, bool LARGE> struct LevelShape {
     static constexpr int kPoints = F > 4 ? 1 : D == 2 ? (F <= 2 ? 2 : 1) : LARGE ? 2 : 1;
     static constexpr int kChunk = kLevelThreads * kPoints; // points of a workgroup
@@ -75,6 +75,32 @@ __device__ __forceinline__ void row_entries(const uint32_t (&cell)[D], uint32_t 
     }
 }
 
+// Whether the two corners of a row are neighbouring entries that one load takes: a level that is not hashed. In two dimensions, where most levels are not
+// (2^18 points in cell order 27.8 -> 25.6 us; three dimensions, 2^20 points 242 -> 240, and 2^22 entries, 2^21 points 1116 -> 1125).
+__host__ __device__ constexpr bool side_by_side(uint32_t n_dims, uint32_t flags, size_t entry_bytes) {
+    return n_dims == 2 && entry_bytes >= 4 && entry_bytes <= 8 && (flags & 31u) == n_dims;
+}
+// Two neighbouring entries in one load (of an entry's alignment, which is at least 4 bytes).
+template <typename P, int F> __device__ __forceinline__ void load_pair(const P *__restrict__ p, float (&near)[F], float (&far)[F]) {
+    typedef P pair_t __attribute__((ext_vector_type(2 * F), aligned(F * sizeof(P))));
+    const pair_t t = *reinterpret_cast<const pair_t *>(p);
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        near[f] = (float)t[f];
+        far[f] = (float)t[F + f];
+    }
+}
+
+// From what a lane loaded for the even and the odd lane's point to the near and the far corner of its own.
+template <int F> __device__ __forceinline__ void exchange_corners(uint32_t side, float (&even)[F], float (&odd)[F]) {
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        const float mine = side ? odd[f] : even[f], other = swap_pair(side ? even[f] : odd[f]);
+        even[f] = side ? other : mine;
+        odd[f] = side ? mine : other;
+    }
+}
+
 template <int D, int F, typename P, typename O, bool ROWS, bool LARGE>
 __global__ void __launch_bounds__(kLevelThreads)
     grid_levels_kernel(const GridLevels lv, const GridParams gp, const LevelPlan plan, const float *__restrict__ xin, const float4 *__restrict__ order,
@@ -109,32 +135,69 @@ __global__ void __launch_bounds__(kLevelThreads)
             for (int d = 0; d < D; ++d) x[u][d] = xin[i * D + d];
         }
     }
-    float even[U][R][F], odd[U][R][F], frac[U][D]; // what this lane loads for the even and the odd lane's point
+    // of a row of corners: what this lane loads for the even and the odd lane's point, and then the near and the far corner of its own
+    float even[U][R][F], odd[U][R][F], frac[U][D];
+    // A level that is not hashed has the two corners side by side: one load for both, unless the index of any of the wave's wraps.
+    bool together = side_by_side(D, flags, F * sizeof(P)) && !nearest;
+    if (together) {
+        uint32_t near[U][R];
+        bool wraps = false;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-        uint32_t cell[D], of_even[D], of_odd[D], a[R], b[R];
-        cell_of<D>(x[u], scale, gp.interpolation, cell, frac[u]);
-        if (nearest) {
-            load_entry<P, F>(level + (size_t)level_index<D>(cell, size, res, flags, gp.hash_type) * F, even[u][0]);
-            continue;
+        for (int u = 0; u < U; ++u) {
+            uint32_t cell[D];
+            cell_of<D>(x[u], scale, gp.interpolation, cell, frac[u]);
+            const uint32_t first = cell[0] + res * cell[1];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                near[u][r] = first + ((r & 1) ? res : 0u); // (two dimensions)
+                wraps |= near[u][r] >= size - 1; // (a level has 8 entries and more)
+            }
         }
+        together = !__any(wraps);
+        if (together) {
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            const uint32_t other = swap_pair(cell[d]);
-            of_even[d] = side ? other : cell[d];
-            of_odd[d] = side ? cell[d] : other;
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int r = 0; r < R; ++r) load_pair<P, F>(level + (size_t)near[u][r] * F, even[u][r], odd[u][r]);
         }
-        row_entries<D>(of_even, side, size, res, flags, gp.hash_type, a);
-        row_entries<D>(of_odd, side, size, res, flags, gp.hash_type, b);
+    }
+    if (!together) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            load_entry<P, F>(level + (size_t)a[r] * F, even[u][r]);
-            load_entry<P, F>(level + (size_t)b[r] * F, odd[u][r]);
+        for (int u = 0; u < U; ++u) {
+            uint32_t cell[D], of_even[D], of_odd[D], a[R], b[R];
+            cell_of<D>(x[u], scale, gp.interpolation, cell, frac[u]);
+            if (nearest) {
+                load_entry<P, F>(level + (size_t)level_index<D>(cell, size, res, flags, gp.hash_type) * F, even[u][0]);
+                continue;
+            }
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                const uint32_t other = swap_pair(cell[d]);
+                of_even[d] = side ? other : cell[d];
+                of_odd[d] = side ? cell[d] : other;
+            }
+            row_entries<D>(of_even, side, size, res, flags, gp.hash_type, a);
+            row_entries<D>(of_odd, side, size, res, flags, gp.hash_type, b);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                load_entry<P, F>(level + (size_t)a[r] * F, even[u][r]);
+                load_entry<P, F>(level + (size_t)b[r] * F, odd[u][r]);
+            }
+        }
+        if (D == 2 && !nearest) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int r = 0; r < R; ++r) exchange_corners<F>(side, even[u][r], odd[u][r]);
         }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const long long i = i0 + u * kLevelThreads;
+        if (D == 3 && !nearest) { // (where they are first used)
+#pragma unroll
+            for (int r = 0; r < R; ++r) exchange_corners<F>(side, even[u][r], odd[u][r]);
+        }
         ovec o;
 #pragma unroll
         for (int f = 0; f < F; ++f) {
@@ -144,8 +207,6 @@ __global__ void __launch_bounds__(kLevelThreads)
             } else {
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
-                    const float mine = side ? odd[u][r][f] : even[u][r][f], other = swap_pair(side ? even[u][r][f] : odd[u][r][f]);
-                    const float near = side ? other : mine, far = side ? mine : other;
                     // the products and the order of encode_levels
                     float near_weight = 1 - frac[u][0], far_weight = frac[u][0];
 #pragma unroll
@@ -154,8 +215,8 @@ __global__ void __launch_bounds__(kLevelThreads)
                         near_weight *= w;
                         far_weight *= w;
                     }
-                    v = __builtin_fmaf(near_weight, near, v);
-                    v = __builtin_fmaf(far_weight, far, v);
+                    v = __builtin_fmaf(near_weight, even[u][r][f], v);
+                    v = __builtin_fmaf(far_weight, odd[u][r][f], v);
                 }
             }
             o[f] = to_out<O>(as_fp32(v)); // (pinned as encode_levels pins it)
@@ -223,7 +284,9 @@ static double level_cost(const GridLevels &lv, uint32_t l, uint32_t n_dims, size
         const double per_cell = (double)M / std::pow((double)lv.resolution[l], (double)n_dims);
         misses /= 1.0 + std::pow(per_cell / (0.1 * std::pow(1.26 / std::max(misses, 1.26), 0.73)), 1.5);
     }
-    return n_dims == 2 ? 29.0 + 43.0 * misses : 49.0 + 95.0 * misses;
+    // (one load for two corners is worth most where lanes share lines: of a batch in the caller's order the lines are what a level costs)
+    const bool pairs = ordered && side_by_side(n_dims, lv.flags[l], entry_bytes);
+    return n_dims == 2 ? (pairs ? 18.0 : 29.0) + 43.0 * misses : 49.0 + 95.0 * misses;
 }
 
 // us a batch takes by levels (3-D, 2^19 entries, 2^20 points: 332 measured, 253 in cell order).

@@ -3,8 +3,8 @@
 //
 // Reference behaviour being reproduced: dpcpp_bindings/tiny_dpcpp_nn/modules.py:357-421, as grid_mlp.inc does in one kernel; the values are
 // the same, bit for bit. The one kernel moves fewer bytes, but its gathers are as the encoding of all levels of a point has them: lines from the memory
-// side, two waves a SIMD to wait for them. (2-D, 16 levels, 2^19 entries, fp32 table, 2^18 points in cell order, two hidden layers of 64: 45.5 us; 33 and 8
-// this way. 3-D, 3000 points: 37 and 5 + 5.)
+// side, two waves a SIMD to wait for them. (2-D, 16 levels, 2^19 entries, fp32 table, 2^18 points in cell order, two hidden layers of 64: 45.5 us; 27 and 15
+// this way. 3-D, 3000 points: 37 and 6 + 6.)
 #include "grid_levels.h"
 #include "mlp_tile.h"
 
