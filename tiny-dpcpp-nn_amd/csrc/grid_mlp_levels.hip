@@ -118,9 +118,18 @@ TNN_API size_t tnn_grid_levels_bytes(const tnn_grid_desc *grid, size_t M) {
 
 TNN_API int tnn_grid_mlp_wants_levels(const tnn_grid_desc *grid, size_t M) {
     if (check_grid_desc(grid) || M == 0) return 0;
-    // As tnn_grid_forward_workspace_bytes has it; and few points of two dimensions are a launch of one tile's latency in one kernel, two otherwise (module,
-    // us, one kernel / levels: 100 points 10.3 / 13.1, 9000 21.4 / 13.1; 3-D 100 points 16.8 / 13.2).
-    if (grid->n_dims == 2 && (M < (size_t(1) << 11) || M >= (size_t(1) << 19))) return 0; // (2^18 points 69 / 55, 2^20 150 / 168)
+    // By levels is two launches, 13 us through the module however few the points are; one kernel takes a tile's gathers in a row: 10 us with 8 levels, more with
+    // each level and corner. Points of a picture's rows share their lines of the table in one kernel nearly as well as by levels, scattered ones do not, and which
+    // they are is not known here: by levels where neither is slower (module, us, one kernel / levels, rows of a picture and scattered points).
+    // 2-D, 16 levels: 100 points 10.3 / 13.1; 6000 14.6 / 13.0 and 21.6 / 13.1; 30000 15.0 / 14.7 and 22.8 / 15.0; 108895 20.2 / 24.0 and 43.2 / 27.0;
+    // 2^18 53 / 38 and 71 / 48 (ordered from there in one kernel); 2^20 scattered 150 / 168. 12 levels: 16000 11.4 / 13.0. 8 levels: 30000 9.6 / 12.1,
+    // 140000 14.4 / 15.7, 2^18 40 / 21.
+    if (grid->n_dims == 2) {
+        if (M >= (size_t(1) << 19) || M < (size_t(1) << 11)) return 0;
+        if (M < (size_t(1) << 18) && (grid->n_levels <= 12 || M >= (size_t(1) << 15))) return 0;
+    }
+    // 3-D, 16 levels: 100 scattered points 16.8 / 13.2, 6000 of a picture 18.0 / 13.2; 8 levels: 30000 12.1 / 12.9 (scattered, 17000: 21.6 / 12.9), 108895 20.6 / 18.9.
+    if (grid->n_dims == 3 && grid->n_levels <= 8 && M < (size_t(1) << 16)) return 0;
     // 2^22 entries (32 MB a level), 3-D, 2^18 points, 2^20, 2^21: 212 / 224, 704 / 704, 1288 / 1265; 2^21 entries, 2^21 points 1271 / 1145.
     const size_t largest = largest_level_bytes(grid);
     if (grid->n_dims == 3) return M < (size_t(1) << 17) || M >= (size_t(1) << 20) || largest <= (size_t(16) << 20);
