@@ -182,7 +182,9 @@ __global__ void __launch_bounds__(kOrderThreads)
 
 // Step 2: one workgroup per bin sorts the bin's records by the next bits of the coordinates, in LDS, in pieces of at most
 // 8 THREADS records (a bin that holds more, because the points cluster, is refined piece by piece). THREADS: about as many as the bins hold records, so
-// that the LDS of the workgroups of a small batch leaves many of them a CU (2^18 points: 8.2 us with 256 threads and 32 KB).
+// that the LDS of the workgroups of a small batch leaves many of them a CU (2^18 points: 8.2 us with 256 threads and 32 KB). 64 threads up to 2^18 points,
+// 2^17 in 3-D: a picture's rows fill one bin in sixteen there (encoding and network, us, 256 threads / 64: 2^19 such points 164 / 171, 2^18 104 / 108; scattered 445 / 441,
+// 248 / 243).
 template <int D, int THREADS>
 __global__ void __launch_bounds__(THREADS)
     order_refine_kernel(const uint32_t *__restrict__ starts, float4 *__restrict__ records, long long M) {
@@ -269,7 +271,7 @@ TNN_API int tnn_grid_order_points(const tnn_grid_desc *desc, const float *d_x, s
         if ((rc = check_launch("order_scan_kernel"))) return rc;                                                                       \
         TNN_LAUNCH((order_scatter_kernel<D_>), dim3(p.n_wg), dim3(kOrderThreads), 0, s, d_x, (long long)M, p.chunk, (const uint32_t *)hist, records); \
         if ((rc = check_launch("order_scatter_kernel"))) return rc;                                                                    \
-        if (M <= (size_t)kOrderBins * 128)                                                                                             \
+        if (M <= (size_t)kOrderBins * (D_ == 2 ? 64 : 32))                                                                             \
             TNN_LAUNCH((order_refine_kernel<D_, 64>), dim3(kOrderBins), dim3(64), 0, s, (const uint32_t *)hist, records, (long long)M);      \
         else                                                                                                                           \
             TNN_LAUNCH((order_refine_kernel<D_, 256>), dim3(kOrderBins), dim3(256), 0, s, (const uint32_t *)hist, records, (long long)M);    \
