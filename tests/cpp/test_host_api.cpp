@@ -8,6 +8,7 @@
 #include <thread>
 
 #include "../../tiny-dpcpp-nn_amd/csrc/lds_reservation.h"
+#include "../../tiny-dpcpp-nn_amd/csrc/level_plan.h"
 #include "tnn/SwiftNetMLP.h"
 #include "tnn/encoding_factory.h"
 #include "tnn/io.h"
@@ -694,6 +695,31 @@ static void test_lds_reservations() {
     CHECK(ask(&a, 0, 90000, set) == 90000 && set == 90000);
 }
 
+// Every item of a launch of the encoding by levels belongs to one XCD, and no plan has 2^32 threads, however unequal the levels' costs are.
+static void test_level_plans() {
+    constexpr uint32_t threads = 256;
+    for (uint32_t n_levels : {1u, 2u, 5u, 16u, 31u, 32u, 127u, 128u}) {
+        const size_t part = tnn::level_part_chunks(n_levels, threads);
+        CHECK(part >= 4096 && part * n_levels * tnn::kXcds * threads < (1ull << 32));
+        for (int costs = 0; costs < 4; ++costs) {
+            std::vector<double> cost(n_levels);
+            for (uint32_t l = 0; l < n_levels; ++l) cost[l] = costs == 0 ? 1.0 : costs == 1 ? (l + 1 == n_levels ? 1000.0 : 1.0) : costs == 2 ? (l == 0 ? 30.0 : 1.0) : 1.0 + l * l;
+            for (size_t n_chunks : {size_t(1), size_t(3), size_t(1000), part - 1, part}) {
+                tnn::LevelPlan plan;
+                plan.n_chunks = (uint32_t)n_chunks;
+                const uint32_t most = tnn::plan_levels(cost.data(), n_levels, &plan);
+                bool in_order = plan.first[0] == 0 && plan.first[tnn::kXcds] == n_levels * n_chunks;
+                uint32_t widest = 0;
+                for (uint32_t k = 0; k < tnn::kXcds; ++k) {
+                    in_order = in_order && plan.first[k] <= plan.first[k + 1];
+                    widest = std::max(widest, plan.first[k + 1] - plan.first[k]);
+                }
+                CHECK(in_order && most == widest && (unsigned long long)most * tnn::kXcds * threads < (1ull << 32));
+            }
+        }
+    }
+}
+
 int main(int argc, char **argv) {
     const bool cpu_only = argc > 1 && std::string(argv[1]) == "--cpu";
     std::printf("storage types\n");
@@ -706,6 +732,8 @@ int main(int argc, char **argv) {
     test_io_files();
     std::printf("LDS reservations\n");
     test_lds_reservations();
+    std::printf("level plans\n");
+    test_level_plans();
     if (!cpu_only) {
         tnn::abi_check(tnn_device_check());
         std::printf("swiftnet\n");

@@ -53,6 +53,19 @@ def test_levels_are_the_rows_of_the_points(tnn, cfg, param_dtype, out_dtype, wid
         assert torch.equal(bits(tnn.grid_forward_ordered(d, tnn.grid_order(d, part), table, width, m, out_dtype)), bits(expected[:m]))
 
 
+@pytest.mark.parametrize("ordered", [False, True])
+def test_a_batch_of_several_launches(tnn, ordered):
+    """32 levels: a launch takes 65535 chunks of 512 points; a batch with more, its last chunk and last 64 points not full."""
+    cfg = dict(BASE, n_levels=32, n_features_per_level=1, log2_hashmap_size=12, per_level_scale=1.2)
+    d = tnn.grid_desc(cfg)
+    gen = torch.Generator(device=tnn.dev).manual_seed(9)
+    table = torch.rand(tnn.grid_n_params(d), device=tnn.dev, generator=gen)
+    M = 65535 * 512 + 5 * 512 + 77
+    x = torch.rand((M, 3), device=tnn.dev, generator=gen)
+    got = by_level(tnn, d, x, tnn.grid_order(d, x) if ordered else None, table, 32, BF16)
+    assert torch.equal(bits(got), bits(tnn.grid_forward(d, x, table, 32, BF16)))
+
+
 @pytest.mark.parametrize("dims,log2,M", [(3, 16, DIRECT), (3, 16, DIRECT + 1), (3, 19, 2 ** 19 + 3), (2, 16, 2 ** 19 - 1), (2, 16, 2 ** 19), (3, 22, 2 ** 17), (3, 14, 2 ** 19 - 1)])
 def test_encoding_module_on_both_sides_of_each_rule(tnn, dims, log2, M):
     """The Python encoding takes whichever route its size says; the C ABI in two calls of half the points, or by points, gives the same rows."""

@@ -15,6 +15,7 @@
 // 2-D, 2^18 points 25.6 and 39 (42 and 76). 5001 points 3-D: 6 us (38).
 // A batch that is small then has a wave for every level, too, and not one wave that walks through all of them.
 #include "grid_levels.h"
+#include "level_plan.h"
 
 #include <algorithm>
 #include <cmath>
@@ -22,7 +23,6 @@
 namespace tnn {
 
 constexpr int kLevelThreads = 256;
-constexpr uint32_t kXcds = 8;
 
 // Points of a thread. Few, so that a batch is many workgroups (us with 1, 2, 4 and 8 points a thread, 2-D: 20 000 points 5.0, 5.6, 6.3, 7.8; 2^16 10.8, 10.7,
 // 11.5, 14.1; 2^18 29.4, 29.8, 32.0, 33.7, before two corners were one load), but two in three dimensions where the batch is large (2^20 points, one and two: 265, 254).
@@ -31,13 +31,6 @@ template <int D, int F, bool LARGE> struct LevelShape {
     static constexpr int kChunk = kLevelThreads * kPoints; // points of a workgroup
 };
 constexpr size_t kLargeBatch = size_t(1) << 19;
-
-// Workgroup b is the (b / 8)-th of XCD b % 8 (workgroups go to the XCDs in turn; were they not, nothing but locality would be lost);
-// XCD k takes the items [first[k], first[k + 1]) of the list of all (level, chunk of points), level by level.
-struct LevelPlan {
-    uint32_t first[kXcds + 1];
-    uint32_t n_chunks;
-};
 
 // The neighbouring lane's value: lanes 2 k and 2 k + 1 exchange (DPP quad_perm).
 __device__ __forceinline__ uint32_t swap_pair(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xf, 0xf, false); }
@@ -221,7 +214,7 @@ __global__ void __launch_bounds__(kLevelThreads)
             }
             o[f] = to_out<O>(as_fp32(v)); // (pinned as encode_levels pins it)
         }
-        if (i >= (ROWS ? M : (long long)pitch)) continue;
+        if (i >= (ROWS ? M : (long long)level_pitch(M))) continue;
         if constexpr (ROWS) {
             O *const to = out + (order ? (size_t)row[u] : (size_t)i) * gp.padded_width;
 #pragma unroll
@@ -296,30 +289,35 @@ static double levels_us(const GridLevels &lv, uint32_t n_levels, uint32_t n_dims
     return cost * (double)M / (double)(1 << 23);
 }
 
+// One launch: the points [begin, begin + M) of a batch.
 template <int D, int F, typename P, typename O>
-static int launch_levels(const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *table, void *out, bool rows, size_t M,
-                         hipStream_t s) {
+static int launch_levels_part(const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *table, O *out, bool rows, bool large,
+                              size_t begin, size_t M, size_t batch, hipStream_t s) {
     LevelPlan plan;
-    const bool large = D == 3 && M >= kLargeBatch && !rows;
     const size_t chunk = large ? LevelShape<D, F, D == 3>::kChunk : LevelShape<D, F, false>::kChunk;
-    const unsigned long long chunks = (M + chunk - 1) / chunk, items = chunks * gp.n_levels;
-    if (items > 0x0fffffffull) return fail(TNN_ERR_UNSUPPORTED, "grid encoding by levels: batch too large for one launch");
-    plan.n_chunks = (uint32_t)chunks;
-    double total = 0.0, cost[TNN_GRID_MAX_LEVELS], before = 0.0;
-    for (uint32_t l = 0; l < gp.n_levels; ++l) total += cost[l] = level_cost(lv, l, D, F * sizeof(P), order != nullptr, M);
-    uint32_t most = 0;
-    for (uint32_t k = 0, l = 0; k <= kXcds; ++k) {
-        const double until = total * k / kXcds;
-        while (l + 1 < gp.n_levels && before + cost[l] < until) before += cost[l++];
-        const double part = std::min(1.0, std::max(0.0, (until - before) / cost[l]));
-        plan.first[k] = k == kXcds ? (uint32_t)items : l * plan.n_chunks + (uint32_t)(part * plan.n_chunks + 0.5);
-        if (k > 0) most = std::max(most, plan.first[k] - plan.first[k - 1]);
-    }
+    plan.n_chunks = (uint32_t)((M + chunk - 1) / chunk);
+    double cost[TNN_GRID_MAX_LEVELS];
+    for (uint32_t l = 0; l < gp.n_levels; ++l) cost[l] = level_cost(lv, l, D, F * sizeof(P), order != nullptr, batch);
+    const uint32_t most = plan_levels(cost, gp.n_levels, &plan);
     auto k = grid_levels_kernel<D, F, P, O, false, false>;
     if (rows) k = grid_levels_kernel<D, F, P, O, true, false>;
     if (large) k = grid_levels_kernel<D, F, P, O, false, D == 3>;
-    TNN_LAUNCH(k, dim3(most * kXcds), dim3(kLevelThreads), 0, s, lv, gp, plan, x, order, (const P *)table, (O *)out, (long long)M, level_pitch(M));
+    TNN_LAUNCH(k, dim3(most * kXcds), dim3(kLevelThreads), 0, s, lv, gp, plan, x ? x + begin * D : nullptr, order ? order + begin : nullptr, (const P *)table,
+               out + (rows ? 0 : begin * F), (long long)M, level_pitch(batch));
     return check_launch("grid_levels_kernel");
+}
+
+template <int D, int F, typename P, typename O>
+static int launch_levels(const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *table, void *out, bool rows, size_t M,
+                         hipStream_t s) {
+    const bool large = D == 3 && M >= kLargeBatch && !rows;
+    const size_t chunk = large ? LevelShape<D, F, D == 3>::kChunk : LevelShape<D, F, false>::kChunk;
+    const size_t part = level_part_chunks(gp.n_levels, kLevelThreads) * chunk;
+    if (rows && M > part) return fail(TNN_ERR_UNSUPPORTED, "grid encoding by levels: rows of small batches only");
+    for (size_t begin = 0; begin < M; begin += part)
+        if (const int rc = launch_levels_part<D, F, P, O>(lv, gp, x, order, table, (O *)out, rows, large, begin, std::min(part, M - begin), M, s))
+            return rc;
+    return TNN_OK;
 }
 
 int launch_grid_levels(const tnn_grid_desc *desc, const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *table, void *out,

@@ -1,0 +1,41 @@
+// Which XCD takes which levels of which points (grid_levels.hip), and how many points one launch may have.
+#pragma once
+
+#include <algorithm>
+#include <cstddef>
+#include <cstdint>
+
+namespace tnn {
+
+constexpr uint32_t kXcds = 8;
+
+// Workgroup b is the (b / 8)-th of XCD b % 8 (workgroups go to the XCDs in turn; were they not, nothing but locality would be lost);
+// XCD k takes the items [first[k], first[k + 1]) of the list of all (level, chunk of points), level by level.
+struct LevelPlan {
+    uint32_t first[kXcds + 1];
+    uint32_t n_chunks;
+};
+
+// Shares of equal cost (of a level: cost[l]). Returns the most items an XCD has: the launch is 8 times as many workgroups.
+inline uint32_t plan_levels(const double *cost, uint32_t n_levels, LevelPlan *plan) {
+    double total = 0.0, before = 0.0;
+    for (uint32_t l = 0; l < n_levels; ++l) total += cost[l];
+    uint32_t most = 0;
+    for (uint32_t k = 0, l = 0; k <= kXcds; ++k) {
+        const double until = total * k / kXcds;
+        while (l + 1 < n_levels && before + cost[l] < until) before += cost[l++];
+        const double part = std::min(1.0, std::max(0.0, (until - before) / cost[l]));
+        plan->first[k] = k == kXcds ? n_levels * plan->n_chunks : l * plan->n_chunks + (uint32_t)(part * plan->n_chunks + 0.5);
+        if (k > 0) most = std::max(most, plan->first[k] - plan->first[k - 1]);
+    }
+    return most;
+}
+
+// The most chunks of a launch, whatever the levels cost: a launch has fewer than 2^32 threads, and one XCD may have nearly all items
+// (16 levels, 256 threads: 2^17 chunks, 2^25 points and more; a level's tables are long in L2 by then).
+inline size_t level_part_chunks(uint32_t n_levels, uint32_t threads) {
+    const size_t items = ((size_t(1) << 32) - 1) / (kXcds * threads);
+    return std::max<size_t>(1, items / n_levels);
+}
+
+} // namespace tnn
