@@ -179,3 +179,25 @@ def test_backward_takes_its_own_forward_passes_order(tnn, dims, log2, M, interpo
         expected = tnn.grid_backward(d, xs[i], dys[i], FP32)
         scale = float(expected.abs().max())
         assert float((enc.params.grad.reshape(-1) - expected.reshape(-1)).abs().max()) <= 1e-5 * scale  # (fp32 sums in another order: the bar of tnn_grid_backward)
+
+
+@pytest.mark.parametrize("dims,config,M,kept", [
+    (2, dict(n_levels=16, log2_hashmap_size=16), 2 ** 19, False), (3, dict(n_levels=16, log2_hashmap_size=16, interpolation="Nearest"), 2 ** 19, False),
+    (3, dict(n_levels=16, log2_hashmap_size=16), 2 ** 19, True), (2, dict(n_levels=1, n_features_per_level=8, log2_hashmap_size=22, base_resolution=2100), 2 ** 18, True)])
+def test_an_order_is_kept_where_the_backward_pass_reads_it(tnn, dims, config, M, kept):
+    """Between its passes an encoding holds a batch's cell order only where the backward pass takes it: in three dimensions and, in two, where bins refuse levels."""
+    import tiny_dpcpp_nn
+    cfg = dict(BASE, n_dims=dims, **config)
+    enc = tiny_dpcpp_nn.Encoding(dims, {"otype": "HashGrid", "type": "Hash", **{k: v for k, v in cfg.items() if k != "n_dims"}})
+    d = tnn.grid_desc(cfg)
+    gen = torch.Generator(device=tnn.dev).manual_seed(10)
+    x = torch.rand((M, dims), device=tnn.dev, generator=gen)
+    dy = torch.randn((M, enc.n_output_dims), device=tnn.dev, generator=gen)
+    before = torch.cuda.memory_allocated()
+    y = enc(x)
+    extra = torch.cuda.memory_allocated() - before - y.numel() * 4
+    assert (extra >= 16 * M) if kept else (extra < 16 * M)
+    y.backward(dy)
+    expected = tnn.grid_backward(d, x, dy, FP32)
+    scale = float(expected.abs().max())
+    assert float((enc.params.grad.reshape(-1) - expected.reshape(-1)).abs().max()) <= 1e-5 * scale  # (fp32 sums in another order: the bar of tnn_grid_backward)

@@ -93,6 +93,13 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
         const bool ordered = forward_scratch_bytes(batch_size) ? tnn_grid_levels_want_order(&m_desc, batch_size) != 0 : batch_size >= kCellOrderMinBatch;
         return ordered ? tnn_grid_order_bytes(&m_desc, batch_size) : 0;
     }
+    /// Whether backward_with_scratch reads an order of batch_size points that is there. One is worth its boxes in three dimensions (2^19 entries, 2^20
+    /// points, whole scatter 723 -> 633 us), not in two, whose rows of dL/dy are then read in another order than they lie in (2^20 points, forward and
+    /// backward 595 -> 603), unless the bins refuse levels. Nearest is the faster for the caller's order either way.
+    bool backward_takes_order(const size_t batch_size) const {
+        if (m_desc.interpolation == TNN_INTERP_NEAREST) return false;
+        return m_desc.n_dims == 3 || tnn_grid_backward_wants_order(&m_desc, batch_size) != 0;
+    }
     void forward_with_scratch(const DeviceMatrixView<float> input, DeviceMatrixView<T> *output, void *scratch, const size_t scratch_bytes, void *order,
                               const size_t order_bytes) {
         if (!check_forward(input, output, false, false)) return;
@@ -170,10 +177,8 @@ template <typename T> class GridEncodingTemplated : public GridEncoding<T> {
     }
     void run_backward(const DeviceMatrixView<float> input, const DeviceMatrixView<T> dL_doutput, DeviceMatrixView<T> *gradients, void *scratch,
                       const size_t scratch_bytes, GradientMode param_gradients_mode, const void *order = nullptr) {
-        // An order that is there is worth its boxes in three dimensions (2^19 entries, 2^20 points, whole scatter 723 -> 633 us), not in two, whose rows of
-        // dL/dy are then read in another order than they lie in (2^20 points, forward and backward 595 -> 603); made for this pass alone it is where the
-        // bins refuse levels. Nearest is the faster for the caller's order either way.
-        if (m_desc.interpolation == TNN_INTERP_NEAREST || m_desc.n_dims == 2) order = nullptr;
+        if (!backward_takes_order(input.m())) order = nullptr;
+        // (made for this pass alone it is worth it where the bins refuse levels)
         if (!order && tnn_grid_backward_wants_order(&m_desc, input.m())) order = ordered(input);
         tnn::abi_check(tnn_grid_backward_binned(&m_desc, input.GetPointer(), order, dL_doutput.GetPointer(), TNN_FP32,
                                                 this->get_padded_output_width(), gradients->GetPointer(),

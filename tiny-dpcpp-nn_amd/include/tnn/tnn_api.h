@@ -312,7 +312,8 @@ template <typename T> class EncodingModule : public Module {
         const torch::Tensor y = forward_pass(x, order);
         if (keep) {
             pass.input = x;
-            pass.order = order;
+            const auto *grid = dynamic_cast<const tinydpcppnn::encodings::grid::GridEncodingTemplated<T> *>(encoding_.get());
+            if (order.defined() && grid->backward_takes_order((size_t)x.size(0))) pass.order = order;
         }
         return y;
     }
