@@ -201,3 +201,67 @@ def test_an_order_is_kept_where_the_backward_pass_reads_it(tnn, dims, config, M,
     expected = tnn.grid_backward(d, x, dy, FP32)
     scale = float(expected.abs().max())
     assert float((enc.params.grad.reshape(-1) - expected.reshape(-1)).abs().max()) <= 1e-5 * scale  # (fp32 sums in another order: the bar of tnn_grid_backward)
+
+
+class MemoryFor:
+    """PyTorch's allocator gives out about `spare` bytes more than are in use, and no more."""
+
+    def __init__(self, spare):
+        self.spare = spare
+
+    def limit(self, spare):
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + spare) / torch.cuda.get_device_properties(0).total_memory)
+
+    def __enter__(self):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        self.limit(0)
+        self.held = []
+        while True:  # (what is left of the blocks it has)
+            try:
+                self.held.append(torch.empty(2 ** 21, dtype=torch.uint8, device="cuda"))
+            except torch.cuda.OutOfMemoryError:
+                break
+        self.limit(self.spare)
+
+    def __exit__(self, *_):
+        del self.held
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+def test_passes_run_where_memory_is_short(tnn):
+    """Without memory for the encoded batch by levels the passes run as they do without it: the same values (a batch that is not put in cell order)."""
+    import tiny_dpcpp_nn
+    M, grid = 131000, {"otype": "HashGrid", "type": "Hash", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": 14, "base_resolution": 16, "per_level_scale": 1.447}
+    tiny_dpcpp_nn.manual_seed(4)
+    gen = torch.Generator(device=tnn.dev).manual_seed(11)
+    model = tiny_dpcpp_nn.NetworkWithInputEncoding(3, 3, {"otype": "FullyFusedMLP", "activation": "ReLU", "output_activation": "None", "n_neurons": 64, "n_hidden_layers": 2}, grid,
+                                                   dtype=torch.float16, use_bias=False)
+    enc = tiny_dpcpp_nn.Encoding(3, grid)
+    x = torch.rand((M, 3), device=tnn.dev, generator=gen)
+    dy = (torch.randn((M, 3), device=tnn.dev, generator=gen) * 1e-3).half()
+    with torch.no_grad():
+        model.encoding.params.copy_(torch.rand(model.encoding.params.shape, device=tnn.dev, generator=gen) - 0.5)
+        enc.params.copy_(model.encoding.params)
+        encoded = enc(x)
+    y = model(x)
+    assert torch.cuda.memory_allocated() > 64 * M  # (the levels that this pass keeps)
+    y.backward(dy)
+    expected = [p.grad.clone() for p in model.parameters()]
+    model.zero_grad()
+    y = y.detach()
+    with torch.no_grad(), MemoryFor(128 * M + 8 * 2 ** 20):  # a result of 128 bytes a point, and not as much again beside it
+        again = enc(x)
+    assert torch.equal(bits(again), bits(encoded))
+    del again, encoded
+    with MemoryFor(6 * 2 ** 20):  # not 64 bytes a point
+        with torch.no_grad():
+            w = model(x)
+        kept = torch.cuda.memory_allocated()
+        z = model(x)
+        assert torch.cuda.memory_allocated() - kept < 16 * M
+    assert torch.equal(bits(z.detach()), bits(y)) and torch.equal(bits(w), bits(y))
+    z.backward(dy)
+    (dtable, dW), (expected_dtable, expected_dW) = [p.grad for p in model.parameters()], expected
+    assert dW.numel() < dtable.numel() and torch.equal(dW, expected_dW)
+    assert float((dtable - expected_dtable).abs().max()) <= 1e-5 * float(expected_dtable.abs().max())  # (fp32 atomics in no defined order: the bar of tnn_grid_backward)

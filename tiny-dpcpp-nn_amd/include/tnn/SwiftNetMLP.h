@@ -234,6 +234,14 @@ template <typename T, int WIDTH> class SwiftNetMLP : public Network<T> {
                                                          dy_scale, result_scale, dW_packed, dW_dtype, grad_table, 1, M, scratch, scratch_bytes,
                                                          this->get_queue().abi()));
     }
+    /// The same where the levels were not kept: formed again from the table, in the caller's order.
+    void backward_with_grid_rows(const tnn_grid_desc &grid, const void *table, const float *positions, const void *dLdy, const int dy_cols, const float dy_scale,
+                                 const float result_scale, void *dW_packed, const int dW_dtype, float *grad_table, const size_t M, void *scratch,
+                                 const size_t scratch_bytes) {
+        const tnn_mlp_desc d = desc();
+        tnn::abi_check(tnn_grid_mlp_backward_rows(&grid, &d, positions, nullptr, table, this->prepared_forward(), this->prepared_backward(), dLdy, dy_cols, dy_scale,
+                                                  result_scale, dW_packed, dW_dtype, grad_table, 1, M, scratch, scratch_bytes, this->get_queue().abi()));
+    }
     /// Width 128: forward pass that keeps the hidden activations only, and the backward pass on them.
     void forward_rows(const void *x, void *hidden, void *y, const int y_cols, const size_t M) {
         const tnn_mlp_desc d = desc();

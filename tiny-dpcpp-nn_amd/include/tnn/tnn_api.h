@@ -84,7 +84,7 @@ class Module {
     struct RowsPass {
         torch::Tensor input;          // what the kernels read: the caller's tensor, or the padded and converted copy of it
         torch::Tensor hidden, output; // width 128: the hidden activations, and the output where its activation needs it
-        torch::Tensor levels, order;  // behind a grid encoding: the encoded batch, and the cell order it is in (undefined: the caller's)
+        torch::Tensor levels, order;  // behind a grid encoding: the encoded batch (undefined: not kept), and the cell order it is in (undefined: the caller's)
         int64_t rows = 0, cols = 0;   // of the caller's input
         c10::ScalarType dtype = torch::kFloat32;
         bool in_workspace = false; // the activations are in the module's own workspace (forward_pass / backward_pass)
@@ -180,6 +180,15 @@ class Module {
     torch::Tensor fresh(at::IntArrayRef sizes, c10::ScalarType dtype) const { return torch::empty(sizes, torch::TensorOptions().dtype(dtype).device(device())); }
     /// Scratch memory of one call, from the pool the caller's tensors come from (stream-ordered, like the results).
     torch::Tensor scratch(size_t bytes) const { return fresh({(int64_t)bytes}, torch::kUInt8); }
+    /// The same for a faster way that a pass can do without: undefined where there is not as much.
+    torch::Tensor scratch_or_none(size_t bytes) const {
+        if (bytes == 0) return torch::Tensor();
+        try {
+            return scratch(bytes);
+        } catch (const c10::OutOfMemoryError &) {
+            return torch::Tensor();
+        }
+    }
     static int abi_dtype(c10::ScalarType t) {
         switch (t) {
         case torch::kFloat32: return TNN_FP32;
@@ -242,10 +251,10 @@ template <typename T> class EncodingModule : public Module {
         auto *grid = dynamic_cast<tinydpcppnn::encodings::grid::GridEncodingTemplated<T> *>(encoding_.get());
         if (grid) {
             const size_t scratch_bytes = grid->forward_scratch_bytes(batch_size), order_bytes = grid->forward_order_bytes(batch_size);
-            const torch::Tensor work = scratch_bytes ? this->scratch(scratch_bytes) : torch::Tensor();
-            if (order_bytes) order = this->scratch(order_bytes);
-            grid->forward_with_scratch(input_dmv, &output_encoding, scratch_bytes ? work.data_ptr() : nullptr, scratch_bytes, order_bytes ? order.data_ptr() : nullptr,
-                                       order_bytes);
+            const torch::Tensor work = this->scratch_or_none(scratch_bytes); // (where memory is short, the kernel that needs none)
+            order = this->scratch_or_none(order_bytes);
+            grid->forward_with_scratch(input_dmv, &output_encoding, work.defined() ? work.data_ptr() : nullptr, scratch_bytes,
+                                       order.defined() ? order.data_ptr() : nullptr, order_bytes);
         } else {
             encoding_->forward_impl(input_dmv, &output_encoding);
         }
@@ -666,14 +675,16 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
         const float *pushed = PushedWithThePass(push, true);
         const int64_t rows = positions.size(0), n_out = visible_columns();
         torch::Tensor y = fresh({rows, n_out}, kType);
-        if (!keep && !tnn_grid_mlp_wants_levels(grid, (size_t)rows)) {
+        torch::Tensor levels, order;
+        if (keep || tnn_grid_mlp_wants_levels(grid, (size_t)rows)) levels = this->scratch_or_none(tnn_grid_levels_bytes(grid, (size_t)rows));
+        if (!levels.defined()) { // (or where memory is short: a backward pass then forms them again)
             network_.inference_with_grid_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), (size_t)rows, y.data_ptr(), (int)n_out, pushed);
             return y;
         }
         const size_t order_bytes = network_.levels_order_bytes(*grid, (size_t)rows, keep);
-        const torch::Tensor levels = this->scratch(tnn_grid_levels_bytes(grid, (size_t)rows)), order = order_bytes ? this->scratch(order_bytes) : torch::Tensor();
+        order = this->scratch_or_none(order_bytes);
         network_.forward_with_levels_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), (size_t)rows, levels.data_ptr(),
-                                          order_bytes ? order.data_ptr() : nullptr, order_bytes, y.data_ptr(), (int)n_out, pushed);
+                                          order.defined() ? order.data_ptr() : nullptr, order_bytes, y.data_ptr(), (int)n_out, pushed);
         if (keep) {
             pass.levels = levels;
             pass.order = order;
@@ -694,6 +705,13 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
         const c10::ScalarType dW_type = params.scalar_type() == kType ? kType : torch::kFloat32;
         torch::Tensor dW = fresh(params.sizes(), dW_type), dtable = fresh(table.sizes(), torch::kFloat32);
         const torch::Tensor work = this->scratch(network_.backward_with_grid_scratch_bytes(*grid, (size_t)rows));
+        if (!pass.levels.defined()) {
+            const torch::Tensor entries = table.detach().to(torch::kFloat32).contiguous();
+            network_.backward_with_grid_rows(*grid, entries.data_ptr(), positions.data_ptr<float>(), g.data_ptr(), (int)g.size(1), (float)loss_scale,
+                                             (float)(1.0 / loss_scale), dW.data_ptr(), this->abi_dtype(dW_type), dtable.data_ptr<float>(), (size_t)rows, work.data_ptr(),
+                                             (size_t)work.numel());
+            return {dW_type == params.scalar_type() ? dW : dW.to(params.scalar_type()), dtable.to(table.scalar_type())};
+        }
         // the caller's tensor is one autograd saved: it is as it was in the forward pass, whose levels and cell order these are
         network_.backward_with_levels_rows(*grid, positions.data_ptr<float>(), pass.levels.data_ptr(), pass.order.defined() ? pass.order.data_ptr() : nullptr,
                                            g.data_ptr(), (int)g.size(1), (float)loss_scale, (float)(1.0 / loss_scale), dW.data_ptr(), this->abi_dtype(dW_type),
