@@ -68,6 +68,35 @@ def test_order_is_a_permutation_and_forward_is_unchanged(tnn, cfg, kind, M):
     assert torch.equal(plain.view(torch.int16), ordered.view(torch.int16))
 
 
+PIECE = 2048  # records of a bin that are sorted at once
+
+
+@pytest.mark.parametrize("cfg", [CFG4, CFG5])
+@pytest.mark.parametrize("spread", [0, 20000, 2 ** 20 + 5])
+@pytest.mark.parametrize("sizes", [(1, 2, 511, 512, 513), (2047, 2048, 2049), (4096, 4097, 6143, 1), (200001, 513), (3 * PIECE,) * 8])
+def test_every_piece_of_a_bin_is_refined(tnn, cfg, spread, sizes):
+    """Bins on both sides of what a wave and a workgroup sort, neighbours and far apart, alone and among evenly spread points: every piece of every bin is in
+    the order of the next bits."""
+    D = cfg["n_dims"]
+    coarse, fine = (6, 3) if D == 2 else (4, 2)
+    rng = np.random.default_rng(len(sizes) + spread)
+    parts = [rng.uniform(0, 1, (spread, D))]
+    for k, size in enumerate(sizes):
+        cell = [(7 * k + 3) % (1 << coarse)] + [2 + k // 3] * (D - 1) if k % 2 else [k, 1, 1][:D]
+        parts.append((np.array(cell) + rng.uniform(0, 1, (size, D))) / (1 << coarse))
+    x = np.minimum(np.concatenate(parts), 1 - 2.0 ** -20).astype(np.float32)
+    rng.shuffle(x)
+    _, rec, rows = records_of(tnn, tnn.grid_desc(cfg, FP16), torch.from_numpy(x).to(tnn.dev))
+    assert np.array_equal(np.sort(rows), np.arange(len(x), dtype=np.uint32)) and np.array_equal(rec[:, :D], x[rows])
+    q = (rec[:, :D] * np.float32(1 << (coarse + fine))).astype(np.int64)
+    key = sum((q[:, d] >> fine) << (coarse * d) for d in range(D))
+    sub = sum((q[:, d] & ((1 << fine) - 1)) << (fine * d) for d in range(D))
+    first = np.concatenate([[0], np.flatnonzero(np.diff(key)) + 1])
+    place = np.arange(len(x)) - np.repeat(first, np.diff(np.concatenate([first, [len(x)]])))
+    inside = (np.diff(key) == 0) & (place[1:] % PIECE != 0)
+    assert np.all(np.diff(key) >= 0) and np.all(np.diff(sub)[inside] >= 0)
+
+
 def test_ordered_forward_matches_the_oracle_and_every_variant(tnn, oracle):
     rng = np.random.default_rng(3)
     for cfg, pd, od in ((dict(CFG5, n_features_per_level=4, n_levels=8, interpolation="Smoothstep"), FP32, FP32),

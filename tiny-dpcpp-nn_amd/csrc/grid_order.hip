@@ -10,7 +10,7 @@
 // Two steps, neither needs a stable order:
 //   1. counting sort by a 12-bit key, the leading bits of every coordinate with the first dimension fastest (x runs along
 //      a table line): per-workgroup histograms in LDS, one small scan kernel, scatter with LDS counters;
-//   2. inside every one of the 4096 bins, a counting sort in LDS by the next bits of every coordinate.
+//   2. inside every one of the 4096 bins, a counting sort by the next bits of every coordinate.
 // A record is 16 bytes: up to three coordinates and the row number.
 #include "grid_device.h"
 
@@ -21,7 +21,7 @@ constexpr int kOrderBins = 4096;      // 12-bit key
 constexpr int kOrderGroups = 64;      // runs of 64 bins, one scan workgroup each
 constexpr int kOrderMaxWg = 256;      // histogram workgroups (the scan keeps a [workgroups][64] tile in LDS)
 constexpr int kOrderAhead = 4;        // points of a thread under way at once (the whole ordering, 2^18 points: 24.8 us one by one, 21.1 with this and the refinement)
-constexpr int kRefineEach = 8;        // records of a thread that a bin's workgroup sorts in LDS at once
+constexpr int kRefineEach = 8;        // records of a thread in a piece of a bin
 constexpr int kRefineBins = 64;       // 6 further bits
 
 struct OrderPlan {
@@ -180,58 +180,97 @@ __global__ void __launch_bounds__(kOrderThreads)
     }
 }
 
-// Step 2: one workgroup per bin sorts the bin's records by the next bits of the coordinates, in LDS, in pieces of at most
-// 8 THREADS records (a bin that holds more, because the points cluster, is refined piece by piece). THREADS: about as many as the bins hold records, so
-// that the LDS of the workgroups of a small batch leaves many of them a CU (2^18 points: 8.2 us with 256 threads and 32 KB). 64 threads up to 2^18 points,
-// 2^17 in 3-D: a picture's rows fill one bin in sixteen there (encoding and network, us, 256 threads / 64: 2^19 such points 164 / 171, 2^18 104 / 108; scattered 445 / 441,
-// 248 / 243).
-template <int D, int THREADS>
-__global__ void __launch_bounds__(THREADS)
+// Step 2: the records of a bin by the next bits of their coordinates, in pieces of at most kRefinePiece that a workgroup sorts in its registers. The first
+// kOrderBins / PER workgroups take the first pieces of PER bins each. Where points crowd a bin is many pieces, and the further workgroups take the others, side
+// by side: workgroup e the piece that starts in [e, e + 1) * kRefinePiece, which is one at most, since the piece in front of it is full and of the same bin.
+// PER 4, up to 256 points a bin on average: bins of few records are a wave's each, so that no wave of the workgroup is idle, unless one of the four is
+// larger (they lie far apart: of a picture's rows one is). PER 1: more workgroups where bins fill them.
+// The whole ordering, us, against pieces that wait in LDS and follow each other in one workgroup of 64 threads (of 256): 2-D, 2^18 points 21.7, 21.8 (25.5),
+// 2^20 45.5, - (47.4), 2^21 63.4, - (64.2); 2^18 points in a square of a twentieth of the side 22.5, 172 (68), of a hundredth 23.5, 615 (194); 3-D, 2^20 points in a cube
+// of a twentieth 41.5, - (831), near a sphere 43.2, - (44.8), the rows of a picture 40.4, - (41.5). Pieces of 1024 (128 threads) are as fast to sort, but gathers
+// behind them share fewer lines (3-D, 2^21 points near a sphere, all levels 831 us for 793).
+constexpr int kRefineThreads = 256;
+constexpr int kRefinePiece = kRefineEach * kRefineThreads;
+
+// Sorts n <= kRefineEach * GROUP records with GROUP threads. Every thread of the workgroup has to come (the groups share its barriers).
+template <int D, int GROUP> __device__ __forceinline__ void refine_piece(float4 *__restrict__ records, int n, int tid, uint32_t *next) {
+    if (tid < kRefineBins) next[tid] = 0;
+    float4 rec[kRefineEach];
+    uint32_t key[kRefineEach];
+#pragma unroll
+    for (int u = 0; u < kRefineEach; ++u) {
+        rec[u] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (tid + u * GROUP < n) rec[u] = records[tid + u * GROUP];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kRefineEach; ++u) {
+        key[u] = 0;
+        if (tid + u * GROUP < n) {
+            float x[D];
+            x[0] = rec[u].x;
+            x[1] = rec[u].y;
+            if (D > 2) x[D - 1] = rec[u].z;
+            key[u] = fine_key<D>(x);
+            atomicAdd(&next[key[u]], 1u);
+        }
+    }
+    __syncthreads(); // (and all records of the piece are in registers)
+    if (tid < kRefineBins) {
+        const uint32_t c = next[tid];
+        uint32_t incl = c;
+#pragma unroll
+        for (int off = 1; off < kRefineBins; off <<= 1) {
+            const uint32_t v = __shfl_up(incl, off, 64);
+            if (tid >= off) incl += v;
+        }
+        next[tid] = incl - c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kRefineEach; ++u)
+        if (tid + u * GROUP < n) records[atomicAdd(&next[key[u]], 1u)] = rec[u];
+    __syncthreads();
+}
+
+template <int D, int PER>
+__global__ void __launch_bounds__(kRefineThreads)
     order_refine_kernel(const uint32_t *__restrict__ starts, float4 *__restrict__ records, long long M) {
-    constexpr int kRefineThreads = THREADS, kRefineCap = kRefineEach * THREADS;
-    __shared__ float4 rec[kRefineCap];
-    __shared__ uint32_t count[kRefineBins], next[kRefineBins];
-    const int bin = blockIdx.x, tid = threadIdx.x;
-    const long long begin = starts[bin]; // workgroup 0's start of a bin is the start of the bin
-    const long long end = (bin + 1 < kOrderBins) ? (long long)starts[bin + 1] : M;
-    for (long long p0 = begin; p0 < end; p0 += kRefineCap) {
-        const int n = (int)((end - p0 < kRefineCap) ? end - p0 : kRefineCap);
-        if (tid < kRefineBins) count[tid] = 0;
-        __syncthreads();
-        uint32_t key[kRefineCap / kRefineThreads];
+    static_assert(kOrderBins == 64 * 64 && kRefineBins == 64, "the search below is two steps of a wave; a wave scans the counts");
+    constexpr int kGroups = kOrderBins / PER;
+    __shared__ uint32_t next[PER][kRefineBins];
+    const int tid = threadIdx.x, lane = tid & 63, block = blockIdx.x;
+    auto begin_of = [&](int bin) { return bin < kOrderBins ? (long long)starts[bin] : M; }; // (workgroup 0's start of a bin is the start of the bin)
+    if (block >= kGroups) {
+        const long long before = (long long)(block - kGroups + 1) * kRefinePiece - 1; // a record of the piece in front, if there is one of this bin
+        int bin = 64 * (__popcll(__ballot((long long)starts[64 * lane] <= before)) - 1);
+        bin += __popcll(__ballot((long long)starts[bin + lane] <= before)) - 1;
+        const long long begin = starts[bin], p0 = begin + ((before - begin) / kRefinePiece + 1) * kRefinePiece, left = begin_of(bin + 1) - p0;
+        if (left > 0) refine_piece<D, kRefineThreads>(records + p0, (int)(left < kRefinePiece ? left : kRefinePiece), tid, next[0]);
+        return;
+    }
+    if constexpr (PER > 1) {
+        static_assert(PER == kRefineThreads / 64, "a wave for each bin");
+        long long begin = 0, most = 0;
+        int n = 0;
 #pragma unroll
-        for (int u = 0; u < kRefineCap / kRefineThreads; ++u) {
-            const int e = tid + u * kRefineThreads;
-            key[u] = 0;
-            if (e < n) {
-                const float4 r = records[p0 + e];
-                rec[e] = r;
-                float x[D];
-                x[0] = r.x;
-                x[1] = r.y;
-                if (D > 2) x[D - 1] = r.z;
-                key[u] = fine_key<D>(x);
-                atomicAdd(&count[key[u]], 1u);
+        for (int k = 0; k < PER; ++k) {
+            const long long first = starts[block + k * kGroups], size = begin_of(block + k * kGroups + 1) - first;
+            most = most > size ? most : size;
+            if (tid / 64 == k) {
+                begin = first;
+                n = (int)size;
             }
         }
-        __syncthreads();
-        if (tid < kRefineBins) {
-            const uint32_t c = count[tid];
-            uint32_t incl = c;
-#pragma unroll
-            for (int off = 1; off < kRefineBins; off <<= 1) {
-                const uint32_t v = __shfl_up(incl, off, 64);
-                if (tid >= off) incl += v;
-            }
-            next[tid] = incl - c;
+        if (most <= kRefineEach * 64) {
+            refine_piece<D, 64>(records + begin, n, lane, next[tid / 64]);
+            return;
         }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < kRefineCap / kRefineThreads; ++u) {
-            const int e = tid + u * kRefineThreads;
-            if (e < n) records[p0 + atomicAdd(&next[key[u]], 1u)] = rec[e];
-        }
-        __syncthreads();
+    }
+#pragma unroll 1
+    for (int k = 0; k < PER; ++k) {
+        const long long first = starts[block + k * kGroups], size = begin_of(block + k * kGroups + 1) - first;
+        if (size > 1) refine_piece<D, kRefineThreads>(records + first, (int)(size < kRefinePiece ? size : kRefinePiece), tid, next[0]);
     }
 }
 
@@ -271,10 +310,10 @@ TNN_API int tnn_grid_order_points(const tnn_grid_desc *desc, const float *d_x, s
         if ((rc = check_launch("order_scan_kernel"))) return rc;                                                                       \
         TNN_LAUNCH((order_scatter_kernel<D_>), dim3(p.n_wg), dim3(kOrderThreads), 0, s, d_x, (long long)M, p.chunk, (const uint32_t *)hist, records); \
         if ((rc = check_launch("order_scatter_kernel"))) return rc;                                                                    \
-        if (M <= (size_t)kOrderBins * (D_ == 2 ? 64 : 32))                                                                             \
-            TNN_LAUNCH((order_refine_kernel<D_, 64>), dim3(kOrderBins), dim3(64), 0, s, (const uint32_t *)hist, records, (long long)M);      \
+        if (M <= (size_t)kOrderBins * 256)                                                                                             \
+            TNN_LAUNCH((order_refine_kernel<D_, 4>), dim3(kOrderBins / 4 + (unsigned)(M / kRefinePiece)), dim3(kRefineThreads), 0, s, (const uint32_t *)hist, records, (long long)M); \
         else                                                                                                                           \
-            TNN_LAUNCH((order_refine_kernel<D_, 256>), dim3(kOrderBins), dim3(256), 0, s, (const uint32_t *)hist, records, (long long)M);    \
+            TNN_LAUNCH((order_refine_kernel<D_, 1>), dim3(kOrderBins + (unsigned)(M / kRefinePiece)), dim3(kRefineThreads), 0, s, (const uint32_t *)hist, records, (long long)M); \
         return check_launch("order_refine_kernel");                                                                                    \
     } while (0)
     if (desc->n_dims == 2) TNN_ORDER(2);
