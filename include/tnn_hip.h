@@ -365,8 +365,8 @@ int tnn_grid_forward_ordered(const tnn_grid_desc *desc, const void *d_order, con
 
 /* tnn_grid_forward, level by level: the levels go to the XCDs in turn, each of which has a level in its L2 while it gathers from it, and a
  * second pass makes rows of them. Same values, bit for bit. d_order (may be NULL): the records of tnn_grid_order_points, then d_x may be
- * NULL. tnn_grid_forward_workspace_bytes: the workspace it takes where it is the faster call for M points, 0 where it is not (small
- * batches, whose rows tnn_grid_forward writes the same way; large ones of two dimensions or of levels beyond 16 MB). Any M runs, with
+ * NULL. tnn_grid_forward_workspace_bytes: the workspace it takes where it is the faster call for M scattered points, 0 where it is not (small
+ * batches, whose rows tnn_grid_forward writes the same way; few levels, or small ones; large batches of two dimensions or of levels beyond 16 MB). Any M runs, with
  * (n_levels * n_features_per_level rounded up to 16) * sizeof(out_dtype) bytes for each of M points rounded up to 64, and 256 more.
  * tnn_grid_levels_want_order: whether it (with tnn_grid_order_points in front) is the faster for cell order. */
 size_t tnn_grid_forward_workspace_bytes(const tnn_grid_desc *desc, int out_dtype, size_t M);

@@ -75,3 +75,26 @@ def test_scatter_workspace_is_as_large_as_the_header_says(lib):
     assert lib.tnn_grid_desc_init(ctypes.byref(d), 2, 16, 2, 19, 16, 1.5, 0, 1, 1, _lib.TNN_FP16) == 0
     step = int(lib.tnn_grid_mlp_train_step_workspace_bytes(ctypes.byref(d), ctypes.byref(mlp), 2 ** 18) / 2 ** 20)
     assert f"({step} MiB for 2^18 points" in header
+
+
+@pytest.mark.parametrize("dims,features,levels,scale,log2,sides", [
+    # the sizes on both sides of each rule of tnn_grid_forward_workspace_bytes: (points, whether by levels)
+    (2, 2, 8, 1.5, 19, ((2 ** 14, 0), (2 ** 14 + 1, 0), (2 ** 17, 0), (2 ** 18 - 1, 0), (2 ** 18, 1), (2 ** 19 - 1, 1), (2 ** 19, 0))),
+    (2, 2, 8, 2.0, 19, ((2 ** 16, 0), (2 ** 16 + 1, 1), (2 ** 18, 1))),
+    (2, 2, 12, 1.5, 14, ((2 ** 15, 0), (2 ** 18 - 1, 0), (2 ** 18, 1), (3 * 2 ** 17 - 1, 1), (3 * 2 ** 17, 0))),
+    (2, 2, 12, 1.5, 19, ((2 ** 14, 0), (2 ** 14 + 1, 1), (2 ** 18, 1), (3 * 2 ** 17, 0))),
+    (2, 2, 12, 2.0, 19, ((3 * 2 ** 17, 1), (2 ** 19 - 1, 1), (2 ** 19, 0))),
+    (2, 2, 13, 1.5, 14, ((2 ** 14 + 1, 1),)), (2, 2, 16, 1.3, 19, ((3 * 2 ** 17 - 1, 1), (3 * 2 ** 17, 0))), (2, 2, 16, 1.5, 19, ((2 ** 14 + 1, 1), (2 ** 19 - 1, 1), (2 ** 19, 0))),
+    (2, 2, 16, 1.5, 22, ((2 ** 14 + 1, 1), (2 ** 15 - 1, 1), (2 ** 15, 0))), (2, 8, 16, 1.447, 14, ((2 ** 15, 1), (2 ** 15 + 1, 0), (2 ** 18, 0))), (2, 8, 8, 1.447, 14, ((2 ** 15, 0),)),
+    (3, 2, 8, 1.447, 14, ((2 ** 14 + 1, 0), (2 ** 16, 0), (2 ** 16 + 1, 1), (7 * 2 ** 16 - 1, 1), (7 * 2 ** 16, 0))),
+    (3, 2, 8, 1.447, 17, ((2 ** 14 + 1, 1), (7 * 2 ** 16, 0))), (3, 2, 8, 2.0, 17, ((7 * 2 ** 16, 1), (2 ** 20, 1))),
+    (3, 2, 4, 1.447, 19, ((2 ** 16, 0), (2 ** 18 - 1, 0), (2 ** 18, 1), (7 * 2 ** 16, 0))), (3, 2, 16, 1.447, 19, ((2 ** 14, 0), (2 ** 14 + 1, 1), (2 ** 20, 1), (2 ** 24, 1))),
+    (3, 2, 16, 1.447, 22, ((2 ** 17 - 1, 1), (2 ** 17, 0))), (3, 2, 12, 1.447, 22, ((2 ** 16 - 1, 1), (2 ** 16, 0))), (3, 2, 16, 1.447, 21, ((7 * 2 ** 16 - 1, 1), (7 * 2 ** 16, 0))),
+    (3, 8, 16, 1.447, 19, ((2 ** 15, 1), (2 ** 15 + 1, 0), (2 ** 16, 0), (2 ** 16 + 1, 1), (2 ** 18, 0))), (3, 8, 8, 1.447, 19, ((2 ** 17, 0),))])
+def test_encodings_go_by_level_where_that_was_measured_to_be_faster(lib, dims, features, levels, scale, log2, sides):
+    from tiny_dpcpp_nn import _lib
+    d = _lib.GridDesc()
+    assert lib.tnn_grid_desc_init(ctypes.byref(d), dims, levels, features, log2, 16, scale, 0, 1, 1, _lib.TNN_FP32) == 0
+    for M, by_level in sides:
+        need = (levels * features + 15) // 16 * 16 * 4 * ((M + 63) // 64 * 64) + 256
+        assert lib.tnn_grid_forward_workspace_bytes(ctypes.byref(d), _lib.TNN_FP32, M) == by_level * need, M

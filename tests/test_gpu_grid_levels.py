@@ -66,12 +66,15 @@ def test_a_batch_of_several_launches(tnn, ordered):
     assert torch.equal(bits(got), bits(tnn.grid_forward(d, x, table, 32, BF16)))
 
 
-@pytest.mark.parametrize("dims,log2,M", [(3, 16, DIRECT), (3, 16, DIRECT + 1), (3, 19, 2 ** 19 + 3), (2, 16, 2 ** 19 - 1), (2, 16, 2 ** 19), (3, 22, 2 ** 17), (3, 14, 2 ** 19 - 1)])
-def test_encoding_module_on_both_sides_of_each_rule(tnn, dims, log2, M):
+@pytest.mark.parametrize("dims,log2,M,levels", [
+    (3, 16, DIRECT, 16), (3, 16, DIRECT + 1, 16), (3, 19, 2 ** 19 + 3, 16), (2, 16, 2 ** 19 - 1, 16), (2, 16, 2 ** 19, 16), (3, 22, 2 ** 17 - 1, 16), (3, 22, 2 ** 17, 16),
+    (3, 14, 2 ** 19 - 1, 16), (2, 19, 2 ** 18 - 1, 8), (2, 19, 2 ** 18, 8), (2, 14, 3 * 2 ** 17 - 1, 12), (2, 14, 3 * 2 ** 17, 12), (2, 22, 2 ** 15 - 1, 16), (2, 22, 2 ** 15, 16),
+    (3, 14, 2 ** 16, 8), (3, 14, 2 ** 16 + 1, 8), (3, 17, 7 * 2 ** 16 - 1, 8), (3, 17, 7 * 2 ** 16, 8), (3, 19, 2 ** 18 - 1, 4), (3, 19, 2 ** 18, 4)])
+def test_encoding_module_on_both_sides_of_each_rule(tnn, dims, log2, M, levels):
     """The Python encoding takes whichever route its size says; the C ABI in two calls of half the points, or by points, gives the same rows."""
     import tiny_dpcpp_nn
-    cfg = dict(BASE, n_dims=dims, log2_hashmap_size=log2)
-    enc = tiny_dpcpp_nn.Encoding(dims, {"otype": "HashGrid", "type": "Hash", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": log2, "base_resolution": 16,
+    cfg = dict(BASE, n_dims=dims, log2_hashmap_size=log2, n_levels=levels)
+    enc = tiny_dpcpp_nn.Encoding(dims, {"otype": "HashGrid", "type": "Hash", "n_levels": levels, "n_features_per_level": 2, "log2_hashmap_size": log2, "base_resolution": 16,
                                         "per_level_scale": 1.447})
     gen = torch.Generator(device=tnn.dev).manual_seed(6)
     with torch.no_grad():
@@ -80,7 +83,7 @@ def test_encoding_module_on_both_sides_of_each_rule(tnn, dims, log2, M):
         y = enc(x)
     d = tnn.grid_desc(cfg)
     x2 = torch.cat([x, x[: DIRECT + 1]]) if M <= DIRECT else x  # (a batch beyond the small ones)
-    assert torch.equal(bits(y), bits(tnn.grid_forward(d, x2, enc.params.detach().reshape(-1), 32, FP32)[:M]))
+    assert torch.equal(bits(y), bits(tnn.grid_forward(d, x2, enc.params.detach().reshape(-1), 2 * levels, FP32)[:M]))
 
 
 @pytest.mark.parametrize("dims,M", [(2, 2 ** 11 - 1), (2, 2 ** 11), (2, 2 ** 19 - 1), (2, 2 ** 19), (3, 1), (3, 2 ** 17)])

@@ -372,14 +372,51 @@ size_t tnn::largest_level_bytes(const tnn_grid_desc *desc) {
     return entries * entry_bytes(desc);
 }
 
+// Whether M points (more than rows are written directly for) are faster by levels and a pass for the rows than by the kernel that walks all levels of a point.
+// Two launches and a scratch allocation are 11 us through the module however little there is to do, the one kernel 7; beyond that it takes a level's gathers
+// after another's, 0.7 us each in two dimensions and 1.4 in three where lines come from L2, up to 2.6 where they do not, as long as a CU's waves hold the batch
+// (2^16 points), and puts points in cell order from 2^18 on. Points of a picture's rows share lines as they walk nearly as well as by levels (16 levels of 2^19 entries,
+// us, walking / by levels: 2-D, 2^15 points 15 / 15, 2^17 25 / 30, 2^18 55 / 45; 3-D, 2^15 31 / 17, 2^17 38 / 37, 2^20 192 / 275, scattered 569 / 353); which they are is not
+// known here, and an encoding on its own stands in front of a model whose points are scattered. Drawn for such points (fp32, two features unless said otherwise):
+static bool levels_pay(const tnn_grid_desc *desc, size_t M) {
+    const uint32_t L = desc->n_levels, F = desc->n_features_per_level;
+    const size_t largest = tnn::largest_level_bytes(desc);
+    uint32_t n_large = 0, n_fine = 0; // levels of 1 MB and more; levels with no more than a point a cell
+    for (uint32_t l = 0; l < L; ++l) {
+        n_large += (desc->offsets[l + 1] - desc->offsets[l]) * entry_bytes(desc) >= (size_t(1) << 20);
+        const double side = desc->resolutions[l];
+        n_fine += side * side * (desc->n_dims == 3 ? side : 1.0) >= (double)M;
+    }
+    if (desc->n_dims == 2) {
+        // Lines of eight features: 8 levels 15 / 20 (2^16 points), 52 / 62 (2^18); 16 levels 28 / 21 (2^15), 66 / 84 (100 000), 110 / 180 (2^18).
+        if (F == 8 && L > 4) return L > 12 && M <= (size_t(1) << 15);
+        // 32 MB a level, 16 levels: 20 / 15 (24 000 points), 27 / 31 (2^16), 74 / 98 (2^18).
+        if (largest > (size_t(8) << 20)) return L > 8 && M < (size_t(1) << 15);
+        // 8 levels of up to 600 KB: 7 / 11 (2^14 points), 12 / 15 (2^17), 20 / 19 (200 000), 35 / 24 (2^18, ordered); three of 4 MB: 33 / 24 (200 000).
+        // 12 levels of up to 128 KB: 10 / 11, 19 / 23, 32 / 32, 41 / 40; of up to 4 MB 12 / 11, 25 / 25, 48 / 34, 42 / 42. 16 levels: 13 / 11 to 46 / 36 and 20 / 13 to 80 / 45.
+        if (M < (size_t(1) << 18)) return L > 12 || (n_large >= 3 && (L > 8 || M > (size_t(1) << 16)));
+        // Ordered points of levels with many of them a cell share lines as they walk: 2^19 points, finest level 820 a side 70 / 79, 1956 66 / 77, 7006 96 / 94, 524288 106 / 87;
+        // 12 levels of up to 1384 61 / 71. 8 levels 51 / 41. From 2^19 on 169 / 190 (2^20 points).
+        return M < (size_t(3) << 17) || (M < (size_t(1) << 19) && (L <= 8 || 8 * n_fine >= 3 * L));
+    }
+    // 32 MB a level, 16 levels: 42 / 30 (24 000 points), 64 / 63 (2^16), 111 / 93 (100 000), 224 / 237 (2^18); 8 levels 21 / 20, 25 / 26, 39 / 37, 61 / 69.
+    if (largest > (size_t(16) << 20)) return L > 4 && M < (size_t(1) << (L > 12 ? 17 : 16));
+    // 4 levels: 7 / 11 (2^14 points), 11 / 13 (100 000), 16 / 16 (150 000), 37 / 22 (2^18, ordered), 49 / 39.
+    if (L <= 4) return M >= (size_t(1) << 18) && M < (size_t(7) << 16);
+    // Eight features, 16 levels of up to 16 MB: 59 / 51 (2^15 points), 79 / 89 (2^16), 139 / 130 (100 000), 313 / 449 (2^18); of 512 KB 47 / 27, 45 / 46, 92 / 63, 176 / 152;
+    // 8 levels of up to 16 MB 70 / 75 (2^17), 100 / 126.
+    const size_t widest = M >= (size_t(1) << 18) ? 2 : L > 8 ? 16 : 8; // MB
+    if (F == 8 && M > (size_t(1) << 15) && (M <= (size_t(1) << 16) || largest > widest << 20)) return false;
+    // 8 levels of up to 128 KB: 11 / 11 (2^14 points), 13 / 15 (2^16), 24 / 21 (2^17), 50 / 38 (2^18); of up to 1 MB 17 / 11, 19 / 15, 32 / 25, 54 / 44. 16 levels: 22 / 11 to 100 / 71,
+    // 41 / 16 to 173 / 100.
+    if (M <= (size_t(1) << 16)) return L > 8 || largest >= (size_t(1) << 19);
+    // 16 MB a level: 116 / 90 (200 000 points), 161 / 157 (2^18), 270 / 303 (2^19).
+    // As in two dimensions: 2^19 points, 8 levels, finest 212 a side 80 / 89, 2048 144 / 94; 16 levels, 4058 303 / 196; 2^20 points 569 / 353, 8 levels 140 / 146.
+    return M < (size_t(7) << 16) || (largest <= (size_t(8) << 20) && 2 * n_fine >= L);
+}
+
 TNN_API size_t tnn_grid_forward_workspace_bytes(const tnn_grid_desc *desc, int out_dtype, size_t M) {
-    if (check_grid_desc(desc) || M == 0 || grid_rows_direct(M)) return 0;
-    // Points in cell order walk all levels (grid_forward_kernel) where lines come from the memory side in either case, and in 2-D from
-    // 2^19 points on, where few lines are not shared and the rows are a pass of their own. us, with the ordering (points / levels and
-    // rows): 3-D, 2^18 points, 2^19, 2^20, 2^22 entries 171 / 103, 208 / 163, 217 / 240; 2-D, 2^18 points, 2^19 entries 72 / 54,
-    // 2^20 points 171 / 177 ordered, 193 not.
-    if (M >= (size_t(1) << 17) && largest_level_bytes(desc) > (desc->n_dims == 3 ? size_t(16) << 20 : size_t(8) << 20)) return 0;
-    if (M >= (size_t(1) << 19) && desc->n_dims == 2) return 0;
+    if (check_grid_desc(desc) || M == 0 || grid_rows_direct(M) || !levels_pay(desc, M)) return 0;
     return levels_elements(desc, M) * dtype_bytes(out_dtype) + 256;
 }
 
