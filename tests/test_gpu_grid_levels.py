@@ -36,6 +36,10 @@ def by_level(tnn, d, x, order, table, width, out_dtype):
     (dict(BASE, n_features_per_level=4), FP32, FP32, 64), (dict(BASE, n_features_per_level=8, n_levels=3, n_dims=2), FP16, FP16, 24),
     (dict(BASE, n_features_per_level=8, n_levels=7), FP32, FP32, 60), (dict(BASE, n_levels=1), FP32, FP32, 2), (dict(BASE, n_levels=5, interpolation="Smoothstep"), FP32, FP32, 10),
     (dict(BASE, interpolation="Nearest"), FP32, FP32, 32), (dict(BASE, hash="Prime"), FP32, FP32, 32), (dict(BASE, hash="ReversedPrime", n_dims=2), FP16, FP16, 32),
+    (dict(BASE, n_dims=2, n_features_per_level=1), FP32, FP32, 17), (dict(BASE, n_dims=2, n_features_per_level=1, interpolation="Smoothstep"), FP16, FP16, 16),
+    (dict(BASE, n_dims=2, n_features_per_level=4), FP16, FP32, 64), (dict(BASE, n_dims=2, n_features_per_level=4, grid_type="Tiled"), FP16, BF16, 70),
+    (dict(BASE, n_dims=2, n_features_per_level=4, n_levels=6), FP32, FP32, 24), (dict(BASE, n_dims=2, grid_type="Tiled", base_resolution=5), FP32, FP32, 32),
+    (dict(BASE, n_dims=2, n_features_per_level=1, grid_type="Dense", n_levels=5), FP32, BF16, 5),
     (dict(BASE, hash="Rng"), FP32, FP32, 32), (dict(BASE, grid_type="Dense", n_levels=5), FP32, FP32, 12), (dict(BASE, grid_type="Tiled"), FP32, FP32, 32)])
 def test_levels_are_the_rows_of_the_points(tnn, cfg, param_dtype, out_dtype, width):
     d = tnn.grid_desc(cfg, param_dtype)
@@ -51,6 +55,21 @@ def test_levels_are_the_rows_of_the_points(tnn, cfg, param_dtype, out_dtype, wid
         part = x[:m].contiguous()
         assert torch.equal(bits(tnn.grid_forward(d, part, table, width, out_dtype)), bits(expected[:m]))
         assert torch.equal(bits(tnn.grid_forward_ordered(d, tnn.grid_order(d, part), table, width, m, out_dtype)), bits(expected[:m]))
+
+
+@pytest.mark.parametrize("features,param_dtype,out_dtype,M", [(1, FP32, FP32, 2 ** 19), (1, FP16, BF16, 2 ** 19 + 77), (4, FP32, FP16, 2 ** 19 + 1), (4, FP16, FP32, 2 ** 19 - 1),
+                                                              (8, FP32, BF16, 2 ** 19 + 513), (8, FP16, FP16, 2 ** 19), (2, FP32, FP32, 2 ** 19 - 1)])
+def test_large_batches_of_three_dimensions(tnn, features, param_dtype, out_dtype, M):
+    """On both sides of the size from which a thread takes two points."""
+    cfg = dict(BASE, n_levels=5, n_features_per_level=features, log2_hashmap_size=13, base_resolution=13, interpolation="Smoothstep")
+    d = tnn.grid_desc(cfg, param_dtype)
+    gen = torch.Generator(device=tnn.dev).manual_seed(12)
+    table = (torch.rand(tnn.grid_n_params(d), device=tnn.dev, generator=gen) * 2 - 1).to(TORCH[param_dtype])
+    x = torch.rand((M, 3), device=tnn.dev, generator=gen)
+    width = 5 * features
+    expected = bits(tnn.grid_forward(d, x, table, width, out_dtype))
+    assert torch.equal(bits(by_level(tnn, d, x, None, table, width, out_dtype)), expected)
+    assert torch.equal(bits(by_level(tnn, d, x, tnn.grid_order(d, x), table, width, out_dtype)), expected)
 
 
 @pytest.mark.parametrize("ordered", [False, True])
@@ -86,19 +105,36 @@ def test_encoding_module_on_both_sides_of_each_rule(tnn, dims, log2, M, levels):
     assert torch.equal(bits(y), bits(tnn.grid_forward(d, x2, enc.params.detach().reshape(-1), 2 * levels, FP32)[:M]))
 
 
-@pytest.mark.parametrize("dims,M", [(2, 2 ** 11 - 1), (2, 2 ** 11), (2, 2 ** 19 - 1), (2, 2 ** 19), (3, 1), (3, 2 ** 17)])
-def test_field_module_on_both_sides_of_each_rule(tnn, dims, M):
-    """NetworkWithInputEncoding without autograd takes the route its size says; with autograd the one that keeps the encoded batch: the same rows."""
+# (dimensions, levels, log2 of a level's entries, points, whether inference goes by levels, whether in cell order): both sides of each rule
+FIELD_SIDES = [
+    (2, 16, 14, 2 ** 11 - 1, 0, 0), (2, 16, 14, 2 ** 11, 1, 0), (2, 13, 14, 2 ** 15 - 1, 1, 0), (2, 12, 14, 2 ** 15 - 1, 0, 0), (2, 16, 14, 2 ** 15, 0, 0), (2, 16, 14, 2 ** 18 - 1, 0, 0),
+    (2, 12, 14, 2 ** 18, 1, 0), (2, 16, 14, 2 ** 19 - 1, 1, 0), (2, 16, 14, 2 ** 19, 0, 0), (2, 16, 21, 2 ** 18, 0, 0), (3, 16, 14, 1, 1, 0), (3, 8, 14, 2 ** 16 - 1, 0, 0),
+    (3, 8, 14, 2 ** 16, 1, 0), (3, 9, 14, 2 ** 16 - 1, 1, 0), (3, 16, 22, 2 ** 17 - 1, 1, 0), (3, 16, 22, 2 ** 17, 0, 0), (3, 16, 22, 2 ** 20 - 1, 0, 0), (3, 16, 22, 2 ** 20, 1, 1),
+    (3, 16, 19, 5 * 2 ** 17 - 1, 1, 0), (3, 16, 19, 5 * 2 ** 17, 1, 1)]
+
+
+@pytest.mark.parametrize("dims,levels,log2,M,by_levels,ordered", FIELD_SIDES)
+def test_field_module_on_both_sides_of_each_rule(tnn, dims, levels, log2, M, by_levels, ordered):
+    """NetworkWithInputEncoding without autograd takes the route its size says; with autograd the one that keeps the encoded batch, a few points alone another: the
+    same rows."""
     import tiny_dpcpp_nn
     tiny_dpcpp_nn.manual_seed(3)
     model = tiny_dpcpp_nn.NetworkWithInputEncoding(
         dims, 3, {"otype": "FullyFusedMLP", "activation": "ReLU", "output_activation": "None", "n_neurons": 64, "n_hidden_layers": 2},
-        {"otype": "HashGrid", "type": "Hash", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": 14, "base_resolution": 16, "per_level_scale": 1.5},
+        {"otype": "HashGrid", "type": "Hash", "n_levels": levels, "n_features_per_level": 2, "log2_hashmap_size": log2, "base_resolution": 16, "per_level_scale": 1.5},
         dtype=torch.float16, use_bias=False)
+    d = tnn.grid_desc(dict(BASE, n_dims=dims, n_levels=levels, log2_hashmap_size=log2, per_level_scale=1.5))
+    assert tnn.lib.tnn_grid_mlp_wants_levels(ctypes.byref(d), M) == by_levels
     x = torch.rand((M, dims), device=tnn.dev)
     with torch.no_grad():
         model.encoding.params.copy_(torch.rand(model.encoding.params.shape, device=tnn.dev) - 0.5)
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
         y = model(x)
+        scratch = torch.cuda.max_memory_allocated() - before - 6 * M
+        if M >= 2 ** 11:  # 2 bytes of 16 or 32 features a point, and 16 bytes and the histograms of an order
+            assert (scratch >= 64 * M * (levels > 8) + 32 * M * (levels <= 8)) == bool(by_levels) and (scratch >= (64 + 16) * M) == bool(ordered)
+        assert torch.equal(bits(y[-1000:]), bits(model(x[-1000:].contiguous())))
     assert torch.equal(bits(y), bits(model(x).detach()))
 
 
