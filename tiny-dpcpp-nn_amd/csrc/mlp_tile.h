@@ -247,6 +247,9 @@ template <typename T, int W> struct Tile {
     // The same store from one offset per tile (that of the lane's 16 bytes in the first of its rows) and a constant per
     // instruction. Rows past the end of the matrix need no flag: their offsets lie past the end of the buffer resource and the
     // range check drops them (the resource covers less than 2^31 bytes, so an offset cannot wrap back into range).
+    // The constant is part of the lane's offset, not the scalar one: behind a store whose offset is a scalar register the compiler leaves no
+    // wait states before the data may be overwritten, and gfx950 needs them there, too (a v_mov into the fourth register right behind the last
+    // store: now and then 16 of the 64 lanes stored what the v_mov had written).
     static __device__ __forceinline__ unsigned int staged_base(long long tile, int lane) {
         return (unsigned int)((tile * 32 + lane / LPR) * (W * (long long)sizeof(T))) + (lane % LPR) * 16;
     }
@@ -255,7 +258,7 @@ template <typename T, int W> struct Tile {
 #pragma unroll
         for (int i = 0; i < NK; ++i)
             __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4 *>(tile_lds + (i * RPI + lane / LPR) * PITCH + (lane % LPR) * 16),
-                                                   rows, base, i * RPI * W * (int)sizeof(T), AUX);
+                                                   rows, base + i * RPI * W * (int)sizeof(T), 0, AUX);
     }
 
     static constexpr int NF = NI * NK; // weight fragments per matrix and lane
