@@ -115,8 +115,8 @@ FIELD_SIDES = [
 
 @pytest.mark.parametrize("dims,levels,log2,M,by_levels,ordered", FIELD_SIDES)
 def test_field_module_on_both_sides_of_each_rule(tnn, dims, levels, log2, M, by_levels, ordered):
-    """NetworkWithInputEncoding without autograd takes the route its size says; with autograd the one that keeps the encoded batch, a few points alone another: the
-    same rows."""
+    """NetworkWithInputEncoding without autograd takes the route its size says, with autograd the one that keeps the encoded batch: the rows of the network on a batch
+    that one kernel encoded, all levels of a point."""
     import tiny_dpcpp_nn
     tiny_dpcpp_nn.manual_seed(3)
     model = tiny_dpcpp_nn.NetworkWithInputEncoding(
@@ -134,7 +134,9 @@ def test_field_module_on_both_sides_of_each_rule(tnn, dims, levels, log2, M, by_
         scratch = torch.cuda.max_memory_allocated() - before - 6 * M
         if M >= 2 ** 11:  # 2 bytes of 16 or 32 features a point, and 16 bytes and the histograms of an order
             assert (scratch >= 64 * M * (levels > 8) + 32 * M * (levels <= 8)) == bool(by_levels) and (scratch >= (64 + 16) * M) == bool(ordered)
-        assert torch.equal(bits(y[-1000:]), bits(model(x[-1000:].contiguous())))
+        x2 = torch.cat([x, torch.rand((DIRECT, dims), device=tnn.dev)])[: max(M, DIRECT + 1)]  # (a batch beyond those that are written by levels)
+        walked = tnn.grid_forward(d, x2, model.encoding.params.detach().reshape(-1), 64, FP32)[:M]
+        assert torch.equal(bits(y), bits(model.network(walked)))
     assert torch.equal(bits(y), bits(model(x).detach()))
 
 

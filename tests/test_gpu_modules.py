@@ -8,6 +8,8 @@ where the kernels round.
 
 Tolerances: tests/tolerances.py (bf16 1e-2 rel / 1e-3 abs, fp16 5e-3 rel / 5e-4 abs; end to end "propagated").
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -372,8 +374,8 @@ def test_training_without_stored_activations_equals_the_stored_route(tcnn, dtype
     (torch.float16, 2, GRID_2D, 2, 4096), (torch.bfloat16, 2, GRID_2D, 1, 1001),
     (torch.float16, 3, {"otype": "HashGrid", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": 14, "base_resolution": 16, "per_level_scale": 1.447}, 3, 2048)])
 def test_network_with_grid_encoding_trains_through_one_kernel(tcnn, oracle, dtype, n_dims, grid, n_hidden, batch):
-    """NetworkWithInputEncoding with autograd on a grid encoding: forward is the fused inference kernel, backward one kernel
-    that forms encoding and activations again plus the scatter. Against the two modules in turn (the reference's only route,
+    """NetworkWithInputEncoding with autograd on a grid encoding, one call each way: the encoding by levels and the network on them, and its
+    backward pass on the same levels plus the scatter. Against the two modules in turn (the reference's only route,
     dpcpp_bindings/tiny_dpcpp_nn/modules.py:389-407) on the same model: output bit for bit, network gradients to a unit in the
     last place of the network's type, table gradients to 1e-5 of their largest; and against the oracle's chain."""
     torch.manual_seed(17)
@@ -392,7 +394,7 @@ def test_network_with_grid_encoding_trains_through_one_kernel(tcnn, oracle, dtyp
         return out.detach(), model.network.params.grad.clone(), model.encoding.params.grad.clone()
 
     y2, dnet2, dtab2 = grads(model.network_with_encoding)   # Encoding.forward, then Network.forward
-    y1, dnet1, dtab1 = grads(model)                        # one kernel each way
+    y1, dnet1, dtab1 = grads(model)                        # one call each way
     assert y1.shape == (batch, 3) and y1.dtype == dtype
     assert torch.equal(y1.view(torch.int16), y2.view(torch.int16))
     net_scale, tab_scale = float(dnet2.abs().max()), float(dtab2.abs().max())
@@ -568,8 +570,8 @@ def test_parameter_free_encodings_through_the_package(tcnn, oracle):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("n_dims, grid, batch", [(2, "GRID_2D", 1001), (3, "GRID_3D", 4096)])
 def test_network_with_grid_encoding_fused_inference(tcnn, dtype, n_dims, grid, batch):
-    """Evaluation without autograd takes the single-kernel route (encoding + network); with autograd enabled the two
-    modules run in turn. Same bits either way, also for a batch that is padded to a multiple of 8."""
+    """Evaluation without autograd is one call (encoding and network, in one kernel or by levels), with the bits of the two modules in turn, also for a
+    batch that is padded to a multiple of 8."""
     cfg = dict(GRID_2D) if grid == "GRID_2D" else {"otype": "HashGrid", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": 15,
                                                    "base_resolution": 16, "per_level_scale": 1.447}
     torch.manual_seed(3)
@@ -579,7 +581,7 @@ def test_network_with_grid_encoding_fused_inference(tcnn, dtype, n_dims, grid, b
     model.eval()
     assert model.network.tnn_module.can_fuse_encoding(model.encoding.tnn_module)
     x = torch.rand((batch, n_dims), device=DEVICE)
-    two_calls = model(x).detach()  # autograd on: Encoding.forward, then Network.forward
+    two_calls = model.network_with_encoding(x).detach()  # Encoding.forward, then Network.forward
     with torch.no_grad():
         fused = model(x)
     assert fused.shape == two_calls.shape == (batch, 5) and fused.dtype == dtype
@@ -732,10 +734,14 @@ def test_modules_follow_the_callers_stream(tcnn):
 
 
 def test_large_batches_take_the_cell_order_route(tcnn):
-    """From 2^18 rows on the grid encoding (alone, and fused with the network) orders the batch by cell first. Row for row the
-    result equals what the same rows give in batches below the threshold."""
-    n = (1 << 19) + 40
-    cfg = {"otype": "HashGrid", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": 17, "base_resolution": 16, "per_level_scale": 1.447}
+    """Large batches of the grid encoding are ordered by cell first, alone from 2^18 rows on and with the network from 5 * 2^17, where that is the faster. Row for row
+    the result equals what the same rows give in batches below the threshold."""
+    n = (5 << 17) + 40
+    cfg = {"otype": "HashGrid", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": 19, "base_resolution": 16, "per_level_scale": 1.447}
+    from tiny_dpcpp_nn import _lib
+    desc = _lib.GridDesc()
+    _lib.check(_lib.load().tnn_grid_desc_init(ctypes.byref(desc), 3, 16, 2, 19, 16, 1.447, 0, 1, 1, _lib.TNN_FP32))
+    assert _lib.load().tnn_grid_levels_want_order(ctypes.byref(desc), n) == 1
     torch.manual_seed(5)
     model = tcnn.NetworkWithInputEncoding(3, 4, net_config(64, 2), cfg, dtype=torch.float16, use_bias=False)
     with torch.no_grad():
@@ -752,9 +758,8 @@ def test_large_batches_take_the_cell_order_route(tcnn):
 
 
 def test_large_batches_scatter_in_cell_order(tcnn):
-    """From 2^17 rows on the grid encoding's backward pass orders the batch by cell and scatters over the ordered points. The
-    gradient of the table is a sum over rows: the large batch's gradient equals the sum of the gradients of its two halves
-    (each below the threshold, scattered in the caller's order) up to fp32 rounding of sums in another order."""
+    """The gradient of the table is a sum over rows: a large batch's gradient equals the sum of the gradients of its two halves up to fp32 rounding of sums
+    in another order."""
     n = 1 << 17
     cfg = {"otype": "HashGrid", "n_levels": 16, "n_features_per_level": 2, "log2_hashmap_size": 15, "base_resolution": 16, "per_level_scale": 1.5}
     torch.manual_seed(6)
