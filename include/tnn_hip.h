@@ -492,9 +492,11 @@ int tnn_grid_mlp_backward_rows(const tnn_grid_desc *grid, const tnn_mlp_desc *ml
  * tnn_grid_mlp_push_inference_rows with the encoding level by level, which leaves the encoded batch in d_levels (tnn_grid_levels_bytes, 16-byte
  * aligned; values in the network's type); and tnn_grid_mlp_backward_rows on these levels instead of the table. The backward pass of a forward
  * pass that was given d_order takes the same records. Same values as those calls, bit for bit.
- * tnn_grid_mlp_wants_levels: whether the forward pass is the faster this way for M points (where not, its bytes of scratch buy nothing). */
+ * tnn_grid_mlp_width_wants_levels: whether the forward pass of a network of that width is the faster this way for M points, scattered ones or those of a
+ * picture's rows (where not, its bytes of scratch buy nothing); tnn_grid_mlp_wants_levels: of width 64. */
 size_t tnn_grid_levels_bytes(const tnn_grid_desc *grid, size_t M);
 int tnn_grid_mlp_wants_levels(const tnn_grid_desc *grid, size_t M);
+int tnn_grid_mlp_width_wants_levels(const tnn_grid_desc *grid, int width, size_t M);
 int tnn_grid_mlp_forward_levels(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_src_packed, int unpadded_input_width,
                                 int unpadded_output_width, int use_bias, void *d_packed_T, void *d_packed_transposed_T, void *d_prepared_fwd,
                                 void *d_prepared_bwd, const float *d_x, const void *d_order, const void *d_table, void *d_levels, void *d_y,

@@ -98,3 +98,22 @@ def test_encodings_go_by_level_where_that_was_measured_to_be_faster(lib, dims, f
     for M, by_level in sides:
         need = (levels * features + 15) // 16 * 16 * 4 * ((M + 63) // 64 * 64) + 256
         assert lib.tnn_grid_forward_workspace_bytes(ctypes.byref(d), _lib.TNN_FP32, M) == by_level * need, M
+
+
+@pytest.mark.parametrize("dims,features,levels,log2,width,sides", [
+    # on both sides of each rule of tnn_grid_mlp_width_wants_levels: (points, whether by levels)
+    (3, 2, 1, 14, 128, ((1, 1), (2 ** 21, 1))), (3, 4, 1, 14, 128, ((1, 0),)), (2, 1, 1, 14, 128, ((1, 1),)), (2, 2, 8, 14, 128, ((2 ** 14, 0),)), (2, 2, 11, 14, 128, ((2 ** 14, 1), (2 ** 18 - 1, 1))),
+    (3, 1, 1, 14, 64, ((1, 1),)), (2, 1, 8, 14, 64, ((1, 0),)), (3, 1, 8, 14, 32, ((1, 0),)), (2, 4, 9, 14, 64, ((2 ** 18, 1),)), (2, 4, 10, 14, 64, ((2 ** 18, 0),)),
+    (2, 2, 8, 14, 64, ((2 ** 18 - 1, 0), (2 ** 18, 1), (2 ** 20, 1), (2 ** 20 + 1, 0))), (2, 2, 16, 20, 64, ((2 ** 18, 1), (2 ** 19 - 1, 1), (2 ** 19, 0))), (2, 2, 16, 21, 64, ((2 ** 18, 0),)),
+    (3, 2, 11, 14, 32, ((2 ** 15 - 1, 1),)), (3, 1, 11, 14, 16, ((2 ** 15 - 1, 0), (2 ** 18, 1))), (3, 4, 11, 14, 64, ((23999, 1), (24000, 0))), (3, 2, 11, 20, 32, ((2 ** 15 - 1, 1), (2 ** 17, 1))),
+    (3, 2, 11, 21, 32, ((23999, 1), (24000, 0), (2 ** 20, 0))), (3, 2, 8, 16, 16, ((2 ** 18 - 1, 0), (2 ** 18, 1))), (3, 2, 8, 18, 16, ((2 ** 18, 0),)), (3, 8, 6, 14, 64, ((2 ** 18, 1), (2 ** 19, 0))),
+    (3, 8, 7, 14, 64, ((2 ** 18, 0),)), (3, 4, 4, 14, 64, ((2 ** 18 - 1, 0), (2 ** 19, 1))), (3, 4, 5, 14, 64, ((2 ** 19, 0),)), (3, 2, 8, 14, 64, ((2 ** 16 - 1, 0), (2 ** 16, 1))),
+    (3, 2, 2, 14, 64, ((2 ** 17 - 1, 0), (2 ** 17, 1))), (3, 2, 8, 14, 32, ((2 ** 18 - 1, 0), (2 ** 18, 1)))])
+def test_networks_go_by_level_where_that_was_measured_to_be_faster(lib, dims, features, levels, log2, width, sides):
+    from tiny_dpcpp_nn import _lib
+    d = _lib.GridDesc()
+    assert lib.tnn_grid_desc_init(ctypes.byref(d), dims, levels, features, log2, 16, 2.0, 0, 1, 1, _lib.TNN_FP32) == 0
+    for M, by_level in sides:
+        assert lib.tnn_grid_mlp_width_wants_levels(ctypes.byref(d), width, M) == by_level, M
+        assert width != 64 or lib.tnn_grid_mlp_wants_levels(ctypes.byref(d), M) == by_level
+    assert lib.tnn_grid_mlp_width_wants_levels(ctypes.byref(d), width, 0) == 0

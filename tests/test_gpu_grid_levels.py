@@ -140,10 +140,11 @@ def test_encoding_module_on_both_sides_of_each_rule(tnn, dims, log2, M, levels):
 
 # (dimensions, levels, log2 of a level's entries, points, whether inference goes by levels, whether in cell order): both sides of each rule
 FIELD_SIDES = [
-    (2, 16, 14, 2 ** 11 - 1, 0, 0), (2, 16, 14, 2 ** 11, 1, 0), (2, 13, 14, 2 ** 15 - 1, 1, 0), (2, 12, 14, 2 ** 15 - 1, 0, 0), (2, 16, 14, 2 ** 15, 0, 0), (2, 16, 14, 2 ** 18 - 1, 0, 0),
-    (2, 12, 14, 2 ** 18, 1, 0), (2, 16, 14, 2 ** 19 - 1, 1, 0), (2, 16, 14, 2 ** 19, 0, 0), (2, 16, 21, 2 ** 18, 0, 0), (3, 16, 14, 1, 1, 0), (3, 8, 14, 2 ** 16 - 1, 0, 0),
-    (3, 8, 14, 2 ** 16, 1, 0), (3, 9, 14, 2 ** 16 - 1, 1, 0), (3, 16, 22, 2 ** 17 - 1, 1, 0), (3, 16, 22, 2 ** 17, 0, 0), (3, 16, 22, 2 ** 20 - 1, 0, 0), (3, 16, 22, 2 ** 20, 1, 1),
-    (3, 16, 19, 5 * 2 ** 17 - 1, 1, 0), (3, 16, 19, 5 * 2 ** 17, 1, 1)]
+    (2, 16, 19, 2 ** 13 - 1, 0, 0), (2, 16, 19, 2 ** 13, 1, 0), (2, 13, 19, 23999, 1, 0), (2, 13, 19, 24000, 0, 0), (2, 12, 19, 2 ** 13, 0, 0), (2, 16, 14, 2 ** 13, 0, 0),
+    (2, 16, 14, 2 ** 18 - 1, 0, 0), (2, 16, 14, 2 ** 18, 1, 0), (2, 16, 14, 2 ** 19, 1, 0), (2, 16, 14, 2 ** 19 + 1, 0, 0), (2, 8, 14, 2 ** 20, 1, 0), (2, 16, 19, 2 ** 19 - 1, 1, 0),
+    (2, 16, 19, 2 ** 19, 0, 0), (2, 16, 21, 2 ** 18, 0, 0), (3, 16, 14, 1, 1, 0), (3, 11, 14, 2 ** 15 - 1, 1, 0), (3, 10, 14, 2 ** 15 - 1, 0, 0), (3, 16, 22, 23999, 1, 0),
+    (3, 16, 22, 24000, 0, 0), (3, 16, 22, 2 ** 20, 0, 0), (3, 8, 14, 2 ** 16 - 1, 0, 0), (3, 8, 14, 2 ** 16, 1, 0), (3, 11, 14, 2 ** 15, 1, 0), (3, 2, 14, 2 ** 17 - 1, 0, 0),
+    (3, 2, 14, 2 ** 17, 1, 0), (3, 16, 19, 5 * 2 ** 17 - 1, 1, 0), (3, 16, 19, 5 * 2 ** 17, 1, 1)]
 
 
 @pytest.mark.parametrize("dims,levels,log2,M,by_levels,ordered", FIELD_SIDES)

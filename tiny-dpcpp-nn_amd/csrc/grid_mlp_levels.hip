@@ -116,25 +116,41 @@ TNN_API size_t tnn_grid_levels_bytes(const tnn_grid_desc *grid, size_t M) {
     return check_grid_desc(grid) || M == 0 ? 0 : levels_elements(grid, M) * 2;
 }
 
-TNN_API int tnn_grid_mlp_wants_levels(const tnn_grid_desc *grid, size_t M) {
-    if (check_grid_desc(grid) || M == 0) return 0;
-    // By levels is two launches, 13 us through the module however few the points are; one kernel takes a tile's gathers in a row: 10 us with 8 levels, more with
-    // each level and corner. Points of a picture's rows share their lines of the table in one kernel nearly as well as by levels, scattered ones do not, and which
-    // they are is not known here: by levels where neither is slower (module, us, one kernel / levels, rows of a picture and scattered points).
-    // 2-D, 16 levels: 100 points 10.3 / 13.1; 6000 14.6 / 13.0 and 21.6 / 13.1; 30000 15.0 / 14.7 and 22.8 / 15.0; 108895 20.2 / 24.0 and 43.2 / 27.0;
-    // 2^18 53 / 38 and 71 / 48 (ordered from there in one kernel); 2^20 scattered 150 / 168. 12 levels: 16000 11.4 / 13.0. 8 levels: 30000 9.6 / 12.1,
-    // 140000 14.4 / 15.7, 2^18 40 / 21.
-    if (grid->n_dims == 2) {
-        if (M >= (size_t(1) << 19) || M < (size_t(1) << 11)) return 0;
-        if (M < (size_t(1) << 18) && (grid->n_levels <= 12 || M >= (size_t(1) << 15))) return 0;
+// Whether M points are faster by levels. That is two launches and a scratch allocation, 11.7 us through the module however few the points are; one kernel is 8 us, and takes
+// a tile's gathers in a row: more with each level and corner, least at small widths, whose registers leave a SIMD more waves. From 2^18 points on it has them in cell order first. Points of a
+// picture's rows share their lines of the table in one kernel as well as by levels or better, scattered ones do not, and which they are is not known here: by levels where
+// neither is slower. Drawn over 11898 configurations (dimensions, levels, features, width, table, resolutions, points; one kernel / levels, us, scattered points and a picture's rows). With this
+// rule 1.0 % of them are more than 10 % slower than one kernel for one or the other; on average they take 0.76 of its time, rows 0.78 (the faster one each time 0.72 and 0.77; a rule
+// that looked at dimensions, points and levels only 0.81 and 0.85, and 6.8 % were slower).
+static bool levels_pay(const tnn_grid_desc *grid, int width, size_t M) {
+    const uint32_t D = grid->n_dims, L = grid->n_levels, F = grid->n_features_per_level;
+    const size_t largest = largest_level_bytes(grid), MB = size_t(1) << 20;
+    // A tile of so many levels in one kernel does not fit its registers: 3-D, width 128, two features 0.05 to 0.23 of its time by levels, width 64, one feature 0.3.
+    if (width == 128 && F <= (D == 3 ? 2u : 1u)) return true;
+    if (width == 64 && F == 1 && D == 3) return true;
+    if (D == 2) {
+        // Width 64, two features. 8 levels of up to 1 MB: 2^18 points 40 / 21, 2^20 0.75 of the time and 0.63; 12 levels 2^20 1.10 and 0.79; 16 levels 2^18 0.78 and 0.69, beyond 2^19 1.16 and 1.12;
+        // of up to 8 MB 0.89 and 0.71, beyond 2^19 1.18 and 1.09; beyond 8 MB 1.1 to 1.3. 8 levels of eight features 1.1 to 1.3.
+        if (M >= (size_t(1) << 18)) return L * F <= 36 && (largest <= MB ? M * L <= (size_t(1) << 23) : largest <= 8 * MB && M < (size_t(1) << 19));
+        if (width == 128) return F > 1 && L > 10; // 0.6 and 0.7
+        // 16 levels of more than 1 MB: 2^13 points 0.60 and 0.84, 2^14 0.72 and 1.05; of less 1.1 and 1.2, and so are fewer levels.
+        return width == 64 && F == 2 && L > 12 && largest > MB && M >= (size_t(1) << 13) && M < 24000;
     }
-    // 3-D, 16 levels: 100 scattered points 16.8 / 13.2, 6000 of a picture 18.0 / 13.2; 8 levels: 30000 12.1 / 12.9 (scattered, 17000: 21.6 / 12.9), 108895 20.6 / 18.9.
-    if (grid->n_dims == 3 && grid->n_levels <= 8 && M < (size_t(1) << 16)) return 0;
-    // 2^22 entries (32 MB a level), 3-D, 2^18 points, 2^20, 2^21: 212 / 224, 704 / 704, 1288 / 1265; 2^21 entries, 2^21 points 1271 / 1145.
-    const size_t largest = largest_level_bytes(grid);
-    if (grid->n_dims == 3) return M < (size_t(1) << 17) || M >= (size_t(1) << 20) || largest <= (size_t(16) << 20);
-    return M < (size_t(1) << 17) || largest <= (size_t(8) << 20);
+    // 12 and 16 levels: 0.3 to 0.7 and 0.5 to 0.9; of more than 8 MB, 2^15 points 0.65 and 0.97, 2^16 0.89 and 1.34. 8 levels 0.8 and 1.0 to 1.1.
+    if (L > 10 && M < (size_t(1) << 15)) return width >= 32 && (M < 24000 || (F <= 2 && largest <= 8 * MB));
+    // Twice an XCD's L2 and more: 16 levels, 2^17 points 0.79 and 1.42, 2^20 0.92 and 1.37 (2^22 entries, 2^21 points 1473 / 1424 and 465 / 725); 8 levels 1.3 and 0.8 (2^18).
+    if (largest > (width == 16 ? 1 : 8) * MB) return false;
+    // Two features: 0.3 to 0.8 and 0.2 to 0.9. Four and eight: 6 levels 2^18 points 0.8 to 1.0 and 0.6, 8 levels 1.0 and 0.9, 2^19 1.1 and 1.4.
+    if (M >= (size_t(1) << 18)) return F <= 2 || (L <= 6 && M < (size_t(1) << 19)) || (L * F <= 16 && largest <= MB);
+    // Between: 16 levels 0.5 and 0.9 (2^15 to 2^16 points 0.6 and 1.0). 8 levels, width 64: 2^15 points 0.7 and 1.1, 2^16 0.6 and 0.9; 4 levels 0.84 and 0.76, 2 levels 2^17 0.65. Four features
+    // 0.55 and 1.1 to 1.8; width 32, 4 levels 2^16 points 1.15, width 16, 8 levels 0.7 and 1.3.
+    if (F > 2 || width < 32) return false;
+    return L > 10 || (width == 64 && M >= (size_t(1) << (L > 2 ? 16 : 17)));
 }
+
+TNN_API int tnn_grid_mlp_width_wants_levels(const tnn_grid_desc *grid, int width, size_t M) { return !check_grid_desc(grid) && M != 0 && levels_pay(grid, width, M); }
+
+TNN_API int tnn_grid_mlp_wants_levels(const tnn_grid_desc *grid, size_t M) { return tnn_grid_mlp_width_wants_levels(grid, 64, M); }
 
 TNN_API int tnn_grid_mlp_forward_levels(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_src_packed, int unpadded_input_width,
                                         int unpadded_output_width, int use_bias, void *d_packed_T, void *d_packed_transposed_T, void *d_prepared_fwd,

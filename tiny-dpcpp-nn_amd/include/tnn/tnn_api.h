@@ -676,7 +676,7 @@ template <typename T, int WIDTH> class NetworkModule : public Module {
         const int64_t rows = positions.size(0), n_out = visible_columns();
         torch::Tensor y = fresh({rows, n_out}, kType);
         torch::Tensor levels, order;
-        if (keep || tnn_grid_mlp_wants_levels(grid, (size_t)rows)) levels = this->scratch_or_none(tnn_grid_levels_bytes(grid, (size_t)rows));
+        if (keep || tnn_grid_mlp_width_wants_levels(grid, WIDTH, (size_t)rows)) levels = this->scratch_or_none(tnn_grid_levels_bytes(grid, (size_t)rows));
         if (!levels.defined()) { // (or where memory is short: a backward pass then forms them again)
             network_.inference_with_grid_rows(*grid, encoding.grid_table(), positions.data_ptr<float>(), (size_t)rows, y.data_ptr(), (int)n_out, pushed);
             return y;

@@ -105,6 +105,7 @@ SIGNATURES = {
                                            c_float, c_void_p, c_int, c_void_p, c_int, c_size_t, c_void_p, c_size_t, c_void_p]),
     "tnn_grid_levels_bytes": (c_size_t, [POINTER(GridDesc), c_size_t]),
     "tnn_grid_mlp_wants_levels": (c_int, [POINTER(GridDesc), c_size_t]),
+    "tnn_grid_mlp_width_wants_levels": (c_int, [POINTER(GridDesc), c_int, c_size_t]),
     "tnn_grid_mlp_forward_levels": (c_int, [POINTER(GridDesc), POINTER(MlpDesc), c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                             c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_size_t, c_void_p]),
     "tnn_grid_mlp_backward_levels_rows": (c_int, [POINTER(GridDesc), POINTER(MlpDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_float,
