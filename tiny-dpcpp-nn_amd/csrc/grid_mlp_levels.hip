@@ -125,7 +125,8 @@ TNN_API size_t tnn_grid_levels_bytes(const tnn_grid_desc *grid, size_t M) {
 static bool levels_pay(const tnn_grid_desc *grid, int width, size_t M) {
     const uint32_t D = grid->n_dims, L = grid->n_levels, F = grid->n_features_per_level;
     const size_t largest = largest_level_bytes(grid), MB = size_t(1) << 20;
-    // A tile of so many levels in one kernel does not fit its registers: 3-D, width 128, two features 0.05 to 0.23 of its time by levels, width 64, one feature 0.3.
+    // The constants of so many levels do not fit one kernel's scalar registers: 3-D, width 128, two features 25 000 of its 100 000 instructions read and write lanes for them, and by levels
+    // takes 0.05 to 0.23 of its time; width 64, one feature 5 000 of 33 000, 0.3.
     if (width == 128 && F <= (D == 3 ? 2u : 1u)) return true;
     if (width == 64 && F == 1 && D == 3) return true;
     if (D == 2) {
