@@ -397,7 +397,8 @@ size_t tnn::largest_level_bytes(const tnn_grid_desc *desc) {
 // after another's, 0.7 us each in two dimensions and 1.4 in three where lines come from L2, up to 2.6 where they do not, as long as a CU's waves hold the batch
 // (2^16 points), and puts points in cell order from 2^18 on. Points of a picture's rows share lines as they walk nearly as well as by levels (16 levels of 2^19 entries,
 // us, walking / by levels: 2-D, 2^15 points 15 / 15, 2^17 25 / 30, 2^18 55 / 45; 3-D, 2^15 31 / 17, 2^17 38 / 37, 2^20 192 / 275, scattered 569 / 353); which they are is not
-// known here, and an encoding on its own stands in front of a model whose points are scattered. Drawn for such points (fp32, two features unless said otherwise):
+// known here, and an encoding on its own stands in front of a model whose points are scattered. Drawn for such points (16028 configurations: 0.83 of the walking kernel's time on average,
+// 1 % more than a tenth longer; rows 0.96, 18 %) (fp32, two features unless said otherwise):
 static bool levels_pay(const tnn_grid_desc *desc, size_t M) {
     const uint32_t L = desc->n_levels, F = desc->n_features_per_level;
     const size_t largest = tnn::largest_level_bytes(desc);
