@@ -198,10 +198,11 @@ __device__ __forceinline__ long long load_point(const float *__restrict__ xin, c
     return i;
 }
 
-// Gradient contributions of one point to one level: visits (entry index, weight) of every corner.
+// Gradient contributions of one point to one level: visits (entry index, weight) of every corner. Bit d of `turn` has the corners
+// of dimension d visited far side first: lanes whose points share a cell then add to different entries in one instruction.
 template <int D, typename Fn>
 __device__ __forceinline__ void for_each_corner(const float (&x)[D], float scale, uint32_t size, uint32_t res, uint32_t flags,
-                                                uint32_t hash_type, uint32_t interpolation, Fn &&fn) {
+                                                uint32_t hash_type, uint32_t interpolation, uint32_t turn, Fn &&fn) {
     uint32_t cell[D];
     float frac[D];
     cell_of<D>(x, scale, interpolation, cell, frac);
@@ -209,19 +210,24 @@ __device__ __forceinline__ void for_each_corner(const float (&x)[D], float scale
         fn(level_index<D>(cell, size, res, flags, hash_type), 1.0f);
         return;
     }
+    float side_weight[D][2];
+    uint32_t side[D][2];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        const uint32_t far = (turn >> d) & 1;
+        side_weight[d][0] = far ? frac[d] : 1 - frac[d];
+        side_weight[d][1] = far ? 1 - frac[d] : frac[d];
+        side[d][0] = cell[d] + far;
+        side[d][1] = cell[d] + 1 - far;
+    }
 #pragma unroll
     for (int c = 0; c < (1 << D); ++c) {
         float weight = 1.0f;
         uint32_t loc[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            if ((c & (1 << d)) == 0) {
-                weight *= 1 - frac[d];
-                loc[d] = cell[d];
-            } else {
-                weight *= frac[d];
-                loc[d] = cell[d] + 1;
-            }
+            weight *= side_weight[d][(c >> d) & 1];
+            loc[d] = side[d][(c >> d) & 1];
         }
         fn(level_index<D>(loc, size, res, flags, hash_type), weight);
     }
@@ -305,7 +311,7 @@ __global__ void __launch_bounds__(kBwdThreads)
         __syncthreads();
         const long long first = (long long)(lds_block % bp.small_blocks) * bp.chunk;
         const long long last = first + bp.chunk < M ? first + bp.chunk : M;
-        // In cell order the lanes of a wave take points a stripe apart, as below: neighbours would queue up on one LDS address.
+        // In cell order the lanes of a wave take points a stripe apart: neighbours would queue up on one LDS address.
         const uint32_t wave_no = threadIdx.x / kGridWave, lane = threadIdx.x % kGridWave;
         const uint32_t start = order ? lane * (bp.chunk / kGridWave) + wave_no : threadIdx.x;
         const uint32_t step = order ? kBwdThreads / kGridWave : kBwdThreads, turns = bp.chunk / kBwdThreads;
@@ -319,10 +325,10 @@ __global__ void __launch_bounds__(kBwdThreads)
 #pragma unroll
             for (int f = 0; f < F; ++f)
                 if (f < (int)n_f) gy[f] = (float)dy[f] * dl.scale;
-            for_each_corner<D>(x, scale, size, res, flags, gp.hash_type, gp.interpolation, [&](uint32_t idx, float w) {
+            for_each_corner<D>(x, scale, size, res, flags, gp.hash_type, gp.interpolation, lane, [&](uint32_t idx, float w) {
 #pragma unroll
                 for (int f = 0; f < F; ++f)
-                    if (f < (int)n_f) lds_add(&priv[idx * n_f + f], w * gy[f]);
+                    if (f < (int)n_f) lds_add(&priv[f * size + idx], w * gy[f]);
             });
         }
         __syncthreads();
@@ -330,7 +336,7 @@ __global__ void __launch_bounds__(kBwdThreads)
         if constexpr (std::is_same<GT, float>::value) {
             // neighbouring lanes take neighbouring values, so that the values of a 32-byte sector leave in one request
             for (uint32_t e = threadIdx.x; e < size * n_f; e += kBwdThreads) {
-                const float v = (float)priv[e];
+                const float v = (float)priv[n_f == F ? e % F * size + e / F : e];
                 if (v != 0.0f) unsafeAtomicAdd(g + (n_f == F ? e : (size_t)e * F), v);
             }
         } else {
@@ -339,7 +345,7 @@ __global__ void __launch_bounds__(kBwdThreads)
                 bool any = false;
 #pragma unroll
                 for (int f = 0; f < F; ++f) {
-                    v[f] = (float)priv[e * F + f];
+                    v[f] = (float)priv[f * size + e];
                     any |= v[f] != 0.0f;
                 }
                 if (any) add_entry<F>(g + (size_t)e * F, v);
@@ -364,8 +370,9 @@ __global__ void __launch_bounds__(kBwdThreads)
         const float scale = lv.scale[l];
         const long long row_first = bin_start[rowno * bp.bins_per_row];
         const long long row_end = rowno + 1 < bp.n_rows ? (long long)bin_start[(rowno + 1) * bp.bins_per_row] : M;
-        // lane L of wave w takes the points L * stripe + w + n_waves * k of the stretch: the lanes of an instruction are a
-        // stripe apart and rarely in the same cell, where consecutive points would queue up on one LDS address
+        // Eight neighbouring lanes take eight consecutive points, which share lines of the records and of dL/dy and lie in few cells, so that they
+        // take the cell's corners each in another order; the next eight lanes are an eighth of the stretch further, in other cells
+        // (2-D, 2^18 points: eight 35.3 us, one 36.4, 64 39.4; corners in the same order and one lane 40.7; 3-D, 2^20 points 151, 151, 149 and 165).
         constexpr uint32_t n_waves = kBwdThreads / kGridWave;
         const uint32_t stripe = chunk / kGridWave, wv = threadIdx.x / kGridWave, ln = threadIdx.x % kGridWave;
         GT *g = grad + (size_t)lv.offset[l] * F;
@@ -395,7 +402,7 @@ __global__ void __launch_bounds__(kBwdThreads)
                 __syncthreads();
             }
             for (uint32_t k = wv; k < stripe; k += n_waves) {
-                const uint32_t pl = ln * stripe + k;
+                const uint32_t pl = (ln / 8) * (stripe * 8) + k * 8 + ln % 8;
                 if (pl >= count) continue;
                 float x[D];
                 const long long row = load_point<D>(xin, order, first + pl, x);
@@ -409,22 +416,32 @@ __global__ void __launch_bounds__(kBwdThreads)
                 bool inside = fits;
 #pragma unroll
                 for (int d = 0; d < D; ++d) inside &= (uint32_t)((int)cell[d] - lo[d]) < ext[d] - 1;
+                float side_weight[D][2];
+                uint32_t side[D][2], place[D][2], stride = 1;
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    const uint32_t far = (ln >> d) & 1; // (as for_each_corner)
+                    side_weight[d][0] = far ? frac[d] : 1 - frac[d];
+                    side_weight[d][1] = far ? 1 - frac[d] : frac[d];
+                    side[d][0] = cell[d] + far;
+                    side[d][1] = cell[d] + 1 - far;
+                    place[d][0] = (uint32_t)((int)side[d][0] - lo[d]) * stride;
+                    place[d][1] = (uint32_t)((int)side[d][1] - lo[d]) * stride;
+                    stride *= ext[d];
+                }
 #pragma unroll
                 for (int c = 0; c < (1 << D); ++c) {
                     float weight = 1.0f;
-                    uint32_t loc[D];
-                    uint32_t local = 0, stride = 1;
+                    uint32_t loc[D], local = 0;
 #pragma unroll
                     for (int d = 0; d < D; ++d) {
-                        const bool far = (c & (1 << d)) != 0;
-                        weight *= far ? frac[d] : 1 - frac[d]; // the products of for_each_corner
-                        loc[d] = far ? cell[d] + 1 : cell[d];
-                        local += (uint32_t)((int)loc[d] - lo[d]) * stride;
-                        stride *= ext[d];
+                        weight *= side_weight[d][(c >> d) & 1];
+                        loc[d] = side[d][(c >> d) & 1];
+                        local += place[d][(c >> d) & 1];
                     }
                     if (inside) {
 #pragma unroll
-                        for (int f = 0; f < F; ++f) lds_add(&priv[local * F + f], weight * gy[f]);
+                        for (int f = 0; f < F; ++f) lds_add(&priv[f * (uint32_t)n_local + local], weight * gy[f]);
                     } else {
                         float v[F];
 #pragma unroll
@@ -442,7 +459,7 @@ __global__ void __launch_bounds__(kBwdThreads)
                 bool any = false;
 #pragma unroll
                 for (uint32_t f = 0; f < F / VL; ++f) {
-                    v[f] = (float)priv[n * (F / VL) + f];
+                    v[f] = (float)priv[(n % VL + f) * (uint32_t)n_local + e];
                     any |= v[f] != 0.0f;
                 }
                 if (!any) continue;
