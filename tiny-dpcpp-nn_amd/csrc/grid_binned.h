@@ -17,6 +17,7 @@ struct BinPlan {
     uint8_t run_log2[kMaxBinned];
     uint16_t places[kMaxBinned];       // entries a bin has room for
     uint32_t first_bin[kMaxBinned + 1]; // bins of the levels in front of this one
+    uint32_t first_quad[kMaxBinned + 1]; // the same in fours of bins
     uint32_t slice_lds;                // LDS bytes of the largest slice
     uint32_t batch;                    // points binned at a time
 };
