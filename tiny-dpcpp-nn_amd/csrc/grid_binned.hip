@@ -30,6 +30,7 @@ namespace tnn {
 constexpr int kBinSumThreads = 1024; // at most
 constexpr uint32_t kBinSumGroup = 8;    // lanes that walk through a share of a bin's records together
 constexpr int kBinPiecesEach = 4;        // pieces a thread of the sums looks up, at most
+constexpr size_t kBinBatch = size_t(1) << 19; // points binned at a time, at most
 constexpr uint32_t kBinNeighbours = 16;  // consecutive bins on an XCD
 constexpr uint32_t kBinPiecePad = 144; // records between two pieces, so that workgroups in step do not all write to the same channels
 
@@ -361,14 +362,17 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
     if ((M << (n_dims - 1)) < size / 16) return false;
     // 128 bins a level: a workgroup's share of a bin is then a run of several lines, and the bins of all levels are enough
     // workgroups for the sums. 256 where 128 would take more than 32 KB of LDS each, so that four workgroups share a CU while some wait
-    // for their first records (2-D, 2^18 points: 29 -> 27 us; 3-D, 2^16: 48 -> 40, 2^19: 182 either way; four features 262 -> 236). Small
+    // for their first records (2-D, 2^18 points: 29 -> 27 us; 3-D, 2^16: 48 -> 40; four features, 2^19 262 -> 236); but up to 64 KB, two workgroups of
+    // 1024 threads, where a bin of 256 would still hold 8192 records, whose runs then share half as many lines with other bins' (256 and 128
+    // bins: 3-D, 2^19 points 119, 108; 2^18 89, 88; 2^17 51, 57; 2-D, 2^19 66, 67; 2^18 22, 27). Small
     // levels have fewer, large ones as many as it takes for a bin to fit LDS.
-    uint32_t n_log2 = (size >> 7) * entry > 32 * 1024 ? 8 : 7;
+    const bool long_bins = (std::min<size_t>(M, kBinBatch) << (n_dims - 1)) >> 8 >= 8192;
+    uint32_t n_log2 = (size >> 7) * entry > (long_bins ? 64 : 32) * 1024 ? 8 : 7;
     while (n_log2 > 0 && (size >> (n_log2 + 4)) == 0) --n_log2;
     while (n_log2 < 31 && ((size >> n_log2) * entry > kBinSliceBytes || (size >> n_log2) > 0x7fff)) ++n_log2;
     const size_t bins = (size_t)1 << n_log2;
     if (bins > kBinMaxBins) return false;
-    p->batch = (uint32_t)std::min<size_t>(M, size_t(1) << 19);
+    p->batch = (uint32_t)std::min<size_t>(M, kBinBatch);
     // A hashed level deals out groups of cells that share a run of x and all of the other coordinates, at random: runs as long as
     // leaves a bin 64 groups, down to 16 entries (a line of two features). A dense level deals out runs of that length: points that
     // crowd a region of it then still meet all of its bins. (Other hashes than the coherent one send every corner by itself,
