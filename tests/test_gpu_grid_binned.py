@@ -30,7 +30,8 @@ def binned(tnn, d, x, g, dtype, ordered=False, grad=None, overwrite=True, short=
 
 @pytest.mark.parametrize("cfg", [CFG2, CFG3, dict(CFG3, log2_hashmap_size=22, n_levels=12), dict(CFG2, n_features_per_level=1, hash="Prime"),
                                  dict(CFG3, n_features_per_level=4, n_levels=8, interpolation="Smoothstep"), dict(CFG2, n_features_per_level=8, n_levels=7),
-                                 dict(CFG3, interpolation="Nearest"), dict(CFG2, grid_type="Dense", n_levels=9), dict(CFG2, grid_type="Tiled")])
+                                 dict(CFG3, interpolation="Nearest"), dict(CFG2, grid_type="Dense", n_levels=9), dict(CFG2, grid_type="Tiled"),
+                                 dict(CFG2, n_levels=34, per_level_scale=1.2)])
 @pytest.mark.parametrize("M,ordered,kind", [(1, False, "uniform"), (513, False, "uniform"), (40007, True, "uniform"), (40007, False, "few"), (2 ** 19 + 9, False, "uniform")])
 def test_binned_scatter_matches_the_oracle(tnn, oracle, cfg, M, ordered, kind):
     """Bins of very different lengths ("few": all points on some twenty cells), a batch of more than one part, edges of bins, every kind of level. fp32 sums

@@ -606,33 +606,48 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
     BackwardPlan bp{};
     bp.chunk = kPrivateChunk;
     bp.budget = ordered ? kPrivateLdsBytesOrdered : kPrivateLdsBytes;
-    const size_t per_chunk = (M < bp.chunk ? M : (size_t)bp.chunk) << (gp.interpolation == TNN_INTERP_NEAREST ? 0 : D);
+    const bool nearest = gp.interpolation == TNN_INTERP_NEAREST;
+    const size_t per_chunk = (M < bp.chunk ? M : (size_t)bp.chunk) << (nearest ? 0 : D);
     uint32_t n_big = 0, lds_bytes = 0;
-    for (uint32_t l = 0; l < gp.n_levels; ++l) {
-        const size_t feature_bytes = (size_t)lv.size[l] * sizeof(double), bytes = feature_bytes * F;
-        // (in cell order only the coarsest levels: the box of a stretch is far smaller than a level from 8 KiB on)
-        const bool worth_it = per_chunk >= 2 * (size_t)lv.size[l];
-        if (worth_it && bytes <= (ordered ? 16384u : bp.budget)) {
-            bp.small_feature[bp.n_small] = kAllFeatures;
-            bp.small_level[bp.n_small++] = (uint8_t)l;
-            if (bytes > lds_bytes) lds_bytes = (uint32_t)bytes;
-        } else if (worth_it && !ordered && fp32_table && F == 2 && feature_bytes <= bp.budget && bp.n_small + 2 <= TNN_GRID_MAX_LEVELS) {
-            for (uint32_t f = 0; f < F; ++f) {
-                bp.small_feature[bp.n_small] = (uint8_t)f;
+    const auto divide = [&](size_t contributions, size_t an_entry) {
+        bp.n_small = n_big = lds_bytes = 0;
+        for (uint32_t l = 0; l < gp.n_levels; ++l) {
+            const size_t feature_bytes = (size_t)lv.size[l] * sizeof(double), bytes = feature_bytes * F;
+            // (in cell order only the coarsest levels: the box of a stretch is far smaller than a level from 8 KiB on)
+            const bool worth_it = per_chunk >= 2 * (size_t)lv.size[l] && contributions >= an_entry * (size_t)lv.size[l];
+            if (worth_it && bytes <= (ordered ? 16384u : bp.budget)) {
+                bp.small_feature[bp.n_small] = kAllFeatures;
                 bp.small_level[bp.n_small++] = (uint8_t)l;
+                if (bytes > lds_bytes) lds_bytes = (uint32_t)bytes;
+            } else if (worth_it && !ordered && fp32_table && F == 2 && feature_bytes <= bp.budget && bp.n_small + 2 <= TNN_GRID_MAX_LEVELS) {
+                for (uint32_t f = 0; f < F; ++f) {
+                    bp.small_feature[bp.n_small] = (uint8_t)f;
+                    bp.small_level[bp.n_small++] = (uint8_t)l;
+                }
+                if (feature_bytes > lds_bytes) lds_bytes = (uint32_t)feature_bytes;
+            } else {
+                bp.big_level[n_big++] = (uint8_t)l;
             }
-            if (feature_bytes > lds_bytes) lds_bytes = (uint32_t)feature_bytes;
-        } else {
-            bp.big_level[n_big++] = (uint8_t)l;
         }
-    }
+    };
+    // Binned from where the atomics it saves (one request per pair of corners, 20e9 a second) take longer than its two launches:
+    // 2^18 requests. (2-D, 11 such levels, 12 000 points: 20 us either way; 2^16 points: 42 against 95.)
+    const auto enough_to_bin = [&] { return bins && ((unsigned long long)M * n_big << (D - 1)) >= (1ull << 18); };
+    divide(0, 0);
+    // Beside binned levels a copy of the whole level has to be worth its additions to the table, for the chunks of 1024 points that a batch is cut into
+    // in the end: a level of more entries than a chunk has contributions is binned, too (whole scatter, 2-D, 2^16 points, 2^15 entries 37.8 -> 32.9 us; 2^18
+    // 81 -> 77; 2^15 points, 2^19 entries 39.3 either way), and in three dimensions, where that leaves none as a rule and so a launch less, one of more than
+    // a quarter as many (20 000 points 52 -> 42.5; 2^16 63.5 -> 54.5; 2^17 93 -> 94, and its records take memory: not from there on; with that rule in two
+    // dimensions 2^16 points 35.9).
+    if (!ordered && !nearest && enough_to_bin() && gp.n_levels <= kMaxBinned)
+        divide(std::min<size_t>(M, 1024) << D, D == 2 || M >= (size_t(1) << 17) ? 1 : 4);
     // Cell order: of the other levels, those where a stretch of consecutive points of one row of the order's coarse cells
     // fills a box of the level's cells that fits the LDS budget take the boxed route, as long as the level has a point for
     // every few cells (beyond that a box holds hardly more than one contribution per entry and saves no atomics). The order
     // (grid_order.hip) walks a lattice of 64^2 (16^3) coarse cells row by row, x fastest: with the points spread evenly a
     // row holds M / 64 (M / 256) of them, and a stretch of C of these spans that share of the level's width plus a coarse
     // cell, and one coarse cell in the other dimensions. A stretch that breaks the estimate is caught in the kernel.
-    if (ordered && gp.n_levels > 0 && gp.interpolation != TNN_INTERP_NEAREST) {
+    if (ordered && gp.n_levels > 0 && !nearest) {
         bp.bins_per_row = (D == 2) ? 64 : 16;
         bp.n_rows = 4096 / bp.bins_per_row;
         const double per_row = (double)M / bp.n_rows, coarse = (double)bp.bins_per_row;
@@ -666,10 +681,8 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
     // (few workgroups of the LDS route leave most of the chip idle: shorter ones then)
     while (bp.chunk > 1024 && (M / bp.chunk) * bp.n_small < 256) bp.chunk /= 2;
     bp.small_blocks = (uint32_t)((M + bp.chunk - 1) / bp.chunk);
-    // Binned from where the atomics it saves (one request per pair of corners, 20e9 a second) take longer than its two launches:
-    // 2^18 requests. (2-D, 11 such levels, 12 000 points: 20 us either way; 2^16 points: 42 against 95.)
     if (bins) *bins = BinPlan{};
-    if (bins && ((unsigned long long)M * n_big << (D - 1)) >= (1ull << 18)) {
+    if (enough_to_bin()) {
         uint32_t kept = 0;
         for (uint32_t i = 0; i < n_big; ++i)
             if (!bin_plan_add(bins, bp.big_level[i], lv, gp, n_dims, F, M)) bp.big_level[kept++] = bp.big_level[i];
