@@ -715,14 +715,14 @@ static int launch_backward128(const tnn_mlp_desc *d, const void *wprep_bwd, cons
     const bool reform = targets && wprep_fwd;
     auto k_top = reform ? mlp_layer_backward128_kernel<T, 3> : (targets ? mlp_layer_backward128_kernel<T, 2> : mlp_layer_backward128_kernel<T, 1>);
     auto k_mid = mlp_layer_backward128_kernel<T, 0>;
-    auto k_pair = mlp_layer_pair_backward128_kernel<T>;
+    auto k_pairs = mlp_layer_pairs_backward128_kernel<T>;
     const float inv_n = 1.0f / (float)(M * W);
     const size_t top_lds = reform ? LayerBwd128::pair_lds_bytes : LayerBwd128::lds_bytes;
     if (!reserve_lds(reinterpret_cast<const void *>(k_top), top_lds))
         return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", top_lds);
     if (!reserve_lds(reinterpret_cast<const void *>(k_mid), LayerBwd128::lds_bytes))
         return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", LayerBwd128::lds_bytes);
-    if (!reserve_lds(reinterpret_cast<const void *>(k_pair), LayerBwd128::pair_lds_bytes))
+    if (!reserve_lds(reinterpret_cast<const void *>(k_pairs), LayerBwd128::pair_lds_bytes))
         return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", LayerBwd128::pair_lds_bytes);
     const T *fwd = static_cast<const T *>(interm_fwd);
     const T *input0 = x0 ? static_cast<const T *>(x0) : fwd; // the first matrix's input: the caller's x, or its copy in front of the activations
@@ -732,20 +732,17 @@ static int launch_backward128(const tnn_mlp_desc *d, const void *wprep_bwd, cons
                                ? reinterpret_cast<float *>(dl + (size_t)(n_mats - 1) * mat) : (float *)nullptr;
     if (targets && loss_sum && !loss_partials) return fail(TNN_ERR_INVALID_ARGUMENT, "no room for the loss sums of %lld workgroups", p.n_chunks);
     const vec8 *wb = static_cast<const vec8 *>(wprep_bwd);
-    // the top layer by itself (it turns dL/dy or the loss into deltas first), then the layers below it two per launch, and
+    // the top layer by itself (it turns dL/dy or the loss into deltas first), then the layers below it two at a time in one launch, and
     // the first matrix by itself when their number is odd
     int l = n_mats - 1;
     while (l >= 0) {
         const bool top = (l == n_mats - 1);
         if (!top && l >= 1) {
-            T *delta_out = l > 1 ? dl + (size_t)(l - 2) * mat : static_cast<T *>(dLdx);
-            TNN_LAUNCH(k_pair, dim3((unsigned)p.n_chunks), dim3(kLayerBwdThreads), LayerBwd128::pair_lds_bytes, s, wb + (size_t)l * per_mat,
-                       wb + (size_t)(l - 1) * per_mat, dl + (size_t)l * mat, fwd + (size_t)l * mat, l > 1 ? fwd + (size_t)(l - 1) * mat : input0,
-                       keep_top_delta ? dl + (size_t)(l - 1) * mat : (T *)nullptr, delta_out, partials, n_mats, l, d->activation,
-                       l > 1 ? d->activation : TNN_ACT_NONE, l > 1 ? 1.0f : tail.result_scale, (long long)M, p.rows_per_chunk);
-            const int rc = check_launch("mlp_layer_pair_backward128_kernel");
+            TNN_LAUNCH(k_pairs, dim3((unsigned)p.n_chunks), dim3(kLayerBwdThreads), LayerBwd128::pair_lds_bytes, s, wb, dl, fwd, input0, static_cast<T *>(dLdx),
+                       keep_top_delta ? 1 : 0, partials, n_mats, l, d->activation, tail.result_scale, (long long)M, p.rows_per_chunk);
+            const int rc = check_launch("mlp_layer_pairs_backward128_kernel");
             if (rc) return rc;
-            l -= 2;
+            l = (l & 1) ? -1 : 0;
             continue;
         }
         const T *delta_in = top ? static_cast<const T *>(dLdy) : dl + (size_t)l * mat;
