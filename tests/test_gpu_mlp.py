@@ -156,6 +156,31 @@ def test_backward_parity_widths(tnn, oracle, dtype, W, n_hidden):
     assert max_norm_rel(tnn.host(dX), dX64) < 1e-2
 
 
+@pytest.mark.parametrize("dtype,n_hidden,M", [(FP16, 1, 8), (BF16, 2, 8), (FP16, 4, 72), (BF16, 5, 200), (FP16, 8, 264), (BF16, 3, 8192 + 40), (FP16, 2, 16384 + 72)])
+def test_width_128_backward_of_few_rows(tnn, oracle, dtype, n_hidden, M):
+    """All pairs of layers in one launch, with the bottom layer in a pair or alone (an odd number of hidden layers leaves an odd
+    number below the top one), workgroups of 64 and 128 rows, rounds that end in the middle of a wave's tile and waves without rows. With the
+    deltas kept and without: the same weight gradients, which are a plain product of the kept deltas and the activations."""
+    W, n_mats = 128, n_hidden + 1
+    ls = 128.0 if dtype == FP16 else 1.0
+    w, x = make_case(oracle, dtype, W, n_mats, M, seed=13)
+    g = oracle.round(np.random.default_rng(8).uniform(-1, 1, (M, W)) * ls / M, dtype)
+    desc = tnn.mlp_desc(dtype, W, n_hidden, "relu", "none")
+    _, pf, pb = tnn.prepare(desc, w)
+    interm_t = tnn.forward(desc, pf, tnn.dev_tensor(x, dtype))
+    interm = tnn.host(interm_t)
+    rib, rdW, rdX = oracle.mlp_backward_T(dtype, W, n_mats, "relu", "none", w, interm, g, round_dw=False)
+    ib, dW, dX = tnn.backward(desc, pb, tnn.dev_tensor(g, dtype), interm_t, dw_fp32=True)
+    _, dW2, _ = tnn.backward(desc, pb, tnn.dev_tensor(g, dtype), interm_t, want_interm=False, want_dx=False, dw_fp32=True)
+    assert np.array_equal(tnn.host(dW), tnn.host(dW2))
+    gib = tnn.host(ib)
+    for l in range(n_mats):
+        assert_propagated(gib[l], rib[l], dtype, f"delta[{l}]", scale=ls / M)
+        assert_close(tnn.host(dW[l]), gib[l].astype(np.float64).T @ interm[l].astype(np.float64), dtype, f"dW[{l}] from the GPU's own deltas", scale=ls)
+    assert_propagated(tnn.host(dX), rdX, dtype, "dL/dx", scale=ls / M)
+    assert_propagated(tnn.host(dW), rdW, dtype, "dW", scale=ls)
+
+
 def test_closed_forms(tnn, oracle):
     # test/doctest_swiftnet.cpp:44-51,79-96 : constant weights 0.01 with padded input / output
     dtype, W, n_hidden, M = BF16, 64, 2, 16

@@ -675,8 +675,11 @@ static DwPlan dw_plan(const tnn_mlp_desc *d, size_t M) {
     const int W = d->width, n_mats = d->n_hidden_layers + 1;
     long long target_chunks = 256;
     long long rpc = ((long long)M + target_chunks - 1) / target_chunks;
-    rpc = (rpc + kDwSlab - 1) / kDwSlab * kDwSlab;
-    if (rpc < kDwSlab) rpc = kDwSlab;
+    // At width 128 a workgroup of few rows has a short round and one partial sum like any other: 128 rows at least where 64 would be half of the chip's workgroups and more
+    // (steps of 8 hidden layers, us, chunks in multiples of 64, 128, 256: 1024 rows 84, 89, 106; 4096 88, 93, 110; 8192 100, 97, 112; 16384 113, 107, 116; 2^15 and more the same).
+    const long long slab = W == 128 && M >= 8192 ? 2 * kDwSlab : kDwSlab;
+    rpc = (rpc + slab - 1) / slab * slab;
+    if (rpc < slab) rpc = slab;
     p.rows_per_chunk = rpc;
     p.n_chunks = M ? ((long long)M + rpc - 1) / rpc : 0;
     p.partials_per_chunk = (W <= 32) ? 4 : 1;
