@@ -169,3 +169,18 @@ def test_binned_workspace_is_checked(tnn):
     with pytest.raises(_lib.TnnError):
         binned(tnn, d, x, torch.rand((40960, 32), device=tnn.dev), FP32, short=4096)
     assert tnn.lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), 0) == 0
+
+
+@pytest.mark.parametrize("M", [28001, 32003, 60001, 64007, 80009])
+@pytest.mark.parametrize("features", [1, 2, 8])
+def test_sums_with_few_and_many_records_a_lane(tnn, oracle, M, features):
+    """Two to six rounds of records of an even spread, which choose how many a lane has in flight; several bins a workgroup, whose sums start from zero for each; and
+    levels whose last entries fill a bin's last pair or not. fp32 results of double sums: the bar of the plain scatter."""
+    cfg = dict(CFG2, n_features_per_level=features, n_levels=16 if features <= 2 else 10)
+    rng = np.random.default_rng(M + features)
+    x = rng.uniform(0, 1, (M, 2)).astype(np.float32)
+    d = tnn.grid_desc(cfg)
+    g = rng.standard_normal((M, cfg["n_levels"] * features)).astype(np.float32)
+    ref = oracle.grid_backward(cfg, x, g, tnn.grid_n_params(d))
+    grad = binned(tnn, d, torch.from_numpy(x).to(tnn.dev), torch.from_numpy(g).to(tnn.dev), FP32)
+    assert np.abs(grad.cpu().numpy() - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())

@@ -853,7 +853,7 @@ namespace tnn {
 // The binned levels are written whole: where they are the last ones, as the finest are, only what lies in front of them is cleared.
 static ClearRange range_to_clear(const tnn_grid_desc *desc, const BinPlan &bins, void *d_grad_table, int grad_dtype) {
     size_t entries = desc->offsets[desc->n_levels];
-    if (bins.n_levels && bins.level[0] + bins.n_levels == desc->n_levels) entries = std::min<size_t>(entries, desc->offsets[bins.level[0]]);
+    if (bins.n_levels && bins.at[0].level + bins.n_levels == desc->n_levels) entries = std::min<size_t>(entries, bins.at[0].offset);
     const size_t bytes = entries * desc->n_features_per_level * (grad_dtype == TNN_FP32 ? sizeof(float) : sizeof(fp16_t));
     ClearRange c;
     c.p = static_cast<float4 *>(d_grad_table);
@@ -912,7 +912,7 @@ int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4
         TNN_DISPATCH_DF(desc, rc = (launch_grid_backward_g<D_, F_, float>(lv, gp, bp, dl, n_big, lds_bytes, d_x, d_order, d_dLdy, dy_dtype,
                                                                           (float *)d_grad_table, M, s)));
         if (rc == TNN_OK && bins.n_levels)
-            rc = launch_grid_binned(bins, lv, gp, dl, desc->n_dims, n_features, d_x, d_x && !dl.by_position ? nullptr : d_order, d_dLdy, dy_dtype, (float *)d_grad_table, overwrite != 0, M,
+            rc = launch_grid_binned(bins, gp, dl, desc->n_dims, n_features, d_x, d_x && !dl.by_position ? nullptr : d_order, d_dLdy, dy_dtype, (float *)d_grad_table, overwrite != 0, M,
                                     reinterpret_cast<void *>(scratch), s);
     } else {
         const uint32_t F = desc->n_features_per_level;

@@ -9,17 +9,25 @@ constexpr uint32_t kMaxBinned = 32;         // levels one launch bins
 constexpr uint32_t kBinMaxBins = 1024;      // bins of a level
 constexpr uint32_t kBinSliceBytes = 128 * 1024; // most of a bin's slice of the table (LDS of a workgroup)
 
+// All that the kernels need of a level, side by side: a workgroup has it after one scalar load.
+struct BinLevel {
+    uint32_t level;
+    uint32_t offset, size, resolution, flags; // as in GridLevels
+    float scale;
+    uint32_t bins_log2, run_log2; // the level's runs of 2^run_log2 entries go to its 2^bins_log2 bins in turn
+    uint32_t places;              // entries a bin has room for
+    uint32_t first_bin;           // bins of the levels in front of this one
+    uint32_t first_quad;          // the same in fours of bins
+};
+
 struct BinPlan {
     uint32_t n_levels;
-    uint32_t n_bins;                   // of all levels
-    uint8_t level[kMaxBinned];
-    uint8_t bins_log2[kMaxBinned];     // the level's runs of 2^run_log2 entries go to its 2^bins_log2 bins in turn
-    uint8_t run_log2[kMaxBinned];
-    uint16_t places[kMaxBinned];       // entries a bin has room for
-    uint32_t first_bin[kMaxBinned + 1]; // bins of the levels in front of this one
-    uint32_t first_quad[kMaxBinned + 1]; // the same in fours of bins
-    uint32_t slice_lds;                // LDS bytes of the largest slice
-    uint32_t batch;                    // points binned at a time
+    uint32_t n_bins;                    // of all levels
+    uint32_t n_quads;                   // the same in fours of bins
+    uint32_t slice_lds;                 // LDS bytes of the largest slice
+    uint32_t batch;                     // points binned at a time
+    uint32_t later_bin[kMaxBinned - 1]; // first bin of the second level and those behind it, ~0 where there is none
+    BinLevel at[kMaxBinned];
 };
 
 // Adds level l to the plan if it can take the route.
@@ -27,7 +35,7 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
 size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_dims, uint32_t n_features);
 // Nothing in the scratch has to be cleared. With `overwrite` every entry of the plan's levels
 // is written, whatever it held.
-int launch_grid_binned(const BinPlan &p, const GridLevels &lv, const GridParams &gp, const GradLayout &dl, uint32_t n_dims, uint32_t n_features, const float *x,
+int launch_grid_binned(const BinPlan &p, const GridParams &gp, const GradLayout &dl, uint32_t n_dims, uint32_t n_features, const float *x,
                        const float4 *order, const void *dLdy, int dy_dtype, float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s);
 
 } // namespace tnn

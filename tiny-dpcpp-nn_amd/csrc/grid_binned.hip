@@ -18,12 +18,13 @@
 // as fast for points spread evenly, but what finds no room has to go elsewhere. 2^20 points, 3-D, 2^19 entries, whole scatter, from
 // points in the inner 90 % of the cube / in a cube of 5 % of the side: the overfull bins summed from the points 4.0 / 5.8 ms, the surplus
 // added with atomics 0.76 / 36 ms, pieces 0.75 / 3.9 ms; evenly spread 0.74, 0.76 and 0.75 ms.)
-// Measured, 2^20 points, 3-D, 2^19 entries, 15 levels this way: 2 x (161 + 184) us; before, the atomics of the ten finest of these
-// levels alone took 1.5 ms.
+// Measured, 2^20 points, 3-D, 2^19 entries, the ten finest levels: 2 x (98 + 96) us; as atomics 1.5 ms.
 #include "grid_binned.h"
+#include "mlp_tile.h"
 
 #include <algorithm>
 #include <cmath>
+#include <iterator>
 
 namespace tnn {
 
@@ -106,34 +107,40 @@ __device__ __forceinline__ void pair_entries(const uint32_t (&cell)[D], uint32_t
     }
 }
 
-// What the threads of a workgroup in front of this one have, and what all have. WAVES: room in wave_sum.
-template <int WAVES> __device__ __forceinline__ uint32_t running_sum(uint32_t mine, uint32_t *__restrict__ wave_sum, uint32_t &total) {
+// The sum up to each lane of a row of 16 (DPP row_shr).
+__device__ __forceinline__ uint32_t row_sums(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
+    return v;
+}
+
+// The sum of the values of the waves in front of this one, and of all: a wave's value a lane.
+__device__ __forceinline__ uint32_t sums_in_front(const uint32_t *__restrict__ of_wave, uint32_t &total) {
+    static_assert(kBinSumThreads / 64 <= 16, "a row of 16 lanes holds the waves' values");
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t upto = row_sums(lane < blockDim.x / 64 ? of_wave[lane] : 0u);
+    total = (uint32_t)__builtin_amdgcn_readlane((int)upto, 15);
+    return wave > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)upto, (int)wave - 1) : 0u;
+}
+
+// What the threads of a workgroup in front of this one have, and what all have.
+__device__ __forceinline__ uint32_t running_sum(uint32_t mine, uint32_t *__restrict__ wave_sum, uint32_t &total) {
     // of the wave's lanes up to this one: rows of 16 lanes first (DPP row_shr), then the last lane of a row to the rows above
-    uint32_t upto = mine;
-    upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x111, 0xf, 0xf, true);
-    upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x112, 0xf, 0xf, true);
-    upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x114, 0xf, 0xf, true);
-    upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x118, 0xf, 0xf, true);
+    uint32_t upto = row_sums(mine);
     upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
     upto += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
     if ((threadIdx.x & 63) == 63) wave_sum[threadIdx.x >> 6] = upto;
     __syncthreads();
-    uint32_t before = upto - mine;
-    total = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < WAVES; ++w) {
-        const uint32_t sum = w < blockDim.x / 64 ? wave_sum[w] : 0u;
-        if (w < threadIdx.x >> 6) before += sum;
-        total += sum;
-    }
-    return before;
+    return upto - mine + sums_in_front(wave_sum, total);
 }
 
 // Where a bin's records in a piece begin and end (two 16-bit numbers): by four bins, then by pieces. A workgroup of the sums reads its bin's
 // of all pieces, eight pieces to a line that it shares with three neighbouring bins; with all bins of a piece side by side it read a
 // line for each (3-D, 2^19 points, 10 levels: 123.5 us, now 119; 2^18 in the caller's order 95, 89).
-__device__ __forceinline__ size_t run_slot(const BinPlan &bp, uint32_t k, uint32_t bin, uint32_t n_stretches, uint32_t stretch) {
-    return ((size_t)(bp.first_quad[k] + bin / 4) * n_stretches + stretch) * 4 + bin % 4;
+__device__ __forceinline__ size_t run_slot(uint32_t first_quad, uint32_t bin, uint32_t n_stretches, uint32_t stretch) {
+    return ((size_t)(first_quad + bin / 4) * n_stretches + stretch) * 4 + bin % 4;
 }
 
 // One workgroup bins kPoints points a thread of one level: it counts its records per bin, which gives every record its place among
@@ -145,7 +152,7 @@ __device__ __forceinline__ size_t run_slot(const BinPlan &bp, uint32_t k, uint32
 // fill reaches 6.9; the vector units are at work half of the time, LDS a quarter, and a wave waits for 43 % of its.
 template <int D, int F, typename G>
 __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
-    grid_bin_kernel(const GridLevels lv, const GridParams gp, const BinPlan bp, const GradLayout dl, const float *__restrict__ xin,
+    grid_bin_kernel(const GridParams gp, const BinPlan bp, const GradLayout dl, const float *__restrict__ xin,
                     const float4 *__restrict__ order, const G *__restrict__ dLdy, uint32_t *__restrict__ runs, BinRecord<F> *__restrict__ records,
                     long long first, long long last, uint32_t n_stretches, uint32_t pitch, uint32_t room) {
     typedef BinShape<D, F> S;
@@ -159,12 +166,13 @@ __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
     if (stretch >= n_stretches) return;
     const long long begin = first + (long long)stretch * (T * P);
     const long long end = begin + T * P < last ? begin + T * P : last;
-    const Bins dealt{bp.bins_log2[k], bp.run_log2[k]};
-    const uint32_t l = bp.level[k], n_bins = 1u << dealt.n_log2;
+    const BinLevel at_level = bp.at[k];
+    const Bins dealt{at_level.bins_log2, at_level.run_log2};
+    const uint32_t l = at_level.level, n_bins = 1u << dealt.n_log2;
     uint32_t *const split = base + n_bins; // the same for far sides in another bin, then the place of the next of them
     uint32_t *const wave_sum = split + n_bins;
-    const uint32_t size = lv.size[l], res = lv.resolution[l], flags = lv.flags[l];
-    const float scale = lv.scale[l];
+    const uint32_t size = at_level.size, res = at_level.resolution, flags = at_level.flags;
+    const float scale = at_level.scale;
     BinRecord<F> *const piece = records + ((size_t)k * n_stretches + stretch) * pitch;
 
     for (uint32_t b = threadIdx.x; b < n_bins; b += T) base[b] = split[b] = 0;
@@ -204,7 +212,7 @@ __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
         apart[e] = any ? split[b0 + e] : 0u;
         mine += count[e] + apart[e];
     }
-    uint32_t at = running_sum<S::kThreads / 64>(mine, wave_sum, total);
+    uint32_t at = running_sum(mine, wave_sum, total);
 #pragma unroll
     for (int e = 0; e < kEach; ++e) {
         if ((uint32_t)e >= each) break;
@@ -213,7 +221,7 @@ __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
             base[b] = at;
             split[b] = at + count[e];
             const uint32_t next = at + count[e] + apart[e];
-            runs[run_slot(bp, k, b, n_stretches, stretch)] = at | (next << 16);
+            runs[run_slot(at_level.first_quad, b, n_stretches, stretch)] = at | (next << 16);
             at = next;
         }
     }
@@ -252,115 +260,161 @@ __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
     for (uint32_t i = threadIdx.x; i < staged * kWords; i += T) __builtin_nontemporal_store(from[i], to + i);
 }
 
-// One workgroup sums one bin and stores (or adds) its entries, a plane of sums a feature (lds_add; interleaved 25.0 -> 22.3 us, 2-D,
-// 2^18 points). Bound by the LDS atomics, two entries of F values a record: LDS is at
-// work 72 % of the time (3-D, 2^19 points, 15 levels, 184 us; 163 with the records read and not added). The bin's runs of records in the pieces follow each other here (`first`: records in front of a piece's run);
-// sixteen lanes take an equal share of them all, whatever the runs' lengths, and walk from run to run. Neighbouring bins, whose
+// A workgroup sums a bin and stores (or adds) its entries, a plane of sums a feature (lds_add; interleaved 25.0 -> 22.3 us, 2-D,
+// 2^18 points), then the bin that lies a grid further on. The bin's runs of records in the pieces follow each other here (`first`: records in front of a
+// piece's run); eight lanes take an equal share of them all, whatever the runs' lengths, and walk from run to run. Neighbouring bins, whose
 // runs share lines, are workgroups of one XCD, sixteen at a time. kAhead: records of a lane in flight.
+// Long bins are bound by the LDS atomics, two entries of F values a record. Short ones were bound by what comes before the first record: a workgroup a
+// bin, 3-D, 2^15 points, took 30 us, 18 of them without a record read or an entry written. So a workgroup stays for several bins: where the next bin's
+// runs lie is loaded while this one's records are summed, and sums are cleared as they are read. What was left of it were instructions, eight and more waves a bin of them:
+// the prefix sums over the waves are a value a lane, a wave without pieces leaves the look-up out, and two entries leave together (3-D, 2^15 points 30 -> 20.3 us,
+// 100 003 46 -> 37.5, 2^19 101 -> 96; 2-D, 20 011 points 11.3 -> 8.2, 2^16 12.3 -> 9.7, 2^18 23.4 -> 20.8).
 template <int F, int kAhead>
-__global__ void __launch_bounds__(kBinSumThreads)
-    grid_bin_sum_kernel(const GridLevels lv, const BinPlan bp, const uint32_t *__restrict__ runs_of, const BinRecord<F> *__restrict__ records,
+__global__ void __launch_bounds__(kBinSumThreads, F <= 2 ? 8 : 4)
+    grid_bin_sum_kernel(const BinPlan bp, const uint32_t *__restrict__ runs_of, const BinRecord<F> *__restrict__ records,
                         float *__restrict__ grad, uint32_t n_stretches, uint32_t pitch, int store) {
     constexpr uint32_t kWaves = kBinSumThreads / 64, kGroup = kBinSumGroup;
-    extern __shared__ double sums[];
-    const uint32_t number = (blockIdx.x / (8 * kBinNeighbours) * 8 + blockIdx.x % 8) * kBinNeighbours + blockIdx.x / 8 % kBinNeighbours;
-    if (number >= bp.n_bins) return;
-    uint32_t k = 0;
-    while (k + 1 < bp.n_levels && number >= bp.first_bin[k + 1]) ++k;
-    const uint32_t l = bp.level[k], bin = number - bp.first_bin[k];
-    const Bins dealt{bp.bins_log2[k], bp.run_log2[k]};
-    const uint32_t size = lv.size[l];
-    const uint32_t n = bp.places[k]; // the last ones may be beyond the level
-    uint32_t *const wave_sum = reinterpret_cast<uint32_t *>(sums + n * F);
+    constexpr int kEach = kBinPiecesEach;
+    extern __shared__ __align__(16) double sums[];
+    uint32_t *const wave_sum = reinterpret_cast<uint32_t *>(sums + bp.slice_lds / sizeof(double));
     uint32_t *const wave_runs = wave_sum + kWaves;
     uint32_t *const group_run = wave_runs + kWaves;       // run that a group's first record is in
     uint32_t *const first = group_run + kBinSumThreads / kGroup; // records in front of a run
     uint32_t *const start = first + n_stretches + 1;       // place of the run's first record in the pieces, less `first`
-    const uint32_t *const runs_here = runs_of + run_slot(bp, k, bin, n_stretches, 0);
-    constexpr int kEach = kBinPiecesEach;
-    const uint32_t each = (n_stretches + blockDim.x - 1) / blockDim.x, s0 = threadIdx.x * each;
+    const uint32_t threads_log2 = 31 - __builtin_clz(blockDim.x); // (a power of two)
+    const uint32_t each = (n_stretches + blockDim.x - 1) >> threads_log2;
+    const bool has_pieces = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u) * each < n_stretches; // (a wave without any has nothing to look up and nothing to add up)
+    const auto first_piece = [&]() __attribute__((always_inline)) {
+        uint32_t s0 = threadIdx.x * each;
+        asm volatile("" : "+v"(s0)); // (what follows from it is formed where it is used: kept over the bins it spills)
+        return s0;
+    };
+    // (the grid is a multiple of 8 kBinNeighbours: a workgroup's bins grow, and are one XCD's)
+    const auto bin_of = [&](uint32_t block) { return (block / (8 * kBinNeighbours) * 8 + block % 8) * kBinNeighbours + block / 8 % kBinNeighbours; };
+    // (the list of the levels' first bins over the lanes and the level's numbers side by side: two loads, where an entry and a number at a time were
+    // waited for one after the other: 3-D, 100 003 points 46.3 -> 44.0 us)
+    const uint32_t lane = threadIdx.x & 63, later_bin = lane < kMaxBinned - 1 ? bp.later_bin[lane] : ~0u;
+    const auto level_of = [&](uint32_t number) { return (uint32_t)__popcll(__ballot(number >= later_bin)); };
     uint32_t ends[kEach]; // where the bin's records begin in the piece, and where the next bin's do
+    const auto look_up = [&](uint32_t number) __attribute__((always_inline)) {
+        const BinLevel &at_level = bp.at[level_of(number)];
+        const uint32_t *const runs_here = runs_of + run_slot(at_level.first_quad, number - at_level.first_bin, n_stretches, 0);
+        const uint32_t s0 = first_piece();
 #pragma unroll
-    for (int e = 0; e < kEach; ++e) {
-        ends[e] = (uint32_t)e < each && s0 + e < n_stretches ? runs_here[(size_t)(s0 + e) * 4] : 0u;
-    }
-    for (uint32_t e = threadIdx.x; e < n * F; e += blockDim.x) sums[e] = 0.0;
-    uint32_t count[kEach], mine = 0, run = 0, runs = 0; // runs that hold any records: in front of this thread's, in its wave
-#pragma unroll
-    for (int e = 0; e < kEach; ++e) {
-        count[e] = (ends[e] >> 16) - (ends[e] & 0xffffu);
-        mine += count[e];
-        const unsigned long long any = __ballot(count[e] != 0);
-        run += __popcll(any & ((1ull << (threadIdx.x & 63)) - 1));
-        runs += __popcll(any);
-    }
-    if ((threadIdx.x & 63) == 0) wave_runs[threadIdx.x >> 6] = runs;
-    uint32_t total, at = running_sum<kWaves>(mine, wave_sum, total), n_runs = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < kWaves; ++w) {
-        const uint32_t sum = w < blockDim.x / 64 ? wave_runs[w] : 0u;
-        if (w < threadIdx.x >> 6) run += sum;
-        n_runs += sum;
-    }
-    // (whole rounds of a group: all but the last groups then have all of their lanes at work)
-    const uint32_t share = (total + blockDim.x - 1) / blockDim.x * kGroup;
-#pragma unroll
-    for (int e = 0; e < kEach; ++e) {
-        if (count[e] == 0) continue;
-        for (uint32_t g = (at + share - 1) / share; g * share < at + count[e]; ++g) group_run[g] = run;
-        first[run] = at;
-        start[run++] = (s0 + e) * pitch + (ends[e] & 0xffffu) - at;
-        at += count[e];
-    }
-    if (threadIdx.x == 0) first[n_runs] = total;
-    __syncthreads();
-    const BinRecord<F> *const rec = records + (size_t)k * n_stretches * pitch;
-    const uint32_t group = threadIdx.x / kGroup, end = (group + 1) * share < total ? (group + 1) * share : total;
-    uint32_t i = group * share + threadIdx.x % kGroup, s = i < end ? group_run[group] : 0u;
-    for (; i < end; i += kAhead * kGroup) {
-        uint32_t at_a[kAhead];
-#pragma unroll
-        for (int a = 0; a < kAhead; ++a) {
-            // (lanes past the end walk to the last run and read its last record)
-            const uint32_t wanted = i + a * kGroup < total ? i + a * kGroup : total - 1;
-            while (wanted >= first[s + 1]) ++s; // (first[n_runs] is beyond every record)
-            at_a[a] = start[s] + wanted;
+        for (int e = 0; e < kEach; ++e) {
+            if ((uint32_t)e >= each) break;
+            ends[e] = s0 + e < n_stretches ? runs_here[(size_t)(s0 + e) * 4] : 0u;
         }
-        BinRecord<F> r[kAhead];
+    };
+    uint32_t number = bin_of(blockIdx.x);
+    if (number >= bp.n_bins) return;
+    look_up(number);
+    for (uint32_t e = threadIdx.x; e < bp.slice_lds / sizeof(double); e += blockDim.x) sums[e] = 0.0;
+    for (uint32_t block = blockIdx.x + gridDim.x;; block += gridDim.x) {
+        const uint32_t k = level_of(number);
+        const BinLevel at_level = bp.at[k];
+        const uint32_t n = at_level.places; // the last ones may be beyond the level
+        uint32_t count[kEach], begin[kEach], mine = 0, run = 0, runs = 0; // runs that hold any records: in front of this thread's, in its wave
+        if (has_pieces) {
 #pragma unroll
-        for (int a = 0; a < kAhead; ++a) r[a] = rec[at_a[a]];
-#pragma unroll
-        for (int a = 0; a < kAhead; ++a) {
-            const uint32_t where = i + a * kGroup < end ? r[a].where : 0u, near = where & 0x7fff, far = (where >> 15) & 0x7fff;
-            if (where & (1u << 30)) {
-#pragma unroll
-                for (int f = 0; f < F; ++f) lds_add(&sums[f * n + near], (1 - r[a].frac) * r[a].g[f]);
-            }
-            if (where & (1u << 31)) {
-#pragma unroll
-                for (int f = 0; f < F; ++f) lds_add(&sums[f * n + far], r[a].frac * r[a].g[f]);
+            for (int e = 0; e < kEach; ++e) {
+                if ((uint32_t)e >= each) break; // (the same for all threads)
+                begin[e] = ends[e] & 0xffffu;
+                count[e] = (ends[e] >> 16) - begin[e];
+                mine += count[e];
+                const unsigned long long any = __ballot(count[e] != 0);
+                run += __popcll(any & ((1ull << lane) - 1));
+                runs += __popcll(any);
             }
         }
-    }
-    __syncthreads();
-    float *const g = grad + (size_t)lv.offset[l] * F;
-    if (store) { // the bin's entries have no other contributions
-        typedef float entry_t __attribute__((ext_vector_type(F), aligned(F < 4 ? F * 4 : 16)));
-        for (uint32_t v = threadIdx.x; v < n; v += blockDim.x) {
-            const uint32_t e = dealt.entry(bin, v);
-            if (e >= size) continue;
-            entry_t sum;
+        if (lane == 0) wave_runs[threadIdx.x >> 6] = runs;
+        uint32_t total, n_runs, at = running_sum(mine, wave_sum, total);
+        run += sums_in_front(wave_runs, n_runs);
+        // (whole rounds of a group: all but the last groups then have all of their lanes at work)
+        const uint32_t share = ((total + blockDim.x - 1) >> threads_log2) * kGroup, s0 = first_piece();
+        if (has_pieces) {
 #pragma unroll
-            for (int f = 0; f < F; ++f) sum[f] = (float)sums[f * n + v];
-            *reinterpret_cast<entry_t *>(g + (size_t)e * F) = sum;
+            for (int e = 0; e < kEach; ++e) {
+                if ((uint32_t)e >= each) break;
+                if (count[e] == 0) continue;
+                for (uint32_t g = (at + share - 1) / share; g * share < at + count[e]; ++g) group_run[g] = run;
+                first[run] = at;
+                start[run++] = (s0 + e) * pitch + begin[e] - at;
+                at += count[e];
+            }
         }
-        return;
-    }
-    for (uint32_t v = threadIdx.x; v < n * F; v += blockDim.x) {
-        const uint32_t e = dealt.entry(bin, v / F);
-        if (e >= size) continue;
-        float *const to = g + (size_t)e * F + v % F;
-        *to += (float)sums[v % F * n + v / F];
+        if (threadIdx.x == 0) first[n_runs] = total;
+        const uint32_t next = bin_of(block);
+        if (next < bp.n_bins) look_up(next);
+        __syncthreads();
+        const BinRecord<F> *const rec = records + (size_t)k * n_stretches * pitch;
+        const uint32_t group = threadIdx.x / kGroup, end = (group + 1) * share < total ? (group + 1) * share : total;
+        uint32_t i = group * share + threadIdx.x % kGroup, s = i < end ? group_run[group] : 0u;
+        for (; i < end; i += kAhead * kGroup) {
+            uint32_t at_a[kAhead];
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                // (lanes past the end walk to the last run and read its last record)
+                const uint32_t wanted = i + a * kGroup < total ? i + a * kGroup : total - 1;
+                while (wanted >= first[s + 1]) ++s; // (first[n_runs] is beyond every record)
+                at_a[a] = start[s] + wanted;
+            }
+            BinRecord<F> r[kAhead];
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) r[a] = rec[at_a[a]];
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                const uint32_t where = i + a * kGroup < end ? r[a].where : 0u, near = where & 0x7fff, far = (where >> 15) & 0x7fff;
+                if (where & (1u << 30)) {
+#pragma unroll
+                    for (int f = 0; f < F; ++f) lds_add(&sums[f * n + near], (1 - r[a].frac) * r[a].g[f]);
+                }
+                if (where & (1u << 31)) {
+#pragma unroll
+                    for (int f = 0; f < F; ++f) lds_add(&sums[f * n + far], r[a].frac * r[a].g[f]);
+                }
+            }
+        }
+        __syncthreads();
+        const Bins dealt{at_level.bins_log2, at_level.run_log2};
+        const uint32_t bin = number - at_level.first_bin, size = at_level.size;
+        float *const g = grad + (size_t)at_level.offset * F;
+        if (store) { // the bin's entries have no other contributions
+            // Two neighbouring entries a thread: a run has an even number, a level's offset and size are multiples of 8, and the table is 16-byte aligned.
+            constexpr int kStore = 2 * F < 4 ? 2 * F : 4;
+            typedef float store_t __attribute__((ext_vector_type(kStore)));
+            typedef double pair_t __attribute__((ext_vector_type(2)));
+            for (uint32_t v = 2 * threadIdx.x; v < n; v += 2 * blockDim.x) {
+                const uint32_t e = dealt.entry(bin, v);
+                float sum[2 * F];
+#pragma unroll
+                for (int f = 0; f < F; ++f) {
+                    pair_t *const both = reinterpret_cast<pair_t *>(sums + f * n + v);
+                    const pair_t d = *both;
+                    *both = pair_t{0.0, 0.0};
+                    sum[f] = (float)d[0];
+                    sum[F + f] = (float)d[1];
+                }
+                if (e >= size) continue;
+                store_t *const to = reinterpret_cast<store_t *>(g + (size_t)e * F);
+#pragma unroll
+                for (int q = 0; q < 2 * F / kStore; ++q) {
+                    store_t w;
+#pragma unroll
+                    for (int j = 0; j < kStore; ++j) w[j] = sum[q * kStore + j];
+                    to[q] = w;
+                }
+            }
+        } else {
+            for (uint32_t v = threadIdx.x; v < n * F; v += blockDim.x) {
+                const uint32_t e = dealt.entry(bin, v / F), from = v % F * n + v / F;
+                const float sum = (float)sums[from];
+                sums[from] = 0.0;
+                if (e < size) g[(size_t)e * F + v % F] += sum;
+            }
+        }
+        if (next >= bp.n_bins) return;
+        number = next;
     }
 }
 
@@ -394,15 +448,11 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
     while (((size_t)1 << (run_log2 + n_log2)) < size && (apart || (hashed && groups(run_log2 + 1) >= 64.0))) ++run_log2;
     const size_t places = ((size + ((size_t)1 << (run_log2 + n_log2)) - 1) >> (run_log2 + n_log2)) << run_log2;
     if (places > 0x7fff || places * entry > kBinSliceBytes) return false;
-    const uint32_t k = p->n_levels++;
-    p->level[k] = (uint8_t)l;
-    p->bins_log2[k] = (uint8_t)n_log2;
-    p->run_log2[k] = (uint8_t)run_log2;
-    p->places[k] = (uint16_t)places;
-    p->first_bin[k] = p->n_bins;
+    if (p->n_levels == 0) std::fill(std::begin(p->later_bin), std::end(p->later_bin), ~0u);
+    else p->later_bin[p->n_levels - 1] = p->n_bins;
+    p->at[p->n_levels++] = BinLevel{l, lv.offset[l], lv.size[l], lv.resolution[l], lv.flags[l], lv.scale[l], n_log2, run_log2, (uint32_t)places, p->n_bins, p->n_quads};
     p->n_bins += (uint32_t)bins;
-    p->first_bin[k + 1] = p->n_bins;
-    p->first_quad[k + 1] = p->first_quad[k] + (uint32_t)((bins + 3) / 4);
+    p->n_quads += (uint32_t)((bins + 3) / 4);
     p->slice_lds = std::max<uint32_t>(p->slice_lds, (uint32_t)(entry * places));
     return true;
 }
@@ -422,7 +472,7 @@ template <int D, int F> static BinLaunch bin_launch(const BinPlan &p) {
     b.n_stretches = (p.batch + b.stretch - 1) / b.stretch;
     b.room = b.stretch * S::kPairs / 8 * 9;
     b.pitch = 2 * b.stretch * S::kPairs + kBinPiecePad; // (were every far side a record of its own)
-    b.offset_bytes = ((size_t)b.n_stretches * p.first_quad[p.n_levels] * 4 * sizeof(uint32_t) + 255) & ~(size_t)255;
+    b.offset_bytes = ((size_t)b.n_stretches * p.n_quads * 4 * sizeof(uint32_t) + 255) & ~(size_t)255;
     b.scratch_bytes = b.offset_bytes + (size_t)p.n_levels * b.n_stretches * b.pitch * sizeof(BinRecord<F>);
     return b;
 }
@@ -440,47 +490,53 @@ size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_dims, uint32_t n_features)
 }
 
 template <int D, int F, typename G>
-static int launch_binned(const BinPlan &p, const GridLevels &lv, const GridParams &gp, const GradLayout &dl, const float *x, const float4 *order, const void *dLdy,
+static int launch_binned(const BinPlan &p, const GridParams &gp, const GradLayout &dl, const float *x, const float4 *order, const void *dLdy,
                          float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s) {
     typedef BinShape<D, F> S;
     const BinLaunch b = bin_launch<D, F>(p);
     uint32_t *const runs = static_cast<uint32_t *>(scratch);
     BinRecord<F> *const records = reinterpret_cast<BinRecord<F> *>(static_cast<char *>(scratch) + b.offset_bytes);
     uint32_t most_bins = 0;
-    for (uint32_t k = 0; k < p.n_levels; ++k) most_bins = std::max(most_bins, 1u << p.bins_log2[k]);
+    for (uint32_t k = 0; k < p.n_levels; ++k) most_bins = std::max(most_bins, 1u << p.at[k].bins_log2);
     const auto bin = grid_bin_kernel<D, F, G>;
     const size_t bin_lds = (size_t)b.room * sizeof(BinRecord<F>) + (2 * most_bins + 16) * sizeof(uint32_t);
     const size_t sum_lds = p.slice_lds + (2 * kBinSumThreads / 64 + kBinSumThreads / kBinSumGroup + 2 * b.n_stretches + 1) * sizeof(uint32_t);
     // (about as many waves on a CU as it holds, whatever LDS the bins need: small bins are over before many are under way)
     unsigned sum_threads = p.slice_lds > 48 * 1024 ? kBinSumThreads : p.slice_lds > 20 * 1024 ? kBinSumThreads / 2 : kBinSumThreads / 4;
     while (sum_threads * kBinPiecesEach < b.n_stretches) sum_threads *= 2;
-    // Up to four records a lane of an even spread, and a few more that are split: five in flight make one round of them (2-D, 2^18 points 27.3 ->
-    // 24.9 us); long bins are no faster for it (3-D, 2^19: 184 and 191).
-    const bool short_bins = ((size_t)p.batch * S::kPairs) / most_bins <= (size_t)4 * sum_threads;
-    const auto sum = short_bins ? grid_bin_sum_kernel<F, 5> : grid_bin_sum_kernel<F, 4>;
+    // Records a lane has of an even spread, and those that are split (one in sixteen of a level with runs of 16 entries): five in flight where four and the
+    // split ones make five (2-D, 2^18 points 27.3 -> 24.9 us; long bins are no faster for it: 3-D, 2^19 184 and 191), two where that is all there are, and
+    // the rest would be instructions for nothing (3-D, 2^15 points, with the stores of two entries: 25.4 -> 20.3).
+    const size_t a_lane = ((size_t)p.batch * S::kPairs / 16 * 17 / most_bins + sum_threads - 1) / sum_threads;
+    const auto sum = a_lane <= 2 ? grid_bin_sum_kernel<F, 2> : a_lane == 5 ? grid_bin_sum_kernel<F, 5> : grid_bin_sum_kernel<F, 4>;
     if (!reserve_lds(reinterpret_cast<const void *>(bin), bin_lds) || !reserve_lds(reinterpret_cast<const void *>(sum), sum_lds))
         return fail(TNN_ERR_HIP, "cannot reserve %zu and %zu bytes of LDS", bin_lds, sum_lds);
+    // As many workgroups of the sums as the CUs hold at once (2048 threads, 160 KB), in whole rounds of bins.
+    constexpr size_t kRound = 8 * kBinNeighbours;
+    size_t sum_blocks = (p.n_bins + kRound - 1) / kRound * kRound;
+    const size_t held = device_info().n_cu * std::min<size_t>(2048 / sum_threads, 160 * 1024 / sum_lds) / kRound * kRound;
+    if (held > 0 && sum_blocks > held) sum_blocks = held;
     for (size_t first = 0; first < M; first += p.batch) {
         const size_t last = std::min(M, first + p.batch);
         const uint32_t n_stretches = (uint32_t)((last - first + b.stretch - 1) / b.stretch);
-        TNN_LAUNCH(bin, dim3((n_stretches + 7) / 8 * 8 * p.n_levels), dim3(b.threads), bin_lds, s, lv, gp, p, dl, x, order, (const G *)dLdy, runs, records,
+        TNN_LAUNCH(bin, dim3((n_stretches + 7) / 8 * 8 * p.n_levels), dim3(b.threads), bin_lds, s, gp, p, dl, x, order, (const G *)dLdy, runs, records,
                    (long long)first, (long long)last, n_stretches, b.pitch, b.room);
         int rc = check_launch("grid_bin_kernel");
         if (rc) return rc;
-        TNN_LAUNCH(sum, dim3((p.n_bins + 8 * kBinNeighbours - 1) / (8 * kBinNeighbours) * (8 * kBinNeighbours)), dim3(sum_threads), sum_lds, s, lv, p, (const uint32_t *)runs, (const BinRecord<F> *)records, grad,
+        TNN_LAUNCH(sum, dim3((unsigned)sum_blocks), dim3(sum_threads), sum_lds, s, p, (const uint32_t *)runs, (const BinRecord<F> *)records, grad,
                    n_stretches, b.pitch, (int)(overwrite && first == 0));
         if ((rc = check_launch("grid_bin_sum_kernel"))) return rc;
     }
     return TNN_OK;
 }
 
-int launch_grid_binned(const BinPlan &p, const GridLevels &lv, const GridParams &gp, const GradLayout &dl, uint32_t n_dims, uint32_t n_features, const float *x,
+int launch_grid_binned(const BinPlan &p, const GridParams &gp, const GradLayout &dl, uint32_t n_dims, uint32_t n_features, const float *x,
                        const float4 *order, const void *dLdy, int dy_dtype, float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s) {
 #define TNN_BIN_G(D, F)                                                                                                                    \
     switch (dy_dtype) {                                                                                                                    \
-    case TNN_FP32: return launch_binned<D, F, float>(p, lv, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s);                            \
-    case TNN_BF16: return launch_binned<D, F, bf16_t>(p, lv, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s);                           \
-    case TNN_FP16: return launch_binned<D, F, fp16_t>(p, lv, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s);                           \
+    case TNN_FP32: return launch_binned<D, F, float>(p, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s);                            \
+    case TNN_BF16: return launch_binned<D, F, bf16_t>(p, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s);                           \
+    case TNN_FP16: return launch_binned<D, F, fp16_t>(p, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s);                           \
     default: return fail(TNN_ERR_UNSUPPORTED, "dy_dtype %d", dy_dtype);                                                                     \
     }
 #define TNN_BIN_F(D)                                                                                                                       \
