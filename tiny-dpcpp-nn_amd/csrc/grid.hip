@@ -655,7 +655,7 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
         for (uint32_t i = 0; i < n_big; ++i) {
             const uint32_t l = bp.big_level[i];
             const double R = (double)lv.resolution[l];
-            const double per_cell = (double)M / std::pow(R, (double)D);
+            const double per_cell = (double)M / (D == 2 ? R * R : R * R * R);
             int chunk_log2 = -1;
             // (short stretches: many workgroups of some ten microseconds each spread over the CUs far more evenly than few long ones)
             for (int c = 10; c >= 9 && chunk_log2 < 0 && bp.n_tiled < kMaxTiled && per_cell >= (bins ? kBoxedMinPerCellBinned : kBoxedMinPerCell); --c) {

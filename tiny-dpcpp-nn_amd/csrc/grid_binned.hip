@@ -443,7 +443,8 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
     // at random: consecutive entries to a bin.)
     const bool hashed = (lv.flags[l] & 16u) != 0, apart = hashed && gp.hash_type != TNN_HASH_COHERENT_PRIME;
     const double R = (double)lv.resolution[l];
-    const auto groups = [&](uint32_t run) { return std::max(R / (double)((size_t)1 << run), 1.0) * std::pow(R, (double)n_dims - 1.0) / (double)bins; };
+    const double rows = n_dims == 2 ? R : R * R; // (a product: std::pow was half of a plan's time, three of which a pass makes)
+    const auto groups = [&](uint32_t run) { return std::max(R / (double)((size_t)1 << run), 1.0) * rows / (double)bins; };
     uint32_t run_log2 = 4;
     while (((size_t)1 << (run_log2 + n_log2)) < size && (apart || (hashed && groups(run_log2 + 1) >= 64.0))) ++run_log2;
     const size_t places = ((size + ((size_t)1 << (run_log2 + n_log2)) - 1) >> (run_log2 + n_log2)) << run_log2;
