@@ -184,3 +184,18 @@ def test_sums_with_few_and_many_records_a_lane(tnn, oracle, M, features):
     ref = oracle.grid_backward(cfg, x, g, tnn.grid_n_params(d))
     grad = binned(tnn, d, torch.from_numpy(x).to(tnn.dev), torch.from_numpy(g).to(tnn.dev), FP32)
     assert np.abs(grad.cpu().numpy() - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
+
+
+@pytest.mark.parametrize("features", [1, 2, 4])
+def test_tiled_levels_of_an_odd_number_of_entries(tnn, oracle, features):
+    """A tiled level has base_resolution^3 entries, 29791 here: the next level begins in the middle of a pair of entries, and the last entry is half of one."""
+    cfg = dict(CFG3, grid_type="Tiled", base_resolution=31, n_features_per_level=features, n_levels=5)
+    rng = np.random.default_rng(features)
+    M = 40007
+    x = rng.uniform(0, 1, (M, 3)).astype(np.float32)
+    d = tnn.grid_desc(cfg)
+    assert d.offsets[1] % 2 == 1
+    g = rng.standard_normal((M, cfg["n_levels"] * features)).astype(np.float32)
+    ref = oracle.grid_backward(cfg, x, g, tnn.grid_n_params(d))
+    grad = binned(tnn, d, torch.from_numpy(x).to(tnn.dev), torch.from_numpy(g).to(tnn.dev), FP32)
+    assert np.abs(grad.cpu().numpy() - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())

@@ -379,8 +379,8 @@ __global__ void __launch_bounds__(kBinSumThreads, F <= 2 ? 8 : 4)
         const Bins dealt{at_level.bins_log2, at_level.run_log2};
         const uint32_t bin = number - at_level.first_bin, size = at_level.size;
         float *const g = grad + (size_t)at_level.offset * F;
-        if (store) { // the bin's entries have no other contributions
-            // Two neighbouring entries a thread: a run has an even number, a level's offset and size are multiples of 8, and the table is 16-byte aligned.
+        if (store && ((size | at_level.offset) & 1) == 0) { // the bin's entries have no other contributions
+            // Two neighbouring entries a thread: a run has an even number, and the table is 16-byte aligned.
             constexpr int kStore = 2 * F < 4 ? 2 * F : 4;
             typedef float store_t __attribute__((ext_vector_type(kStore)));
             typedef double pair_t __attribute__((ext_vector_type(2)));
@@ -405,12 +405,14 @@ __global__ void __launch_bounds__(kBinSumThreads, F <= 2 ? 8 : 4)
                     to[q] = w;
                 }
             }
-        } else {
+        } else { // (a tiled level may have any number of entries, and begin anywhere)
             for (uint32_t v = threadIdx.x; v < n * F; v += blockDim.x) {
                 const uint32_t e = dealt.entry(bin, v / F), from = v % F * n + v / F;
                 const float sum = (float)sums[from];
                 sums[from] = 0.0;
-                if (e < size) g[(size_t)e * F + v % F] += sum;
+                if (e >= size) continue;
+                float *const to = g + (size_t)e * F + v % F;
+                *to = store ? sum : *to + sum;
             }
         }
         if (next >= bp.n_bins) return;
