@@ -393,8 +393,8 @@ int tnn_grid_backward_ordered(const tnn_grid_desc *desc, const void *d_order, co
  * summed on chip, where the calls above add each of them to the table with atomics. The same contributions in another order
  * of addition. Nothing in the workspace has to be cleared. Its size, tnn_grid_backward_workspace_bytes, grows with the batch up to 2^19
  * points, which are sorted at a time, and no further: room for two records a pair of corners along the first dimension (12, 16, 24
- * or 40 bytes with 1, 2, 4 or 8 features), point and level that is sorted. 16 levels of two features and 2^19 entries: 201 MiB for 2^18
- * points of a 2-D grid, 402 from 2^19 on; 504 and 1001 MiB in 3-D; 836 and 1672 MiB with four features, 1385 and 2768 with eight.
+ * or 40 bytes with 1, 2, 4 or 8 features), point and level that is sorted. 16 levels of two features and 2^19 entries: 183 MiB for 2^18
+ * points of a 2-D grid, 366 from 2^19 on; 500 and 1000 MiB in 3-D; 829 and 1658 MiB with four features, 1377 and 2754 with eight.
  * A caller without that much to spare sorts parts of the batch (overwrite = 0 after the first) or calls the routines above, which need
  * no workspace. */
 size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size_t M);

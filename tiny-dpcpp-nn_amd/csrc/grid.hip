@@ -174,6 +174,8 @@ constexpr uint8_t kAllFeatures = 255;
 // binned; one of 0.7, 4.8 and 7.7; 1.6: 3.8 and 6.4; 3.5: 3.1 and 7.5; 7.9: 2.6 and 6.3).
 constexpr double kBoxedMinPerCell = 0.3, kBoxedMinPerCellBinned = 0.5;
 
+constexpr size_t kMoreBinnedBelow = size_t(1) << 17; // points of a batch in the caller's order that bins more levels (plan_backward)
+
 constexpr int kGridWave = 64;                    // lanes of a wave
 constexpr int kBwdThreads = 512;                 // the backward kernel's workgroups
 constexpr int kDirectPasses = 8;                 // groups of kBwdThreads / lanes-per-point points a direct-route workgroup takes
@@ -635,12 +637,12 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
     const auto enough_to_bin = [&] { return bins && ((unsigned long long)M * n_big << (D - 1)) >= (1ull << 18); };
     divide(0, 0);
     // Beside binned levels a copy of the whole level has to be worth its additions to the table, for the chunks of 1024 points that a batch is cut into
-    // in the end: a level of more entries than a chunk has contributions is binned, too (whole scatter, 2-D, 2^16 points, 2^15 entries 37.8 -> 32.9 us; 2^18
-    // 81 -> 77; 2^15 points, 2^19 entries 39.3 either way), and in three dimensions, where that leaves none as a rule and so a launch less, one of more than
-    // a quarter as many (20 000 points 52 -> 42.5; 2^16 63.5 -> 54.5; 2^17 93 -> 94, and its records take memory: not from there on; with that rule in two
-    // dimensions 2^16 points 35.9).
-    if (!ordered && !nearest && enough_to_bin() && gp.n_levels <= kMaxBinned)
-        divide(std::min<size_t>(M, 1024) << D, D == 2 || M >= (size_t(1) << 17) ? 1 : 4);
+    // in the end: a level of more entries than a chunk has contributions is binned, too (whole scatter, 2-D, 2^16 points, 2^15 entries 37.8 -> 32.9 us;
+    // 2^15 points, 2^19 entries 39.3 either way), and in three dimensions, where that leaves none as a rule and so a launch less, one of more than
+    // a quarter as many (20 000 points 52 -> 42.5; 2^16 63.5 -> 54.5; 2^17 93 -> 94; with that rule in two
+    // dimensions 2^16 points 35.9). The records of such levels take memory, a tenth more, for which 2^18 points would gain 4 of 81: not from 2^17 on.
+    if (!ordered && !nearest && M < kMoreBinnedBelow && enough_to_bin() && gp.n_levels <= kMaxBinned)
+        divide(std::min<size_t>(M, 1024) << D, D == 2 ? 1 : 4);
     // Cell order: of the other levels, those where a stretch of consecutive points of one row of the order's coarse cells
     // fills a box of the level's cells that fits the LDS budget take the boxed route, as long as the level has a point for
     // every few cells (beyond that a box holds hardly more than one contribution per entry and saves no atomics). The order
@@ -949,12 +951,15 @@ TNN_API size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size
     GridParams gp;
     if (check_grid_desc(desc) || grid_common(desc, desc->n_levels * desc->n_features_per_level, M, &lv, &gp)) return 0;
     size_t most = 0;
-    for (const bool ordered : {false, true}) {
+    const auto room_for = [&](bool ordered, size_t points) {
         BinPlan bins{};
         uint32_t n_big, lds;
-        (void)plan_backward(lv, gp, desc->n_dims, desc->n_features_per_level, ordered, true, M, &bins, &n_big, &lds);
+        (void)plan_backward(lv, gp, desc->n_dims, desc->n_features_per_level, ordered, true, points, &bins, &n_big, &lds);
         most = std::max(most, bin_scratch_bytes(bins, desc->n_dims, desc->n_features_per_level));
-    }
+    };
+    room_for(false, M);
+    room_for(true, M);
+    if (M >= kMoreBinnedBelow) room_for(false, kMoreBinnedBelow - 1); // (what holds a batch holds a smaller one)
     return most + 256;
 }
 

@@ -24,6 +24,7 @@ struct BinPlan {
     uint32_t n_levels;
     uint32_t n_bins;                    // of all levels
     uint32_t n_quads;                   // the same in fours of bins
+    uint32_t n_ends;                    // 16-bit numbers of a piece's runs, as bin_launch counts the workspace
     uint32_t slice_lds;                 // LDS bytes of the largest slice
     uint32_t batch;                     // points binned at a time
     uint32_t later_bin[kMaxBinned - 1]; // first bin of the second level and those behind it, ~0 where there is none

@@ -33,7 +33,7 @@ constexpr uint32_t kBinSumGroup = 8;    // lanes that walk through a share of a 
 constexpr int kBinPiecesEach = 4;        // pieces a thread of the sums looks up, at most
 constexpr size_t kBinBatch = size_t(1) << 19; // points binned at a time, at most
 constexpr uint32_t kBinNeighbours = 16;  // consecutive bins on an XCD
-constexpr uint32_t kBinPiecePad = 144; // records between two pieces, so that workgroups in step do not all write to the same channels
+constexpr uint32_t kBinPiecePad = 144; // records between two pieces, at most (bin_launch), so that workgroups in step do not all write to the same channels
 
 // A binning workgroup: its threads (at most), the points of a thread, and the pairs of corners it sorts in LDS. 2048 records of 16
 // bytes let four workgroups of 8 waves share a CU, whose phases (loads, LDS, stores) then overlap; wider records take half as many.
@@ -455,6 +455,7 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
     else p->later_bin[p->n_levels - 1] = p->n_bins;
     p->at[p->n_levels++] = BinLevel{l, lv.offset[l], lv.size[l], lv.resolution[l], lv.flags[l], lv.scale[l], n_log2, run_log2, (uint32_t)places, p->n_bins, p->n_quads};
     p->n_bins += (uint32_t)bins;
+    p->n_ends += std::max<uint32_t>((uint32_t)bins, (size >> 7) * entry > 32 * 1024 ? 256u : 1u) + 1u;
     p->n_quads += (uint32_t)((bins + 3) / 4);
     p->slice_lds = std::max<uint32_t>(p->slice_lds, (uint32_t)(entry * places));
     return true;
@@ -474,9 +475,13 @@ template <int D, int F> static BinLaunch bin_launch(const BinPlan &p) {
     b.stretch = b.threads * S::kPoints;
     b.n_stretches = (p.batch + b.stretch - 1) / b.stretch;
     b.room = b.stretch * S::kPairs / 8 * 9;
-    b.pitch = 2 * b.stretch * S::kPairs + kBinPiecePad; // (were every far side a record of its own)
+    // The workspace has room for two records a pair of corners (were every far side a record of its own), kBinPiecePad records a piece, and a 16-bit number a bin and
+    // piece. A run takes two such numbers, the second out of the pads (3-D, 2^19 entries: 32 records of 144 a piece).
+    const size_t pieces = (size_t)p.n_levels * b.n_stretches, least = 2 * b.stretch * S::kPairs;
+    const size_t counted = (((size_t)b.n_stretches * p.n_ends * sizeof(uint16_t) + 255) & ~(size_t)255) + pieces * (least + kBinPiecePad) * sizeof(BinRecord<F>);
     b.offset_bytes = ((size_t)b.n_stretches * p.n_quads * 4 * sizeof(uint32_t) + 255) & ~(size_t)255;
-    b.scratch_bytes = b.offset_bytes + (size_t)p.n_levels * b.n_stretches * b.pitch * sizeof(BinRecord<F>);
+    b.pitch = (uint32_t)std::max(least, (counted - b.offset_bytes) / (pieces * sizeof(BinRecord<F>)) / 8 * 8);
+    b.scratch_bytes = std::max(counted, b.offset_bytes + pieces * b.pitch * sizeof(BinRecord<F>));
     return b;
 }
 
