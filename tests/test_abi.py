@@ -77,6 +77,15 @@ def test_scatter_workspace_is_as_large_as_the_header_says(lib):
     assert f"({step} MiB for 2^18 points" in header
 
 
+def test_workspace_of_8192_rows_of_width_128_holds_fewer(lib):
+    """From 8192 rows on a workgroup takes 128 rows instead of 64 and leaves half as many partial sums."""
+    from tiny_dpcpp_nn import _lib
+    wide = _lib.MlpDesc(_lib.TNN_FP16, 128, 8, _lib.ACT_RELU, _lib.ACT_NONE)
+    for query in (lib.tnn_mlp_backward_workspace_bytes, lib.tnn_mlp_train_step_workspace_bytes):
+        sizes = [query(ctypes.byref(wide), m) for m in (4096, 8128, 8184, 8192, 8256, 16384)]
+        assert sizes == sorted(sizes)
+
+
 @pytest.mark.parametrize("dims,features,levels,scale,log2,sides", [
     # the sizes on both sides of each rule of tnn_grid_forward_workspace_bytes: (points, whether by levels)
     (2, 2, 8, 1.5, 19, ((2 ** 14, 0), (2 ** 14 + 1, 0), (2 ** 17, 0), (2 ** 18 - 1, 0), (2 ** 18, 1), (2 ** 19 - 1, 1), (2 ** 19, 0))),

@@ -675,15 +675,17 @@ static DwPlan dw_plan(const tnn_mlp_desc *d, size_t M) {
     const int W = d->width, n_mats = d->n_hidden_layers + 1;
     long long target_chunks = 256;
     long long rpc = ((long long)M + target_chunks - 1) / target_chunks;
-    // At width 128 a workgroup of few rows has a short round and one partial sum like any other: 128 rows at least where 64 would be half of the chip's workgroups and more
-    // (steps of 8 hidden layers, us, chunks in multiples of 64, 128, 256: 1024 rows 84, 89, 106; 4096 88, 93, 110; 8192 100, 97, 112; 16384 113, 107, 116; 2^15 and more the same).
-    const long long slab = W == 128 && M >= 8192 ? 2 * kDwSlab : kDwSlab;
-    rpc = (rpc + slab - 1) / slab * slab;
-    if (rpc < slab) rpc = slab;
-    p.rows_per_chunk = rpc;
-    p.n_chunks = M ? ((long long)M + rpc - 1) / rpc : 0;
+    rpc = (rpc + kDwSlab - 1) / kDwSlab * kDwSlab;
+    if (rpc < kDwSlab) rpc = kDwSlab;
+    const auto chunks = [&] { return M ? ((long long)M + rpc - 1) / rpc : 0; };
     p.partials_per_chunk = (W <= 32) ? 4 : 1;
-    p.partial_bytes = (size_t)p.n_chunks * p.partials_per_chunk * n_mats * W * W * sizeof(float);
+    // (room for chunks in multiples of 64 rows, however many there are: what holds 8192 rows holds fewer)
+    p.partial_bytes = (size_t)chunks() * p.partials_per_chunk * n_mats * W * W * sizeof(float);
+    // At width 128 a workgroup of few rows has a short round and one partial sum like any other: 128 rows where 64 would be half of the chip's workgroups and more
+    // (steps of 8 hidden layers, us, chunks in multiples of 64, 128, 256: 1024 rows 84, 89, 106; 4096 88, 93, 110; 8192 100, 97, 112; 16384 113, 107, 116; 2^15 and more the same).
+    if (W == 128 && M >= 8192 && rpc < 2 * kDwSlab) rpc = 2 * kDwSlab;
+    p.rows_per_chunk = rpc;
+    p.n_chunks = chunks();
     p.delta_bytes = (size_t)n_mats * M * W * 2;
     return p;
 }
