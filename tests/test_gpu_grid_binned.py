@@ -130,6 +130,51 @@ def test_crowded_points_take_about_as_long_as_even_ones(tnn, cfg):
         assert time(kind) <= 2 * even, kind
 
 
+def scatter_time(tnn, cfg, x):
+    """Of nine samples of ten calls, the third."""
+    d, M = tnn.grid_desc(cfg), x.shape[0]
+    g = torch.randn((M, cfg["n_levels"] * cfg["n_features_per_level"]), device=tnn.dev)
+    grad = torch.empty(tnn.grid_n_params(d), device=tnn.dev)
+    work = torch.empty(tnn.lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), M), dtype=torch.uint8, device=tnn.dev)
+    times = []
+    for _ in range(9):
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        ev[0].record()
+        for _ in range(10):
+            assert tnn.lib.tnn_grid_backward_binned(ctypes.byref(d), x.data_ptr(), None, g.data_ptr(), FP32, g.shape[1], grad.data_ptr(), 1, M, work.data_ptr(), work.numel(), tnn.stream()) == 0
+        ev[1].record()
+        ev[1].synchronize()
+        times.append(ev[0].elapsed_time(ev[1]))
+    return sorted(times)[2]
+
+
+@pytest.mark.parametrize("cfg,most", [(CFG2, 2.7), (dict(CFG2, log2_hashmap_size=19), 2.3)])
+def test_points_in_a_corner_of_coarse_levels(tnn, cfg, most):
+    """All points in a square of 5 % of the side, where the coarse levels are binned: 2.1 and 1.8 times as long as even ones, and 3.3 and 2.6 to 3.1 without copies of the sums."""
+    M, rng = 2 ** 16, np.random.default_rng(3)
+    even, small = (scatter_time(tnn, cfg, torch.from_numpy(crowded(kind, cfg, M, rng)).to(tnn.dev)) for kind in ("even", "small"))
+    assert small <= most * even
+
+
+@pytest.mark.parametrize("features", [1, 2, 4, 8])
+@pytest.mark.parametrize("cfg", [CFG2, CFG3, dict(CFG3, grid_type="Tiled", base_resolution=15)])
+@pytest.mark.parametrize("crowd", [1500, 3000, 6000, 12000, 40007])
+def test_bins_with_copies_of_their_sums(tnn, oracle, cfg, features, crowd):
+    """So many points of 40007 in one cell: a bin has copies from eight records a lane on, which are one or more of such a point and 256, 512 or 1024 lanes. Every bin's
+    sums are followed by others', with and without copies, in the same LDS; levels of an odd number of entries (tiled) take the other store. The bar of even points."""
+    cfg = dict(cfg, n_features_per_level=features, n_levels=16 if features <= 2 else 10)
+    M, rng = 40007, np.random.default_rng(crowd + features)
+    x = rng.uniform(0, 1, (M, cfg["n_dims"])).astype(np.float32)
+    x[rng.permutation(M)[:crowd]] = 0.4321
+    d = tnn.grid_desc(cfg)
+    g = rng.standard_normal((M, cfg["n_levels"] * features)).astype(np.float32)
+    ref = oracle.grid_backward(cfg, x, g, tnn.grid_n_params(d))
+    table = np.full(tnn.grid_n_params(d), 0.5, np.float32)
+    for overwrite in (True, False):
+        grad = binned(tnn, d, torch.from_numpy(x).to(tnn.dev), torch.from_numpy(g).to(tnn.dev), FP32, grad=torch.from_numpy(table).to(tnn.dev), overwrite=overwrite)
+        assert np.abs(grad.cpu().numpy() - (0 if overwrite else 0.5) - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
+
+
 @pytest.mark.parametrize("cfg", [CFG2, CFG3, dict(CFG3, log2_hashmap_size=22, n_levels=12), dict(CFG3, n_features_per_level=8, n_levels=6, per_level_scale=2.0),
                                  dict(CFG2, interpolation="Nearest"), dict(CFG2, n_features_per_level=1, grid_type="Dense", n_levels=9)])
 @pytest.mark.parametrize("kind", ["even", "small"])

@@ -16,6 +16,7 @@ struct BinLevel {
     float scale;
     uint32_t bins_log2, run_log2; // the level's runs of 2^run_log2 entries go to its 2^bins_log2 bins in turn
     uint32_t places;              // entries a bin has room for
+    uint32_t copies_log2;         // copies of its sums that a crowded bin has
     uint32_t first_bin;           // bins of the levels in front of this one
     uint32_t first_quad;          // the same in fours of bins
 };

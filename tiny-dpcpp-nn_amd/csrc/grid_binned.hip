@@ -31,6 +31,9 @@ namespace tnn {
 constexpr int kBinSumThreads = 1024; // at most
 constexpr uint32_t kBinSumGroup = 8;    // lanes that walk through a share of a bin's records together
 constexpr int kBinPiecesEach = 4;        // pieces a thread of the sums looks up, at most
+// Copies of the sums of a crowded bin (grid_bin_sum_kernel): at most sixteen, in 8 KB and what keeps an entry's copies in different banks. Bins of more than 4 KB have one.
+constexpr uint32_t kBinCopiesLog2 = 4, kBinCopySkew = 2; // (doubles between two copies)
+constexpr size_t kBinCopiesBytes = 8 * 1024 + (sizeof(double) * kBinCopySkew << kBinCopiesLog2);
 constexpr size_t kBinBatch = size_t(1) << 19; // points binned at a time, at most
 constexpr uint32_t kBinNeighbours = 16;  // consecutive bins on an XCD
 constexpr uint32_t kBinPiecePad = 144; // records between two pieces, at most (bin_launch), so that workgroups in step do not all write to the same channels
@@ -269,6 +272,9 @@ __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
 // runs lie is loaded while this one's records are summed, and sums are cleared as they are read. What was left of it were instructions, eight and more waves a bin of them:
 // the prefix sums over the waves are a value a lane, a wave without pieces leaves the look-up out, and two entries leave together (3-D, 2^15 points 30 -> 20.3 us,
 // 100 003 46 -> 37.5, 2^19 101 -> 96; 2-D, 20 011 points 11.3 -> 8.2, 2^16 12.3 -> 9.7, 2^18 23.4 -> 20.8).
+// Points that crowd a part of the volume meet a few of a coarse level's entries only: lanes queue up on them, and the longest bin is the kernel's time. A small bin
+// has room for copies of its sums, and short bins take one as if they had not (whole scatter, 2^16 points, even / in a square or cube of 5 % of the side, before the
+// coarsest levels were binned, then, with copies: 2-D, 2^19 entries 51 / 77, 40 / 124, 40 / 72 us; 3-D 66 / 313, 48 / 394, 48 / 231; 2-D, 2^15 entries 43 / 84, 35 / 120, 35 / 72).
 template <int F, int kAhead>
 __global__ void __launch_bounds__(kBinSumThreads, F <= 2 ? 8 : 4)
     grid_bin_sum_kernel(const BinPlan bp, const uint32_t *__restrict__ runs_of, const BinRecord<F> *__restrict__ records,
@@ -349,6 +355,9 @@ __global__ void __launch_bounds__(kBinSumThreads, F <= 2 ? 8 : 4)
         __syncthreads();
         const BinRecord<F> *const rec = records + (size_t)k * n_stretches * pitch;
         const uint32_t group = threadIdx.x / kGroup, end = (group + 1) * share < total ? (group + 1) * share : total;
+        // Of a bin with more than eight records a lane, whose points are crowded where even ones leave it a fraction of that, neighbouring lanes add to copies of their own.
+        const uint32_t copies = total > 8 * blockDim.x ? 1u << at_level.copies_log2 : 1u, copy = n * F + kBinCopySkew;
+        double *const own = sums + (threadIdx.x & (copies - 1)) * copy;
         uint32_t i = group * share + threadIdx.x % kGroup, s = i < end ? group_run[group] : 0u;
         for (; i < end; i += kAhead * kGroup) {
             uint32_t at_a[kAhead];
@@ -367,11 +376,11 @@ __global__ void __launch_bounds__(kBinSumThreads, F <= 2 ? 8 : 4)
                 const uint32_t where = i + a * kGroup < end ? r[a].where : 0u, near = where & 0x7fff, far = (where >> 15) & 0x7fff;
                 if (where & (1u << 30)) {
 #pragma unroll
-                    for (int f = 0; f < F; ++f) lds_add(&sums[f * n + near], (1 - r[a].frac) * r[a].g[f]);
+                    for (int f = 0; f < F; ++f) lds_add(&own[f * n + near], (1 - r[a].frac) * r[a].g[f]);
                 }
                 if (where & (1u << 31)) {
 #pragma unroll
-                    for (int f = 0; f < F; ++f) lds_add(&sums[f * n + far], r[a].frac * r[a].g[f]);
+                    for (int f = 0; f < F; ++f) lds_add(&own[f * n + far], r[a].frac * r[a].g[f]);
                 }
             }
         }
@@ -390,8 +399,13 @@ __global__ void __launch_bounds__(kBinSumThreads, F <= 2 ? 8 : 4)
 #pragma unroll
                 for (int f = 0; f < F; ++f) {
                     pair_t *const both = reinterpret_cast<pair_t *>(sums + f * n + v);
-                    const pair_t d = *both;
+                    pair_t d = *both;
                     *both = pair_t{0.0, 0.0};
+                    for (uint32_t c = 1; c < copies; ++c) {
+                        pair_t *const other = reinterpret_cast<pair_t *>(sums + c * copy + f * n + v);
+                        d += *other;
+                        *other = pair_t{0.0, 0.0};
+                    }
                     sum[f] = (float)d[0];
                     sum[F + f] = (float)d[1];
                 }
@@ -408,11 +422,14 @@ __global__ void __launch_bounds__(kBinSumThreads, F <= 2 ? 8 : 4)
         } else { // (a tiled level may have any number of entries, and begin anywhere)
             for (uint32_t v = threadIdx.x; v < n * F; v += blockDim.x) {
                 const uint32_t e = dealt.entry(bin, v / F), from = v % F * n + v / F;
-                const float sum = (float)sums[from];
-                sums[from] = 0.0;
+                double sum = 0.0;
+                for (uint32_t c = 0; c < copies; ++c) {
+                    sum += sums[c * copy + from];
+                    sums[c * copy + from] = 0.0;
+                }
                 if (e >= size) continue;
                 float *const to = g + (size_t)e * F + v % F;
-                *to = store ? sum : *to + sum;
+                *to = store ? (float)sum : *to + (float)sum;
             }
         }
         if (next >= bp.n_bins) return;
@@ -451,13 +468,16 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
     while (((size_t)1 << (run_log2 + n_log2)) < size && (apart || (hashed && groups(run_log2 + 1) >= 64.0))) ++run_log2;
     const size_t places = ((size + ((size_t)1 << (run_log2 + n_log2)) - 1) >> (run_log2 + n_log2)) << run_log2;
     if (places > 0x7fff || places * entry > kBinSliceBytes) return false;
+    const auto sums_bytes = [&](uint32_t copies) { return copies ? (entry * places + sizeof(double) * kBinCopySkew) << copies : entry * places; };
+    uint32_t copies_log2 = 0;
+    while (copies_log2 < kBinCopiesLog2 && sums_bytes(copies_log2 + 1) <= kBinCopiesBytes) ++copies_log2;
     if (p->n_levels == 0) std::fill(std::begin(p->later_bin), std::end(p->later_bin), ~0u);
     else p->later_bin[p->n_levels - 1] = p->n_bins;
-    p->at[p->n_levels++] = BinLevel{l, lv.offset[l], lv.size[l], lv.resolution[l], lv.flags[l], lv.scale[l], n_log2, run_log2, (uint32_t)places, p->n_bins, p->n_quads};
+    p->at[p->n_levels++] = BinLevel{l, lv.offset[l], lv.size[l], lv.resolution[l], lv.flags[l], lv.scale[l], n_log2, run_log2, (uint32_t)places, copies_log2, p->n_bins, p->n_quads};
     p->n_bins += (uint32_t)bins;
     p->n_ends += std::max<uint32_t>((uint32_t)bins, (size >> 7) * entry > 32 * 1024 ? 256u : 1u) + 1u;
     p->n_quads += (uint32_t)((bins + 3) / 4);
-    p->slice_lds = std::max<uint32_t>(p->slice_lds, (uint32_t)(entry * places));
+    p->slice_lds = std::max<uint32_t>(p->slice_lds, (uint32_t)sums_bytes(copies_log2));
     return true;
 }
 
