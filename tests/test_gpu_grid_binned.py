@@ -156,6 +156,15 @@ def test_points_in_a_corner_of_coarse_levels(tnn, cfg, most):
     assert small <= most * even
 
 
+@pytest.mark.parametrize("seed", [2, 3])
+def test_long_bins_do_not_wait_for_each_other(tnn, seed):
+    """All of 2^18 points are one of twenty: 4.0 and 4.4 times as long as even ones, and 6.1 and 6.2 where a workgroup takes the second of its long bins after the first."""
+    cfg, M, rng = dict(CFG2, log2_hashmap_size=19), 2 ** 18, np.random.default_rng(seed)
+    twenty = rng.uniform(0, 1, (20, 2))[rng.integers(0, 20, M)]
+    few, even = (scatter_time(tnn, cfg, torch.from_numpy(x.astype(np.float32)).to(tnn.dev)) for x in (twenty, rng.uniform(0, 1, (M, 2))))
+    assert few <= 5.2 * even
+
+
 @pytest.mark.parametrize("features", [1, 2, 4, 8])
 @pytest.mark.parametrize("cfg", [CFG2, CFG3, dict(CFG3, grid_type="Tiled", base_resolution=15)])
 @pytest.mark.parametrize("crowd", [1500, 3000, 6000, 12000, 40007])

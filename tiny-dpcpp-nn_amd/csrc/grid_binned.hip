@@ -268,7 +268,7 @@ __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
 // piece's run); eight lanes take an equal share of them all, whatever the runs' lengths, and walk from run to run. Neighbouring bins, whose
 // runs share lines, are workgroups of one XCD, sixteen at a time. kAhead: records of a lane in flight.
 // Long bins are bound by the LDS atomics, two entries of F values a record. Short ones were bound by what comes before the first record: a workgroup a
-// bin, 3-D, 2^15 points, took 30 us, 18 of them without a record read or an entry written. So a workgroup stays for several bins: where the next bin's
+// bin, 3-D, 2^15 points, took 30 us, 18 of them without a record read or an entry written. So a workgroup stays for several of the shortest (launch_binned): where the next bin's
 // runs lie is loaded while this one's records are summed, and sums are cleared as they are read. What was left of it were instructions, eight and more waves a bin of them:
 // the prefix sums over the waves are a value a lane, a wave without pieces leaves the look-up out, and two entries leave together (3-D, 2^15 points 30 -> 20.3 us,
 // 100 003 46 -> 37.5, 2^19 101 -> 96; 2-D, 20 011 points 11.3 -> 8.2, 2^16 12.3 -> 9.7, 2^18 23.4 -> 20.8).
@@ -539,11 +539,18 @@ static int launch_binned(const BinPlan &p, const GridParams &gp, const GradLayou
     const auto sum = a_lane <= 2 ? grid_bin_sum_kernel<F, 2> : a_lane == 5 ? grid_bin_sum_kernel<F, 5> : grid_bin_sum_kernel<F, 4>;
     if (!reserve_lds(reinterpret_cast<const void *>(bin), bin_lds) || !reserve_lds(reinterpret_cast<const void *>(sum), sum_lds))
         return fail(TNN_ERR_HIP, "cannot reserve %zu and %zu bytes of LDS", bin_lds, sum_lds);
-    // As many workgroups of the sums as the CUs hold at once (2048 threads, 160 KB), in whole rounds of bins.
+    // A workgroup stays for several bins (as many workgroups as threads and LDS of the CUs allow, in whole rounds of bins; the registers of eight features let three in of four,
+    // and the fourth starts where one is through: 3-D, 2^17 entries, 2^13 points 26.3 us, with three 25.8, but of twenty points 59 and 67) where what comes before a bin's first record is most of its
+    // time: bins of 256 records, of 128 with eight features. Longer ones have a workgroup each, which starts wherever one is through: a workgroup that met several bins
+    // of crowded points was the kernel's time. Twenty points only, whole scatter, us, before workgroups stayed for bins, for all of them, now: 2-D, 2^19 entries, 2^16 points
+    // 113, 137, 106; 2^18 358, 631, 321; 3-D, 2^17 points 317, 411, 294; eight features 766, 1087, 686. Even points, for all of them, now: 2-D, 2^16 points 39.9, 41.7; 2^18
+    // 75.6, 78.3; 3-D, 2^15 points 35.4, 38.7; 2^16 48.1, 48.4; 2^18 151, 146; 2^19 268, 255. Bins of 256 records, a workgroup each, now: 3-D, 2^14 points 32.5, 30.1.
     constexpr size_t kRound = 8 * kBinNeighbours;
     size_t sum_blocks = (p.n_bins + kRound - 1) / kRound * kRound;
-    const size_t held = device_info().n_cu * std::min<size_t>(2048 / sum_threads, 160 * 1024 / sum_lds) / kRound * kRound;
-    if (held > 0 && sum_blocks > held) sum_blocks = held;
+    if ((size_t)p.batch * S::kPairs / most_bins <= (F == 8 ? 128 : 256)) {
+        const size_t held = device_info().n_cu * std::min<size_t>(2048 / sum_threads, 160 * 1024 / sum_lds) / kRound * kRound;
+        if (held > 0 && sum_blocks > held) sum_blocks = held;
+    }
     for (size_t first = 0; first < M; first += p.batch) {
         const size_t last = std::min(M, first + p.batch);
         const uint32_t n_stretches = (uint32_t)((last - first + b.stretch - 1) / b.stretch);
