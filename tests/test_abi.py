@@ -77,6 +77,28 @@ def test_scatter_workspace_is_as_large_as_the_header_says(lib):
     assert f"({step} MiB for 2^18 points" in header
 
 
+@pytest.mark.parametrize("dims,features,levels,log2,scale,base,grid_type", [
+    (2, 2, 16, 15, 1.5, 16, 0), (2, 2, 16, 19, 1.5, 16, 0), (2, 2, 12, 16, 1.5, 16, 0), (2, 2, 16, 22, 1.5, 16, 0), (2, 1, 16, 12, 1.3, 16, 0), (2, 8, 8, 17, 2.0, 16, 0), (2, 2, 40, 19, 1.2, 16, 0),
+    (3, 2, 16, 19, 1.447, 16, 0), (3, 2, 8, 20, 1.447, 16, 0), (3, 2, 4, 19, 1.3, 16, 1), (3, 2, 16, 19, 1.447, 16, 2), (3, 4, 12, 14, 1.6, 16, 0), (3, 8, 3, 21, 1.2, 128, 0), (3, 1, 2, 23, 1.5, 300, 0)])
+def test_scatter_workspace_of_a_batch_holds_smaller_ones(lib, dims, features, levels, log2, scale, base, grid_type):
+    """Over the sizes where the binning's workgroups are halved, levels leave the bins for boxes, and coarse levels are binned or not. From 2^17 points on the size is the points' share of that for 2^18."""
+    from tiny_dpcpp_nn import _lib
+    d, mlp = _lib.GridDesc(), _lib.MlpDesc(_lib.TNN_FP16, 64, 2, _lib.ACT_RELU, _lib.ACT_NONE)
+    assert lib.tnn_grid_desc_init(ctypes.byref(d), dims, levels, features, log2, base, scale, grid_type, 1, 1, _lib.TNN_FP32) == 0
+    sizes = {2 ** k + e for k in range(8, 22) for e in (-1, 0, 1)} | {int(2 ** (8 + i / 12)) for i in range(156)}
+    for halved in (2 ** 18, 2 ** 19, 2 ** 17):  # points times levels
+        sizes |= {halved // n + e for n in range(1, levels + 1) for e in (-1, 0, 1)}
+    for l in range(levels):
+        sizes |= {min(2 ** 21, d.resolutions[l] ** dims // 2) + e for e in (-1, 0, 1)}
+    sizes = sorted(m for m in sizes if m > 0)
+    for query in (lambda m: lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), m), lambda m: lib.tnn_grid_mlp_train_step_workspace_bytes(ctypes.byref(d), ctypes.byref(mlp), m)):
+        needs = [query(m) for m in sizes]
+        assert needs == sorted(needs), [m for m, a, b in zip(sizes, needs, needs[1:]) if b < a]
+    half, whole = (lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), m) for m in (2 ** 17, 2 ** 18))
+    if levels > 2 and (log2, grid_type) not in ((12, 0), (14, 0), (19, 2)):  # (2^17 points of two levels have the smaller workgroups; levels of small tables are in boxes at 2^18, in cell order)
+        assert half <= whole * 0.51
+
+
 def test_workspace_of_8192_rows_of_width_128_holds_fewer(lib):
     """From 8192 rows on a workgroup takes 128 rows instead of 64 and leaves half as many partial sums."""
     from tiny_dpcpp_nn import _lib

@@ -216,6 +216,20 @@ def test_encoding_orders_a_batch_whose_finest_levels_are_not_binned(tnn):
     assert float((got.reshape(-1) - ref.reshape(-1)).abs().max()) <= 1e-5 * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("cfg,M", [(CFG3, 16384), (dict(CFG3, n_levels=8, log2_hashmap_size=20), 32768), (dict(CFG2, n_levels=12, log2_hashmap_size=16), 65536), (CFG3, 2 ** 17)])
+def test_workspace_of_a_batch_holds_a_smaller_one(tnn, cfg, M):
+    """Just below these sizes the scatter has twice as many workgroups or bins more levels, and needs more."""
+    from tiny_dpcpp_nn import _lib
+    d = tnn.grid_desc(cfg)
+    work = torch.empty(tnn.lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), M), dtype=torch.uint8, device=tnn.dev)
+    for m in (M, M - 1, M * 15 // 16, M * 14 // 15):
+        x, g = torch.rand((m, cfg["n_dims"]), device=tnn.dev), torch.randn((m, 2 * cfg["n_levels"]), device=tnn.dev)
+        grad = torch.empty(tnn.grid_n_params(d), device=tnn.dev)
+        _lib.check(tnn.lib.tnn_grid_backward_binned(ctypes.byref(d), x.data_ptr(), None, g.data_ptr(), FP32, g.shape[1], grad.data_ptr(), 1, m, work.data_ptr(), work.numel(), tnn.stream()))
+        ref = tnn.grid_backward(d, x, g, FP32)
+        assert float((grad - ref).abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max()))
+
+
 def test_binned_workspace_is_checked(tnn):
     from tiny_dpcpp_nn import _lib
     d = tnn.grid_desc(CFG3)

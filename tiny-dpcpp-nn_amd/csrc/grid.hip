@@ -166,6 +166,7 @@ struct BackwardPlan {
     uint8_t tiled_pieces[16];     // workgroups per row of the order's coarse cells; they take the row's stretches in turn
     uint32_t bins_per_row;        // coarse cells in a row (64 in 2-D, 16 in 3-D), n_rows rows
     uint32_t n_rows;
+    size_t more_up_to;            // points up to which a batch in the caller's order bins more levels, 0: none does
 };
 constexpr uint32_t kMaxTiled = 16;
 constexpr uint8_t kAllFeatures = 255;
@@ -174,7 +175,7 @@ constexpr uint8_t kAllFeatures = 255;
 // binned; one of 0.7, 4.8 and 7.7; 1.6: 3.8 and 6.4; 3.5: 3.1 and 7.5; 7.9: 2.6 and 6.3).
 constexpr double kBoxedMinPerCell = 0.3, kBoxedMinPerCellBinned = 0.5;
 
-constexpr size_t kMoreBinnedBelow = size_t(1) << 17; // points of a batch in the caller's order that bins more levels (plan_backward)
+constexpr size_t kMoreBinnedBelow = size_t(1) << 17; // points of a batch in the caller's order that may bin more levels (plan_backward)
 
 constexpr int kGridWave = 64;                    // lanes of a wave
 constexpr int kBwdThreads = 512;                 // the backward kernel's workgroups
@@ -183,6 +184,7 @@ constexpr uint32_t kPrivateLdsBytes = 64 * 1024; // LDS budget of a workgroup; t
 // In cell order more levels take an LDS route, and the launch's LDS size holds for every workgroup, also for those of the
 // direct route, which need none: four workgroups of 40 KiB fill a CU's wave slots.
 constexpr uint32_t kPrivateLdsBytesOrdered = 40 * 1024;
+constexpr uint32_t kCopiedBytesOrdered = 16 * 1024; // and of a level that is copied whole
 constexpr uint32_t kPrivateChunk = 4096;         // points per workgroup on the LDS route
 
 // Coordinates and row number of the i-th point: row i of x, or the i-th record of the cell order (grid_order.hip).
@@ -598,6 +600,30 @@ static int launch_grid_forward_p(const tnn_grid_desc *d, const GridLevels &lv, c
     return launch_grid_forward_o<D, F, fp16_t>(lv, gp, x, order, table, out, out_dtype, M, s);
 }
 
+// Coarse cells of the order along a dimension (grid_order.hip), and rows of them.
+static uint32_t coarse_cells(uint32_t n_dims) { return n_dims == 2 ? 64 : 16; }
+
+// Cell order: log2 of the points of a stretch whose box of the level's cells fits the LDS budget, -1 where none does or the level has too few points a
+// cell for it (beyond that a box holds hardly more than one contribution per entry and saves no atomics). The order walks a lattice of 64^2 (16^3)
+// coarse cells row by row, x fastest: with the points spread evenly a row holds M / 64 (M / 256) of them, and a stretch of C of these spans that share of the
+// level's width plus a coarse cell, and one coarse cell in the other dimensions. A stretch that breaks the estimate is caught in the kernel.
+// (Short stretches: many workgroups of some ten microseconds each spread over the CUs far more evenly than few long ones.) A level that has boxes has them in every larger batch.
+static int boxed_chunk_log2(uint32_t resolution, uint32_t n_dims, uint32_t F, double min_per_cell, size_t M) {
+    const double R = (double)resolution, coarse = (double)coarse_cells(n_dims), per_row = (double)M * coarse / 4096.0;
+    if ((double)M / (n_dims == 2 ? R * R : R * R * R) < min_per_cell) return -1;
+    for (int c = 10; c >= 9; --c) {
+        const double share = std::min(1.0, (double)(1u << c) / std::max(per_row, 1.0));
+        double cells = (share * R + R / coarse + 2.0) * (R / coarse + 2.0);
+        if (n_dims == 3) cells *= R / coarse + 2.0;
+        if (cells * F * sizeof(double) <= 0.9 * (double)kPrivateLdsBytesOrdered) return c;
+    }
+    return -1;
+}
+
+// Binned from where the atomics it saves (one request per pair of corners, 20e9 a second) take longer than its two launches:
+// 2^18 requests. (2-D, 11 such levels, 12 000 points: 20 us either way; 2^16 points: 42 against 95.)
+static bool enough_to_bin(size_t M, uint32_t n_levels, uint32_t n_dims) { return ((unsigned long long)M * n_levels << (n_dims - 1)) >= (1ull << 18); }
+
 // Which route every level takes: n_big levels are left for the direct one (bp->big_level), those of `bins` for the binned one
 // (grid_binned.hip), which needs scratch memory and is planned for only when `bins` is given.
 static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, uint32_t n_dims, uint32_t F, bool ordered, bool fp32_table, size_t M, BinPlan *bins,
@@ -617,7 +643,7 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
             const size_t feature_bytes = (size_t)lv.size[l] * sizeof(double), bytes = feature_bytes * F;
             // (in cell order only the coarsest levels: the box of a stretch is far smaller than a level from 8 KiB on)
             const bool worth_it = per_chunk >= 2 * (size_t)lv.size[l] && contributions >= an_entry * (size_t)lv.size[l];
-            if (worth_it && bytes <= (ordered ? 16384u : bp.budget)) {
+            if (worth_it && bytes <= (ordered ? kCopiedBytesOrdered : bp.budget)) {
                 bp.small_feature[bp.n_small] = kAllFeatures;
                 bp.small_level[bp.n_small++] = (uint8_t)l;
                 if (bytes > lds_bytes) lds_bytes = (uint32_t)bytes;
@@ -632,40 +658,29 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
             }
         }
     };
-    // Binned from where the atomics it saves (one request per pair of corners, 20e9 a second) take longer than its two launches:
-    // 2^18 requests. (2-D, 11 such levels, 12 000 points: 20 us either way; 2^16 points: 42 against 95.)
-    const auto enough_to_bin = [&] { return bins && ((unsigned long long)M * n_big << (D - 1)) >= (1ull << 18); };
+    const auto bin_others = [&] { return bins && enough_to_bin(M, n_big, n_dims); };
     divide(0, 0);
     // Beside binned levels a copy of the whole level has to be worth its additions to the table, for the chunks of 1024 points that a batch is cut into
     // in the end: a level of more entries than a chunk has contributions is binned, too (whole scatter, 2-D, 2^16 points, 2^15 entries 37.8 -> 32.9 us;
     // 2^15 points, 2^19 entries 39.3 either way), and in three dimensions, where that leaves none as a rule and so a launch less, one of more than
     // a quarter as many (20 000 points 52 -> 42.5; 2^16 63.5 -> 54.5; 2^17 93 -> 94; with that rule in two
-    // dimensions 2^16 points 35.9). The records of such levels take memory, a tenth more, for which 2^18 points would gain 4 of 81: not from 2^17 on.
-    if (!ordered && !nearest && M < kMoreBinnedBelow && enough_to_bin() && gp.n_levels <= kMaxBinned)
+    // dimensions 2^16 points 35.9). The records of such levels take memory: batches that need more of it for them than 2^17 points do
+    // without (16 levels in 3-D: 122 880 points), and that many and more, for which 2^18 points would gain 4 of 81, do not have them.
+    if (!ordered && !nearest && bin_others() && gp.n_levels <= kMaxBinned) {
+        const size_t without = n_big;
         divide(std::min<size_t>(M, 1024) << D, D == 2 ? 1 : 4);
-    // Cell order: of the other levels, those where a stretch of consecutive points of one row of the order's coarse cells
-    // fills a box of the level's cells that fits the LDS budget take the boxed route, as long as the level has a point for
-    // every few cells (beyond that a box holds hardly more than one contribution per entry and saves no atomics). The order
-    // (grid_order.hip) walks a lattice of 64^2 (16^3) coarse cells row by row, x fastest: with the points spread evenly a
-    // row holds M / 64 (M / 256) of them, and a stretch of C of these spans that share of the level's width plus a coarse
-    // cell, and one coarse cell in the other dimensions. A stretch that breaks the estimate is caught in the kernel.
+        if (n_big > without) bp.more_up_to = std::min(kMoreBinnedBelow / 1024 * without / n_big * 1024, kMoreBinnedBelow - 1);
+        if (M > bp.more_up_to) divide(0, 0);
+    }
+    // Cell order: of the other levels, those with boxes take the boxed route.
     if (ordered && gp.n_levels > 0 && !nearest) {
-        bp.bins_per_row = (D == 2) ? 64 : 16;
+        bp.bins_per_row = coarse_cells(n_dims);
         bp.n_rows = 4096 / bp.bins_per_row;
-        const double per_row = (double)M / bp.n_rows, coarse = (double)bp.bins_per_row;
+        const double per_row = (double)M / bp.n_rows;
         uint32_t kept = 0;
         for (uint32_t i = 0; i < n_big; ++i) {
             const uint32_t l = bp.big_level[i];
-            const double R = (double)lv.resolution[l];
-            const double per_cell = (double)M / (D == 2 ? R * R : R * R * R);
-            int chunk_log2 = -1;
-            // (short stretches: many workgroups of some ten microseconds each spread over the CUs far more evenly than few long ones)
-            for (int c = 10; c >= 9 && chunk_log2 < 0 && bp.n_tiled < kMaxTiled && per_cell >= (bins ? kBoxedMinPerCellBinned : kBoxedMinPerCell); --c) {
-                const double share = std::min(1.0, (double)(1u << c) / std::max(per_row, 1.0));
-                double cells = (share * R + R / coarse + 2.0) * (R / coarse + 2.0);
-                if (D == 3) cells *= R / coarse + 2.0;
-                if (cells * F * sizeof(double) <= 0.9 * (double)bp.budget) chunk_log2 = c;
-            }
+            const int chunk_log2 = bp.n_tiled < kMaxTiled ? boxed_chunk_log2(lv.resolution[l], n_dims, F, bins ? kBoxedMinPerCellBinned : kBoxedMinPerCell, M) : -1;
             if (chunk_log2 >= 0) {
                 const uint32_t pieces = (uint32_t)std::min(64.0, std::ceil(per_row / (double)(1u << chunk_log2)) + 1.0);
                 bp.tiled_level[bp.n_tiled] = (uint8_t)l;
@@ -684,7 +699,7 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
     while (bp.chunk > 1024 && (M / bp.chunk) * bp.n_small < 256) bp.chunk /= 2;
     bp.small_blocks = (uint32_t)((M + bp.chunk - 1) / bp.chunk);
     if (bins) *bins = BinPlan{};
-    if (enough_to_bin()) {
+    if (bin_others()) {
         uint32_t kept = 0;
         for (uint32_t i = 0; i < n_big; ++i)
             if (!bin_plan_add(bins, bp.big_level[i], lv, gp, n_dims, F, M)) bp.big_level[kept++] = bp.big_level[i];
@@ -950,16 +965,67 @@ TNN_API size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size
     GridLevels lv;
     GridParams gp;
     if (check_grid_desc(desc) || grid_common(desc, desc->n_levels * desc->n_features_per_level, M, &lv, &gp)) return 0;
-    size_t most = 0;
-    const auto room_for = [&](bool ordered, size_t points) {
-        BinPlan bins{};
-        uint32_t n_big, lds;
-        (void)plan_backward(lv, gp, desc->n_dims, desc->n_features_per_level, ordered, true, points, &bins, &n_big, &lds);
-        most = std::max(most, bin_scratch_bytes(bins, desc->n_dims, desc->n_features_per_level));
+    // What holds a batch holds a smaller one: the most that any batch of up to M points needs, in either order.
+    const uint32_t D = desc->n_dims, F = desc->n_features_per_level;
+    size_t most = 0, most_points = 0; // (points times levels)
+    uint32_t n_big, lds;
+    BinPlan bins{};
+    const bool followed = gp.n_levels <= kMaxBinned; // (of more levels than are ever binned as many as are are taken to be, at every size)
+    if (followed) {
+        // The caller's order: as many levels at every size, but more up to one size (plan_backward).
+        const size_t more = plan_backward(lv, gp, D, F, false, true, M, &bins, &n_big, &lds).more_up_to;
+        most = bin_scratch_bytes_up_to(bins, D, F);
+        most_points = (size_t)bins.batch * bins.n_levels;
+        if (more && M > more) {
+            (void)plan_backward(lv, gp, D, F, false, true, more, &bins, &n_big, &lds);
+            most = std::max(most, bin_scratch_bytes_up_to(bins, D, F));
+        }
+    }
+    // Cell order: levels that are not copied leave the bins for boxes one by one as the batch grows, each at a size of its own.
+    uint32_t n = 0, level[TNN_GRID_MAX_LEVELS], most_bins = 0;
+    size_t boxed_from[TNN_GRID_MAX_LEVELS];
+    for (uint32_t l = 0; l < gp.n_levels; ++l) {
+        if (lv.size[l] * F * sizeof(double) <= kCopiedBytesOrdered) continue;
+        const double R = (double)lv.resolution[l], enough = std::ceil(kBoxedMinPerCellBinned * (D == 2 ? R * R : R * R * R));
+        const auto boxed = [&](size_t points) { return boxed_chunk_log2(lv.resolution[l], D, F, kBoxedMinPerCellBinned, points) >= 0; };
+        level[n] = l;
+        boxed_from[n] = ~(size_t)0;
+        if (followed && enough <= (double)M) {
+            size_t no = (size_t)enough - 1, yes = (size_t)enough;
+            if (!boxed(yes)) { // (its boxes do not fit yet)
+                no = yes;
+                yes = boxed(M) ? M : boxed_from[n];
+            }
+            while (yes - no > 1 && yes <= M) (boxed((no + yes) / 2) ? yes : no) = (no + yes) / 2;
+            boxed_from[n] = yes;
+        }
+        ++n;
+    }
+    bool is_binned[TNN_GRID_MAX_LEVELS];
+    const auto in_order = [&](size_t points) {
+        const size_t batch = std::min(points, kBinBatch);
+        uint32_t in_boxes = 0, others = 0, binned = 0;
+        for (uint32_t i = 0; i < n; ++i) others += boxed_from[i] > points || in_boxes++ >= kMaxTiled;
+        // (by a quarter fewer points and levels need less, whatever their workgroups and tables)
+        if (!enough_to_bin(points, others, D) || (batch + 1024) * others * 4 <= most_points * 3) return;
+        if (most_bins == 0) {
+            for (uint32_t i = 0; i < n; ++i) {
+                bins = BinPlan{};
+                is_binned[i] = bin_plan_add(&bins, level[i], lv, gp, D, F, M);
+                most_bins = std::max(most_bins, bins.room_bins);
+            }
+        }
+        in_boxes = 0;
+        for (uint32_t i = 0; i < n; ++i) binned += (boxed_from[i] > points || in_boxes++ >= kMaxTiled) && is_binned[i];
+        bins.n_levels = std::min(binned, kMaxBinned);
+        bins.room_bins = bins.n_levels * most_bins;
+        bins.n_quads = (bins.room_bins + 3) / 4;
+        bins.batch = (uint32_t)batch;
+        most = std::max(most, bin_scratch_bytes_up_to(bins, D, F));
     };
-    room_for(false, M);
-    room_for(true, M);
-    if (M >= kMoreBinnedBelow) room_for(false, kMoreBinnedBelow - 1); // (what holds a batch holds a smaller one)
+    in_order(M);
+    for (uint32_t i = 0; i < n; ++i)
+        if (boxed_from[i] <= M && boxed_from[i] > 1) in_order(boxed_from[i] - 1);
     return most + 256;
 }
 

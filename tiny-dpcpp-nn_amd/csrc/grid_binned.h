@@ -6,6 +6,7 @@
 namespace tnn {
 
 constexpr uint32_t kMaxBinned = 32;         // levels one launch bins
+constexpr size_t kBinBatch = size_t(1) << 19; // points binned at a time, at most
 constexpr uint32_t kBinMaxBins = 1024;      // bins of a level
 constexpr uint32_t kBinSliceBytes = 128 * 1024; // most of a bin's slice of the table (LDS of a workgroup)
 
@@ -25,7 +26,7 @@ struct BinPlan {
     uint32_t n_levels;
     uint32_t n_bins;                    // of all levels
     uint32_t n_quads;                   // the same in fours of bins
-    uint32_t n_ends;                    // 16-bit numbers of a piece's runs, as bin_launch counts the workspace
+    uint32_t room_bins;                 // bins that the workspace has room for: those that the levels have in a short batch
     uint32_t slice_lds;                 // LDS bytes of the largest slice
     uint32_t batch;                     // points binned at a time
     uint32_t later_bin[kMaxBinned - 1]; // first bin of the second level and those behind it, ~0 where there is none
@@ -35,6 +36,8 @@ struct BinPlan {
 // Adds level l to the plan if it can take the route.
 bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams &gp, uint32_t n_dims, uint32_t n_features, size_t M);
 size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_dims, uint32_t n_features);
+// What the plan's levels need for its batch and for any smaller one.
+size_t bin_scratch_bytes_up_to(BinPlan p, uint32_t n_dims, uint32_t n_features);
 // Nothing in the scratch has to be cleared. With `overwrite` every entry of the plan's levels
 // is written, whatever it held.
 int launch_grid_binned(const BinPlan &p, const GridParams &gp, const GradLayout &dl, uint32_t n_dims, uint32_t n_features, const float *x,

@@ -34,7 +34,6 @@ constexpr int kBinPiecesEach = 4;        // pieces a thread of the sums looks up
 // Copies of the sums of a crowded bin (grid_bin_sum_kernel): at most sixteen, in 8 KB and what keeps an entry's copies in different banks. Bins of more than 4 KB have one.
 constexpr uint32_t kBinCopiesLog2 = 4, kBinCopySkew = 2; // (doubles between two copies)
 constexpr size_t kBinCopiesBytes = 8 * 1024 + (sizeof(double) * kBinCopySkew << kBinCopiesLog2);
-constexpr size_t kBinBatch = size_t(1) << 19; // points binned at a time, at most
 constexpr uint32_t kBinNeighbours = 16;  // consecutive bins on an XCD
 constexpr uint32_t kBinPiecePad = 144; // records between two pieces, at most (bin_launch), so that workgroups in step do not all write to the same channels
 
@@ -450,9 +449,13 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
     // bins: 3-D, 2^19 points 119, 108; 2^18 89, 88; 2^17 51, 57; 2-D, 2^19 66, 67; 2^18 22, 27). Small
     // levels have fewer, large ones as many as it takes for a bin to fit LDS.
     const bool long_bins = (std::min<size_t>(M, kBinBatch) << (n_dims - 1)) >> 8 >= 8192;
-    uint32_t n_log2 = (size >> 7) * entry > (long_bins ? 64 : 32) * 1024 ? 8 : 7;
-    while (n_log2 > 0 && (size >> (n_log2 + 4)) == 0) --n_log2;
-    while (n_log2 < 31 && ((size >> n_log2) * entry > kBinSliceBytes || (size >> n_log2) > 0x7fff)) ++n_log2;
+    const auto bins_log2 = [&](size_t slice) {
+        uint32_t n = (size >> 7) * entry > slice ? 8 : 7;
+        while (n > 0 && (size >> (n + 4)) == 0) --n;
+        while (n < 31 && ((size >> n) * entry > kBinSliceBytes || (size >> n) > 0x7fff)) ++n;
+        return n;
+    };
+    const uint32_t short_log2 = bins_log2(32 * 1024), n_log2 = long_bins ? bins_log2(64 * 1024) : short_log2;
     const size_t bins = (size_t)1 << n_log2;
     if (bins > kBinMaxBins) return false;
     p->batch = (uint32_t)std::min<size_t>(M, kBinBatch);
@@ -475,7 +478,7 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
     else p->later_bin[p->n_levels - 1] = p->n_bins;
     p->at[p->n_levels++] = BinLevel{l, lv.offset[l], lv.size[l], lv.resolution[l], lv.flags[l], lv.scale[l], n_log2, run_log2, (uint32_t)places, copies_log2, p->n_bins, p->n_quads};
     p->n_bins += (uint32_t)bins;
-    p->n_ends += std::max<uint32_t>((uint32_t)bins, (size >> 7) * entry > 32 * 1024 ? 256u : 1u) + 1u;
+    p->room_bins += 1u << short_log2;
     p->n_quads += (uint32_t)((bins + 3) / 4);
     p->slice_lds = std::max<uint32_t>(p->slice_lds, (uint32_t)sums_bytes(copies_log2));
     return true;
@@ -487,21 +490,24 @@ struct BinLaunch {
     uint32_t room, pitch;                   // records that fit its LDS; from one piece to the next
     size_t offset_bytes, scratch_bytes;
 };
+// A batch of fewer points times levels has binning workgroups of half as many threads, and twice as many of them: fewer than two for every CU otherwise.
+template <int D, int F> constexpr size_t kSmallBatch = size_t(512) * BinShape<D, F>::kThreads * BinShape<D, F>::kPoints;
+
 template <int D, int F> static BinLaunch bin_launch(const BinPlan &p) {
     typedef BinShape<D, F> S;
     BinLaunch b;
-    // (a small batch: half as many threads, twice as many workgroups, while there are fewer than two for every CU)
-    b.threads = (size_t)p.batch * p.n_levels < size_t(512) * S::kThreads * S::kPoints ? S::kThreads / 2 : S::kThreads;
+    b.threads = (size_t)p.batch * p.n_levels < kSmallBatch<D, F> ? S::kThreads / 2 : S::kThreads;
     b.stretch = b.threads * S::kPoints;
     b.n_stretches = (p.batch + b.stretch - 1) / b.stretch;
     b.room = b.stretch * S::kPairs / 8 * 9;
-    // The workspace has room for two records a pair of corners (were every far side a record of its own), kBinPiecePad records a piece, and a 16-bit number a bin and
-    // piece. A run takes two such numbers, the second out of the pads (3-D, 2^19 entries: 32 records of 144 a piece).
+    // Room for two records a pair of corners (were every far side a record of its own), and for kBinPiecePad records a piece and two bytes a bin and piece, which hold the table of
+    // runs, four bytes each, and leave the rest between the pieces (3-D, 2^19 entries: 112 records of 144 a piece).
     const size_t pieces = (size_t)p.n_levels * b.n_stretches, least = 2 * b.stretch * S::kPairs;
-    const size_t counted = (((size_t)b.n_stretches * p.n_ends * sizeof(uint16_t) + 255) & ~(size_t)255) + pieces * (least + kBinPiecePad) * sizeof(BinRecord<F>);
+    const size_t room = (((size_t)b.n_stretches * p.room_bins * 2 + 255) & ~(size_t)255) + pieces * (least + kBinPiecePad) * sizeof(BinRecord<F>);
     b.offset_bytes = ((size_t)b.n_stretches * p.n_quads * 4 * sizeof(uint32_t) + 255) & ~(size_t)255;
-    b.pitch = (uint32_t)std::max(least, (counted - b.offset_bytes) / (pieces * sizeof(BinRecord<F>)) / 8 * 8);
-    b.scratch_bytes = std::max(counted, b.offset_bytes + pieces * b.pitch * sizeof(BinRecord<F>));
+    b.pitch = (uint32_t)least;
+    if (room > b.offset_bytes) b.pitch = (uint32_t)std::max(least, (room - b.offset_bytes) / (pieces * sizeof(BinRecord<F>)) / 8 * 8);
+    b.scratch_bytes = std::max(room, b.offset_bytes + pieces * b.pitch * sizeof(BinRecord<F>));
     return b;
 }
 
@@ -515,6 +521,18 @@ size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_dims, uint32_t n_features)
     default: return TNN_BIN_BYTES(8);
     }
 #undef TNN_BIN_BYTES
+}
+
+size_t bin_scratch_bytes_up_to(BinPlan p, uint32_t n_dims, uint32_t n_features) {
+    if (!p.n_levels) return 0;
+    // (the largest batch of small workgroups has twice the pads and tables of a slightly larger one)
+#define TNN_BIN_SMALL(F) (n_dims == 2 ? kSmallBatch<2, F> : kSmallBatch<3, F>)
+    const size_t small = n_features == 1 ? TNN_BIN_SMALL(1) : n_features == 2 ? TNN_BIN_SMALL(2) : n_features == 4 ? TNN_BIN_SMALL(4) : TNN_BIN_SMALL(8);
+#undef TNN_BIN_SMALL
+    const size_t bytes = bin_scratch_bytes(p, n_dims, n_features);
+    if ((size_t)p.batch * p.n_levels < small) return bytes;
+    p.batch = (uint32_t)((small - 1) / p.n_levels);
+    return std::max(bytes, bin_scratch_bytes(p, n_dims, n_features));
 }
 
 template <int D, int F, typename G>
