@@ -108,6 +108,19 @@ def test_workspace_of_8192_rows_of_width_128_holds_fewer(lib):
         assert sizes == sorted(sizes)
 
 
+@pytest.mark.parametrize("width,hidden", [(16, 9), (32, 2), (64, 4), (64, 9), (128, 1), (128, 8)])
+def test_workspace_of_a_batch_holds_fewer_rows(lib, width, hidden):
+    """The partial sums become fewer where a workgroup takes 64 rows more: behind 16384, 32768, ... rows."""
+    from tiny_dpcpp_nn import _lib
+    desc = _lib.MlpDesc(_lib.TNN_FP16, width, hidden, _lib.ACT_RELU, _lib.ACT_NONE)
+    rows = sorted({8, 64, 4096, 24576, 200000} | {k * 8192 + e for k in range(1, 33) for e in (-8, 0, 8)})
+    for query in (lib.tnn_mlp_backward_workspace_bytes, lib.tnn_mlp_train_step_workspace_bytes):
+        sizes = [query(ctypes.byref(desc), m) for m in rows]
+        assert sizes == sorted(sizes), [m for m, a, b in zip(rows, sizes, sizes[1:]) if b < a]
+    if (width, hidden) == (128, 8):  # as many partial sums as there are: 128 of nine matrices, and nine of deltas
+        assert lib.tnn_mlp_backward_workspace_bytes(ctypes.byref(desc), 16384) == 9 * 128 * 128 * 4 * 128 + 9 * 16384 * 128 * 2 + 512
+
+
 @pytest.mark.parametrize("dims,features,levels,scale,log2,sides", [
     # the sizes on both sides of each rule of tnn_grid_forward_workspace_bytes: (points, whether by levels)
     (2, 2, 8, 1.5, 19, ((2 ** 14, 0), (2 ** 14 + 1, 0), (2 ** 17, 0), (2 ** 18 - 1, 0), (2 ** 18, 1), (2 ** 19 - 1, 1), (2 ** 19, 0))),

@@ -181,6 +181,23 @@ def test_width_128_backward_of_few_rows(tnn, oracle, dtype, n_hidden, M):
     assert_propagated(tnn.host(dW), rdW, dtype, "dW", scale=ls)
 
 
+@pytest.mark.parametrize("W,n_hidden,rows,fewer", [(128, 2, 16392, 16384), (128, 3, 32776, 32768), (128, 1, 8192, 8184), (64, 9, 16392, 16384)])
+def test_a_workspace_holds_fewer_rows(tnn, W, n_hidden, rows, fewer):
+    """The smaller batch has more partial sums, or as many: it runs in the larger one's workspace, with the weight gradients of a workspace of its own."""
+    rng = np.random.default_rng(3)
+    w = (rng.uniform(-1, 1, (n_hidden + 1, W, W)) / np.sqrt(W)).astype(np.float32)
+    desc = tnn.mlp_desc(FP16, W, n_hidden, "relu", "none")
+    _, pf, pb = tnn.prepare(desc, w)
+    x, g = (tnn.dev_tensor(rng.uniform(-1, 1, (fewer, W)).astype(np.float32), FP16) for _ in range(2))
+    interm = tnn.forward(desc, pf, x)
+    work = torch.empty(tnn.lib.tnn_mlp_backward_workspace_bytes(ctypes.byref(desc), rows), dtype=torch.uint8, device=tnn.dev)
+    dW = torch.empty((n_hidden + 1, W, W), device=tnn.dev)
+    rc = tnn.lib.tnn_mlp_backward(ctypes.byref(desc), pb.data_ptr(), g.data_ptr(), interm.data_ptr(), None, dW.data_ptr(), 1, None, fewer, work.data_ptr(), work.numel(), tnn.stream())
+    assert rc == 0, tnn.lib.tnn_last_error()
+    _, own, _ = tnn.backward(desc, pb, g, interm, want_interm=False, want_dx=False, dw_fp32=True)
+    assert torch.equal(dW, own)
+
+
 def test_closed_forms(tnn, oracle):
     # test/doctest_swiftnet.cpp:44-51,79-96 : constant weights 0.01 with padded input / output
     dtype, W, n_hidden, M = BF16, 64, 2, 16

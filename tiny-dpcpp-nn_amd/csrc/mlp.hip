@@ -677,16 +677,29 @@ static DwPlan dw_plan(const tnn_mlp_desc *d, size_t M) {
     long long rpc = ((long long)M + target_chunks - 1) / target_chunks;
     rpc = (rpc + kDwSlab - 1) / kDwSlab * kDwSlab;
     if (rpc < kDwSlab) rpc = kDwSlab;
-    const auto chunks = [&] { return M ? ((long long)M + rpc - 1) / rpc : 0; };
     p.partials_per_chunk = (W <= 32) ? 4 : 1;
-    // (room for chunks in multiples of 64 rows, however many there are: what holds 8192 rows holds fewer)
-    p.partial_bytes = (size_t)chunks() * p.partials_per_chunk * n_mats * W * W * sizeof(float);
     // At width 128 a workgroup of few rows has a short round and one partial sum like any other: 128 rows where 64 would be half of the chip's workgroups and more
     // (steps of 8 hidden layers, us, chunks in multiples of 64, 128, 256: 1024 rows 84, 89, 106; 4096 88, 93, 110; 8192 100, 97, 112; 16384 113, 107, 116; 2^15 and more the same).
     if (W == 128 && M >= 8192 && rpc < 2 * kDwSlab) rpc = 2 * kDwSlab;
     p.rows_per_chunk = rpc;
-    p.n_chunks = chunks();
+    p.n_chunks = M ? ((long long)M + rpc - 1) / rpc : 0;
+    p.partial_bytes = (size_t)p.n_chunks * p.partials_per_chunk * n_mats * W * W * sizeof(float);
     p.delta_bytes = (size_t)n_mats * M * W * 2;
+    return p;
+}
+
+static size_t backward_bytes(const DwPlan &p) { return ((p.partial_bytes + 255) & ~(size_t)255) + p.delta_bytes + 512; }
+size_t backward_needs(const tnn_mlp_desc *d, size_t M) { return backward_bytes(dw_plan(d, M)); }
+
+// The plan with the most chunks that a batch of up to M rows has: their number falls where the chunks grow by 64 rows.
+static DwPlan dw_plan_up_to(const tnn_mlp_desc *d, size_t M) {
+    DwPlan p = dw_plan(d, M);
+    const auto most = [&](size_t rows) { // the last batch with chunks of that length
+        if (M > rows) p.partial_bytes = std::max(p.partial_bytes, dw_plan(d, rows).partial_bytes);
+    };
+    if (d->width == 128) most(8191);
+    most(size_t(256) * kDwSlab);     // 256 chunks, as many as any batch has,
+    most(size_t(256) * 2 * kDwSlab); // and at width 128, where chunks have 128 rows by then
     return p;
 }
 
@@ -790,7 +803,7 @@ int backward128_from_loss(const tnn_mlp_desc *desc, const void *wprep_bwd, const
                           const void *wprep_fwd_if_no_output, const TrainTail &tail) {
     const DwPlan p = dw_plan(desc, M);
     const size_t partial_rounded = (p.partial_bytes + 255) & ~(size_t)255;
-    const size_t need = partial_rounded + p.delta_bytes + 512;
+    const size_t need = backward_bytes(p);
     if (!workspace || workspace_bytes < need) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
     uintptr_t base = (reinterpret_cast<uintptr_t>(workspace) + 255) & ~(uintptr_t)255;
     float *partials = reinterpret_cast<float *>(base);
@@ -1041,7 +1054,7 @@ TNN_API int tnn_mlp_backward_rows(const tnn_mlp_desc *desc, const void *d_prepar
         return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
     TrainTail tail;
     if ((rc = rows_tail(desc, desc->width, dy_scale, result_scale, d_dW_packed, dW_dtype, M, &tail))) return rc;
-    const size_t need = tnn_mlp_backward_workspace_bytes(desc, M);
+    const size_t need = backward_needs(desc, M);
     if (!d_workspace || workspace_bytes < need) return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
     uintptr_t base = (reinterpret_cast<uintptr_t>(d_workspace) + 255) & ~(uintptr_t)255;
     float *partials = reinterpret_cast<float *>(base);
@@ -1057,8 +1070,7 @@ TNN_API int tnn_mlp_backward_rows(const tnn_mlp_desc *desc, const void *d_prepar
 
 TNN_API size_t tnn_mlp_backward_workspace_bytes(const tnn_mlp_desc *desc, size_t M) {
     if (check_mlp_desc(desc)) return 0;
-    const DwPlan p = dw_plan(desc, M);
-    return ((p.partial_bytes + 255) & ~(size_t)255) + p.delta_bytes + 512;
+    return backward_bytes(dw_plan_up_to(desc, M)); // (what holds a batch holds a smaller one)
 }
 
 TNN_API int tnn_mlp_backward(const tnn_mlp_desc *desc, const void *d_prepared_bwd, const void *d_dLdy,

@@ -38,6 +38,7 @@ int fused_train_step(const tnn_mlp_desc *d, const void *wf, const void *wb, cons
                      hipStream_t s);
 size_t fused_train_workspace_bytes(const tnn_mlp_desc *d, size_t M);
 // mlp.hip
+size_t backward_needs(const tnn_mlp_desc *d, size_t M); // for this batch, where tnn_mlp_backward_workspace_bytes is for smaller ones, too
 int forward128_for_training(const tnn_mlp_desc *desc, const void *wprep, const void *x, void *interm_fwd, size_t M, hipStream_t s, bool without_output);
 int backward128_from_loss(const tnn_mlp_desc *desc, const void *wprep_bwd, const void *x, const void *interm_fwd, const float *targets, float loss_scale,
                           float *loss_sum, void *dW, int dW_is_fp32, void *dLdx, size_t M, void *workspace, size_t workspace_bytes, hipStream_t s,
@@ -47,14 +48,18 @@ int backward128_from_loss(const tnn_mlp_desc *desc, const void *wprep_bwd, const
 
 using namespace tnn;
 
-TNN_API size_t tnn_mlp_train_step_workspace_bytes(const tnn_mlp_desc *desc, size_t M) {
-    if (check_mlp_desc(desc)) return 0;
+static size_t step_bytes(const tnn_mlp_desc *desc, size_t M, size_t backward) {
     const size_t fused = fused_train_workspace_bytes(desc, M);
     if (fused) return fused;
     const size_t mat = M * desc->width * 2;
     // activations, dL/dy, the backward pass's own workspace, and fp32 weight gradients for tnn_mlp_train_step_l2_adam
-    return align256((size_t)(desc->n_hidden_layers + 2) * mat) + align256(mat) + align256(tnn_mlp_backward_workspace_bytes(desc, M)) +
-           align256(unfused_dw_bytes(desc)) + 512;
+    return align256((size_t)(desc->n_hidden_layers + 2) * mat) + align256(mat) + align256(backward) + align256(unfused_dw_bytes(desc)) + 512;
+}
+static size_t step_needs(const tnn_mlp_desc *desc, size_t M) { return step_bytes(desc, M, backward_needs(desc, M)); }
+
+TNN_API size_t tnn_mlp_train_step_workspace_bytes(const tnn_mlp_desc *desc, size_t M) {
+    if (check_mlp_desc(desc)) return 0;
+    return step_bytes(desc, M, tnn_mlp_backward_workspace_bytes(desc, M));
 }
 
 static int unfused_train_step(const tnn_mlp_desc *desc, const void *d_prepared_fwd, const void *d_prepared_bwd, const void *d_x, const float *d_targets,
@@ -69,7 +74,7 @@ TNN_API int tnn_mlp_train_step_l2(const tnn_mlp_desc *desc, const void *d_prepar
     if (rc) return rc;
     if (!d_prepared_fwd || !d_prepared_bwd || !d_x || !d_targets || !d_dW) return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
     if (loss_scale == 0.0f) return fail(TNN_ERR_INVALID_ARGUMENT, "loss_scale must not be 0");
-    const size_t need = tnn_mlp_train_step_workspace_bytes(desc, M);
+    const size_t need = step_needs(desc, M);
     if (!d_workspace || workspace_bytes < need)
         return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
     hipStream_t s = as_stream(stream);
@@ -97,7 +102,7 @@ static int unfused_train_step(const tnn_mlp_desc *desc, const void *d_prepared_f
     void *dLdy = reinterpret_cast<void *>(base);
     base += align256(mat);
     void *bwd_ws = reinterpret_cast<void *>(base);
-    const size_t bwd_ws_bytes = align256(tnn_mlp_backward_workspace_bytes(desc, M));
+    const size_t bwd_ws_bytes = align256(backward_needs(desc, M));
 
     // width 128 when nobody asks for the network's output: the forward pass ends at the last hidden layer and the backward
     // pass's first launch forms the output again on chip (one matrix less to write and to read)
@@ -135,7 +140,7 @@ TNN_API int tnn_mlp_train_step_l2_adam(const tnn_mlp_desc *desc, void *d_prepare
         return fail(TNN_ERR_INVALID_ARGUMENT, "NULL pointer argument");
     if (loss_scale == 0.0f) return fail(TNN_ERR_INVALID_ARGUMENT, "loss_scale must not be 0");
     if (step < 1) return fail(TNN_ERR_INVALID_ARGUMENT, "step counts from 1");
-    const size_t need = tnn_mlp_train_step_workspace_bytes(desc, M);
+    const size_t need = step_needs(desc, M);
     if (!d_workspace || workspace_bytes < need)
         return fail(TNN_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
     if (M == 0 || (M % 8) != 0) return fail(TNN_ERR_INVALID_ARGUMENT, "batch size %zu is not a positive multiple of 8", M);
@@ -269,7 +274,7 @@ TNN_API int tnn_mlp_train_step_l2_static(const tnn_mlp_desc *desc, const void *d
                                          void *d_dW, int dW_is_fp32, void *d_dLdx, size_t M, tnn_stream_t stream) {
     int rc = check_mlp_desc(desc);
     if (rc) return rc;
-    const size_t need = tnn_mlp_train_step_workspace_bytes(desc, M);
+    const size_t need = step_needs(desc, M);
     if (need > kStaticScratchBytes)
         return fail(TNN_ERR_WORKSPACE,
                     "this shape and batch size need %zu bytes of scratch memory, the static buffer holds %zu: use "
