@@ -242,8 +242,8 @@ def test_binned_workspace_is_checked(tnn):
 @pytest.mark.parametrize("M", [28001, 32003, 60001, 64007, 80009])
 @pytest.mark.parametrize("features", [1, 2, 8])
 def test_sums_with_few_and_many_records_a_lane(tnn, oracle, M, features):
-    """Two to six rounds of records of an even spread, which choose how many a lane has in flight; several bins a workgroup, whose sums start from zero for each; and
-    levels whose last entries fill a bin's last pair or not. fp32 results of double sums: the bar of the plain scatter."""
+    """Two to six rounds of records of an even spread, which choose how many a lane has in flight, and levels whose last entries fill a bin's last pair or not. fp32 results
+    of double sums: the bar of the plain scatter."""
     cfg = dict(CFG2, n_features_per_level=features, n_levels=16 if features <= 2 else 10)
     rng = np.random.default_rng(M + features)
     x = rng.uniform(0, 1, (M, 2)).astype(np.float32)
@@ -252,6 +252,24 @@ def test_sums_with_few_and_many_records_a_lane(tnn, oracle, M, features):
     ref = oracle.grid_backward(cfg, x, g, tnn.grid_n_params(d))
     grad = binned(tnn, d, torch.from_numpy(x).to(tnn.dev), torch.from_numpy(g).to(tnn.dev), FP32)
     assert np.abs(grad.cpu().numpy() - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
+
+
+@pytest.mark.parametrize("features,log2,levels,M", [(1, 19, 16, 8192), (2, 19, 16, 8209), (2, 19, 16, 16384), (4, 17, 16, 8191), (8, 17, 12, 8191)])
+@pytest.mark.parametrize("crowd", [0, 5000])
+def test_workgroups_that_stay_for_several_bins(tnn, oracle, features, log2, levels, M, crowd):
+    """Bins of 256 records at most, 128 with eight features, and 1500 to 3000 of them, 32 KB each, where 256 CUs hold four workgroups: the sums start from zero for each, also behind a
+    long bin, with copies, of points in one cell. The bar of the plain scatter."""
+    cfg = dict(CFG3, n_features_per_level=features, log2_hashmap_size=log2, n_levels=levels)
+    rng = np.random.default_rng(M + features)
+    x = rng.uniform(0, 1, (M, 3)).astype(np.float32)
+    x[rng.permutation(M)[:crowd]] = 0.4321
+    d = tnn.grid_desc(cfg)
+    g = rng.standard_normal((M, levels * features)).astype(np.float32)
+    ref = oracle.grid_backward(cfg, x, g, tnn.grid_n_params(d))
+    table = torch.full((tnn.grid_n_params(d),), 0.5, device=tnn.dev)
+    for overwrite in (True, False):
+        grad = binned(tnn, d, torch.from_numpy(x).to(tnn.dev), torch.from_numpy(g).to(tnn.dev), FP32, grad=table.clone(), overwrite=overwrite)
+        assert np.abs(grad.cpu().numpy() - (0 if overwrite else 0.5) - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
 
 
 @pytest.mark.parametrize("features", [1, 2, 4])
