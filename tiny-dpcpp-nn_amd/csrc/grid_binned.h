@@ -28,6 +28,7 @@ struct BinPlan {
     uint32_t n_quads;                   // the same in fours of bins
     uint32_t room_bins;                 // bins that the workspace has room for: those that the levels have in a short batch
     uint32_t slice_lds;                 // LDS bytes of the largest slice
+    uint32_t sums_lds;                  // the same with copies of short slices
     uint32_t batch;                     // points binned at a time
     uint32_t later_bin[kMaxBinned - 1]; // first bin of the second level and those behind it, ~0 where there is none
     BinLevel at[kMaxBinned];

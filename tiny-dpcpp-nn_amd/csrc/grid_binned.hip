@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(kBinSumThreads, F <= 2 ? 8 : 4)
     constexpr uint32_t kWaves = kBinSumThreads / 64, kGroup = kBinSumGroup;
     constexpr int kEach = kBinPiecesEach;
     extern __shared__ __align__(16) double sums[];
-    uint32_t *const wave_sum = reinterpret_cast<uint32_t *>(sums + bp.slice_lds / sizeof(double));
+    uint32_t *const wave_sum = reinterpret_cast<uint32_t *>(sums + bp.sums_lds / sizeof(double));
     uint32_t *const wave_runs = wave_sum + kWaves;
     uint32_t *const group_run = wave_runs + kWaves;       // run that a group's first record is in
     uint32_t *const first = group_run + kBinSumThreads / kGroup; // records in front of a run
@@ -349,13 +349,15 @@ __global__ void __launch_bounds__(kBinSumThreads, F <= 2 ? 8 : 4)
             }
         }
         if (threadIdx.x == 0) first[n_runs] = total;
+        // Of a bin with more than eight records a lane, whose points are crowded where even ones leave it a fraction of that, neighbouring lanes add to copies of their own.
+        const uint32_t copies = total > 8 * blockDim.x ? 1u << at_level.copies_log2 : 1u, copy = n * F + kBinCopySkew;
+        if (copies > 1)
+            for (uint32_t e = n * F + threadIdx.x; e < copies * copy; e += blockDim.x) sums[e] = 0.0;
         const uint32_t next = bin_of(block);
         if (next < bp.n_bins) look_up(next);
         __syncthreads();
         const BinRecord<F> *const rec = records + (size_t)k * n_stretches * pitch;
         const uint32_t group = threadIdx.x / kGroup, end = (group + 1) * share < total ? (group + 1) * share : total;
-        // Of a bin with more than eight records a lane, whose points are crowded where even ones leave it a fraction of that, neighbouring lanes add to copies of their own.
-        const uint32_t copies = total > 8 * blockDim.x ? 1u << at_level.copies_log2 : 1u, copy = n * F + kBinCopySkew;
         double *const own = sums + (threadIdx.x & (copies - 1)) * copy;
         uint32_t i = group * share + threadIdx.x % kGroup, s = i < end ? group_run[group] : 0u;
         for (; i < end; i += kAhead * kGroup) {
@@ -480,7 +482,8 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
     p->n_bins += (uint32_t)bins;
     p->room_bins += 1u << short_log2;
     p->n_quads += (uint32_t)((bins + 3) / 4);
-    p->slice_lds = std::max<uint32_t>(p->slice_lds, (uint32_t)sums_bytes(copies_log2));
+    p->slice_lds = std::max<uint32_t>(p->slice_lds, (uint32_t)sums_bytes(0));
+    p->sums_lds = std::max<uint32_t>(p->sums_lds, (uint32_t)sums_bytes(copies_log2));
     return true;
 }
 
@@ -546,7 +549,7 @@ static int launch_binned(const BinPlan &p, const GridParams &gp, const GradLayou
     for (uint32_t k = 0; k < p.n_levels; ++k) most_bins = std::max(most_bins, 1u << p.at[k].bins_log2);
     const auto bin = grid_bin_kernel<D, F, G>;
     const size_t bin_lds = (size_t)b.room * sizeof(BinRecord<F>) + (2 * most_bins + 16) * sizeof(uint32_t);
-    const size_t sum_lds = p.slice_lds + (2 * kBinSumThreads / 64 + kBinSumThreads / kBinSumGroup + 2 * b.n_stretches + 1) * sizeof(uint32_t);
+    const size_t sum_lds = p.sums_lds + (2 * kBinSumThreads / 64 + kBinSumThreads / kBinSumGroup + 2 * b.n_stretches + 1) * sizeof(uint32_t);
     // (about as many waves on a CU as it holds, whatever LDS the bins need: small bins are over before many are under way)
     unsigned sum_threads = p.slice_lds > 48 * 1024 ? kBinSumThreads : p.slice_lds > 20 * 1024 ? kBinSumThreads / 2 : kBinSumThreads / 4;
     while (sum_threads * kBinPiecesEach < b.n_stretches) sum_threads *= 2;
