@@ -601,7 +601,7 @@ class Bench:
     def leg_train_w128(self):
         # BASELINE config 3's widest network: width 128, 8 hidden layers, fp16, 2^20 rows. Its nine matrices do not fit one
         # kernel: a forward pass that stores the activations, the top layer's backward launch with the loss in it, then
-        # one backward launch per two layers. Parity at this size: tests/test_gpu_mlp.py::test_baseline_config_3_full_size.
+        # one backward launch for the layers below it. Parity at this size: tests/test_gpu_mlp.py::test_baseline_config_3_full_size.
         np, torch, t, lib = self.np, self.torch, self.t, self.lib
         from tiny_dpcpp_nn.cabi import ptr
         from tolerances import FP16, FP32
@@ -641,7 +641,7 @@ class Bench:
         roof = {"bound": "mfma", "achieved": ach, "peak": PEAK_MFMA_BF16, "unit": "TFLOP/s", "frac": ach / PEAK_MFMA_BF16,
                 "traffic": MEASURED_TRAFFIC_BYTES.get(("train_w128", lg)),
                 "kernel": "whole step: mlp_forward_stream_kernel, mlp_layer_backward128_kernel (top layer + loss), "
-                          "mlp_layer_pair_backward128_kernel x (n_hidden / 2), train_reduce_kernel (with Adam)",
+                          "mlp_layer_pairs_backward128_kernel (all layers below), train_reduce_kernel (with Adam)",
                 "kernel_ms": tm["ms"], "algorithmic_flops_per_launch": flops}
         return line("fused-MLP training samples/s (w128, 8 hidden layers, fp16, batch 2^20); % fp16 MFMA peak", "samples/s", "f16",
                     f"training step: w128, 8 hidden layers (9 matmuls), ReLU/linear, fp16, batch 2^{lg}, L2 loss, Adam on fp32 masters (BASELINE config 3, widest)",

@@ -664,7 +664,8 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
     // in the end: a level of more entries than a chunk has contributions is binned, too (whole scatter, 2-D, 2^16 points, 2^15 entries 37.8 -> 32.9 us;
     // 2^15 points, 2^19 entries 39.3 either way), and in three dimensions, where that leaves none as a rule and so a launch less, one of more than
     // a quarter as many (20 000 points 52 -> 42.5; 2^16 63.5 -> 54.5; 2^17 93 -> 94; with that rule in two
-    // dimensions 2^16 points 35.9). The records of such levels take memory: batches that need more of it for them than 2^17 points do
+    // dimensions 2^16 points 35.9; points in a square or cube of 5 % of the side, which meet few of such a level's entries, 2^16 points 2-D 84 -> 72,
+    // 3-D 312 -> 218, since crowded bins have copies of their sums, 120 and 393 without). The records of such levels take memory: batches that need more of it for them than 2^17 points do
     // without (16 levels in 3-D: 122 880 points), and that many and more, for which 2^18 points would gain 4 of 81, do not have them.
     if (!ordered && !nearest && bin_others() && gp.n_levels <= kMaxBinned) {
         const size_t without = n_big;

@@ -17,8 +17,8 @@
 // make some bins longer than others, and that is all. (Bins of a fixed size, filled by all workgroups through shared cursors, are
 // as fast for points spread evenly, but what finds no room has to go elsewhere. 2^20 points, 3-D, 2^19 entries, whole scatter, from
 // points in the inner 90 % of the cube / in a cube of 5 % of the side: the overfull bins summed from the points 4.0 / 5.8 ms, the surplus
-// added with atomics 0.76 / 36 ms, pieces 0.75 / 3.9 ms; evenly spread 0.74, 0.76 and 0.75 ms.)
-// Measured, 2^20 points, 3-D, 2^19 entries, the ten finest levels: 2 x (98 + 96) us; as atomics 1.5 ms.
+// added with atomics 0.76 / 36 ms, pieces 0.75 / 3.9 ms; evenly spread 0.74, 0.76 and 0.75 ms. Pieces now: 0.54 / 3.1 ms, evenly spread 0.54.)
+// Measured, 2^20 points, 3-D, 2^19 entries, the ten finest levels: 2 x (99 + 97) us; as atomics 1.5 ms.
 #include "grid_binned.h"
 #include "mlp_tile.h"
 
@@ -138,7 +138,7 @@ __device__ __forceinline__ uint32_t running_sum(uint32_t mine, uint32_t *__restr
     return upto - mine + sums_in_front(wave_sum, total);
 }
 
-// Where a bin's records in a piece begin and end (two 16-bit numbers): by four bins, then by pieces. A workgroup of the sums reads its bin's
+// Where a bin's records in a piece begin and end (two 16-bit numbers, side by side in a word): by four bins, then by pieces. A workgroup of the sums reads its bin's
 // of all pieces, eight pieces to a line that it shares with three neighbouring bins; with all bins of a piece side by side it read a
 // line for each (3-D, 2^19 points, 10 levels: 123.5 us, now 119; 2^18 in the caller's order 95, 89).
 __device__ __forceinline__ size_t run_slot(uint32_t first_quad, uint32_t bin, uint32_t n_stretches, uint32_t stretch) {
@@ -150,8 +150,8 @@ __device__ __forceinline__ size_t run_slot(uint32_t first_quad, uint32_t bin, ui
 // lies in another bin than the near side is a record of its own; LDS has room for one in eight, those beyond go to the
 // piece directly. The levels of the same points are consecutive workgroups of one XCD, which shares the rows of dL/dy between
 // them in its L2.
-// No one unit bounds it (3-D, 2^19 points, 15 levels, 161 us): 507 MB written, all in whole 64-byte requests, at 3.1 TB/s where a
-// fill reaches 6.9; the vector units are at work half of the time, LDS a quarter, and a wave waits for 43 % of its.
+// No one unit bounds it (3-D, 2^19 points, 10 levels, 99 us): 346 MB written, the records all in whole 64-byte requests, at 3.5 TB/s where a
+// fill reaches 6.9; the vector units are at work 45 % of the time, LDS a sixth, and a wave waits for 41 % of its.
 template <int D, int F, typename G>
 __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
     grid_bin_kernel(const GridParams gp, const BinPlan bp, const GradLayout dl, const float *__restrict__ xin,
@@ -266,7 +266,7 @@ __global__ void __launch_bounds__((BinShape<D, F>::kThreads))
 // 2^18 points), then the bin that lies a grid further on. The bin's runs of records in the pieces follow each other here (`first`: records in front of a
 // piece's run); eight lanes take an equal share of them all, whatever the runs' lengths, and walk from run to run. Neighbouring bins, whose
 // runs share lines, are workgroups of one XCD, sixteen at a time. kAhead: records of a lane in flight.
-// Long bins are bound by the LDS atomics, two entries of F values a record. Short ones were bound by what comes before the first record: a workgroup a
+// Long bins are bound by the LDS atomics, two entries of F values a record (3-D, 2^19 points, 10 levels, 97 us: LDS at work 66 % of the time, 490 MB read). Short ones were bound by what comes before the first record: a workgroup a
 // bin, 3-D, 2^15 points, took 30 us, 18 of them without a record read or an entry written. So a workgroup stays for several of the shortest (launch_binned): where the next bin's
 // runs lie is loaded while this one's records are summed, and sums are cleared as they are read. What was left of it were instructions, eight and more waves a bin of them:
 // the prefix sums over the waves are a value a lane, a wave without pieces leaves the look-up out, and two entries leave together (3-D, 2^15 points 30 -> 20.3 us,

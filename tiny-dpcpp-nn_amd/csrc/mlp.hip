@@ -715,7 +715,8 @@ static int launch_dw(const tnn_mlp_desc *d, const void *interm_bwd, const void *
     return launch_train_reduce<T>(partials, nullptr, (int)(p.n_chunks * p.partials_per_chunk), n_mats * W * W, dW, dW_is_fp32, nullptr, TrainTail{}, s);
 }
 
-// Width 128: one launch per layer that forms delta_{l-1} and dW_l together (mlp_backward128.inc), then the reduction.
+// Width 128: delta_{l-1} and dW_l together (mlp_backward128.inc), one launch for the top layer, one for the pairs of layers below it and, with an odd
+// number of those, one for the first matrix, then the reduction.
 // With `targets` the top layer's launch forms dL/dy itself from the network's output (the last matrix of interm_fwd) and leaves
 // the loss values as one sum per workgroup, which the reduction adds into *loss_sum; dLdy is then not read, and `tail` may ask
 // for Adam on the reduced gradients inside the reduction (dW may then be null).
