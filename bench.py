@@ -640,8 +640,8 @@ class Bench:
         ach = flops / (tm["ms"] * 1e-3) / 1e12
         roof = {"bound": "mfma", "achieved": ach, "peak": PEAK_MFMA_BF16, "unit": "TFLOP/s", "frac": ach / PEAK_MFMA_BF16,
                 "traffic": MEASURED_TRAFFIC_BYTES.get(("train_w128", lg)),
-                "kernel": "whole step: mlp_forward_stream_kernel, mlp_layer_backward128_kernel (top layer + loss), "
-                          "mlp_layer_pairs_backward128_kernel (all layers below), train_reduce_kernel (with Adam)",
+                "kernel": "whole step: mlp_forward_stream_kernel, mlp_layers_backward128_kernel (loss and all layers' "
+                          "backward passes), train_reduce_kernel (with Adam)",
                 "kernel_ms": tm["ms"], "algorithmic_flops_per_launch": flops}
         return line("fused-MLP training samples/s (w128, 8 hidden layers, fp16, batch 2^20); % fp16 MFMA peak", "samples/s", "f16",
                     f"training step: w128, 8 hidden layers (9 matmuls), ReLU/linear, fp16, batch 2^{lg}, L2 loss, Adam on fp32 masters (BASELINE config 3, widest)",

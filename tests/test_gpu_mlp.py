@@ -158,7 +158,7 @@ def test_backward_parity_widths(tnn, oracle, dtype, W, n_hidden):
 
 @pytest.mark.parametrize("dtype,n_hidden,M", [(FP16, 1, 8), (BF16, 2, 8), (FP16, 4, 72), (BF16, 5, 200), (FP16, 8, 264), (BF16, 3, 8192 + 40), (FP16, 2, 16384 + 72)])
 def test_width_128_backward_of_few_rows(tnn, oracle, dtype, n_hidden, M):
-    """All pairs of layers in one launch, with the bottom layer in a pair or alone (an odd number of hidden layers leaves an odd
+    """All layers in one launch, with the bottom layer in a pair or alone (an odd number of hidden layers leaves an odd
     number below the top one), workgroups of 64 and 128 rows, rounds that end in the middle of a wave's tile and waves without rows. With the
     deltas kept and without: the same weight gradients, which are a plain product of the kept deltas and the activations."""
     W, n_mats = 128, n_hidden + 1
@@ -179,6 +179,37 @@ def test_width_128_backward_of_few_rows(tnn, oracle, dtype, n_hidden, M):
         assert_close(tnn.host(dW[l]), gib[l].astype(np.float64).T @ interm[l].astype(np.float64), dtype, f"dW[{l}] from the GPU's own deltas", scale=ls)
     assert_propagated(tnn.host(dX), rdX, dtype, "dL/dx", scale=ls / M)
     assert_propagated(tnn.host(dW), rdW, dtype, "dW", scale=ls)
+
+
+@pytest.mark.parametrize("n_hidden,M", [(1, 131072 + 8), (2, 65536), (3, 65536 + 8), (4, 131072), (5, 131072 + 8), (8, 196608 + 64)])
+def test_width_128_rounds_of_layers_take_turns(tnn, n_hidden, M):
+    """One, two, three and four rounds of 256 rows a workgroup, whole and ragged: every other pair of layers takes them from the last one on, and the deltas of the
+    round where they turn stay in registers. A row's deltas and dL/dx are those of the same row in a batch of one round, bit for bit, whether the deltas
+    are kept or not. dW is an fp32 sum of M products in shares of at most 1024 rows and up to 256 shares: its error is at most (1024 + 256) half units of the last place of
+    the sum of their absolute values."""
+    W, n_mats = 128, n_hidden + 1
+    gen = torch.Generator(device=tnn.dev).manual_seed(n_hidden)
+    rng = np.random.default_rng(21)
+    w = (rng.uniform(-1, 1, (n_mats, W, W)) * np.sqrt(3.0 / W)).astype(np.float32)
+    desc = tnn.mlp_desc(FP16, W, n_hidden, "relu", "none")
+    _, pf, pb = tnn.prepare(desc, w)
+    x = (torch.rand((M, W), device=tnn.dev, generator=gen) * 2 - 1).to(torch.float16)
+    g = (torch.rand((M, W), device=tnn.dev, generator=gen) * 2 - 1).to(torch.float16)
+    interm = tnn.forward(desc, pf, x).view(n_mats + 1, M, W)
+    deltas, dW, dX = tnn.backward(desc, pb, g, interm, dw_fp32=True)
+    _, dW2, dX2 = tnn.backward(desc, pb, g, interm, want_interm=False, dw_fp32=True)
+    assert torch.equal(dW, dW2) and torch.equal(dX.view(torch.int16), dX2.view(torch.int16))
+    _, dW3, _ = tnn.backward(desc, pb, g, interm, want_interm=False, want_dx=False, dw_fp32=True)
+    assert torch.equal(dW, dW3)
+    deltas = deltas.view(n_mats, M, W)
+    for at in range(0, M, 65536):
+        rows = slice(at, min(at + 65536, M))
+        part, _, part_dX = tnn.backward(desc, pb, g[rows].contiguous(), interm[:, rows].contiguous(), dw_fp32=True)
+        assert torch.equal(part.view(n_mats, -1, W).view(torch.int16), deltas[:, rows].view(torch.int16))
+        assert torch.equal(part_dX.view(torch.int16), dX[rows].view(torch.int16))
+    for l in range(n_mats):
+        d, a = deltas[l].double(), interm[l].double()
+        assert ((dW[l].double() - d.t() @ a).abs() <= (1024 + 256) * 2.0 ** -24 * (d.abs().t() @ a.abs())).all(), l
 
 
 @pytest.mark.parametrize("W,n_hidden,rows,fewer", [(128, 2, 16392, 16384), (128, 3, 32776, 32768), (128, 1, 8192, 8184), (64, 9, 16392, 16384)])
@@ -554,7 +585,7 @@ def test_baseline_config_3_full_size(tnn, oracle, W, n_hidden):
                                                           (FP16, 2, "sigmoid", "none", (1 << 17) + 8), (BF16, 5, "relu", "relu", (1 << 16) + 2048)])
 def test_width_128_step_without_stored_output(tnn, oracle, dtype, n_hidden, act, out_act, M):
     """A width-128 training step that is not asked for the network's output ends its forward pass at the last hidden layer;
-    the top launch of its backward pass forms the output again with the forward pass's arithmetic. Everything it returns
+    its backward pass forms the output again with the forward pass's arithmetic. Everything it returns
     must be what the step with the output stored returns: dL/dx bit for bit, the weight gradients bit for bit as well (same
     partial sums over the same values), the loss to the rounding of its sum. Odd and even numbers of matrices (the bottom
     layer alone or in a pair), ragged last rounds, every output activation; the batch sizes are those of the streaming

@@ -715,16 +715,16 @@ static int launch_dw(const tnn_mlp_desc *d, const void *interm_bwd, const void *
     return launch_train_reduce<T>(partials, nullptr, (int)(p.n_chunks * p.partials_per_chunk), n_mats * W * W, dW, dW_is_fp32, nullptr, TrainTail{}, s);
 }
 
-// Width 128: delta_{l-1} and dW_l together (mlp_backward128.inc), one launch for the top layer, one for the pairs of layers below it and, with an odd
+// Width 128: delta_{l-1} and dW_l together (mlp_backward128.inc), one launch for the top layer and the pairs of layers below it and, with an odd
 // number of those, one for the first matrix, then the reduction.
-// With `targets` the top layer's launch forms dL/dy itself from the network's output (the last matrix of interm_fwd) and leaves
+// With `targets` the launch forms dL/dy itself from the network's output (the last matrix of interm_fwd) and leaves
 // the loss values as one sum per workgroup, which the reduction adds into *loss_sum; dLdy is then not read, and `tail` may ask
 // for Adam on the reduced gradients inside the reduction (dW may then be null).
 template <typename T>
 static int launch_backward128(const tnn_mlp_desc *d, const void *wprep_bwd, const void *dLdy, const void *interm_fwd, void *deltas,
                               bool keep_top_delta, void *dW, int dW_is_fp32, void *dLdx, size_t M, float *partials, hipStream_t s,
                               const float *targets = nullptr, float loss_scale = 0.0f, float *loss_sum = nullptr, const void *x0 = nullptr,
-                              const void *wprep_fwd = nullptr, // (with targets): the network's output is not in interm_fwd, the top launch forms it
+                              const void *wprep_fwd = nullptr, // (with targets): the network's output is not in interm_fwd, the launch forms it
                               const TrainTail &tail = TrainTail{}, const void *y = nullptr) { // y: the network's output, null: behind the activations
     typedef typename Storage<T>::vec8 vec8;
     constexpr int W = 128;
@@ -732,16 +732,12 @@ static int launch_backward128(const tnn_mlp_desc *d, const void *wprep_bwd, cons
     const DwPlan p = dw_plan(d, M);
     const size_t mat = M * W, per_mat = (size_t)4 * 8 * 64;
     const bool reform = targets && wprep_fwd;
-    auto k_top = reform ? mlp_layer_backward128_kernel<T, 3> : (targets ? mlp_layer_backward128_kernel<T, 2> : mlp_layer_backward128_kernel<T, 1>);
-    auto k_mid = mlp_layer_backward128_kernel<T, 0>;
-    auto k_pairs = mlp_layer_pairs_backward128_kernel<T>;
+    auto k_bottom = mlp_bottom_layer_backward128_kernel<T>;
+    auto k_all = reform ? mlp_layers_backward128_kernel<T, 3> : (targets ? mlp_layers_backward128_kernel<T, 2> : mlp_layers_backward128_kernel<T, 1>);
     const float inv_n = 1.0f / (float)(M * W);
-    const size_t top_lds = reform ? LayerBwd128::pair_lds_bytes : LayerBwd128::lds_bytes;
-    if (!reserve_lds(reinterpret_cast<const void *>(k_top), top_lds))
-        return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", top_lds);
-    if (!reserve_lds(reinterpret_cast<const void *>(k_mid), LayerBwd128::lds_bytes))
+    if (!reserve_lds(reinterpret_cast<const void *>(k_bottom), LayerBwd128::lds_bytes))
         return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", LayerBwd128::lds_bytes);
-    if (!reserve_lds(reinterpret_cast<const void *>(k_pairs), LayerBwd128::pair_lds_bytes))
+    if (!reserve_lds(reinterpret_cast<const void *>(k_all), LayerBwd128::pair_lds_bytes))
         return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", LayerBwd128::pair_lds_bytes);
     const T *fwd = static_cast<const T *>(interm_fwd);
     const T *input0 = x0 ? static_cast<const T *>(x0) : fwd; // the first matrix's input: the caller's x, or its copy in front of the activations
@@ -751,30 +747,19 @@ static int launch_backward128(const tnn_mlp_desc *d, const void *wprep_bwd, cons
                                ? reinterpret_cast<float *>(dl + (size_t)(n_mats - 1) * mat) : (float *)nullptr;
     if (targets && loss_sum && !loss_partials) return fail(TNN_ERR_INVALID_ARGUMENT, "no room for the loss sums of %lld workgroups", p.n_chunks);
     const vec8 *wb = static_cast<const vec8 *>(wprep_bwd);
-    // the top layer by itself (it turns dL/dy or the loss into deltas first), then the layers below it two at a time in one launch, and
-    // the first matrix by itself when their number is odd
-    int l = n_mats - 1;
-    while (l >= 0) {
-        const bool top = (l == n_mats - 1);
-        if (!top && l >= 1) {
-            TNN_LAUNCH(k_pairs, dim3((unsigned)p.n_chunks), dim3(kLayerBwdThreads), LayerBwd128::pair_lds_bytes, s, wb, dl, fwd, input0, static_cast<T *>(dLdx),
-                       keep_top_delta ? 1 : 0, partials, n_mats, l, d->activation, tail.result_scale, (long long)M, p.rows_per_chunk);
-            const int rc = check_launch("mlp_layer_pairs_backward128_kernel");
-            if (rc) return rc;
-            l = (l & 1) ? -1 : 0;
-            continue;
-        }
-        const T *delta_in = top ? static_cast<const T *>(dLdy) : dl + (size_t)l * mat;
-        T *delta_out = l > 0 ? dl + (size_t)(l - 1) * mat : static_cast<T *>(dLdx);
-        const int gate = l > 0 ? d->activation : TNN_ACT_NONE;
-        TNN_LAUNCH((top ? k_top : k_mid), dim3((unsigned)p.n_chunks), dim3(kLayerBwdThreads), top ? top_lds : LayerBwd128::lds_bytes, s,
-                   wb + (size_t)l * per_mat, delta_in, l > 0 ? fwd + (size_t)l * mat : input0, y ? static_cast<const T *>(y) : fwd + (size_t)n_mats * mat,
-                   (top && keep_top_delta) ? dl + (size_t)l * mat : (T *)nullptr, delta_out, partials, n_mats, l, gate, d->output_activation, (long long)M,
-                   p.rows_per_chunk, targets, targets ? loss_scale : tail.dy_scale, inv_n, loss_partials, l > 0 ? 1.0f : tail.result_scale,
-                   (top && reform) ? static_cast<const vec8 *>(wprep_fwd) + (size_t)l * per_mat : (const vec8 *)nullptr);
-        const int rc = check_launch("mlp_layer_backward128_kernel");
-        if (rc) return rc;
-        l -= 1;
+    const T *top_y = y ? static_cast<const T *>(y) : fwd + (size_t)n_mats * mat;
+    // the top layer (it turns dL/dy or the loss into deltas first) and the layers below it two at a time in one launch, and the first
+    // matrix by itself when the number of layers below the top one is odd
+    TNN_LAUNCH(k_all, dim3((unsigned)p.n_chunks), dim3(kLayerBwdThreads), LayerBwd128::pair_lds_bytes, s, wb, static_cast<const T *>(dLdy), top_y, dl, fwd, input0,
+               static_cast<T *>(dLdx), keep_top_delta ? 1 : 0, partials, n_mats, d->activation, d->output_activation, tail.result_scale, (long long)M,
+               p.rows_per_chunk, targets, targets ? loss_scale : tail.dy_scale, inv_n, loss_partials,
+               reform ? static_cast<const vec8 *>(wprep_fwd) + (size_t)(n_mats - 1) * per_mat : (const vec8 *)nullptr);
+    int rc = check_launch("mlp_layers_backward128_kernel");
+    if (rc) return rc;
+    if (n_mats % 2 == 0) {
+        TNN_LAUNCH(k_bottom, dim3((unsigned)p.n_chunks), dim3(kLayerBwdThreads), LayerBwd128::lds_bytes, s, wb, dl, input0, static_cast<T *>(dLdx), partials,
+                   n_mats, (long long)M, p.rows_per_chunk, tail.result_scale);
+        if ((rc = check_launch("mlp_bottom_layer_backward128_kernel"))) return rc;
     }
     if (tail.main_done && hipEventRecord(tail.main_done, s) != hipSuccess) return fail(TNN_ERR_HIP, "hipEventRecord failed");
     return launch_train_reduce<T>(partials, loss_partials, (int)p.n_chunks, n_mats * W * W, dW, dW_is_fp32, loss_partials ? loss_sum : nullptr, tail, s);
@@ -782,7 +767,7 @@ static int launch_backward128(const tnn_mlp_desc *d, const void *wprep_bwd, cons
 
 // For tnn_mlp_train_step_l2 on width 128. The forward pass with stored activations that does not copy the input in front of
 // them where its kernel can leave that out (2^20 rows: 268 MB less to write), ...
-// without_output: the last layer is left out (the backward pass's top launch forms the network's output again from the last
+// without_output: the last layer is left out (the backward pass forms the network's output again from the last
 // hidden layer, which lies where it always does); needs at least two hidden layers.
 int forward128_for_training(const tnn_mlp_desc *desc, const void *wprep, const void *x, void *interm_fwd, size_t M, hipStream_t s, bool without_output) {
     tnn_mlp_desc d = *desc;
@@ -796,7 +781,7 @@ int forward128_for_training(const tnn_mlp_desc *desc, const void *wprep, const v
     return launch_forward<fp16_t, 128, true>(&d, wprep, x, interm_fwd, M, s, io);
 }
 
-// ... and loss and backward pass over those activations, the loss folded into the top layer's launch and the first matrix's
+// ... and loss and backward pass over those activations, the loss folded into the layers' launch and the first matrix's
 // input read from `x`. Workspace as tnn_mlp_backward's.
 // wprep_fwd_if_no_output: the operand-order weights of the forward pass when interm_fwd holds no network output (see above), else null.
 int backward128_from_loss(const tnn_mlp_desc *desc, const void *wprep_bwd, const void *x, const void *interm_fwd, const float *targets, float loss_scale,
