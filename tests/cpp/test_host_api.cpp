@@ -720,6 +720,31 @@ static void test_level_plans() {
     }
 }
 
+// With shared levels, too, every (level, chunk) is an item of one XCD, once.
+static void test_shared_level_plans() {
+    for (uint32_t n_levels : {1u, 2u, 7u, 16u}) {
+        for (uint32_t n_own = 0; n_own <= n_levels; ++n_own) {
+            const std::vector<double> cost(n_levels, 2.0);
+            for (uint32_t n_chunks : {1u, 2u, 7u, 8u, 9u, 63u, 64u, 1001u}) {
+                tnn::LevelPlan plan;
+                plan.n_chunks = n_chunks;
+                const uint32_t most = tnn::plan_shared_levels(cost.data(), n_own, n_levels, &plan);
+                std::vector<int> seen((size_t)n_levels * n_chunks, 0);
+                for (uint32_t xcd = 0; xcd < tnn::kXcds; ++xcd)
+                    for (uint32_t turn = 0; turn < most; ++turn) {
+                        uint32_t level, chunk;
+                        if (tnn::plan_item(plan, n_levels, xcd, turn, &level, &chunk)) ++seen[(size_t)level * n_chunks + chunk];
+                    }
+                CHECK(std::all_of(seen.begin(), seen.end(), [](int n) { return n == 1; }));
+            }
+        }
+        const size_t part = tnn::level_part_chunks(n_levels, 256);
+        tnn::LevelPlan plan;
+        plan.n_chunks = (uint32_t)part;
+        CHECK((unsigned long long)tnn::plan_shared_levels(nullptr, 0, n_levels, &plan) * tnn::kXcds * 256 < (1ull << 32));
+    }
+}
+
 int main(int argc, char **argv) {
     const bool cpu_only = argc > 1 && std::string(argv[1]) == "--cpu";
     std::printf("storage types\n");
@@ -734,6 +759,7 @@ int main(int argc, char **argv) {
     test_lds_reservations();
     std::printf("level plans\n");
     test_level_plans();
+    test_shared_level_plans();
     if (!cpu_only) {
         tnn::abi_check(tnn_device_check());
         std::printf("swiftnet\n");

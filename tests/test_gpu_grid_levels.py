@@ -105,6 +105,41 @@ def test_large_batches_of_three_dimensions(tnn, features, param_dtype, out_dtype
     assert torch.equal(bits(by_level(tnn, d, x, tnn.grid_order(d, x), table, width, out_dtype)), expected)
 
 
+@pytest.mark.parametrize("dims,log2,features,levels,M", [
+    (3, 22, 2, 16, 1), (3, 22, 2, 16, 300), (3, 22, 2, 12, 5001), (3, 22, 2, 16, 20000), (2, 22, 2, 16, 5001), (3, 21, 2, 16, 2 ** 18), (3, 21, 2, 16, 2 ** 18 - 1),
+    (3, 20, 2, 16, 2 ** 19 + 77), (3, 20, 4, 9, 4097), (3, 16, 2, 16, 3 * 2 ** 18), (3, 19, 2, 16, 2 ** 20 + 511)])
+def test_levels_that_all_xcds_share(tnn, dims, log2, features, levels, M):
+    """All levels shared, none, and the large ones behind coarse ones that are not; batches of fewer chunks than XCDs, and that are no whole eighths."""
+    d = tnn.grid_desc(dict(BASE, n_dims=dims, n_levels=levels, n_features_per_level=features, log2_hashmap_size=log2))
+    gen = torch.Generator(device=tnn.dev).manual_seed(7)
+    table = torch.rand(tnn.grid_n_params(d), device=tnn.dev, generator=gen) * 2 - 1
+    x = torch.rand((M, dims), device=tnn.dev, generator=gen)
+    width = levels * features
+    x2 = torch.cat([x, torch.rand((DIRECT + 1, dims), device=tnn.dev)])[: max(M, DIRECT + 1)]  # (a batch beyond those that are written by levels)
+    expected = bits(tnn.grid_forward(d, x2, table, width, FP32)[:M])
+    assert torch.equal(bits(by_level(tnn, d, x, None, table, width, FP32)), expected)
+    assert torch.equal(bits(by_level(tnn, d, x, tnn.grid_order(d, x), table, width, FP32)), expected)
+
+
+@pytest.mark.parametrize("features,levels,log2,M", [(2, 16, 21, 2 ** 20 + 8), (1, 16, 22, 2 ** 20 + 1)])
+def test_a_large_field_by_levels(tnn, features, levels, log2, M):
+    """Beyond the size from which large levels pay in inference: the rows of the same points in batches that one kernel takes."""
+    import tiny_dpcpp_nn
+    tiny_dpcpp_nn.manual_seed(3)
+    model = tiny_dpcpp_nn.NetworkWithInputEncoding(
+        3, 3, {"otype": "FullyFusedMLP", "activation": "ReLU", "output_activation": "None", "n_neurons": 32, "n_hidden_layers": 2},
+        {"otype": "HashGrid", "type": "Hash", "n_levels": levels, "n_features_per_level": features, "log2_hashmap_size": log2, "base_resolution": 16, "per_level_scale": 1.5},
+        dtype=torch.float16, use_bias=False)
+    d = tnn.grid_desc(dict(BASE, n_levels=levels, n_features_per_level=features, log2_hashmap_size=log2, per_level_scale=1.5))
+    assert [tnn.lib.tnn_grid_mlp_width_wants_levels(ctypes.byref(d), 32, m) for m in (2 ** 20, M, 2 ** 19)] == [0, 1, 0]
+    x = torch.rand((M, 3), device=tnn.dev)
+    with torch.no_grad():
+        model.encoding.params.copy_(torch.rand(model.encoding.params.shape, device=tnn.dev) - 0.5)
+        y = model(x)
+        for rows in (slice(0, 2 ** 19), slice(2 ** 19, 2 ** 20), slice(M - 100000, M)):
+            assert torch.equal(bits(y[rows]), bits(model(x[rows].contiguous())))
+
+
 @pytest.mark.parametrize("ordered", [False, True])
 def test_a_batch_of_several_launches(tnn, ordered):
     """32 levels: a launch takes 65535 chunks of 512 points; a batch with more, its last chunk and last 64 points not full."""

@@ -6,7 +6,8 @@
 // What bounds a gather is where its line comes from: lines of 128 bytes at random arrive 66 * 10^9 times a second from the memory
 // side and 265 * 10^9 times from an XCD's own 4 MB of L2 (64 bytes a cycle and CU), whether 4, 8 or 16 bytes of a line are wanted.
 // A kernel whose waves walk all levels of their points (grid_forward_kernel) has the whole table in use at once, in every XCD. Here
-// an XCD takes a level at a time, for all points: its L2 holds that level, and a level is fetched by one or two XCDs instead of eight.
+// an XCD takes a level at a time, for all points: its L2 holds that level, and a level is fetched by one or two XCDs instead of eight. Levels that L2 does
+// not hold, and those of which a batch takes every line many times, all XCDs take one after the other, an eighth of the points each (shared_level).
 // The corners of a cell along the first dimension lie in one line nearly always. Two loads of a lane fetch it twice, because
 // the lines that a CU's waves have under way are many times what its vector cache holds; here two neighbouring lanes load the two
 // corners of a row, of one's point and then of the other's, and exchange what they loaded.
@@ -121,10 +122,10 @@ __global__ void __launch_bounds__(kLevelThreads)
             return;
         }
     }
-    const uint32_t xcd = blockIdx.x % kXcds, item = plan.first[xcd] + blockIdx.x / kXcds;
-    if (item >= plan.first[xcd + 1]) return;
-    const uint32_t l = item / plan.n_chunks;
-    const long long i0 = (long long)(item % plan.n_chunks) * S::kChunk + threadIdx.x;
+    const uint32_t xcd = blockIdx.x % kXcds, turn = blockIdx.x / kXcds;
+    uint32_t l, chunk;
+    if (!plan_item(plan, gp.n_levels, xcd, turn, &l, &chunk)) return;
+    const long long i0 = (long long)chunk * S::kChunk + threadIdx.x;
     const uint32_t size = lv.size[l], res = lv.resolution[l], flags = lv.flags[l];
     const float scale = lv.scale[l];
     const P *const level = table + (size_t)lv.offset[l] * F;
@@ -307,6 +308,21 @@ static double levels_us(const GridLevels &lv, uint32_t n_levels, uint32_t n_dims
     return cost * (double)M / (double)(1 << 23);
 }
 
+// Whether all XCDs take a level at a time, an eighth of the points each, instead of one or two of them the whole level. In cell order an eighth is a part of
+// space. Two or three large levels are in use at once then and not eight: 32 MB a level is what the 256 MB in front of the memory hold, and there is nothing to balance by
+// a guess of what levels cost, which is wrong where points share more lines than scattered ones (a picture's rows). But eight XCDs fetch the level,
+// which scattered points have to make up for: as many rows of corners for each of its lines. Field, 3-D, 16 levels, us, by XCDs / shared, scattered and a picture's rows (in
+// cell order from 5 * 2^17 points): 4 MB a level, 2^18 points 96 / 114 and 50 / 45, 2^19 180 / 198 and 81 / 69, 2^20 341 / 339 and 238 / 159; 2 MB, 2^19 162 / 162 and 76 / 66; 256 KB and
+// 1 MB, 2^19 152 / 157 and 164 / 168, rows 77 / 70 and 79 / 71, 2^20 281 / 267 and 297 / 282, 210 / 152 and 219 / 153; 8 MB, 2^18 158 / 168 and 64 / 51, 2^19 303 / 307 and 101 / 79, 2^20 512 / 491 and 304 / 175; 16 MB, 2^17 104 / 113, 2^18 198 / 204 and 83 / 58, 2^20 636 / 597 and 362 / 186;
+// 32 MB, 20 000 points 35 / 30 and 21 / 16, 2^17 121 / 122 and 62 / 40, 2^21 1286 / 1177 and 774 / 339. 2-D, 4 MB, 2^19 93 / 99, 2^20 173 / 177; 8 MB, 2^19 123 / 128, 2^20 199 / 196; 16 MB,
+// 2^19 152 / 149; 32 MB, 2^16 32 / 30, 2^20 252 / 219. (Two shared levels at a time, a coarse one's chunks between a fine one's: 32 MB 1170 -> 1145, 4 MB 328 -> 438.)
+static bool shared_level(size_t bytes, uint32_t n_dims, size_t M) {
+    const size_t MB = size_t(1) << 20, rows = M << (n_dims - 1), lines = bytes / 128;
+    if (bytes > 16 * MB) return true;
+    if (bytes > 4 * MB) return rows >= (bytes > 8 * MB ? 8 : 32) * lines;
+    return M >= (size_t(3) << 18) && rows >= 128 * lines;
+}
+
 // One launch: the points [begin, begin + M) of a batch.
 template <int D, int F, typename P, typename O>
 static int launch_levels_part(const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *table, O *out, bool rows, bool large,
@@ -316,7 +332,9 @@ static int launch_levels_part(const GridLevels &lv, const GridParams &gp, const 
     plan.n_chunks = (uint32_t)((M + chunk - 1) / chunk);
     double cost[TNN_GRID_MAX_LEVELS];
     for (uint32_t l = 0; l < gp.n_levels; ++l) cost[l] = level_cost(lv, l, D, F * sizeof(P), order != nullptr, batch);
-    const uint32_t most = plan_levels(cost, gp.n_levels, &plan);
+    uint32_t n_own = gp.n_levels;
+    while (n_own > 0 && shared_level(lv.size[n_own - 1] * F * sizeof(P), D, batch)) --n_own;
+    const uint32_t most = plan_shared_levels(cost, n_own, gp.n_levels, &plan);
     auto k = grid_levels_kernel<D, F, P, O, false, false>;
     if (rows) k = grid_levels_kernel<D, F, P, O, true, false>;
     if (large) k = grid_levels_kernel<D, F, P, O, false, D == 3>;

@@ -139,8 +139,11 @@ static bool levels_pay(const tnn_grid_desc *grid, int width, size_t M) {
     }
     // 12 and 16 levels: 0.3 to 0.7 and 0.5 to 0.9; of more than 8 MB, 2^15 points 0.65 and 0.97, 2^16 0.89 and 1.34. 8 levels 0.8 and 1.0 to 1.1.
     if (L > 10 && M < (size_t(1) << 15)) return width >= 32 && (M < 24000 || (F <= 2 && largest <= 8 * MB));
-    // Twice an XCD's L2 and more: 16 levels, 2^17 points 0.79 and 1.42, 2^20 0.92 and 1.37 (2^22 entries, 2^21 points 1473 / 1424 and 465 / 725); 8 levels 1.3 and 0.8 (2^18).
-    if (largest > (width == 16 ? 1 : 8) * MB) return false;
+    // Four times an XCD's L2 and more, which all XCDs share (shared_level): 16 levels of 32 MB, 2^17 points 138 / 121 and 37 / 41, 2^20 713 / 653 and 231 / 194, 2^21 1304 / 1170 and 430 / 328;
+    // one feature, 16 MB, 2^20 350 / 306 and 231 / 130. Four features, 8 levels, 2^19 209 / 215 and 76 / 99. (In cell order 2^19 points are 391 / 361 and 132 / 126, too: up to 2^20 points such a field
+    // is one that is evaluated without scratch memory, and stays so.)
+    if (largest > 8 * MB) return F <= 2 && M > (size_t(1) << 20);
+    if (largest > MB && width == 16) return false;
     // Two features: 0.3 to 0.8 and 0.2 to 0.9. Four and eight: 6 levels 2^18 points 0.8 to 1.0 and 0.6, 8 levels 1.0 and 0.9, 2^19 1.1 and 1.4.
     if (M >= (size_t(1) << 18)) return F <= 2 || (L <= 6 && M < (size_t(1) << 19)) || (L * F <= 16 && largest <= MB);
     // Between: 16 levels 0.5 and 0.9 (2^15 to 2^16 points 0.6 and 1.0). 8 levels, width 64: 2^15 points 0.7 and 1.1, 2^16 0.6 and 0.9; 4 levels 0.84 and 0.76, 2 levels 2^17 0.65. Four features

@@ -10,10 +10,12 @@ namespace tnn {
 constexpr uint32_t kXcds = 8;
 
 // Workgroup b is the (b / 8)-th of XCD b % 8 (workgroups go to the XCDs in turn; were they not, nothing but locality would be lost);
-// XCD k takes the items [first[k], first[k + 1]) of the list of all (level, chunk of points), level by level.
+// XCD k takes the items [first[k], first[k + 1]) of the list of all (level, chunk of points) of the levels up to `n_own`, level by level, and then
+// an eighth of the chunks of each further level, `each` at most.
 struct LevelPlan {
     uint32_t first[kXcds + 1];
     uint32_t n_chunks;
+    uint32_t n_own, each;
 };
 
 // Shares of equal cost (of a level: cost[l]). Returns the most items an XCD has: the launch is 8 times as many workgroups.
@@ -29,6 +31,30 @@ inline uint32_t plan_levels(const double *cost, uint32_t n_levels, LevelPlan *pl
         if (k > 0) most = std::max(most, plan->first[k] - plan->first[k - 1]);
     }
     return most;
+}
+
+// The levels from n_own on are shared, those in front dealt out by cost. Returns the most items an XCD has.
+inline uint32_t plan_shared_levels(const double *cost, uint32_t n_own, uint32_t n_levels, LevelPlan *plan) {
+    plan->n_own = n_own;
+    plan->each = (plan->n_chunks + kXcds - 1) / kXcds;
+    for (uint32_t k = 0; k <= kXcds; ++k) plan->first[k] = 0;
+    return (n_own ? plan_levels(cost, n_own, plan) : 0) + plan->each * (n_levels - n_own);
+}
+
+// The turn-th item of an XCD; false where there is none.
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline bool plan_item(const LevelPlan &plan, uint32_t n_levels, uint32_t xcd, uint32_t turn, uint32_t *level, uint32_t *chunk) {
+    const uint32_t own = plan.first[xcd + 1] - plan.first[xcd];
+    if (turn < own) {
+        *level = (plan.first[xcd] + turn) / plan.n_chunks;
+        *chunk = (plan.first[xcd] + turn) % plan.n_chunks;
+        return true;
+    }
+    *level = plan.n_own + (turn - own) / plan.each;
+    *chunk = (xcd + *level) % kXcds * plan.each + (turn - own) % plan.each; // (another eighth in every level: a batch of few chunks is not one XCD's)
+    return *level < n_levels && *chunk < plan.n_chunks;
 }
 
 // The most chunks of a launch, whatever the levels cost: a launch has fewer than 2^32 threads, and one XCD may have nearly all items
