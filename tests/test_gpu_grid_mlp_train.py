@@ -135,6 +135,26 @@ def test_fused_step_equals_the_three_calls(tnn, case, ordered):
     assert float(ga.abs().max()) > 0
 
 
+@pytest.mark.parametrize("dims,levels,dtype,n_hidden,M,overwrite", [
+    (2, 8, FP16, 2, 2 ** 14 - 8, True), (2, 8, FP16, 2, 2 ** 14 + 8, True),  # levels that are binned on both sides of 2^18 requests
+    (2, 16, BF16, 4, 30000, False), (2, 16, FP16, 1, 47000, True),           # 256 and 512 threads, most partials; a table that is added to
+    (3, 9, BF16, 3, 9000, True), (3, 16, FP16, 4, 65536 + 8, False),
+    (2, 4, FP16, 1, 2 ** 19 + 8, True)])                                     # binned in two parts: a reduction of its own
+def test_the_reduction_goes_with_the_binning(tnn, dims, levels, dtype, n_hidden, M, overwrite):
+    """The sums of the weight gradients, Adam, the loss and the cleared table as the first workgroups of the scatter's first launch: what they are in a launch of their own."""
+    cfg = dict(n_dims=dims, n_levels=levels, n_features_per_level=2, log2_hashmap_size=17, base_resolution=16, per_level_scale=1.6)
+    c = setup(tnn, cfg, FP32, dtype, n_hidden, M, seed=M % 97)
+    a, b = state(tnn, c), state(tnn, c)
+    before = torch.full((c["n"],), float("nan") if overwrite else 0.25, device=tnn.dev)
+    ga, gb = before.clone(), before.clone()
+    for step in (1, 2):
+        chain_step(tnn, c, a, step, 1.0 * M, ga, overwrite, False)
+        fused_step(tnn, c, b, step, 1.0 * M, gb, overwrite, False)
+        same_state(a, b, False, f"step {step}")
+        assert torch.isfinite(gb).all()
+        assert float((ga - gb).abs().max()) <= 1e-5 * float(ga.abs().max())
+
+
 def test_table_gradient_against_the_oracle(tnn, oracle):
     cfg = dict(n_dims=2, n_levels=16, n_features_per_level=2, log2_hashmap_size=15, base_resolution=16, per_level_scale=1.5)
     c = setup(tnn, cfg, FP16, FP16, 2, 8192, seed=5)

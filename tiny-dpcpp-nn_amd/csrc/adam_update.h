@@ -109,6 +109,7 @@ __device__ __forceinline__ void clear_range(const ClearRange &c, uint32_t block,
     if (i < c.n_tail) reinterpret_cast<float *>(c.p + c.n4)[i] = 0.0f;
 }
 
+struct TrainReduce;
 // What follows the main kernel of the fused training step.
 struct TrainTail {
     bool use_adam = false;       // apply Adam to the reduced gradients inside the reduction kernel
@@ -121,6 +122,7 @@ struct TrainTail {
     int dy_cols = 0;
     float dy_scale = 1.0f, result_scale = 1.0f;
     PackedGradient packed{};
+    TrainReduce *later = nullptr; // the reduction is not launched but left here for the caller (train_reduce.h)
     ClearRange clear{}; // cleared by further workgroups of the reduction (a launch of its own in front of the scatter took 5 us)
 };
 

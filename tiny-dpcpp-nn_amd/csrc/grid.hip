@@ -897,7 +897,7 @@ int grid_backward_clear(const tnn_grid_desc *desc, bool ordered, bool with_works
 // d_x may be given beside d_order, for the routes that read the rows of a row-major dL/dy better in the caller's order.
 int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4 *d_order, const void *d_dLdy, int dy_dtype, uint32_t padded_width,
                        const GradLayout &dl, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
-                       hipStream_t s, bool cleared) {
+                       hipStream_t s, bool cleared, const ReduceInFront *front) {
     GridLevels lv;
     GridParams gp;
     int rc = grid_common(desc, padded_width, M, &lv, &gp);
@@ -917,6 +917,12 @@ int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4
     if (bins.n_levels && workspace_bytes < bin_scratch_bytes(bins, desc->n_dims, n_features) + (scratch - reinterpret_cast<uintptr_t>(d_workspace)))
         return fail(TNN_ERR_WORKSPACE, "grid backward: workspace of %zu bytes given, %zu needed", workspace_bytes, bin_scratch_bytes(bins, desc->n_dims, n_features) + 256);
     if (overwrite && (reinterpret_cast<uintptr_t>(d_grad_table) & 15)) return fail(TNN_ERR_INVALID_ARGUMENT, "d_grad_table must be 16-byte aligned");
+    const auto launch_bins = [&](BinStage stage, const TrainReduce *reduce) {
+        return launch_grid_binned(bins, gp, dl, desc->n_dims, n_features, d_x, d_x && !dl.by_position ? nullptr : d_order, d_dLdy, dy_dtype, (float *)d_grad_table, overwrite != 0, M,
+                                  reinterpret_cast<void *>(scratch), s, stage, reduce);
+    };
+    const bool together = front && bins.n_levels && bins_take_reduction(bins, n_features, dy_dtype, M, *front->reduce);
+    if (front && (rc = together ? launch_bins(kBinning, front->reduce) : front->launch(*front->reduce, s))) return rc;
     if (overwrite && !cleared) {
         // a fill kernel rather than a memset node, so the call can be captured into a HIP graph
         const ClearRange clear = range_to_clear(desc, bins, d_grad_table, grad_dtype);
@@ -929,9 +935,7 @@ int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4
     if (grad_dtype == TNN_FP32) {
         TNN_DISPATCH_DF(desc, rc = (launch_grid_backward_g<D_, F_, float>(lv, gp, bp, dl, n_big, lds_bytes, d_x, d_order, d_dLdy, dy_dtype,
                                                                           (float *)d_grad_table, M, s)));
-        if (rc == TNN_OK && bins.n_levels)
-            rc = launch_grid_binned(bins, gp, dl, desc->n_dims, n_features, d_x, d_x && !dl.by_position ? nullptr : d_order, d_dLdy, dy_dtype, (float *)d_grad_table, overwrite != 0, M,
-                                    reinterpret_cast<void *>(scratch), s);
+        if (rc == TNN_OK && bins.n_levels) rc = launch_bins(together ? kSums : kBinningAndSums, nullptr);
     } else {
         const uint32_t F = desc->n_features_per_level;
 #define TNN_PACKED(D_, F_) \

@@ -39,9 +39,13 @@ bool bin_plan_add(BinPlan *p, uint32_t l, const GridLevels &lv, const GridParams
 size_t bin_scratch_bytes(const BinPlan &p, uint32_t n_dims, uint32_t n_features);
 // What the plan's levels need for its batch and for any smaller one.
 size_t bin_scratch_bytes_up_to(BinPlan p, uint32_t n_dims, uint32_t n_features);
+// Whether the binning's launch can take the reduction with it, and then it is the first launch of a scatter (kBinning alone), before any that adds to the table.
+bool bins_take_reduction(const BinPlan &p, uint32_t n_features, int dy_dtype, size_t M, const TrainReduce &r);
+enum BinStage { kBinning = 1, kSums = 2, kBinningAndSums = 3 };
 // Nothing in the scratch has to be cleared. With `overwrite` every entry of the plan's levels
 // is written, whatever it held.
 int launch_grid_binned(const BinPlan &p, const GridParams &gp, const GradLayout &dl, uint32_t n_dims, uint32_t n_features, const float *x,
-                       const float4 *order, const void *dLdy, int dy_dtype, float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s);
+                       const float4 *order, const void *dLdy, int dy_dtype, float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s,
+                       BinStage stage = kBinningAndSums, const TrainReduce *reduce = nullptr);
 
 } // namespace tnn

@@ -21,6 +21,7 @@
 // Measured, 2^20 points, 3-D, 2^19 entries, the ten finest levels: 2 x (99 + 97) us; as atomics 1.5 ms.
 #include "grid_binned.h"
 #include "mlp_tile.h"
+#include "train_reduce.h"
 
 #include <algorithm>
 #include <cmath>
@@ -152,19 +153,46 @@ __device__ __forceinline__ size_t run_slot(uint32_t first_quad, uint32_t bin, ui
 // them in its L2.
 // No one unit bounds it (3-D, 2^19 points, 10 levels, 99 us): 346 MB written, the records all in whole 64-byte requests, at 3.5 TB/s where a
 // fill reaches 6.9; the vector units are at work 45 % of the time, LDS a sixth, and a wave waits for 41 % of its.
-template <int D, int F, typename G>
-__global__ void __launch_bounds__((BinShape<D, F>::kThreads))
+// TAKEN: the reduction of the training kernel that left dL/dy (and what it clears) is the first workgroups of this launch: both wait for that kernel only, and what adds to the table
+// waits for both. It was a launch of its own of 4 to 7 us, a chain of loads and one sum (optimisation step with the ordering, us, before / now: 2-D, 20 000 points 68.4 / 64.6, 2^16 82.0 / 77.4, 2^18
+// 210 / 203; 3-D, 2^17 257 / 253; a module's forward and backward pass, 2-D, 2^18 177 / 171). Registers for eight waves a SIMD, as without.
+template <int D, int F, typename G, typename TAKEN = std::false_type>
+__global__ void __launch_bounds__((BinShape<D, F>::kThreads), (std::is_same<TAKEN, TrainReduce>::value ? 8 : 1))
     grid_bin_kernel(const GridParams gp, const BinPlan bp, const GradLayout dl, const float *__restrict__ xin,
                     const float4 *__restrict__ order, const G *__restrict__ dLdy, uint32_t *__restrict__ runs, BinRecord<F> *__restrict__ records,
-                    long long first, long long last, uint32_t n_stretches, uint32_t pitch, uint32_t room) {
+                    long long first, long long last, uint32_t n_stretches, uint32_t pitch, uint32_t room, const TAKEN taken, uint32_t taken_blocks) {
     typedef BinShape<D, F> S;
     constexpr int NP = S::kPairs, P = S::kPoints;
     static_assert(S::kRecords <= 4096 && kBinMaxBins <= 1024, "a record's place is packed into 12 + 10 + 10 bits");
     const uint32_t T = blockDim.x;
     extern __shared__ __align__(16) unsigned char bin_smem[];
+    if constexpr (std::is_same<TAKEN, TrainReduce>::value) {
+        if (blockIdx.x < taken_blocks) { // (a multiple of 8: the others' numbers say which XCD they are on)
+            const uint32_t n = taken.clear.reduce_blocks;
+            if (blockIdx.x >= n) {
+                clear_range(taken.clear, blockIdx.x - n, taken_blocks - n);
+                return;
+            }
+            float4(*const red)[16] = reinterpret_cast<float4(*)[16]>(bin_smem);
+            const auto reduce = [&](auto adam, auto threads) __attribute__((always_inline)) {
+                train_reduce_block<G, decltype(adam)::value, decltype(threads)::value, true>(taken.partials, taken.loss_partials, taken.n_partials, taken.n_elems,
+                                                                                            static_cast<G *>(taken.dW_T), taken.dW_f32, taken.loss_sum, taken.adam,
+                                                                                            taken.packed, blockIdx.x, red);
+            };
+            if (T == 512) {
+                if (taken.use_adam) reduce(std::true_type{}, std::integral_constant<int, 512>{});
+                else reduce(std::false_type{}, std::integral_constant<int, 512>{});
+            } else {
+                if (taken.use_adam) reduce(std::true_type{}, std::integral_constant<int, 256>{});
+                else reduce(std::false_type{}, std::integral_constant<int, 256>{});
+            }
+            return;
+        }
+    }
+    const uint32_t block = blockIdx.x - (std::is_same<TAKEN, TrainReduce>::value ? taken_blocks : 0u);
     BinRecord<F> *const sorted = reinterpret_cast<BinRecord<F> *>(bin_smem);
     uint32_t *const base = reinterpret_cast<uint32_t *>(sorted + room); // records per bin, then the place of the bin's first one
-    const uint32_t turn = blockIdx.x / 8, k = turn % bp.n_levels, stretch = (turn / bp.n_levels) * 8 + blockIdx.x % 8;
+    const uint32_t turn = block / 8, k = turn % bp.n_levels, stretch = (turn / bp.n_levels) * 8 + block % 8;
     if (stretch >= n_stretches) return;
     const long long begin = first + (long long)stretch * (T * P);
     const long long end = begin + T * P < last ? begin + T * P : last;
@@ -540,7 +568,7 @@ size_t bin_scratch_bytes_up_to(BinPlan p, uint32_t n_dims, uint32_t n_features) 
 
 template <int D, int F, typename G>
 static int launch_binned(const BinPlan &p, const GridParams &gp, const GradLayout &dl, const float *x, const float4 *order, const void *dLdy,
-                         float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s) {
+                         float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s, BinStage stage, const TrainReduce *reduce) {
     typedef BinShape<D, F> S;
     const BinLaunch b = bin_launch<D, F>(p);
     uint32_t *const runs = static_cast<uint32_t *>(scratch);
@@ -576,10 +604,24 @@ static int launch_binned(const BinPlan &p, const GridParams &gp, const GradLayou
     for (size_t first = 0; first < M; first += p.batch) {
         const size_t last = std::min(M, first + p.batch);
         const uint32_t n_stretches = (uint32_t)((last - first + b.stretch - 1) / b.stretch);
-        TNN_LAUNCH(bin, dim3((n_stretches + 7) / 8 * 8 * p.n_levels), dim3(b.threads), bin_lds, s, gp, p, dl, x, order, (const G *)dLdy, runs, records,
-                   (long long)first, (long long)last, n_stretches, b.pitch, b.room);
-        int rc = check_launch("grid_bin_kernel");
-        if (rc) return rc;
+        const unsigned bin_blocks = (n_stretches + 7) / 8 * 8 * p.n_levels;
+        int rc = TNN_OK;
+        if constexpr (F == 2 && !std::is_same<G, float>::value) {
+            if (reduce) { // (one part: bins_take_reduction)
+                const unsigned taken = (reduce->blocks() + 7) / 8 * 8;
+                const auto both = grid_bin_kernel<D, F, G, TrainReduce>;
+                if (!reserve_lds(reinterpret_cast<const void *>(both), bin_lds)) return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", bin_lds);
+                TNN_LAUNCH(both, dim3(taken + bin_blocks), dim3(b.threads), bin_lds, s, gp, p, dl, x, order, (const G *)dLdy, runs, records, (long long)first,
+                           (long long)last, n_stretches, b.pitch, b.room, *reduce, taken);
+                if ((rc = check_launch("grid_bin_kernel with a reduction"))) return rc;
+            }
+        }
+        if ((stage & kBinning) && !reduce) {
+            TNN_LAUNCH(bin, dim3(bin_blocks), dim3(b.threads), bin_lds, s, gp, p, dl, x, order, (const G *)dLdy, runs, records, (long long)first, (long long)last,
+                       n_stretches, b.pitch, b.room, std::false_type{}, 0u);
+            if ((rc = check_launch("grid_bin_kernel"))) return rc;
+        }
+        if (!(stage & kSums)) continue;
         TNN_LAUNCH(sum, dim3((unsigned)sum_blocks), dim3(sum_threads), sum_lds, s, p, (const uint32_t *)runs, (const BinRecord<F> *)records, grad,
                    n_stretches, b.pitch, (int)(overwrite && first == 0));
         if ((rc = check_launch("grid_bin_sum_kernel"))) return rc;
@@ -587,13 +629,19 @@ static int launch_binned(const BinPlan &p, const GridParams &gp, const GradLayou
     return TNN_OK;
 }
 
+// The binning is one launch, the threads hold all partials at once, and dL/dy is of the network's type, as the training kernel writes it.
+bool bins_take_reduction(const BinPlan &p, uint32_t n_features, int dy_dtype, size_t M, const TrainReduce &r) {
+    return n_features == 2 && dy_dtype != TNN_FP32 && M <= p.batch && r.n_partials <= 256;
+}
+
 int launch_grid_binned(const BinPlan &p, const GridParams &gp, const GradLayout &dl, uint32_t n_dims, uint32_t n_features, const float *x,
-                       const float4 *order, const void *dLdy, int dy_dtype, float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s) {
+                       const float4 *order, const void *dLdy, int dy_dtype, float *grad, bool overwrite, size_t M, void *scratch, hipStream_t s, BinStage stage,
+                       const TrainReduce *reduce) {
 #define TNN_BIN_G(D, F)                                                                                                                    \
     switch (dy_dtype) {                                                                                                                    \
-    case TNN_FP32: return launch_binned<D, F, float>(p, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s);                            \
-    case TNN_BF16: return launch_binned<D, F, bf16_t>(p, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s);                           \
-    case TNN_FP16: return launch_binned<D, F, fp16_t>(p, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s);                           \
+    case TNN_FP32: return launch_binned<D, F, float>(p, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s, stage, reduce); \
+    case TNN_BF16: return launch_binned<D, F, bf16_t>(p, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s, stage, reduce); \
+    case TNN_FP16: return launch_binned<D, F, fp16_t>(p, gp, dl, x, order, dLdy, grad, overwrite, M, scratch, s, stage, reduce); \
     default: return fail(TNN_ERR_UNSUPPORTED, "dy_dtype %d", dy_dtype);                                                                     \
     }
 #define TNN_BIN_F(D)                                                                                                                       \

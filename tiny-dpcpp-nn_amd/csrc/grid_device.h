@@ -57,10 +57,16 @@ template <> struct OrderBits<3> { static constexpr int coarse = 4, fine = 2; };
 int check_grid_desc(const tnn_grid_desc *d);
 // `cleared`: of a table that is overwritten, what grid_backward_clear names has been cleared already.
 struct ClearRange;
+struct TrainReduce;
+// The reduction of the kernel that left dL/dy, not launched yet: it goes in front of the scatter, as a launch of its own by `launch` where no other can take it.
+struct ReduceInFront {
+    const TrainReduce *reduce;
+    int (*launch)(const TrainReduce &, hipStream_t);
+};
 int grid_backward_clear(const tnn_grid_desc *desc, bool ordered, bool with_workspace, void *d_grad_table, int grad_dtype, size_t M, ClearRange *clear);
 int grid_backward_impl(const tnn_grid_desc *desc, const float *d_x, const float4 *d_order, const void *d_dLdy, int dy_dtype, uint32_t padded_width,
                        const GradLayout &dl, void *d_grad_table, int grad_dtype, int overwrite, size_t M, void *d_workspace, size_t workspace_bytes,
-                       hipStream_t s, bool cleared = false);
+                       hipStream_t s, bool cleared = false, const ReduceInFront *front = nullptr);
 int grid_common(const tnn_grid_desc *desc, uint32_t padded_width, size_t M, GridLevels *lv, GridParams *gp);
 
 template <int D> __device__ __forceinline__ uint32_t hash_pos(const uint32_t (&p)[D], uint32_t hash_type) {

@@ -4,6 +4,7 @@
 #include "adam_update.h"
 #include "grid_levels.h"
 #include "mlp_train_shape.h"
+#include "train_reduce.h"
 
 #include <algorithm>
 
@@ -14,7 +15,8 @@ namespace tnn {
                                   float *partials, float *loss_partials, const TrainTail &tail, hipStream_t s);                                        \
     int grid_mlp_given_launch_##T(const tnn_mlp_desc *d, const FusedPlan &p, const void *levels, uint32_t n_levels, const float4 *order, const void *wf, \
                                   const void *wb, const void *dLdy, void *d_enc, size_t M, float *partials, float *loss_partials, const TrainTail &tail, \
-                                  hipStream_t s);
+                                  hipStream_t s);                                                                                                       \
+    int grid_mlp_reduce_launch_##T(const TrainReduce &r, hipStream_t s);
 TNN_DECLARE(bf16)
 TNN_DECLARE(fp16)
 #undef TNN_DECLARE
@@ -69,13 +71,14 @@ struct GridTrainMemory {
     }
 };
 
-// (The reduction behind the network's kernel has cleared the table's gradient where that is overwritten.)
+// (The reduction behind the network's kernel clears the table's gradient where that is overwritten. It is launched with the scatter.)
 // dL/d(encoding), in the network's type, by levels and in the order the kernel took the points, into the table's gradient
 static int scatter_levels(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const float4 *order, const GridTrainMemory &m, float scale,
-                          float *d_grad_table, int overwrite, size_t M, hipStream_t s) {
+                          float *d_grad_table, int overwrite, size_t M, const TrainReduce &reduce, hipStream_t s) {
+    ReduceInFront front{&reduce, mlp->dtype == TNN_BF16 ? grid_mlp_reduce_launch_bf16 : grid_mlp_reduce_launch_fp16};
     const GradLayout dl{grid->n_features_per_level, level_pitch(M) * grid->n_features_per_level, 1, scale};
     return grid_backward_impl(grid, order ? nullptr : d_x, order, m.enc_grad, mlp->dtype, (uint32_t)mlp->width, dl, d_grad_table, TNN_FP32, overwrite, M, m.scatter,
-                              m.scatter_bytes, s, overwrite != 0);
+                              m.scatter_bytes, s, overwrite != 0, &front);
 }
 
 TNN_API size_t tnn_grid_mlp_train_step_workspace_bytes(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, size_t M) {
@@ -108,6 +111,8 @@ TNN_API int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn
     hipStream_t s = as_stream(stream);
 
     TrainTail tail;
+    TrainReduce reduce;
+    tail.later = &reduce;
     tail.use_adam = true;
     tail.adam = make_adam_args(d_master_packed, d_m, d_v, 1.0f / loss_scale, step, lr, beta1, beta2, eps, d_packed_T, d_prepared_fwd, d_prepared_bwd,
                                mlp->width);
@@ -118,7 +123,7 @@ TNN_API int tnn_grid_mlp_train_step_l2_adam(const tnn_grid_desc *grid, const tnn
     if ((rc = launch(mlp, plan, m.levels, grid->n_levels, order, d_prepared_fwd, d_prepared_bwd, d_targets, loss_scale, d_y, d_loss_sum, m.enc_grad, M, m.partials,
                      m.loss_partials, tail, s)))
         return rc;
-    return scatter_levels(grid, mlp, d_x, order, m, 1.0f, d_grad_table, overwrite, M, s);
+    return scatter_levels(grid, mlp, d_x, order, m, 1.0f, d_grad_table, overwrite, M, reduce, s);
 }
 
 // d_levels: the encoded batch as a forward pass left it, or null, and it is formed from d_table.
@@ -143,12 +148,14 @@ static int grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp,
         if ((rc = launch_grid_levels(grid, lv, gp, d_x, order, d_table, m.levels, mlp->dtype, 0, M, s))) return rc;
         d_levels = m.levels;
     }
+    TrainReduce reduce;
+    if (d_grad_table) tail.later = &reduce;
     // without a gradient table the network's gradients are all that is asked for: no dL/d(encoding) leaves the kernel
     const auto launch = mlp->dtype == TNN_BF16 ? grid_mlp_given_launch_bf16 : grid_mlp_given_launch_fp16;
     rc = launch(mlp, plan, d_levels, grid->n_levels, order, d_prepared_fwd, d_prepared_bwd, d_dLdy, d_grad_table ? m.enc_grad : nullptr, M, m.partials, m.loss_partials,
                 tail, s);
     if (rc || !d_grad_table) return rc;
-    return scatter_levels(grid, mlp, d_x, order, m, tail.result_scale, d_grad_table, overwrite, M, s);
+    return scatter_levels(grid, mlp, d_x, order, m, tail.result_scale, d_grad_table, overwrite, M, reduce, s);
 }
 
 TNN_API int tnn_grid_mlp_backward(const tnn_grid_desc *grid, const tnn_mlp_desc *mlp, const float *d_x, const void *d_order, const void *d_table,

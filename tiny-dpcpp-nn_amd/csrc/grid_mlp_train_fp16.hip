@@ -7,4 +7,5 @@ int grid_mlp_train_launch_fp16(const tnn_mlp_desc *d, const FusedPlan &p, const 
                                float *loss_partials, const TrainTail &tail, hipStream_t s) {
     return launch_levels_train_n<fp16_t>(d, p, levels, n_levels, order, wf, wb, targets, loss_scale, y, loss_sum, d_enc, M, partials, loss_partials, tail, s);
 }
+int grid_mlp_reduce_launch_fp16(const TrainReduce &r, hipStream_t s) { return launch_train_reduce<fp16_t>(r, s); }
 } // namespace tnn
