@@ -230,6 +230,27 @@ def test_workspace_of_a_batch_holds_a_smaller_one(tnn, cfg, M):
         assert float((grad - ref).abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max()))
 
 
+@pytest.mark.parametrize("features,levels,base,M", [(2, 16, 16, 122880), (2, 16, 16, 122881), (2, 8, 16, 5000), (1, 16, 16, 40000), (4, 6, 16, 20000), (2, 16, 8, 40000), (8, 3, 16, 16384)])
+def test_batches_in_cell_order_without_boxes(tnn, oracle, features, levels, base, M):
+    """Three dimensions, on both sides of the size up to which all levels are binned, and with levels that are copied (base 8), whose launch boxes share. The bar of the plain scatter."""
+    cfg = dict(CFG3, n_features_per_level=features, n_levels=levels, base_resolution=base)
+    rng = np.random.default_rng(M + features)
+    x = rng.uniform(0, 1, (M, 3)).astype(np.float32)
+    x[: M // 8] = x[0] * 0.9 + 0.01 * x[: M // 8]  # (some points crowd)
+    d = tnn.grid_desc(cfg)
+    g = rng.standard_normal((M, levels * features)).astype(np.float32)
+    ref = oracle.grid_backward(cfg, x, g, tnn.grid_n_params(d))
+    xt, gt = torch.from_numpy(x).to(tnn.dev), torch.from_numpy(g).to(tnn.dev)
+    order = tnn.grid_order(d, xt)
+    for rows in (None, xt):  # from the order alone, and with the points beside it
+        grad = torch.full((tnn.grid_n_params(d),), float("nan"), device=tnn.dev)
+        need = tnn.lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), M)
+        work = torch.empty(max(need, 1), dtype=torch.uint8, device=tnn.dev)
+        assert tnn.lib.tnn_grid_backward_binned(ctypes.byref(d), None if rows is None else rows.data_ptr(), order.data_ptr(), gt.data_ptr(), FP32, gt.shape[1], grad.data_ptr(), 1, M,
+                                                work.data_ptr(), work.numel(), tnn.stream()) == 0, tnn.lib.tnn_last_error()
+        assert np.abs(grad.cpu().numpy() - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
+
+
 def test_binned_workspace_is_checked(tnn):
     from tiny_dpcpp_nn import _lib
     d = tnn.grid_desc(CFG3)

@@ -620,6 +620,33 @@ static int boxed_chunk_log2(uint32_t resolution, uint32_t n_dims, uint32_t F, do
     return -1;
 }
 
+// From and up to how many points boxes do not pay beside bins. Where no level is copied whole either, as in three dimensions, and the bins take all, batches without boxes have no launch
+// for them: optimisation step with the ordering, 3-D, us, with boxes / all levels binned: 16 levels of 2^15 entries, 2^12 points 59 / 49, 2^13 63 / 52, 2^15 85 / 71, 114 688 160 / 144; of
+// 2^19 2^13 142 / 129, 2^15 165 / 150, 114 688 234 / 217; 8 levels of 2^17 entries 64 / 52, 77 / 65, 124 / 112; of 2^19 72 / 60, 89 / 73, 133 / 121, 2^18 184 / 190. (Where the bins refuse
+// levels of too few points the launch stays: 16 levels of 2^19, 2^12 points 136 / 144. 2-D, where the coarsest levels are copied, 2^13 55 / 56, 2^16 77 / 82.) Up to as many points as take no more
+// memory for it than 2^17 in the caller's order, which copy some levels (122 880 for 16 levels, one of them copied).
+struct NoBoxes {
+    size_t from = 1, to = 0;
+    bool operator()(size_t M) const { return M >= from && M <= to; }
+};
+static NoBoxes no_boxes_for(const GridLevels &lv, const GridParams &gp, uint32_t n_dims, uint32_t F) {
+    NoBoxes r;
+    if (n_dims != 3 || gp.n_levels > kMaxBinned) return r;
+    uint32_t copied = 0, largest = 0;
+    for (uint32_t l = 0; l < gp.n_levels; ++l) {
+        if (lv.size[l] * F * sizeof(double) <= kCopiedBytesOrdered) return r;
+        copied += lv.size[l] * (F == 2 ? 1 : F) * sizeof(double) <= kPrivateLdsBytes;
+        largest = std::max(largest, lv.size[l]);
+    }
+    const size_t to = std::min(kMoreBinnedBelow * (gp.n_levels - copied) / gp.n_levels, kMoreBinnedBelow - 1);
+    BinPlan bins{};
+    for (uint32_t l = 0; l < gp.n_levels; ++l)
+        if (!bin_plan_add(&bins, l, lv, gp, n_dims, F, to)) return r;
+    while (r.from < to && (r.from << (n_dims - 1)) < largest / 16) r.from *= 2; // (as bin_plan_add refuses them, to a power of two)
+    r.to = to;
+    return r;
+}
+
 // Binned from where the atomics it saves (one request per pair of corners, 20e9 a second) take longer than its two launches:
 // 2^18 requests. (2-D, 11 such levels, 12 000 points: 20 us either way; 2^16 points: 42 against 95.)
 static bool enough_to_bin(size_t M, uint32_t n_levels, uint32_t n_dims) { return ((unsigned long long)M * n_levels << (n_dims - 1)) >= (1ull << 18); }
@@ -674,7 +701,7 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
         if (M > bp.more_up_to) divide(0, 0);
     }
     // Cell order: of the other levels, those with boxes take the boxed route.
-    if (ordered && gp.n_levels > 0 && !nearest) {
+    if (ordered && gp.n_levels > 0 && !nearest && !(M < kMoreBinnedBelow && bin_others() && no_boxes_for(lv, gp, n_dims, F)(M))) {
         bp.bins_per_row = coarse_cells(n_dims);
         bp.n_rows = 4096 / bp.bins_per_row;
         const double per_row = (double)M / bp.n_rows;
@@ -986,13 +1013,17 @@ TNN_API size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size
             most = std::max(most, bin_scratch_bytes_up_to(bins, D, F));
         }
     }
+    const NoBoxes without = no_boxes_for(lv, gp, D, F);
+    const size_t no_boxes = M >= without.from ? without.to : 0; // (below `from` a batch has boxes and needs less)
     // Cell order: levels that are not copied leave the bins for boxes one by one as the batch grows, each at a size of its own.
     uint32_t n = 0, level[TNN_GRID_MAX_LEVELS], most_bins = 0;
     size_t boxed_from[TNN_GRID_MAX_LEVELS];
     for (uint32_t l = 0; l < gp.n_levels; ++l) {
         if (lv.size[l] * F * sizeof(double) <= kCopiedBytesOrdered) continue;
         const double R = (double)lv.resolution[l], enough = std::ceil(kBoxedMinPerCellBinned * (D == 2 ? R * R : R * R * R));
-        const auto boxed = [&](size_t points) { return boxed_chunk_log2(lv.resolution[l], D, F, kBoxedMinPerCellBinned, points) >= 0; };
+        const auto boxed = [&](size_t points) {
+            return boxed_chunk_log2(lv.resolution[l], D, F, kBoxedMinPerCellBinned, points) >= 0 && points > no_boxes;
+        };
         level[n] = l;
         boxed_from[n] = ~(size_t)0;
         if (followed && enough <= (double)M) {
@@ -1008,6 +1039,11 @@ TNN_API size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size
     }
     bool is_binned[TNN_GRID_MAX_LEVELS];
     const auto in_order = [&](size_t points) {
+        if (followed && points <= no_boxes) { // (the levels of one plan)
+            (void)plan_backward(lv, gp, D, F, true, true, points, &bins, &n_big, &lds);
+            most = std::max(most, bin_scratch_bytes_up_to(bins, D, F));
+            return;
+        }
         const size_t batch = std::min(points, kBinBatch);
         uint32_t in_boxes = 0, others = 0, binned = 0;
         for (uint32_t i = 0; i < n; ++i) others += boxed_from[i] > points || in_boxes++ >= kMaxTiled;
