@@ -137,6 +137,26 @@ def test_ordered_forward_matches_the_oracle_and_every_variant(tnn, oracle):
         assert torch.equal(out.view(torch.uint8), tnn.grid_forward(d, xt, tt, width, od).view(torch.uint8))
 
 
+@pytest.mark.parametrize("D", [2, 3])
+@pytest.mark.parametrize("M", [1, 63, 1023, 1025, 2048, 2049, 4096, 4097, 8191, 8192, 8193])
+def test_batches_that_one_workgroup_orders(tnn, D, M):
+    """Up to 2, 4 and 8 points a thread, and the first batch beyond: every row once with its own coordinates, sorted by coarse cell, and the positions where the coarse cells start."""
+    d = tnn.grid_desc(dict(n_dims=D, n_levels=4, n_features_per_level=2, log2_hashmap_size=12, base_resolution=16, per_level_scale=1.5))
+    rng = np.random.default_rng(M + D)
+    x = rng.uniform(-0.05, 1.05, (M, D)).astype(np.float32)
+    x[: M // 3] = rng.uniform(0.5, 0.5 + 2.0 ** -8, (M // 3, D))  # (a crowded cell)
+    order = tnn.grid_order(d, torch.from_numpy(x).to(tnn.dev)).cpu().numpy().view(np.uint8).reshape(-1)
+    rec = order[: 16 * M].view(np.float32).reshape(M, 4)
+    rows = rec[:, 3].copy().view(np.uint32)
+    assert np.array_equal(np.sort(rows), np.arange(M, dtype=np.uint32)) and np.array_equal(rec[:, :D], x[rows])
+    coarse = 6 if D == 2 else 4
+    q = np.clip(np.floor(rec[:, :D] * np.float32(1 << coarse)), 0, (1 << coarse) - 1).astype(np.int64)
+    key = sum(q[:, k] << (coarse * k) for k in range(D))
+    assert (np.diff(key) >= 0).all()
+    at = (16 * M + 255) // 256 * 256
+    assert np.array_equal(order[at: at + 4 * 4096].view(np.uint32), np.searchsorted(key, np.arange(4096)))
+
+
 def test_order_buffer_checks(tnn):
     from tiny_dpcpp_nn import _lib
     d = tnn.grid_desc(CFG5, FP16)

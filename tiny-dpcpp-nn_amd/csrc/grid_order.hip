@@ -23,6 +23,7 @@ constexpr int kOrderMaxWg = 256;      // histogram workgroups (the scan keeps a 
 constexpr int kOrderAhead = 4;        // points of a thread under way at once (the whole ordering, 2^18 points: 24.8 us one by one, 21.1 with this and the refinement)
 constexpr int kRefineEach = 8;        // records of a thread in a piece of a bin
 constexpr int kRefineBins = 64;       // 6 further bits
+constexpr size_t kSmallOrder = 8192; // points that one workgroup puts into their bins (order_small_kernel)
 
 struct OrderPlan {
     int n_wg;
@@ -180,6 +181,53 @@ __global__ void __launch_bounds__(kOrderThreads)
     }
 }
 
+// Step 1 of a batch that one workgroup holds in its registers: histogram, starting positions and places in one launch instead of three, each of which was some 3 us
+// for nothing but its latency. What bounds it are the records that one CU writes to places of their own (optimisation step with the ordering, 2-D, us, three launches / one: 1024 points
+// 49.4 / 43.3, 2048 50.8 / 44.0, 4096 52.2 / 45.5, 8192 54.7 / 50.7, with sixteen points a thread 12 288 58.9 / 58.7, 16 384 57.1 / 59.3; 3-D, 4096 48.6 / 42.2, 8192 51.9 / 48.2).
+template <int D, int EACH>
+__global__ void __launch_bounds__(kOrderThreads)
+    order_small_kernel(const float *__restrict__ xin, uint32_t M, uint32_t *__restrict__ starts, float4 *__restrict__ records) {
+    __shared__ uint4 h4[kOrderBins / 4];
+    __shared__ uint32_t wave_sum[kOrderThreads / 64];
+    static_assert(kOrderBins == 4 * kOrderThreads, "four bins a thread");
+    uint32_t *const h = reinterpret_cast<uint32_t *>(h4);
+    const uint32_t tid = threadIdx.x;
+    float x[EACH][D];
+#pragma unroll
+    for (int u = 0; u < EACH; ++u) load_point<D>(xin, tid + u * kOrderThreads < M ? tid + u * kOrderThreads : M - 1, x[u]);
+    h4[tid] = uint4{0u, 0u, 0u, 0u};
+    __syncthreads();
+    uint32_t key[EACH], rank[EACH];
+#pragma unroll
+    for (int u = 0; u < EACH; ++u) {
+        key[u] = coarse_key<D>(x[u]);
+        rank[u] = tid + u * kOrderThreads < M ? atomicAdd(&h[key[u]], 1u) : 0u;
+    }
+    __syncthreads();
+    const uint4 c = h4[tid];
+    uint32_t incl = c.x + c.y + c.z + c.w;
+    const uint32_t mine = incl;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t v = __shfl_up(incl, off, 64);
+        if ((int)(tid & 63) >= off) incl += v;
+    }
+    if ((tid & 63) == 63) wave_sum[tid >> 6] = incl;
+    __syncthreads();
+    uint32_t at = incl - mine;
+#pragma unroll
+    for (uint32_t w = 0; w < kOrderThreads / 64; ++w) at += w < tid >> 6 ? wave_sum[w] : 0u;
+    const uint4 start{at, at + c.x, at + c.x + c.y, at + c.x + c.y + c.z};
+    h4[tid] = start;
+    reinterpret_cast<uint4 *>(starts)[tid] = start;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < EACH; ++u) {
+        const uint32_t i = tid + u * kOrderThreads;
+        if (i < M) records[h[key[u]] + rank[u]] = float4{x[u][0], x[u][1], D > 2 ? x[u][D - 1] : 0.0f, __uint_as_float(i)};
+    }
+}
+
 // Step 2: the records of a bin by the next bits of their coordinates, in pieces of at most kRefinePiece that a workgroup sorts in its registers. The first
 // kOrderBins / PER workgroups take the first pieces of PER bins each. Where points crowd a bin is many pieces, and the further workgroups take the others, side
 // by side: workgroup e the piece that starts in [e, e + 1) * kRefinePiece, which is one at most, since the piece in front of it is full and of the same bin.
@@ -304,12 +352,20 @@ TNN_API int tnn_grid_order_points(const tnn_grid_desc *desc, const float *d_x, s
         return fail(TNN_ERR_HIP, "cannot reserve %zu bytes of LDS", scan_lds);
 #define TNN_ORDER(D_)                                                                                                                  \
     do {                                                                                                                               \
-        TNN_LAUNCH((order_hist_kernel<D_>), dim3(p.n_wg), dim3(kOrderThreads), 0, s, d_x, (long long)M, p.chunk, hist, groups);         \
-        if ((rc = check_launch("order_hist_kernel"))) return rc;                                                                       \
-        TNN_LAUNCH(order_scan_kernel, dim3(kOrderGroups), dim3(kScanThreads), scan_lds, s, hist, (const uint32_t *)groups, p.n_wg);              \
-        if ((rc = check_launch("order_scan_kernel"))) return rc;                                                                       \
-        TNN_LAUNCH((order_scatter_kernel<D_>), dim3(p.n_wg), dim3(kOrderThreads), 0, s, d_x, (long long)M, p.chunk, (const uint32_t *)hist, records); \
-        if ((rc = check_launch("order_scatter_kernel"))) return rc;                                                                    \
+        if (M <= kSmallOrder) {                                                                                                        \
+            auto small = order_small_kernel<D_, kSmallOrder / kOrderThreads>;                                                          \
+            if (M <= 4 * kOrderThreads) small = order_small_kernel<D_, 4>;                                                             \
+            if (M <= 2 * kOrderThreads) small = order_small_kernel<D_, 2>;                                                             \
+            TNN_LAUNCH(small, dim3(1), dim3(kOrderThreads), 0, s, d_x, (uint32_t)M, hist, records);                                    \
+            if ((rc = check_launch("order_small_kernel"))) return rc;                                                                  \
+        } else {                                                                                                                       \
+            TNN_LAUNCH((order_hist_kernel<D_>), dim3(p.n_wg), dim3(kOrderThreads), 0, s, d_x, (long long)M, p.chunk, hist, groups);     \
+            if ((rc = check_launch("order_hist_kernel"))) return rc;                                                                   \
+            TNN_LAUNCH(order_scan_kernel, dim3(kOrderGroups), dim3(kScanThreads), scan_lds, s, hist, (const uint32_t *)groups, p.n_wg); \
+            if ((rc = check_launch("order_scan_kernel"))) return rc;                                                                   \
+            TNN_LAUNCH((order_scatter_kernel<D_>), dim3(p.n_wg), dim3(kOrderThreads), 0, s, d_x, (long long)M, p.chunk, (const uint32_t *)hist, records); \
+            if ((rc = check_launch("order_scatter_kernel"))) return rc;                                                                \
+        }                                                                                                                              \
         if (M <= (size_t)kOrderBins * 256)                                                                                             \
             TNN_LAUNCH((order_refine_kernel<D_, 4>), dim3(kOrderBins / 4 + (unsigned)(M / kRefinePiece)), dim3(kRefineThreads), 0, s, (const uint32_t *)hist, records, (long long)M); \
         else                                                                                                                           \
