@@ -138,9 +138,9 @@ def test_ordered_forward_matches_the_oracle_and_every_variant(tnn, oracle):
 
 
 @pytest.mark.parametrize("D", [2, 3])
-@pytest.mark.parametrize("M", [1, 63, 1023, 1025, 2048, 2049, 4096, 4097, 8191, 8192, 8193])
+@pytest.mark.parametrize("M", [1, 63, 1023, 1025, 2048, 2049, 4096, 4097, 8191, 8192, 8193, 65537, 69633, 2 ** 20 + 1])
 def test_batches_that_one_workgroup_orders(tnn, D, M):
-    """Up to 2, 4 and 8 points a thread, and the first batch beyond: every row once with its own coordinates, sorted by coarse cell, and the positions where the coarse cells start."""
+    """Up to 2, 4 and 8 points a thread, and beyond 3, 17, 18 and 256 histograms: every row once with its own coordinates, sorted by coarse cell, and the positions where the coarse cells start."""
     d = tnn.grid_desc(dict(n_dims=D, n_levels=4, n_features_per_level=2, log2_hashmap_size=12, base_resolution=16, per_level_scale=1.5))
     rng = np.random.default_rng(M + D)
     x = rng.uniform(-0.05, 1.05, (M, D)).astype(np.float32)
