@@ -46,14 +46,12 @@ inline uint32_t plan_shared_levels(const double *cost, uint32_t n_own, uint32_t 
 __host__ __device__
 #endif
 inline bool plan_item(const LevelPlan &plan, uint32_t n_levels, uint32_t xcd, uint32_t turn, uint32_t *level, uint32_t *chunk) {
-    const uint32_t own = plan.first[xcd + 1] - plan.first[xcd];
-    if (turn < own) {
-        *level = (plan.first[xcd] + turn) / plan.n_chunks;
-        *chunk = (plan.first[xcd] + turn) % plan.n_chunks;
-        return true;
-    }
-    *level = plan.n_own + (turn - own) / plan.each;
-    *chunk = (xcd + *level) % kXcds * plan.each + (turn - own) % plan.each; // (another eighth in every level: a batch of few chunks is not one XCD's)
+    // (one division for both kinds: it is what a workgroup of a small batch waits for)
+    const uint32_t first = plan.first[xcd], end = plan.first[xcd + 1], item = first + turn;
+    const bool own = item < end;
+    const uint32_t number = own ? item : item - end, chunks = own ? plan.n_chunks : plan.each, l = number / chunks;
+    *level = l + (own ? 0u : plan.n_own);
+    *chunk = number - l * chunks + (own ? 0u : (xcd + *level) % kXcds * plan.each); // (another eighth in every level: a batch of few chunks is not one XCD's)
     return *level < n_levels && *chunk < plan.n_chunks;
 }
 
