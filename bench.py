@@ -49,8 +49,8 @@ MEASURED_TRAFFIC_BYTES = {
     ("grid_mlp_ordered", 21): (3915783.4 * 2.0 + 264728.9) * 1024,
     ("grid_train", 18): (108943.2 * 2.0 + 236762.7) * 1024,  # the scatter kernel; an atomic request counts as a 32-byte write
     ("grid_train_ordered", 18): (248862.1 * 2.0 + 126583.5) * 1024,
-    # the whole width-128 step: forward, top launch, four pair launches, reduction with Adam
-    ("train_w128", 20): ((138126.3 + 403751.0 + 4 * 393607.4 + 77222.7) * 2.0 + (2098630.8 + 283206.9 + 4 * 229381.6 + 8674.3)) * 1024,
+    # the whole width-128 step: forward, all layers' backward passes, reduction with Adam
+    ("train_w128", 20): ((138539.8 + 1935638.5 + 77225.3) * 2.0 + (2099993.6 + 1131668.8 + 8677.4)) * 1024,
 }
 
 
@@ -600,8 +600,8 @@ class Bench:
     # --------------------------------------------------------------------------------------------------------------
     def leg_train_w128(self):
         # BASELINE config 3's widest network: width 128, 8 hidden layers, fp16, 2^20 rows. Its nine matrices do not fit one
-        # kernel: a forward pass that stores the activations, the top layer's backward launch with the loss in it, then
-        # one backward launch for the layers below it. Parity at this size: tests/test_gpu_mlp.py::test_baseline_config_3_full_size.
+        # kernel: a forward pass that stores the activations, then one launch for all layers' backward passes with the loss
+        # in it. Parity at this size: tests/test_gpu_mlp.py::test_baseline_config_3_full_size.
         np, torch, t, lib = self.np, self.torch, self.t, self.lib
         from tiny_dpcpp_nn.cabi import ptr
         from tolerances import FP16, FP32

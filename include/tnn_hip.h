@@ -363,7 +363,7 @@ int tnn_grid_order_points(const tnn_grid_desc *desc, const float *d_x, size_t M,
 int tnn_grid_forward_ordered(const tnn_grid_desc *desc, const void *d_order, const void *d_table, void *d_out, int out_dtype,
                              uint32_t padded_width, size_t M, tnn_stream_t stream);
 
-/* tnn_grid_forward, level by level: the levels go to the XCDs in turn, each of which has a level in its L2 while it gathers from it, and a
+/* tnn_grid_forward, level by level: the levels go to the XCDs, each of which has a level in its L2 while it gathers from it (large levels all XCDs take in turn), and a
  * second pass makes rows of them. Same values, bit for bit. d_order (may be NULL): the records of tnn_grid_order_points, then d_x may be
  * NULL. tnn_grid_forward_workspace_bytes: the workspace it takes where it is the faster call for M scattered points, 0 where it is not (small
  * batches, whose rows tnn_grid_forward writes the same way; few levels, or small ones; large batches of two dimensions or of levels beyond 16 MB). Any M runs, with
