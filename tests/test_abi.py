@@ -99,6 +99,48 @@ def test_scatter_workspace_of_a_batch_holds_smaller_ones(lib, dims, features, le
         assert half <= whole * 0.51
 
 
+def scatter_need(lib, d, M, ordered):
+    """Bytes that the scatter of M points says it needs where it has none to speak of, 0 where it needs none. Planned on the host and then refused: for the workspace, or
+    for its table's alignment."""
+    from tiny_dpcpp_nn import _lib
+    rc = lib.tnn_grid_backward_binned(ctypes.byref(d), None if ordered else 4096, 4096 if ordered else None, 4096, _lib.TNN_FP32, d.n_levels * d.n_features_per_level, 4100, 1, M, 4096, 1, None)
+    if rc == _lib.TNN_ERR_INVALID_ARGUMENT:
+        return 0
+    assert rc == _lib.TNN_ERR_WORKSPACE
+    return int(lib.tnn_last_error().decode().rsplit(", ", 1)[1].split()[0])
+
+
+@pytest.mark.parametrize("dims,features,levels,log2,scale,base,sides", [
+    # (points in cell order, whether all levels are binned)
+    (3, 2, 16, 19, 1.447, 16, ((4096, 0), (8192, 1), (90235, 1), (90236, 0), (114688, 0))), (3, 2, 16, 17, 1.3, 16, ((5000, 1), (73075, 1), (73076, 0))), (3, 1, 8, 19, 2.0, 16, ((8192, 1), (57344, 1), (57345, 0))),
+    (3, 2, 16, 17, 1.3, 32, ((5000, 1), (131071, 1), (131072, 0))), (3, 2, 8, 16, 1.25, 11, ((8192, 1), (10828, 1), (10829, 0))), (2, 2, 16, 19, 1.447, 16, ((65536, 0),)), (3, 2, 16, 17, 1.447, 8, ((16384, 0),)),
+    (3, 4, 8, 19, 2.0, 16, ((8192, 0), (32768, 0))), (3, 8, 8, 19, 2.0, 16, ((8192, 0), (32768, 0))), (3, 8, 6, 16, 1.25, 8, ((16387, 0), (65536, 0)))])
+def test_batches_have_boxes_where_a_cell_has_many_points(lib, dims, features, levels, log2, scale, base, sides):
+    """Up to two points a cell on the mean of the levels, and for one and two features. Boxes take levels away from the bins, which have room for two records of every pair of corners of each level."""
+    from tiny_dpcpp_nn import _lib
+    d = _lib.GridDesc()
+    assert lib.tnn_grid_desc_init(ctypes.byref(d), dims, levels, features, log2, base, scale, 0, 1, 1, _lib.TNN_FP32) == 0
+    for M, binned in sides:
+        assert (scatter_need(lib, d, M, True) >= 2 * (M << (dims - 1)) * levels * (8 + 4 * features)) == binned, M
+
+
+@pytest.mark.parametrize("features,levels,log2,scale,base", [(2, 16, 19, 1.447, 16), (2, 16, 15, 1.5, 16), (2, 8, 17, 2.0, 16), (2, 16, 17, 1.3, 32), (1, 16, 19, 1.3, 16), (1, 4, 20, 2.0, 14), (2, 12, 14, 1.25, 11), (4, 8, 19, 2.0, 16),
+                                                         (8, 6, 16, 1.25, 8)])
+def test_scatter_workspace_holds_every_smaller_plan_in_either_order(lib, features, levels, log2, scale, base):
+    """Around the sizes between which batches have no boxes, and the powers of two from which the bins take a level."""
+    from tiny_dpcpp_nn import _lib
+    d = _lib.GridDesc()
+    assert lib.tnn_grid_desc_init(ctypes.byref(d), 3, levels, features, log2, base, scale, 0, 1, 1, _lib.TNN_FP32) == 0
+    dense = int(2 * levels / sum(float(d.resolutions[l]) ** -3 for l in range(levels)))
+    sizes = sorted({2 ** k + e for k in range(8, 19) for e in (-1, 0, 1)} | {int(2 ** (8 + i / 6)) for i in range(60)} | {dense + e for e in (-1, 0, 1, 2)} | {2 ** 17 * n // levels + e for n in range(1, levels + 1) for e in (-1, 0, 1)})
+    most = 0
+    for M in sizes:
+        if M < 1:
+            continue
+        most = max([most] + [scatter_need(lib, d, M, ordered) for ordered in (False, True)])
+        assert lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), M) >= most, M
+
+
 def test_workspace_of_8192_rows_of_width_128_holds_fewer(lib):
     """From 8192 rows on a workgroup takes 128 rows instead of 64 and leaves half as many partial sums."""
     from tiny_dpcpp_nn import _lib
