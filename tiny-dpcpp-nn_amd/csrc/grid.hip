@@ -668,7 +668,7 @@ static bool enough_to_bin(size_t M, uint32_t n_levels, uint32_t n_dims) { return
 // Which route every level takes: n_big levels are left for the direct one (bp->big_level), those of `bins` for the binned one
 // (grid_binned.hip), which needs scratch memory and is planned for only when `bins` is given.
 static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, uint32_t n_dims, uint32_t F, bool ordered, bool fp32_table, size_t M, BinPlan *bins,
-                                  uint32_t *n_big_levels, uint32_t *lds) {
+                                  uint32_t *n_big_levels, uint32_t *lds, const NoBoxes *without = nullptr) { // (`without`: what no_boxes_for says of any batch)
     const int D = (int)n_dims;
     // A level goes the LDS route when its slice fits the budget and a chunk of points makes clearly more atomics
     // than the flush of the private copy does (chunk * 2^D contributions against `size` entries).
@@ -715,7 +715,7 @@ static BackwardPlan plan_backward(const GridLevels &lv, const GridParams &gp, ui
         if (M > bp.more_up_to) divide(0, 0);
     }
     // Cell order: of the other levels, those with boxes take the boxed route.
-    if (ordered && gp.n_levels > 0 && !nearest && !(bin_others() && no_boxes_for(lv, gp, n_dims, F, M)(M))) {
+    if (ordered && gp.n_levels > 0 && !nearest && !(bin_others() && (without ? *without : no_boxes_for(lv, gp, n_dims, F, M))(M))) {
         bp.bins_per_row = coarse_cells(n_dims);
         bp.n_rows = 4096 / bp.bins_per_row;
         const double per_row = (double)M / bp.n_rows;
@@ -1052,9 +1052,12 @@ TNN_API size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size
         ++n;
     }
     bool is_binned[TNN_GRID_MAX_LEVELS];
+    size_t asked = 0;
     const auto in_order = [&](size_t points) {
+        if (points == asked) return; // (levels that have boxes from the same size on, as all do that batches without boxes hold back)
+        asked = points;
         if (followed && points <= no_boxes) { // (the levels of one plan)
-            (void)plan_backward(lv, gp, D, F, true, true, points, &bins, &n_big, &lds);
+            (void)plan_backward(lv, gp, D, F, true, true, points, &bins, &n_big, &lds, &without);
             most = std::max(most, bin_scratch_bytes_up_to(bins, D, F));
             return;
         }
