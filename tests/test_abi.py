@@ -203,3 +203,16 @@ def test_networks_go_by_level_where_that_was_measured_to_be_faster(lib, dims, fe
         assert lib.tnn_grid_mlp_width_wants_levels(ctypes.byref(d), width, M) == by_level, M
         assert width != 64 or lib.tnn_grid_mlp_wants_levels(ctypes.byref(d), M) == by_level
     assert lib.tnn_grid_mlp_width_wants_levels(ctypes.byref(d), width, 0) == 0
+
+
+@pytest.mark.parametrize("features,levels,log2,base,scale,width,beyond", [
+    # 3-D, levels of more than 8 MB: whether by levels beyond 2^20 points
+    (2, 16, 22, 16, 1.447, 64, 1), (2, 4, 22, 16, 2.0, 64, 1), (2, 4, 22, 16, 2.0, 32, 1), (2, 3, 22, 64, 2.0, 64, 0), (2, 3, 22, 64, 2.0, 32, 0), (2, 1, 22, 256, 2.0, 32, 0),  # two features: by the number of levels,
+    (2, 7, 22, 16, 2.0, 16, 1), (2, 6, 22, 16, 2.0, 16, 0), (2, 2, 22, 256, 2.0, 16, 0), (1, 8, 22, 16, 2.0, 32, 1), (1, 7, 22, 16, 2.0, 32, 0), (1, 8, 22, 16, 2.0, 16, 1),  # at width 16 and of one feature of the large ones
+    (1, 7, 22, 16, 2.0, 16, 0), (4, 8, 21, 16, 2.0, 64, 0), (4, 4, 20, 64, 2.0, 16, 0)])
+def test_large_fields_go_by_level_where_that_was_measured_to_be_faster(lib, features, levels, log2, base, scale, width, beyond):
+    from tiny_dpcpp_nn import _lib
+    d = _lib.GridDesc()
+    assert lib.tnn_grid_desc_init(ctypes.byref(d), 3, levels, features, log2, base, scale, 0, 1, 1, _lib.TNN_FP32) == 0
+    assert max(d.offsets[l + 1] - d.offsets[l] for l in range(levels)) * features * 4 > 2 ** 23
+    assert [lib.tnn_grid_mlp_width_wants_levels(ctypes.byref(d), width, M) for M in (2 ** 18, 2 ** 20, 2 ** 20 + 1, 2 ** 22)] == [0, 0, beyond, beyond]

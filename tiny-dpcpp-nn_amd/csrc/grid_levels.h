@@ -38,6 +38,7 @@ __device__ __forceinline__ void load_level_pieces(typename Storage<T>::vec8 (&r)
 // entries, direct / one thread a point (grid_forward_kernel): 16 000 points 8 / 22, 16 / 41, 22 / 41; 65 000 points 23 / 26, 46 / 49, 74 / 64. (2-D 7.7 / 13,
 // 8.8 / 19, 11.5 / 19; 23 / 16, 33 / 24, 43 / 27.)
 bool grid_rows_direct(size_t M);
+size_t level_bytes(const tnn_grid_desc *desc, uint32_t l);
 size_t largest_level_bytes(const tnn_grid_desc *desc);
 // out: by levels (padded_width 0), or rows of padded_width values.
 int launch_grid_levels(const tnn_grid_desc *desc, const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *table, void *out,

@@ -404,10 +404,12 @@ using namespace tnn;
 static size_t dtype_bytes(int dtype) { return dtype == TNN_FP32 ? 4 : 2; }
 static size_t entry_bytes(const tnn_grid_desc *desc) { return desc->n_features_per_level * dtype_bytes(desc->param_dtype); }
 
+size_t tnn::level_bytes(const tnn_grid_desc *desc, uint32_t l) { return (size_t)(desc->offsets[l + 1] - desc->offsets[l]) * entry_bytes(desc); }
+
 size_t tnn::largest_level_bytes(const tnn_grid_desc *desc) {
-    size_t entries = 0;
-    for (uint32_t l = 0; l < desc->n_levels; ++l) entries = std::max<size_t>(entries, desc->offsets[l + 1] - desc->offsets[l]);
-    return entries * entry_bytes(desc);
+    size_t bytes = 0;
+    for (uint32_t l = 0; l < desc->n_levels; ++l) bytes = std::max(bytes, tnn::level_bytes(desc, l));
+    return bytes;
 }
 
 // Whether M points (more than rows are written directly for) are faster by levels and a pass for the rows than by the kernel that walks all levels of a point.
