@@ -720,6 +720,17 @@ static void test_level_plans() {
     }
 }
 
+// Levels of more than 16 MB are shared by any batch, also where their bytes take more than 32 bits; smaller ones from a number of points on.
+static void test_which_levels_are_shared() {
+    for (uint32_t n_dims : {2u, 3u})
+        for (size_t entry : {size_t(2), size_t(8), size_t(16), size_t(32)})
+            for (size_t entries = (size_t(16) << 20) / entry + 8; entries < (size_t(1) << 32); entries += entries / 4)
+                CHECK(tnn::shared_level((uint32_t)entries, entry, n_dims, 1));
+    CHECK(tnn::shared_level(1u << 30, 16, 3, 1) && tnn::shared_level(1u << 29, 32, 3, 1)); // 16 GB, in 32 bits nothing
+    CHECK(!tnn::shared_level(1u << 19, 8, 3, (size_t(1) << 20) - 1) && tnn::shared_level(1u << 19, 8, 3, size_t(1) << 20)); // 4 MB
+    CHECK(!tnn::shared_level(1u << 21, 8, 3, (size_t(1) << 18) - 1) && tnn::shared_level(1u << 21, 8, 3, size_t(1) << 18)); // 16 MB
+}
+
 // With shared levels, too, every (level, chunk) is an item of one XCD, once.
 static void test_shared_level_plans() {
     for (uint32_t n_levels : {1u, 2u, 7u, 16u}) {
@@ -759,6 +770,7 @@ int main(int argc, char **argv) {
     test_lds_reservations();
     std::printf("level plans\n");
     test_level_plans();
+    test_which_levels_are_shared();
     test_shared_level_plans();
     if (!cpu_only) {
         tnn::abi_check(tnn_device_check());

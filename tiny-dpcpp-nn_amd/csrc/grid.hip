@@ -1033,7 +1033,7 @@ TNN_API size_t tnn_grid_backward_workspace_bytes(const tnn_grid_desc *desc, size
     uint32_t n = 0, level[TNN_GRID_MAX_LEVELS], most_bins = 0;
     size_t boxed_from[TNN_GRID_MAX_LEVELS];
     for (uint32_t l = 0; l < gp.n_levels; ++l) {
-        if (lv.size[l] * F * sizeof(double) <= kCopiedBytesOrdered) continue;
+        if ((size_t)lv.size[l] * F * sizeof(double) <= kCopiedBytesOrdered) continue;
         const double R = (double)lv.resolution[l], enough = std::ceil(kBoxedMinPerCellBinned * (D == 2 ? R * R : R * R * R));
         const auto boxed = [&](size_t points) {
             return boxed_chunk_log2(lv.resolution[l], D, F, kBoxedMinPerCellBinned, points) >= 0 && points > no_boxes;

@@ -308,21 +308,6 @@ static double levels_us(const GridLevels &lv, uint32_t n_levels, uint32_t n_dims
     return cost * (double)M / (double)(1 << 23);
 }
 
-// Whether all XCDs take a level at a time, an eighth of the points each, instead of one or two of them the whole level. In cell order an eighth is a part of
-// space. Two or three large levels are in use at once then and not eight: 32 MB a level is what the 256 MB in front of the memory hold, and there is nothing to balance by
-// a guess of what levels cost, which is wrong where points share more lines than scattered ones (a picture's rows). But eight XCDs fetch the level,
-// which scattered points have to make up for: as many rows of corners for each of its lines. Field, 3-D, 16 levels, us, by XCDs / shared, scattered and a picture's rows (in
-// cell order from 5 * 2^17 points): 4 MB a level, 2^18 points 96 / 114 and 50 / 45, 2^19 180 / 198 and 81 / 69, 2^20 341 / 339 and 238 / 159; 2 MB, 2^19 162 / 162 and 76 / 66; 256 KB and
-// 1 MB, 2^19 152 / 157 and 164 / 168, rows 77 / 70 and 79 / 71, 2^20 281 / 267 and 297 / 282, 210 / 152 and 219 / 153; 8 MB, 2^18 158 / 168 and 64 / 51, 2^19 303 / 307 and 101 / 79, 2^20 512 / 491 and 304 / 175; 16 MB, 2^17 104 / 113, 2^18 198 / 204 and 83 / 58, 2^20 636 / 597 and 362 / 186;
-// 32 MB, 20 000 points 35 / 30 and 21 / 16, 2^17 121 / 122 and 62 / 40, 2^21 1286 / 1177 and 774 / 339. 2-D, 4 MB, 2^19 93 / 99, 2^20 173 / 177; 8 MB, 2^19 123 / 128, 2^20 199 / 196; 16 MB,
-// 2^19 152 / 149; 32 MB, 2^16 32 / 30, 2^20 252 / 219. (Two shared levels at a time, a coarse one's chunks between a fine one's: 32 MB 1170 -> 1145, 4 MB 328 -> 438.)
-static bool shared_level(size_t bytes, uint32_t n_dims, size_t M) {
-    const size_t MB = size_t(1) << 20, rows = M << (n_dims - 1), lines = bytes / 128;
-    if (bytes > 16 * MB) return true;
-    if (bytes > 4 * MB) return rows >= (bytes > 8 * MB ? 8 : 32) * lines;
-    return M >= (size_t(3) << 18) && rows >= 128 * lines;
-}
-
 // One launch: the points [begin, begin + M) of a batch.
 template <int D, int F, typename P, typename O>
 static int launch_levels_part(const GridLevels &lv, const GridParams &gp, const float *x, const float4 *order, const void *table, O *out, bool rows, bool large,
@@ -333,7 +318,7 @@ static int launch_levels_part(const GridLevels &lv, const GridParams &gp, const 
     double cost[TNN_GRID_MAX_LEVELS];
     for (uint32_t l = 0; l < gp.n_levels; ++l) cost[l] = level_cost(lv, l, D, F * sizeof(P), order != nullptr, batch);
     uint32_t n_own = gp.n_levels;
-    while (n_own > 0 && shared_level(lv.size[n_own - 1] * F * sizeof(P), D, batch)) --n_own;
+    while (n_own > 0 && shared_level(lv.size[n_own - 1], F * sizeof(P), D, batch)) --n_own;
     const uint32_t most = plan_shared_levels(cost, n_own, gp.n_levels, &plan);
     auto k = grid_levels_kernel<D, F, P, O, false, false>;
     if (rows) k = grid_levels_kernel<D, F, P, O, true, false>;

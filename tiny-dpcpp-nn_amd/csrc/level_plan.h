@@ -33,6 +33,21 @@ inline uint32_t plan_levels(const double *cost, uint32_t n_levels, LevelPlan *pl
     return most;
 }
 
+// Whether all XCDs take a level at a time, an eighth of the points each, instead of one or two of them the whole level. In cell order an eighth is a part of
+// space. Two or three large levels are in use at once then and not eight: 32 MB a level is what the 256 MB in front of the memory hold, and there is nothing to balance by
+// a guess of what levels cost, which is wrong where points share more lines than scattered ones (a picture's rows). But eight XCDs fetch the level,
+// which scattered points have to make up for: as many rows of corners for each of its lines. Field, 3-D, 16 levels, us, by XCDs / shared, scattered and a picture's rows (in
+// cell order from 5 * 2^17 points): 4 MB a level, 2^18 points 96 / 114 and 50 / 45, 2^19 180 / 198 and 81 / 69, 2^20 341 / 339 and 238 / 159; 2 MB, 2^19 162 / 162 and 76 / 66; 256 KB and
+// 1 MB, 2^19 152 / 157 and 164 / 168, rows 77 / 70 and 79 / 71, 2^20 281 / 267 and 297 / 282, 210 / 152 and 219 / 153; 8 MB, 2^18 158 / 168 and 64 / 51, 2^19 303 / 307 and 101 / 79, 2^20 512 / 491 and 304 / 175; 16 MB, 2^17 104 / 113, 2^18 198 / 204 and 83 / 58, 2^20 636 / 597 and 362 / 186;
+// 32 MB, 20 000 points 35 / 30 and 21 / 16, 2^17 121 / 122 and 62 / 40, 2^21 1286 / 1177 and 774 / 339. 2-D, 4 MB, 2^19 93 / 99, 2^20 173 / 177; 8 MB, 2^19 123 / 128, 2^20 199 / 196; 16 MB,
+// 2^19 152 / 149; 32 MB, 2^16 32 / 30, 2^20 252 / 219. (Two shared levels at a time, a coarse one's chunks between a fine one's: 32 MB 1170 -> 1145, 4 MB 328 -> 438.)
+inline bool shared_level(uint32_t entries, size_t entry_bytes, uint32_t n_dims, size_t M) {
+    const size_t MB = size_t(1) << 20, bytes = entries * entry_bytes, rows = M << (n_dims - 1), lines = bytes / 128;
+    if (bytes > 16 * MB) return true;
+    if (bytes > 4 * MB) return rows >= (bytes > 8 * MB ? 8 : 32) * lines;
+    return M >= (size_t(3) << 18) && rows >= 128 * lines;
+}
+
 // The levels from n_own on are shared, those in front dealt out by cost. Returns the most items an XCD has.
 inline uint32_t plan_shared_levels(const double *cost, uint32_t n_own, uint32_t n_levels, LevelPlan *plan) {
     plan->n_own = n_own;
