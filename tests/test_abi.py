@@ -141,6 +141,17 @@ def test_scatter_workspace_holds_every_smaller_plan_in_either_order(lib, feature
         assert lib.tnn_grid_backward_workspace_bytes(ctypes.byref(d), M) >= most, M
 
 
+def test_order_buffer_has_what_its_route_needs(lib):
+    """16 bytes a point; up to 8192 points where the 4096 coarse cells start, beyond a histogram for 4096 points (256 at most) and the cells' totals. A buffer holds every smaller batch."""
+    from tiny_dpcpp_nn import _lib
+    d = _lib.GridDesc()
+    assert lib.tnn_grid_desc_init(ctypes.byref(d), 3, 16, 2, 19, 16, 1.447, 0, 1, 1, _lib.TNN_FP32) == 0
+    sizes = [1, 16, 17, 4096, 4097, 8192, 8193, 12288, 12289, 2 ** 18, 2 ** 20, 2 ** 20 + 1, 2 ** 22]
+    needs = [lib.tnn_grid_order_bytes(ctypes.byref(d), M) for M in sizes]
+    assert needs == [(16 * M + 255) // 256 * 256 + 16384 * (1 if M <= 8192 else min(256, (M + 4095) // 4096) + 1) + 256 for M in sizes]
+    assert needs == sorted(needs)
+
+
 def test_workspace_of_8192_rows_of_width_128_holds_fewer(lib):
     """From 8192 rows on a workgroup takes 128 rows instead of 64 and leaves half as many partial sums."""
     from tiny_dpcpp_nn import _lib

@@ -39,8 +39,9 @@ static OrderPlan order_plan(size_t M) {
     long long chunk = ((long long)M + wg - 1) / wg;
     p.chunk = (chunk + kOrderThreads - 1) / kOrderThreads * kOrderThreads;
     p.record_bytes = order_record_bytes(M);
-    p.hist_bytes = (size_t)p.n_wg * kOrderBins * sizeof(uint32_t);
-    p.total_bytes = kOrderBins * sizeof(uint32_t);
+    // (one workgroup's points need the starts of the bins alone)
+    p.hist_bytes = (M <= kSmallOrder ? 1 : (size_t)p.n_wg) * kOrderBins * sizeof(uint32_t);
+    p.total_bytes = M <= kSmallOrder ? 0 : kOrderBins * sizeof(uint32_t);
     return p;
 }
 
