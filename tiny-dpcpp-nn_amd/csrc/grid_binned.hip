@@ -154,8 +154,9 @@ __device__ __forceinline__ size_t run_slot(uint32_t first_quad, uint32_t bin, ui
 // No one unit bounds it (3-D, 2^19 points, 10 levels, 99 us): 346 MB written, the records all in whole 64-byte requests, at 3.5 TB/s where a
 // fill reaches 6.9; the vector units are at work 45 % of the time, LDS a sixth, and a wave waits for 41 % of its.
 // TAKEN: the reduction of the training kernel that left dL/dy (and what it clears) is the first workgroups of this launch: both wait for that kernel only, and what adds to the table
-// waits for both. It was a launch of its own of 4 to 7 us, a chain of loads and one sum (optimisation step with the ordering, us, before / now: 2-D, 20 000 points 68.4 / 64.6, 2^16 82.0 / 77.4, 2^18
-// 210 / 203; 3-D, 2^17 257 / 253; a module's forward and backward pass, 2-D, 2^18 177 / 171). Registers for eight waves a SIMD, as without.
+// waits for both. It was a launch of its own of 4 to 7 us, a chain of loads and one sum, and makes this one longer (2-D, 2^18 points, with Adam: 6.9 us gone, 15.3 -> 18.1 here). Optimisation step with the
+// ordering, 16 levels, us, before / now: 2-D, 2^17 entries a level, 20 000 points 68.4 / 64.6, 2^15, 2^16 points 82.0 / 77.4, 2^19, 2^18 210 / 203; 3-D, 2^19, 2^17 257 / 253; a module's forward and backward pass,
+// 2-D, 2^19, 2^18 177 / 171. Registers for eight waves a SIMD, as without.
 template <int D, int F, typename G, typename TAKEN = std::false_type>
 __global__ void __launch_bounds__((BinShape<D, F>::kThreads), (std::is_same<TAKEN, TrainReduce>::value ? 8 : 1))
     grid_bin_kernel(const GridParams gp, const BinPlan bp, const GradLayout dl, const float *__restrict__ xin,

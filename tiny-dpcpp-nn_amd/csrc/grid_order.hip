@@ -109,7 +109,7 @@ __device__ __forceinline__ uint4 bin_starts(const uint4 c, uint32_t at) { return
 // Step 1b: what the workgroups in front of a workgroup have in each bin, in place, and every bin's total; where the bins start follows from the totals, which
 // every workgroup of the next step adds up by itself. A workgroup takes sixteen bins, a lane of it every sixteenth histogram's count of one, all under way at once; in a bin the histograms lie
 // in that order, the first one first. (With the bins' starts formed here, 64 workgroups read all totals of runs of bins, and a bin's counts one after the other in LDS: 256 histograms
-// 14.3 us, 64 histograms 5.5. Optimisation step, 2-D, 2^18 points 171.0 -> 166.4 us; encoding, 3-D, 2^20 points, forward and backward 887 -> 873; a field of a picture's rows 167 -> 158.)
+// 14.1 -> 6.1 us, 64 histograms 5.5 -> 4.1. Optimisation step, 2-D, 16 levels of 2^17 entries, 2^18 points 171.0 -> 166.4 us; encoding, 3-D, 2^20 points, forward and backward 887 -> 873; a field of a picture's rows 167 -> 158.)
 constexpr int kScanThreads = 256;
 constexpr int kScanBins = 16;
 __global__ void __launch_bounds__(kScanThreads)
@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(kOrderThreads)
 }
 
 // Step 1 of a batch that one workgroup holds in its registers: histogram, starting positions and places in one launch instead of three, each of which was some 3 us
-// for nothing but its latency. What bounds it are the records that one CU writes to places of their own (optimisation step with the ordering, 2-D, us, three launches / one: 1024 points
+// for nothing but its latency. What bounds it are the records that one CU writes to places of their own (optimisation step with the ordering, 16 levels of 2^15 entries, 2-D, us, three launches / one: 1024 points
 // 49.4 / 43.3, 2048 50.8 / 44.0, 4096 52.2 / 45.5, 8192 54.7 / 50.7, with sixteen points a thread 12 288 58.9 / 58.7, 16 384 57.1 / 59.3; 3-D, 4096 48.6 / 42.2, 8192 51.9 / 48.2).
 template <int D, int EACH>
 __global__ void __launch_bounds__(kOrderThreads)
