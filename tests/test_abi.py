@@ -218,9 +218,9 @@ def test_networks_go_by_level_where_that_was_measured_to_be_faster(lib, dims, fe
 
 @pytest.mark.parametrize("features,levels,log2,base,scale,width,beyond", [
     # 3-D, levels of more than 8 MB: whether by levels beyond 2^20 points
-    (2, 16, 22, 16, 1.447, 64, 1), (2, 4, 22, 16, 2.0, 64, 1), (2, 4, 22, 16, 2.0, 32, 1), (2, 3, 22, 64, 2.0, 64, 0), (2, 3, 22, 64, 2.0, 32, 0), (2, 1, 22, 256, 2.0, 32, 0),  # two features: by the number of levels,
-    (2, 7, 22, 16, 2.0, 16, 1), (2, 6, 22, 16, 2.0, 16, 0), (2, 2, 22, 256, 2.0, 16, 0), (1, 8, 22, 16, 2.0, 32, 1), (1, 7, 22, 16, 2.0, 32, 0), (1, 8, 22, 16, 2.0, 16, 1),  # at width 16 and of one feature of the large ones
-    (1, 7, 22, 16, 2.0, 16, 0), (4, 8, 21, 16, 2.0, 64, 0), (4, 4, 20, 64, 2.0, 16, 0)])
+    (2, 16, 22, 16, 1.447, 64, 1), (2, 3, 22, 64, 2.0, 64, 1), (2, 3, 22, 64, 2.0, 32, 1), (2, 1, 22, 256, 2.0, 32, 1),  # two features, width 32 and more: all;
+    (2, 7, 22, 16, 2.0, 16, 1), (2, 6, 22, 16, 2.0, 16, 0), (2, 2, 22, 256, 2.0, 16, 0), (2, 3, 22, 256, 2.0, 16, 1), (2, 1, 22, 128, 2.0, 16, 0),  # at width 16 and of one feature by how many are
+    (1, 7, 22, 16, 2.0, 32, 1), (1, 6, 22, 16, 2.0, 32, 0), (1, 7, 22, 16, 2.0, 16, 1), (1, 6, 22, 16, 2.0, 16, 0), (4, 8, 21, 16, 2.0, 64, 0), (4, 4, 20, 64, 2.0, 16, 0)])  # as large as the largest
 def test_large_fields_go_by_level_where_that_was_measured_to_be_faster(lib, features, levels, log2, base, scale, width, beyond):
     from tiny_dpcpp_nn import _lib
     d = _lib.GridDesc()

@@ -139,17 +139,18 @@ static bool levels_pay(const tnn_grid_desc *grid, int width, size_t M) {
     }
     // 12 and 16 levels: 0.3 to 0.7 and 0.5 to 0.9; of more than 8 MB, 2^15 points 0.65 and 0.97, 2^16 0.89 and 1.34. 8 levels 0.8 and 1.0 to 1.1.
     if (L > 10 && M < (size_t(1) << 15)) return width >= 32 && (M < 24000 || (F <= 2 && largest <= 8 * MB));
-    // Twice an XCD's L2 and more, which all XCDs share (shared_level). Drawn with 1 to 24 levels, one and two features, widths 16 to 64 and 2^20 to 2^22 points (2650 configurations; one kernel's time = 1,
-    // scattered points and a picture's rows): with four such levels or more, or two features, width 32 and more than three levels, 0.87 and 0.73, 1.5 % more than a tenth slower for one or the
-    // other; all others 1.09 (up to 1.44) and 0.86, 47 %. 16 levels of 32 MB, width 64, 2^21 points 1304 / 1170 us and 430 / 328; 8 levels of 16 MB, width 16, one feature 429 / 419 and 219 / 149; two levels
-    // of 32 MB, width 16 243 / 270 and 119 / 102; three, width 64, 300 / 330 and 265 / 168. Four features, 8 levels, 2^19 points 209 / 215 and 76 / 99.
+    // Twice an XCD's L2 and more, which all XCDs share (shared_level). Drawn with 1 to 24 levels, one and two features, widths 16 to 64 and 2^20 to 2^22 points (4906 configurations, half of them of one to
+    // five levels; one kernel's time = 1, scattered points and a picture's rows): two features and width 32 and more 0.91 and 0.62; of the others, whose waves are more, those with three levels as large as
+    // the largest (whose tables are full: the levels that cost lines) 0.89 and 0.79; in all 4 % more than a tenth slower for one or the other. With fewer such levels 1.09 (up to 1.57) and 0.81, 50 %. 16 levels of
+    // 32 MB, width 64, 2^21 points 1304 / 1170 us and 430 / 328; three, two of them of more than 8 MB 248 / 199 and 222 / 152; two of 32 MB, width 16 243 / 270 and 119 / 102. Four features, 8 levels,
+    // 2^19 points 209 / 215 and 76 / 99.
     // The points are in cell order from 5 * 2^17 on, and without it 2^19 take 1.0 to 1.3 of one kernel's time for 12 levels and fewer, 0.92 to 1.0 for 16 of two features. Between, such fields would be as much faster as
     // beyond (16 levels of 32 MB, 3 * 2^18 points 0.88 and 0.91, 2^20 0.87 and 1.0). They are one kernel up to 2^20 points not because that were faster, but because callers and tests
     // count on its taking no scratch memory there.
     if (largest > 8 * MB) {
-        uint32_t n_large = 0;
-        for (uint32_t l = 0; l < L; ++l) n_large += level_bytes(grid, l) > 8 * MB;
-        return F <= 2 && M > (size_t(1) << 20) && (n_large > 3 || (F == 2 && width >= 32 && L > 3));
+        uint32_t n_largest = 0;
+        for (uint32_t l = 0; l < L; ++l) n_largest += level_bytes(grid, l) == largest;
+        return F <= 2 && M > (size_t(1) << 20) && ((F == 2 && width >= 32) || n_largest > 2);
     }
     if (largest > MB && width == 16) return false;
     // Two features: 0.3 to 0.8 and 0.2 to 0.9. Four and eight: 6 levels 2^18 points 0.8 to 1.0 and 0.6, 8 levels 1.0 and 0.9, 2^19 1.1 and 1.4.
