@@ -112,11 +112,11 @@ def scatter_need(lib, d, M, ordered):
 
 @pytest.mark.parametrize("dims,features,levels,log2,scale,base,sides", [
     # (points in cell order, whether all levels are binned)
-    (3, 2, 16, 19, 1.447, 16, ((4096, 0), (8192, 1), (90235, 1), (90236, 0), (114688, 0))), (3, 2, 16, 17, 1.3, 16, ((5000, 1), (73075, 1), (73076, 0))), (3, 1, 8, 19, 2.0, 16, ((8192, 1), (57344, 1), (57345, 0))),
-    (3, 2, 16, 17, 1.3, 32, ((5000, 1), (131071, 1), (131072, 0))), (3, 2, 8, 16, 1.25, 11, ((8192, 1), (10828, 1), (10829, 0))), (2, 2, 16, 19, 1.447, 16, ((65536, 0),)), (3, 2, 16, 17, 1.447, 8, ((16384, 0),)),
+    (3, 2, 16, 19, 1.447, 16, ((4096, 0), (8192, 1), (122880, 1), (122881, 0))), (3, 1, 8, 19, 2.0, 16, ((8192, 1), (114688, 1), (114689, 0))), (3, 2, 8, 16, 1.3, 16, ((8192, 1), (109817, 1), (109818, 0))),
+    (3, 2, 16, 17, 1.3, 32, ((5000, 1), (131071, 1), (131072, 0))), (3, 2, 7, 19, 2.0, 16, ((16384, 1), (50176, 1), (50177, 0))), (3, 2, 16, 17, 1.3, 15, ((5000, 1), (60489, 1), (60490, 0))), (3, 2, 8, 16, 1.25, 11, ((8192, 1), (10828, 1), (10829, 0))), (2, 2, 16, 19, 1.447, 16, ((65536, 0),)), (3, 2, 16, 17, 1.447, 8, ((16384, 0),)),
     (3, 4, 8, 19, 2.0, 16, ((8192, 0), (32768, 0))), (3, 8, 8, 19, 2.0, 16, ((8192, 0), (32768, 0))), (3, 8, 6, 16, 1.25, 8, ((16387, 0), (65536, 0)))])
 def test_batches_have_boxes_where_a_cell_has_many_points(lib, dims, features, levels, log2, scale, base, sides):
-    """Up to two points a cell on the mean of the levels, and for one and two features. Boxes take levels away from the bins, which have room for two records of every pair of corners of each level."""
+    """Up to two points a cell on the mean of the levels, six of eight levels and more from 16 cells a side on, and for one and two features. Boxes take levels away from the bins, which have room for two records of every pair of corners of each level."""
     from tiny_dpcpp_nn import _lib
     d = _lib.GridDesc()
     assert lib.tnn_grid_desc_init(ctypes.byref(d), dims, levels, features, log2, base, scale, 0, 1, 1, _lib.TNN_FP32) == 0
@@ -132,7 +132,7 @@ def test_scatter_workspace_holds_every_smaller_plan_in_either_order(lib, feature
     d = _lib.GridDesc()
     assert lib.tnn_grid_desc_init(ctypes.byref(d), 3, levels, features, log2, base, scale, 0, 1, 1, _lib.TNN_FP32) == 0
     dense = int(2 * levels / sum(float(d.resolutions[l]) ** -3 for l in range(levels)))
-    sizes = sorted({2 ** k + e for k in range(8, 19) for e in (-1, 0, 1)} | {int(2 ** (8 + i / 6)) for i in range(60)} | {dense + e for e in (-1, 0, 1, 2)} | {2 ** 17 * n // levels + e for n in range(1, levels + 1) for e in (-1, 0, 1)})
+    sizes = sorted({2 ** k + e for k in range(8, 19) for e in (-1, 0, 1)} | {int(2 ** (8 + i / 6)) for i in range(60)} | {n * dense + e for n in (1, 3) for e in (-1, 0, 1, 2, 3)} | {2 ** 17 * n // levels + e for n in range(1, levels + 1) for e in (-1, 0, 1)})
     most = 0
     for M in sizes:
         if M < 1:

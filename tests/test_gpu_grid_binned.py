@@ -230,9 +230,9 @@ def test_workspace_of_a_batch_holds_a_smaller_one(tnn, cfg, M):
         assert float((grad - ref).abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max()))
 
 
-@pytest.mark.parametrize("features,levels,base,M", [(2, 16, 16, 90235), (2, 16, 16, 90236), (2, 16, 16, 122880), (2, 16, 16, 122881), (2, 8, 16, 5000), (1, 16, 16, 40000), (4, 6, 16, 20000), (2, 16, 8, 40000), (8, 3, 16, 16384)])
+@pytest.mark.parametrize("features,levels,base,M", [(2, 16, 16, 122880), (2, 16, 16, 122881), (2, 6, 12, 14358), (2, 6, 12, 14359), (2, 8, 16, 5000), (1, 16, 16, 40000), (4, 6, 16, 20000), (2, 16, 8, 40000), (8, 3, 16, 16384)])
 def test_batches_in_cell_order_without_boxes(tnn, oracle, features, levels, base, M):
-    """Three dimensions, on both sides of the size up to which all levels are binned (two points a cell on their mean), and with boxes: larger batches, four and eight features, and levels that are
+    """Three dimensions, on both sides of the size up to which all levels are binned (2^17 points less what copies save, or two points a cell on the mean of the levels), and with boxes: larger batches, four and eight features, and levels that are
     copied (base 8), whose launch boxes share. The bar of the plain scatter."""
     cfg = dict(CFG3, n_features_per_level=features, n_levels=levels, base_resolution=base)
     rng = np.random.default_rng(M + features)

@@ -621,15 +621,15 @@ static int boxed_chunk_log2(uint32_t resolution, uint32_t n_dims, uint32_t F, do
 }
 
 // From and up to how many points boxes do not pay beside bins. Where no level is copied whole either, as in three dimensions, and the bins take all, batches without boxes have no launch
-// for them: optimisation step with the ordering, 3-D, us, with boxes / all levels binned: 16 levels of 2^15 entries, 2^12 points 59 / 49, 2^13 63 / 52, 2^15 85 / 71; of
-// 2^19 2^13 142 / 129, 2^15 165 / 150; 8 levels of 2^17 entries 64 / 52, 77 / 65; of 2^19 72 / 60, 89 / 73. (Where the bins refuse
+// for them: optimisation step with the ordering, 3-D, us, with boxes / all levels binned: 16 levels of 2^15 entries, 2^12 points 59 / 49, 2^13 63 / 52, 2^15 85 / 71, 114 688 160 / 144; of
+// 2^19 2^13 142 / 129, 2^15 165 / 150, 114 688 234 / 217; 8 levels of 2^17 entries 64 / 52, 77 / 65, 124 / 112; of 2^19 72 / 60, 89 / 73, 133 / 121, 2^18 184 / 190. (Where the bins refuse
 // levels of too few points the launch stays: 16 levels of 2^19, 2^12 points 136 / 144. 2-D, where the coarsest levels are copied, 2^13 55 / 56, 2^16 77 / 82.)
-// Up to two points a cell, on the mean of the levels: points that crowd a part of the volume queue up on the few entries of coarse levels, which boxes hold as well as even ones. The scatter
-// alone, all levels binned over boxes, 815 drawn grids of one and two features and batches of 2^12 to 122 000 points, on average, and how many are more than a tenth slower: up to two points
-// a cell even ones 0.68 (none), a picture's rows 0.79 (1 %), normally distributed 0.77 (1 %), in a cube of half the side 0.76 (none), of a fifth 0.83 (6 %), of a twentieth 0.81 (9 %); two to
-// four 0.72 (1), 0.97 (22), 0.94 (23), 0.90 (9), 1.10 (47), 0.97 (35); beyond 0.84, 1.15, 1.19, 1.15, 1.38, 1.22. (Two features, 16 levels of 2^17 entries, scale 1.3, 114 688 points, 3.2 a cell: 81 / 64 and, in a
-// cube of a twentieth, 371 / 630.) Records of four and eight features lose at either end: 8 levels of 2^19 entries, 2^13 even points 32 / 36 and 40 / 56, 2^15 in a cube of a twentieth 212 / 327 and 397 / 640;
-// eight features, 6 small levels (base 8, scale 1.25), 2^16 points 65 / 95 and 294 / 1190.
+// Points that crowd a part of the volume queue up on the few entries of coarse levels, which boxes hold as well as even ones, the more of them a cell has on the mean of the levels and the more of the levels are
+// such. The scatter alone, all levels binned over boxes, 815 drawn grids of one and two features and batches of 2^12 to 122 000 points, on average, and how many are more than a tenth slower: up to
+// two points a cell even ones 0.68 (none), a picture's rows 0.79 (1 %), normally distributed 0.77 (1 %), in a cube of half the side 0.76 (none), of a fifth 0.83 (6 %), of a twentieth 0.81 (9 %); two
+// to six, 8 levels and more from 16 cells a side on, 0.75 (none), 0.94, 0.81, 0.87, 0.95, 1.13 (56 %: what lies in one of 8000 parts of the volume); fewer or coarser levels two to
+// four 0.72, 0.98, 0.98, 0.92, 1.14, 0.94, beyond 0.85, 1.16, 1.21, 1.17, 1.41, 1.23, and these have boxes there. Records of four and eight features lose at either end: 8 levels of 2^19 entries, 2^13 even points
+// 32 / 36 and 40 / 56, 2^15 in a cube of a twentieth 212 / 327 and 397 / 640; eight features, 6 small levels (base 8, scale 1.25), 2^16 points 65 / 95 and 294 / 1190.
 // And up to as many points as take no more memory for it than 2^17 in the caller's order, which copy some levels (122 880 for 16 levels, one of them copied); smaller batches may take more
 // than in the caller's order (8 levels of 2^19 entries, 2^13 points 9 MB and none; 8 small levels, base 11, scale 1.25, 10 828 points 12 MB and none).
 struct NoBoxes {
@@ -640,17 +640,19 @@ struct NoBoxes {
 static NoBoxes no_boxes_for(const GridLevels &lv, const GridParams &gp, uint32_t n_dims, uint32_t F, size_t M = 0) {
     NoBoxes r;
     if (n_dims != 3 || F > 2 || gp.n_levels > kMaxBinned || M >= kMoreBinnedBelow) return r;
-    uint32_t copied = 0, largest = 0;
+    uint32_t copied = 0, largest = 0, coarsest = ~0u;
     double per_cell = 0.0; // of one point, on all levels
     for (uint32_t l = 0; l < gp.n_levels; ++l) {
         const size_t feature_bytes = (size_t)lv.size[l] * sizeof(double);
         if (feature_bytes * F <= kCopiedBytesOrdered) return r;
         copied += feature_bytes <= kPrivateLdsBytes;
         largest = std::max(largest, lv.size[l]);
+        coarsest = std::min(coarsest, lv.resolution[l]);
         const double R = (double)lv.resolution[l];
         per_cell += 1.0 / (R * R * R);
     }
-    const size_t crowded = (size_t)std::min(2.0 * gp.n_levels / per_cell, (double)kMoreBinnedBelow);
+    const double a_cell = gp.n_levels >= 8 && coarsest >= 16 ? 6.0 : 2.0;
+    const size_t crowded = (size_t)std::min(a_cell * gp.n_levels / per_cell, (double)kMoreBinnedBelow);
     const size_t to = std::min({kMoreBinnedBelow * (gp.n_levels - copied) / gp.n_levels, kMoreBinnedBelow - 1, crowded});
     if (M > to) return r;
     BinPlan bins{};
