@@ -37,12 +37,12 @@ inline uint32_t plan_levels(const double *cost, uint32_t n_levels, LevelPlan *pl
 // space. Two or three large levels are in use at once then and not eight: 32 MB a level is what the 256 MB in front of the memory hold, and there is nothing to balance by
 // a guess of what levels cost, which is wrong where points share more lines than scattered ones (a picture's rows). But eight XCDs fetch the level,
 // which scattered points have to make up for: as many rows of corners for each of its lines. Field, 3-D, 16 levels, us, by XCDs / shared, scattered and a picture's rows (in
-// cell order from 5 * 2^17 points): 4 MB a level, 2^18 points 96 / 114 and 50 / 45, 2^19 180 / 198 and 81 / 69, 2^20 341 / 339 and 238 / 159; 2 MB, 2^19 162 / 162 and 76 / 66; 256 KB and
+// cell order from 5 * 2^17 points): 4 MB a level, 2^18 points 96 / 114 and 50 / 45, 2^19 180 / 198 and 81 / 69, 700 000 207 / 213 and 147 / 101, 10^6 289 / 292 and 204 / 133, 2^20 341 / 339 and 238 / 159 (8 levels 122 / 132 and 63 / 56, 170 / 180 and 88 / 78); 2 MB, 2^19 162 / 162 and 76 / 66; 256 KB and
 // 1 MB, 2^19 152 / 157 and 164 / 168, rows 77 / 70 and 79 / 71, 2^20 281 / 267 and 297 / 282, 210 / 152 and 219 / 153; 8 MB, 2^18 158 / 168 and 64 / 51, 2^19 303 / 307 and 101 / 79, 2^20 512 / 491 and 304 / 175; 16 MB, 2^17 104 / 113, 2^18 198 / 204 and 83 / 58, 2^20 636 / 597 and 362 / 186;
 // 32 MB, 20 000 points 35 / 30 and 21 / 16, 2^17 121 / 122 and 62 / 40, 2^21 1286 / 1177 and 774 / 339. 8 levels, 2^20 4 MB 157 / 154 and 111 / 73, 32 MB 281 / 253 and 181 / 81. 2-D, 4 MB, 2^19 93 / 99, 2^20 173 / 177; 8 MB, 2^19 123 / 128, 2^20 199 / 196; 16 MB,
 // 2^19 152 / 149; 32 MB, 2^16 32 / 30, 2^20 252 / 219;
 // 256 KB and 2 MB, 8 levels, 2^20 86 / 86 and 89 / 89, rows 60 / 54 and 61 / 53, 16 levels 122 / 121 and 120 / 125, rows 103 / 98 and 102 / 101. So scattered points lose 1 to 5 % at the sizes from which a rule
-// begins (8 MB, 2^19; 16 MB, 2^18; 2-D, 2 MB, 2^20), for the up to 30 % that rows gain there. Levels of up to 4 MB are an XCD's own as long as its L2 holds them, and begin at 3 * 2^18 points only:
+// begins (8 MB, 2^19; 16 MB, 2^18; 2-D, 2 MB, 2^20), for the up to 30 % that rows gain there. Levels of up to 4 MB an XCD's own L2 holds, and they are shared from 3 * 2^18 points on only:
 // a level of 8 MB is shared by fewer points than one of 2 MB. (Two shared levels at a time, a coarse one's chunks between a fine one's: 32 MB 1170 -> 1145, 4 MB 328 -> 438.)
 inline bool shared_level(uint32_t entries, size_t entry_bytes, uint32_t n_dims, size_t M) {
     const size_t MB = size_t(1) << 20, bytes = entries * entry_bytes, rows = M << (n_dims - 1), lines = bytes / 128;
